@@ -38,10 +38,11 @@ const char* vrwkv_last_error(void);      /* thread-local, never NULL */
 
 /* Tuning / testing switches, process-wide (no counterpart in the reference).  Names: "biwkv_l", "biwkv_s",
  * "biwkv_grid", "biwkv_no_stage", "biwkv_no_resident", "biwkv_bwd_serial", "wkv6_fwd_scalar", "wkv6_bwd_scalar",
- * "wkv6_bwd_unfused"; 0 = default behaviour.  The initial value of <name> is that of the environment variable
+ * "wkv6_bwd_unfused", "wkv6_segments"; 0 = default behaviour.  The initial value of <name> is that of the environment variable
  * VRWKV_<NAME> when the library first looks at any switch; the entry points never read the environment afterwards.
  * vrwkv_set_option rejects (VRWKV_INVALID_ARG) a value the plans would ignore: biwkv_l takes 0, 4, 8, 16, 25, 28 (tokens
- * per wave), biwkv_s 0 or 2..8 (waves per workgroup), biwkv_grid 0 or a positive workgroup count, the others 0 or 1. */
+ * per wave), biwkv_s 0 or 2..8 (waves per workgroup), biwkv_grid 0 or a positive workgroup count, wkv6_segments 0..64 (segments a sequence
+ * is cut into), the others 0 or 1. */
 int vrwkv_set_option(const char* name, int value);
 int vrwkv_get_option(const char* name, int* value);
 
@@ -107,8 +108,9 @@ int vrwkv_biwkv_bwd(const float* w, const float* u, const void* k, const void* v
  * w_is_ew = 0: w is the raw decay logit and the kernel uses d = exp(-exp(w)), i.e. it folds in
  *              the `ew = -exp(w)` of WKV_6.forward (vrwkv6.py:48);
  * w_is_ew = 1: w already holds ew = -exp(w_raw), as the reference extension receives it.
- * State and accumulation are fp32.  No limit on T (T*C < 2^29).  No workspace is needed: the size
- * function returns 0 and workspace may be NULL (both kept so that every operator has the same shape). */
+ * State and accumulation are fp32.  No limit on T (T*C < 2^29).  workspace: the size function returns 0 unless the call has
+ * few, long sequences, which are then cut into segments that exchange their states through it; 16-byte aligned.  It may
+ * be NULL (or too small) for every call: the sequences then run uncut. */
 size_t vrwkv_wkv6_fwd_workspace_bytes(int B, int T, int C, int H);
 int vrwkv_wkv6_fwd(const void* r, const void* k, const void* v, const void* w, const float* u,
                    float* y, int B, int T, int C, int H, int rkv_dtype, int w_dtype, int w_is_ew,

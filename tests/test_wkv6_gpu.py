@@ -153,3 +153,26 @@ def test_phase_stamping_entry_point(ops):
     assert lib.vrwkv_wkv6_fwd_phases(*args, st.data_ptr(), nb - 8, stream) == 5
     assert lib.vrwkv_wkv6_fwd_phases(*args, None, nb, stream) == 1
     assert lib.vrwkv_wkv6_fwd_phases_bytes(0, T, H) == 0
+
+
+@pytest.mark.parametrize("T,segments", [(33, 2), (64, 2), (65, 3), (250, 4), (250, 8), (577, 5), (2080, 64)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_sequences_cut_into_segments(ops, T, segments, dtype):
+    """Sequences handed to several workgroups (a forced number of segments: one chunk each, a last segment of one token,
+    the most there are) meet the oracle like whole ones."""
+    from oracle import clib
+    r, k, v, w, u = gen(2, T, 2, seed=T + segments, w_mean=-3.0, w_std=1.0)
+    with ops.option("wkv6_segments", segments):
+        y, *inputs = run(ops, r, k, v, w, u, 2, dtype, dtype)
+    assert rel_err(y, clib.wkv6_fwd(*inputs, u, 2)) <= TOL
+
+
+def test_cut_sequence_with_a_decay_out_of_range(ops):
+    """One of four sequences decays by more than e^-60 inside a chunk of its last segment: it is redone by the sequential
+    recurrence, the others are not disturbed."""
+    from oracle import clib
+    r, k, v, w, u = gen(2, 200, 2, seed=7, w_mean=-3.0, w_std=1.0)
+    w[1, 180:190, 64:] = 3.0
+    with ops.option("wkv6_segments", 3):
+        y, *inputs = run(ops, r, k, v, w, u, 2)
+    assert rel_err(y, clib.wkv6_fwd(*inputs, u, 2)) <= TOL

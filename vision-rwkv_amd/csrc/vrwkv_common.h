@@ -27,6 +27,7 @@ enum Option {
     OPT_WKV6_FWD_SCALAR,    // sequential-state wkv6 forward kernel
     OPT_WKV6_BWD_SCALAR,    // sequential wkv6 backward sweeps
     OPT_WKV6_BWD_UNFUSED,   // one launch per wkv6 backward scan
+    OPT_WKV6_SEGMENTS,      // segments a wkv6 sequence is cut into
     N_OPTIONS
 };
 int option(Option o);

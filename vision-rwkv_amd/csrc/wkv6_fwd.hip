@@ -34,6 +34,22 @@ int validate(int B, int T, int C, int H, int rkv_dtype, int w_dtype) {
     return VRWKV_OK;
 }
 
+// Segments per sequence of a call (1: not split); OPT_WKV6_SEGMENTS forces a number (testing).
+int segments(int B, int T, int H) {
+    const int nchunk = (T + LC - 1) / LC, forced = option(OPT_WKV6_SEGMENTS);
+    if (forced > 0) {
+        const int n = forced < nchunk ? forced : nchunk, cps = (nchunk + n - 1) / n;
+        return (nchunk + cps - 1) / cps;
+    }
+    return wkv6_segments((long long)B * H, nchunk, device_cus());
+}
+
+// the state kernel reads two neighbouring channels at a time
+template <typename IO, typename WT>
+bool pairs_aligned(const void* k, const void* v, const void* w) {
+    return !((((uintptr_t)k | (uintptr_t)v) & (2 * sizeof(IO) - 1)) || ((uintptr_t)w & (2 * sizeof(WT) - 1)));
+}
+
 template <typename IO, typename WT>
 int launch_scalar(const void* r, const void* k, const void* v, const void* w, const float* u, float* y,
                   int B, int T, int C, int H, bool w_is_ew, hipStream_t st) {
@@ -52,20 +68,32 @@ int launch_scalar(const void* r, const void* k, const void* v, const void* w, co
     return check_launch("wkv6_fwd");
 }
 
-// One launch: both passes of a (b,h) sequence side by side in one workgroup, out-of-range sequences
-// redone in place by the sequential recurrence.
-template <typename IO, typename WT>
-int launch_chunked(const void* r, const void* k, const void* v, const void* w, const float* u, float* y,
-                   int B, int T, int C, int H, bool w_is_ew, hipStream_t st) {
-    const dim3 grid(B * H), block(64 * FW_WAVES);
+// Both passes of a (b,h) sequence side by side in one workgroup, out-of-range sequences redone in place by the sequential
+// recurrence; few long sequences are cut into segments first (wkv6_segment.h) when the caller's workspace allows it.
+template <typename IO, typename WT, bool EW>
+int launch_chunked(const void* r, const void* k, const void* v, const void* w, const float* u, float* y, void* ws, size_t ws_bytes,
+                   int B, int T, int C, int H, hipStream_t st) {
+    const dim3 block(64 * FW_WAVES);
     const IO* rr = static_cast<const IO*>(r);
     const IO* kk = static_cast<const IO*>(k);
     const IO* vv = static_cast<const IO*>(v);
     const WT* ww = static_cast<const WT*>(w);
-    if (w_is_ew)
-        hipLaunchKernelGGL((wkv6_fwd_chunk_kernel<IO, WT, true>), grid, block, 0, st, rr, kk, vv, ww, u, y, T, C, H, nullptr);
-    else
-        hipLaunchKernelGGL((wkv6_fwd_chunk_kernel<IO, WT, false>), grid, block, 0, st, rr, kk, vv, ww, u, y, T, C, H, nullptr);
+    const long long sequences = (long long)B * H;
+    int nseg = segments(B, T, H);
+    if (!ws || ws_bytes < seg_workspace_bytes(sequences, nseg) || ((uintptr_t)ws & 15) || !pairs_aligned<IO, WT>(k, v, w)) nseg = 1;
+    float* states = nullptr;
+    int* flags = nullptr;
+    unsigned grid = (unsigned)sequences;
+    if (nseg > 1) {
+        states = static_cast<float*>(ws);
+        flags = reinterpret_cast<int*>(states + (size_t)sequences * nseg * SEG_FLOATS);
+        grid = seg_grid(sequences, nseg);
+        hipLaunchKernelGGL((wkv6_seg_state_kernel<IO, WT, EW>), dim3(grid), dim3(256), 0, st, kk, vv, ww, states, flags, T, C, H,
+                           sequences, nseg);
+        hipLaunchKernelGGL(wkv6_seg_fold_kernel, dim3(4, 2, (unsigned)sequences), dim3(256), 0, st, states, nseg);
+    }
+    hipLaunchKernelGGL((wkv6_fwd_chunk_kernel<IO, WT, EW>), dim3(grid), block, 0, st, rr, kk, vv, ww, u, y, T, C, H, (int)sequences,
+                       nseg, states, flags, nullptr);
     return check_launch("wkv6_fwd (chunked)");
 }
 
@@ -73,10 +101,10 @@ bool force_scalar() { return option(OPT_WKV6_FWD_SCALAR) != 0; }   // testing ov
 
 template <typename IO, typename WT>
 int launch_any(const void* r, const void* k, const void* v, const void* w, const float* u, float* y,
-               void* ws, int B, int T, int C, int H, bool w_is_ew, hipStream_t st) {
-    (void)ws;
+               void* ws, size_t ws_bytes, int B, int T, int C, int H, bool w_is_ew, hipStream_t st) {
     if (force_scalar()) return launch_scalar<IO, WT>(r, k, v, w, u, y, B, T, C, H, w_is_ew, st);
-    return launch_chunked<IO, WT>(r, k, v, w, u, y, B, T, C, H, w_is_ew, st);
+    return w_is_ew ? launch_chunked<IO, WT, true>(r, k, v, w, u, y, ws, ws_bytes, B, T, C, H, st)
+                   : launch_chunked<IO, WT, false>(r, k, v, w, u, y, ws, ws_bytes, B, T, C, H, st);
 }
 
 }  // namespace
@@ -108,13 +136,15 @@ extern "C" int vrwkv_wkv6_fwd_phases(const void* r, const void* k, const void* v
     hipLaunchKernelGGL((wkv6_fwd_chunk_kernel<__hip_bfloat16, float, false, true>), dim3(B * H), dim3(64 * FW_WAVES), 0,
                        static_cast<hipStream_t>(hip_stream), static_cast<const __hip_bfloat16*>(r),
                        static_cast<const __hip_bfloat16*>(k), static_cast<const __hip_bfloat16*>(v),
-                       static_cast<const float*>(w), u, y, T, C, H, static_cast<unsigned long long*>(stamps));
+                       static_cast<const float*>(w), u, y, T, C, H, B * H, 1, (const float*)nullptr, (const int*)nullptr,
+                       static_cast<unsigned long long*>(stamps));
     return check_launch("wkv6_fwd_phases");
 }
 
 extern "C" size_t vrwkv_wkv6_fwd_workspace_bytes(int B, int T, int C, int H) {
-    (void)B; (void)T; (void)C; (void)H;
-    return 0;                                            // no workspace is needed (kept for ABI symmetry)
+    (void)C;
+    if (B <= 0 || T <= 0 || H <= 0) return 0;
+    return seg_workspace_bytes((long long)B * H, segments(B, T, H));
 }
 
 extern "C" int vrwkv_wkv6_fwd(const void* r, const void* k, const void* v, const void* w, const float* u,
@@ -122,7 +152,6 @@ extern "C" int vrwkv_wkv6_fwd(const void* r, const void* k, const void* v, const
                               void* workspace, size_t workspace_bytes, void* hip_stream) {
     int rc = validate(B, T, C, H, rkv_dtype, w_dtype);
     if (rc != VRWKV_OK) return rc;
-    (void)workspace_bytes;
     if (!r || !k || !v || !w || !u || !y) {
         set_error("wkv6_fwd: null pointer argument");
         return VRWKV_INVALID_ARG;
@@ -137,15 +166,15 @@ extern "C" int vrwkv_wkv6_fwd(const void* r, const void* k, const void* v, const
     const bool ew = w_is_ew != 0;
     switch (rkv_dtype) {
         case VRWKV_F32:
-            return launch_any<float, float>(r, k, v, w, u, y, workspace, B, T, C, H, ew, st);
+            return launch_any<float, float>(r, k, v, w, u, y, workspace, workspace_bytes, B, T, C, H, ew, st);
         case VRWKV_BF16:
             return w_dtype == VRWKV_F32
-                       ? launch_any<__hip_bfloat16, float>(r, k, v, w, u, y, workspace, B, T, C, H, ew, st)
-                       : launch_any<__hip_bfloat16, __hip_bfloat16>(r, k, v, w, u, y, workspace, B, T, C, H, ew, st);
+                       ? launch_any<__hip_bfloat16, float>(r, k, v, w, u, y, workspace, workspace_bytes, B, T, C, H, ew, st)
+                       : launch_any<__hip_bfloat16, __hip_bfloat16>(r, k, v, w, u, y, workspace, workspace_bytes, B, T, C, H, ew, st);
         case VRWKV_F16:
             return w_dtype == VRWKV_F32
-                       ? launch_any<__half, float>(r, k, v, w, u, y, workspace, B, T, C, H, ew, st)
-                       : launch_any<__half, __half>(r, k, v, w, u, y, workspace, B, T, C, H, ew, st);
+                       ? launch_any<__half, float>(r, k, v, w, u, y, workspace, workspace_bytes, B, T, C, H, ew, st)
+                       : launch_any<__half, __half>(r, k, v, w, u, y, workspace, workspace_bytes, B, T, C, H, ew, st);
     }
     return VRWKV_UNSUPPORTED_DTYPE;
 }

@@ -34,11 +34,15 @@
 // which keeps the result within ~3e-5 of the fp32 recurrence (one bf16 rounding of any of them
 // alone costs ~1e-2).  v is exact in bf16 for bf16 input and split in two for fp16 / fp32 input.
 //
+// Few long sequences: with nseg > 1 a workgroup owns one segment of a sequence (a run of chunks) and starts both passes
+// from the states that wkv6_segment.h provides; everything else is the same.
+//
 // Range: the factorisation needs |P31| <= 60 in every chunk (decay over 32 tokens no stronger
 // than e^-60).  A (b,h) sequence with a chunk outside that range is redone from scratch by the same
-// workgroup with the sequential-state recurrence.
+// workgroup with the sequential-state recurrence (a split sequence by the workgroup of its first segment: the state
+// kernel, which saw every chunk, has set the flag before any of them starts).
 #pragma once
-#include "wkv6_chunk_common.h"
+#include "wkv6_segment.h"
 
 namespace vrwkv {
 namespace wkv6_detail {
@@ -97,7 +101,8 @@ template <typename IO, typename WT, bool W_IS_EW, bool STAMPS = false>
 __global__ __launch_bounds__(64 * FW_WAVES, 4)   // four waves per SIMD: at most 128 registers
 void wkv6_fwd_chunk_kernel(const IO* __restrict__ r_, const IO* __restrict__ k_, const IO* __restrict__ v_,
                            const WT* __restrict__ w_, const float* __restrict__ u_, float* __restrict__ y_,
-                           int T, int C, int H, unsigned long long* __restrict__ stamps = nullptr)
+                           int T, int C, int H, int sequences, int nseg, const float* __restrict__ seg_ws,
+                           const int* __restrict__ seg_flags, unsigned long long* __restrict__ stamps = nullptr)
 {
     constexpr bool VSPLIT = !(sizeof(IO) == 2 && __is_same(IO, __hip_bfloat16));
     __shared__ FwdLds<VSPLIT> lds[2];
@@ -109,10 +114,15 @@ void wkv6_fwd_chunk_kernel(const IO* __restrict__ r_, const IO* __restrict__ k_,
     const int w4 = wave & 3;                     // token quarter in stage E, value-column quarter in stage M
     const bool asc = wave >= 4;                  // waves 4-7: ascending pass (with the bonus)
     FwdLds<VSPLIT>& L = lds[asc ? 1 : 0];
-    const int bh = blockIdx.x;
+    int bh = blockIdx.x, seg = 0;
+    if (nseg > 1) {
+        seg_of_block(blockIdx.x, nseg, bh, seg);
+        if (bh >= sequences) return;
+    }
     const int b = bh / H, h = bh % H;
     const size_t base = (size_t)b * T * C + (size_t)h * HN;
-    const int nchunk = (T + LC - 1) / LC;
+    const int cps = ((T + LC - 1) / LC + nseg - 1) / nseg, c0 = seg * cps;       // this segment's chunks: c0 .. c0 + nchunk - 1
+    const int nchunk = min(cps, (T + LC - 1) / LC - c0);
     const float uj = asc ? u_[h * HN + lane] : 0.f;
     if (threadIdx.x < 2) sFlag[threadIdx.x] = 0;
     __syncthreads();
@@ -130,6 +140,18 @@ void wkv6_fwd_chunk_kernel(const IO* __restrict__ r_, const IO* __restrict__ k_,
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt) S[jt] = f32x4v{0.f, 0.f, 0.f, 0.f};
     bool bail = false;
+    if (nseg > 1) {
+        const int f = lane < nseg ? seg_flags[(size_t)bh * nseg + lane] : 0;
+        if (__builtin_amdgcn_ballot_w64(f != 0) != 0ull) {               // the whole sequence is left to its first segment
+            if (seg != 0) return;
+            bail = true;
+        } else {
+            const float* in = seg_ws + ((size_t)bh * nseg + seg) * SEG_FLOATS + (asc ? 0 : SEG_STATE);
+#pragma unroll
+            for (int jt = 0; jt < 4; ++jt) S[jt] = *reinterpret_cast<const f32x4v*>(in + seg_frag(w4, jt, lane));
+        }
+    }
+    if (!bail) {
 
     // The decay rows of a chunk are fetched one step ahead (when the previous step enters its matrix stage),
     // so the cumulative decay can start at once; r, k, v follow at the top of the step and are needed only
@@ -149,7 +171,7 @@ void wkv6_fwd_chunk_kernel(const IO* __restrict__ r_, const IO* __restrict__ k_,
     // Pass index n = 0..31 inside a chunk is token 32c + n (ascending) or 32c + 31 - n (descending); tokens
     // past T (only in the last chunk; for the descending pass they come first) read zeros and count as
     // k = 0, d = 1 (their own y rows are dropped by the store's range check).
-    auto chunk_of = [&](int ch) { return asc ? ch : nchunk - 1 - ch; };
+    auto chunk_of = [&](int ch) { return c0 + (asc ? ch : nchunk - 1 - ch); };
     const int sgn = asc ? 1 : -1, n0 = asc ? 0 : LC - 1;
     auto token_of = [&](int c, int n) { return c * LC + n0 + sgn * n; };
     // Row offsets walk the 8 tokens of this wave's block with one scalar add each (the scalar offset of the access;
@@ -248,15 +270,15 @@ void wkv6_fwd_chunk_kernel(const IO* __restrict__ r_, const IO* __restrict__ k_,
         asm volatile("" : "+v"(lane_e));
         int w4s = w4, hps = hp;                                           // the same for what depends on the wave number
         asm volatile("" : "+s"(w4s), "+s"(hps));
-        const int cy = chunk_of(ch);
-        // the other pass's M of chunk cy on the common clock: the descending one runs in half 2 (nchunk - cy), the
-        // ascending one in half 2 cy + 1; this step's E runs in half hp, its M in half hp + 1
-        const int other_m = asc ? 2 * (nchunk - cy) : 2 * cy + 1;
+        const int cy = chunk_of(ch), cl = cy - c0;                        // its number in the sequence and in the segment
+        // the other pass's M of chunk cl on the common clock: the descending one runs in half 2 (nchunk - cl), the
+        // ascending one in half 2 cl + 1; this step's E runs in half hp, its M in half hp + 1
+        const int other_m = asc ? 2 * (nchunk - cl) : 2 * cl + 1;
         const bool y_second = other_m < hp + 1, y_late = other_m == hp;   // wave-uniform
         // ... and if the other pass runs its E of chunk cy in the half of this step's M, it fetches this step's y rows
         // right behind the barrier that ends that half: then the stores are waited for before that barrier (the barrier
         // orders the instructions' issue, not the arrival of the data)
-        const bool y_drain = (asc ? 2 * (nchunk - 1 - cy) + 1 : 2 * cy) == hp + 1;
+        const bool y_drain = (asc ? 2 * (nchunk - 1 - cl) + 1 : 2 * cl) == hp + 1;
         {
             // =============================== stage E: elementwise =================================
             // wave w4s of the pass prepares tokens n = 8 w4s .. 8 w4s + 7 of the chunk; lane = channel j (and i for v)
@@ -275,7 +297,7 @@ void wkv6_fwd_chunk_kernel(const IO* __restrict__ r_, const IO* __restrict__ k_,
             const float m0 = w4s == 0 ? 1.f : 0.f, m1 = w4s <= 1 ? 1.f : 0.f, m2 = w4s <= 2 ? 1.f : 0.f;     // wave-uniform
             const float rest = fmaf(m0, t0, fmaf(m1, t1, fmaf(m2, t2, t3)));
             const float p31 = (t0 + t1) + (t2 + t3);
-            if (w4s == 0 && __builtin_amdgcn_ballot_w64(!(p31 >= -SAFE_DECAY * LOG2E)) != 0ull && lane == 0) sFlag[hps & 1] = 1;
+            if (nseg == 1 && w4s == 0 && __builtin_amdgcn_ballot_w64(!(p31 >= -SAFE_DECAY * LOG2E)) != 0ull && lane == 0) sFlag[hps & 1] = 1;
             // Z = diag(e^P31) S, in place, split into head and tail for MFMA 3 (done here, while the r, k, v rows are still
             // on their way): a lane needs e^P31 of the channels its state rows belong to, taken from the wave's own copy
             L.C2[w4s][lane_e] = fast_exp2(p31);
@@ -501,6 +523,7 @@ void wkv6_fwd_chunk_kernel(const IO* __restrict__ r_, const IO* __restrict__ k_,
         if (sFlag[(hps + 1) & 1]) { bail = true; break; }
     }
     if (asc && !bail) sync_step();
+    }
 
     if (bail) {
         // Some chunk decays faster than the factorisation can represent: recompute the whole sequence
