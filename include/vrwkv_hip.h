@@ -140,6 +140,13 @@ int vrwkv_wkv6_bwd(const void* r, const void* k, const void* v, const void* w, c
                    const float* gy, float* gr, float* gk, float* gv, float* gw, float* gu,
                    int B, int T, int C, int H, int rkv_dtype, int w_dtype, int w_is_ew,
                    void* workspace, size_t workspace_bytes, void* hip_stream);
+/* The same with the gradients in their inputs' types: gr, gk, gv of rkv_dtype, gw of w_dtype (rounded once from the fp32
+ * sums), as an autograd engine hands them on. */
+size_t vrwkv_wkv6_bwd_like_workspace_bytes(int B, int T, int C, int H, int rkv_dtype, int w_dtype);
+int vrwkv_wkv6_bwd_like(const void* r, const void* k, const void* v, const void* w, const float* u,
+                        const float* gy, void* gr, void* gk, void* gv, void* gw, float* gu,
+                        int B, int T, int C, int H, int rkv_dtype, int w_dtype, int w_is_ew,
+                        void* workspace, size_t workspace_bytes, void* hip_stream);
 
 /* ---- fused Q-Shift + token mix (the elementwise step in front of the r/k/v projections) -----
  * Replaces q_shift (classification/mmcls_custom/models/backbones/vrwkv.py:68-79) followed by the

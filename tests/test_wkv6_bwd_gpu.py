@@ -245,3 +245,47 @@ def test_decay_regimes_mixed_over_the_heads_of_one_call(ops, seed, B, T, H, dtyp
             assert T <= 3 or e <= (5e-3 if top < 1 else 6e-2), (name, e)
         else:
             assert e <= TOL, (name, e)
+
+
+@pytest.mark.parametrize("T,segments", [(33, 2), (65, 3), (200, 3), (250, 8), (577, 5)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_backward_of_sequences_cut_into_segments(ops, T, segments, dtype):
+    """Forced numbers of segments (one chunk each, a last segment of one token) against the uncut sequences, which the
+    tests above hold to the oracle: the same sums with the states between segments formed another way, so both carry the
+    split operands' 3e-5.  gw: each side within the 1e-3 that the tests above allow against the oracle, 2e-3 apart."""
+    B, H = 2, 2
+    g = torch.Generator().manual_seed(T)
+    r, k, v = (torch.randn(B, T, 64 * H, generator=g).to(dtype).cuda() for _ in range(3))
+    w = (torch.randn(B, T, 64 * H, generator=g) - 3).to(dtype).cuda()
+    u, gy = (0.3 * torch.randn(H, 64, generator=g)).cuda(), torch.randn(B, T, 64 * H, generator=g).cuda()
+    with ops.option("wkv6_segments", 1):
+        want = ops.wkv6_backward(B, T, 64 * H, H, r, k, v, w, u, gy)
+    with ops.option("wkv6_segments", segments):
+        got = ops.wkv6_backward(B, T, 64 * H, H, r, k, v, w, u, gy)
+        like = ops.wkv6_backward(B, T, 64 * H, H, r, k, v, w, u, gy, like_inputs=True)
+    for a, b, c, name in zip(got, want, like, ("gr", "gk", "gv", "gw", "gu")):
+        assert rel_err(a.cpu().numpy(), b.cpu().numpy()) <= (2e-3 if name == "gw" else 1e-4), name
+        assert torch.equal(c, a.to(c.dtype)), name                       # the same sums, rounded once
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_backward_of_a_cut_sequence_with_a_decay_out_of_range(ops, dtype):
+    """One of four sequences decays by more than e^-60 inside its last segment: redone by the sequential sweeps, in every
+    result type; the reference is the sequential path itself, bit for bit for that sequence."""
+    B, T, H = 2, 200, 2
+    g = torch.Generator().manual_seed(9)
+    r, k, v = (torch.randn(B, T, 64 * H, generator=g).to(dtype).cuda() for _ in range(3))
+    w = torch.randn(B, T, 64 * H, generator=g) - 3
+    w[1, 180:190, 64:] = 3.0
+    w = w.to(dtype).cuda()
+    u, gy = (0.3 * torch.randn(H, 64, generator=g)).cuda(), torch.randn(B, T, 64 * H, generator=g).cuda()
+    with ops.option("wkv6_bwd_scalar", 1):
+        want = ops.wkv6_backward(B, T, 64 * H, H, r, k, v, w, u, gy, like_inputs=True)
+    for segments in (1, 3):
+        with ops.option("wkv6_segments", segments):
+            got = ops.wkv6_backward(B, T, 64 * H, H, r, k, v, w, u, gy, like_inputs=True)
+        for a, b, name in zip(got[:4], want[:4], ("gr", "gk", "gv", "gw")):
+            assert torch.equal(a[1, :, 64:], b[1, :, 64:]), name
+            tol = 2e-3 if dtype == torch.float32 else 1e-2               # gw at the file's tolerance; bf16 results round
+            assert rel_err(a.float().cpu().numpy(), b.float().cpu().numpy()) <= tol, name
+        assert rel_err(got[4].cpu().numpy(), want[4].cpu().numpy()) <= 1e-4

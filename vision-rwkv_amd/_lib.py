@@ -73,6 +73,10 @@ def _declare(lib):
     lib.vrwkv_wkv6_bwd_workspace_bytes.restype = sz
     lib.vrwkv_wkv6_bwd.argtypes = [vp, vp, vp, vp, fp, fp, fp, fp, fp, fp, fp, i, i, i, i, i, i, i, vp, sz, vp]
     lib.vrwkv_wkv6_bwd.restype = i
+    lib.vrwkv_wkv6_bwd_like_workspace_bytes.argtypes = [i, i, i, i, i, i]
+    lib.vrwkv_wkv6_bwd_like_workspace_bytes.restype = sz
+    lib.vrwkv_wkv6_bwd_like.argtypes = lib.vrwkv_wkv6_bwd.argtypes
+    lib.vrwkv_wkv6_bwd_like.restype = i
     lib.vrwkv_qshift_mix.argtypes = [vp, fp, c.POINTER(c.c_void_p), i, i, i, i, i, i, i, i, i, i, vp]
     lib.vrwkv_qshift_mix.restype = i
     lib.vrwkv_qshift_mix_bwd_workspace_bytes.argtypes = [i, i, i, i]

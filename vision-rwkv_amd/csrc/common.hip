@@ -51,9 +51,12 @@ int option(Option o) {
 }
 
 int device_cus() {
+    static std::atomic<int> cus[64];                     // per device, 0 = not asked yet
     int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-        n = 256;
+    if (hipGetDevice(&dev) != hipSuccess) return 256;
+    if (dev >= 0 && dev < 64 && (n = cus[dev].load(std::memory_order_relaxed)) > 0) return n;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
+    if (dev >= 0 && dev < 64) cus[dev].store(n, std::memory_order_relaxed);
     return n;
 }
 

@@ -41,13 +41,7 @@ int segments(int B, int T, int H) {
         const int n = forced < nchunk ? forced : nchunk, cps = (nchunk + n - 1) / n;
         return (nchunk + cps - 1) / cps;
     }
-    return wkv6_segments((long long)B * H, nchunk, device_cus());
-}
-
-// the state kernel reads two neighbouring channels at a time
-template <typename IO, typename WT>
-bool pairs_aligned(const void* k, const void* v, const void* w) {
-    return !((((uintptr_t)k | (uintptr_t)v) & (2 * sizeof(IO) - 1)) || ((uintptr_t)w & (2 * sizeof(WT) - 1)));
+    return wkv6_segments((long long)B * H, nchunk, device_cus(), SEG_FWD);
 }
 
 template <typename IO, typename WT>
@@ -80,7 +74,7 @@ int launch_chunked(const void* r, const void* k, const void* v, const void* w, c
     const WT* ww = static_cast<const WT*>(w);
     const long long sequences = (long long)B * H;
     int nseg = segments(B, T, H);
-    if (!ws || ws_bytes < seg_workspace_bytes(sequences, nseg) || ((uintptr_t)ws & 15) || !pairs_aligned<IO, WT>(k, v, w)) nseg = 1;
+    if (!ws || ws_bytes < seg_bytes(sequences, nseg, SEG_FLOATS) || ((uintptr_t)ws & 15)) nseg = 1;
     float* states = nullptr;
     int* flags = nullptr;
     unsigned grid = (unsigned)sequences;
@@ -90,7 +84,7 @@ int launch_chunked(const void* r, const void* k, const void* v, const void* w, c
         grid = seg_grid(sequences, nseg);
         hipLaunchKernelGGL((wkv6_seg_state_kernel<IO, WT, EW>), dim3(grid), dim3(256), 0, st, kk, vv, ww, states, flags, T, C, H,
                            sequences, nseg);
-        hipLaunchKernelGGL(wkv6_seg_fold_kernel, dim3(4, 2, (unsigned)sequences), dim3(256), 0, st, states, nseg);
+        hipLaunchKernelGGL((wkv6_seg_fold_kernel<2, false>), dim3(4, 2, (unsigned)sequences), dim3(256), 0, st, states, nseg);
     }
     hipLaunchKernelGGL((wkv6_fwd_chunk_kernel<IO, WT, EW>), dim3(grid), block, 0, st, rr, kk, vv, ww, u, y, T, C, H, (int)sequences,
                        nseg, states, flags, nullptr);
@@ -144,7 +138,7 @@ extern "C" int vrwkv_wkv6_fwd_phases(const void* r, const void* k, const void* v
 extern "C" size_t vrwkv_wkv6_fwd_workspace_bytes(int B, int T, int C, int H) {
     (void)C;
     if (B <= 0 || T <= 0 || H <= 0) return 0;
-    return seg_workspace_bytes((long long)B * H, segments(B, T, H));
+    return seg_bytes((long long)B * H, segments(B, T, H), SEG_FLOATS);
 }
 
 extern "C" int vrwkv_wkv6_fwd(const void* r, const void* k, const void* v, const void* w, const float* u,

@@ -22,24 +22,30 @@ namespace wkv6_detail {
 
 constexpr int SEG_MAX = 64;                          // segments per sequence (one flag per lane of a wave)
 constexpr int SEG_STATE = HN * HN;                   // floats of one state
-constexpr int SEG_FLOATS = 2 * SEG_STATE + HN;       // up state, down state, total decay per channel
+constexpr int SEG_FLOATS = 2 * SEG_STATE + HN;       // forward: up state, down state, total decay per channel
+constexpr int BWD_SEG_FLOATS = 4 * SEG_STATE + HN;   // backward: S up, G up, S down, G down, total decay per channel
 
-// Segments of a sequence: the number with the least estimated time, in microseconds measured on bf16 calls.  Per chunk, a
-// workgroup of the main kernel takes 2.8 when the chip is nearly empty, 3.6 with one on every CU, 5.6 with two (the most
-// that fit), one of the state kernel 1.55 / 2.4; the scan takes 4 to 8, the two extra launches about 7 more.  Measured at
-// 24 sequences of 130 chunks: uncut 358, 2 segments 276, 6 103, 10 69, 21 64, 32 72; at 48 sequences of 32 chunks: uncut
-// 90, 10 segments 44; at 192 sequences of 32 chunks uncut 93, best cut 108.
-inline int wkv6_segments(long long sequences, int nchunk, int cus) {
+// Segments of a sequence: the number with the least estimated time, where that is a fifth less than uncut.  Sequences of up to
+// 256 tokens stay whole: the results of a (b,h) then do not depend on how many others are in the call.  Costs are microseconds measured on bf16 calls: a step
+// (one chunk) of the main kernel while its CU holds one workgroup, and more per further workgroup that its CU has to run
+// (two at a time fit); the state kernel's step per workgroup on a CU; the scan and the extra launches.
+struct SegCosts { double one, each, state, fixed, per_segment; };
+// forward: at 24 sequences of 130 chunks uncut 358, 6 segments 103, 10 69, 21 64, 32 72; at 48 of 32 chunks uncut 90, 10
+// segments 44, of 19 chunks uncut 57, 10 segments 45; at 192 of 32 chunks uncut 93, best cut 108
+constexpr SegCosts SEG_FWD = {3.2, 2.8, 1.3, 20.0, 0.1};
+// backward (both sweeps): at 24 sequences of 130 chunks uncut 1381, 10 segments 194, 21 163, 32 193; at 192 of 32 chunks
+// uncut 376, 4 segments 310; at 9 of 7 chunks uncut 78, 7 segments 42; at 192 of 7 chunks uncut 84, best cut 103
+constexpr SegCosts SEG_BWD = {11.5, 9.0, 1.5, 32.0, 0.1};
+inline int wkv6_segments(long long sequences, int nchunk, int cus, const SegCosts& k) {
     auto time = [&](int nseg) {
         const int cps = (nchunk + nseg - 1) / nseg;
-        const long long groups = sequences * nseg;
-        const double rounds = (double)((groups + 2 * cus - 1) / (2 * cus));
-        if (nseg == 1) return 2.0 + rounds * cps * (groups > cus ? 4.5 : 2.8);
-        return 20.0 + 0.1 * nseg + rounds * cps * (groups > cus ? 5.6 + 2.4 : 3.6 + 1.55);
+        const long long per_cu = (sequences * nseg + cus - 1) / cus;
+        const double main = cps * (per_cu == 1 ? k.one : k.each * per_cu);
+        return nseg == 1 ? main : main + cps * k.state * per_cu + k.fixed + k.per_segment * nseg;
     };
     int best = 1;
-    double best_time = 0.9 * time(1);
-    for (int nseg = 2; nseg <= SEG_MAX && nseg <= nchunk && sequences * nseg <= 4LL * cus; ++nseg) {
+    double best_time = 0.8 * time(1);
+    for (int nseg = 2; nchunk > 8 && nseg <= SEG_MAX && nseg <= nchunk && sequences * nseg <= 4LL * cus; ++nseg) {
         const double t = time(nseg);
         if (t < best_time) { best = nseg; best_time = t; }
     }
@@ -56,27 +62,31 @@ __device__ __forceinline__ void seg_of_block(unsigned block, int nseg, int& bh, 
     seg = (int)(y % nseg);
 }
 
-inline size_t seg_workspace_bytes(long long sequences, int nseg) {
-    return nseg > 1 ? (size_t)sequences * nseg * (SEG_FLOATS * sizeof(float) + sizeof(int)) : 0;
+// bytes of the segments' states (floats_per_segment each) and flags
+inline size_t seg_bytes(long long sequences, int nseg, int floats_per_segment) {
+    return nseg > 1 ? (size_t)sequences * nseg * (floats_per_segment * sizeof(float) + sizeof(int)) : 0;
 }
 
 // State fragment of a wave in the main kernel's accumulator order: tile jt of wave w4 holds rows j = 16 jt + 4 g4 + r,
 // column i = 16 w4 + c16, as one 16-byte piece per lane.
 __device__ __forceinline__ size_t seg_frag(int w4, int jt, int lane) { return (size_t)((w4 * 4 + jt) * 64 + lane) * 4; }
 
-// Exclusive scan over the segments of a sequence: the local states are replaced in place by the states entering the
-// segments.  A thread owns four rows of one column in one direction; its loads over the segments are independent of each
-// other and go out eight at a time.  Grid: (4, 2, sequences), block 256.  (Folding in the main kernel instead, every
-// segment reading all segments before it, moved 160 MB through the L2s at 24 sequences of 21 segments: 10 us more.)
-__global__ __launch_bounds__(256) inline void wkv6_seg_fold_kernel(float* __restrict__ ws, int nseg)
+// Exclusive scan over the segments of a sequence: the local states (NMAT of them per segment, the upward ones first) are
+// replaced in place by the states entering the segments.  A thread owns four neighbouring values of one state -- rows of a
+// column, with the decay per row, or (COLS) the other way round; its loads over the segments are independent of each other
+// and go out eight at a time.  Grid: (4, NMAT, sequences), block 256.  (Folding in the main kernel instead, every segment
+// reading all segments before it, moved 160 MB through the L2s at 24 sequences of 21 segments: 10 us more.)
+template <int NMAT, bool COLS>
+__global__ __launch_bounds__(256) void wkv6_seg_fold_kernel(float* __restrict__ ws, int nseg)
 {
-    const int piece = blockIdx.x * 256 + threadIdx.x;                     // 16-byte piece of the state
-    const bool up = blockIdx.y == 0;
-    const int j0 = 16 * ((piece >> 6) & 3) + 4 * ((piece >> 4) & 3);      // its rows (see seg_frag)
-    const ptrdiff_t step = up ? SEG_FLOATS : -(ptrdiff_t)SEG_FLOATS;
-    float* p = ws + ((size_t)blockIdx.z * nseg + (up ? 0 : nseg - 1)) * SEG_FLOATS;
-    float* l = p + (up ? 0 : SEG_STATE) + 4 * piece;
-    const float* d = p + 2 * SEG_STATE + j0;
+    constexpr int FLOATS = NMAT * SEG_STATE + HN;
+    const int piece = blockIdx.x * 256 + threadIdx.x;                     // 16-byte piece of the state (see seg_frag)
+    const bool up = blockIdx.y < NMAT / 2;
+    const int j0 = COLS ? 16 * (piece >> 8) + (piece & 15) : 16 * ((piece >> 6) & 3) + 4 * ((piece >> 4) & 3);
+    const ptrdiff_t step = up ? FLOATS : -(ptrdiff_t)FLOATS;
+    float* p = ws + ((size_t)blockIdx.z * nseg + (up ? 0 : nseg - 1)) * FLOATS;
+    float* l = p + blockIdx.y * SEG_STATE + 4 * piece;
+    const float* d = p + NMAT * SEG_STATE + j0;
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
     constexpr int U = 8;
     for (int q = 0; q < nseg; q += U) {
@@ -85,7 +95,8 @@ __global__ __launch_bounds__(256) inline void wkv6_seg_fold_kernel(float* __rest
         for (int i = 0; i < U; ++i)
             if (q + i < nseg) {
                 lv[i] = *reinterpret_cast<const f32x4*>(l + i * step);
-                dv[i] = *reinterpret_cast<const f32x4*>(d + i * step);
+                if (COLS) { const float x = d[i * step]; dv[i] = f32x4{x, x, x, x}; }
+                else dv[i] = *reinterpret_cast<const f32x4*>(d + i * step);
             }
 #pragma unroll
         for (int i = 0; i < U; ++i)
@@ -105,8 +116,6 @@ template <typename IO> struct SegLds {
     float C2[HN], Tot[2][8][HN];
 };
 
-// Element-wise stage: a half wave owns four tokens of the chunk, a lane two neighbouring channels (one 4- or 8-byte
-// load per row).
 template <typename IO, typename WT, bool W_IS_EW>
 __global__ __launch_bounds__(256)
 void wkv6_seg_state_kernel(const IO* __restrict__ k_, const IO* __restrict__ v_, const WT* __restrict__ w_,
@@ -142,19 +151,9 @@ void wkv6_seg_state_kernel(const IO* __restrict__ k_, const IO* __restrict__ v_,
             vraw[s][m] = BufRaw<2 * sizeof(IO)>::ld(rsv, e * (unsigned)sizeof(IO), 0);
         }
     };
-    auto two = [](RawIO raw, float (&o)[2]) { IO t[2]; __builtin_memcpy(t, &raw, sizeof(raw)); o[0] = to_f32(t[0]); o[1] = to_f32(t[1]); };
     float p[2][4];                                                        // cumulative log2 decays inside the group
     auto decays = [&](int c, int s) {
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            WT t[2];
-            __builtin_memcpy(t, &wraw[s][m], sizeof(wraw[s][m]));
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const float fw = to_f32(t[e]);
-                p[e][m] = W_IS_EW ? fw * LOG2E : -fast_exp2(fmaf(fw, LOG2E, LOG2_LOG2E));
-            }
-        }
+        pair_log_decays<WT, W_IS_EW>(wraw[s], p);
         if ((c + 1) * LC > T) {                                           // wave-uniform: some token of the chunk is past T
 #pragma unroll
             for (int m = 0; m < 4; ++m)
@@ -175,23 +174,8 @@ void wkv6_seg_state_kernel(const IO* __restrict__ k_, const IO* __restrict__ v_,
     lds_barrier();
     auto step = [&](int c, auto buf_) {
         constexpr int buf = buf_;
-        // log2 decay in front of the lane's group and behind it: sums over the groups of the other waves with wave-uniform
-        // weights, then this wave's other half
-        float before[2] = {0.f, 0.f}, rest[2] = {0.f, 0.f};
-        const bool upper = lane >= 32;
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const f32x2 t = *reinterpret_cast<const f32x2*>(&L.Tot[buf][g][cp]);
-            const float wb = (g >> 1) < w4 ? 1.f : 0.f, wr = (g >> 1) > w4 ? 1.f : 0.f;
-#pragma unroll
-            for (int e = 0; e < 2; ++e) { before[e] = fmaf(wb, t[e], before[e]); rest[e] = fmaf(wr, t[e], rest[e]); }
-        }
-        const f32x2 sib = *reinterpret_cast<const f32x2*>(&L.Tot[buf][grp ^ 1][cp]);
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            before[e] += upper ? sib[e] : 0.f;
-            rest[e] += upper ? 0.f : sib[e];
-        }
+        float before[2], rest[2];                                         // log2 decay in front of the lane's group and behind it
+        pair_group_sums(L.Tot[buf], w4, lane, cp, before, rest);
         unsigned ah[2][2], al[2][2], dh[2][2], dl[2][2], vh[2][2], vl[2][2];
         float p31[2];
 #pragma unroll
@@ -202,8 +186,8 @@ void wkv6_seg_state_kernel(const IO* __restrict__ k_, const IO* __restrict__ v_,
 #pragma unroll
         for (int m = 0; m < 4; m += 2) {
             float k0[2], k1[2], v0[2], v1[2];
-            two(kraw[buf][m], k0); two(kraw[buf][m + 1], k1);
-            two(vraw[buf][m], v0); two(vraw[buf][m + 1], v1);
+            pair_widen<IO>(kraw[buf][m], k0); pair_widen<IO>(kraw[buf][m + 1], k1);
+            pair_widen<IO>(vraw[buf][m], v0); pair_widen<IO>(vraw[buf][m + 1], v1);
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 const float tail = p[e][3] + rest[e];
@@ -212,11 +196,11 @@ void wkv6_seg_state_kernel(const IO* __restrict__ k_, const IO* __restrict__ v_,
                 const float fd0 = fast_exp2(m ? pre + p[e][m - 1] : pre), fd1 = fast_exp2(pre + p[e][m]);
                 const float a0 = k0[e] * fa0, a1 = k1[e] * fa1, d0 = k0[e] * fd0, d1 = k1[e] * fd1;
                 ah[e][m / 2] = pack_bf16(a0, a1);
-                al[e][m / 2] = pack_bf16(a0 - bf16_lo(ah[e][m / 2]), a1 - bf16_hi(ah[e][m / 2]));
+                al[e][m / 2] = tail_bf16(a0, a1, ah[e][m / 2]);
                 dh[e][m / 2] = pack_bf16(d0, d1);
-                dl[e][m / 2] = pack_bf16(d0 - bf16_lo(dh[e][m / 2]), d1 - bf16_hi(dh[e][m / 2]));
+                dl[e][m / 2] = tail_bf16(d0, d1, dh[e][m / 2]);
                 vh[e][m / 2] = pack_bf16(v0[e], v1[e]);
-                if constexpr (VSPLIT) vl[e][m / 2] = pack_bf16(v0[e] - bf16_lo(vh[e][m / 2]), v1[e] - bf16_hi(vh[e][m / 2]));
+                if constexpr (VSPLIT) vl[e][m / 2] = tail_bf16(v0[e], v1[e], vh[e][m / 2]);
             }
         }
 #pragma unroll
@@ -268,6 +252,165 @@ void wkv6_seg_state_kernel(const IO* __restrict__ k_, const IO* __restrict__ v_,
     // every wave's half waves saw the same chunk totals: wave 0's first half speaks for all
     if (w4 == 0) {
         if (lane < 32) *reinterpret_cast<f32x2*>(out + 2 * SEG_STATE + cp) = f32x2{fast_exp2(base_p[0]), fast_exp2(base_p[1])};
+        const bool any = __builtin_amdgcn_ballot_w64(out_of_range) != 0ull;
+        if (lane == 0) flags[(size_t)bh * nseg + seg] = any ? 1 : 0;
+    }
+}
+
+// The same for the backward's sweeps, which carry two states each: S (k, v) and the adjoint state G (r, gy), up and down.
+// A wave owns 16 columns j and the rows i of all four (the order in which the sweeps read them).
+template <typename IO> struct BwdSegLds {
+    static constexpr bool VSPLIT = !__is_same(IO, __hip_bfloat16);
+    __bf16 Op[4][2][HN][PS];                                              // k up, r up, k down, r down: head, tail
+    __bf16 Vt[HN][PS], Vtl[VSPLIT ? HN : 1][PS], Gh[HN][PS], Gl[HN][PS];
+    float C2[HN], Tot[8][HN];
+};
+template <typename IO, typename WT, bool W_IS_EW>
+__global__ __launch_bounds__(256, 2)
+void wkv6_bwd_seg_state_kernel(const IO* __restrict__ r_, const IO* __restrict__ k_, const IO* __restrict__ v_, const WT* __restrict__ w_,
+                               const float* __restrict__ gy_, float* __restrict__ ws, int* __restrict__ flags, int T, int C, int H,
+                               long long sequences, int nseg)
+{
+    constexpr bool VSPLIT = BwdSegLds<IO>::VSPLIT;
+    constexpr unsigned ES = (unsigned)sizeof(IO), WS = (unsigned)sizeof(WT);
+    __shared__ __attribute__((aligned(16))) BwdSegLds<IO> L;
+    const int lane = threadIdx.x & 63;
+    const int w4 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int bh, seg;
+    seg_of_block(blockIdx.x, nseg, bh, seg);
+    if (bh >= sequences) return;
+    const int b = bh / H, h = bh % H;
+    const size_t base = (size_t)b * T * C + (size_t)h * HN;
+    const int nchunk = (T + LC - 1) / LC, cps = (nchunk + nseg - 1) / nseg;
+    const int c0 = seg * cps, c1 = min(c0 + cps, nchunk);
+    const int grp = 2 * w4 + (lane >> 5), cp = 2 * (lane & 31);
+    using RawIO = typename BufRaw<2 * ES>::type;
+    using RawW = typename BufRaw<2 * WS>::type;
+    const unsigned n_el = (unsigned)((size_t)(T - 1) * C + HN);
+    const __amdgpu_buffer_rsrc_t rsr = make_rsrc(r_ + base, n_el * ES), rsk = make_rsrc(k_ + base, n_el * ES), rsv = make_rsrc(v_ + base, n_el * ES),
+                                 rsw = make_rsrc(w_ + base, n_el * WS), rsg = make_rsrc(gy_ + base, n_el * 4);
+    RawIO rraw[4], kraw[4], vraw[4];
+    RawW wraw[4];
+    f32x2 graw[4];
+    auto fetch = [&](int c) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const unsigned e = (unsigned)(c * LC + 4 * grp + m) * C + cp;
+            wraw[m] = BufRaw<2 * WS>::ld(rsw, e * WS, 0);
+            rraw[m] = BufRaw<2 * ES>::ld(rsr, e * ES, 0);
+            kraw[m] = BufRaw<2 * ES>::ld(rsk, e * ES, 0);
+            vraw[m] = BufRaw<2 * ES>::ld(rsv, e * ES, 0);
+            graw[m] = __builtin_bit_cast(f32x2, BufRaw<8>::ld(rsg, e * 4u, 0));
+        }
+    };
+    float p[2][4];
+    auto decays = [&](int c) {
+        pair_log_decays<WT, W_IS_EW>(wraw, p);
+        if ((c + 1) * LC > T) {
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+                if (c * LC + 4 * grp + m >= T) p[0][m] = p[1][m] = 0.f;
+        }
+#pragma unroll
+        for (int m = 1; m < 4; ++m) { p[0][m] += p[0][m - 1]; p[1][m] += p[1][m - 1]; }
+        *reinterpret_cast<f32x2*>(&L.Tot[grp][cp]) = f32x2{p[0][3], p[1][3]};
+    };
+    f32x4 st[4][4];                                                       // S up, G up, S down, G down; tile it: rows i = 16 it + 4 g4 + r
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int it = 0; it < 4; ++it) st[q][it] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float base_p[2] = {0.f, 0.f};
+    bool out_of_range = false;
+    fetch(c0);
+    decays(c0);
+    lds_barrier();
+    for (int c = c0; c < c1; ++c) {
+        float before[2], rest[2], tail[2], pre[2], p31[2];
+        pair_group_sums(L.Tot, w4, lane, cp, before, rest);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            tail[e] = p[e][3] + rest[e];
+            p31[e] = before[e] + tail[e];
+            pre[e] = base_p[e] + before[e];
+            out_of_range |= !(p31[e] >= -SAFE_DECAY * LOG2E);
+        }
+        unsigned op[4][2][2][2], vh[2][2], vl[2][2], gh[2][2], gl[2][2];  // [operand][head, tail][channel][token pair]
+        auto split = [&](float x0, float x1, unsigned& hi, unsigned& lo) {
+            hi = pack_bf16(x0, x1);
+            lo = tail_bf16(x0, x1, hi);
+        };
+#pragma unroll
+        for (int m = 0; m < 4; m += 2) {
+            float r0[2], r1[2], k0[2], k1[2], v0[2], v1[2];
+            pair_widen<IO>(rraw[m], r0); pair_widen<IO>(rraw[m + 1], r1);
+            pair_widen<IO>(kraw[m], k0); pair_widen<IO>(kraw[m + 1], k1);
+            pair_widen<IO>(vraw[m], v0); pair_widen<IO>(vraw[m + 1], v1);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const float fa0 = fast_exp2(tail[e] - p[e][m]), fa1 = fast_exp2(tail[e] - p[e][m + 1]);
+                const float fd0 = fast_exp2(m ? pre[e] + p[e][m - 1] : pre[e]), fd1 = fast_exp2(pre[e] + p[e][m]);
+                split(k0[e] * fa0, k1[e] * fa1, op[0][0][e][m / 2], op[0][1][e][m / 2]);
+                split(r0[e] * fa0, r1[e] * fa1, op[1][0][e][m / 2], op[1][1][e][m / 2]);
+                split(k0[e] * fd0, k1[e] * fd1, op[2][0][e][m / 2], op[2][1][e][m / 2]);
+                split(r0[e] * fd0, r1[e] * fd1, op[3][0][e][m / 2], op[3][1][e][m / 2]);
+                split(graw[m][e], graw[m + 1][e], gh[e][m / 2], gl[e][m / 2]);
+                split(v0[e], v1[e], vh[e][m / 2], vl[e][m / 2]);
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            auto put = [&](__bf16 (*arr)[PS], const unsigned (&x)[2]) { *reinterpret_cast<uint2*>(&arr[cp + e][4 * grp]) = make_uint2(x[0], x[1]); };
+#pragma unroll
+            for (int q = 0; q < 4; ++q) { put(L.Op[q][0], op[q][0][e]); put(L.Op[q][1], op[q][1][e]); }
+            put(L.Vt, vh[e]);
+            if constexpr (VSPLIT) put(L.Vtl, vl[e]);
+            put(L.Gh, gh[e]);
+            put(L.Gl, gl[e]);
+            base_p[e] += p31[e];
+        }
+        if (grp == 0) *reinterpret_cast<f32x2*>(&L.C2[cp]) = f32x2{fast_exp2(p31[0]), fast_exp2(p31[1])};
+        lds_barrier();
+        if (c + 1 < c1) fetch(c + 1);
+        {
+            const int g4 = lane >> 4, c16 = lane & 15, j = 16 * w4 + c16;
+            const float c2 = L.C2[j];
+            bf16x8 bh_[4], bl_[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                bh_[q] = *reinterpret_cast<const bf16x8*>(&L.Op[q][0][j][8 * g4]);
+                bl_[q] = *reinterpret_cast<const bf16x8*>(&L.Op[q][1][j][8 * g4]);
+            }
+#pragma unroll
+            for (int it = 0; it < 4; ++it) {
+                const bf16x8 av = *reinterpret_cast<const bf16x8*>(&L.Vt[16 * it + c16][8 * g4]);
+                bf16x8 avl;
+                if constexpr (VSPLIT) avl = *reinterpret_cast<const bf16x8*>(&L.Vtl[16 * it + c16][8 * g4]);
+                const bf16x8 ag = *reinterpret_cast<const bf16x8*>(&L.Gh[16 * it + c16][8 * g4]);
+                const bf16x8 agl = *reinterpret_cast<const bf16x8*>(&L.Gl[16 * it + c16][8 * g4]);
+                st[0][it] *= c2;
+                st[1][it] *= c2;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const bool g = q & 1;
+                    st[q][it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g ? ag : av, bh_[q], st[q][it], 0, 0, 0);
+                    st[q][it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g ? ag : av, bl_[q], st[q][it], 0, 0, 0);
+                    if (g) st[q][it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(agl, bh_[q], st[q][it], 0, 0, 0);
+                    if constexpr (VSPLIT)
+                        if (!g) st[q][it] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(avl, bh_[q], st[q][it], 0, 0, 0);
+                }
+            }
+        }
+        if (c + 1 < c1) decays(c + 1);
+        lds_barrier();
+    }
+    float* out = ws + ((size_t)bh * nseg + seg) * BWD_SEG_FLOATS;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int it = 0; it < 4; ++it) *reinterpret_cast<f32x4*>(out + q * SEG_STATE + seg_frag(w4, it, lane)) = st[q][it];
+    if (w4 == 0) {
+        if (lane < 32) *reinterpret_cast<f32x2*>(out + 4 * SEG_STATE + cp) = f32x2{fast_exp2(base_p[0]), fast_exp2(base_p[1])};
         const bool any = __builtin_amdgcn_ballot_w64(out_of_range) != 0ull;
         if (lane == 0) flags[(size_t)bh * nseg + seg] = any ? 1 : 0;
     }

@@ -169,11 +169,12 @@ def RUN_CUDA(*args):
 HEAD_SIZE = 64   # vrwkv6.py:23
 
 
-def wkv6_forward(B, T, C, H, r, k, v, w, u, w_is_ew=False, out=None):
+def wkv6_forward(B, T, C, H, r, k, v, w, u, w_is_ew=False, out=None, whole=False):
     """Extension-level entry (wkv6_op.cpp:7-9): r,k,v (B,T,C) fp32/bf16/fp16, w (B,T,C) fp32 or
     that dtype, u (H,64); returns y (B,T,C) fp32.  With w_is_ew=False, w is the raw decay logit
     (the kernel applies d = exp(-exp(w))); with True it is ew = -exp(w_raw) as the reference
-    extension receives it."""
+    extension receives it.  whole: no sequence is cut into segments (a call without workspace), so that y of a sequence
+    does not depend on how many there are."""
     for t, n in ((r, "r"), (k, "k"), (v, "v"), (w, "w"), (u, "u")):
         _check_input(t, n)
     if tuple(r.shape) != (B, T, C) or k.shape != r.shape or v.shape != r.shape or w.shape != r.shape:
@@ -190,7 +191,7 @@ def wkv6_forward(B, T, C, H, r, k, v, w, u, w_is_ew=False, out=None):
          else _check_out(out, "y", (B, T, C), torch.float32, r))      # the reference passes y in (wkv6_op.cpp:7-9)
     if y.numel() == 0:
         return y
-    ws_bytes = L.vrwkv_wkv6_fwd_workspace_bytes(B, T, C, H)
+    ws_bytes = 0 if whole else L.vrwkv_wkv6_fwd_workspace_bytes(B, T, C, H)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=r.device) if ws_bytes else None
     with torch.cuda.device(r.device):
         _lib.check(L.vrwkv_wkv6_fwd(r.data_ptr(), k.data_ptr(), v.data_ptr(), w.data_ptr(), uf.data_ptr(),
@@ -200,9 +201,10 @@ def wkv6_forward(B, T, C, H, r, k, v, w, u, w_is_ew=False, out=None):
     return y
 
 
-def wkv6_backward(B, T, C, H, r, k, v, w, u, gy, w_is_ew=False, out=None):
+def wkv6_backward(B, T, C, H, r, k, v, w, u, gy, w_is_ew=False, out=None, like_inputs=False):
     """Extension-level entry (wkv6_op.cpp:10-12): returns (gr, gk, gv, gw) as (B,T,C) fp32 and gu as
-    (H,64) fp32 (already summed over the batch); gw is the gradient w.r.t. the raw decay logit."""
+    (H,64) fp32 (already summed over the batch); gw is the gradient w.r.t. the raw decay logit.
+    like_inputs: gr, gk, gv, gw of their inputs' types, rounded from the fp32 sums by the kernel."""
     for t, n in ((r, "r"), (k, "k"), (v, "v"), (w, "w"), (u, "u"), (gy, "gy")):
         _check_input(t, n)
     if tuple(r.shape) != (B, T, C) or any(x.shape != r.shape for x in (k, v, w, gy)):
@@ -215,18 +217,21 @@ def wkv6_backward(B, T, C, H, r, k, v, w, u, gy, w_is_ew=False, out=None):
     gyf = gy if gy.dtype == torch.float32 else gy.float()
     L = _lib.lib()
     if out is None:
-        mk = lambda: torch.empty((B, T, C), device=r.device, dtype=torch.float32)
-        gr, gk, gv, gw = mk(), mk(), mk(), mk()
+        mk = lambda x: torch.empty((B, T, C), device=r.device, dtype=x.dtype if like_inputs else torch.float32)
+        gr, gk, gv, gw = mk(r), mk(k), mk(v), mk(w)
         gu = torch.empty((H, C // H), device=r.device, dtype=torch.float32)
     else:                                                             # caller-allocated (gr, gk, gv, gw, gu)
         gr, gk, gv, gw = (_check_out(t, n, (B, T, C), torch.float32, r) for t, n in zip(out[:4], ("gr", "gk", "gv", "gw")))
         gu = _check_out(out[4], "gu", (H, C // H), torch.float32, r)
     if gr.numel() == 0:
         return gr, gk, gv, gw, gu.zero_()
-    ws_bytes = L.vrwkv_wkv6_bwd_workspace_bytes(B, T, C, H)
+    if like_inputs:
+        fn, ws_bytes = L.vrwkv_wkv6_bwd_like, L.vrwkv_wkv6_bwd_like_workspace_bytes(B, T, C, H, _DT[r.dtype], _DT[w.dtype])
+    else:
+        fn, ws_bytes = L.vrwkv_wkv6_bwd, L.vrwkv_wkv6_bwd_workspace_bytes(B, T, C, H)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=r.device)
     with torch.cuda.device(r.device):
-        _lib.check(L.vrwkv_wkv6_bwd(r.data_ptr(), k.data_ptr(), v.data_ptr(), w.data_ptr(), uf.data_ptr(),
+        _lib.check(fn(r.data_ptr(), k.data_ptr(), v.data_ptr(), w.data_ptr(), uf.data_ptr(),
                                     gyf.data_ptr(), gr.data_ptr(), gk.data_ptr(), gv.data_ptr(), gw.data_ptr(),
                                     gu.data_ptr(), B, T, C, H, _DT[r.dtype], _DT[w.dtype], 1 if w_is_ew else 0,
                                     ws.data_ptr(), ws_bytes, _stream_ptr(r.device)))
@@ -249,15 +254,21 @@ class WKV_6(torch.autograd.Function):
             assert w.is_contiguous()
             assert u.is_contiguous()
             ctx.save_for_backward(r, k, v, w, u)
-            return wkv6_forward(B, T, C, H, r, k, v, w, u)
+            # A 16-bit network in training rounds y again in every block and amplifies last-bit differences from block to
+            # block (the weight gradients of twelve bf16 blocks move by 3e-2), so up to the sizes of image backbones its
+            # sequences stay whole and a sample's y is the same in any batch; cut into segments, 24 sequences of 1024
+            # tokens would take 45 instead of 90 us.
+            whole = T <= 1056 and r.dtype != torch.float32 and any(ctx.needs_input_grad)
+            return wkv6_forward(B, T, C, H, r, k, v, w, u, whole=whole)
 
     @staticmethod
     def backward(ctx, gy):
-        # vrwkv6.py:55-70: fp32 gradients, gu summed over the batch and shaped (H, C//H)
+        # vrwkv6.py:55-70: gu summed over the batch and shaped (H, C//H); the fp32 gradients leave the kernel rounded to
+        # their inputs' types, which is what autograd makes of them next
         with torch.no_grad():
             assert gy.is_contiguous()
             r, k, v, w, u = ctx.saved_tensors
-            gr, gk, gv, gw, gu = wkv6_backward(ctx.B, ctx.T, ctx.C, ctx.H, r, k, v, w, u, gy)
+            gr, gk, gv, gw, gu = wkv6_backward(ctx.B, ctx.T, ctx.C, ctx.H, r, k, v, w, u, gy, like_inputs=True)
             return (None, None, None, None, gr, gk, gv, gw, gu)
 
 
