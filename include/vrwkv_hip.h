@@ -222,6 +222,13 @@ int vrwkv_groupnorm_gate_bwd(const void* y, const void* gate, const void* gn_wei
                              float eps, int y_dtype, int io_dtype, void* workspace, size_t workspace_bytes,
                              void* hip_stream);
 
+/* ---- bicubic resampling of a position table (detection/mmdet_custom/models/utils/embed.py:6-47) ----
+ * adjoint 0: src (Hi*Wi, C) -> dst (Ho*Wo, C), cubic convolution (A = -0.75, sample points (o + 0.5) Hi/Ho - 0.5, taps
+ * clamped to the border); adjoint 1: src (Ho*Wo, C) = gradient of that result -> dst (Hi*Wi, C).  Row-major tokens, both of
+ * `dtype`, fp32 arithmetic.  The reference has no native code here. */
+int vrwkv_pos_resize(const void* src, void* dst, int Hi, int Wi, int Ho, int Wo, int C, int adjoint, int dtype,
+                     void* hip_stream);
+
 #ifdef __cplusplus
 }
 #endif

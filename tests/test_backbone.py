@@ -261,6 +261,34 @@ def test_pos_embed_resize_restates_the_interpolation():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("src,dst,C,dtype", [((14, 14), (24, 32), 768, torch.float32), ((12, 12), (24, 24), 1024, torch.bfloat16),
+                                             ((14, 14), (7, 9), 192, torch.float16), ((1, 3), (5, 1), 257, torch.float32),
+                                             ((40, 30), (3, 4), 33, torch.bfloat16), ((5, 4), (50, 84), 2, torch.float32)])
+def test_pos_embed_resize_kernel_against_the_interpolation_in_float64(src, dst, C, dtype):
+    """Result and gradient of the resampling kernel, with an extra token in front (whose slice makes odd row pitches and
+    offsets), against F.interpolate in float64: 16 products of weights of at most 1 and fp32 sample points (their rounding,
+    84 * 2^-24, shifts a weight by at most 1.5 times as much); the gradient adds up to 16 * (dst/src) products."""
+    from vision_rwkv_amd.backbone import resize_pos_embed
+    import torch.nn.functional as F
+    torch.manual_seed(2)
+    n = src[0] * src[1]
+    pe = torch.randn(1, 1 + n, C).to(dtype)
+    g = torch.randn(1, 1 + dst[0] * dst[1], C).to(dtype)
+    ref_in = pe.double().requires_grad_()
+    grid = ref_in[:, 1:].reshape(1, *src, C).permute(0, 3, 1, 2)
+    ref = F.interpolate(grid, size=dst, mode="bicubic", align_corners=False).flatten(2).transpose(1, 2)
+    ref = torch.cat((ref_in[:, :1], ref), 1)
+    gref, = torch.autograd.grad(ref, ref_in, g.double())
+    x = pe.cuda().requires_grad_()
+    out = resize_pos_embed(x, src, dst, "bicubic", num_extra_tokens=1)
+    gx, = torch.autograd.grad(out, x, g.cuda())
+    assert out.dtype == dtype and gx.dtype == dtype
+    eps = {torch.float32: 2e-5, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for a, r in ((out, ref), (gx, gref)):
+        assert (a.double().cpu() - r.detach()).abs().max() <= eps * max(1.0, r.abs().max().item())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("N,dtype", [(1024, torch.bfloat16), (4096, torch.bfloat16), (768, torch.float32),
                                      (3072, torch.float32), (64, torch.float16), (8192, torch.bfloat16),
                                      (768, torch.bfloat16), (2048, torch.bfloat16), (1032, torch.bfloat16)])

@@ -101,6 +101,8 @@ def _declare(lib):
     lib.vrwkv_groupnorm_gate_bwd_workspace_bytes.restype = sz
     lib.vrwkv_groupnorm_gate_bwd.argtypes = [vp, vp, vp, vp, vp, vp, vp, fp, c.c_longlong, i, i, c.c_float, i, i, vp, sz, vp]
     lib.vrwkv_groupnorm_gate_bwd.restype = i
+    lib.vrwkv_pos_resize.argtypes = [vp, vp, i, i, i, i, i, i, i, vp]
+    lib.vrwkv_pos_resize.restype = i
     return lib
 
 

@@ -14,8 +14,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .ops import (RUN_CUDA, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, PRE_NONE, PRE_RELU_SQ, POST_NONE, POST_SIGMOID_GATE,
-                  POST_RESIDUAL)
+from .ops import (RUN_CUDA, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, PRE_NONE, PRE_RELU_SQ, POST_NONE,
+                  POST_SIGMOID_GATE, POST_RESIDUAL)
 
 
 def resize_pos_embed(pos_embed, src_shape, dst_shape, mode="bicubic", num_extra_tokens=0):
@@ -28,6 +28,9 @@ def resize_pos_embed(pos_embed, src_shape, dst_shape, mode="bicubic", num_extra_
     if L != src_shape[0] * src_shape[1] + num_extra_tokens:
         raise RuntimeError(f"pos_embed has {L} tokens, expected {src_shape[0]}*{src_shape[1]}+{num_extra_tokens}")
     extra, grid = pos_embed[:, :num_extra_tokens], pos_embed[:, num_extra_tokens:]
+    w = resize_table(grid, src_shape, dst_shape) if mode == "bicubic" else None
+    if w is not None:
+        return torch.cat((extra, w), dim=1) if num_extra_tokens else w
     w = grid.reshape(1, src_shape[0], src_shape[1], C).permute(0, 3, 1, 2)
     w = F.interpolate(w.float(), size=dst_shape, align_corners=False, mode=mode).to(pos_embed.dtype)
     w = torch.flatten(w, 2).transpose(1, 2)

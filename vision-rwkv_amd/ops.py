@@ -647,3 +647,46 @@ def q_shift_mix_autograd(x, mixes, shift_pixel=1, gamma=1 / 4, patch_resolution=
         xx = q_shift(x, shift_pixel, gamma, patch_resolution)
         return [(x.float() * m + xx.float() * (1 - m)).to(x.dtype) for m in table]
     return list(_QShiftMix.apply(x, table, shift_pixel, gamma, Hp, Wp, head_dim))
+
+
+class _TableResize(torch.autograd.Function):
+    """Bicubic resampling of a (1, Hs*Ws, C) table, or its adjoint (vrwkv_pos_resize): linear maps, each the other's
+    derivative, so gradients of any order and forward-mode tangents go through the same two kernels."""
+
+    @staticmethod
+    def forward(ctx, table, src, dst, adjoint):
+        ctx.meta = (src, dst, adjoint)
+        return _table_resize_launch(table, src, dst, adjoint)
+
+    @staticmethod
+    def backward(ctx, g):
+        src, dst, adjoint = ctx.meta
+        return _TableResize.apply(g, src, dst, not adjoint), None, None, None
+
+    @staticmethod
+    def jvp(ctx, t, *_):
+        return _TableResize.apply(t, *ctx.meta)
+
+
+def _table_resize_launch(table, src, dst, adjoint):
+    table = table.contiguous()
+    n, C = (src if adjoint else dst), table.shape[-1]
+    out = torch.empty((1, n[0] * n[1], C), dtype=table.dtype, device=table.device)
+    with torch.cuda.device(table.device):
+        _lib.check(_lib.lib().vrwkv_pos_resize(table.data_ptr(), out.data_ptr(), src[0], src[1], dst[0], dst[1], C,
+                                               1 if adjoint else 0, _DT[table.dtype], _stream_ptr(table.device)))
+    return out
+
+
+def resize_table(table, src_shape, dst_shape):
+    """A (1, Hs*Ws, C) position table resampled bicubically to the grid dst_shape in one HIP kernel (and one for its
+    gradient): fp32 arithmetic, result of the table's type.  None where the kernel does not apply (off the GPU, other types
+    of tensor, traced or transformed calls, empty grids)."""
+    src, dst = tuple(int(n) for n in src_shape), tuple(int(n) for n in dst_shape)
+    if (not table.is_cuda or table.dtype not in _DT or table.dim() != 3 or table.shape[0] != 1
+            or type(table) not in (torch.Tensor, torch.nn.Parameter) or len(src) != 2 or len(dst) != 2
+            or min(src + dst) <= 0 or table.shape[1] != src[0] * src[1] or table.shape[2] == 0
+            or torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or torch._C._functorch.peek_interpreter_stack() is not None):
+        return None
+    return _TableResize.apply(table, src, dst, False)
