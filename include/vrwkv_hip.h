@@ -38,7 +38,7 @@ const char* vrwkv_last_error(void);      /* thread-local, never NULL */
 
 /* Tuning / testing switches, process-wide (no counterpart in the reference).  Names: "biwkv_l", "biwkv_s",
  * "biwkv_grid", "biwkv_no_stage", "biwkv_no_resident", "biwkv_bwd_serial", "wkv6_fwd_scalar", "wkv6_bwd_scalar",
- * "wkv6_bwd_unfused", "wkv6_segments"; 0 = default behaviour.  The initial value of <name> is that of the environment variable
+ * "wkv6_bwd_unfused", "wkv6_segments", "linear_tile"; 0 = default behaviour.  The initial value of <name> is that of the environment variable
  * VRWKV_<NAME> when the library first looks at any switch; the entry points never read the environment afterwards.
  * vrwkv_set_option rejects (VRWKV_INVALID_ARG) a value the plans would ignore: biwkv_l takes 0, 4, 8, 16, 25, 28 (tokens
  * per wave), biwkv_s 0 or 2..8 (waves per workgroup), biwkv_grid 0 or a positive workgroup count, wkv6_segments 0..64 (segments a sequence
@@ -228,6 +228,31 @@ int vrwkv_groupnorm_gate_bwd(const void* y, const void* gate, const void* gn_wei
  * `dtype`, fp32 arithmetic.  The reference has no native code here. */
 int vrwkv_pos_resize(const void* src, void* dst, int Hi, int Wi, int Ho, int Wo, int C, int adjoint, int dtype,
                      void* hip_stream);
+
+/* ---- inference of one VRWKV / VRWKV6 block on few tokens (.../backbones/vrwkv.py:265-319, vrwkv6.py:288-343) ----
+ * x -> out, both (B, T, C) of dtype (bf16 or fp16) like every weight; projections (out, in) row-major; C and hidden multiples
+ * of 32, hidden <= 8192; every pointer 16-byte aligned.  gamma1, gamma2 and the key_norm vectors (*_kn_*) may be NULL.
+ * att_mix: (3, C) [VRWKV: k, v, r] or (2, C) [VRWKV6: zeros, 1 - time_maa_x], ffn_mix: (2, C), both fp32 as for vrwkv_qshift_mix.
+ * VRWKV (heads = 0): w, u = decay and bonus divided by T, fp32; quarter = width of a shifted channel group.
+ * VRWKV6 (heads = C / 64): u (heads, 64) fp32; maa (5, C) fp32; maa_w1 (160, C), maa_w2 (5, C, 32), decay_w1 (64, C) and
+ * decay_w2 (C, 64) are the low-rank matrices with the contraction index innermost; att_kn_* are fp32.
+ * The reference has no native code here (PyTorch modules around the operator). */
+typedef struct vrwkv_block_args {
+    const void *x;
+    void *out, *workspace;
+    size_t workspace_bytes;
+    const void *ln1_w, *ln1_b, *ln2_w, *ln2_b, *gamma1, *gamma2;
+    const float *att_mix, *ffn_mix, *w, *u;
+    const void *key, *value, *receptance, *output, *att_kn_w, *att_kn_b;
+    const void *ffn_key, *ffn_receptance, *ffn_value, *ffn_kn_w, *ffn_kn_b;
+    const void *gate;
+    const float *maa;
+    const void *maa_w1, *maa_w2, *decay, *decay_w1, *decay_w2, *gn_w, *gn_b;
+    int B, T, C, hidden, heads, Hp, Wp, shift_pixel, quarter, post_norm, dtype;
+    float ln1_eps, ln2_eps, att_kn_eps, ffn_kn_eps, gn_eps;
+} vrwkv_block_args;
+size_t vrwkv_block_fwd_workspace_bytes(int B, int T, int C, int hidden, int heads, int dtype);
+int vrwkv_block_fwd(const vrwkv_block_args* args, void* hip_stream);
 
 #ifdef __cplusplus
 }

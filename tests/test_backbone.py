@@ -610,3 +610,74 @@ def test_split_weight_gradient_of_the_block_projections():
     assert "SplitK" not in type(bb._bmm(lo[:, :64], w2).grad_fn).__name__
     with torch.no_grad():
         assert bb._proj(lin, x).grad_fn is None
+
+
+def _small_backbone(kind, C, dtype, key_norm, post_norm, cls, hw):
+    import vision_rwkv_amd as ops
+    torch.manual_seed(11)
+    kw = dict(img_size=hw[0] * 16, embed_dims=C, depth=2, key_norm=key_norm, post_norm=post_norm, init_values=0.3 if post_norm else None)
+    net = ops.VRWKV6(num_heads=C // 64, with_cls_token=cls, **kw) if kind == "v6" else ops.VRWKV(**kw)
+    with torch.no_grad():
+        for n, p in net.named_parameters():
+            if "time_maa_w" in n and p.dim() > 1 and n[-1] in "12" or "decay_w" in n:
+                p.normal_(0, 0.02)
+            elif p.dim() < 2 or p.shape[0] == 1:
+                p.add_(0.05 * torch.randn_like(p))
+    return net.cuda().to(dtype).eval()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [0, 1, 2, 4])
+@pytest.mark.parametrize("kind,C,dtype,key_norm,post_norm,cls,hw,batch", [
+    ("v4", 192, torch.bfloat16, False, False, False, (14, 14), 1), ("v4", 64, torch.float16, True, False, False, (1, 3), 24),
+    ("v4", 416, torch.bfloat16, False, True, False, (7, 9), 3), ("v4", 256, torch.float16, True, True, False, (16, 15), 2),
+    ("v6", 192, torch.bfloat16, False, False, True, (14, 14), 1), ("v6", 64, torch.float16, True, True, False, (1, 1), 96),
+    ("v6", 384, torch.bfloat16, True, False, False, (9, 7), 3), ("v6", 128, torch.float16, False, True, True, (5, 13), 2)])
+def test_native_block_is_no_further_from_the_fp32_model_than_its_operators(kind, C, dtype, key_norm, post_norm, cls, hw, batch, tile):
+    """Two blocks as native calls and operator by operator, both against the same weights and image in fp32.  The native call
+    rounds at a subset of the places where the operators round, so its error may not exceed theirs.  Both norms are random:
+    the errors of one token move together (one normalised vector: 1.4 apart for a single token of 64 channels), so a norm
+    over n tokens scatters by about 1 / sqrt(2 n), their ratio by 1 / sqrt(n); with 65 or more tokens 1.25 is two of those
+    at least."""
+    net = _small_backbone(kind, C, dtype, key_norm, post_norm, cls, hw)
+    img = torch.randn(batch, 3, hw[0] * 16, hw[1] * 16, device="cuda").to(dtype)
+    from vision_rwkv_amd import ops as impl, option
+    with torch.no_grad():
+        x, res = net.embed(img)
+        x = x if not cls else torch.cat((x, x[:, :1]), 1)
+        assert all(l._native(x, res) is not None for l in net.layers)
+        with option("linear_tile", tile):
+            got = net(img).double()
+        impl.BLOCK_FUSE_ENABLED = False
+        try:
+            assert net.layers[0]._native(x, res) is None
+            plain = net(img).double()
+            ref = net.float()(img.float()).double()
+        finally:
+            impl.BLOCK_FUSE_ENABLED = True
+    assert (got - ref).norm() <= 1.25 * (plain - ref).norm()
+
+
+@pytest.mark.gpu
+def test_native_block_leaves_changed_modules_to_their_own_code():
+    net = _small_backbone("v4", 192, torch.bfloat16, False, False, False, (14, 14))
+    img = torch.randn(1, 3, 224, 224, device="cuda").bfloat16()
+    blk = net.layers[0]
+    with torch.no_grad():
+        x, res = net.embed(img)
+        base = net(img)
+        calls = []
+        h = blk.att.key.register_forward_hook(lambda *a: calls.append(1))
+        assert blk._native(x, res) is None
+        assert torch.allclose(net(img), base, rtol=0.1, atol=0.1) and calls
+        h.remove()
+        blk.ffn.key = torch.nn.Linear(192, 768, bias=True).cuda().bfloat16()
+        assert blk._native(x, res) is None and net.layers[1]._native(x, res) is not None
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert net.layers[1]._native(x, res) is None
+        assert net.layers[1]._native(x.transpose(0, 1).transpose(0, 1).expand(2, -1, -1), res) is None      # not contiguous
+        net.layers[1].att.output.weight.data = net.layers[1].att.output.weight.data.t()                     # transposed storage
+        assert net.layers[1]._native(x, res) is None
+        net.layers[1].float()
+        assert net.layers[1]._native(x, res) is None
+    assert net.layers[1]._native(x.detach().requires_grad_(), res) is None                                  # autograd on

@@ -17,6 +17,18 @@ STATUS_NAMES = {0: "OK", 1: "INVALID_ARG", 2: "UNSUPPORTED_DTYPE", 3: "UNSUPPORT
 _lib = None
 
 
+class BlockArgs(ctypes.Structure):
+    """vrwkv_block_args of include/vrwkv_hip.h."""
+    POINTERS_A = ("x", "out", "workspace")
+    POINTERS_B = ("ln1_w", "ln1_b", "ln2_w", "ln2_b", "gamma1", "gamma2", "att_mix", "ffn_mix", "w", "u", "key", "value",
+                  "receptance", "output", "att_kn_w", "att_kn_b", "ffn_key", "ffn_receptance", "ffn_value", "ffn_kn_w", "ffn_kn_b",
+                  "gate", "maa", "maa_w1", "maa_w2", "decay", "decay_w1", "decay_w2", "gn_w", "gn_b")
+    INTS = ("B", "T", "C", "hidden", "heads", "Hp", "Wp", "shift_pixel", "quarter", "post_norm", "dtype")
+    FLOATS = ("ln1_eps", "ln2_eps", "att_kn_eps", "ffn_kn_eps", "gn_eps")
+    _fields_ = ([(n, ctypes.c_void_p) for n in POINTERS_A] + [("workspace_bytes", ctypes.c_size_t)]
+                + [(n, ctypes.c_void_p) for n in POINTERS_B] + [(n, ctypes.c_int) for n in INTS] + [(n, ctypes.c_float) for n in FLOATS])
+
+
 class VrwkvError(RuntimeError):
     """Non-zero status from the C ABI (mirrors the RuntimeError TORCH_CHECK raises at
     classification/mmcls_custom/models/backbones/cuda_new/bi_wkv.cpp:6-8)."""
@@ -103,6 +115,10 @@ def _declare(lib):
     lib.vrwkv_groupnorm_gate_bwd.restype = i
     lib.vrwkv_pos_resize.argtypes = [vp, vp, i, i, i, i, i, i, i, vp]
     lib.vrwkv_pos_resize.restype = i
+    lib.vrwkv_block_fwd_workspace_bytes.argtypes = [i, i, i, i, i, i]
+    lib.vrwkv_block_fwd_workspace_bytes.restype = sz
+    lib.vrwkv_block_fwd.argtypes = [c.POINTER(BlockArgs), vp]
+    lib.vrwkv_block_fwd.restype = i
     return lib
 
 

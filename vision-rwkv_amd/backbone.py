@@ -13,8 +13,9 @@ import math
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules import module as _hooks
 
-from .ops import (RUN_CUDA, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, PRE_NONE, PRE_RELU_SQ, POST_NONE,
+from .ops import (RUN_CUDA, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, block_takes, block_weights_fit, block_forward, _equal_quarters, PRE_NONE, PRE_RELU_SQ, POST_NONE,
                   POST_SIGMOID_GATE, POST_RESIDUAL)
 
 
@@ -176,6 +177,65 @@ def _layer_norm(ln, x):
     return row_fuse(x, None, ln.weight, ln.bias, None, PRE_NONE, POST_NONE, ln.eps)
 
 
+# Multiplications per (C, C) projection up to which a block runs as one native call (vrwkv_block_fwd).  Twelve bf16 blocks,
+# operator by operator -> native, eager / replayed as a graph (GPU time alone), in us: 196 x 192 4037 -> 781 / 991 -> 499, 3136 x 384
+# 4000 -> 1425 / 1426 -> 1408, 784 x 768 3995 -> 1449 / 1426 -> 1428; VRWKV6 196 x 192 6496 -> 1107 / 1536 -> 900, 784 x 768
+# 6505 -> 2014 / 2346 -> 1990.  Beyond, the library's larger tiles win on the GPU (1568 x 768 1619 / 2023) while the calls
+# still take longer than the GPU work; the line is where neither loses.
+NATIVE_BLOCK_WORK = 470_000_000
+
+
+def _as_built(module, kind):
+    """True when calling `module` does what `kind`'s own forward does with the module's parameters and nothing else."""
+    return (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks and "forward" not in module.__dict__)
+
+
+def _block_weights(block, att, ffn, C):
+    """The weights of a block that one native call can run (its linear maps with the shapes and without the biases they are
+    built with, the norms with both vectors) and the numbers that go with them, as fields of vrwkv_block_args; None for any
+    other block."""
+    am, fm, bm = att._modules, ffn._modules, block._modules
+    key = fm["key"]
+    hidden = key._parameters["weight"].shape[0] if type(key) is nn.Linear else 0
+    if not (C % 32 == 0 and hidden % 32 == 0 and 0 < hidden <= 8192 and att.fused_shift and ffn.fused_shift
+            and att.shift_pixel == ffn.shift_pixel):
+        return None
+    w, num = {}, dict(hidden=hidden, shift_pixel=att.shift_pixel, post_norm=int(block.post_norm))
+    for name, lin, shape in (("key", am["key"], (C, C)), ("value", am["value"], (C, C)), ("receptance", am["receptance"], (C, C)),
+                             ("output", am["output"], (C, C)), ("ffn_key", key, (hidden, C)),
+                             ("ffn_receptance", fm["receptance"], (C, C)), ("ffn_value", fm["value"], (C, hidden))):
+        if not _as_built(lin, nn.Linear):
+            return None
+        p = lin._parameters
+        if p["bias"] is not None or p["weight"].shape != shape:
+            return None
+        w[name] = p["weight"]
+    for name, ln, n in (("ln1", bm["ln1"], C), ("ln2", bm["ln2"], C), ("att_kn", am.get("key_norm"), C),
+                        ("ffn_kn", fm.get("key_norm"), hidden)):
+        if ln is None and name.endswith("kn"):
+            continue
+        if not _as_built(ln, nn.LayerNorm) or ln.normalized_shape != (n,):
+            return None
+        p = ln._parameters
+        if p["weight"] is None or p["bias"] is None:
+            return None
+        w[name + "_w"], w[name + "_b"] = p["weight"], p["bias"]
+        num[name + "_eps"] = ln.eps
+    if block.layer_scale:
+        for name in ("gamma1", "gamma2"):
+            w[name] = block._parameters[name]
+            if w[name].shape != (C,):
+                return None
+    return w, num
+
+
+def _block_may_fuse(block, att_kind, ffn_kind, x):
+    """The checks that come before a look at the weights."""
+    return (not torch.is_grad_enabled() and x.numel() * x.shape[-1] <= NATIVE_BLOCK_WORK and block_takes(x)
+            and not _hooks._global_forward_hooks and not _hooks._global_forward_pre_hooks
+            and _as_built(block._modules["att"], att_kind) and _as_built(block._modules["ffn"], ffn_kind))
+
+
 class VRWKV_SpatialMix(nn.Module):
     def __init__(self, n_embd, n_layer, layer_id, channel_gamma=1 / 4, shift_pixel=1, key_norm=False, fused_shift=True):
         super().__init__()
@@ -269,9 +329,34 @@ class Block(nn.Module):
             self.gamma1 = nn.Parameter(init_values * torch.ones(n_embd))
             self.gamma2 = nn.Parameter(init_values * torch.ones(n_embd))
 
+    def _native(self, x, res):
+        """The block in one native call (vrwkv_block_fwd) where that computes the same; None elsewhere."""
+        if not _block_may_fuse(self, VRWKV_SpatialMix, VRWKV_ChannelMix, x):
+            return None
+        att, ffn = self._modules["att"], self._modules["ffn"]
+        T, C = x.shape[1:]
+        wn = _block_weights(self, att, ffn, C)
+        if (wn is None or not block_weights_fit(x, wn[0].values()) or T != res[0] * res[1] or not att.fused_gate or att.shift_pixel <= 0
+                or att.channel_gamma != ffn.channel_gamma or not _equal_quarters(C, att.channel_gamma, 0)):
+            return None
+        w, num = wn
+        ap, fp = att._parameters, ffn._parameters
+        decay, first = ap["spatial_decay"], ap["spatial_first"]
+        if decay.dtype != x.dtype:
+            return None
+        am, fm = [ap["spatial_mix_k"], ap["spatial_mix_v"], ap["spatial_mix_r"]], [fp["spatial_mix_k"], fp["spatial_mix_r"]]
+        w["w"], w["u"] = eval_cached(att, "wu", (decay, first), T,
+                                     lambda: ((decay / T).float().contiguous(), (first / T).float().contiguous()))
+        w["att_mix"] = eval_cached(att, "mix_table", am, x.device, lambda: stack_mixes(am, x.device))
+        w["ffn_mix"] = eval_cached(ffn, "mix_table", fm, x.device, lambda: stack_mixes(fm, x.device))
+        return block_forward(x, w, Hp=res[0], Wp=res[1], quarter=int(C * att.channel_gamma), **num)
+
     def forward(self, x, patch_resolution):
         if self.layer_id == 0:
             x = _layer_norm(self.ln0, x)
+        y = self._native(x, patch_resolution)
+        if y is not None:
+            return y
         g1 = self.gamma1 if self.layer_scale else None
         g2 = self.gamma2 if self.layer_scale else None
         # residual with layer scale (vrwkv.py:300-313): x + gamma * ln(branch(x)) or x + gamma * branch(ln(x)), the

@@ -10,8 +10,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .backbone import VRWKV, eval_cached, _proj, _matmul, _bmm
-from .ops import (HEAD_SIZE, RUN_CUDA_RWKV6, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, maa_mix, groupnorm_gate, PRE_NONE, PRE_RELU_SQ, POST_NONE,
+from .backbone import VRWKV, eval_cached, _proj, _matmul, _bmm, _as_built, _block_may_fuse, _block_weights
+from .ops import (HEAD_SIZE, RUN_CUDA_RWKV6, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, maa_mix, groupnorm_gate, block_weights_fit, block_forward, PRE_NONE, PRE_RELU_SQ, POST_NONE,
                   POST_SIGMOID_GATE, POST_RESIDUAL)
 
 
@@ -148,9 +148,48 @@ class Block6(nn.Module):
             self.gamma1 = nn.Parameter(init_values * torch.ones(n_embd))
             self.gamma2 = nn.Parameter(init_values * torch.ones(n_embd))
 
+    def _native(self, x, res):
+        """The block in one native call (vrwkv_block_fwd) where that computes the same; None elsewhere."""
+        if not _block_may_fuse(self, VRWKV_SpatialMix_V6, VRWKV_ChannelMix_V6, x):
+            return None
+        att, ffn = self._modules["att"], self._modules["ffn"]
+        T, C = x.shape[1:]
+        wn = _block_weights(self, att, ffn, C)
+        if wn is None:
+            return None
+        w, num = wn
+        ap, fp, ln_x, gate = att._parameters, ffn._parameters, att._modules["ln_x"], att._modules["gate"]
+        low = (ap["time_maa_w1"], ap["time_maa_w2"], ap["time_decay_w1"], ap["time_decay_w2"])
+        if (not _as_built(gate, nn.Linear) or gate.bias is not None or gate.weight.shape != (C, C)
+                or not _as_built(ln_x, nn.GroupNorm) or ln_x.num_groups * HEAD_SIZE != C or ln_x.num_channels != C or not ln_x.affine
+                or att.n_head * HEAD_SIZE != C or ap["time_decay"].numel() != C or ap["time_faaaa"].numel() != C
+                or tuple(t.shape for t in low) != ((C, 160), (5, 32, C), (C, 64), (64, C))
+                or T != res[0] * res[1] + (1 if att.with_cls_token else 0) or att.with_cls_token != ffn.with_cls_token):
+            return None
+        w.update(gate=gate.weight, decay=ap["time_decay"], gn_w=ln_x.weight, gn_b=ln_x.bias)
+        if not block_weights_fit(x, (*w.values(), *low)):
+            return None
+        cm = (fp["spatial_mix_k"], fp["spatial_mix_r"])
+        maas = tuple(ap["time_maa_" + n] for n in "wkvrg")
+        mx, first = ap["time_maa_x"], ap["time_faaaa"]
+        # the low-rank matrices with the contraction index innermost, like every other projection's
+        w["maa_w1"], w["maa_w2"], w["decay_w1"], w["decay_w2"] = eval_cached(
+            att, "low_rank", low, None, lambda: [t.detach().transpose(-1, -2).contiguous() for t in low])
+        w["u"] = eval_cached(att, "u", (first,), None, lambda: first.detach().float().contiguous())
+        w["att_mix"] = eval_cached(att, "mix_table", (mx,), x.device, lambda: stack_mixes([torch.zeros_like(mx), 1 - mx], x.device))
+        w["ffn_mix"] = eval_cached(ffn, "mix_table", cm, x.device, lambda: stack_mixes(cm, x.device))
+        w["maa"] = eval_cached(att, "maa_table", maas, x.device, lambda: stack_mixes(maas, x.device))
+        if "att_kn_w" in w:                                  # normalises the operator's fp32 result
+            kn = (w["att_kn_w"], w["att_kn_b"])
+            w["att_kn_w"], w["att_kn_b"] = eval_cached(att, "kn32", kn, None, lambda: [p.detach().float() for p in kn])
+        return block_forward(x, w, Hp=res[0], Wp=res[1], heads=att.n_head, quarter=HEAD_SIZE // 4, gn_eps=ln_x.eps, **num)
+
     def forward(self, x, patch_resolution):
         if self.layer_id == 0:
             x = _layer_norm(self.ln0, x)
+        y = self._native(x, patch_resolution)
+        if y is not None:
+            return y
         g1 = self.gamma1 if self.layer_scale else None
         g2 = self.gamma2 if self.layer_scale else None
         if self.post_norm:                                   # scale, add and post-norm in one pass

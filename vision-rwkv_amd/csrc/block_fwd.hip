@@ -1,0 +1,312 @@
+// Inference of one whole VRWKV / VRWKV6 block on few tokens: one entry point issues the block's kernels, with the
+// projections on matrix cores here, several of them in one launch and the element-wise steps around them in their epilogues.
+//
+// A block of one 224 x 224 image (196 tokens) is 16 (VRWKV) or 26 (VRWKV6) operator calls of 2-20 us of GPU work each, and a call
+// through the Python operators and the library costs about 20 us of host time, so the host sets the pace; on top the
+// library picks tiles of 192 x 256 for 196 x 192 results (13 us a product).  Issued from here a VRWKV block is 9 launches:
+//   LN | shift + mixes | key, value, receptance | Bi-WKV with gate | output + residual
+//   LN | shift + mixes | key with relu^2, receptance | value, gate, residual
+#include "vrwkv_common.h"
+#include <algorithm>
+#include <type_traits>
+
+namespace vrwkv {
+namespace {
+
+// ---- the projections ---------------------------------------------------------------------------------------------------
+// out = epilogue(A W^T): A (M, K) with row pitch lda, W (N, K), out (M, N), 16-bit with fp32 accumulation.  Both operands have
+// the contraction index innermost, which is the order of the MFMA fragments (16 x 16 x 32: lane l holds row l & 15, eight
+// k from 8 (l >> 4)), so they go from global memory to registers in 16-byte pieces without a stage in LDS.  At these sizes
+// everything lies in the L2s and latency counts: a workgroup owns a tile of (16 MT)^2 results, its four waves take every
+// fourth slice of 32 k each with D slices requested ahead, and add up through LDS in a fixed order.  The weights are the
+// first operand, so a lane ends up with four neighbouring channels of a token: 8-byte accesses in the epilogue.
+enum { EPI_RELU_SQ = 1, EPI_TANH = 2, EPI_ADD_VEC = 4 };
+struct LinProblem {
+    const void *a, *w;
+    void* out;
+    const void *gate, *vec, *res;   // all optional: v *= sigmoid(gate); v *= vec (or v += vec with EPI_ADD_VEC); v += res
+    int N, K, lda, epi, tile0;
+};
+constexpr int LIN_MAX = 5;
+struct LinGroup {
+    LinProblem p[LIN_MAX];
+    int n, M;
+};
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+template <typename IO> __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
+    if constexpr (std::is_same<IO, __hip_bfloat16>::value)
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
+template <typename IO, int MT>
+__global__ __launch_bounds__(256)
+void linear_group_kernel(LinGroup G)
+{
+    constexpr int TILE = 16 * MT, D = MT == 4 ? 2 : 3;
+    __shared__ f32x4 red[4][MT * MT][WAVE];
+    const int lane = threadIdx.x & 63, g4 = lane >> 4, c16 = lane & 15;
+    const int w4 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int q = 0;
+    while (q + 1 < G.n && (int)blockIdx.x >= G.p[q + 1].tile0) ++q;
+    const LinProblem& P = G.p[q];
+    const int N = P.N, K = P.K, M = G.M, nt = (N + TILE - 1) / TILE;
+    const int tile = (int)blockIdx.x - P.tile0, m0 = tile / nt * TILE, n0 = tile % nt * TILE;
+    // rows past M or N lie outside the descriptors and read 0
+    const __amdgpu_buffer_rsrc_t rsa = make_rsrc(P.a, ((unsigned)(M - 1) * P.lda + K) * 2u), rsw = make_rsrc(P.w, (unsigned)N * K * 2u);
+    unsigned oa[MT], ow[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        oa[i] = (unsigned)(m0 + 16 * i + c16) * P.lda * 2u + 16u * g4;
+        ow[i] = (unsigned)(n0 + 16 * i + c16) * K * 2u + 16u * g4;
+    }
+    u32x4 fa[D][MT], fw[D][MT];
+    auto fetch = [&](int s, int d) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            fw[d][i] = BufRaw<16>::ld(rsw, ow[i], 64u * s);
+            fa[d][i] = BufRaw<16>::ld(rsa, oa[i], 64u * s);
+        }
+    };
+    f32x4 acc[MT][MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int steps = K / 32;
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (w4 + 4 * d < steps) fetch(w4 + 4 * d, d);
+    for (int s = w4; s < steps; s += 4 * D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            const int cur = s + 4 * d;
+            if (cur >= steps) break;                      // wave-uniform
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < MT; ++j) acc[i][j] = mfma<IO>(fw[d][j], fa[d][i], acc[i][j]);
+            if (cur + 4 * D < steps) fetch(cur + 4 * D, d);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) red[w4][i * MT + j][lane] = acc[i][j];
+    __syncthreads();
+    const IO *gate = (const IO*)P.gate, *vec = (const IO*)P.vec, *res = (const IO*)P.res;
+    IO* out = (IO*)P.out;
+    for (int t = w4; t < MT * MT; t += 4) {
+        const int m = m0 + 16 * (t / MT) + c16, n = n0 + 16 * (t % MT) + 4 * g4;
+        if (m >= M || n >= N) continue;
+        const f32x4 s = (red[0][t][lane] + red[1][t][lane]) + (red[2][t][lane] + red[3][t][lane]);
+        float v[4], x[4];
+        const size_t off = (size_t)m * N + n;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = s[e];
+            if (P.epi & EPI_RELU_SQ) { const float r = fmaxf(v[e], 0.f); v[e] = r * r; }
+            if (P.epi & EPI_TANH) v[e] = tanhf(v[e]);
+        }
+        if (gate) {
+            load_vec<IO, 4>(gate + off, x);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] *= fast_rcp(1.f + fast_exp2(-LOG2E * x[e]));
+        }
+        if (vec) {
+            load_vec<IO, 4>(vec + n, x);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = P.epi & EPI_ADD_VEC ? v[e] + x[e] : v[e] * x[e];
+        }
+        if (res) {
+            load_vec<IO, 4>(res + off, x);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += x[e];
+        }
+        store_vec<IO, 4>(out + off, v);
+    }
+}
+
+template <int MT>
+void launch_group(LinGroup& G, int dtype, hipStream_t st) {
+    int tiles = 0;
+    for (int i = 0; i < G.n; ++i) {
+        G.p[i].tile0 = tiles;
+        tiles += ((G.M + 16 * MT - 1) / (16 * MT)) * ((G.p[i].N + 16 * MT - 1) / (16 * MT));
+    }
+    if (dtype == VRWKV_BF16) hipLaunchKernelGGL((linear_group_kernel<__hip_bfloat16, MT>), dim3(tiles), dim3(256), 0, st, G);
+    else hipLaunchKernelGGL((linear_group_kernel<__half, MT>), dim3(tiles), dim3(256), 0, st, G);
+}
+// The largest tile that still gives every compute unit a workgroup: larger tiles read less from the L2s, smaller ones
+// shorten the chain of a wave.
+int linear_group(LinGroup& G, int dtype, hipStream_t st) {
+    long long area = 0;
+    for (int i = 0; i < G.n; ++i) area += (long long)G.M * G.p[i].N;
+    const int force = option(OPT_LINEAR_TILE);
+    const int mt = force ? force : area >= 64LL * 64 * 256 ? 4 : area >= 32LL * 32 * 128 ? 2 : 1;
+    if (mt == 4) launch_group<4>(G, dtype, st);
+    else if (mt == 2) launch_group<2>(G, dtype, st);
+    else launch_group<1>(G, dtype, st);
+    return check_launch("linear_group");
+}
+LinProblem linear(const void* a, const void* w, void* out, int N, int K, int lda = 0, int epi = 0) {
+    return LinProblem{a, w, out, nullptr, nullptr, nullptr, N, K, lda ? lda : K, epi, 0};
+}
+
+// ---- the block -----------------------------------------------------------------------------------------------------------
+size_t al(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
+// token tensors of C channels that live at the same time: LN result, up to six mixes, x after the attention half, and the
+// operator's tensors
+struct Layout { size_t n, hidden, op, total; };
+Layout layout(int B, int T, int C, int hidden, int heads, int dtype) {
+    Layout l;
+    l.n = al((size_t)B * T * C * 2);
+    l.hidden = al((size_t)B * T * hidden * 2);
+    l.op = heads ? al(vrwkv_wkv6_fwd_workspace_bytes(B, T, C, heads)) : al(vrwkv_biwkv_fwd_workspace_bytes(B, T, C, dtype));
+    // VRWKV: 9 tensors; VRWKV6: x1, LN, sx, xxx, five mixes, five maps (later r, k, v, w, gate), two fp32 tensors, low-rank rows
+    const size_t tokens = heads ? 2 + 2 + 5 + 5 + 4 : 9;
+    const size_t low = heads ? al((size_t)B * T * 160 * 2) + al((size_t)B * T * 64 * 2) : 0;
+    l.total = tokens * l.n + 2 * l.hidden + low + l.op;           // (hidden rows twice: before and after their norm)
+    return l;
+}
+
+}  // namespace
+}  // namespace vrwkv
+
+#define TRY(call) do { const int rc_ = (call); if (rc_ != VRWKV_OK) return rc_; } while (0)
+
+extern "C" size_t vrwkv_block_fwd_workspace_bytes(int B, int T, int C, int hidden, int heads, int dtype)
+{
+    if (B <= 0 || T <= 0 || C <= 0 || hidden <= 0 || heads < 0) return 0;
+    return vrwkv::layout(B, T, C, hidden, heads, dtype).total;
+}
+
+extern "C" int vrwkv_block_fwd(const vrwkv_block_args* a, void* hip_stream)
+{
+    using namespace vrwkv;
+    if (!a || !a->x || !a->out || !a->workspace || !a->ln1_w || !a->ln1_b || !a->ln2_w || !a->ln2_b || !a->att_mix || !a->ffn_mix ||
+        !a->u || !a->key || !a->value || !a->receptance || !a->output || !a->ffn_key || !a->ffn_receptance || !a->ffn_value ||
+        (a->heads ? !a->gate || !a->maa || !a->maa_w1 || !a->maa_w2 || !a->decay || !a->decay_w1 || !a->decay_w2 || !a->gn_w || !a->gn_b
+                  : !a->w) ||
+        (!a->att_kn_w != !a->att_kn_b) || (!a->ffn_kn_w != !a->ffn_kn_b)) {
+        set_error("block_fwd: null pointer argument");
+        return VRWKV_INVALID_ARG;
+    }
+    const int B = a->B, T = a->T, C = a->C, hidden = a->hidden, H = a->heads, dt = a->dtype;
+    if (dt != VRWKV_BF16 && dt != VRWKV_F16) {
+        set_error("block_fwd: dtype must be bf16 or fp16");
+        return VRWKV_UNSUPPORTED_DTYPE;
+    }
+    const long long M = (long long)B * T;
+    if (B <= 0 || T <= 0 || C <= 0 || C % 32 || hidden <= 0 || hidden % 32 || hidden > 8192 || C > 8192 || H < 0 || (H && C != 64 * H) ||
+        M * std::max(C, hidden) * 2 >= (1LL << 30) || (long long)C * hidden * 2 >= (1LL << 30)) {
+        set_error("block_fwd: unsupported sizes (B=%d T=%d C=%d hidden=%d heads=%d)", B, T, C, hidden, H);
+        return VRWKV_UNSUPPORTED_SHAPE;
+    }
+    const void* aligned[] = {a->x, a->out, a->workspace, a->ln1_w, a->ln1_b, a->ln2_w, a->ln2_b, a->gamma1, a->gamma2, a->key, a->value, a->receptance,
+                             a->output, a->att_kn_w, a->att_kn_b, a->ffn_key, a->ffn_receptance, a->ffn_value, a->ffn_kn_w, a->ffn_kn_b,
+                             a->gate, a->maa_w1, a->maa_w2, a->decay, a->decay_w1, a->decay_w2, a->gn_w, a->gn_b, a->w, a->u, a->att_mix, a->ffn_mix, a->maa};
+    for (const void* p : aligned)
+        if ((size_t)p & 15) {
+            set_error("block_fwd: every tensor must be 16-byte aligned");
+            return VRWKV_INVALID_ARG;
+        }
+    const Layout L = layout(B, T, C, hidden, H, dt);
+    if (a->workspace_bytes < L.total) {
+        set_error("block_fwd: workspace of %zu bytes, %zu needed", a->workspace_bytes, L.total);
+        return VRWKV_WORKSPACE_TOO_SMALL;
+    }
+    char* at = (char*)a->workspace;
+    auto take = [&](size_t bytes) { void* p = at; at += bytes; return p; };
+    hipStream_t st = static_cast<hipStream_t>(hip_stream);
+    const int hd = H ? 64 : 0;
+    void *x1 = take(L.n), *ln = take(L.n), *hid = take(L.hidden), *hid_raw = take(L.hidden), *op_ws = take(L.op);
+    LinGroup G;
+    G.M = (int)M;
+    // branch -> x: gamma * branch + x in the projection's epilogue, or with the post-norm in a row kernel
+    auto residual = [&](LinProblem p, const void* x, void* out, const void* gamma, const void* w, const void* b, float eps, void* tmp) {
+        G.n = 1;
+        if (!a->post_norm) { p.vec = gamma; p.res = x; p.out = out; }
+        else p.out = tmp;
+        G.p[0] = p;
+        TRY(linear_group(G, dt, st));
+        return a->post_norm ? vrwkv_rowfuse(tmp, x, w, b, gamma, out, M, C, 0, 2, eps, dt, st) : (int)VRWKV_OK;
+    };
+
+    const void* x = a->x;
+    const void* src = x;                                  // input of a half
+    if (!a->post_norm) { TRY(vrwkv_rowfuse(x, nullptr, a->ln1_w, a->ln1_b, nullptr, ln, M, C, 0, 0, a->ln1_eps, dt, st)); src = ln; }
+    char* half = at;                                      // both halves use what follows
+    void* y;
+    if (!H) {
+        void* m[3] = {take(L.n), take(L.n), take(L.n)};
+        void *k = take(L.n), *v = take(L.n), *r = take(L.n);
+        TRY(vrwkv_qshift_mix(src, a->att_mix, m, 3, B, T, C, a->Hp, a->Wp, a->shift_pixel, a->quarter, 0, dt, st));
+        G.n = 3;
+        G.p[0] = linear(m[0], a->key, k, C, C);
+        G.p[1] = linear(m[1], a->value, v, C, C);
+        G.p[2] = linear(m[2], a->receptance, r, C, C);
+        TRY(linear_group(G, dt, st));
+        y = m[0];
+        if (a->att_kn_w) {
+            TRY(vrwkv_biwkv_fwd(a->w, a->u, k, v, m[1], B, T, C, dt, L.op ? op_ws : nullptr, L.op, st));
+            TRY(vrwkv_rowfuse(m[1], r, a->att_kn_w, a->att_kn_b, nullptr, y, M, C, 0, 1, a->att_kn_eps, dt, st));
+        } else {
+            TRY(vrwkv_biwkv_fwd_gate(a->w, a->u, k, v, r, y, B, T, C, dt, L.op ? op_ws : nullptr, L.op, st));
+        }
+    } else {
+        void* s[2] = {take(L.n), take(L.n)};              // shifted x, the mix that feeds the low-rank maps
+        char* maps = at;
+        void* five[5];
+        for (void*& p : five) p = take(L.n);
+        void* m[5];
+        for (void*& p : m) p = take(L.n);
+        float *yf = (float*)take(2 * L.n), *yn = (float*)take(2 * L.n);
+        void *lo = take(al((size_t)M * 160 * 2)), *dlo = take(al((size_t)M * 64 * 2));
+        TRY(vrwkv_qshift_mix(src, a->att_mix, s, 2, B, T, C, a->Hp, a->Wp, a->shift_pixel, 16, hd, dt, st));
+        G.n = 1;
+        G.p[0] = linear(s[1], a->maa_w1, lo, 160, C, 0, EPI_TANH);
+        TRY(linear_group(G, dt, st));
+        G.n = 5;
+        for (int i = 0; i < 5; ++i)                       // the five maps as one (5, M, C) tensor
+            G.p[i] = linear((const char*)lo + 64 * i, (const char*)a->maa_w2 + (size_t)i * C * 64, maps + (size_t)i * M * C * 2, C, 32, 160);
+        TRY(linear_group(G, dt, st));
+        TRY(vrwkv_maa_mix(src, s[0], maps, a->maa, m, M, C, dt, st));                 // w, k, v, r, g
+        G.p[0] = linear(m[0], a->decay_w1, dlo, 64, C, 0, EPI_TANH);
+        G.p[1] = linear(m[1], a->key, five[1], C, C);
+        G.p[2] = linear(m[2], a->value, five[2], C, C);
+        G.p[3] = linear(m[3], a->receptance, five[3], C, C);
+        G.p[4] = linear(m[4], a->gate, five[4], C, C);
+        TRY(linear_group(G, dt, st));
+        G.n = 1;
+        G.p[0] = linear(dlo, a->decay_w2, five[0], C, 64, 0, EPI_ADD_VEC);
+        G.p[0].vec = a->decay;
+        TRY(linear_group(G, dt, st));
+        TRY(vrwkv_wkv6_fwd(five[3], five[1], five[2], five[0], a->u, yf, B, T, C, H, dt, dt, 0, L.op ? op_ws : nullptr, L.op, st));
+        if (a->att_kn_w) {
+            TRY(vrwkv_rowfuse(yf, nullptr, a->att_kn_w, a->att_kn_b, nullptr, yn, M, C, 0, 0, a->att_kn_eps, VRWKV_F32, st));
+            yf = yn;
+        }
+        y = m[0];
+        TRY(vrwkv_groupnorm_gate(yf, five[4], a->gn_w, a->gn_b, y, M, C, 64, a->gn_eps, VRWKV_F32, dt, st));
+    }
+    TRY(residual(linear(y, a->output, nullptr, C, C), x, x1, a->gamma1, a->ln1_w, a->ln1_b, a->ln1_eps, ln));
+    at = half;
+    src = x1;
+    if (!a->post_norm) { TRY(vrwkv_rowfuse(x1, nullptr, a->ln2_w, a->ln2_b, nullptr, ln, M, C, 0, 0, a->ln2_eps, dt, st)); src = ln; }
+    void *f[2] = {take(L.n), take(L.n)}, *fr = take(L.n), *ftmp = take(L.n);
+    TRY(vrwkv_qshift_mix(src, a->ffn_mix, f, 2, B, T, C, a->Hp, a->Wp, a->shift_pixel, H ? 16 : a->quarter, hd, dt, st));
+    G.n = 2;
+    G.p[0] = linear(f[0], a->ffn_key, a->ffn_kn_w ? hid_raw : hid, hidden, C, 0, a->ffn_kn_w ? 0 : EPI_RELU_SQ);
+    G.p[1] = linear(f[1], a->ffn_receptance, fr, C, C);
+    TRY(linear_group(G, dt, st));
+    if (a->ffn_kn_w) TRY(vrwkv_rowfuse(hid_raw, nullptr, a->ffn_kn_w, a->ffn_kn_b, nullptr, hid, M, hidden, 1, 0, a->ffn_kn_eps, dt, st));
+    LinProblem p = linear(hid, a->ffn_value, nullptr, C, hidden);
+    p.gate = fr;
+    return residual(p, x1, a->out, a->gamma2, a->ln2_w, a->ln2_b, a->ln2_eps, ftmp);
+}

@@ -678,6 +678,13 @@ def _table_resize_launch(table, src, dst, adjoint):
     return out
 
 
+def _transformed():
+    """True inside torch.compile, jit tracing, a functorch transform or a dispatch / function mode, which are to see the
+    tensor ops."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0)
+
+
 def resize_table(table, src_shape, dst_shape):
     """A (1, Hs*Ws, C) position table resampled bicubically to the grid dst_shape in one HIP kernel (and one for its
     gradient): fp32 arithmetic, result of the table's type.  None where the kernel does not apply (off the GPU, other types
@@ -686,7 +693,48 @@ def resize_table(table, src_shape, dst_shape):
     if (not table.is_cuda or table.dtype not in _DT or table.dim() != 3 or table.shape[0] != 1
             or type(table) not in (torch.Tensor, torch.nn.Parameter) or len(src) != 2 or len(dst) != 2
             or min(src + dst) <= 0 or table.shape[1] != src[0] * src[1] or table.shape[2] == 0
-            or torch.compiler.is_compiling() or torch.jit.is_tracing()
-            or torch._C._functorch.peek_interpreter_stack() is not None):
+            or _transformed()):
         return None
     return _TableResize.apply(table, src, dst, False)
+
+
+BLOCK_FUSE_ENABLED = True    # set False to make the blocks run operator by operator everywhere (for comparisons)
+
+
+def block_takes(x):
+    """True where vrwkv_block_fwd may stand in for a block's operators: no autograd, a plain contiguous 16-bit GPU tensor
+    outside every kind of transform."""
+    return (BLOCK_FUSE_ENABLED and ROW_FUSE_ENABLED and not torch.is_grad_enabled() and type(x) is torch.Tensor and x.is_cuda
+            and x.dtype in (torch.bfloat16, torch.float16) and x.dim() == 3 and x.numel() > 0 and x.is_contiguous()
+            and not torch.is_autocast_enabled("cuda") and not _transformed())
+
+
+def block_weights_fit(x, weights):
+    """True when every weight is a plain contiguous parameter of x's type and device."""
+    dt, dev, kind = x.dtype, x.get_device(), torch.nn.Parameter
+    for p in weights:
+        if type(p) is not kind or p.dtype != dt or p.get_device() != dev or not p.is_contiguous():
+            return False
+    return True
+
+
+def block_forward(x, tensors, **scalars):
+    """vrwkv_block_fwd on the current stream: tensors and scalars fill the like-named fields of vrwkv_block_args.  None when
+    a tensor is not aligned for 16-byte accesses."""
+    L = _lib.lib()
+    B, T, C = x.shape
+    out = torch.empty_like(x)
+    ptrs = {n: t.data_ptr() for n, t in tensors.items()}
+    ptrs["x"], ptrs["out"] = x.data_ptr(), out.data_ptr()
+    bits = 0
+    for p in ptrs.values():
+        bits |= p
+    if bits & 15:
+        return None
+    a = _lib.BlockArgs(B=B, T=T, C=C, dtype=_DT[x.dtype], **ptrs, **scalars)
+    a.workspace_bytes = L.vrwkv_block_fwd_workspace_bytes(B, T, C, a.hidden, a.heads, a.dtype)
+    ws = torch.empty(a.workspace_bytes, dtype=torch.uint8, device=x.device)
+    a.workspace = ws.data_ptr()
+    with torch.cuda.device(x.device):
+        _lib.check(L.vrwkv_block_fwd(ctypes.byref(a), _stream_ptr(x.device)))
+    return out
