@@ -38,7 +38,7 @@ const char* vrwkv_last_error(void);      /* thread-local, never NULL */
 
 /* Tuning / testing switches, process-wide (no counterpart in the reference).  Names: "biwkv_l", "biwkv_s",
  * "biwkv_grid", "biwkv_no_stage", "biwkv_no_resident", "biwkv_bwd_serial", "wkv6_fwd_scalar", "wkv6_bwd_scalar",
- * "wkv6_bwd_unfused", "wkv6_segments", "linear_tile"; 0 = default behaviour.  The initial value of <name> is that of the environment variable
+ * "wkv6_bwd_unfused", "wkv6_segments", "linear_tile", "wgrad_splits"; 0 = default behaviour.  The initial value of <name> is that of the environment variable
  * VRWKV_<NAME> when the library first looks at any switch; the entry points never read the environment afterwards.
  * vrwkv_set_option rejects (VRWKV_INVALID_ARG) a value the plans would ignore: biwkv_l takes 0, 4, 8, 16, 25, 28 (tokens
  * per wave), biwkv_s 0 or 2..8 (waves per workgroup), biwkv_grid 0 or a positive workgroup count, wkv6_segments 0..64 (segments a sequence
@@ -253,6 +253,15 @@ typedef struct vrwkv_block_args {
 } vrwkv_block_args;
 size_t vrwkv_block_fwd_workspace_bytes(int B, int T, int C, int hidden, int heads, int dtype);
 int vrwkv_block_fwd(const vrwkv_block_args* args, void* hip_stream);
+
+/* ---- weight gradients of the projections ----
+ * out[z] (O, I) = sum over m of g[z][m][o] x[z][m][i], z < n: rows of g and x at pitches ldg, ldx (elements, multiples of 8),
+ * stacks at strides stride_g, stride_x; 16-bit operands and result (dtype), fp32 sums rounded once; O and I multiples of 8,
+ * every pointer 16-byte aligned.  workspace: vrwkv_wgrad_workspace_bytes(n, M, O, I) bytes.  The reference has no native code
+ * here (autograd of nn.Linear). */
+size_t vrwkv_wgrad_workspace_bytes(int n, int M, int O, int I);
+int vrwkv_wgrad(const void* g, const void* x, void* out, int n, int M, int O, int I, int ldg, int ldx, long long stride_g,
+                long long stride_x, int dtype, void* workspace, size_t workspace_bytes, void* hip_stream);
 
 #ifdef __cplusplus
 }

@@ -681,3 +681,44 @@ def test_native_block_leaves_changed_modules_to_their_own_code():
         net.layers[1].float()
         assert net.layers[1]._native(x, res) is None
     assert net.layers[1]._native(x.detach().requires_grad_(), res) is None                                  # autograd on
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("splits", [0, 1, 3])
+@pytest.mark.parametrize("n,M,O,I,dtype", [(1, 1, 8, 8, torch.bfloat16), (1, 31, 8, 136, torch.float16), (1, 33, 128, 120, torch.bfloat16),
+                                           (2, 300, 136, 264, torch.float16), (5, 1000, 32, 768, torch.bfloat16),
+                                           (1, 4096, 160, 384, torch.bfloat16), (1, 4099, 1024, 1024, torch.float16)])
+def test_weight_gradient_kernel_against_float64(n, M, O, I, dtype, splits):
+    """a^T b over the tokens at tile edges and remainders, with rows in their own tensors, inside wider ones, at odd addresses
+    and transposed: one rounding of the result (8 / 11 significant bits: at most 2^-8 / 2^-11 of the value) and fp32 sums of M terms (2^-24 M of the
+    magnitudes' sum)."""
+    from vision_rwkv_amd import option
+    from vision_rwkv_amd.ops import weight_grad
+    torch.manual_seed(5)
+    a, b = (torch.randn(n, M, c, device="cuda").to(dtype) for c in (O, I))
+    wide = torch.full((M, n, O + 24), float("nan"), device="cuda", dtype=dtype)
+    wide[..., 8:8 + O] = a.transpose(0, 1)
+    odd = torch.empty(n * M * I + 1, device="cuda", dtype=dtype)[1:].view(n, M, I).copy_(b)
+    ref = a.double().transpose(1, 2) @ b.double()
+    mag = a.double().abs().transpose(1, 2) @ b.double().abs()
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    bound = unit * 1.01 * ref.abs() + (M + 4) * 2.0 ** -24 * mag + 1e-7
+    with option("wgrad_splits", splits):
+        outs = [weight_grad(a, b), weight_grad(wide[..., 8:8 + O].transpose(0, 1), odd),
+                weight_grad(a, b.transpose(1, 2).contiguous().transpose(1, 2))]
+        if n == 1:
+            outs.append(weight_grad(a[0], b[0])[None])
+    for got in outs:
+        assert got.dtype == dtype and got.shape == ref.shape and bool(((got.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.gpu
+def test_second_derivative_of_a_projection_goes_through_tensor_ops():
+    from vision_rwkv_amd.backbone import _SplitKLinear
+    torch.manual_seed(6)
+    x = torch.randn(4096, 64, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    w = torch.randn(64, 64, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    y = _SplitKLinear.apply(x, w, 8)
+    gw, = torch.autograd.grad(y.float().square().sum(), w, create_graph=True)
+    ggx, = torch.autograd.grad(gw.float().sum(), x)
+    assert ggx.shape == x.shape and bool(torch.isfinite(ggx).all()) and ggx.abs().max() > 0

@@ -119,6 +119,11 @@ def _declare(lib):
     lib.vrwkv_block_fwd_workspace_bytes.restype = sz
     lib.vrwkv_block_fwd.argtypes = [c.POINTER(BlockArgs), vp]
     lib.vrwkv_block_fwd.restype = i
+    ll = c.c_longlong
+    lib.vrwkv_wgrad_workspace_bytes.argtypes = [i, i, i, i]
+    lib.vrwkv_wgrad_workspace_bytes.restype = sz
+    lib.vrwkv_wgrad.argtypes = [vp, vp, vp, i, i, i, i, i, i, ll, ll, i, vp, sz, vp]
+    lib.vrwkv_wgrad.restype = i
     return lib
 
 

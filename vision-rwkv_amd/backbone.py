@@ -15,7 +15,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch.nn.modules import module as _hooks
 
-from .ops import (RUN_CUDA, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, block_takes, block_weights_fit, block_forward, _equal_quarters, PRE_NONE, PRE_RELU_SQ, POST_NONE,
+from .ops import (RUN_CUDA, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, weight_grad, block_takes, block_weights_fit, block_forward, _equal_quarters, PRE_NONE, PRE_RELU_SQ, POST_NONE,
                   POST_SIGMOID_GATE, POST_RESIDUAL)
 
 
@@ -62,10 +62,27 @@ def _mix(module, x, mixes, shift_pixel, gamma, patch_resolution, fused, head_dim
     return [x * m + xx * (1 - m) for m in mixes]
 
 
+# Elements of a weight up to which its gradient is the framework's own kernel: 12544 tokens, own / the library's batched
+# partial products and their sum, in us: 768 x 768 34 / 43, 384 x 384 22 / 37, 1536 x 384 33 / 42, 192 x 192 15 / 25, 160 x 768 22 / 36,
+# five of 32 x 768 24 / 44; 3072 x 768 88 / 76.
+OWN_WEIGHT_GRAD = 1 << 20
+
+
+def _token_product(a, b, splits):
+    """a^T b over the rows (tokens) of a (M, O), b (M, I) or of stacks of them: the own kernel (fp32 sums, rounded once), or
+    `splits` batched partial products of the library.  A gradient that is itself to be differentiated takes tensor ops."""
+    (M, O), I = a.shape[-2:], b.shape[-1]
+    if (not torch.is_grad_enabled() and O * I <= OWN_WEIGHT_GRAD and O % 8 == 0 and I % 8 == 0 and a.dtype == b.dtype
+            and M * max(a.stride(-2), b.stride(-2), O, I) < 1 << 30):
+        return weight_grad(a, b)
+    S = splits if M % splits == 0 else 1
+    part = torch.matmul(a.reshape(a.shape[:-2] + (S, M // S, O)).transpose(-1, -2), b.reshape(b.shape[:-2] + (S, M // S, I)))
+    return part.sum(-3)                   # one kernel: the sum of 16-bit values accumulates in fp32 and is rounded once
+
+
 class _SplitKLinear(torch.autograd.Function):
     """x @ W^T whose weight gradient g^T x -- a contraction over all B*T tokens into a small (out, in) matrix, which the
-    library's GEMM runs as one deep sum on too few workgroups -- is computed as `splits` batched partial products that
-    are added in fp32.  Forward and input gradient are the library's plain GEMMs."""
+    library's GEMM runs as one deep sum on too few workgroups -- is split over the tokens (_token_product).  Forward and input gradient are the library's plain GEMMs."""
 
     @staticmethod
     def forward(ctx, x, weight, splits):
@@ -80,10 +97,7 @@ class _SplitKLinear(torch.autograd.Function):
         gx = g @ weight if ctx.needs_input_grad[0] else None
         gw = None
         if ctx.needs_input_grad[1]:
-            g2, x2 = g.reshape(-1, g.shape[-1]), x.reshape(-1, x.shape[-1])
-            M = g2.shape[0]
-            part = torch.bmm(g2.view(S, M // S, -1).transpose(1, 2), x2.view(S, M // S, -1))
-            gw = part.sum(0)              # one kernel: the sum of 16-bit values accumulates in fp32 and is rounded once
+            gw = _token_product(g.reshape(-1, g.shape[-1]), x.reshape(-1, x.shape[-1]), S)
         return gx, gw, None
 
 
@@ -103,10 +117,7 @@ class _SplitKMatmul(torch.autograd.Function):
         gx = g @ weight.t() if ctx.needs_input_grad[0] else None
         gw = None
         if ctx.needs_input_grad[1]:
-            g2, x2 = g.reshape(-1, g.shape[-1]), x.reshape(-1, x.shape[-1])
-            M = g2.shape[0]
-            part = torch.bmm(x2.view(S, M // S, -1).transpose(1, 2), g2.view(S, M // S, -1))
-            gw = part.sum(0)              # accumulated in fp32, rounded once
+            gw = _token_product(x.reshape(-1, x.shape[-1]), g.reshape(-1, g.shape[-1]), S)
         return gx, gw, None
 
 
@@ -128,11 +139,7 @@ class _SplitKBmm(torch.autograd.Function):
         gx = torch.bmm(g, weight.transpose(1, 2)) if ctx.needs_input_grad[0] else None
         gw = None
         if ctx.needs_input_grad[1]:
-            n, M, _ = x.shape
-            x4 = x.reshape(n, S, M // S, x.shape[-1])
-            g4 = g.reshape(n, S, M // S, g.shape[-1])
-            part = torch.matmul(x4.transpose(2, 3), g4)               # (n, S, in, out)
-            gw = part.sum(1)              # accumulated in fp32, rounded once
+            gw = _token_product(x, g, S)
         return gx, gw, None
 
 

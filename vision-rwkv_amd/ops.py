@@ -35,7 +35,8 @@ def _check_out(t, name, shape, dtype, like):
 
 
 def _stream_ptr(device):
-    return torch.cuda.current_stream(device).cuda_stream
+    # the handle itself: building a Stream object around it takes 2 us of every call
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def bi_wkv_forward(w, u, k, v, out=None, gate=None):
@@ -737,4 +738,33 @@ def block_forward(x, tensors, **scalars):
     a.workspace = ws.data_ptr()
     with torch.cuda.device(x.device):
         _lib.check(L.vrwkv_block_fwd(ctypes.byref(a), _stream_ptr(x.device)))
+    return out
+
+
+def _token_rows(t):
+    """t (n, M, C) with every row in 16-byte pieces, copied where it is not laid out so."""
+    sn, sm, sc = t.stride()
+    if sc == 1 and sm >= t.shape[2] and not (sn | sm) & 7 and not t.data_ptr() & 15:
+        return t
+    return t.clone(memory_format=torch.contiguous_format)
+
+
+def weight_grad(g, x):
+    """sum over t of g[.., t, o] x[.., t, i] for token matrices g (M, O), x (M, I) or stacks (n, M, O), (n, M, I) of one 16-bit
+    type, O and I multiples of 8: the gradient of a projection's weight (O, I), fp32 sums rounded once.  Rows may lie at any
+    pitch of 16-byte pieces; other layouts are copied."""
+    stack = g.dim() == 3
+    g3, x3 = (_token_rows(g), _token_rows(x)) if stack else (_token_rows(g[None]), _token_rows(x[None]))
+    n, M, O = g3.shape
+    I = x3.shape[2]
+    out = torch.empty((n, O, I) if stack else (O, I), dtype=g.dtype, device=g.device)
+    if out.numel() == 0 or M == 0:
+        return out.zero_()
+    L = _lib.lib()
+    ws_bytes = L.vrwkv_wgrad_workspace_bytes(n, M, O, I)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=g.device)
+    gs, xs = g3.stride(), x3.stride()
+    with torch.cuda.device(g.device):
+        _lib.check(L.vrwkv_wgrad(g3.data_ptr(), x3.data_ptr(), out.data_ptr(), n, M, O, I, gs[1], xs[1], gs[0], xs[0],
+                                 _DT[g.dtype], ws.data_ptr(), ws_bytes, _stream_ptr(g.device)))
     return out
