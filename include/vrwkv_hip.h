@@ -230,8 +230,8 @@ int vrwkv_pos_resize(const void* src, void* dst, int Hi, int Wi, int Ho, int Wo,
                      void* hip_stream);
 
 /* ---- inference of one VRWKV / VRWKV6 block on few tokens (.../backbones/vrwkv.py:265-319, vrwkv6.py:288-343) ----
- * x -> out, both (B, T, C) of dtype (bf16 or fp16) like every weight; projections (out, in) row-major; C and hidden multiples
- * of 32, hidden <= 8192; every pointer 16-byte aligned.  gamma1, gamma2 and the key_norm vectors (*_kn_*) may be NULL.
+ * x -> out, both (B, T, C) of dtype like every weight; projections (out, in) row-major; C and hidden multiples of 32, hidden <= 8192
+ * (fp32: 4096); every pointer 16-byte aligned.  gamma1, gamma2 and the key_norm vectors (*_kn_*) may be NULL.
  * att_mix: (3, C) [VRWKV: k, v, r] or (2, C) [VRWKV6: zeros, 1 - time_maa_x], ffn_mix: (2, C), both fp32 as for vrwkv_qshift_mix.
  * VRWKV (heads = 0): w, u = decay and bonus divided by T, fp32; quarter = width of a shifted channel group.
  * VRWKV6 (heads = C / 64): u (heads, 64) fp32; maa (5, C) fp32; maa_w1 (160, C), maa_w2 (5, C, 32), decay_w1 (64, C) and

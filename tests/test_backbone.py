@@ -632,7 +632,9 @@ def _small_backbone(kind, C, dtype, key_norm, post_norm, cls, hw):
     ("v4", 192, torch.bfloat16, False, False, False, (14, 14), 1), ("v4", 64, torch.float16, True, False, False, (1, 3), 24),
     ("v4", 416, torch.bfloat16, False, True, False, (7, 9), 3), ("v4", 256, torch.float16, True, True, False, (16, 15), 2),
     ("v6", 192, torch.bfloat16, False, False, True, (14, 14), 1), ("v6", 64, torch.float16, True, True, False, (1, 1), 96),
-    ("v6", 384, torch.bfloat16, True, False, False, (9, 7), 3), ("v6", 128, torch.float16, False, True, True, (5, 13), 2)])
+    ("v6", 384, torch.bfloat16, True, False, False, (9, 7), 3), ("v4", 160, torch.float32, True, False, False, (9, 7), 2),
+    ("v4", 192, torch.float32, False, True, False, (14, 14), 1), ("v6", 192, torch.float32, True, False, True, (14, 13), 1),
+    ("v6", 128, torch.float16, False, True, True, (5, 13), 2)])
 def test_native_block_is_no_further_from_the_fp32_model_than_its_operators(kind, C, dtype, key_norm, post_norm, cls, hw, batch, tile):
     """Two blocks as native calls and operator by operator, both against the same weights and image in fp32.  The native call
     rounds at a subset of the places where the operators round, so its error may not exceed theirs.  Both norms are random:
@@ -652,10 +654,15 @@ def test_native_block_is_no_further_from_the_fp32_model_than_its_operators(kind,
         try:
             assert net.layers[0]._native(x, res) is None
             plain = net(img).double()
-            ref = net.float()(img.float()).double()
+            ref = net.float()(img.float()).double() if dtype != torch.float32 else plain
         finally:
             impl.BLOCK_FUSE_ENABLED = True
-    assert (got - ref).norm() <= 1.25 * (plain - ref).norm()
+    if dtype == torch.float32:
+        # two fp32 paths: products of up to 4 C = 768 terms, sqrt(768) 2^-24 = 1.7e-6 each, eight of them in a row and as
+        # much again in VRWKV6's normalised, exponentiated decays
+        assert (got - plain).norm() <= 2.8e-5 * plain.norm()
+    else:
+        assert (got - ref).norm() <= 1.25 * (plain - ref).norm()
 
 
 @pytest.mark.gpu

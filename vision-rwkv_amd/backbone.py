@@ -189,7 +189,21 @@ def _layer_norm(ln, x):
 # 4000 -> 1425 / 1426 -> 1408, 784 x 768 3995 -> 1449 / 1426 -> 1428; VRWKV6 196 x 192 6496 -> 1107 / 1536 -> 900, 784 x 768
 # 6505 -> 2014 / 2346 -> 1990.  Beyond, the library's larger tiles win on the GPU (1568 x 768 1619 / 2023) while the calls
 # still take longer than the GPU work; the line is where neither loses.
+# fp32: 196 x 192 4773 -> 747, 3136 x 384 3740 -> 2485 / 2448 -> 2463, 392 x 768 3697 -> 1807 / 1920 -> 1792, but 784 x 768 2307 / 2535 and
+# 1568 x 768 3415 / 3919 on the GPU; from 3136 x 768 on (7064 / 6371, 6272 x 768 12392 / 11386) the library is behind again.
 NATIVE_BLOCK_WORK = 470_000_000
+NATIVE_BLOCK_WORK_FP32 = (420_000_000, 1_700_000_000)                      # up to the first, and from the second on
+
+
+def _native_size(x, hidden):
+    """The rule above, and 32-bit byte offsets inside every token matrix of the call."""
+    M, C = x.shape[0] * x.shape[1], x.shape[2]
+    if M * max(C, hidden, 160) * x.element_size() >= 1 << 30:
+        return False
+    if x.dtype == torch.float32:
+        lo, hi = NATIVE_BLOCK_WORK_FP32
+        return not lo < M * C * C < hi
+    return M * C * C <= NATIVE_BLOCK_WORK
 
 
 def _as_built(module, kind):
@@ -197,15 +211,15 @@ def _as_built(module, kind):
     return (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks and "forward" not in module.__dict__)
 
 
-def _block_weights(block, att, ffn, C):
+def _block_weights(block, att, ffn, x):
     """The weights of a block that one native call can run (its linear maps with the shapes and without the biases they are
     built with, the norms with both vectors) and the numbers that go with them, as fields of vrwkv_block_args; None for any
     other block."""
-    am, fm, bm = att._modules, ffn._modules, block._modules
+    am, fm, bm, C = att._modules, ffn._modules, block._modules, x.shape[2]
     key = fm["key"]
     hidden = key._parameters["weight"].shape[0] if type(key) is nn.Linear else 0
-    if not (C % 32 == 0 and hidden % 32 == 0 and 0 < hidden <= 8192 and att.fused_shift and ffn.fused_shift
-            and att.shift_pixel == ffn.shift_pixel):
+    if not (C % 32 == 0 and hidden % 32 == 0 and 0 < hidden <= 4096 and att.fused_shift and ffn.fused_shift
+            and att.shift_pixel == ffn.shift_pixel and _native_size(x, hidden)):
         return None
     w, num = {}, dict(hidden=hidden, shift_pixel=att.shift_pixel, post_norm=int(block.post_norm))
     for name, lin, shape in (("key", am["key"], (C, C)), ("value", am["value"], (C, C)), ("receptance", am["receptance"], (C, C)),
@@ -238,7 +252,7 @@ def _block_weights(block, att, ffn, C):
 
 def _block_may_fuse(block, att_kind, ffn_kind, x):
     """The checks that come before a look at the weights."""
-    return (not torch.is_grad_enabled() and x.numel() * x.shape[-1] <= NATIVE_BLOCK_WORK and block_takes(x)
+    return (block_takes(x)
             and not _hooks._global_forward_hooks and not _hooks._global_forward_pre_hooks
             and _as_built(block._modules["att"], att_kind) and _as_built(block._modules["ffn"], ffn_kind))
 
@@ -342,7 +356,7 @@ class Block(nn.Module):
             return None
         att, ffn = self._modules["att"], self._modules["ffn"]
         T, C = x.shape[1:]
-        wn = _block_weights(self, att, ffn, C)
+        wn = _block_weights(self, att, ffn, x)
         if (wn is None or not block_weights_fit(x, wn[0].values()) or T != res[0] * res[1] or not att.fused_gate or att.shift_pixel <= 0
                 or att.channel_gamma != ffn.channel_gamma or not _equal_quarters(C, att.channel_gamma, 0)):
             return None

@@ -154,7 +154,7 @@ class Block6(nn.Module):
             return None
         att, ffn = self._modules["att"], self._modules["ffn"]
         T, C = x.shape[1:]
-        wn = _block_weights(self, att, ffn, C)
+        wn = _block_weights(self, att, ffn, x)
         if wn is None:
             return None
         w, num = wn

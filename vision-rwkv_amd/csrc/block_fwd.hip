@@ -14,11 +14,11 @@ namespace vrwkv {
 namespace {
 
 // ---- the projections ---------------------------------------------------------------------------------------------------
-// out = epilogue(A W^T): A (M, K) with row pitch lda, W (N, K), out (M, N), 16-bit with fp32 accumulation.  Both operands have
+// out = epilogue(A W^T): A (M, K) with row pitch lda, W (N, K), out (M, N), of one type, with fp32 accumulation.  Both operands have
 // the contraction index innermost, which is the order of the MFMA fragments (16 x 16 x 32: lane l holds row l & 15, eight
 // k from 8 (l >> 4)), so they go from global memory to registers in 16-byte pieces without a stage in LDS.  At these sizes
 // everything lies in the L2s and latency counts: a workgroup owns a tile of (16 MT)^2 results, its four waves take every
-// fourth slice of 32 k each with D slices requested ahead, and add up through LDS in a fixed order.  The weights are the
+// fourth slice of 64 bytes of k each with D slices requested ahead, and add up through LDS in a fixed order.  The weights are the
 // first operand, so a lane ends up with four neighbouring channels of a token: 8-byte accesses in the epilogue.
 enum { EPI_RELU_SQ = 1, EPI_TANH = 2, EPI_ADD_VEC = 4 };
 struct LinProblem {
@@ -37,8 +37,15 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+// one 16-byte fragment of either operand: 32 k in 16 bits; in fp32 16 k as four products of 4, lane group g taking the k
+// 4 g .. of both operands
 template <typename IO> __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
-    if constexpr (std::is_same<IO, __hip_bfloat16>::value)
+    if constexpr (std::is_same<IO, float>::value) {
+        const f32x4 fa = __builtin_bit_cast(f32x4, a), fb = __builtin_bit_cast(f32x4, b);   // (of one element it takes element 0)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[e], fb[e], c, 0, 0, 0);
+        return c;
+    } else if constexpr (std::is_same<IO, __hip_bfloat16>::value)
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
     else
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
@@ -49,6 +56,7 @@ __global__ __launch_bounds__(256)
 void linear_group_kernel(LinGroup G)
 {
     constexpr int TILE = 16 * MT, D = MT == 4 ? 2 : 3;
+    constexpr unsigned ES = sizeof(IO);
     __shared__ f32x4 red[4][MT * MT][WAVE];
     const int lane = threadIdx.x & 63, g4 = lane >> 4, c16 = lane & 15;
     const int w4 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -58,12 +66,12 @@ void linear_group_kernel(LinGroup G)
     const int N = P.N, K = P.K, M = G.M, nt = (N + TILE - 1) / TILE;
     const int tile = (int)blockIdx.x - P.tile0, m0 = tile / nt * TILE, n0 = tile % nt * TILE;
     // rows past M or N lie outside the descriptors and read 0
-    const __amdgpu_buffer_rsrc_t rsa = make_rsrc(P.a, ((unsigned)(M - 1) * P.lda + K) * 2u), rsw = make_rsrc(P.w, (unsigned)N * K * 2u);
+    const __amdgpu_buffer_rsrc_t rsa = make_rsrc(P.a, ((unsigned)(M - 1) * P.lda + K) * ES), rsw = make_rsrc(P.w, (unsigned)N * K * ES);
     unsigned oa[MT], ow[MT];
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
-        oa[i] = (unsigned)(m0 + 16 * i + c16) * P.lda * 2u + 16u * g4;
-        ow[i] = (unsigned)(n0 + 16 * i + c16) * K * 2u + 16u * g4;
+        oa[i] = (unsigned)(m0 + 16 * i + c16) * P.lda * ES + 16u * g4;
+        ow[i] = (unsigned)(n0 + 16 * i + c16) * K * ES + 16u * g4;
     }
     u32x4 fa[D][MT], fw[D][MT];
     auto fetch = [&](int s, int d) {
@@ -78,7 +86,7 @@ void linear_group_kernel(LinGroup G)
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int steps = K / 32;
+    const int steps = K * ES / 64;
 #pragma unroll
     for (int d = 0; d < D; ++d)
         if (w4 + 4 * d < steps) fetch(w4 + 4 * d, d);
@@ -140,7 +148,8 @@ void launch_group(LinGroup& G, int dtype, hipStream_t st) {
         tiles += ((G.M + 16 * MT - 1) / (16 * MT)) * ((G.p[i].N + 16 * MT - 1) / (16 * MT));
     }
     if (dtype == VRWKV_BF16) hipLaunchKernelGGL((linear_group_kernel<__hip_bfloat16, MT>), dim3(tiles), dim3(256), 0, st, G);
-    else hipLaunchKernelGGL((linear_group_kernel<__half, MT>), dim3(tiles), dim3(256), 0, st, G);
+    else if (dtype == VRWKV_F16) hipLaunchKernelGGL((linear_group_kernel<__half, MT>), dim3(tiles), dim3(256), 0, st, G);
+    else hipLaunchKernelGGL((linear_group_kernel<float, MT>), dim3(tiles), dim3(256), 0, st, G);
 }
 // The largest tile that still gives every compute unit a workgroup: larger tiles read less from the L2s, smaller ones
 // shorten the chain of a wave.
@@ -165,12 +174,13 @@ size_t al(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
 struct Layout { size_t n, hidden, op, total; };
 Layout layout(int B, int T, int C, int hidden, int heads, int dtype) {
     Layout l;
-    l.n = al((size_t)B * T * C * 2);
-    l.hidden = al((size_t)B * T * hidden * 2);
+    const size_t es = dtype == VRWKV_F32 ? 4 : 2;
+    l.n = al((size_t)B * T * C * es);
+    l.hidden = al((size_t)B * T * hidden * es);
     l.op = heads ? al(vrwkv_wkv6_fwd_workspace_bytes(B, T, C, heads)) : al(vrwkv_biwkv_fwd_workspace_bytes(B, T, C, dtype));
     // VRWKV: 9 tensors; VRWKV6: x1, LN, sx, xxx, five mixes, five maps (later r, k, v, w, gate), two fp32 tensors, low-rank rows
     const size_t tokens = heads ? 2 + 2 + 5 + 5 + 4 : 9;
-    const size_t low = heads ? al((size_t)B * T * 160 * 2) + al((size_t)B * T * 64 * 2) : 0;
+    const size_t low = heads ? al((size_t)B * T * 160 * es) + al((size_t)B * T * 64 * es) : 0;
     l.total = tokens * l.n + 2 * l.hidden + low + l.op;           // (hidden rows twice: before and after their norm)
     return l;
 }
@@ -198,13 +208,14 @@ extern "C" int vrwkv_block_fwd(const vrwkv_block_args* a, void* hip_stream)
         return VRWKV_INVALID_ARG;
     }
     const int B = a->B, T = a->T, C = a->C, hidden = a->hidden, H = a->heads, dt = a->dtype;
-    if (dt != VRWKV_BF16 && dt != VRWKV_F16) {
-        set_error("block_fwd: dtype must be bf16 or fp16");
+    const size_t es = dt == VRWKV_F32 ? 4 : 2;
+    if (dt != VRWKV_F32 && dt != VRWKV_BF16 && dt != VRWKV_F16) {
+        set_error("block_fwd: unknown dtype %d", dt);
         return VRWKV_UNSUPPORTED_DTYPE;
     }
     const long long M = (long long)B * T;
-    if (B <= 0 || T <= 0 || C <= 0 || C % 32 || hidden <= 0 || hidden % 32 || hidden > 8192 || C > 8192 || H < 0 || (H && C != 64 * H) ||
-        M * std::max(C, hidden) * 2 >= (1LL << 30) || (long long)C * hidden * 2 >= (1LL << 30)) {
+    if (B <= 0 || T <= 0 || C <= 0 || C % 32 || hidden <= 0 || hidden % 32 || hidden > 16384 / (int)es || C > 8192 || H < 0 || (H && C != 64 * H) ||
+        M * std::max({C, hidden, 160}) * (long long)es >= (1LL << 30) || (long long)C * hidden * (long long)es >= (1LL << 30)) {
         set_error("block_fwd: unsupported sizes (B=%d T=%d C=%d hidden=%d heads=%d)", B, T, C, hidden, H);
         return VRWKV_UNSUPPORTED_SHAPE;
     }
@@ -267,14 +278,14 @@ extern "C" int vrwkv_block_fwd(const vrwkv_block_args* a, void* hip_stream)
         void* m[5];
         for (void*& p : m) p = take(L.n);
         float *yf = (float*)take(2 * L.n), *yn = (float*)take(2 * L.n);
-        void *lo = take(al((size_t)M * 160 * 2)), *dlo = take(al((size_t)M * 64 * 2));
+        void *lo = take(al((size_t)M * 160 * es)), *dlo = take(al((size_t)M * 64 * es));
         TRY(vrwkv_qshift_mix(src, a->att_mix, s, 2, B, T, C, a->Hp, a->Wp, a->shift_pixel, 16, hd, dt, st));
         G.n = 1;
         G.p[0] = linear(s[1], a->maa_w1, lo, 160, C, 0, EPI_TANH);
         TRY(linear_group(G, dt, st));
         G.n = 5;
         for (int i = 0; i < 5; ++i)                       // the five maps as one (5, M, C) tensor
-            G.p[i] = linear((const char*)lo + 64 * i, (const char*)a->maa_w2 + (size_t)i * C * 64, maps + (size_t)i * M * C * 2, C, 32, 160);
+            G.p[i] = linear((const char*)lo + 32 * es * i, (const char*)a->maa_w2 + (size_t)i * C * 32 * es, maps + (size_t)i * M * C * es, C, 32, 160);
         TRY(linear_group(G, dt, st));
         TRY(vrwkv_maa_mix(src, s[0], maps, a->maa, m, M, C, dt, st));                 // w, k, v, r, g
         G.p[0] = linear(m[0], a->decay_w1, dlo, 64, C, 0, EPI_TANH);

@@ -703,10 +703,10 @@ BLOCK_FUSE_ENABLED = True    # set False to make the blocks run operator by oper
 
 
 def block_takes(x):
-    """True where vrwkv_block_fwd may stand in for a block's operators: no autograd, a plain contiguous 16-bit GPU tensor
+    """True where vrwkv_block_fwd may stand in for a block's operators: no autograd, a plain contiguous GPU tensor
     outside every kind of transform."""
-    return (BLOCK_FUSE_ENABLED and ROW_FUSE_ENABLED and not torch.is_grad_enabled() and type(x) is torch.Tensor and x.is_cuda
-            and x.dtype in (torch.bfloat16, torch.float16) and x.dim() == 3 and x.numel() > 0 and x.is_contiguous()
+    return (not torch.is_grad_enabled() and BLOCK_FUSE_ENABLED and ROW_FUSE_ENABLED and type(x) is torch.Tensor and x.is_cuda
+            and x.dtype in _DT and x.dim() == 3 and x.numel() > 0 and x.is_contiguous()
             and not torch.is_autocast_enabled("cuda") and not _transformed())
 
 
