@@ -180,3 +180,17 @@ def test_long_sequence_tiled_equals_sequential(ops, force):
     _, _, rk, rv = biwkv.biwkv_grads_closed(f(w[64:128]), f(u[64:128]), f(k[sl]), f(v[sl]), f(gy[sl]))
     assert rel_err(f(got[2][sl]), rk) <= 1e-4 and rel_err(f(got[3][sl]), rv) <= 1e-4
     assert (got[3].sum(1) - gy.sum(1)).abs().max().item() <= 1e-4 * gy.abs().sum(1).max().item()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,T,C", [(1, 1, 1), (3, 50, 33), (2, 300, 200)])
+def test_parameter_gradients_of_the_inputs_type_are_the_rounded_fp32_sums(B, T, C, dtype):
+    from vision_rwkv_amd import bi_wkv_backward
+    torch.manual_seed(3)
+    w, u = (torch.randn(C, device="cuda") / T for _ in range(2))
+    k, v, gy = (torch.randn(B, T, C, device="cuda").to(dtype) for _ in range(3))
+    full = bi_wkv_backward(w, u, k, v, gy)
+    like = bi_wkv_backward(w, u, k, v, gy, like_inputs=True)
+    assert all(a.dtype == dtype for a in like)
+    assert all(torch.equal(a.to(dtype), b) for a, b in zip(full, like))

@@ -124,6 +124,9 @@ def _declare(lib):
     lib.vrwkv_wgrad_workspace_bytes.restype = sz
     lib.vrwkv_wgrad.argtypes = [vp, vp, vp, i, i, i, i, i, i, ll, ll, i, vp, sz, vp]
     lib.vrwkv_wgrad.restype = i
+    for name in ("rowfuse_bwd", "qshift_mix_bwd", "groupnorm_gate_bwd", "biwkv_bwd"):
+        like = getattr(lib, f"vrwkv_{name}_like")
+        like.argtypes, like.restype = getattr(lib, f"vrwkv_{name}").argtypes, i
     return lib
 
 

@@ -117,7 +117,7 @@ void launch_tiled(const BwdPlan& p, const float* w, const float* u, const IO* k,
 }
 
 template <typename IO>
-int launch(const float* w, const float* u, const void* k, const void* v, const void* gy, float* gw, float* gu,
+int launch(const float* w, const float* u, const void* k, const void* v, const void* gy, SumOut gw, SumOut gu,
            void* gk, void* gv, float* ws, int B, int T, int C, hipStream_t st) {
     const BwdPlan p = make_bwd_plan(B, T, C);
     float* agg1 = ws + p.planes;
@@ -139,7 +139,7 @@ int launch(const float* w, const float* u, const void* k, const void* v, const v
             hipLaunchKernelGGL((biwkv_bwd_serial_kernel<IO>), dim3((C + 63) / 64, B), dim3(64), 0, st, w, u,
                                kk, vv, gg, ok, ov, ws, gw_part, gu_part, B, T, C);
     }
-    hipLaunchKernelGGL(batch_sum_kernel, dim3((C + BATCH_SUM_COLS - 1) / BATCH_SUM_COLS), dim3(BATCH_SUM_THREADS), 0, st, gw_part, gw, gu_part, gu, B * p.nSC, C);
+    launch_batch_sum(gw_part, gw, gu_part, gu, B * p.nSC, C, st);
     return check_launch("biwkv_bwd");
 }
 
@@ -153,9 +153,10 @@ extern "C" size_t vrwkv_biwkv_bwd_workspace_bytes(int B, int T, int C, int io_dt
     return make_bwd_plan(B, T, C).total * sizeof(float);
 }
 
-extern "C" int vrwkv_biwkv_bwd(const float* w, const float* u, const void* k, const void* v, const void* gy,
-                               float* gw, float* gu, void* gk, void* gv, int B, int T, int C, int io_dtype,
-                               void* workspace, size_t workspace_bytes, void* hip_stream) {
+static int biwkv_bwd(const float* w, const float* u, const void* k, const void* v, const void* gy,
+                               SumOut gw, SumOut gu, void* gk, void* gv, int B, int T, int C, int io_dtype,
+                               void* workspace, size_t workspace_bytes, void* hip_stream)
+{
     int rc = validate(B, T, C, io_dtype);
     if (rc != VRWKV_OK) return rc;
     if (!w || !u || !k || !v || !gy || !gw || !gu || !gk || !gv) {
@@ -169,7 +170,8 @@ extern "C" int vrwkv_biwkv_bwd(const float* w, const float* u, const void* k, co
     }
     const size_t esz = io_dtype == VRWKV_F32 ? 4 : 2;
     if ((((uintptr_t)k | (uintptr_t)v | (uintptr_t)gy | (uintptr_t)gk | (uintptr_t)gv) & (esz - 1)) ||
-        (((uintptr_t)w | (uintptr_t)u | (uintptr_t)gw | (uintptr_t)gu | (uintptr_t)workspace) & 3)) {
+        (((uintptr_t)w | (uintptr_t)u | (uintptr_t)workspace) & 3) ||
+        (((uintptr_t)gw.p | (uintptr_t)gu.p) & (gw.dtype == VRWKV_F32 ? 3 : 1))) {
         set_error("biwkv_bwd: pointers must be aligned to their element size");
         return VRWKV_INVALID_ARG;
     }
@@ -182,3 +184,16 @@ extern "C" int vrwkv_biwkv_bwd(const float* w, const float* u, const void* k, co
     }
     return VRWKV_UNSUPPORTED_DTYPE;
 }
+
+extern "C" int vrwkv_biwkv_bwd(const float* w, const float* u, const void* k, const void* v, const void* gy,
+                               float* gw, float* gu, void* gk, void* gv, int B, int T, int C, int io_dtype,
+                               void* workspace, size_t workspace_bytes, void* hip_stream) {
+    return biwkv_bwd(w, u, k, v, gy, gw, gu, gk, gv, B, T, C, io_dtype, workspace, workspace_bytes, hip_stream);
+}
+
+extern "C" int vrwkv_biwkv_bwd_like(const float* w, const float* u, const void* k, const void* v, const void* gy,
+                               void* gw, void* gu, void* gk, void* gv, int B, int T, int C, int io_dtype,
+                               void* workspace, size_t workspace_bytes, void* hip_stream) {
+    return biwkv_bwd(w, u, k, v, gy, SumOut(gw, io_dtype), SumOut(gu, io_dtype), gk, gv, B, T, C, io_dtype, workspace, workspace_bytes, hip_stream);
+}
+

@@ -298,7 +298,7 @@ void groupnorm_gate_bwd_kernel(const YT* __restrict__ y_, const IO* __restrict__
 
 template <typename YT, typename IO>
 int launch_gn_bwd(const void* y, const void* gate, const void* w, const void* b, const void* g, void* gy, void* ggate,
-                  float* gparam, float* part, long long rows, int C, int group, float eps, hipStream_t st) {
+                  SumOut gparam, float* part, long long rows, int C, int group, float eps, hipStream_t st) {
     const long long nblk = (rows + 4 * GN_RPW - 1) / (4 * GN_RPW);
     const dim3 block(256), grid((unsigned)nblk);
     const size_t lds = (size_t)4 * 2 * C * sizeof(float);
@@ -317,8 +317,7 @@ int launch_gn_bwd(const void* y, const void* gate, const void* w, const void* b,
     }
 #undef VRWKV_GNB
     const int wide = 2 * C;                                   // gparam: (2, C) = g_weight, g_bias
-    hipLaunchKernelGGL(batch_sum_kernel, dim3((wide + BATCH_SUM_COLS - 1) / BATCH_SUM_COLS), dim3(BATCH_SUM_THREADS), 0, st, part, gparam, (const float*)nullptr,
-                       (float*)nullptr, (int)nblk, wide);
+    launch_batch_sum(part, gparam, nullptr, SumOut((float*)nullptr), (int)nblk, wide, st);
     return check_launch("groupnorm_gate_bwd");
 }
 
@@ -438,8 +437,7 @@ extern "C" int vrwkv_maa_mix_bwd(const void* x, const void* sx, const void* m, c
     }
 #undef VRWKV_MAAB
     const int wide = 5 * C;
-    hipLaunchKernelGGL(batch_sum_kernel, dim3((wide + BATCH_SUM_COLS - 1) / BATCH_SUM_COLS), dim3(BATCH_SUM_THREADS), 0, st, part, gmaa, (const float*)nullptr,
-                       (float*)nullptr, (int)nrb, wide);
+    launch_batch_sum(part, gmaa, nullptr, SumOut((float*)nullptr), (int)nrb, wide, st);
     return check_launch("maa_mix_bwd");
 }
 
@@ -448,10 +446,11 @@ extern "C" size_t vrwkv_groupnorm_gate_bwd_workspace_bytes(long long rows, int C
     return (size_t)((rows + 4 * GN_RPW - 1) / (4 * GN_RPW)) * 2 * C * sizeof(float);
 }
 
-extern "C" int vrwkv_groupnorm_gate_bwd(const void* y, const void* gate, const void* gn_weight, const void* gn_bias,
-                                        const void* gout, void* gy, void* ggate, float* gparam, long long rows, int C,
+static int groupnorm_gate_bwd(const void* y, const void* gate, const void* gn_weight, const void* gn_bias,
+                                        const void* gout, void* gy, void* ggate, SumOut gparam, long long rows, int C,
                                         int group, float eps, int y_dtype, int io_dtype,
-                                        void* workspace, size_t workspace_bytes, void* hip_stream) {
+                                        void* workspace, size_t workspace_bytes, void* hip_stream)
+{
     if (rows <= 0 || C <= 0 || group <= 0 || !y || !gate || !gn_weight || !gn_bias || !gout || !gy || !ggate || !gparam) {
         set_error("groupnorm_gate_bwd: bad arguments (rows=%lld C=%d group=%d)", rows, C, group);
         return VRWKV_INVALID_ARG;
@@ -484,3 +483,18 @@ extern "C" int vrwkv_groupnorm_gate_bwd(const void* y, const void* gate, const v
     if (y_dtype == VRWKV_F32) return launch_gn_bwd<float, __half>(y, gate, gn_weight, gn_bias, gout, gy, ggate, gparam, part, rows, C, group, eps, st);
     return launch_gn_bwd<__half, __half>(y, gate, gn_weight, gn_bias, gout, gy, ggate, gparam, part, rows, C, group, eps, st);
 }
+
+extern "C" int vrwkv_groupnorm_gate_bwd(const void* y, const void* gate, const void* gn_weight, const void* gn_bias,
+                                        const void* gout, void* gy, void* ggate, float* gparam, long long rows, int C,
+                                        int group, float eps, int y_dtype, int io_dtype,
+                                        void* workspace, size_t workspace_bytes, void* hip_stream) {
+    return groupnorm_gate_bwd(y, gate, gn_weight, gn_bias, gout, gy, ggate, gparam, rows, C, group, eps, y_dtype, io_dtype, workspace, workspace_bytes, hip_stream);
+}
+
+extern "C" int vrwkv_groupnorm_gate_bwd_like(const void* y, const void* gate, const void* gn_weight, const void* gn_bias,
+                                        const void* gout, void* gy, void* ggate, void* gparam, long long rows, int C,
+                                        int group, float eps, int y_dtype, int io_dtype,
+                                        void* workspace, size_t workspace_bytes, void* hip_stream) {
+    return groupnorm_gate_bwd(y, gate, gn_weight, gn_bias, gout, gy, ggate, SumOut(gparam, io_dtype), rows, C, group, eps, y_dtype, io_dtype, workspace, workspace_bytes, hip_stream);
+}
+

@@ -220,7 +220,7 @@ void qshift_mix_bwd_kernel(const IO* __restrict__ x_, const float* __restrict__ 
 }
 
 template <typename IO, int VEC>
-int launch_bwd(const void* x, const float* mix, const void* const* gout, void* gx, float* gmix, float* part, int n_mix,
+int launch_bwd(const void* x, const float* mix, const void* const* gout, void* gx, SumOut gmix, float* part, int n_mix,
                int B, int T, int C, int Hp, int Wp, int shift, int g, int head_dim, int n_grid, hipStream_t st) {
     const int ncv = C / VEC;
     const dim3 block(QS_CX * QS_TY);
@@ -248,13 +248,12 @@ int launch_bwd(const void* x, const float* mix, const void* const* gout, void* g
     }
     // gmix[m][c] = sum over the B * n_tchunk partial rows: the rows are (n_mix * C) wide
     const int wide = n_mix * C;
-    hipLaunchKernelGGL(batch_sum_kernel, dim3((wide + BATCH_SUM_COLS - 1) / BATCH_SUM_COLS), dim3(BATCH_SUM_THREADS), 0, st, part, gmix, (const float*)nullptr,
-                       (float*)nullptr, B * n_tchunk, wide);
+    launch_batch_sum(part, gmix, nullptr, SumOut((float*)nullptr), B * n_tchunk, wide, st);
     return check_launch("qshift_mix_bwd");
 }
 
 template <typename IO>
-int launch_bwd_io(const void* x, const float* mix, const void* const* gout, void* gx, float* gmix, float* part, int n_mix,
+int launch_bwd_io(const void* x, const float* mix, const void* const* gout, void* gx, SumOut gmix, float* part, int n_mix,
                   int B, int T, int C, int Hp, int Wp, int shift, int g, int head_dim, int n_grid, bool vec_ok, hipStream_t st) {
     // four channels per thread: 16-byte accesses of fp32, 8-byte ones of 16-bit elements (eight channels per thread
     // cost 153 registers with three mixes, three waves per SIMD: measured 10-13 % slower)
@@ -355,10 +354,11 @@ extern "C" size_t vrwkv_qshift_mix_bwd_workspace_bytes(int n_mix, int B, int T, 
     return (size_t)B * ((T + QS_TCH - 1) / QS_TCH) * n_mix * C * sizeof(float);
 }
 
-extern "C" int vrwkv_qshift_mix_bwd(const void* x, const float* mix, const void* const* gout, int n_mix,
-                                    void* gx, float* gmix, int B, int T, int C, int Hp, int Wp, int shift_pixel,
+static int qshift_mix_bwd(const void* x, const float* mix, const void* const* gout, int n_mix,
+                                    void* gx, SumOut gmix, int B, int T, int C, int Hp, int Wp, int shift_pixel,
                                     int quarter_width, int head_dim, int io_dtype,
-                                    void* workspace, size_t workspace_bytes, void* hip_stream) {
+                                    void* workspace, size_t workspace_bytes, void* hip_stream)
+{
     if (B <= 0 || T <= 0 || C <= 0 || Hp <= 0 || Wp <= 0 || n_mix < 1 || n_mix > 3 || shift_pixel < 0) {
         set_error("qshift_mix_bwd: bad sizes (B=%d T=%d C=%d Hp=%d Wp=%d n_mix=%d shift=%d)", B, T, C, Hp, Wp, n_mix, shift_pixel);
         return VRWKV_INVALID_ARG;
@@ -405,3 +405,18 @@ extern "C" int vrwkv_qshift_mix_bwd(const void* x, const float* mix, const void*
     }
     return VRWKV_UNSUPPORTED_DTYPE;
 }
+
+extern "C" int vrwkv_qshift_mix_bwd(const void* x, const float* mix, const void* const* gout, int n_mix,
+                                    void* gx, float* gmix, int B, int T, int C, int Hp, int Wp, int shift_pixel,
+                                    int quarter_width, int head_dim, int io_dtype,
+                                    void* workspace, size_t workspace_bytes, void* hip_stream) {
+    return qshift_mix_bwd(x, mix, gout, n_mix, gx, gmix, B, T, C, Hp, Wp, shift_pixel, quarter_width, head_dim, io_dtype, workspace, workspace_bytes, hip_stream);
+}
+
+extern "C" int vrwkv_qshift_mix_bwd_like(const void* x, const float* mix, const void* const* gout, int n_mix,
+                                    void* gx, void* gmix, int B, int T, int C, int Hp, int Wp, int shift_pixel,
+                                    int quarter_width, int head_dim, int io_dtype,
+                                    void* workspace, size_t workspace_bytes, void* hip_stream) {
+    return qshift_mix_bwd(x, mix, gout, n_mix, gx, SumOut(gmix, io_dtype), B, T, C, Hp, Wp, shift_pixel, quarter_width, head_dim, io_dtype, workspace, workspace_bytes, hip_stream);
+}
+

@@ -441,7 +441,7 @@ static long long bwd_sums_workgroups(long long rows, int waves, int max_wg) {
 
 template <typename IO, int V, int VPL, int POST, bool LN>
 int launch_bwd_sums_mode(const void* a, const void* other, const void* lnw, const void* lnb, const void* gamma,
-                         const void* g, void* ga, void* go, float* gparam, float* part, long long rows, int N, int pre,
+                         const void* g, void* ga, void* go, SumOut gparam, float* part, long long rows, int N, int pre,
                          float eps, hipStream_t st) {
     using Shape = BwsShape<IO, V, VPL, POST>;
     const int nwg = (int)bwd_sums_workgroups(rows, Shape::WAVES, Shape::MAX_WG);
@@ -452,14 +452,13 @@ int launch_bwd_sums_mode(const void* a, const void* other, const void* lnw, cons
                        static_cast<const IO*>(lnb), static_cast<const IO*>(gamma), static_cast<const IO*>(g),
                        static_cast<IO*>(ga), static_cast<IO*>(go), part, rows, N, eps, pre);
     const int wide = 3 * N;                                   // gparam: (3, N) = g_weight, g_bias, g_gamma
-    hipLaunchKernelGGL(batch_sum_kernel, dim3((wide + BATCH_SUM_COLS - 1) / BATCH_SUM_COLS), dim3(BATCH_SUM_THREADS), 0, st, part, gparam,
-                       (const float*)nullptr, (float*)nullptr, nwg, wide);
+    launch_batch_sum(part, gparam, nullptr, SumOut((float*)nullptr), nwg, wide, st);
     return check_launch("rowfuse_bwd");
 }
 
 template <typename IO, int V, int VPL>
 int launch_bwd_sums(const void* a, const void* other, const void* lnw, const void* lnb, const void* gamma, const void* g,
-                    void* ga, void* go, float* gparam, float* part, long long rows, int N, int pre, int post, float eps,
+                    void* ga, void* go, SumOut gparam, float* part, long long rows, int N, int pre, int post, float eps,
                     hipStream_t st) {
 #define VRWKV_SUMS(POST, LN) return launch_bwd_sums_mode<IO, V, VPL, POST, LN>(a, other, lnw, lnb, gamma, g, ga, go, gparam, part, rows, N, pre, eps, st)
     if (post == POST_SIGMOID_GATE) VRWKV_SUMS(POST_SIGMOID_GATE, true);
@@ -482,7 +481,7 @@ int launch_bwd_plain(const void* a, const void* other, const void* g, void* ga, 
 
 template <typename IO>
 int launch_bwd_io(const void* a, const void* other, const void* lnw, const void* lnb, const void* gamma, const void* g,
-                  void* ga, void* go, float* gparam, float* part, long long rows, int N, int pre, int post, float eps,
+                  void* ga, void* go, SumOut gparam, float* part, long long rows, int N, int pre, int post, float eps,
                   hipStream_t st) {
     constexpr int V = 16 / (int)sizeof(IO);
     const int per_lane = (N / V + WAVE - 1) / WAVE;
@@ -614,10 +613,11 @@ extern "C" size_t vrwkv_rowfuse_bwd_workspace_bytes(long long rows, int N) {
     return (size_t)bwd_sums_workgroups(rows, 4, BWS_MAX_PARTIAL_ROWS) * 3 * N * sizeof(float);
 }
 
-extern "C" int vrwkv_rowfuse_bwd(const void* a, const void* other, const void* ln_weight, const void* ln_bias,
-                                 const void* gamma, const void* gout, void* ga, void* gother, float* gparam,
+static int rowfuse_bwd(const void* a, const void* other, const void* ln_weight, const void* ln_bias,
+                                 const void* gamma, const void* gout, void* ga, void* gother, SumOut gparam,
                                  long long rows, int N, int pre, int post, float eps, int io_dtype,
-                                 void* workspace, size_t workspace_bytes, void* hip_stream) {
+                                 void* workspace, size_t workspace_bytes, void* hip_stream)
+{
     if (rows <= 0 || N <= 0 || pre < 0 || pre > 1 || post < 0 || post > 2) {
         set_error("rowfuse_bwd: bad arguments (rows=%lld N=%d pre=%d post=%d)", rows, N, pre, post);
         return VRWKV_INVALID_ARG;
@@ -660,3 +660,18 @@ extern "C" int vrwkv_rowfuse_bwd(const void* a, const void* other, const void* l
     }
     return VRWKV_UNSUPPORTED_DTYPE;
 }
+
+extern "C" int vrwkv_rowfuse_bwd(const void* a, const void* other, const void* ln_weight, const void* ln_bias,
+                                 const void* gamma, const void* gout, void* ga, void* gother, float* gparam,
+                                 long long rows, int N, int pre, int post, float eps, int io_dtype,
+                                 void* workspace, size_t workspace_bytes, void* hip_stream) {
+    return rowfuse_bwd(a, other, ln_weight, ln_bias, gamma, gout, ga, gother, gparam, rows, N, pre, post, eps, io_dtype, workspace, workspace_bytes, hip_stream);
+}
+
+extern "C" int vrwkv_rowfuse_bwd_like(const void* a, const void* other, const void* ln_weight, const void* ln_bias,
+                                 const void* gamma, const void* gout, void* ga, void* gother, void* gparam,
+                                 long long rows, int N, int pre, int post, float eps, int io_dtype,
+                                 void* workspace, size_t workspace_bytes, void* hip_stream) {
+    return rowfuse_bwd(a, other, ln_weight, ln_bias, gamma, gout, ga, gother, SumOut(gparam, io_dtype), rows, N, pre, post, eps, io_dtype, workspace, workspace_bytes, hip_stream);
+}
+

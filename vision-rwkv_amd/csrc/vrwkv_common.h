@@ -192,8 +192,10 @@ __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcp
 // (512 partial rows in one round of loads); the slices are added in a fixed order (deterministic).
 // Grid: ceil(C / BATCH_SUM_COLS), block: BATCH_SUM_THREADS.
 constexpr int BATCH_SUM_THREADS = 1024, BATCH_SUM_COLS = 32, BATCH_SUM_SLICES = BATCH_SUM_THREADS / BATCH_SUM_COLS;
-__global__ __launch_bounds__(1024) inline void batch_sum_kernel(const float* __restrict__ part0, float* __restrict__ out0,
-                                                                const float* __restrict__ part1, float* __restrict__ out1,
+// The sums leave as O: fp32, or rounded to the type of the parameter they are the gradient of (a cast kernel per gradient less).
+template <typename O>
+__global__ __launch_bounds__(1024) inline void batch_sum_kernel(const float* __restrict__ part0, O* __restrict__ out0,
+                                                                const float* __restrict__ part1, O* __restrict__ out1,
                                                                 int B, int C) {
     constexpr int NS = BATCH_SUM_SLICES, U = 16;
     __shared__ float red[2][NS][BATCH_SUM_COLS];
@@ -224,9 +226,24 @@ __global__ __launch_bounds__(1024) inline void batch_sum_kernel(const float* __r
         float t0 = 0.f, t1 = 0.f;
 #pragma unroll
         for (int i = 0; i < NS; ++i) { t0 += red[0][i][cl]; t1 += red[1][i][cl]; }
-        out0[c] = t0;
-        if (part1) out1[c] = t1;
+        out0[c] = from_f32<O>(t0);
+        if (part1) out1[c] = from_f32<O>(t1);
     }
+}
+// Where the sums go, and as what.
+struct SumOut {
+    void* p;
+    int dtype;
+    SumOut(float* q) : p(q), dtype(VRWKV_F32) {}
+    SumOut(void* q, int dt) : p(q), dtype(dt) {}
+    explicit operator bool() const { return p != nullptr; }
+};
+inline void launch_batch_sum(const float* part0, SumOut out0, const float* part1, SumOut out1, int B, int C, hipStream_t st) {
+    const dim3 grid((C + BATCH_SUM_COLS - 1) / BATCH_SUM_COLS), block(BATCH_SUM_THREADS);
+    if (out0.dtype == VRWKV_F32) hipLaunchKernelGGL((batch_sum_kernel<float>), grid, block, 0, st, part0, (float*)out0.p, part1, (float*)out1.p, B, C);
+    else if (out0.dtype == VRWKV_BF16)
+        hipLaunchKernelGGL((batch_sum_kernel<__hip_bfloat16>), grid, block, 0, st, part0, (__hip_bfloat16*)out0.p, part1, (__hip_bfloat16*)out1.p, B, C);
+    else hipLaunchKernelGGL((batch_sum_kernel<__half>), grid, block, 0, st, part0, (__half*)out0.p, part1, (__half*)out1.p, B, C);
 }
 #endif
 

@@ -131,8 +131,7 @@ int launch_all(const void* r, const void* k, const void* v, const void* w, const
         if (p.w16) hipLaunchKernelGGL((round_kernel<WT>), rg, block, 0, st, A.pw, static_cast<WT*>(gw), p.n);
     }
     // torch.sum(gu, 0), vrwkv6.py:69
-    hipLaunchKernelGGL(batch_sum_kernel, dim3((C + BATCH_SUM_COLS - 1) / BATCH_SUM_COLS), dim3(BATCH_SUM_THREADS), 0, st, A.gu_part, gu,
-                       (const float*)nullptr, (float*)nullptr, part_rows, C);
+    launch_batch_sum(A.gu_part, gu, nullptr, SumOut((float*)nullptr), part_rows, C, st);
     return check_launch("wkv6_bwd");
 }
 

@@ -39,6 +39,21 @@ def _stream_ptr(device):
     return torch._C._cuda_getCurrentRawStream(device.index)
 
 
+class _on:
+    """torch.cuda.device for a tensor's device, without the look-up of device arguments of other kinds."""
+    __slots__ = ("index", "previous")
+
+    def __init__(self, device):
+        self.index = device.index
+
+    def __enter__(self):
+        self.previous = torch._C._cuda_exchangeDevice(self.index)
+
+    def __exit__(self, *exc):
+        torch._C._cuda_maybeExchangeDevice(self.previous)
+        return False
+
+
 def bi_wkv_forward(w, u, k, v, out=None, gate=None):
     """Extension-level entry (bi_wkv.cpp:23-33): w,u (C,) fp32; k,v (B,T,C) of one dtype
     (fp32, bf16 or fp16); returns y (B,T,C) of that dtype.  State and arithmetic are fp32.
@@ -64,7 +79,7 @@ def bi_wkv_forward(w, u, k, v, out=None, gate=None):
         return y
     ws_bytes = L.vrwkv_biwkv_fwd_workspace_bytes(B, T, C, dt)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=k.device) if ws_bytes else None
-    with torch.cuda.device(k.device):
+    with _on(k.device):
         tail = (B, T, C, dt, ws.data_ptr() if ws is not None else None, ws_bytes, _stream_ptr(k.device))
         if gate is None:
             _lib.check(L.vrwkv_biwkv_fwd(w.data_ptr(), u.data_ptr(), k.data_ptr(), v.data_ptr(), y.data_ptr(), *tail))
@@ -74,10 +89,11 @@ def bi_wkv_forward(w, u, k, v, out=None, gate=None):
     return y
 
 
-def bi_wkv_backward(w, u, k, v, gy, out=None):
+def bi_wkv_backward(w, u, k, v, gy, out=None, like_inputs=False):
     """Extension-level entry (bi_wkv.cpp:35-47): w,u (C,) fp32; k,v,gy (B,T,C) of one dtype;
     returns [gw, gu, gk, gv] with gw, gu (C,) fp32 summed over batch and tokens and gk, gv of the
-    dtype of k.  out: caller-allocated (gw, gu, gk, gv)."""
+    dtype of k.  out: caller-allocated (gw, gu, gk, gv).  like_inputs: gw, gu of the dtype of k as well, rounded from the
+    fp32 sums by the kernel."""
     for t, n in ((w, "w"), (u, "u"), (k, "k"), (v, "v"), (gy, "gy")):
         _check_input(t, n)
     if k.dim() != 3 or v.shape != k.shape or gy.shape != k.shape:
@@ -90,8 +106,8 @@ def bi_wkv_backward(w, u, k, v, gy, out=None):
     L = _lib.lib()
     dt = _DT[k.dtype]
     if out is None:
-        gw = torch.empty(C, dtype=torch.float32, device=k.device)
-        gu = torch.empty(C, dtype=torch.float32, device=k.device)
+        gw = torch.empty(C, dtype=k.dtype if like_inputs else torch.float32, device=k.device)
+        gu = torch.empty_like(gw)
         gk = torch.empty_like(k)
         gv = torch.empty_like(k)
     else:
@@ -101,10 +117,11 @@ def bi_wkv_backward(w, u, k, v, gy, out=None):
         return [gw.zero_(), gu.zero_(), gk, gv]
     ws_bytes = L.vrwkv_biwkv_bwd_workspace_bytes(B, T, C, dt)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=k.device)
-    with torch.cuda.device(k.device):
-        _lib.check(L.vrwkv_biwkv_bwd(w.data_ptr(), u.data_ptr(), k.data_ptr(), v.data_ptr(), gy.data_ptr(),
-                                     gw.data_ptr(), gu.data_ptr(), gk.data_ptr(), gv.data_ptr(),
-                                     B, T, C, dt, ws.data_ptr(), ws_bytes, _stream_ptr(k.device)))
+    with _on(k.device):
+        fn = L.vrwkv_biwkv_bwd_like if like_inputs and out is None else L.vrwkv_biwkv_bwd
+        _lib.check(fn(w.data_ptr(), u.data_ptr(), k.data_ptr(), v.data_ptr(), gy.data_ptr(),
+                      gw.data_ptr(), gu.data_ptr(), gk.data_ptr(), gv.data_ptr(),
+                      B, T, C, dt, ws.data_ptr(), ws_bytes, _stream_ptr(k.device)))
     return [gw, gu, gk, gv]
 
 
@@ -132,10 +149,8 @@ class WKV(torch.autograd.Function):
         wf, uf, k, v = ctx.saved_tensors
         out_dtype = ctx.out_dtype
         if k.dtype == out_dtype and v.dtype == out_dtype and out_dtype != torch.float32:
-            gw, gu, gk, gv = bi_wkv_backward(wf, uf, k.contiguous(), v.contiguous(), gy.to(out_dtype).contiguous())
-        else:
-            gw, gu, gk, gv = bi_wkv_backward(wf, uf, k.float().contiguous(), v.float().contiguous(),
-                                             gy.float().contiguous())
+            return tuple(bi_wkv_backward(wf, uf, k.contiguous(), v.contiguous(), gy.to(out_dtype).contiguous(), like_inputs=True))
+        gw, gu, gk, gv = bi_wkv_backward(wf, uf, k.float().contiguous(), v.float().contiguous(), gy.float().contiguous())
         if out_dtype == torch.float32:
             return (gw, gu, gk, gv)
         gwu = torch.stack((gw, gu)).to(out_dtype)           # one cast for both parameter gradients
@@ -194,7 +209,7 @@ def wkv6_forward(B, T, C, H, r, k, v, w, u, w_is_ew=False, out=None, whole=False
         return y
     ws_bytes = 0 if whole else L.vrwkv_wkv6_fwd_workspace_bytes(B, T, C, H)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=r.device) if ws_bytes else None
-    with torch.cuda.device(r.device):
+    with _on(r.device):
         _lib.check(L.vrwkv_wkv6_fwd(r.data_ptr(), k.data_ptr(), v.data_ptr(), w.data_ptr(), uf.data_ptr(),
                                     y.data_ptr(), B, T, C, H, _DT[r.dtype], _DT[w.dtype], 1 if w_is_ew else 0,
                                     ws.data_ptr() if ws is not None else None, ws_bytes,
@@ -231,7 +246,7 @@ def wkv6_backward(B, T, C, H, r, k, v, w, u, gy, w_is_ew=False, out=None, like_i
     else:
         fn, ws_bytes = L.vrwkv_wkv6_bwd, L.vrwkv_wkv6_bwd_workspace_bytes(B, T, C, H)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=r.device)
-    with torch.cuda.device(r.device):
+    with _on(r.device):
         _lib.check(fn(r.data_ptr(), k.data_ptr(), v.data_ptr(), w.data_ptr(), uf.data_ptr(),
                                     gyf.data_ptr(), gr.data_ptr(), gk.data_ptr(), gv.data_ptr(), gw.data_ptr(),
                                     gu.data_ptr(), B, T, C, H, _DT[r.dtype], _DT[w.dtype], 1 if w_is_ew else 0,
@@ -339,7 +354,7 @@ def q_shift_mix(x, mixes, shift_pixel=1, gamma=1 / 4, patch_resolution=None, hea
         return outs
     ptrs = (ctypes.c_void_p * len(outs))(*[o.data_ptr() for o in outs])
     g = head_dim // 4 if head_dim else int(C * gamma)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         _lib.check(_lib.lib().vrwkv_qshift_mix(x.data_ptr(), mix.data_ptr(), ptrs, len(outs), B, T, C, Hp, Wp,
                                                shift_pixel, g, head_dim, _DT[x.dtype], _stream_ptr(x.device)))
     return outs
@@ -392,16 +407,16 @@ class _RowFuse(torch.autograd.Function):
         gparam = ws = None
         ws_bytes = 0
         if sums:
-            gparam = torch.empty(3, N, dtype=torch.float32, device=a.device)
+            gparam = torch.empty(3, N, dtype=a.dtype, device=a.device)    # rounded once from the fp32 sums
             ws_bytes = L.vrwkv_rowfuse_bwd_workspace_bytes(rows, N)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device)
         ptr = lambda t: t.data_ptr() if t is not None else None
-        with torch.cuda.device(a.device):
-            _lib.check(L.vrwkv_rowfuse_bwd(a.data_ptr(), ptr(other), ptr(ln_weight), ptr(ln_bias), ptr(gamma),
+        with _on(a.device):
+            _lib.check(L.vrwkv_rowfuse_bwd_like(a.data_ptr(), ptr(other), ptr(ln_weight), ptr(ln_bias), ptr(gamma),
                                            gout.data_ptr(), ga.data_ptr(), ptr(go), ptr(gparam), rows, N, pre, post,
                                            float(eps), _DT[a.dtype], ptr(ws), ws_bytes, _stream_ptr(a.device)))
         g_other = go if post == POST_SIGMOID_GATE else (gout if post == POST_RESIDUAL else None)
-        gp = gparam.to(a.dtype) if sums else None            # one cast for the three parameter gradients
+        gp = gparam
         g_w = gp[0] if ln_weight is not None else None
         g_b = gp[1] if ln_bias is not None else None
         g_g = gp[2] if (gamma is not None and post == POST_RESIDUAL) else None
@@ -412,7 +427,7 @@ def _row_fuse_launch(a, other, ln_weight, ln_bias, gamma, pre, post, eps):
     out = torch.empty_like(a)
     N = a.shape[-1]
     ptr = lambda t: t.data_ptr() if t is not None else None
-    with torch.cuda.device(a.device):
+    with _on(a.device):
         _lib.check(_lib.lib().vrwkv_rowfuse(a.data_ptr(), ptr(other), ptr(ln_weight), ptr(ln_bias), ptr(gamma), out.data_ptr(),
                                             a.numel() // N, N, pre, post, float(eps), _DT[a.dtype], _stream_ptr(a.device)))
     return out
@@ -480,7 +495,7 @@ class _MaaMix(torch.autograd.Function):
         ws_bytes = L.vrwkv_maa_mix_bwd_workspace_bytes(rows, C)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
         ptrs = (ctypes.c_void_p * 5)(*[g.data_ptr() for g in gs])
-        with torch.cuda.device(x.device):
+        with _on(x.device):
             _lib.check(L.vrwkv_maa_mix_bwd(x.data_ptr(), sx.data_ptr(), m.data_ptr(), table.data_ptr(), ptrs, gx.data_ptr(),
                                            gsx.data_ptr(), gm.data_ptr(), gmaa.data_ptr(), rows, C, _DT[x.dtype],
                                            ws.data_ptr(), ws_bytes, _stream_ptr(x.device)))
@@ -491,7 +506,7 @@ def _maa_mix_launch(x, sx, m, table):
     C = x.shape[-1]
     outs = [torch.empty_like(x) for _ in range(5)]
     ptrs = (ctypes.c_void_p * 5)(*[o.data_ptr() for o in outs])
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         _lib.check(_lib.lib().vrwkv_maa_mix(x.data_ptr(), sx.data_ptr(), m.data_ptr(), table.data_ptr(), ptrs,
                                             x.numel() // C, C, _DT[x.dtype], _stream_ptr(x.device)))
     return outs
@@ -514,7 +529,7 @@ def maa_mix(x, sx, m, maas, maa_table=None):
     if not _vec_ok(xc, sxc, mc):
         return maa_mix_tensor_ops(x, sx, m, maas)
     if need_grad:
-        table = torch.stack([a.reshape(-1).float() for a in maas])      # differentiable: the vectors' gradients flow through it
+        table = torch.stack([a.reshape(-1) for a in maas]).float()      # differentiable; one cast for the five vectors
         return list(_MaaMix.apply(xc, sxc, mc, table))
     table = maa_table if maa_table is not None else stack_mixes(maas, x.device)
     if tuple(table.shape) != (5, C) or table.dtype != torch.float32 or not table.is_contiguous():
@@ -555,21 +570,21 @@ class _GroupNormGate(torch.autograd.Function):
         rows = y.numel() // C
         gout = gout.to(gate.dtype).contiguous()
         gy, gg = torch.empty_like(y), torch.empty_like(gate)
-        gparam = torch.empty(2, C, dtype=torch.float32, device=y.device)
+        gparam = torch.empty(2, C, dtype=gate.dtype, device=y.device)
         L = _lib.lib()
         ws_bytes = L.vrwkv_groupnorm_gate_bwd_workspace_bytes(rows, C)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=y.device)
-        with torch.cuda.device(y.device):
-            _lib.check(L.vrwkv_groupnorm_gate_bwd(y.data_ptr(), gate.data_ptr(), w.data_ptr(), b.data_ptr(), gout.data_ptr(),
+        with _on(y.device):
+            _lib.check(L.vrwkv_groupnorm_gate_bwd_like(y.data_ptr(), gate.data_ptr(), w.data_ptr(), b.data_ptr(), gout.data_ptr(),
                                                   gy.data_ptr(), gg.data_ptr(), gparam.data_ptr(), rows, C, group, float(eps),
                                                   _DT[y.dtype], _DT[gate.dtype], ws.data_ptr(), ws_bytes, _stream_ptr(y.device)))
-        return gy, gg, gparam[0].to(w.dtype), gparam[1].to(b.dtype), None, None
+        return gy, gg, gparam[0], gparam[1], None, None
 
 
 def _groupnorm_gate_launch(y, gate, w, b, group, eps):
     C = y.shape[-1]
     out = torch.empty_like(gate)
-    with torch.cuda.device(y.device):
+    with _on(y.device):
         _lib.check(_lib.lib().vrwkv_groupnorm_gate(y.data_ptr(), gate.data_ptr(), w.data_ptr(), b.data_ptr(), out.data_ptr(),
                                                    y.numel() // C, C, group, float(eps), _DT[y.dtype], _DT[gate.dtype],
                                                    _stream_ptr(y.device)))
@@ -603,13 +618,14 @@ def groupnorm_gate(y, gate, gn_weight, gn_bias, n_groups, eps=1e-5):
 
 class _QShiftMix(torch.autograd.Function):
     """q_shift + mix lerps with a hand-written backward (vrwkv_qshift_mix / vrwkv_qshift_mix_bwd); the mix vectors
-    enter as one (n_mix, C) fp32 table, so whatever produced them (parameters, 1 - parameter, ...) is differentiated
+    enter as one (n_mix, C) table of their own type, so whatever produced them (parameters, 1 - parameter, ...) is differentiated
     by autograd outside."""
 
     @staticmethod
     def forward(ctx, x, table, shift_pixel, gamma, Hp, Wp, head_dim):
         x = x.contiguous()
-        table = table.contiguous()
+        ctx.table_dtype = table.dtype
+        table = table.float().contiguous()
         ctx.save_for_backward(x, table)
         ctx.meta = (shift_pixel, gamma, Hp, Wp, head_dim)
         outs = q_shift_mix(x, [None] * table.shape[0], shift_pixel, gamma, (Hp, Wp), head_dim, mix_table=table)
@@ -623,17 +639,19 @@ class _QShiftMix(torch.autograd.Function):
         n_mix = table.shape[0]
         gs = [g.to(x.dtype).contiguous() for g in gouts]
         gx = torch.empty_like(x)
-        gmix = torch.empty_like(table)
+        like = ctx.table_dtype == x.dtype                        # the table's gradient rounded by the kernel, or cast below
+        gmix = torch.empty_like(table, dtype=x.dtype if like else torch.float32)
         L = _lib.lib()
         ws_bytes = L.vrwkv_qshift_mix_bwd_workspace_bytes(n_mix, B, T, C)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
         ptrs = (ctypes.c_void_p * n_mix)(*[g.data_ptr() for g in gs])
         g = head_dim // 4 if head_dim else int(C * gamma)
-        with torch.cuda.device(x.device):
-            _lib.check(L.vrwkv_qshift_mix_bwd(x.data_ptr(), table.data_ptr(), ptrs, n_mix, gx.data_ptr(), gmix.data_ptr(),
-                                              B, T, C, Hp, Wp, shift_pixel, g, head_dim, _DT[x.dtype],
-                                              ws.data_ptr(), ws_bytes, _stream_ptr(x.device)))
-        return gx, gmix, None, None, None, None, None
+        with _on(x.device):
+            fn = L.vrwkv_qshift_mix_bwd_like if like else L.vrwkv_qshift_mix_bwd
+            _lib.check(fn(x.data_ptr(), table.data_ptr(), ptrs, n_mix, gx.data_ptr(), gmix.data_ptr(),
+                          B, T, C, Hp, Wp, shift_pixel, g, head_dim, _DT[x.dtype],
+                          ws.data_ptr(), ws_bytes, _stream_ptr(x.device)))
+        return gx, gmix.to(ctx.table_dtype), None, None, None, None, None
 
 
 def q_shift_mix_autograd(x, mixes, shift_pixel=1, gamma=1 / 4, patch_resolution=None, head_dim=0):
@@ -642,9 +660,10 @@ def q_shift_mix_autograd(x, mixes, shift_pixel=1, gamma=1 / 4, patch_resolution=
     _check_input(x, "x")
     if x.dim() != 3 or x.dtype not in _DT:
         raise RuntimeError("x must be (B,T,C) float32 / bfloat16 / float16")
-    table = torch.stack([m.reshape(-1) for m in mixes]).float()       # one cast, differentiated as one
+    table = torch.stack([m.reshape(-1) for m in mixes])
     Hp, Wp = patch_resolution
     if not _equal_quarters(x.shape[-1], gamma, head_dim):
+        table = table.float()
         xx = q_shift(x, shift_pixel, gamma, patch_resolution)
         return [(x.float() * m + xx.float() * (1 - m)).to(x.dtype) for m in table]
     return list(_QShiftMix.apply(x, table, shift_pixel, gamma, Hp, Wp, head_dim))
@@ -673,7 +692,7 @@ def _table_resize_launch(table, src, dst, adjoint):
     table = table.contiguous()
     n, C = (src if adjoint else dst), table.shape[-1]
     out = torch.empty((1, n[0] * n[1], C), dtype=table.dtype, device=table.device)
-    with torch.cuda.device(table.device):
+    with _on(table.device):
         _lib.check(_lib.lib().vrwkv_pos_resize(table.data_ptr(), out.data_ptr(), src[0], src[1], dst[0], dst[1], C,
                                                1 if adjoint else 0, _DT[table.dtype], _stream_ptr(table.device)))
     return out
@@ -736,7 +755,7 @@ def block_forward(x, tensors, **scalars):
     a.workspace_bytes = L.vrwkv_block_fwd_workspace_bytes(B, T, C, a.hidden, a.heads, a.dtype)
     ws = torch.empty(a.workspace_bytes, dtype=torch.uint8, device=x.device)
     a.workspace = ws.data_ptr()
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         _lib.check(L.vrwkv_block_fwd(ctypes.byref(a), _stream_ptr(x.device)))
     return out
 
@@ -764,7 +783,7 @@ def weight_grad(g, x):
     ws_bytes = L.vrwkv_wgrad_workspace_bytes(n, M, O, I)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=g.device)
     gs, xs = g3.stride(), x3.stride()
-    with torch.cuda.device(g.device):
+    with _on(g.device):
         _lib.check(L.vrwkv_wgrad(g3.data_ptr(), x3.data_ptr(), out.data_ptr(), n, M, O, I, gs[1], xs[1], gs[0], xs[0],
                                  _DT[g.dtype], ws.data_ptr(), ws_bytes, _stream_ptr(g.device)))
     return out
