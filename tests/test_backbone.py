@@ -627,7 +627,7 @@ def _small_backbone(kind, C, dtype, key_norm, post_norm, cls, hw):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tile", [0, 1, 2, 4])
+@pytest.mark.parametrize("tile", [0, 1, 2, 4, 8])
 @pytest.mark.parametrize("kind,C,dtype,key_norm,post_norm,cls,hw,batch", [
     ("v4", 192, torch.bfloat16, False, False, False, (14, 14), 1), ("v4", 64, torch.float16, True, False, False, (1, 3), 24),
     ("v4", 416, torch.bfloat16, False, True, False, (7, 9), 3), ("v4", 256, torch.float16, True, True, False, (16, 15), 2),

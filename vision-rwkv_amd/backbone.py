@@ -184,18 +184,21 @@ def _layer_norm(ln, x):
     return row_fuse(x, None, ln.weight, ln.bias, None, PRE_NONE, POST_NONE, ln.eps)
 
 
-# Multiplications per (C, C) projection up to which a block runs as one native call (vrwkv_block_fwd).  Twelve bf16 blocks,
-# operator by operator -> native, eager / replayed as a graph (GPU time alone), in us: 196 x 192 4037 -> 781 / 991 -> 499, 3136 x 384
-# 4000 -> 1425 / 1426 -> 1408, 784 x 768 3995 -> 1449 / 1426 -> 1428; VRWKV6 196 x 192 6496 -> 1107 / 1536 -> 900, 784 x 768
-# 6505 -> 2014 / 2346 -> 1990.  Beyond, the library's larger tiles win on the GPU (1568 x 768 1619 / 2023) while the calls
-# still take longer than the GPU work; the line is where neither loses.
-# fp32: 196 x 192 4773 -> 747, 3136 x 384 3740 -> 2485 / 2448 -> 2463, 392 x 768 3697 -> 1807 / 1920 -> 1792, but 784 x 768 2307 / 2535 and
-# 1568 x 768 3415 / 3919 on the GPU; from 3136 x 768 on (7064 / 6371, 6272 x 768 12392 / 11386) the library is behind again.
-NATIVE_BLOCK_WORK = 470_000_000
+# Multiplications per (C, C) projection up to which a block runs as one native call (vrwkv_block_fwd).  Twelve bf16 blocks of
+# tokens x channels, operator by operator -> native, eager | replayed as a graph (GPU time alone), in us:
+#   VRWKV   196 x 192 4037 -> 781 | 991 -> 499      3136 x 384 3594 -> 1273 | 1427 -> 1257    784 x 768 3602 -> 1377 | 1428 -> 1360
+#           3136 x 768 3623 -> 2115 | 1992 -> 2115   6272 x 768 3714 -> 3121 | 3163 -> 3062   12544 x 768 5077 -> 5546
+#           1568 x 1024 3673 -> 2296 | 1977 -> 2282  6272 x 1024 3823 -> 4252
+#   VRWKV6  196 x 192 6496 -> 1107 | 1536 -> 900    784 x 768 6055 -> 1950 | 2287 -> 1920    12544 x 768 7919 -> 7880 | 7897 -> 7854
+# The host sets the pace of the operators up to about 4 (7) ms; the GPU work alone is a few percent behind the library's larger
+# tiles from about 1000 tokens of 768 or more channels on, so the line is where the eager call stops gaining.
+NATIVE_BLOCK_WORK, NATIVE_BLOCK_WORK_V6 = 3_800_000_000, 7_500_000_000
+# fp32: 196 x 192 4773 -> 747, 3136 x 384 3740 -> 2485 | 2448 -> 2463, 392 x 768 3697 -> 1807 | 1920 -> 1792, but 784 x 768 2307 / 2535
+# and 1568 x 768 3769 -> 3937 | 3415 -> 3919; from 3136 x 768 on (7064 / 6371, 6272 x 768 12392 / 11386) the library is behind again.
 NATIVE_BLOCK_WORK_FP32 = (420_000_000, 1_700_000_000)                      # up to the first, and from the second on
 
 
-def _native_size(x, hidden):
+def _native_size(x, hidden, v6):
     """The rule above, and 32-bit byte offsets inside every token matrix of the call."""
     M, C = x.shape[0] * x.shape[1], x.shape[2]
     if M * max(C, hidden, 160) * x.element_size() >= 1 << 30:
@@ -203,7 +206,7 @@ def _native_size(x, hidden):
     if x.dtype == torch.float32:
         lo, hi = NATIVE_BLOCK_WORK_FP32
         return not lo < M * C * C < hi
-    return M * C * C <= NATIVE_BLOCK_WORK
+    return M * C * C <= (NATIVE_BLOCK_WORK_V6 if v6 else NATIVE_BLOCK_WORK)
 
 
 def _as_built(module, kind):
@@ -219,7 +222,7 @@ def _block_weights(block, att, ffn, x):
     key = fm["key"]
     hidden = key._parameters["weight"].shape[0] if type(key) is nn.Linear else 0
     if not (C % 32 == 0 and hidden % 32 == 0 and 0 < hidden <= 4096 and att.fused_shift and ffn.fused_shift
-            and att.shift_pixel == ffn.shift_pixel and _native_size(x, hidden)):
+            and att.shift_pixel == ffn.shift_pixel and _native_size(x, hidden, "gate" in am)):
         return None
     w, num = {}, dict(hidden=hidden, shift_pixel=att.shift_pixel, post_norm=int(block.post_norm))
     for name, lin, shape in (("key", am["key"], (C, C)), ("value", am["value"], (C, C)), ("receptance", am["receptance"], (C, C)),

@@ -6,7 +6,7 @@
 // library picks tiles of 192 x 256 for 196 x 192 results (13 us a product).  Issued from here a VRWKV block is 9 launches:
 //   LN | shift + mixes | key, value, receptance | Bi-WKV with gate | output + residual
 //   LN | shift + mixes | key with relu^2, receptance | value, gate, residual
-#include "vrwkv_common.h"
+#include "gemm_tile.h"
 #include <algorithm>
 #include <type_traits>
 
@@ -33,10 +33,8 @@ struct LinGroup {
     int n, M;
 };
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+using gemm::f32x4;
+using gemm::u32x4;
 // one 16-byte fragment of either operand: 32 k in 16 bits; in fp32 16 k as four products of 4, lane group g taking the k
 // 4 g .. of both operands
 template <typename IO> __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
@@ -45,10 +43,39 @@ template <typename IO> __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f
 #pragma unroll
         for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[e], fb[e], c, 0, 0, 0);
         return c;
-    } else if constexpr (std::is_same<IO, __hip_bfloat16>::value)
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+    } else {
+        return gemm::mfma16<IO>(a, b, c);
+    }
+}
+
+// epilogue of four neighbouring channels n .. of token m
+template <typename IO>
+__device__ __forceinline__ void finish(const LinProblem& P, int m, int n, f32x4 s) {
+    const IO *gate = (const IO*)P.gate, *vec = (const IO*)P.vec, *res = (const IO*)P.res;
+    float v[4], x[4];
+    const size_t off = (size_t)m * P.N + n;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v[e] = s[e];
+        if (P.epi & EPI_RELU_SQ) { const float r = fmaxf(v[e], 0.f); v[e] = r * r; }
+        if (P.epi & EPI_TANH) v[e] = tanhf(v[e]);
+    }
+    if (gate) {
+        load_vec<IO, 4>(gate + off, x);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] *= fast_rcp(1.f + fast_exp2(-LOG2E * x[e]));
+    }
+    if (vec) {
+        load_vec<IO, 4>(vec + n, x);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = P.epi & EPI_ADD_VEC ? v[e] + x[e] : v[e] * x[e];
+    }
+    if (res) {
+        load_vec<IO, 4>(res + off, x);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += x[e];
+    }
+    store_vec<IO, 4>((IO*)P.out + off, v);
 }
 
 template <typename IO, int MT>
@@ -107,58 +134,71 @@ void linear_group_kernel(LinGroup G)
 #pragma unroll
         for (int j = 0; j < MT; ++j) red[w4][i * MT + j][lane] = acc[i][j];
     __syncthreads();
-    const IO *gate = (const IO*)P.gate, *vec = (const IO*)P.vec, *res = (const IO*)P.res;
-    IO* out = (IO*)P.out;
     for (int t = w4; t < MT * MT; t += 4) {
         const int m = m0 + 16 * (t / MT) + c16, n = n0 + 16 * (t % MT) + 4 * g4;
         if (m >= M || n >= N) continue;
-        const f32x4 s = (red[0][t][lane] + red[1][t][lane]) + (red[2][t][lane] + red[3][t][lane]);
-        float v[4], x[4];
-        const size_t off = (size_t)m * N + n;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] = s[e];
-            if (P.epi & EPI_RELU_SQ) { const float r = fmaxf(v[e], 0.f); v[e] = r * r; }
-            if (P.epi & EPI_TANH) v[e] = tanhf(v[e]);
-        }
-        if (gate) {
-            load_vec<IO, 4>(gate + off, x);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] *= fast_rcp(1.f + fast_exp2(-LOG2E * x[e]));
-        }
-        if (vec) {
-            load_vec<IO, 4>(vec + n, x);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = P.epi & EPI_ADD_VEC ? v[e] + x[e] : v[e] * x[e];
-        }
-        if (res) {
-            load_vec<IO, 4>(res + off, x);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] += x[e];
-        }
-        store_vec<IO, 4>(out + off, v);
+        finish<IO>(P, m, n, (red[0][t][lane] + red[1][t][lane]) + (red[2][t][lane] + red[3][t][lane]));
     }
 }
 
-template <int MT>
-void launch_group(LinGroup& G, int dtype, hipStream_t st) {
+// The same with 128 x 128 tiles staged in LDS, for 16-bit calls that fill enough compute units with them: 64 x 64 tiles read
+// every operand piece twice as often straight from the L2s (12544 x 768, twelve blocks: 9957 us, with these 5472 us).
+template <typename IO>
+__global__ __launch_bounds__(256, 2)
+void linear_tile_kernel(LinGroup G)
+{
+    __shared__ __attribute__((aligned(16))) char lds[gemm::Stage<false>::LDS];
+    const int lane = threadIdx.x & 63, g4 = lane >> 4, c16 = lane & 15, w4 = threadIdx.x >> 6;
+    // a contiguous eighth of the tiles per XCD: tiles of the same tokens share an L2
+    int id = blockIdx.x;
+    const int whole = gridDim.x / 8 * 8;
+    if (id < whole) id = (id & 7) * (whole / 8) + (id >> 3);
+    int q = 0;
+    while (q + 1 < G.n && id >= G.p[q + 1].tile0) ++q;
+    const LinProblem& P = G.p[q];
+    const int nt = (P.N + gemm::TILE - 1) / gemm::TILE, tile = id - P.tile0;
+    const int m0 = tile / nt * gemm::TILE, n0 = tile % nt * gemm::TILE;
+    gemm::f32x4 acc[4][4];
+    gemm::tile_product<IO, false>(lds, (const IO*)P.w, (const IO*)P.a, n0, m0, P.N, G.M, P.K, P.K, P.lda, 0, (P.K + 63) / 64, acc);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int n = n0 + 64 * (w4 & 1) + 16 * i + 4 * g4, m = m0 + 64 * (w4 >> 1) + 16 * j + c16;
+            if (m < G.M && n < P.N) finish<IO>(P, m, n, acc[i][j]);
+        }
+}
+
+int number_tiles(LinGroup& G, int side) {
     int tiles = 0;
     for (int i = 0; i < G.n; ++i) {
         G.p[i].tile0 = tiles;
-        tiles += ((G.M + 16 * MT - 1) / (16 * MT)) * ((G.p[i].N + 16 * MT - 1) / (16 * MT));
+        tiles += ((G.M + side - 1) / side) * ((G.p[i].N + side - 1) / side);
     }
-    if (dtype == VRWKV_BF16) hipLaunchKernelGGL((linear_group_kernel<__hip_bfloat16, MT>), dim3(tiles), dim3(256), 0, st, G);
+    return tiles;
+}
+template <int MT>
+void launch_group(LinGroup& G, int dtype, hipStream_t st) {
+    const int tiles = number_tiles(G, 16 * MT);
+    if constexpr (MT == 8) {
+        if (dtype == VRWKV_BF16) hipLaunchKernelGGL((linear_tile_kernel<__hip_bfloat16>), dim3(tiles), dim3(256), 0, st, G);
+        else hipLaunchKernelGGL((linear_tile_kernel<__half>), dim3(tiles), dim3(256), 0, st, G);
+    } else if (dtype == VRWKV_BF16) hipLaunchKernelGGL((linear_group_kernel<__hip_bfloat16, MT>), dim3(tiles), dim3(256), 0, st, G);
     else if (dtype == VRWKV_F16) hipLaunchKernelGGL((linear_group_kernel<__half, MT>), dim3(tiles), dim3(256), 0, st, G);
     else hipLaunchKernelGGL((linear_group_kernel<float, MT>), dim3(tiles), dim3(256), 0, st, G);
 }
-// The largest tile that still gives every compute unit a workgroup: larger tiles read less from the L2s, smaller ones
-// shorten the chain of a wave.
+// Tile by the size of the result: larger tiles read less from the L2s, smaller ones give more workgroups and shorten the
+// chain of a wave.  Twelve bf16 blocks replayed as a graph, tiles of 64 / 128 on a side throughout, in us: 1568 x 768 2010 / 1751
+// (mixed by this rule 1721), 3136 x 384 1398 / 1297, 6272 x 384 2064 / 1550, 12544 x 768 9957 / 5472, 784 x 768 1339 / 1660; of
+// 16 / 32 / 64, eager: 784 x 768 2509 / 1672 / 1359, 3136 x 384 2499 / 1607 / 1417, 392 x 768 1544 / 1204 / 1163.
 int linear_group(LinGroup& G, int dtype, hipStream_t st) {
     long long area = 0;
     for (int i = 0; i < G.n; ++i) area += (long long)G.M * G.p[i].N;
     const int force = option(OPT_LINEAR_TILE);
-    const int mt = force ? force : area >= 64LL * 64 * 256 ? 4 : area >= 32LL * 32 * 128 ? 2 : 1;
-    if (mt == 4) launch_group<4>(G, dtype, st);
+    const bool wide = dtype != VRWKV_F32;                // 128 x 128 tiles are for 16 bits
+    const int mt = force && (wide || force < 8) ? force : wide && area >= 128LL * 128 * 110 ? 8 : area >= 64LL * 64 * 256 ? 4 : area >= 32LL * 32 * 128 ? 2 : 1;
+    if (mt == 8) launch_group<8>(G, dtype, st);
+    else if (mt == 4) launch_group<4>(G, dtype, st);
     else if (mt == 2) launch_group<2>(G, dtype, st);
     else launch_group<1>(G, dtype, st);
     return check_launch("linear_group");
