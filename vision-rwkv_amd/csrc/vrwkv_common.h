@@ -26,7 +26,7 @@ enum Option {
     OPT_BIWKV_BWD_SERIAL,   // sequential Bi-WKV backward kernel
     OPT_WKV6_FWD_SCALAR,    // sequential-state wkv6 forward kernel
     OPT_WKV6_BWD_SCALAR,    // sequential wkv6 backward sweeps
-    OPT_WKV6_BWD_UNFUSED,   // one launch per wkv6 backward scan
+    OPT_WKV6_BWD_UNFUSED,   // accepted, no effect (the backward is one kernel)
     OPT_WKV6_SEGMENTS,      // segments a wkv6 sequence is cut into
     OPT_LINEAR_TILE,        // tile of the block entry's projections (1, 2, 4, 8: 16 to 128 results on a side)
     OPT_WGRAD_SPLITS,       // token ranges of a weight gradient
