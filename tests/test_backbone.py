@@ -729,3 +729,48 @@ def test_second_derivative_of_a_projection_goes_through_tensor_ops():
     gw, = torch.autograd.grad(y.float().square().sum(), w, create_graph=True)
     ggx, = torch.autograd.grad(gw.float().sum(), x)
     assert ggx.shape == x.shape and bool(torch.isfinite(ggx).all()) and ggx.abs().max() > 0
+
+
+@pytest.mark.parametrize("kind", ["linear", "matmul", "bmm"])
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_weight_gradients_of_a_batch_of_cotangents(kind, device, monkeypatch):
+    """is_grads_batched runs the backward of a projection on batched tensors, which have no memory of their own: tensor ops,
+    the same gradients as one cotangent at a time (eight partial sums, each below half the largest value, and two results
+    rounded to bf16, 2^-9 each: below 2^-6 of the largest)."""
+    from vision_rwkv_amd import backbone as bb
+    if device == "cpu":                              # stands in for the kernel, which needs addresses
+        def product(a, b):
+            a.data_ptr(), b.data_ptr()
+            return (a.float().transpose(-1, -2) @ b.float()).to(a.dtype)
+        monkeypatch.setattr(bb, "weight_grad", product)
+    torch.manual_seed(7)
+    mk = lambda *s: torch.randn(*s, device=device, dtype=torch.bfloat16)
+    shape = (2,) if kind == "bmm" else ()
+    x, w, gs = mk(*shape, 256, 64), mk(*shape, 64, 64).requires_grad_(), mk(3, *shape, 256, 64)
+    fn = {"linear": bb._SplitKLinear, "matmul": bb._SplitKMatmul, "bmm": bb._SplitKBmm}[kind]
+    y = fn.apply(x, w, 8)
+    batched, = torch.autograd.grad(y, w, gs, is_grads_batched=True, retain_graph=True)
+    single = torch.stack([torch.autograd.grad(y, w, g, retain_graph=True)[0] for g in gs])
+    assert (batched.float() - single.float()).abs().max() <= 2.0 ** -6 * single.float().abs().max()
+
+
+@pytest.mark.parametrize("adjoint", [False, True])
+def test_table_resize_of_a_batch_of_cotangents(adjoint, monkeypatch):
+    """The derivative of either map on a batch of cotangents: tensor ops, equal to one at a time (fp32, taps of 4 x 4)."""
+    from vision_rwkv_amd import ops
+    def launch(t, src, dst, adj):                    # stands in for the kernel, which needs addresses
+        t.data_ptr()
+        return ops._table_resize_ops(t, src, dst, adj)
+    monkeypatch.setattr(ops, "_table_resize_launch", launch)
+    torch.manual_seed(8)
+    src, dst = (5, 7), (8, 6)
+    (n, m) = (48, 35) if adjoint else (35, 48)
+    t = torch.randn(1, n, 4, requires_grad=True)
+    y = ops._TableResize.apply(t, src, dst, adjoint)
+    gs = torch.randn(3, 1, m, 4)
+    batched, = torch.autograd.grad(y, t, gs, is_grads_batched=True, retain_graph=True)
+    for b, g in zip(batched, gs):
+        single, = torch.autograd.grad(y, t, g, retain_graph=True)
+        assert torch.allclose(b, single, rtol=1e-5, atol=1e-5)
+        # the pair are each other's adjoint
+        assert abs(float((y.detach() * g).sum() - (t.detach() * single).sum())) < 1e-3

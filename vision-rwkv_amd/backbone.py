@@ -15,7 +15,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch.nn.modules import module as _hooks
 
-from .ops import (RUN_CUDA, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, weight_grad, block_takes, block_weights_fit, block_forward, _equal_quarters, PRE_NONE, PRE_RELU_SQ, POST_NONE,
+from .ops import (RUN_CUDA, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, weight_grad, block_takes, block_weights_fit, block_forward, _equal_quarters, _transformed, batched_cotangent, PRE_NONE, PRE_RELU_SQ, POST_NONE,
                   POST_SIGMOID_GATE, POST_RESIDUAL)
 
 
@@ -70,9 +70,11 @@ OWN_WEIGHT_GRAD = 1 << 20
 
 def _token_product(a, b, splits):
     """a^T b over the rows (tokens) of a (M, O), b (M, I) or of stacks of them: the own kernel (fp32 sums, rounded once), or
-    `splits` batched partial products of the library.  A gradient that is itself to be differentiated takes tensor ops."""
+    `splits` batched partial products of the library.  A gradient that is itself to be differentiated, batched or traced takes tensor
+    ops."""
     (M, O), I = a.shape[-2:], b.shape[-1]
     if (not torch.is_grad_enabled() and O * I <= OWN_WEIGHT_GRAD and O % 8 == 0 and I % 8 == 0 and a.dtype == b.dtype
+            and not batched_cotangent(a, b) and not _transformed()
             and M * max(a.stride(-2), b.stride(-2), O, I) < 1 << 30):
         return weight_grad(a, b)
     S = splits if M % splits == 0 else 1

@@ -681,11 +681,23 @@ class _TableResize(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         src, dst, adjoint = ctx.meta
-        return _TableResize.apply(g, src, dst, not adjoint), None, None, None
+        resize = _table_resize_ops if batched_cotangent(g) else _TableResize.apply
+        return resize(g, src, dst, not adjoint), None, None, None
 
     @staticmethod
     def jvp(ctx, t, *_):
         return _TableResize.apply(t, *ctx.meta)
+
+
+def _table_resize_ops(table, src, dst, adjoint):
+    """The same two maps as tensor ops, for tensors without memory of their own."""
+    n, C = (dst if adjoint else src), table.shape[-1]
+    t = table.float().reshape(1, n[0], n[1], C).permute(0, 3, 1, 2)
+    if adjoint:
+        t = torch.ops.aten.upsample_bicubic2d_backward(t, dst, (1, C) + src, False)
+    else:
+        t = torch.nn.functional.interpolate(t, size=dst, mode="bicubic", align_corners=False)
+    return t.reshape(1, C, -1).transpose(1, 2).to(table.dtype)
 
 
 def _table_resize_launch(table, src, dst, adjoint):
@@ -696,6 +708,11 @@ def _table_resize_launch(table, src, dst, adjoint):
         _lib.check(_lib.lib().vrwkv_pos_resize(table.data_ptr(), out.data_ptr(), src[0], src[1], dst[0], dst[1], C,
                                                1 if adjoint else 0, _DT[table.dtype], _stream_ptr(table.device)))
     return out
+
+
+def batched_cotangent(*tensors):
+    """True where a backward runs on a batch of cotangents (is_grads_batched): plain to Python, but without memory."""
+    return any(torch._C._functorch.is_legacy_batchedtensor(t) for t in tensors)
 
 
 def _transformed():
