@@ -64,7 +64,7 @@ def _mix(module, x, mixes, shift_pixel, gamma, patch_resolution, fused, head_dim
 
 # Elements of a weight up to which its gradient is the framework's own kernel: 12544 tokens, own / the library's batched
 # partial products and their sum, in us: 768 x 768 34 / 43, 384 x 384 22 / 37, 1536 x 384 33 / 42, 192 x 192 15 / 25, 160 x 768 22 / 36,
-# five of 32 x 768 24 / 44; 3072 x 768 88 / 76.
+# five of 32 x 768 24 / 44; 3072 x 768 112 / 74.
 OWN_WEIGHT_GRAD = 1 << 20
 
 
