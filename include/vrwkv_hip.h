@@ -254,6 +254,16 @@ typedef struct vrwkv_block_args {
 } vrwkv_block_args;
 size_t vrwkv_block_fwd_workspace_bytes(int B, int T, int C, int hidden, int heads, int dtype);
 int vrwkv_block_fwd(const vrwkv_block_args* args, void* hip_stream);
+/* The same for a VRWKV6 block (heads > 0) whose low-rank matrices and vectors lie as the modules hold them: maa_w1 (C, 160), maa_w2
+ * (5, 32, C), decay_w1 (C, 64), decay_w2 (64, C) and att_kn_* (C) of `dtype`; maa_x, maa (w, k, v, r, g), ffn_mix_k, ffn_mix_r
+ * and u of `dtype`, or fp32 where their bit of fp32_vectors is set (0: maa_x, 1..5: maa, 6: ffn_mix_k, 7: ffn_mix_r, 8: u).
+ * Aligned to their elements; every call reads them anew.  The fields of `args` they stand for (att_mix, ffn_mix, u, maa, maa_w1,
+ * maa_w2, decay_w1, decay_w2, att_kn_*) are not looked at.  The same workspace. */
+typedef struct vrwkv_block6_params {
+    const void *maa_w1, *maa_w2, *decay_w1, *decay_w2, *maa_x, *maa[5], *ffn_mix_k, *ffn_mix_r, *u, *att_kn_w, *att_kn_b;
+    int fp32_vectors;
+} vrwkv_block6_params;
+int vrwkv_block6_fwd(const vrwkv_block_args* args, const vrwkv_block6_params* params, void* hip_stream);
 
 /* ---- weight gradients of the projections ----
  * out[z] (O, I) = sum over m of g[z][m][o] x[z][m][i], z < n: rows of g and x at pitches ldg, ldx (elements, multiples of 8),

@@ -666,6 +666,60 @@ def test_native_block_is_no_further_from_the_fp32_model_than_its_operators(kind,
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("C,dtype,key_norm,fp32_vectors", [(64, torch.bfloat16, False, False), (192, torch.float16, True, False),
+                                                           (320, torch.bfloat16, True, True), (768, torch.float32, True, False),
+                                                           (960, torch.bfloat16, False, True)])
+def test_native_v6_block_reads_its_weights_as_the_modules_hold_them(C, dtype, key_norm, fp32_vectors, monkeypatch):
+    """The low-rank matrices and vectors laid out inside the call against the same block given them laid out by tensor ops:
+    bit-identical results.  1 - time_maa_x rounds to its own type in both."""
+    from vision_rwkv_amd import backbone6
+    from vision_rwkv_amd.ops import block_forward
+    net = _small_backbone("v6", C, dtype, key_norm, True, False, (5, 7))
+    if fp32_vectors:
+        for l in net.layers:
+            for m, names in ((l.att, ["time_maa_" + n for n in "xwkvrg"] + ["time_faaaa"]), (l.ffn, ["spatial_mix_r"])):
+                for n in names:
+                    getattr(m, n).data = getattr(m, n).data.float()
+    calls = []
+
+    def both(x, w, params, **num):
+        flat = lambda n: params[n].detach().reshape(-1)
+        laid_out = {n: params[n].detach().transpose(-1, -2).contiguous() for n in ("maa_w1", "maa_w2", "decay_w1", "decay_w2")}
+        laid_out.update({n: params[n].detach().float() for n in ("att_kn_w", "att_kn_b") if n in params}, u=flat("u").float(),
+                        att_mix=torch.stack([torch.zeros(C, device="cuda"), (1 - flat("maa_x")).float()]),
+                        ffn_mix=torch.stack([flat("ffn_mix_k").float(), flat("ffn_mix_r").float()]),
+                        maa=torch.stack([flat("maa_" + n).float() for n in "wkvrg"]))
+        got, want = block_forward(x, w, params, **num), block_forward(x, {**w, **laid_out}, **num)
+        calls.append(bool(torch.isfinite(want).all()) and torch.equal(got, want))
+        return got
+
+    monkeypatch.setattr(backbone6, "block_forward", both)
+    with torch.no_grad():
+        net(torch.randn(2, 3, 80, 112, device="cuda").to(dtype))
+    assert calls == [True, True]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("key_norm,cls", [(False, True), (True, False)])
+def test_native_v6_block_sees_writes_through_data(key_norm, cls):
+    """A write to p.data leaves the parameter's version and address alone; the next inference must use it all the same:
+    bit-identical to a model that is loaded with the new values."""
+    import copy
+    net = _small_backbone("v6", 128, torch.bfloat16, key_norm, True, cls, (6, 5))
+    fresh = copy.deepcopy(net)
+    img = torch.randn(2, 3, 96, 80, device="cuda").bfloat16()
+    with torch.no_grad():
+        before = net(img)
+        for l in net.layers:
+            for p in l.parameters():
+                p.data.copy_(p.data * 1.25 + 0.01)
+        got = net(img)
+        fresh.load_state_dict(net.state_dict())
+        want = fresh(img)
+    assert not torch.equal(got, before) and torch.equal(got, want)
+
+
+@pytest.mark.gpu
 def test_native_block_leaves_changed_modules_to_their_own_code():
     net = _small_backbone("v4", 192, torch.bfloat16, False, False, False, (14, 14))
     img = torch.randn(1, 3, 224, 224, device="cuda").bfloat16()

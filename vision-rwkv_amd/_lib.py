@@ -29,6 +29,13 @@ class BlockArgs(ctypes.Structure):
                 + [(n, ctypes.c_void_p) for n in POINTERS_B] + [(n, ctypes.c_int) for n in INTS] + [(n, ctypes.c_float) for n in FLOATS])
 
 
+class Block6Params(ctypes.Structure):
+    """vrwkv_block6_params of include/vrwkv_hip.h."""
+    POINTERS = ("maa_w1", "maa_w2", "decay_w1", "decay_w2", "maa_x", "maa_w", "maa_k", "maa_v", "maa_r", "maa_g", "ffn_mix_k", "ffn_mix_r",
+                "u", "att_kn_w", "att_kn_b")
+    _fields_ = [(n, ctypes.c_void_p) for n in POINTERS] + [("fp32_vectors", ctypes.c_int)]
+
+
 class VrwkvError(RuntimeError):
     """Non-zero status from the C ABI (mirrors the RuntimeError TORCH_CHECK raises at
     classification/mmcls_custom/models/backbones/cuda_new/bi_wkv.cpp:6-8)."""
@@ -119,6 +126,8 @@ def _declare(lib):
     lib.vrwkv_block_fwd_workspace_bytes.restype = sz
     lib.vrwkv_block_fwd.argtypes = [c.POINTER(BlockArgs), vp]
     lib.vrwkv_block_fwd.restype = i
+    lib.vrwkv_block6_fwd.argtypes = [c.POINTER(BlockArgs), c.POINTER(Block6Params), vp]
+    lib.vrwkv_block6_fwd.restype = i
     ll = c.c_longlong
     lib.vrwkv_wgrad_workspace_bytes.argtypes = [i, i, i, i]
     lib.vrwkv_wgrad_workspace_bytes.restype = sz

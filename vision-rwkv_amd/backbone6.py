@@ -159,30 +159,22 @@ class Block6(nn.Module):
             return None
         w, num = wn
         ap, fp, ln_x, gate = att._parameters, ffn._parameters, att._modules["ln_x"], att._modules["gate"]
-        low = (ap["time_maa_w1"], ap["time_maa_w2"], ap["time_decay_w1"], ap["time_decay_w2"])
+        low = {"maa_w1": ap["time_maa_w1"], "maa_w2": ap["time_maa_w2"], "decay_w1": ap["time_decay_w1"], "decay_w2": ap["time_decay_w2"]}
+        vec = {"maa_" + n: ap["time_maa_" + n] for n in "xwkvrg"}
+        vec.update(ffn_mix_k=fp["spatial_mix_k"], ffn_mix_r=fp["spatial_mix_r"], u=ap["time_faaaa"])
         if (not _as_built(gate, nn.Linear) or gate.bias is not None or gate.weight.shape != (C, C)
                 or not _as_built(ln_x, nn.GroupNorm) or ln_x.num_groups * HEAD_SIZE != C or ln_x.num_channels != C or not ln_x.affine
-                or att.n_head * HEAD_SIZE != C or ap["time_decay"].numel() != C or ap["time_faaaa"].numel() != C
-                or tuple(t.shape for t in low) != ((C, 160), (5, 32, C), (C, 64), (64, C))
+                or att.n_head * HEAD_SIZE != C or ap["time_decay"].numel() != C
+                or tuple(t.shape for t in low.values()) != ((C, 160), (5, 32, C), (C, 64), (64, C))
+                or any(t.numel() != C or t.dtype not in (x.dtype, torch.float32) or t.get_device() != x.get_device() or not t.is_contiguous()
+                       for t in vec.values())
                 or T != res[0] * res[1] + (1 if att.with_cls_token else 0) or att.with_cls_token != ffn.with_cls_token):
             return None
         w.update(gate=gate.weight, decay=ap["time_decay"], gn_w=ln_x.weight, gn_b=ln_x.bias)
-        if not block_weights_fit(x, (*w.values(), *low)):
+        if not block_weights_fit(x, (*w.values(), *low.values())):
             return None
-        cm = (fp["spatial_mix_k"], fp["spatial_mix_r"])
-        maas = tuple(ap["time_maa_" + n] for n in "wkvrg")
-        mx, first = ap["time_maa_x"], ap["time_faaaa"]
-        # the low-rank matrices with the contraction index innermost, like every other projection's
-        w["maa_w1"], w["maa_w2"], w["decay_w1"], w["decay_w2"] = eval_cached(
-            att, "low_rank", low, None, lambda: [t.detach().transpose(-1, -2).contiguous() for t in low])
-        w["u"] = eval_cached(att, "u", (first,), None, lambda: first.detach().float().contiguous())
-        w["att_mix"] = eval_cached(att, "mix_table", (mx,), x.device, lambda: stack_mixes([torch.zeros_like(mx), 1 - mx], x.device))
-        w["ffn_mix"] = eval_cached(ffn, "mix_table", cm, x.device, lambda: stack_mixes(cm, x.device))
-        w["maa"] = eval_cached(att, "maa_table", maas, x.device, lambda: stack_mixes(maas, x.device))
-        if "att_kn_w" in w:                                  # normalises the operator's fp32 result
-            kn = (w["att_kn_w"], w["att_kn_b"])
-            w["att_kn_w"], w["att_kn_b"] = eval_cached(att, "kn32", kn, None, lambda: [p.detach().float() for p in kn])
-        return block_forward(x, w, Hp=res[0], Wp=res[1], heads=att.n_head, quarter=HEAD_SIZE // 4, gn_eps=ln_x.eps, **num)
+        params = {**low, **vec, **{n: w.pop(n) for n in ("att_kn_w", "att_kn_b") if n in w}}
+        return block_forward(x, w, params, Hp=res[0], Wp=res[1], heads=att.n_head, quarter=HEAD_SIZE // 4, gn_eps=ln_x.eps, **num)
 
     def forward(self, x, patch_resolution):
         if self.layer_id == 0:

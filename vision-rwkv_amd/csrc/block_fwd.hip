@@ -211,7 +211,7 @@ LinProblem linear(const void* a, const void* w, void* out, int N, int K, int lda
 size_t al(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
 // token tensors of C channels that live at the same time: LN result, up to six mixes, x after the attention half, and the
 // operator's tensors
-struct Layout { size_t n, hidden, op, total; };
+struct Layout { size_t n, hidden, op, weights, total; };
 Layout layout(int B, int T, int C, int hidden, int heads, int dtype) {
     Layout l;
     const size_t es = dtype == VRWKV_F32 ? 4 : 2;
@@ -221,8 +221,65 @@ Layout layout(int B, int T, int C, int hidden, int heads, int dtype) {
     // VRWKV: 9 tensors; VRWKV6: x1, LN, sx, xxx, five mixes, five maps (later r, k, v, w, gate), two fp32 tensors, low-rank rows
     const size_t tokens = heads ? 2 + 2 + 5 + 5 + 4 : 9;
     const size_t low = heads ? al((size_t)B * T * 160 * es) + al((size_t)B * T * 64 * es) : 0;
-    l.total = tokens * l.n + 2 * l.hidden + low + l.op;           // (hidden rows twice: before and after their norm)
+    l.weights = heads ? al((size_t)448 * C * es) + al((size_t)12 * C * sizeof(float)) : 0;   // (see weights6_kernel)
+    l.total = tokens * l.n + 2 * l.hidden + low + l.op + l.weights;       // (hidden rows twice: before and after their norm)
     return l;
+}
+
+// ---- VRWKV6: the weights that the block wants otherwise than the modules hold them -----------------------------------------
+// The low-rank matrices with the contraction index innermost (32 x 32 tiles turned through LDS) and the vectors in fp32.  Formed
+// in every call, so that a write to a parameter leaves nothing behind: 448 C values, one launch of 3 us (twelve blocks of 784 x 768
+// bf16 1953 -> 1990 us, of 196 x 192 893 -> 935, against copies kept between calls).
+// Grid: 14 C / 32 tiles, then C / 256 (rounded up) workgroups for the vectors.
+struct Weights6 {
+    vrwkv_block6_params p;
+    void *maa_w1, *maa_w2, *decay_w1, *decay_w2;
+    float *att_mix, *ffn_mix, *maa, *u, *kn_w, *kn_b;
+};
+template <typename IO>
+__global__ __launch_bounds__(256)
+void weights6_kernel(Weights6 W, int C)
+{
+    __shared__ IO tile[32][33];
+    const int per = C / 32;
+    int id = blockIdx.x;
+    if (id >= 14 * per) {
+        const int c = (id - 14 * per) * 256 + threadIdx.x;
+        if (c >= C) return;
+        auto get = [&](const void* p, int bit) { return W.p.fp32_vectors >> bit & 1 ? ((const float*)p)[c] : to_f32(((const IO*)p)[c]); };
+        const float x = 1.f - get(W.p.maa_x, 0);          // rounded to its own type, like the tensor operation
+        W.att_mix[c] = 0.f;
+        W.att_mix[C + c] = W.p.fp32_vectors & 1 ? x : to_f32(from_f32<IO>(x));
+        for (int i = 0; i < 5; ++i) W.maa[i * C + c] = get(W.p.maa[i], 1 + i);
+        W.ffn_mix[c] = get(W.p.ffn_mix_k, 6);
+        W.ffn_mix[C + c] = get(W.p.ffn_mix_r, 7);
+        W.u[c] = get(W.p.u, 8);
+        if (W.p.att_kn_w) {
+            W.kn_w[c] = to_f32(((const IO*)W.p.att_kn_w)[c]);
+            W.kn_b[c] = to_f32(((const IO*)W.p.att_kn_b)[c]);
+        }
+        return;
+    }
+    const IO* src;
+    IO* dst;
+    int rows, cols, tr, tc;                               // the matrix as it lies, and the tile's place in it
+    if (id < 5 * per) {
+        src = (const IO*)W.p.maa_w1; dst = (IO*)W.maa_w1; rows = C; cols = 160; tr = id / 5; tc = id % 5;
+    } else if ((id -= 5 * per) < 5 * per) {
+        const size_t z = (size_t)(id / per) * 32 * C;
+        src = (const IO*)W.p.maa_w2 + z; dst = (IO*)W.maa_w2 + z; rows = 32; cols = C; tr = 0; tc = id % per;
+    } else if ((id -= 5 * per) < 2 * per) {
+        src = (const IO*)W.p.decay_w1; dst = (IO*)W.decay_w1; rows = C; cols = 64; tr = id / 2; tc = id % 2;
+    } else {
+        id -= 2 * per;
+        src = (const IO*)W.p.decay_w2; dst = (IO*)W.decay_w2; rows = 64; cols = C; tr = id / per; tc = id % per;
+    }
+    const int x = threadIdx.x & 31, y = threadIdx.x >> 5;
+#pragma unroll
+    for (int i = 0; i < 32; i += 8) tile[y + i][x] = src[(size_t)(32 * tr + y + i) * cols + 32 * tc + x];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 32; i += 8) dst[(size_t)(32 * tc + y + i) * rows + 32 * tr + x] = tile[x][y + i];
 }
 
 }  // namespace
@@ -236,9 +293,30 @@ extern "C" size_t vrwkv_block_fwd_workspace_bytes(int B, int T, int C, int hidde
     return vrwkv::layout(B, T, C, hidden, heads, dtype).total;
 }
 
-extern "C" int vrwkv_block_fwd(const vrwkv_block_args* a, void* hip_stream)
+static int block_fwd(const vrwkv_block_args* args, const vrwkv_block6_params* params, void* hip_stream)
 {
     using namespace vrwkv;
+    vrwkv_block_args with_params;
+    const vrwkv_block_args* a = args;
+    Weights6 W;
+    if (args && params && args->heads > 0 && args->C > 0 && args->workspace) {
+        // the fields that `params` stands for: the end of the workspace, filled below once the sizes are checked
+        const size_t es = args->dtype == VRWKV_F32 ? 4 : 2, n = (size_t)args->C;
+        const Layout L = layout(args->B, args->T, args->C, args->hidden, args->heads, args->dtype);
+        char* m = (char*)args->workspace + L.total - L.weights;
+        float* f = (float*)(m + al(448 * n * es));
+        W = Weights6{*params, m, m + 160 * n * es, m + 320 * n * es, m + 384 * n * es, f, f + 2 * n, f + 4 * n, f + 9 * n, f + 10 * n, f + 11 * n};
+        with_params = *args;
+        a = &with_params;
+        with_params.maa_w1 = W.maa_w1; with_params.maa_w2 = W.maa_w2; with_params.decay_w1 = W.decay_w1; with_params.decay_w2 = W.decay_w2;
+        with_params.att_mix = W.att_mix; with_params.ffn_mix = W.ffn_mix; with_params.maa = W.maa; with_params.u = W.u;
+        with_params.att_kn_w = params->att_kn_w ? W.kn_w : nullptr;
+        with_params.att_kn_b = params->att_kn_b ? W.kn_b : nullptr;
+        bool all = params->maa_w1 && params->maa_w2 && params->decay_w1 && params->decay_w2 && params->maa_x && params->ffn_mix_k &&
+                   params->ffn_mix_r && params->u;
+        for (const void* p : params->maa) all = all && p;
+        if (!all) a = nullptr;
+    }
     if (!a || !a->x || !a->out || !a->workspace || !a->ln1_w || !a->ln1_b || !a->ln2_w || !a->ln2_b || !a->att_mix || !a->ffn_mix ||
         !a->u || !a->key || !a->value || !a->receptance || !a->output || !a->ffn_key || !a->ffn_receptance || !a->ffn_value ||
         (a->heads ? !a->gate || !a->maa || !a->maa_w1 || !a->maa_w2 || !a->decay || !a->decay_w1 || !a->decay_w2 || !a->gn_w || !a->gn_b
@@ -275,6 +353,13 @@ extern "C" int vrwkv_block_fwd(const vrwkv_block_args* a, void* hip_stream)
     char* at = (char*)a->workspace;
     auto take = [&](size_t bytes) { void* p = at; at += bytes; return p; };
     hipStream_t st = static_cast<hipStream_t>(hip_stream);
+    if (a != args) {
+        const dim3 grid((unsigned)(14 * (C / 32) + (C + 255) / 256)), block(256);
+        if (dt == VRWKV_F32) hipLaunchKernelGGL((weights6_kernel<float>), grid, block, 0, st, W, C);
+        else if (dt == VRWKV_BF16) hipLaunchKernelGGL((weights6_kernel<__hip_bfloat16>), grid, block, 0, st, W, C);
+        else hipLaunchKernelGGL((weights6_kernel<__half>), grid, block, 0, st, W, C);
+        TRY(check_launch("block_fwd (weights)"));
+    }
     const int hd = H ? 64 : 0;
     void *x1 = take(L.n), *ln = take(L.n), *hid = take(L.hidden), *hid_raw = take(L.hidden), *op_ws = take(L.op);
     LinGroup G;
@@ -360,4 +445,15 @@ extern "C" int vrwkv_block_fwd(const vrwkv_block_args* a, void* hip_stream)
     LinProblem p = linear(hid, a->ffn_value, nullptr, C, hidden);
     p.gate = fr;
     return residual(p, x1, a->out, a->gamma2, a->ln2_w, a->ln2_b, a->ln2_eps, ftmp);
+}
+
+extern "C" int vrwkv_block_fwd(const vrwkv_block_args* args, void* hip_stream) { return block_fwd(args, nullptr, hip_stream); }
+
+extern "C" int vrwkv_block6_fwd(const vrwkv_block_args* args, const vrwkv_block6_params* params, void* hip_stream)
+{
+    if (!args || !params || args->heads <= 0) {
+        vrwkv::set_error("block6_fwd: null argument or no heads");
+        return VRWKV_INVALID_ARG;
+    }
+    return block_fwd(args, params, hip_stream);
 }

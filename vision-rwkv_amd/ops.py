@@ -755,9 +755,9 @@ def block_weights_fit(x, weights):
     return True
 
 
-def block_forward(x, tensors, **scalars):
-    """vrwkv_block_fwd on the current stream: tensors and scalars fill the like-named fields of vrwkv_block_args.  None when
-    a tensor is not aligned for 16-byte accesses."""
+def block_forward(x, tensors, params=None, **scalars):
+    """vrwkv_block_fwd on the current stream: tensors and scalars fill the like-named fields of vrwkv_block_args; with params
+    (fields of vrwkv_block6_params) vrwkv_block6_fwd.  None when a tensor is not aligned for 16-byte accesses."""
     L = _lib.lib()
     B, T, C = x.shape
     out = torch.empty_like(x)
@@ -773,7 +773,12 @@ def block_forward(x, tensors, **scalars):
     ws = torch.empty(a.workspace_bytes, dtype=torch.uint8, device=x.device)
     a.workspace = ws.data_ptr()
     with _on(x.device):
-        _lib.check(L.vrwkv_block_fwd(ctypes.byref(a), _stream_ptr(x.device)))
+        if params is None:
+            _lib.check(L.vrwkv_block_fwd(ctypes.byref(a), _stream_ptr(x.device)))
+        else:
+            fp32 = sum(1 << i for i, n in enumerate(_lib.Block6Params.POINTERS[4:13]) if params[n].dtype == torch.float32)
+            p = _lib.Block6Params(fp32_vectors=fp32, **{n: t.data_ptr() for n, t in params.items()})
+            _lib.check(L.vrwkv_block6_fwd(ctypes.byref(a), ctypes.byref(p), _stream_ptr(x.device)))
     return out
 
 
