@@ -719,6 +719,26 @@ def test_native_v6_block_sees_writes_through_data(key_norm, cls):
     assert not torch.equal(got, before) and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("copied", [False, True])
+def test_kept_tables_follow_a_module_that_is_cast_away_and_back(copied):
+    """Casting a module gives its parameters new memory, possibly where the old lay, and leaves their versions alone: the kept
+    value must be rebuilt, also in a copy whose original is gone."""
+    import copy
+    from vision_rwkv_amd.backbone import eval_cached
+    torch.manual_seed(12)
+    for n in [500] * 50 + [3, 1000, 70000]:              # (the same address again in a third of the first kind)
+        m = torch.nn.Linear(n, 1, bias=False)
+        take = lambda m: eval_cached(m, "table", (m.weight,), None, lambda: m.weight.detach().clone())
+        assert torch.equal(take(m), m.weight) and take(m) is take(m)
+        if copied:
+            m = copy.deepcopy(m)
+        m.half().float()
+        assert torch.equal(take(m), m.weight), n
+        with torch.no_grad():
+            m.weight.add_(1)
+        assert torch.equal(take(m), m.weight), n
+
+
 @pytest.mark.gpu
 def test_native_block_leaves_changed_modules_to_their_own_code():
     net = _small_backbone("v4", 192, torch.bfloat16, False, False, False, (14, 14))

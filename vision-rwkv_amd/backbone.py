@@ -40,12 +40,14 @@ def resize_pos_embed(pos_embed, src_shape, dst_shape, mode="bicubic", num_extra_
 
 def eval_cached(module, name, params, extra, make):
     """Value derived from parameters (a dtype conversion, a stacked table), kept on the module between forward passes
-    without autograd and rebuilt when a parameter was written to (its version counter), moved or cast."""
-    key = (extra,) + tuple((p._version, p.dtype, p.device, p.data_ptr()) for p in params)
+    without autograd and rebuilt when a parameter was written to (its version counter), moved or cast.  The entry holds on to
+    the memory it was derived from, so that no later parameter can be found at the same address.  A write through p.data
+    counts as no new version: after one, the next in-place write, cast or move of the parameter brings the value up to date."""
+    key = (extra,) + tuple((p._version, p.dtype, p.device) for p in params)
     slot = module.__dict__.setdefault("_eval_cache", {})
     hit = slot.get(name)
-    if hit is None or hit[0] != key:
-        hit = (key, make())
+    if hit is None or hit[0] != key or any(m.data_ptr() != p.data_ptr() for m, p in zip(hit[2], params)):
+        hit = (key, make(), [p.detach() for p in params])
         slot[name] = hit
     return hit[1]
 
