@@ -612,7 +612,7 @@ def test_split_weight_gradient_of_the_block_projections():
         assert bb._proj(lin, x).grad_fn is None
 
 
-def _small_backbone(kind, C, dtype, key_norm, post_norm, cls, hw):
+def _small_backbone(kind, C, dtype, key_norm, post_norm, cls, hw, device="cuda"):
     import vision_rwkv_amd as ops
     torch.manual_seed(11)
     kw = dict(img_size=hw[0] * 16, embed_dims=C, depth=2, key_norm=key_norm, post_norm=post_norm, init_values=0.3 if post_norm else None)
@@ -623,7 +623,7 @@ def _small_backbone(kind, C, dtype, key_norm, post_norm, cls, hw):
                 p.normal_(0, 0.02)
             elif p.dim() < 2 or p.shape[0] == 1:
                 p.add_(0.05 * torch.randn_like(p))
-    return net.cuda().to(dtype).eval()
+    return net.to(device, dtype).eval()
 
 
 @pytest.mark.gpu
@@ -717,6 +717,64 @@ def test_native_v6_block_sees_writes_through_data(key_norm, cls):
         fresh.load_state_dict(net.state_dict())
         want = fresh(img)
     assert not torch.equal(got, before) and torch.equal(got, want)
+
+
+def _as_buffer(module, name):
+    value = getattr(module, name).detach()
+    delattr(module, name)
+    module.register_buffer(name, value)
+
+
+class _Twice(torch.nn.Module):
+    def forward(self, x):
+        return 2 * x
+
+
+_CHANGES = {
+    "pruned ffn key": lambda b, nn: nn.utils.prune.l1_unstructured(b.ffn.key, "weight", 0.3),
+    "weight norm": lambda b, nn: nn.utils.weight_norm(b.ffn.key),
+    "spectral norm": lambda b, nn: nn.utils.spectral_norm(b.ffn.key),
+    "parametrised ffn key": lambda b, nn: nn.utils.parametrize.register_parametrization(b.ffn.key, "weight", _Twice()),
+    "pruned layer scale": lambda b, nn: nn.utils.prune.l1_unstructured(b, "gamma1", 0.3),
+    "parametrised layer scale": lambda b, nn: nn.utils.parametrize.register_parametrization(b, "gamma2", _Twice()),
+    "pruned att key": lambda b, nn: nn.utils.prune.l1_unstructured(b.att.key, "weight", 0.3),
+    "pruned mix": lambda b, nn: nn.utils.prune.l1_unstructured(b.ffn, "spatial_mix_k", 0.3),
+    "pruned norm": lambda b, nn: nn.utils.prune.l1_unstructured(b.ln1, "bias", 0.3),
+    "ffn key as a buffer": lambda b, nn: _as_buffer(b.ffn.key, "weight"),
+    "output as a buffer": lambda b, nn: _as_buffer(b.att.output, "weight"),
+    "mix as a buffer": lambda b, nn: _as_buffer(b.ffn, "spatial_mix_r"),
+    "decay as a buffer": lambda b, nn: _as_buffer(b.att, "time_decay" if hasattr(b.att, "time_decay") else "spatial_decay"),
+    "bonus as a buffer": lambda b, nn: _as_buffer(b.att, "time_faaaa" if hasattr(b.att, "time_faaaa") else "spatial_first"),
+    "norm as a buffer": lambda b, nn: _as_buffer(b.ln2, "weight"),
+    "layer scale as a buffer": lambda b, nn: _as_buffer(b, "gamma2"),
+    "no ffn norm": lambda b, nn: setattr(b, "ln2", nn.Identity()),
+}
+
+
+@pytest.mark.parametrize("kind", ["v4", "v6"])
+@pytest.mark.parametrize("change", list(_CHANGES))
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_blocks_whose_weights_are_held_otherwise_run_their_operators(device, change, kind, monkeypatch):
+    """Pruned, normed, parametrised weights and parameters made buffers are not what the native call could read: it declines
+    (on the CPU asked with its first check stood in for), and the model computes what its operators compute."""
+    import torch.nn.utils.parametrize, torch.nn.utils.prune
+    from vision_rwkv_amd import ops as impl, backbone, backbone6
+    net = _small_backbone(kind, 64, torch.float32, False, True, False, (3, 4), device)
+    if device == "cpu":
+        monkeypatch.setattr(backbone, "block_takes", lambda x: True)
+        for m in (backbone, backbone6):
+            monkeypatch.setattr(m, "block_forward", lambda *a, **kw: "native")
+    x = torch.randn(2, 12, 64, device=device)
+    with torch.no_grad():
+        assert all(l._native(x, (3, 4)) is not None for l in net.layers)
+        for l in net.layers:
+            _CHANGES[change](l, torch.nn)
+        assert all(l._native(x, (3, 4)) is None for l in net.layers)
+        if device == "cuda" and change != "no ffn norm":
+            img = torch.randn(2, 3, 48, 64, device="cuda")
+            got = net(img)
+            monkeypatch.setattr(impl, "BLOCK_FUSE_ENABLED", False)
+            assert torch.equal(got, net(img))
 
 
 @pytest.mark.parametrize("copied", [False, True])

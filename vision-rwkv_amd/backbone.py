@@ -214,7 +214,8 @@ def _native_size(x, hidden, v6):
 
 
 def _as_built(module, kind):
-    """True when calling `module` does what `kind`'s own forward does with the module's parameters and nothing else."""
+    """True when calling `module` does what `kind`'s own forward does with the module's parameters and nothing else.  (What stands
+    in another place -- pruned, normed or parametrised weights, buffers -- is missing from _parameters, or None, also then.)"""
     return (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks and "forward" not in module.__dict__)
 
 
@@ -223,36 +224,37 @@ def _block_weights(block, att, ffn, x):
     built with, the norms with both vectors) and the numbers that go with them, as fields of vrwkv_block_args; None for any
     other block."""
     am, fm, bm, C = att._modules, ffn._modules, block._modules, x.shape[2]
-    key = fm["key"]
-    hidden = key._parameters["weight"].shape[0] if type(key) is nn.Linear else 0
+    key = fm.get("key")
+    weight = key._parameters.get("weight") if _as_built(key, nn.Linear) else None      # (a pruned or normed layer has none)
+    hidden = weight.shape[0] if weight is not None else 0
     if not (C % 32 == 0 and hidden % 32 == 0 and 0 < hidden <= 4096 and att.fused_shift and ffn.fused_shift
             and att.shift_pixel == ffn.shift_pixel and _native_size(x, hidden, "gate" in am)):
         return None
     w, num = {}, dict(hidden=hidden, shift_pixel=att.shift_pixel, post_norm=int(block.post_norm))
-    for name, lin, shape in (("key", am["key"], (C, C)), ("value", am["value"], (C, C)), ("receptance", am["receptance"], (C, C)),
-                             ("output", am["output"], (C, C)), ("ffn_key", key, (hidden, C)),
-                             ("ffn_receptance", fm["receptance"], (C, C)), ("ffn_value", fm["value"], (C, hidden))):
+    for name, lin, shape in (("key", am.get("key"), (C, C)), ("value", am.get("value"), (C, C)), ("receptance", am.get("receptance"), (C, C)),
+                             ("output", am.get("output"), (C, C)), ("ffn_key", key, (hidden, C)),
+                             ("ffn_receptance", fm.get("receptance"), (C, C)), ("ffn_value", fm.get("value"), (C, hidden))):
         if not _as_built(lin, nn.Linear):
             return None
         p = lin._parameters
-        if p["bias"] is not None or p["weight"].shape != shape:
+        if p.get("bias") is not None or p.get("weight") is None or p["weight"].shape != shape:
             return None
         w[name] = p["weight"]
-    for name, ln, n in (("ln1", bm["ln1"], C), ("ln2", bm["ln2"], C), ("att_kn", am.get("key_norm"), C),
+    for name, ln, n in (("ln1", bm.get("ln1"), C), ("ln2", bm.get("ln2"), C), ("att_kn", am.get("key_norm"), C),
                         ("ffn_kn", fm.get("key_norm"), hidden)):
         if ln is None and name.endswith("kn"):
             continue
         if not _as_built(ln, nn.LayerNorm) or ln.normalized_shape != (n,):
             return None
         p = ln._parameters
-        if p["weight"] is None or p["bias"] is None:
+        if p.get("weight") is None or p.get("bias") is None:
             return None
         w[name + "_w"], w[name + "_b"] = p["weight"], p["bias"]
         num[name + "_eps"] = ln.eps
     if block.layer_scale:
         for name in ("gamma1", "gamma2"):
-            w[name] = block._parameters[name]
-            if w[name].shape != (C,):
+            w[name] = block._parameters.get(name)
+            if w[name] is None or w[name].shape != (C,):
                 return None
     return w, num
 
@@ -261,7 +263,7 @@ def _block_may_fuse(block, att_kind, ffn_kind, x):
     """The checks that come before a look at the weights."""
     return (block_takes(x)
             and not _hooks._global_forward_hooks and not _hooks._global_forward_pre_hooks
-            and _as_built(block._modules["att"], att_kind) and _as_built(block._modules["ffn"], ffn_kind))
+            and _as_built(block._modules.get("att"), att_kind) and _as_built(block._modules.get("ffn"), ffn_kind))
 
 
 class VRWKV_SpatialMix(nn.Module):
@@ -369,10 +371,10 @@ class Block(nn.Module):
             return None
         w, num = wn
         ap, fp = att._parameters, ffn._parameters
-        decay, first = ap["spatial_decay"], ap["spatial_first"]
-        if decay.dtype != x.dtype:
+        decay, first = ap.get("spatial_decay"), ap.get("spatial_first")
+        am, fm = [ap.get("spatial_mix_" + n) for n in "kvr"], [fp.get("spatial_mix_" + n) for n in "kr"]
+        if any(p is None for p in (decay, first, *am, *fm)) or decay.dtype != x.dtype:
             return None
-        am, fm = [ap["spatial_mix_k"], ap["spatial_mix_v"], ap["spatial_mix_r"]], [fp["spatial_mix_k"], fp["spatial_mix_r"]]
         w["w"], w["u"] = eval_cached(att, "wu", (decay, first), T,
                                      lambda: ((decay / T).float().contiguous(), (first / T).float().contiguous()))
         w["att_mix"] = eval_cached(att, "mix_table", am, x.device, lambda: stack_mixes(am, x.device))

@@ -158,11 +158,13 @@ class Block6(nn.Module):
         if wn is None:
             return None
         w, num = wn
-        ap, fp, ln_x, gate = att._parameters, ffn._parameters, att._modules["ln_x"], att._modules["gate"]
-        low = {"maa_w1": ap["time_maa_w1"], "maa_w2": ap["time_maa_w2"], "decay_w1": ap["time_decay_w1"], "decay_w2": ap["time_decay_w2"]}
-        vec = {"maa_" + n: ap["time_maa_" + n] for n in "xwkvrg"}
-        vec.update(ffn_mix_k=fp["spatial_mix_k"], ffn_mix_r=fp["spatial_mix_r"], u=ap["time_faaaa"])
-        if (not _as_built(gate, nn.Linear) or gate.bias is not None or gate.weight.shape != (C, C)
+        ap, fp, ln_x, gate = att._parameters, ffn._parameters, att._modules.get("ln_x"), att._modules.get("gate")
+        low = {n: ap.get("time_" + n) for n in ("maa_w1", "maa_w2", "decay_w1", "decay_w2")}
+        vec = {"maa_" + n: ap.get("time_maa_" + n) for n in "xwkvrg"}
+        vec.update(ffn_mix_k=fp.get("spatial_mix_k"), ffn_mix_r=fp.get("spatial_mix_r"), u=ap.get("time_faaaa"))
+        if any(p is None for p in (*low.values(), *vec.values(), ap.get("time_decay"))):
+            return None
+        if (not _as_built(gate, nn.Linear) or gate.bias is not None or gate._parameters.get("weight") is None or gate.weight.shape != (C, C)
                 or not _as_built(ln_x, nn.GroupNorm) or ln_x.num_groups * HEAD_SIZE != C or ln_x.num_channels != C or not ln_x.affine
                 or att.n_head * HEAD_SIZE != C or ap["time_decay"].numel() != C
                 or tuple(t.shape for t in low.values()) != ((C, 160), (5, 32, C), (C, 64), (64, C))
