@@ -777,6 +777,32 @@ def test_blocks_whose_weights_are_held_otherwise_run_their_operators(device, cha
             assert torch.equal(got, net(img))
 
 
+@pytest.mark.parametrize("kind", ["v4", "v6"])
+@pytest.mark.parametrize("part,name", [("att", "spatial_mix_k"), ("ffn", "spatial_mix_r"), ("att", "spatial_decay"), ("att", "spatial_first"),
+                                       ("att", "time_maa_x"), ("att", "time_maa_g"), ("att", "time_faaaa"), ("att", "time_decay"),
+                                       ("att", "time_maa_w2")])
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_native_block_declines_vectors_of_another_size_or_device(device, part, name, kind, monkeypatch):
+    """The operators refuse a vector that has not one element per channel, or lies elsewhere than x; the native call, which
+    would read past its end, is not to be made (and is stood in for here)."""
+    from vision_rwkv_amd import backbone, backbone6
+    net = _small_backbone(kind, 64, torch.float32, False, True, False, (3, 4), device)
+    monkeypatch.setattr(backbone, "block_takes", lambda x: True)
+    for m in (backbone, backbone6):
+        monkeypatch.setattr(m, "block_forward", lambda *a, **kw: "native")
+    block, x = net.layers[1], torch.randn(2, 12, 64, device=device)
+    module = getattr(block, part)
+    if not hasattr(module, name):
+        return
+    old = getattr(module, name)
+    with torch.no_grad():
+        for new in [torch.zeros(n, device=device) for n in (1, 32, 128)] + ([old.cpu()] if device == "cuda" else []):
+            setattr(module, name, torch.nn.Parameter(new))
+            assert block._native(x, (3, 4)) is None, tuple(new.shape)
+        setattr(module, name, old)
+        assert block._native(x, (3, 4)) == "native"
+
+
 @pytest.mark.parametrize("copied", [False, True])
 def test_kept_tables_follow_a_module_that_is_cast_away_and_back(copied):
     """Casting a module gives its parameters new memory, possibly where the old lay, and leaves their versions alone: the kept

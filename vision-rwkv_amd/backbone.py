@@ -373,7 +373,7 @@ class Block(nn.Module):
         ap, fp = att._parameters, ffn._parameters
         decay, first = ap.get("spatial_decay"), ap.get("spatial_first")
         am, fm = [ap.get("spatial_mix_" + n) for n in "kvr"], [fp.get("spatial_mix_" + n) for n in "kr"]
-        if any(p is None for p in (decay, first, *am, *fm)) or decay.dtype != x.dtype:
+        if any(p is None or p.numel() != C or p.get_device() != x.get_device() for p in (decay, first, *am, *fm)) or decay.dtype != x.dtype:
             return None
         w["w"], w["u"] = eval_cached(att, "wu", (decay, first), T,
                                      lambda: ((decay / T).float().contiguous(), (first / T).float().contiguous()))
