@@ -289,3 +289,16 @@ def test_backward_of_a_cut_sequence_with_a_decay_out_of_range(ops, dtype):
             tol = 2e-3 if dtype == torch.float32 else 1e-2               # gw at the file's tolerance; bf16 results round
             assert rel_err(a.float().cpu().numpy(), b.float().cpu().numpy()) <= tol, name
         assert rel_err(got[4].cpu().numpy(), want[4].cpu().numpy()) <= 1e-4
+
+
+@pytest.mark.gpu
+def test_results_passed_in_are_fp32_whatever_types_are_asked_for():
+    import vision_rwkv_amd as ops
+    torch.manual_seed(2)
+    B, T, H = 2, 65, 2
+    mk = lambda: torch.randn(B, T, 64 * H, device="cuda").bfloat16()
+    r, k, v, w, u, gy = mk(), mk(), mk(), mk() - 4, torch.randn(H, 64, device="cuda"), torch.randn(B, T, 64 * H, device="cuda")
+    want = ops.wkv6_backward(B, T, 64 * H, H, r, k, v, w, u, gy)
+    out = [torch.full_like(t, float("nan")) for t in want]
+    ops.wkv6_backward(B, T, 64 * H, H, r, k, v, w, u, gy, out=out, like_inputs=True)
+    assert all(torch.equal(a, b) for a, b in zip(out, want))

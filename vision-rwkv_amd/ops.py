@@ -220,7 +220,9 @@ def wkv6_forward(B, T, C, H, r, k, v, w, u, w_is_ew=False, out=None, whole=False
 def wkv6_backward(B, T, C, H, r, k, v, w, u, gy, w_is_ew=False, out=None, like_inputs=False):
     """Extension-level entry (wkv6_op.cpp:10-12): returns (gr, gk, gv, gw) as (B,T,C) fp32 and gu as
     (H,64) fp32 (already summed over the batch); gw is the gradient w.r.t. the raw decay logit.
-    like_inputs: gr, gk, gv, gw of their inputs' types, rounded from the fp32 sums by the kernel."""
+    like_inputs: gr, gk, gv, gw of their inputs' types, rounded from the fp32 sums by the kernel (results passed in as `out`
+    are fp32 throughout)."""
+    like_inputs = like_inputs and out is None
     for t, n in ((r, "r"), (k, "k"), (v, "v"), (w, "w"), (u, "u"), (gy, "gy")):
         _check_input(t, n)
     if tuple(r.shape) != (B, T, C) or any(x.shape != r.shape for x in (k, v, w, gy)):
