@@ -927,6 +927,8 @@ def test_table_resize_of_a_batch_of_cotangents(adjoint, monkeypatch):
     y = ops._TableResize.apply(t, src, dst, adjoint)
     gs = torch.randn(3, 1, m, 4)
     batched, = torch.autograd.grad(y, t, gs, is_grads_batched=True, retain_graph=True)
+    mapped = torch.vmap(lambda g: torch.autograd.grad(y, t, g, retain_graph=True)[0])(gs)
+    assert torch.equal(mapped, batched)
     for b, g in zip(batched, gs):
         single, = torch.autograd.grad(y, t, g, retain_graph=True)
         assert torch.allclose(b, single, rtol=1e-5, atol=1e-5)

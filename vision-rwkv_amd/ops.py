@@ -683,12 +683,17 @@ class _TableResize(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         src, dst, adjoint = ctx.meta
-        resize = _table_resize_ops if batched_cotangent(g) else _TableResize.apply
-        return resize(g, src, dst, not adjoint), None, None, None
+        return _TableResize.of(g)(g, src, dst, not adjoint), None, None, None
 
     @staticmethod
     def jvp(ctx, t, *_):
-        return _TableResize.apply(t, *ctx.meta)
+        return _TableResize.of(t)(t, *ctx.meta)
+
+    @staticmethod
+    def of(t):
+        """The map for a cotangent or tangent: tensor ops for a batch of them of either kind and wherever else t may not have
+        memory of its own or a function of this class may not be applied."""
+        return _table_resize_ops if batched_cotangent(t) or _transformed() else _TableResize.apply
 
 
 def _table_resize_ops(table, src, dst, adjoint):
