@@ -176,3 +176,37 @@ def test_cut_sequence_with_a_decay_out_of_range(ops):
     with ops.option("wkv6_segments", 3):
         y, *inputs = run(ops, r, k, v, w, u, 2)
     assert rel_err(y, clib.wkv6_fwd(*inputs, u, 2)) <= TOL
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T", [300, 577, 1056, 1057])
+def test_one_rule_cuts_sequences_with_and_without_gradients(ops, T, dtype):
+    """The call that autograd records, the same call under no_grad with the bonus as a parameter, and the plain entry run the
+    same kernels on the same segments: bit-identical y."""
+    H = 3
+    assert ops.lib().vrwkv_wkv6_fwd_workspace_bytes(1, T, 64 * H, H) > 0
+    r, k, v, w, u = (torch.from_numpy(x).cuda() for x in gen(1, T, H, seed=T, w_mean=-3.0, w_std=0.5))
+    r, k, v, w = (x.to(dtype) for x in (r, k, v, w))
+    u = torch.nn.Parameter(u)
+    want = ops.wkv6_forward(1, T, 64 * H, H, r, k, v, w, u.detach())
+    trained = ops.RUN_CUDA_RWKV6(1, T, 64 * H, H, r.requires_grad_(), k, v, w, u)
+    with torch.no_grad():
+        evaluated = ops.RUN_CUDA_RWKV6(1, T, 64 * H, H, r, k, v, w, u)
+    assert trained.grad_fn is not None and torch.equal(trained, want) and torch.equal(evaluated, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T", [196, 256])
+def test_results_of_a_sequence_of_up_to_256_tokens_do_not_depend_on_the_batch(ops, T, dtype):
+    H, B = 2, 40
+    x = [torch.from_numpy(a).cuda() for a in gen(B, T, H, seed=T, w_mean=-3.0, w_std=0.5)]
+    u = x.pop()
+    x = [a.to(dtype).requires_grad_() for a in x]
+    y = ops.RUN_CUDA_RWKV6(B, T, 64 * H, H, *x, u)
+    gy = torch.randn_like(y)
+    grads = torch.autograd.grad(y, x, gy)
+    for b in (0, B - 1):
+        one = [a.detach()[b:b + 1].requires_grad_() for a in x]
+        yb = ops.RUN_CUDA_RWKV6(1, T, 64 * H, H, *one, u)
+        assert torch.equal(yb[0], y[b])
+        assert all(torch.equal(p[0], q[b]) for p, q in zip(torch.autograd.grad(yb, one, gy[b:b + 1].contiguous()), grads))
