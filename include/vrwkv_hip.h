@@ -110,8 +110,9 @@ int vrwkv_biwkv_bwd(const float* w, const float* u, const void* k, const void* v
  *              the `ew = -exp(w)` of WKV_6.forward (vrwkv6.py:48);
  * w_is_ew = 1: w already holds ew = -exp(w_raw), as the reference extension receives it.
  * State and accumulation are fp32.  No limit on T (T*C < 2^29).  workspace: the size function returns 0 unless the call has
- * few, long sequences, which are then cut into segments that exchange their states through it; 16-byte aligned.  It may
- * be NULL (or too small) for every call: the sequences then run uncut. */
+ * few, long sequences, which are then cut into segments that exchange their states through it.  It may be NULL (or too small,
+ * or not on 16 bytes) for every call: the sequences then run uncut, as they do when 16-bit k, v or w are not on 4 bytes.  Every
+ * tensor: aligned to its elements. */
 size_t vrwkv_wkv6_fwd_workspace_bytes(int B, int T, int C, int H);
 int vrwkv_wkv6_fwd(const void* r, const void* k, const void* v, const void* w, const float* u,
                    float* y, int B, int T, int C, int H, int rkv_dtype, int w_dtype, int w_is_ew,
@@ -135,7 +136,9 @@ int vrwkv_wkv6_fwd_phases(const void* r, const void* k, const void* v, const voi
  *    .../cuda_v6/wkv6_cuda.cu:355-362, kernels :99-346), without its T <= 256 limit.
  * r, k, v, w, u as in vrwkv_wkv6_fwd; gy, gr, gk, gv, gw: (B,T,C) fp32, fully overwritten; gw is the
  * gradient w.r.t. the raw decay logit (wkv6_cuda.cu:248,277); gu: (H,64) fp32 already summed over
- * the batch (the reference returns (B,C) and sums in Python, vrwkv6.py:69). */
+ * the batch (the reference returns (B,C) and sums in Python, vrwkv6.py:69).  Every tensor aligned to its elements, the
+ * workspace to 4 bytes (VRWKV_INVALID_ARG otherwise); sequences run uncut where it is not on 16 bytes, or 16-bit r, k, v or w
+ * not on 4. */
 size_t vrwkv_wkv6_bwd_workspace_bytes(int B, int T, int C, int H);
 int vrwkv_wkv6_bwd(const void* r, const void* k, const void* v, const void* w, const float* u,
                    const float* gy, float* gr, float* gk, float* gv, float* gw, float* gu,

@@ -132,6 +132,23 @@ def test_elementwise_entry_points_validate_without_device(lib):
     assert gb(one, one, one, one, one, one, one, one, 4, 128, 64, 1e-5, 0, 1, None, 0, None) == 5     # workspace missing
 
 
+def test_wkv6_backward_refuses_misaligned_pointers_without_device(lib):
+    """Each tensor off its element size, and a workspace off 4 bytes, before anything is launched."""
+    B, T, C, H = 1, 300, 64, 1
+    for fn, like in ((lib.vrwkv_wkv6_bwd, False), (lib.vrwkv_wkv6_bwd_like, True)):
+        for rkv, w in ((0, 0), (1, 0), (1, 1), (2, 2)):
+            es, ws = (4 if rkv == 0 else 2), (4 if w == 0 else 2)
+            out, outw = (es, ws) if like else (4, 4)
+            #          r   k   v   w   u  gy gr   gk   gv   gw    gu workspace
+            elements = [es, es, es, ws, 4, 4, out, out, out, outw, 4, 4]
+            need = lib.vrwkv_wkv6_bwd_like_workspace_bytes(B, T, C, H, rkv, w) if like else lib.vrwkv_wkv6_bwd_workspace_bytes(B, T, C, H)
+            for bad in range(len(elements)):
+                p = [ctypes.c_void_p(4096 + (elements[i] // 2 if i == bad else 0)) for i in range(len(elements))]
+                if fn(*[ctypes.cast(x, t) for x, t in zip(p[:11], fn.argtypes)], B, T, C, H, rkv, w, 0, p[11], need, None) != 1:
+                    raise AssertionError((like, rkv, w, bad))
+                assert b"aligned" in lib.vrwkv_last_error()
+
+
 def test_python_boundary_errors_without_device():
     import torch
     import vision_rwkv_amd as ops

@@ -7,6 +7,8 @@ closed forms those reduce to (no oracle call is needed for them: the expected va
   wkv6,  T = 2: y_0 = (r_0 . (u k_0)) v_0 + (r_0 . k_1) v_1  (adjacent tokens: empty decay product).
 Tolerances: 1e-4 fp32, 1e-2 16-bit I/O (Bi-WKV); 1e-3 (wkv6) of max(|ref|, rms(ref)).
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -159,6 +161,69 @@ def test_wkv6_tensors_that_are_not_16_byte_aligned(ops):
     assert torch.equal(y1, y0)
     for a, b in zip(g1, g0):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype,w_dtype", [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.float16, torch.float16),
+                                           (torch.float32, torch.float32)])
+@pytest.mark.parametrize("offset", [1, 2])
+def test_wkv6_cut_sequences_that_are_not_16_byte_aligned(ops, offset, dtype, w_dtype):
+    """Three segments asked for: 16-bit rows one element into their allocation run uncut (bit for bit like the aligned uncut call),
+    on 4 bytes and in fp32 cut like the aligned ones; each tensor alone decides."""
+    B, T, H = 2, 100, 2
+    C = H * 64
+    g = torch.Generator(device="cpu").manual_seed(3)
+    r, k, v = (torch.randn(B, T, C, generator=g).to(DEV).to(dtype) for _ in range(3))
+    w = (torch.randn(B, T, C, generator=g) * 0.5 - 3).to(DEV).to(w_dtype)
+    u = (0.1 * torch.randn(H, 64, generator=g)).to(DEV)
+    gy = torch.randn(B, T, C, generator=g).to(DEV)
+    x = [r, k, v, w]
+    fwd, bwd = ops.wkv6_forward, lambda *a: ops.wkv6_backward(*a, gy, like_inputs=True)
+    results = {}
+    for segments in (1, 3):
+        with ops.option("wkv6_segments", segments):
+            results[segments] = (fwd(B, T, C, H, *x, u), bwd(B, T, C, H, *x, u))
+    assert not torch.equal(results[1][0], results[3][0])
+    with ops.option("wkv6_segments", 3):
+        for moved in range(4):
+            y = [_offset_copy(t, offset) if i == moved else t for i, t in enumerate(x)]
+            uncut = offset == 1 and y[moved].element_size() == 2
+            want_y = results[1 if uncut and moved > 0 else 3][0]                  # (the forward's state kernel does not read r)
+            want_g = results[1 if uncut else 3][1]
+            assert torch.equal(fwd(B, T, C, H, *y, u), want_y), moved
+            assert all(torch.equal(a, b) for a, b in zip(bwd(B, T, C, H, *y, u), want_g)), moved
+        assert torch.equal(fwd(B, T, C, H, *x, _offset_copy(u)), results[3][0])
+        assert all(torch.equal(a, b) for a, b in zip(ops.wkv6_backward(B, T, C, H, *x, u, _offset_copy(gy), like_inputs=True), results[3][1]))
+
+
+@pytest.mark.parametrize("segments", [1, 3])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_wkv6_backward_results_and_workspace_that_are_not_16_byte_aligned(ops, dtype, segments):
+    """Through the C entry: 16-bit results one element into their allocations, and a workspace on 4 bytes (then uncut)."""
+    B, T, H = 2, 100, 2
+    C, L = H * 64, ops.lib()
+    g = torch.Generator(device="cpu").manual_seed(4)
+    r, k, v, w = (torch.randn(B, T, C, generator=g).to(DEV).to(dtype) for _ in range(4))
+    w -= 3
+    u, gy = (0.1 * torch.randn(H, 64, generator=g)).to(DEV), torch.randn(B, T, C, generator=g).to(DEV)
+    w[1, 40:44, 64:] = 4                                     # one sequence beyond the chunked kernel's range
+    with ops.option("wkv6_segments", 1):
+        uncut = ops.wkv6_backward(B, T, C, H, r, k, v, w, u, gy, like_inputs=True)
+    code = 1 if dtype == torch.bfloat16 else 2
+    with ops.option("wkv6_segments", segments):
+        cut = ops.wkv6_backward(B, T, C, H, r, k, v, w, u, gy, like_inputs=True)
+        need = L.vrwkv_wkv6_bwd_like_workspace_bytes(B, T, C, H, code, code)
+        for out_off, ws_off in ((0, 0), (1, 0), (2, 0), (0, 4), (1, 4)):
+            outs = [torch.full((t.numel() + 4,), float("nan"), dtype=t.dtype, device=DEV) for t in cut]
+            grads = [o[out_off:out_off + t.numel()] for o, t in zip(outs[:4], cut)] + [outs[4][:cut[4].numel()]]
+            ws = torch.empty(need + 16, dtype=torch.uint8, device=DEV)[ws_off:]
+            ptr = lambda t, i: ctypes.cast(t.data_ptr(), L.vrwkv_wkv6_bwd_like.argtypes[i])
+            rc = L.vrwkv_wkv6_bwd_like(*[ptr(t, i) for i, t in enumerate((r, k, v, w, u, gy, *grads))], B, T, C, H, code, code, 0,
+                                       ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream)
+            assert rc == 0, L.vrwkv_last_error()
+            want = uncut if ws_off else cut
+            for a, o, b in zip(grads, outs, want):
+                assert torch.equal(a.view(b.shape), b), (out_off, ws_off)
+                assert int(torch.isnan(o).sum()) == 4                       # nothing written beside them
 
 
 def test_tensors_larger_than_4_gib(ops):

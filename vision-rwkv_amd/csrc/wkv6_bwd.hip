@@ -69,11 +69,11 @@ struct Plan {
     int nseg;
     size_t n, sums, states, bytes;                       // elements of a tensor; floats in front of `a`; bytes of the state block
 };
-Plan plan(int B, int T, int C, int H, int rkv_dtype, int w_dtype, int grad_dtypes_of_inputs) {
+Plan plan(int B, int T, int C, int H, int rkv_dtype, int w_dtype, int grad_dtypes_of_inputs, bool cut = true) {
     Plan p;
     p.out16 = grad_dtypes_of_inputs && rkv_dtype != VRWKV_F32;
     p.w16 = grad_dtypes_of_inputs && w_dtype != VRWKV_F32;
-    p.nseg = segments(B, T, H);
+    p.nseg = cut ? segments(B, T, H) : 1;
     p.n = (size_t)B * T * C;
     p.sums = (p.out16 ? 3 * p.n : 0) + (p.w16 ? p.n : 0);
     p.states = seg_bytes((long long)B * H, p.nseg, BWD_SEG_FLOATS);
@@ -96,13 +96,22 @@ int launch_all(const void* r, const void* k, const void* v, const void* w, const
     A.a = take(p.n);
     A.gu_part = take((size_t)B * p.nseg * C);
     q = ws + (((size_t)(q - ws) + 3) & ~(size_t)3);      // states: 16-byte aligned
-    A.T = T; A.C = C; A.H = H; A.sequences = B * H; A.nseg = p.nseg; A.out16 = p.out16; A.w16 = p.w16;
+    // gv leaves the sweep in pieces of four channels; where its 16-bit rows do not lie on 4 bytes, the sums are rounded afterwards
+    const bool apart = p.out16 && ((uintptr_t)gv & 3);
+    if (apart) { A.gr = A.pr; A.gk = A.pk; A.gv = A.pv; }
+    A.T = T; A.C = C; A.H = H; A.sequences = B * H; A.nseg = p.nseg; A.out16 = p.out16 && !apart; A.w16 = p.w16;
     A.seg_ws = q;
     int* flags = reinterpret_cast<int*>(q + (size_t)A.sequences * p.nseg * BWD_SEG_FLOATS);
     A.seg_flags = flags;
     const IO *rr = static_cast<const IO*>(r), *kk = static_cast<const IO*>(k), *vv = static_cast<const IO*>(v);
     const WT* ww = static_cast<const WT*>(w);
     int part_rows = B;
+    auto round_rkv = [&]() {
+        const dim3 rg((unsigned)((p.n + 1023) / 1024 < 8192 ? (p.n + 1023) / 1024 : 8192)), block(256);
+        hipLaunchKernelGGL((round_kernel<IO>), rg, block, 0, st, A.pr, static_cast<IO*>(gr), p.n);
+        hipLaunchKernelGGL((round_kernel<IO>), rg, block, 0, st, A.pk, static_cast<IO*>(gk), p.n);
+        hipLaunchKernelGGL((round_kernel<IO>), rg, block, 0, st, A.pv, static_cast<IO*>(gv), p.n);
+    };
     if (!option(OPT_WKV6_BWD_SCALAR)) {                  // the option forces the sequential sweeps (testing)
         unsigned grid = (unsigned)A.sequences;
         if (p.nseg > 1) {
@@ -113,6 +122,7 @@ int launch_all(const void* r, const void* k, const void* v, const void* w, const
         }
         hipLaunchKernelGGL((wkv6_bwd_sweep_kernel<IO, WT, EW>), dim3(grid), dim3(512), 0, st, A);
         part_rows = B * p.nseg;
+        if (apart) round_rkv();
     } else {
         const dim3 grid(A.sequences), block(256);
         // descending pass first (writes), ascending pass second (accumulates), as in the forward
@@ -123,11 +133,7 @@ int launch_all(const void* r, const void* k, const void* v, const void* w, const
         hipLaunchKernelGGL((wkv6_bwd_seq_g<IO, WT, 0, EW>), grid, block, 0, st, rr, kk, vv, ww, u, gy, A.a, A.pk, A.pw, T, C, H);
         hipLaunchKernelGGL((wkv6_bwd_seq_v<IO, WT, 0, EW>), grid, block, 0, st, rr, kk, ww, u, gy, A.pv, T, C, H);
         const dim3 rg((unsigned)((p.n + 1023) / 1024 < 8192 ? (p.n + 1023) / 1024 : 8192));
-        if (p.out16) {
-            hipLaunchKernelGGL((round_kernel<IO>), rg, block, 0, st, A.pr, static_cast<IO*>(gr), p.n);
-            hipLaunchKernelGGL((round_kernel<IO>), rg, block, 0, st, A.pk, static_cast<IO*>(gk), p.n);
-            hipLaunchKernelGGL((round_kernel<IO>), rg, block, 0, st, A.pv, static_cast<IO*>(gv), p.n);
-        }
+        if (p.out16) round_rkv();
         if (p.w16) hipLaunchKernelGGL((round_kernel<WT>), rg, block, 0, st, A.pw, static_cast<WT*>(gw), p.n);
     }
     // torch.sum(gu, 0), vrwkv6.py:69
@@ -163,7 +169,16 @@ int backward(const void* r, const void* k, const void* v, const void* w, const f
         set_error("wkv6_bwd: tensor too large");
         return VRWKV_UNSUPPORTED_SHAPE;
     }
-    const Plan p = plan(B, T, C, H, rkv_dtype, w_dtype, like_inputs);
+    const size_t es = rkv_dtype == VRWKV_F32 ? 4 : 2, ws_el = w_dtype == VRWKV_F32 ? 4 : 2;
+    if ((((uintptr_t)r | (uintptr_t)k | (uintptr_t)v) & (es - 1)) || ((uintptr_t)w & (ws_el - 1)) ||
+        (((uintptr_t)u | (uintptr_t)gy | (uintptr_t)gu | (uintptr_t)workspace) & 3) ||
+        (((uintptr_t)gr | (uintptr_t)gk | (uintptr_t)gv) & ((like_inputs ? es : 4) - 1)) || ((uintptr_t)gw & ((like_inputs ? ws_el : 4) - 1))) {
+        set_error("wkv6_bwd: pointers must be aligned to their element size, the workspace to 4 bytes");
+        return VRWKV_INVALID_ARG;
+    }
+    // the state kernel reads pairs of elements (4-byte accesses of 16-bit rows) and keeps its states in 16-byte pieces
+    const bool cut = !(((uintptr_t)r | (uintptr_t)k | (uintptr_t)v | (uintptr_t)w) & 3) && !((uintptr_t)workspace & 15);
+    const Plan p = plan(B, T, C, H, rkv_dtype, w_dtype, like_inputs, cut);
     if (!workspace || workspace_bytes < p.bytes) {
         set_error("wkv6_bwd: workspace of %zu bytes required (got %zu)", p.bytes, workspace ? workspace_bytes : (size_t)0);
         return VRWKV_WORKSPACE_TOO_SMALL;

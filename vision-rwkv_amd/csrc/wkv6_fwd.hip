@@ -74,7 +74,8 @@ int launch_chunked(const void* r, const void* k, const void* v, const void* w, c
     const WT* ww = static_cast<const WT*>(w);
     const long long sequences = (long long)B * H;
     int nseg = segments(B, T, H);
-    if (!ws || ws_bytes < seg_bytes(sequences, nseg, SEG_FLOATS) || ((uintptr_t)ws & 15)) nseg = 1;
+    // (the state kernel reads pairs of elements: 4-byte accesses of 16-bit rows; wider accesses need no more than 4 bytes either)
+    if (!ws || ws_bytes < seg_bytes(sequences, nseg, SEG_FLOATS) || ((uintptr_t)ws & 15) || (((uintptr_t)k | (uintptr_t)v | (uintptr_t)w) & 3)) nseg = 1;
     float* states = nullptr;
     int* flags = nullptr;
     unsigned grid = (unsigned)sequences;
