@@ -149,6 +149,16 @@ def test_wkv6_backward_refuses_misaligned_pointers_without_device(lib):
                 assert b"aligned" in lib.vrwkv_last_error()
 
 
+def test_more_sequences_than_a_grid_holds_are_not_cut(lib):
+    """A forced number of segments does not apply to more sequences than the fold kernel's grid has rows."""
+    import vision_rwkv_amd as ops
+    with ops.option("wkv6_segments", 3):
+        assert lib.vrwkv_wkv6_fwd_workspace_bytes(65535, 100, 64, 1) > 0
+        assert lib.vrwkv_wkv6_fwd_workspace_bytes(65536, 100, 64, 1) == 0
+        cut, uncut = (lib.vrwkv_wkv6_bwd_workspace_bytes(B, 100, 64, 1) / B for B in (65535, 65536))
+    assert uncut == 101 * 64 * 4 and cut > 2 * 4 * 64 * 64 * 4         # two of two chunks each
+
+
 def test_python_boundary_errors_without_device():
     import torch
     import vision_rwkv_amd as ops

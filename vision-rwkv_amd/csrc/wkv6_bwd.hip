@@ -56,11 +56,11 @@ void round_kernel(const float* __restrict__ x, OT* __restrict__ y, size_t n) {
 // Segments per sequence of a call (1: not cut); OPT_WKV6_SEGMENTS forces a number (testing).
 int segments(int B, int T, int H) {
     const int nchunk = (T + LC - 1) / LC, forced = option(OPT_WKV6_SEGMENTS);
-    if (forced > 0) {
+    if (forced > 0 && (long long)B * H <= SEG_SEQUENCES) {
         const int n = forced < nchunk ? forced : nchunk, cps = (nchunk + n - 1) / n;
         return (nchunk + cps - 1) / cps;
     }
-    return wkv6_segments((long long)B * H, nchunk, device_cus(), SEG_BWD);
+    return forced > 0 ? 1 : wkv6_segments((long long)B * H, nchunk, device_cus(), SEG_BWD);
 }
 
 // Workspace: [fp32 sums gr, gk, gv (16-bit results only)] [gw (16-bit decay logits only)] [a] [partial gu] [states] [flags]

@@ -37,11 +37,11 @@ int validate(int B, int T, int C, int H, int rkv_dtype, int w_dtype) {
 // Segments per sequence of a call (1: not split); OPT_WKV6_SEGMENTS forces a number (testing).
 int segments(int B, int T, int H) {
     const int nchunk = (T + LC - 1) / LC, forced = option(OPT_WKV6_SEGMENTS);
-    if (forced > 0) {
+    if (forced > 0 && (long long)B * H <= SEG_SEQUENCES) {
         const int n = forced < nchunk ? forced : nchunk, cps = (nchunk + n - 1) / n;
         return (nchunk + cps - 1) / cps;
     }
-    return wkv6_segments((long long)B * H, nchunk, device_cus(), SEG_FWD);
+    return forced > 0 ? 1 : wkv6_segments((long long)B * H, nchunk, device_cus(), SEG_FWD);
 }
 
 template <typename IO, typename WT>

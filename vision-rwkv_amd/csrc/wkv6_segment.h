@@ -21,6 +21,7 @@ namespace vrwkv {
 namespace wkv6_detail {
 
 constexpr int SEG_MAX = 64;                          // segments per sequence (one flag per lane of a wave)
+constexpr int SEG_SEQUENCES = 65535;                 // sequences of a cut call (the fold kernel's grid; by the rule below, 4 per CU at most)
 constexpr int SEG_STATE = HN * HN;                   // floats of one state
 constexpr int SEG_FLOATS = 2 * SEG_STATE + HN;       // forward: up state, down state, total decay per channel
 constexpr int BWD_SEG_FLOATS = 4 * SEG_STATE + HN;   // backward: S up, G up, S down, G down, total decay per channel
