@@ -719,6 +719,23 @@ def test_native_v6_block_sees_writes_through_data(key_norm, cls):
     assert not torch.equal(got, before) and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("v6,dtype,M,C,called", [
+    (False, torch.bfloat16, 196, 192, True), (False, torch.bfloat16, 3136, 384, True), (False, torch.bfloat16, 12544, 512, True),
+    (False, torch.bfloat16, 784, 768, True), (False, torch.float16, 1568, 768, True), (False, torch.bfloat16, 392, 1024, True),
+    (False, torch.bfloat16, 784, 1024, True), (False, torch.bfloat16, 3136, 1024, True), (False, torch.bfloat16, 6272, 1024, False),
+    (False, torch.bfloat16, 12544, 768, False), (True, torch.bfloat16, 6272, 768, True), (True, torch.bfloat16, 3136, 1024, True),
+    (True, torch.float16, 6272, 1024, True), (True, torch.bfloat16, 12544, 1024, False),
+    (False, torch.float32, 3136, 384, True), (False, torch.float32, 6272, 512, True), (False, torch.float32, 392, 768, True),
+    (False, torch.float32, 784, 768, True), (False, torch.float32, 1568, 768, False), (False, torch.float32, 3136, 768, True),
+    (False, torch.float32, 784, 1024, False), (False, torch.float32, 1568, 1024, True), (True, torch.float32, 784, 768, True),
+    (True, torch.float32, 1568, 768, True), (True, torch.float32, 1568, 1024, True), (False, torch.bfloat16, 1 << 21, 64, False)])
+def test_native_blocks_where_they_measured_faster(v6, dtype, M, C, called):
+    """The rule against the measured points, called eagerly (the last one: 32-bit offsets)."""
+    from vision_rwkv_amd.backbone import _native_size
+    x = torch.empty(1, M, C, dtype=dtype, device="meta")
+    assert _native_size(x, 4 * C, v6) == called
+
+
 def _as_buffer(module, name):
     value = getattr(module, name).detach()
     delattr(module, name)

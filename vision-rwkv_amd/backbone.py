@@ -188,18 +188,25 @@ def _layer_norm(ln, x):
     return row_fuse(x, None, ln.weight, ln.bias, None, PRE_NONE, POST_NONE, ln.eps)
 
 
-# Multiplications per (C, C) projection up to which a block runs as one native call (vrwkv_block_fwd).  Twelve bf16 blocks of
-# tokens x channels, operator by operator -> native, eager | replayed as a graph (GPU time alone), in us:
-#   VRWKV   196 x 192 4037 -> 781 | 991 -> 499      3136 x 384 3594 -> 1273 | 1427 -> 1257    784 x 768 3602 -> 1377 | 1428 -> 1360
-#           3136 x 768 3623 -> 2115 | 1992 -> 2115   6272 x 768 3714 -> 3121 | 3163 -> 3062   12544 x 768 5077 -> 5546
-#           1568 x 1024 3673 -> 2296 | 1977 -> 2282  6272 x 1024 3823 -> 4252
-#   VRWKV6  196 x 192 6496 -> 1107 | 1536 -> 900    784 x 768 6055 -> 1950 | 2287 -> 1920    12544 x 768 7919 -> 7880 | 7897 -> 7854
-# The host sets the pace of the operators up to about 4 (7) ms; the GPU work alone is a few percent behind the library's larger
-# tiles from about 1000 tokens of 768 or more channels on, so the line is where the eager call stops gaining.
-NATIVE_BLOCK_WORK, NATIVE_BLOCK_WORK_V6 = 3_800_000_000, 7_500_000_000
-# fp32: 196 x 192 4773 -> 747, 3136 x 384 3740 -> 2485 | 2448 -> 2463, 392 x 768 3697 -> 1807 | 1920 -> 1792, but 784 x 768 2307 / 2535
-# and 1568 x 768 3769 -> 3937 | 3415 -> 3919; from 3136 x 768 on (7064 / 6371, 6272 x 768 12392 / 11386) the library is behind again.
-NATIVE_BLOCK_WORK_FP32 = (420_000_000, 1_700_000_000)                      # up to the first, and from the second on
+# Whether a block runs as one native call (vrwkv_block_fwd), by M C C, the multiplications of a (C, C) projection on M tokens.
+# Operator by operator the host takes 290 us a block (VRWKV6 490) and sets the pace up to some thousand tokens; the native call
+# takes it 58 (83), so called eagerly it gains until its time on the GPU reaches the host's or the library's, whichever is longer.
+# Up to 512 channels it is ahead on the GPU as well, at every size measured.  Twelve blocks of tokens x channels, operators ->
+# native, eager | replayed, in us:
+#   VRWKV  bf16  784 x 768   3535 -> 1371 | 1415 -> 1362      1568 x 768   3532 -> 1704 | 1597 -> 1693      392 x 1024 3512 -> 1377 | 1508 -> 1375
+#                784 x 1024  3506 -> 1874 | 1648 -> 1868      3136 x 1024  3514 -> 2813 | 2466 -> 2806      6272 x 768 3566 -> 2964 | 3047 -> 2966
+#                6272 x 1024 3665 -> 4118 | 3674 -> 4109      12544 x 768  4892 -> 5334 | 4866 -> 5316      196 x 192  3529 ->  702 | 1492 ->  469
+#                3136 x 512  3528 -> 1452 | 1587 -> 1444      12544 x 512  3530 -> 2944 | 3287 -> 2926      12544 x 192 3521 -> 1388 | 1473 -> 1379
+#   VRWKV6 bf16  6272 x 768  6010 -> 4367 | 4720 -> 4335      3136 x 1024  5971 -> 3795 | 3830 -> 3766      6272 x 1024 5938 -> 5711 | 5628 -> 5680
+#                12544 x 768 7758 -> 7692 | 7659 -> 7660      12544 x 1024 8965 -> 10822 | 8879 -> 10797
+# fp32: the library's 1568 x 768 and 784 x 1024 products fill the chip exactly and are ahead; half and twice the tokens they are behind.
+#   VRWKV        392 x 768   3446 -> 1761 | 1892 -> 1760      784 x 768    3476 -> 2494 | 2274 -> 2485      1568 x 768 3481 -> 3915 | 3326 -> 3907
+#                3136 x 768  7010 -> 6330 | 6990 -> 6325      784 x 1024   3539 -> 3860 | 3394 -> 3853      1568 x 1024 5558 -> 5423 | 5524 -> 5411
+#                3136 x 384  3490 -> 2452 | 2400 -> 2438      6272 x 384   5768 -> 4026 | 5742 -> 3995      3136 x 512 3799 -> 3322 | 3752 -> 3292
+#   VRWKV6       784 x 768   5810 -> 3363 | 3357 -> 3339      1568 x 768   5825 -> 4994 | 4637 -> 4960      1568 x 1024 7193 -> 6854 | 7101 -> 6826
+NATIVE_NARROW = 512                                   # channels up to which the native call is ahead on the GPU as well
+NATIVE_BLOCK_WORK = {(False, False): 3_800_000_000, (False, True): 7_500_000_000, (True, False): 600_000_000, (True, True): 1_500_000_000}   # (fp32, VRWKV6)
+NATIVE_BLOCK_WORK_FP32 = 1_500_000_000                # fp32: native again from here on
 
 
 def _native_size(x, hidden, v6):
@@ -207,10 +214,10 @@ def _native_size(x, hidden, v6):
     M, C = x.shape[0] * x.shape[1], x.shape[2]
     if M * max(C, hidden, 160) * x.element_size() >= 1 << 30:
         return False
-    if x.dtype == torch.float32:
-        lo, hi = NATIVE_BLOCK_WORK_FP32
-        return not lo < M * C * C < hi
-    return M * C * C <= (NATIVE_BLOCK_WORK_V6 if v6 else NATIVE_BLOCK_WORK)
+    work, fp32 = M * C * C, x.dtype == torch.float32
+    if fp32 and (C <= NATIVE_NARROW or work >= NATIVE_BLOCK_WORK_FP32):
+        return True
+    return work <= NATIVE_BLOCK_WORK[fp32, v6]
 
 
 def _as_built(module, kind):
