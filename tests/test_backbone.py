@@ -719,21 +719,60 @@ def test_native_v6_block_sees_writes_through_data(key_norm, cls):
     assert not torch.equal(got, before) and torch.equal(got, want)
 
 
-@pytest.mark.parametrize("v6,dtype,M,C,called", [
-    (False, torch.bfloat16, 196, 192, True), (False, torch.bfloat16, 3136, 384, True), (False, torch.bfloat16, 12544, 512, True),
-    (False, torch.bfloat16, 784, 768, True), (False, torch.float16, 1568, 768, True), (False, torch.bfloat16, 392, 1024, True),
-    (False, torch.bfloat16, 784, 1024, True), (False, torch.bfloat16, 3136, 1024, True), (False, torch.bfloat16, 6272, 1024, False),
-    (False, torch.bfloat16, 12544, 768, False), (True, torch.bfloat16, 6272, 768, True), (True, torch.bfloat16, 3136, 1024, True),
-    (True, torch.float16, 6272, 1024, True), (True, torch.bfloat16, 12544, 1024, False),
-    (False, torch.float32, 3136, 384, True), (False, torch.float32, 6272, 512, True), (False, torch.float32, 392, 768, True),
-    (False, torch.float32, 784, 768, True), (False, torch.float32, 1568, 768, False), (False, torch.float32, 3136, 768, True),
-    (False, torch.float32, 784, 1024, False), (False, torch.float32, 1568, 1024, True), (True, torch.float32, 784, 768, True),
-    (True, torch.float32, 1568, 768, True), (True, torch.float32, 1568, 1024, True), (False, torch.bfloat16, 1 << 21, 64, False)])
-def test_native_blocks_where_they_measured_faster(v6, dtype, M, C, called):
-    """The rule against the measured points, called eagerly (the last one: 32-bit offsets)."""
+@pytest.mark.parametrize("v6,dtype,M,C,called,recorded", [
+    (False, torch.bfloat16, 196, 192, True, True), (False, torch.bfloat16, 3136, 384, True, True), (False, torch.bfloat16, 12544, 512, True, True),
+    (False, torch.bfloat16, 784, 768, True, True), (False, torch.float16, 1568, 768, True, False), (False, torch.bfloat16, 392, 1024, True, True),
+    (False, torch.bfloat16, 784, 1024, True, False), (False, torch.bfloat16, 3136, 1024, True, False), (False, torch.bfloat16, 6272, 1024, False, False),
+    (False, torch.bfloat16, 12544, 768, False, False), (True, torch.bfloat16, 6272, 768, True, True), (True, torch.bfloat16, 3136, 1024, True, True),
+    (True, torch.float16, 6272, 1024, True, False), (True, torch.bfloat16, 12544, 1024, False, False),
+    (False, torch.float32, 3136, 384, True, True), (False, torch.float32, 6272, 512, True, True), (False, torch.float32, 392, 768, True, True),
+    (False, torch.float32, 784, 768, True, False), (False, torch.float32, 1568, 768, False, False), (False, torch.float32, 3136, 768, True, True),
+    (False, torch.float32, 784, 1024, False, False), (False, torch.float32, 1568, 1024, True, True), (True, torch.float32, 784, 768, True, True),
+    (True, torch.float32, 1568, 768, True, False), (True, torch.float32, 1568, 1024, True, True), (False, torch.bfloat16, 1 << 21, 64, False, False)])
+def test_native_blocks_where_they_measured_faster(v6, dtype, M, C, called, recorded, monkeypatch):
+    """The rule against the measured points: called eagerly, and recorded into a graph (the last one: 32-bit offsets)."""
     from vision_rwkv_amd.backbone import _native_size
     x = torch.empty(1, M, C, dtype=dtype, device="meta")
-    assert _native_size(x, 4 * C, v6) == called
+    for capturing, want in ((False, called), (True, recorded)):
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+        assert _native_size(x, 4 * C, v6) == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,C,batch,hw,native", [("v4", 768, 8, (14, 14), False), ("v6", 1024, 8, (28, 28), False), ("v6", 192, 1, (14, 14), True)])
+def test_inference_recorded_into_a_graph(kind, C, batch, hw, native):
+    """A forward recorded after an eager one, where the two take different routes (and where they do not): the tables that the
+    recording forms are not found by a later eager call, and every replay on new images equals the eager call of its route."""
+    from vision_rwkv_amd import ops as impl
+    net = _small_backbone(kind, C, torch.bfloat16, False, False, False, hw)
+    image = lambda: torch.randn(batch, 3, hw[0] * 16, hw[1] * 16, device="cuda").bfloat16()
+
+    def eager(x, fuse):
+        impl.BLOCK_FUSE_ENABLED = fuse
+        try:
+            return net(x)
+        finally:
+            impl.BLOCK_FUSE_ENABLED = True
+
+    with torch.no_grad():
+        x = image()
+        assert net.layers[0]._native(net.embed(x)[0], hw) is not None
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            net(x)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = net(x)
+        first = eager(x, native)                          # before any replay
+        assert bool(torch.isfinite(first).all())
+        for i in range(3):
+            if i:
+                x.copy_(image())
+            graph.replay()
+            torch.cuda.synchronize()
+            want = eager(x, native)
+            assert torch.equal(y, want) and (i or torch.equal(first, want))
 
 
 def _as_buffer(module, name):

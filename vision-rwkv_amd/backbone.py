@@ -42,12 +42,15 @@ def eval_cached(module, name, params, extra, make):
     """Value derived from parameters (a dtype conversion, a stacked table), kept on the module between forward passes
     without autograd and rebuilt when a parameter was written to (its version counter), moved or cast.  The entry holds on to
     the memory it was derived from, so that no later parameter can be found at the same address.  A write through p.data
-    counts as no new version: after one, the next in-place write, cast or move of the parameter brings the value up to date."""
+    counts as no new version: after one, the next in-place write, cast or move of the parameter brings the value up to date.
+    A value made while the stream is recorded into a graph exists when the graph runs, and is not kept."""
     key = (extra,) + tuple((p._version, p.dtype, p.device) for p in params)
     slot = module.__dict__.setdefault("_eval_cache", {})
     hit = slot.get(name)
     if hit is None or hit[0] != key or any(m.data_ptr() != p.data_ptr() for m, p in zip(hit[2], params)):
         hit = (key, make(), [p.detach() for p in params])
+        if params[0].is_cuda and torch.cuda.is_current_stream_capturing():
+            return hit[1]
         slot[name] = hit
     return hit[1]
 
@@ -191,7 +194,9 @@ def _layer_norm(ln, x):
 # Whether a block runs as one native call (vrwkv_block_fwd), by M C C, the multiplications of a (C, C) projection on M tokens.
 # Operator by operator the host takes 290 us a block (VRWKV6 490) and sets the pace up to some thousand tokens; the native call
 # takes it 58 (83), so called eagerly it gains until its time on the GPU reaches the host's or the library's, whichever is longer.
-# Up to 512 channels it is ahead on the GPU as well, at every size measured.  Twelve blocks of tokens x channels, operators ->
+# Recorded into a graph only the time on the GPU counts.  There the native call saves launches and passes over the tokens, and
+# its products are slower than the library's where the contraction is long: 6 to 15 % of a 16-bit block from about 1000 tokens of 768
+# or more channels on.  Up to 512 channels it is ahead at every size measured.  Twelve blocks of tokens x channels, operators ->
 # native, eager | replayed, in us:
 #   VRWKV  bf16  784 x 768   3535 -> 1371 | 1415 -> 1362      1568 x 768   3532 -> 1704 | 1597 -> 1693      392 x 1024 3512 -> 1377 | 1508 -> 1375
 #                784 x 1024  3506 -> 1874 | 1648 -> 1868      3136 x 1024  3514 -> 2813 | 2466 -> 2806      6272 x 768 3566 -> 2964 | 3047 -> 2966
@@ -205,7 +210,9 @@ def _layer_norm(ln, x):
 #                3136 x 384  3490 -> 2452 | 2400 -> 2438      6272 x 384   5768 -> 4026 | 5742 -> 3995      3136 x 512 3799 -> 3322 | 3752 -> 3292
 #   VRWKV6       784 x 768   5810 -> 3363 | 3357 -> 3339      1568 x 768   5825 -> 4994 | 4637 -> 4960      1568 x 1024 7193 -> 6854 | 7101 -> 6826
 NATIVE_NARROW = 512                                   # channels up to which the native call is ahead on the GPU as well
-NATIVE_BLOCK_WORK = {(False, False): 3_800_000_000, (False, True): 7_500_000_000, (True, False): 600_000_000, (True, True): 1_500_000_000}   # (fp32, VRWKV6)
+NATIVE_BLOCK_WORK = {                                 # (fp32, VRWKV6): most work recorded into a graph beyond that width, most work at all
+    (False, False): (600_000_000, 3_800_000_000), (False, True): (4_000_000_000, 7_500_000_000),
+    (True, False): (300_000_000, 600_000_000), (True, True): (600_000_000, 1_500_000_000)}
 NATIVE_BLOCK_WORK_FP32 = 1_500_000_000                # fp32: native again from here on
 
 
@@ -214,10 +221,11 @@ def _native_size(x, hidden, v6):
     M, C = x.shape[0] * x.shape[1], x.shape[2]
     if M * max(C, hidden, 160) * x.element_size() >= 1 << 30:
         return False
-    work, fp32 = M * C * C, x.dtype == torch.float32
-    if fp32 and (C <= NATIVE_NARROW or work >= NATIVE_BLOCK_WORK_FP32):
+    work, fp32, narrow = M * C * C, x.dtype == torch.float32, C <= NATIVE_NARROW
+    if fp32 and (narrow or work >= NATIVE_BLOCK_WORK_FP32):
         return True
-    return work <= NATIVE_BLOCK_WORK[fp32, v6]
+    recorded, called = NATIVE_BLOCK_WORK[fp32, v6]
+    return work <= called and (narrow or work <= recorded or not torch.cuda.is_current_stream_capturing())
 
 
 def _as_built(module, kind):
