@@ -725,7 +725,9 @@ def test_native_v6_block_sees_writes_through_data(key_norm, cls):
     (False, torch.bfloat16, 784, 1024, True, False), (False, torch.bfloat16, 3136, 1024, True, False), (False, torch.bfloat16, 6272, 1024, False, False),
     (False, torch.bfloat16, 12544, 768, False, False), (True, torch.bfloat16, 6272, 768, True, True), (True, torch.bfloat16, 3136, 1024, True, True),
     (True, torch.float16, 6272, 1024, True, False), (True, torch.bfloat16, 12544, 1024, False, False),
-    (False, torch.float32, 3136, 384, True, True), (False, torch.float32, 6272, 512, True, True), (False, torch.float32, 392, 768, True, True),
+    (False, torch.float32, 3136, 384, True, False), (False, torch.float32, 1960, 512, True, False),
+    (False, torch.float32, 1568, 512, True, True), (False, torch.float32, 3136, 448, True, True), (False, torch.float32, 6272, 512, True, True),
+    (True, torch.float32, 2352, 512, True, True), (False, torch.float32, 392, 768, True, True),
     (False, torch.float32, 784, 768, True, False), (False, torch.float32, 1568, 768, False, False), (False, torch.float32, 3136, 768, True, True),
     (False, torch.float32, 784, 1024, False, False), (False, torch.float32, 1568, 1024, True, True), (True, torch.float32, 784, 768, True, True),
     (True, torch.float32, 1568, 768, True, False), (True, torch.float32, 1568, 1024, True, True), (False, torch.bfloat16, 1 << 21, 64, False, False)])

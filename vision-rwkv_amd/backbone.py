@@ -196,7 +196,7 @@ def _layer_norm(ln, x):
 # takes it 58 (83), so called eagerly it gains until its time on the GPU reaches the host's or the library's, whichever is longer.
 # Recorded into a graph only the time on the GPU counts.  There the native call saves launches and passes over the tokens, and
 # its products are slower than the library's where the contraction is long: 6 to 15 % of a 16-bit block from about 1000 tokens of 768
-# or more channels on.  Up to 512 channels it is ahead at every size measured.  Twelve blocks of tokens x channels, operators ->
+# or more channels on.  Up to 512 channels it is ahead in 16 bits.  Twelve blocks of tokens x channels, operators ->
 # native, eager | replayed, in us:
 #   VRWKV  bf16  784 x 768   3535 -> 1371 | 1415 -> 1362      1568 x 768   3532 -> 1704 | 1597 -> 1693      392 x 1024 3512 -> 1377 | 1508 -> 1375
 #                784 x 1024  3506 -> 1874 | 1648 -> 1868      3136 x 1024  3514 -> 2813 | 2466 -> 2806      6272 x 768 3566 -> 2964 | 3047 -> 2966
@@ -204,16 +204,19 @@ def _layer_norm(ln, x):
 #                3136 x 512  3528 -> 1452 | 1587 -> 1444      12544 x 512  3530 -> 2944 | 3287 -> 2926      12544 x 192 3521 -> 1388 | 1473 -> 1379
 #   VRWKV6 bf16  6272 x 768  6010 -> 4367 | 4720 -> 4335      3136 x 1024  5971 -> 3795 | 3830 -> 3766      6272 x 1024 5938 -> 5711 | 5628 -> 5680
 #                12544 x 768 7758 -> 7692 | 7659 -> 7660      12544 x 1024 8965 -> 10822 | 8879 -> 10797
-# fp32: the library's 1568 x 768 and 784 x 1024 products fill the chip exactly and are ahead; half and twice the tokens they are behind.
+# fp32: a gap between few tokens, where launches count, and many, where the products of either are alike and the passes over the
+# tokens count: there the library's products are ahead (784 x 768, 1568 x 768, 392 and 784 x 1024, 1960 and 2352 x 512).
 #   VRWKV        392 x 768   3446 -> 1761 | 1892 -> 1760      784 x 768    3476 -> 2494 | 2274 -> 2485      1568 x 768 3481 -> 3915 | 3326 -> 3907
 #                3136 x 768  7010 -> 6330 | 6990 -> 6325      784 x 1024   3539 -> 3860 | 3394 -> 3853      1568 x 1024 5558 -> 5423 | 5524 -> 5411
-#                3136 x 384  3490 -> 2452 | 2400 -> 2438      6272 x 384   5768 -> 4026 | 5742 -> 3995      3136 x 512 3799 -> 3322 | 3752 -> 3292
+#                3136 x 384  3490 -> 2452 | 2400 -> 2438      6272 x 384   5768 -> 4026 | 5742 -> 3995      1568 x 512  3454 -> 2254 | 2349 -> 2233
+#                1960 x 512  3521 -> 2452 | 2174 -> 2454      3136 x 448   3859 -> 2970 | 3829 -> 2957      43904 x 192 7935 -> 8006 | 7917 -> 7999
 #   VRWKV6       784 x 768   5810 -> 3363 | 3357 -> 3339      1568 x 768   5825 -> 4994 | 4637 -> 4960      1568 x 1024 7193 -> 6854 | 7101 -> 6826
-NATIVE_NARROW = 512                                   # channels up to which the native call is ahead on the GPU as well
-NATIVE_BLOCK_WORK = {                                 # (fp32, VRWKV6): most work recorded into a graph beyond that width, most work at all
-    (False, False): (600_000_000, 3_800_000_000), (False, True): (4_000_000_000, 7_500_000_000),
-    (True, False): (300_000_000, 600_000_000), (True, True): (600_000_000, 1_500_000_000)}
-NATIVE_BLOCK_WORK_FP32 = 1_500_000_000                # fp32: native again from here on
+#                2352 x 512  5943 -> 4005 | 4012 -> 3945      25088 x 192  7842 -> 7431 | 7718 -> 7419      3136 x 1024 13259 -> 12425 | 13180 -> 12409
+NATIVE_NARROW = 512
+NATIVE_WORK = {False: (600_000_000, 3_800_000_000), True: (4_000_000_000, 7_500_000_000)}       # VRWKV6: most work recorded if wider, most work
+NATIVE_FP32_GAP = {                                   # (VRWKV6, narrow): the work left to the operators, recorded and called
+    (False, True): ((420_000_000, 620_000_000), (0, 0)), (False, False): ((300_000_000, 1_500_000_000), (600_000_000, 1_500_000_000)),
+    (True, True): ((0, 0), (0, 0)), (True, False): ((600_000_000, 1_500_000_000), (0, 0))}
 
 
 def _native_size(x, hidden, v6):
@@ -221,11 +224,13 @@ def _native_size(x, hidden, v6):
     M, C = x.shape[0] * x.shape[1], x.shape[2]
     if M * max(C, hidden, 160) * x.element_size() >= 1 << 30:
         return False
-    work, fp32, narrow = M * C * C, x.dtype == torch.float32, C <= NATIVE_NARROW
-    if fp32 and (narrow or work >= NATIVE_BLOCK_WORK_FP32):
-        return True
-    recorded, called = NATIVE_BLOCK_WORK[fp32, v6]
-    return work <= called and (narrow or work <= recorded or not torch.cuda.is_current_stream_capturing())
+    work, narrow = M * C * C, C <= NATIVE_NARROW
+    if x.dtype == torch.float32:
+        recorded, called = (not lo < work < hi for lo, hi in NATIVE_FP32_GAP[v6, narrow])
+    else:
+        recorded, called = (work <= most for most in NATIVE_WORK[v6])
+        recorded |= narrow
+    return called and (recorded or not torch.cuda.is_current_stream_capturing())
 
 
 def _as_built(module, kind):
