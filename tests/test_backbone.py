@@ -666,6 +666,36 @@ def test_native_block_is_no_further_from_the_fp32_model_than_its_operators(kind,
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("C,dtype,key_norm,post_norm,cls,hw,batch,segments", [
+    (192, torch.bfloat16, False, False, False, (17, 18), 1, 0), (192, torch.float16, True, True, True, (24, 24), 1, 0),
+    (64, torch.float32, True, False, True, (24, 24), 3, 0), (192, torch.float32, False, True, False, (17, 18), 1, 0),
+    (768, torch.bfloat16, True, False, False, (28, 28), 2, 0), (128, torch.bfloat16, True, True, False, (5, 13), 3, 3),
+    (64, torch.float16, False, False, True, (1, 33), 5, 2), (320, torch.float32, True, False, True, (8, 16), 2, 64)])
+def test_native_v6_block_on_sequences_cut_into_segments(C, dtype, key_norm, post_norm, cls, hw, batch, segments):
+    """Few long sequences, and short ones with a forced number of segments: the wkv6 operator inside the block exchanges states
+    through its part of the block's workspace.  Held against the operators as above."""
+    net = _small_backbone("v6", C, dtype, key_norm, post_norm, cls, hw)
+    img = torch.randn(batch, 3, hw[0] * 16, hw[1] * 16, device="cuda").to(dtype)
+    from vision_rwkv_amd import lib, ops as impl, option
+    with torch.no_grad(), option("wkv6_segments", segments):
+        assert lib().vrwkv_wkv6_fwd_workspace_bytes(batch, hw[0] * hw[1] + cls, C, C // 64) > 0
+        x, res = net.embed(img)
+        x = x if not cls else torch.cat((x, x[:, :1]), 1)
+        assert all(l._native(x, res) is not None for l in net.layers)
+        got = net(img).double()
+        impl.BLOCK_FUSE_ENABLED = False
+        try:
+            plain = net(img).double()
+            ref = net.float()(img.float()).double() if dtype != torch.float32 else plain
+        finally:
+            impl.BLOCK_FUSE_ENABLED = True
+    if dtype == torch.float32:
+        assert (got - plain).norm() <= 2.8e-5 * plain.norm()
+    else:
+        assert (got - ref).norm() <= 1.25 * (plain - ref).norm()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("C,dtype,key_norm,fp32_vectors", [(64, torch.bfloat16, False, False), (192, torch.float16, True, False),
                                                            (320, torch.bfloat16, True, True), (768, torch.float32, True, False),
                                                            (960, torch.bfloat16, False, True)])

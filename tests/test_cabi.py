@@ -149,6 +149,30 @@ def test_wkv6_backward_refuses_misaligned_pointers_without_device(lib):
                 assert b"aligned" in lib.vrwkv_last_error()
 
 
+def test_block_entries_validate_without_device(lib):
+    """vrwkv_block6_fwd takes a VRWKV6 block and all its parameters; null pointers and a short workspace are refused."""
+    import vision_rwkv_amd as ops
+    from vision_rwkv_amd import _lib
+    B, T, C = 1, 12, 64
+    size = lib.vrwkv_block_fwd_workspace_bytes(B, T, C, 256, 1, 1)
+    names = ("ln1_w", "ln1_b", "ln2_w", "ln2_b", "key", "value", "receptance", "output", "ffn_key", "ffn_receptance", "ffn_value", "gate",
+             "decay", "gn_w", "gn_b", "x", "out", "workspace")
+
+    def call(missing=None, heads=1, bytes_=size, params=True):
+        a = _lib.BlockArgs(B=B, T=T, C=C, hidden=256, heads=heads, Hp=3, Wp=4, shift_pixel=1, quarter=16, dtype=1, workspace_bytes=bytes_,
+                           **{n: 4096 for n in names if n != missing})
+        p = _lib.Block6Params(**{n: 4096 for n in _lib.Block6Params.POINTERS if n != missing})
+        return lib.vrwkv_block6_fwd(ctypes.byref(a), ctypes.byref(p) if params else None, None)
+
+    assert call(params=False) == 1 and call(heads=0) == 1
+    for n in names + _lib.Block6Params.POINTERS[:13]:
+        assert call(missing=n) == 1, n
+    assert call(missing="att_kn_w") == 1                     # a norm's weight without its bias, and the other way round
+    assert call(missing="att_kn_b") == 1
+    assert call(bytes_=size - 1) == 5
+    assert lib.vrwkv_block6_fwd(None, None, None) == 1 and lib.vrwkv_block_fwd(None, None) == 1
+
+
 def test_more_sequences_than_a_grid_holds_are_not_cut(lib):
     """A forced number of segments does not apply to more sequences than the fold kernel's grid has rows."""
     import vision_rwkv_amd as ops
