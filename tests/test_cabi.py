@@ -180,7 +180,7 @@ def test_more_sequences_than_a_grid_holds_are_not_cut(lib):
         assert lib.vrwkv_wkv6_fwd_workspace_bytes(65535, 100, 64, 1) > 0
         assert lib.vrwkv_wkv6_fwd_workspace_bytes(65536, 100, 64, 1) == 0
         cut, uncut = (lib.vrwkv_wkv6_bwd_workspace_bytes(B, 100, 64, 1) / B for B in (65535, 65536))
-    assert uncut == 101 * 64 * 4 and cut > 2 * 4 * 64 * 64 * 4         # two of two chunks each
+    assert uncut == 201 * 64 * 4 and cut > 2 * 4 * 64 * 64 * 4         # two of two chunks each
 
 
 def test_python_boundary_errors_without_device():

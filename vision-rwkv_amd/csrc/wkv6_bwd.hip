@@ -63,7 +63,7 @@ int segments(int B, int T, int H) {
     return forced > 0 ? 1 : wkv6_segments((long long)B * H, nchunk, device_cus(), SEG_BWD);
 }
 
-// Workspace: [fp32 sums gr, gk, gv (16-bit results only)] [gw (16-bit decay logits only)] [a] [partial gu] [states] [flags]
+// Workspace: [fp32 sums gr, gk, gv (16-bit results only)] [gw (16-bit decay logits only)] [a of both passes] [partial gu] [states] [flags]
 struct Plan {
     bool out16, w16;
     int nseg;
@@ -77,7 +77,7 @@ Plan plan(int B, int T, int C, int H, int rkv_dtype, int w_dtype, int grad_dtype
     p.n = (size_t)B * T * C;
     p.sums = (p.out16 ? 3 * p.n : 0) + (p.w16 ? p.n : 0);
     p.states = seg_bytes((long long)B * H, p.nseg, BWD_SEG_FLOATS);
-    p.bytes = ((p.sums + p.n + (size_t)B * p.nseg * C + 3) & ~(size_t)3) * sizeof(float) + p.states;
+    p.bytes = ((p.sums + 2 * p.n + (size_t)B * p.nseg * C + 3) & ~(size_t)3) * sizeof(float) + p.states;
     return p;
 }
 
@@ -93,7 +93,8 @@ int launch_all(const void* r, const void* k, const void* v, const void* w, const
     A.pk = p.out16 ? take(p.n) : static_cast<float*>(gk);
     A.pv = p.out16 ? take(p.n) : static_cast<float*>(gv);
     A.pw = p.w16 ? take(p.n) : static_cast<float*>(gw);
-    A.a = take(p.n);
+    A.a = take(2 * p.n);
+    A.a_size = p.n;
     A.gu_part = take((size_t)B * p.nseg * C);
     q = ws + (((size_t)(q - ws) + 3) & ~(size_t)3);      // states: 16-byte aligned
     // gv leaves the sweep in pieces of four channels; where its 16-bit rows do not lie on 4 bytes, the sums are rounded afterwards

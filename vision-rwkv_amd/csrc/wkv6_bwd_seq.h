@@ -42,7 +42,7 @@ void seq_sweep_s(int bh, const IO* __restrict__ r_, const IO* __restrict__ k_, c
 {
     float (*s_row)[3][HN] = reinterpret_cast<float (*)[3][HN]>(stage);   // [wave][v, gy][i]
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
     const int b = bh / H, h = bh % H;
     const int sq = lane & 3, j = wave * 16 + (lane >> 2);
     const size_t base = (size_t)b * T * C + (size_t)h * HN;
@@ -95,7 +95,7 @@ void seq_sweep_g(int bh, const IO* __restrict__ r_, const IO* __restrict__ k_, c
 {
     float (*s_row)[3][HN] = reinterpret_cast<float (*)[3][HN]>(stage);
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
     const int b = bh / H, h = bh % H;
     const int sq = lane & 3, j = wave * 16 + (lane >> 2);
     const size_t base = (size_t)b * T * C + (size_t)h * HN;
@@ -148,7 +148,7 @@ void seq_sweep_v(int bh, const IO* __restrict__ r_, const IO* __restrict__ k_,
 {
     float (*s_row)[3][HN] = reinterpret_cast<float (*)[3][HN]>(stage);   // [wave][r, k, d][j]
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
     const int b = bh / H, h = bh % H;
     const int sq = lane & 3, i = wave * 16 + (lane >> 2);
     const size_t base = (size_t)b * T * C + (size_t)h * HN;

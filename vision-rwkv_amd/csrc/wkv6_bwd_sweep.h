@@ -50,7 +50,8 @@ struct BwdArgs {
     const float *u, *gy;
     void *gr, *gk, *gv, *gw;                         // results: IO / WT when out16 / w16, else fp32
     float *pr, *pk, *pv, *pw;                        // fp32 sums of the upward sweep (the results themselves when they are fp32)
-    float *a, *gu_part;                              // sequential fallback's (B,T,C) scratch; (B*nseg, C) partial gu
+    float *a, *gu_part;                              // sequential fallback's (2, B,T,C) scratch; (B*nseg, C) partial gu
+    size_t a_size;                                   // elements of a tensor
     const float* seg_ws;                             // states entering the segments (nseg > 1)
     const int* seg_flags;
     int T, C, H, sequences, nseg, out16, w16;
@@ -260,7 +261,7 @@ void wkv6_bwd_sweep_kernel(BwdArgs A)
     using Lds = BwdLds<!EXACT>;
     __shared__ Lds L;
     __shared__ int sFlag;
-    static_assert(sizeof(Lds) >= SEQ_STAGE_FLOATS * sizeof(float), "the sequential sweeps' staging must fit");
+    static_assert(sizeof(Lds) >= 2 * SEQ_STAGE_FLOATS * sizeof(float), "the sequential sweeps' staging must fit");
 
     const int lane = threadIdx.x & 63;                                    // channel in the element-wise and closing stages
     const int w8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // token group there (tokens 4 w8 .. 4 w8 + 3 of the chunk)
@@ -631,21 +632,23 @@ void wkv6_bwd_sweep_kernel(BwdArgs A)
         return;
     }
     }
-    // Some chunk decays faster than the factors can represent: the whole sequence with the sequential sweeps (four waves wide),
-    // which add into fp32 buffers; 16-bit results are rounded from those afterwards.
+    // Some chunk decays faster than the factors can represent: the whole sequence with the sequential sweeps, which add into fp32
+    // buffers; 16-bit results are rounded from those afterwards.  The sweeps are four waves wide and a chain over the tokens, so
+    // two run side by side: waves 0..3 gr of both passes and then half of gv, waves 4..7 the other half of gv and then gk and gw,
+    // which need gr's `a` of the same pass (768 sequences of 196 tokens, bf16: 1140 us; one after the other 2010).
     __syncthreads();
-    float* const stage = reinterpret_cast<float*>(&L);
-    if (w8 < 4) {
-        const IO *r = static_cast<const IO*>(A.r), *k = static_cast<const IO*>(A.k), *v = static_cast<const IO*>(A.v);
-        const WT* w = static_cast<const WT*>(A.w);
-        float* const gu_row = A.gu_part + (size_t)b * nseg * C + h * HN;
-        seq_sweep_s<IO, WT, 1, W_IS_EW>(bh, r, k, v, w, A.u, A.gy, A.pr, A.a, gu_row, stage, T, C, A.H);
-        seq_sweep_g<IO, WT, 1, W_IS_EW>(bh, r, k, v, w, A.u, A.gy, A.a, A.pk, A.pw, stage, T, C, A.H);
-        seq_sweep_v<IO, WT, 1, W_IS_EW>(bh, r, k, w, A.u, A.gy, A.pv, stage, T, C, A.H);
-        seq_sweep_s<IO, WT, 0, W_IS_EW>(bh, r, k, v, w, A.u, A.gy, A.pr, A.a, gu_row, stage, T, C, A.H);
-        seq_sweep_g<IO, WT, 0, W_IS_EW>(bh, r, k, v, w, A.u, A.gy, A.a, A.pk, A.pw, stage, T, C, A.H);
-        seq_sweep_v<IO, WT, 0, W_IS_EW>(bh, r, k, w, A.u, A.gy, A.pv, stage, T, C, A.H);
-    }
+    float* const stage = reinterpret_cast<float*>(&L) + (w8 >> 2) * SEQ_STAGE_FLOATS;
+    const IO *r = static_cast<const IO*>(A.r), *k = static_cast<const IO*>(A.k), *v = static_cast<const IO*>(A.v);
+    const WT* w = static_cast<const WT*>(A.w);
+    float* const gu_row = A.gu_part + (size_t)b * nseg * C + h * HN;
+    if (w8 < 4) seq_sweep_s<IO, WT, 1, W_IS_EW>(bh, r, k, v, w, A.u, A.gy, A.pr, A.a, gu_row, stage, T, C, A.H);
+    else seq_sweep_v<IO, WT, 1, W_IS_EW>(bh, r, k, w, A.u, A.gy, A.pv, stage, T, C, A.H);
+    __syncthreads();
+    if (w8 < 4) seq_sweep_s<IO, WT, 0, W_IS_EW>(bh, r, k, v, w, A.u, A.gy, A.pr, A.a + A.a_size, gu_row, stage, T, C, A.H);
+    else seq_sweep_g<IO, WT, 1, W_IS_EW>(bh, r, k, v, w, A.u, A.gy, A.a, A.pk, A.pw, stage, T, C, A.H);
+    __syncthreads();
+    if (w8 < 4) seq_sweep_v<IO, WT, 0, W_IS_EW>(bh, r, k, w, A.u, A.gy, A.pv, stage, T, C, A.H);
+    else seq_sweep_g<IO, WT, 0, W_IS_EW>(bh, r, k, v, w, A.u, A.gy, A.a + A.a_size, A.pk, A.pw, stage, T, C, A.H);
     if ((ES == 2 && A.out16) || (WS == 2 && A.w16)) {
         __syncthreads();
         for (size_t q = threadIdx.x; q < (size_t)T * HN; q += 512) {
