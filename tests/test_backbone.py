@@ -966,6 +966,20 @@ def test_weight_gradient_kernel_against_float64(n, M, O, I, dtype, splits):
 
 
 @pytest.mark.gpu
+def test_weight_gradient_of_many_tokens_in_more_ranges():
+    """200000 tokens into 96 x 40: 260 ranges, against float64 with the bound of the test above."""
+    from vision_rwkv_amd import lib
+    from vision_rwkv_amd.ops import weight_grad
+    torch.manual_seed(6)
+    M, O, I = 200003, 96, 40
+    assert lib().vrwkv_wgrad_workspace_bytes(1, M, O, I) > 200 * O * I * 4
+    a, b = (torch.randn(M, c, device="cuda").bfloat16() for c in (O, I))
+    got = weight_grad(a, b).double()
+    ref, mag = a.double().t() @ b.double(), a.double().abs().t() @ b.double().abs()
+    assert bool(((got - ref).abs() <= 2.0 ** -8 * 1.01 * ref.abs() + (M + 4) * 2.0 ** -24 * mag + 1e-7).all())
+
+
+@pytest.mark.gpu
 def test_second_derivative_of_a_projection_goes_through_tensor_ops():
     from vision_rwkv_amd.backbone import _SplitKLinear
     torch.manual_seed(6)

@@ -3,7 +3,8 @@
 // result and a range of the tokens and leaves its fp32 partial sum, a second kernel adds the ranges in a fixed order and
 // rounds once.  Bound by the LDS reads of 64 x 64 quadrants and, with many ranges, by the partial sums' way through memory
 // (14 ranges of 768 x 768: 33 MB out and in): two workgroups per compute unit (14 ranges; 7: 41 us, 28: 41 us) and at most 32
-// ranges measure best (192 x 192: 28 ranges 15 us, 98 ranges 23 us).  12544 tokens, bf16, own / the library's batched partial
+// ranges, or ranges of 24 slices where that is more, measure best (192 x 192 on 12544 tokens: 28 ranges 15 us, 98 ranges 23 us; on
+// 100352: 32 ranges 61 us, 64 39, 128 35, 256 45; 96 x 96 on 301056: 32 ranges 162 us, 128 56, 256 47).  12544 tokens, bf16, own / the library's batched partial
 // products in bf16 and their sum: 768 x 768 34 / 43 us, 384 x 384 22 / 37, 1536 x 384 33 / 42, 768 x 64 16 / 25; error against
 // float64 1.7e-3 (the result's rounding) / 2.4e-3.
 #include "gemm_tile.h"
@@ -69,7 +70,7 @@ Plan plan(int n, int M, int O, int I) {
     const int slices = (M + 31) / 32, forced = option(OPT_WGRAD_SPLITS);
     const long long tiles = (long long)n * p.tiles_o * p.tiles_i;
     int s = forced ? forced : (int)std::max(1LL, 2LL * device_cus() / tiles);
-    if (!forced) s = std::min(s, 32);
+    if (!forced) s = std::min(s, std::max(32, slices / 24));
     s = std::min(s, std::max(1, slices / 4));
     p.slices_per = (slices + s - 1) / s;
     p.splits = (slices + p.slices_per - 1) / p.slices_per;
