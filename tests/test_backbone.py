@@ -979,6 +979,19 @@ def test_weight_gradient_of_many_tokens_in_more_ranges():
     assert bool(((got - ref).abs() <= 2.0 ** -8 * 1.01 * ref.abs() + (M + 4) * 2.0 ** -24 * mag + 1e-7).all())
 
 
+@pytest.mark.parametrize("M,O,I,own", [(4096, 1024, 1024, True), (9408, 4096, 256, True), (12544, 1024, 1024, False), (25088, 1024, 768, False),
+                                       (12544, 768, 768, True), (100352, 768, 768, True), (301056, 768, 768, False), (301056, 64, 768, True),
+                                       (301056, 96, 96, True), (12544, 3072, 768, False), (6272, 2048, 512, True)])
+def test_weight_gradients_where_they_measured_faster(M, O, I, own, monkeypatch):
+    """The rule against the measured points: the kernel is asked, or the library's partial products (on tensors without data)."""
+    from vision_rwkv_amd import backbone as bb
+    monkeypatch.setattr(bb, "weight_grad", lambda a, b: "own")
+    monkeypatch.setattr(bb, "_transformed", lambda: False)
+    a, b = (torch.empty(M, c, dtype=torch.bfloat16, device="meta") for c in (O, I))
+    with torch.no_grad():
+        assert (isinstance(bb._token_product(a, b, 8), str)) == own
+
+
 @pytest.mark.gpu
 def test_second_derivative_of_a_projection_goes_through_tensor_ops():
     from vision_rwkv_amd.backbone import _SplitKLinear

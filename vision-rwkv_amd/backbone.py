@@ -67,10 +67,13 @@ def _mix(module, x, mixes, shift_pixel, gamma, patch_resolution, fused, head_dim
     return [x * m + xx * (1 - m) for m in mixes]
 
 
-# Elements of a weight up to which its gradient is the framework's own kernel: 12544 tokens, own / the library's batched
-# partial products and their sum, in us: 768 x 768 34 / 43, 384 x 384 22 / 37, 1536 x 384 33 / 42, 192 x 192 15 / 25, 160 x 768 22 / 36,
-# five of 32 x 768 24 / 44; 3072 x 768 112 / 74.
-OWN_WEIGHT_GRAD = 1 << 20
+# Whose weight gradient is the framework's own kernel, by the weight's elements and the multiplications: its deep split pays until
+# the library's partial products fill the chip for long, which weights beyond about 0.6 million elements do sooner.  Own / the
+# library's batched partial products and their sum, in us:
+#   12544 tokens   768 x 768 34 / 44     384 x 384 23 / 40   1536 x 384 34 / 43   192 x 192 18 / 33   160 x 768 22 / 39   5 of 32 x 768 24 / 45
+#                  1024 x 1024 45 / 43   9408 tokens: 4096 x 256 39 / 42           25088: 1024 x 1024 73 / 65, 1024 x 768 62 / 59
+#   100352 tokens  768 x 768 189 / 274   384 x 384 60 / 118  192 x 192 35 / 98    1024 x 1024 317 / 230     301056: 768 x 768 537 / 408
+OWN_WEIGHT_GRAD = ((650_000, 100_000_000_000), (1 << 20, 10_000_000_000))           # elements up to, multiplications up to
 
 
 def _token_product(a, b, splits):
@@ -78,7 +81,7 @@ def _token_product(a, b, splits):
     `splits` batched partial products of the library.  A gradient that is itself to be differentiated, batched or traced takes tensor
     ops."""
     (M, O), I = a.shape[-2:], b.shape[-1]
-    if (not torch.is_grad_enabled() and O * I <= OWN_WEIGHT_GRAD and O % 8 == 0 and I % 8 == 0 and a.dtype == b.dtype
+    if (not torch.is_grad_enabled() and any(O * I <= n and M * O * I <= work for n, work in OWN_WEIGHT_GRAD) and O % 8 == 0 and I % 8 == 0 and a.dtype == b.dtype
             and not batched_cotangent(a, b) and not _transformed()
             and M * max(a.stride(-2), b.stride(-2), O, I) < 1 << 30):
         return weight_grad(a, b)
