@@ -38,20 +38,32 @@ def resize_pos_embed(pos_embed, src_shape, dst_shape, mode="bicubic", num_extra_
     return torch.cat((extra, w), dim=1) if num_extra_tokens else w
 
 
+class _Kept(dict):
+    """What eval_cached keeps on a module; a copy of the module starts without."""
+
+    def __deepcopy__(self, memo):
+        return _Kept()
+
+    def __reduce__(self):
+        return _Kept, ()
+
+
 def eval_cached(module, name, params, extra, make):
     """Value derived from parameters (a dtype conversion, a stacked table), kept on the module between forward passes
     without autograd and rebuilt when a parameter was written to (its version counter), moved or cast.  The entry holds on to
     the memory it was derived from, so that no later parameter can be found at the same address.  A write through p.data
     counts as no new version: after one, the next in-place write, cast or move of the parameter brings the value up to date.
     A value made while the stream is recorded into a graph exists when the graph runs, and is not kept."""
-    key = (extra,) + tuple((p._version, p.dtype, p.device) for p in params)
-    slot = module.__dict__.setdefault("_eval_cache", {})
-    hit = slot.get(name)
-    if hit is None or hit[0] != key or any(m.data_ptr() != p.data_ptr() for m, p in zip(hit[2], params)):
+    key = (extra,) + tuple((p._version, p.dtype, p.device, p.data_ptr()) for p in params)
+    kept = module.__dict__.get("_eval_cache")
+    if kept is None:
+        kept = module.__dict__.setdefault("_eval_cache", _Kept())
+    hit = kept.get(name)
+    if hit is None or hit[0] != key:
         hit = (key, make(), [p.detach() for p in params])
         if params[0].is_cuda and torch.cuda.is_current_stream_capturing():
             return hit[1]
-        slot[name] = hit
+        kept[name] = hit
     return hit[1]
 
 
@@ -229,54 +241,54 @@ def _native_size(x, hidden, v6):
         return False
     work, narrow = M * C * C, C <= NATIVE_NARROW
     if x.dtype == torch.float32:
-        recorded, called = (not lo < work < hi for lo, hi in NATIVE_FP32_GAP[v6, narrow])
+        (lo, hi), (lo2, hi2) = NATIVE_FP32_GAP[v6, narrow]
+        recorded, called = not lo < work < hi, not lo2 < work < hi2
     else:
-        recorded, called = (work <= most for most in NATIVE_WORK[v6])
-        recorded |= narrow
+        most, most2 = NATIVE_WORK[v6]
+        recorded, called = narrow or work <= most, work <= most2
     return called and (recorded or not torch.cuda.is_current_stream_capturing())
 
 
 def _as_built(module, kind):
-    """True when calling `module` does what `kind`'s own forward does with the module's parameters and nothing else.  (What stands
-    in another place -- pruned, normed or parametrised weights, buffers -- is missing from _parameters, or None, also then.)"""
+    """True when calling `module` does what `kind`'s own forward does with the module's parameters and nothing else."""
     return (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks and "forward" not in module.__dict__)
 
 
 def _block_weights(block, att, ffn, x):
     """The weights of a block that one native call can run (its linear maps with the shapes and without the biases they are
     built with, the norms with both vectors) and the numbers that go with them, as fields of vrwkv_block_args; None for any
-    other block."""
+    other block, KeyError where a name is missing (pruned, normed, parametrised weights and buffers stand elsewhere)."""
     am, fm, bm, C = att._modules, ffn._modules, block._modules, x.shape[2]
-    key = fm.get("key")
-    weight = key._parameters.get("weight") if _as_built(key, nn.Linear) else None      # (a pruned or normed layer has none)
+    key = fm["key"]
+    weight = key._parameters["weight"] if type(key) is nn.Linear else None
     hidden = weight.shape[0] if weight is not None else 0
     if not (C % 32 == 0 and hidden % 32 == 0 and 0 < hidden <= 4096 and att.fused_shift and ffn.fused_shift
             and att.shift_pixel == ffn.shift_pixel and _native_size(x, hidden, "gate" in am)):
         return None
     w, num = {}, dict(hidden=hidden, shift_pixel=att.shift_pixel, post_norm=int(block.post_norm))
-    for name, lin, shape in (("key", am.get("key"), (C, C)), ("value", am.get("value"), (C, C)), ("receptance", am.get("receptance"), (C, C)),
-                             ("output", am.get("output"), (C, C)), ("ffn_key", key, (hidden, C)),
-                             ("ffn_receptance", fm.get("receptance"), (C, C)), ("ffn_value", fm.get("value"), (C, hidden))):
+    for name, lin, shape in (("key", am["key"], (C, C)), ("value", am["value"], (C, C)), ("receptance", am["receptance"], (C, C)),
+                             ("output", am["output"], (C, C)), ("ffn_key", key, (hidden, C)),
+                             ("ffn_receptance", fm["receptance"], (C, C)), ("ffn_value", fm["value"], (C, hidden))):
         if not _as_built(lin, nn.Linear):
             return None
         p = lin._parameters
-        if p.get("bias") is not None or p.get("weight") is None or p["weight"].shape != shape:
+        if p["bias"] is not None or p["weight"] is None or p["weight"].shape != shape:
             return None
         w[name] = p["weight"]
-    for name, ln, n in (("ln1", bm.get("ln1"), C), ("ln2", bm.get("ln2"), C), ("att_kn", am.get("key_norm"), C),
+    for name, ln, n in (("ln1", bm["ln1"], C), ("ln2", bm["ln2"], C), ("att_kn", am.get("key_norm"), C),
                         ("ffn_kn", fm.get("key_norm"), hidden)):
         if ln is None and name.endswith("kn"):
             continue
         if not _as_built(ln, nn.LayerNorm) or ln.normalized_shape != (n,):
             return None
         p = ln._parameters
-        if p.get("weight") is None or p.get("bias") is None:
+        if p["weight"] is None or p["bias"] is None:
             return None
         w[name + "_w"], w[name + "_b"] = p["weight"], p["bias"]
         num[name + "_eps"] = ln.eps
     if block.layer_scale:
         for name in ("gamma1", "gamma2"):
-            w[name] = block._parameters.get(name)
+            w[name] = block._parameters[name]
             if w[name] is None or w[name].shape != (C,):
                 return None
     return w, num
@@ -286,7 +298,7 @@ def _block_may_fuse(block, att_kind, ffn_kind, x):
     """The checks that come before a look at the weights."""
     return (block_takes(x)
             and not _hooks._global_forward_hooks and not _hooks._global_forward_pre_hooks
-            and _as_built(block._modules.get("att"), att_kind) and _as_built(block._modules.get("ffn"), ffn_kind))
+            and _as_built(block._modules["att"], att_kind) and _as_built(block._modules["ffn"], ffn_kind))
 
 
 class VRWKV_SpatialMix(nn.Module):
@@ -384,6 +396,13 @@ class Block(nn.Module):
 
     def _native(self, x, res):
         """The block in one native call (vrwkv_block_fwd) where that computes the same; None elsewhere."""
+        try:
+            fields = self._native_fields(x, res)
+        except KeyError:                                     # a parameter or module that is held otherwise than built
+            return None
+        return None if fields is None else block_forward(x, *fields[:-1], **fields[-1])
+
+    def _native_fields(self, x, res):
         if not _block_may_fuse(self, VRWKV_SpatialMix, VRWKV_ChannelMix, x):
             return None
         att, ffn = self._modules["att"], self._modules["ffn"]
@@ -394,15 +413,32 @@ class Block(nn.Module):
             return None
         w, num = wn
         ap, fp = att._parameters, ffn._parameters
-        decay, first = ap.get("spatial_decay"), ap.get("spatial_first")
-        am, fm = [ap.get("spatial_mix_" + n) for n in "kvr"], [fp.get("spatial_mix_" + n) for n in "kr"]
-        if any(p is None or p.numel() != C or p.get_device() != x.get_device() for p in (decay, first, *am, *fm)) or decay.dtype != x.dtype:
+        vectors = (ap["spatial_decay"], ap["spatial_first"], ap["spatial_mix_k"], ap["spatial_mix_v"], ap["spatial_mix_r"],
+                   fp["spatial_mix_k"], fp["spatial_mix_r"])
+        for p in vectors:
+            if p is None:
+                return None
+        if vectors[0].dtype != x.dtype:
             return None
-        w["w"], w["u"] = eval_cached(att, "wu", (decay, first), T,
-                                     lambda: ((decay / T).float().contiguous(), (first / T).float().contiguous()))
-        w["att_mix"] = eval_cached(att, "mix_table", am, x.device, lambda: stack_mixes(am, x.device))
-        w["ffn_mix"] = eval_cached(ffn, "mix_table", fm, x.device, lambda: stack_mixes(fm, x.device))
-        return block_forward(x, w, Hp=res[0], Wp=res[1], quarter=int(C * att.channel_gamma), **num)
+        device = x.device
+        wu = eval_cached(self, "native_wu", vectors[:2], (T, device), lambda: self._native_tables(vectors[:2], x, divided=True))
+        mixes = eval_cached(self, "native_mix", vectors[2:], device, lambda: self._native_tables(vectors[2:], x))
+        if wu is None or mixes is None:
+            return None
+        w["w"], w["u"] = wu
+        w["att_mix"], w["ffn_mix"] = mixes
+        return w, dict(num, Hp=res[0], Wp=res[1], quarter=int(C * att.channel_gamma))
+
+    @staticmethod
+    def _native_tables(vectors, x, divided=False):
+        """Decay and bonus divided by T, or the mix tables, as the native call takes them; None for vectors that the operators
+        refuse or move (other sizes, another device)."""
+        T, C = x.shape[1:]
+        if any(p.numel() != C or p.device != x.device for p in vectors):
+            return None
+        if divided:
+            return [(p / T).float().reshape(-1).contiguous() for p in vectors]
+        return stack_mixes(vectors[:3], x.device), stack_mixes(vectors[3:], x.device)
 
     def forward(self, x, patch_resolution):
         if self.layer_id == 0:

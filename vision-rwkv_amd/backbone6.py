@@ -149,7 +149,14 @@ class Block6(nn.Module):
             self.gamma2 = nn.Parameter(init_values * torch.ones(n_embd))
 
     def _native(self, x, res):
-        """The block in one native call (vrwkv_block_fwd) where that computes the same; None elsewhere."""
+        """The block in one native call (vrwkv_block6_fwd) where that computes the same; None elsewhere."""
+        try:
+            fields = self._native_fields(x, res)
+        except KeyError:                                     # a parameter or module that is held otherwise than built
+            return None
+        return None if fields is None else block_forward(x, *fields[:-1], **fields[-1])
+
+    def _native_fields(self, x, res):
         if not _block_may_fuse(self, VRWKV_SpatialMix_V6, VRWKV_ChannelMix_V6, x):
             return None
         att, ffn = self._modules["att"], self._modules["ffn"]
@@ -158,13 +165,14 @@ class Block6(nn.Module):
         if wn is None:
             return None
         w, num = wn
-        ap, fp, ln_x, gate = att._parameters, ffn._parameters, att._modules.get("ln_x"), att._modules.get("gate")
-        low = {n: ap.get("time_" + n) for n in ("maa_w1", "maa_w2", "decay_w1", "decay_w2")}
-        vec = {"maa_" + n: ap.get("time_maa_" + n) for n in "xwkvrg"}
-        vec.update(ffn_mix_k=fp.get("spatial_mix_k"), ffn_mix_r=fp.get("spatial_mix_r"), u=ap.get("time_faaaa"))
-        if any(p is None for p in (*low.values(), *vec.values(), ap.get("time_decay"))):
-            return None
-        if (not _as_built(gate, nn.Linear) or gate.bias is not None or gate._parameters.get("weight") is None or gate.weight.shape != (C, C)
+        ap, fp, ln_x, gate = att._parameters, ffn._parameters, att._modules["ln_x"], att._modules["gate"]
+        low = {n: ap["time_" + n] for n in ("maa_w1", "maa_w2", "decay_w1", "decay_w2")}
+        vec = {"maa_" + n: ap["time_maa_" + n] for n in "xwkvrg"}
+        vec.update(ffn_mix_k=fp["spatial_mix_k"], ffn_mix_r=fp["spatial_mix_r"], u=ap["time_faaaa"])
+        for p in (*low.values(), *vec.values(), ap["time_decay"]):
+            if p is None:
+                return None
+        if (not _as_built(gate, nn.Linear) or gate.bias is not None or gate._parameters["weight"] is None or gate.weight.shape != (C, C)
                 or not _as_built(ln_x, nn.GroupNorm) or ln_x.num_groups * HEAD_SIZE != C or ln_x.num_channels != C or not ln_x.affine
                 or att.n_head * HEAD_SIZE != C or ap["time_decay"].numel() != C
                 or tuple(t.shape for t in low.values()) != ((C, 160), (5, 32, C), (C, 64), (64, C))
@@ -176,7 +184,7 @@ class Block6(nn.Module):
         if not block_weights_fit(x, (*w.values(), *low.values())):
             return None
         params = {**low, **vec, **{n: w.pop(n) for n in ("att_kn_w", "att_kn_b") if n in w}}
-        return block_forward(x, w, params, Hp=res[0], Wp=res[1], heads=att.n_head, quarter=HEAD_SIZE // 4, gn_eps=ln_x.eps, **num)
+        return w, params, dict(num, Hp=res[0], Wp=res[1], heads=att.n_head, quarter=HEAD_SIZE // 4, gn_eps=ln_x.eps)
 
     def forward(self, x, patch_resolution):
         if self.layer_id == 0:
