@@ -38,7 +38,7 @@ const char* vrwkv_last_error(void);      /* thread-local, never NULL */
 
 /* Tuning / testing switches, process-wide (no counterpart in the reference).  Names: "biwkv_l", "biwkv_s",
  * "biwkv_grid", "biwkv_no_stage", "biwkv_no_resident", "biwkv_bwd_serial", "wkv6_fwd_scalar", "wkv6_bwd_scalar",
- * "wkv6_bwd_unfused", "wkv6_segments", "linear_tile", "wgrad_splits"; 0 = default behaviour.  The initial value of <name> is
+ * "wkv6_bwd_unfused" (no effect: the backward is one kernel), "wkv6_segments", "linear_tile", "wgrad_splits"; 0 = default behaviour.  The initial value of <name> is
  * that of the environment variable VRWKV_<NAME> when the library first looks at any switch; the entry points never read the environment afterwards.
  * vrwkv_set_option rejects (VRWKV_INVALID_ARG) a value the plans would ignore: biwkv_l takes 0, 4, 8, 16, 25, 28 (tokens
  * per wave), biwkv_s 0 or 2..8 (waves per workgroup), biwkv_grid 0 or a positive workgroup count, wkv6_segments 0..64 (segments a sequence

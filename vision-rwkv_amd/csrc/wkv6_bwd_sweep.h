@@ -25,7 +25,7 @@
 // what hides the LDS and matrix latencies of the step.  Measured at 64 x 196 x 768 bf16: 190-215 us; four waves with 256
 // registers each, two per SIMD, 278; six scans with 1.35 GB of traffic, one per result and pass, 310.  What bounds it is the
 // step's latency and the vector ALUs (46 % busy; per step and workgroup 4700 vector instructions beside 480 MFMA), not
-// memory (0.6 GB).  A chunk step is an element-wise stage (wave: four tokens, lane: channel), a matrix stage and a closing
+// memory (0.61 GB by FETCH_SIZE and WRITE_SIZE).  A chunk step is an element-wise stage (wave: four tokens, lane: channel), a matrix stage and a closing
 // stage in the element-wise stage's layout, two LDS-only barriers (the decay sums of the next chunk and gw of the previous
 // one ride on them).  In the matrix stage the waves divide the three results: waves 0, 1 form gr and own S (half its
 // columns j each, 64 x 32 in their accumulators), waves 2, 3 gk and G with the value channel as the contraction, waves
@@ -37,7 +37,7 @@
 // runs in phases that read their operands anew instead of keeping them.
 //
 // Range: the factors need |P31| <= 60 in every chunk.  A sequence with a chunk outside that range is redone by the same
-// workgroup with the sequential sweeps of wkv6_bwd.hip.
+// workgroup with the sequential sweeps of wkv6_bwd_seq.h.
 #pragma once
 #include "wkv6_segment.h"
 #include "wkv6_bwd_seq.h"
