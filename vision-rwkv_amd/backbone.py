@@ -54,7 +54,9 @@ def eval_cached(module, name, params, extra, make):
     the memory it was derived from, so that no later parameter can be found at the same address.  A write through p.data
     counts as no new version: after one, the next in-place write, cast or move of the parameter brings the value up to date.
     A value made while the stream is recorded into a graph exists when the graph runs, and is not kept."""
-    key = (extra,) + tuple((p._version, p.dtype, p.device, p.data_ptr()) for p in params)
+    key = [extra]
+    for p in params:
+        key += (p._version, p.dtype, p.get_device(), p.data_ptr())
     kept = module.__dict__.get("_eval_cache")
     if kept is None:
         kept = module.__dict__.setdefault("_eval_cache", _Kept())
@@ -211,7 +213,9 @@ def _layer_norm(ln, x):
 # takes it 58 (83), so called eagerly it gains until its time on the GPU reaches the host's or the library's, whichever is longer.
 # Recorded into a graph only the time on the GPU counts.  There the native call saves launches and passes over the tokens, and
 # its products are slower than the library's where the contraction is long: 6 to 15 % of a 16-bit block from about 1000 tokens of 768
-# or more channels on.  Up to 512 channels it is ahead in 16 bits.  Twelve blocks of tokens x channels, operators ->
+# or more channels on.  Up to 512 channels it is ahead in 16 bits.  (VRWKV6, whose operators are more, is within 1 % on the GPU at the
+# eager line; its operators would also record the forming of their tables, which its native call does not leave behind.)  Twelve blocks
+# of tokens x channels, operators ->
 # native, eager | replayed, in us:
 #   VRWKV  bf16  784 x 768   3535 -> 1371 | 1415 -> 1362      1568 x 768   3532 -> 1704 | 1597 -> 1693      392 x 1024 3512 -> 1377 | 1508 -> 1375
 #                784 x 1024  3506 -> 1874 | 1648 -> 1868      3136 x 1024  3514 -> 2813 | 2466 -> 2806      6272 x 768 3566 -> 2964 | 3047 -> 2966
@@ -228,19 +232,20 @@ def _layer_norm(ln, x):
 #   VRWKV6       784 x 768   5810 -> 3363 | 3357 -> 3339      1568 x 768   5825 -> 4994 | 4637 -> 4960      1568 x 1024 7193 -> 6854 | 7101 -> 6826
 #                2352 x 512  5943 -> 4005 | 4012 -> 3945      25088 x 192  7842 -> 7431 | 7718 -> 7419      3136 x 1024 13259 -> 12425 | 13180 -> 12409
 NATIVE_NARROW = 512
-NATIVE_WORK = {False: (600_000_000, 3_800_000_000), True: (4_000_000_000, 7_500_000_000)}       # VRWKV6: most work recorded if wider, most work
+NATIVE_WORK = {False: (600_000_000, 3_800_000_000), True: (7_500_000_000, 7_500_000_000)}       # VRWKV6: most work recorded if wider, most work
 NATIVE_FP32_GAP = {                                   # (VRWKV6, narrow): the work left to the operators, recorded and called
     (False, True): ((420_000_000, 620_000_000), (0, 0)), (False, False): ((300_000_000, 1_500_000_000), (600_000_000, 1_500_000_000)),
-    (True, True): ((0, 0), (0, 0)), (True, False): ((600_000_000, 1_500_000_000), (0, 0))}
+    (True, True): ((0, 0), (0, 0)), (True, False): ((0, 0), (0, 0))}
 
 
 def _native_size(x, hidden, v6):
     """The rule above, and 32-bit byte offsets inside every token matrix of the call."""
-    M, C = x.shape[0] * x.shape[1], x.shape[2]
-    if M * max(C, hidden, 160) * x.element_size() >= 1 << 30:
+    B, T, C = x.shape
+    M, fp32 = B * T, x.dtype == torch.float32
+    if M * max(C, hidden, 160) * (4 if fp32 else 2) >= 1 << 30:
         return False
     work, narrow = M * C * C, C <= NATIVE_NARROW
-    if x.dtype == torch.float32:
+    if fp32:
         (lo, hi), (lo2, hi2) = NATIVE_FP32_GAP[v6, narrow]
         recorded, called = not lo < work < hi, not lo2 < work < hi2
     else:
@@ -294,10 +299,9 @@ def _block_weights(block, att, ffn, x):
     return w, num
 
 
-def _block_may_fuse(block, att_kind, ffn_kind, x):
+def _block_may_fuse(block, att_kind, ffn_kind):
     """The checks that come before a look at the weights."""
-    return (block_takes(x)
-            and not _hooks._global_forward_hooks and not _hooks._global_forward_pre_hooks
+    return (not _hooks._global_forward_hooks and not _hooks._global_forward_pre_hooks
             and _as_built(block._modules["att"], att_kind) and _as_built(block._modules["ffn"], ffn_kind))
 
 
@@ -396,14 +400,16 @@ class Block(nn.Module):
 
     def _native(self, x, res):
         """The block in one native call (vrwkv_block_fwd) where that computes the same; None elsewhere."""
+        if not block_takes(x):
+            return None
         try:
             fields = self._native_fields(x, res)
         except KeyError:                                     # a parameter or module that is held otherwise than built
             return None
-        return None if fields is None else block_forward(x, *fields[:-1], **fields[-1])
+        return block_forward(x, fields[0], **fields[1]) if fields is not None else None
 
     def _native_fields(self, x, res):
-        if not _block_may_fuse(self, VRWKV_SpatialMix, VRWKV_ChannelMix, x):
+        if not _block_may_fuse(self, VRWKV_SpatialMix, VRWKV_ChannelMix):
             return None
         att, ffn = self._modules["att"], self._modules["ffn"]
         T, C = x.shape[1:]
@@ -413,32 +419,24 @@ class Block(nn.Module):
             return None
         w, num = wn
         ap, fp = att._parameters, ffn._parameters
-        vectors = (ap["spatial_decay"], ap["spatial_first"], ap["spatial_mix_k"], ap["spatial_mix_v"], ap["spatial_mix_r"],
-                   fp["spatial_mix_k"], fp["spatial_mix_r"])
-        for p in vectors:
-            if p is None:
-                return None
-        if vectors[0].dtype != x.dtype:
+        decay, first = ap["spatial_decay"], ap["spatial_first"]
+        am = [ap["spatial_mix_k"], ap["spatial_mix_v"], ap["spatial_mix_r"]]
+        fm = [fp["spatial_mix_k"], fp["spatial_mix_r"]]
+        if (decay is None or first is None or am[0] is None or am[1] is None or am[2] is None or fm[0] is None or fm[1] is None
+                or decay.dtype != x.dtype):
             return None
+        # under the operators' names: what an eager native call formed, a recorded forward that takes the operators finds
         device = x.device
-        wu = eval_cached(self, "native_wu", vectors[:2], (T, device), lambda: self._native_tables(vectors[:2], x, divided=True))
-        mixes = eval_cached(self, "native_mix", vectors[2:], device, lambda: self._native_tables(vectors[2:], x))
-        if wu is None or mixes is None:
-            return None
-        w["w"], w["u"] = wu
-        w["att_mix"], w["ffn_mix"] = mixes
-        return w, dict(num, Hp=res[0], Wp=res[1], quarter=int(C * att.channel_gamma))
-
-    @staticmethod
-    def _native_tables(vectors, x, divided=False):
-        """Decay and bonus divided by T, or the mix tables, as the native call takes them; None for vectors that the operators
-        refuse or move (other sizes, another device)."""
-        T, C = x.shape[1:]
-        if any(p.numel() != C or p.device != x.device for p in vectors):
-            return None
-        if divided:
-            return [(p / T).float().reshape(-1).contiguous() for p in vectors]
-        return stack_mixes(vectors[:3], x.device), stack_mixes(vectors[3:], x.device)
+        wd, u = eval_cached(att, "wu", (decay, first), T, lambda: ((decay / T).float().contiguous(), (first / T).float().contiguous()))
+        att_mix = eval_cached(att, "mix_table", am, device, lambda: stack_mixes(am, device))
+        ffn_mix = eval_cached(ffn, "mix_table", fm, device, lambda: stack_mixes(fm, device))
+        index = x.get_device()
+        if (wd.numel() != C or u.numel() != C or att_mix.numel() != 3 * C or ffn_mix.numel() != 2 * C
+                or wd.get_device() != index or u.get_device() != index):
+            return None                                      # (the operators refuse these)
+        w["w"], w["u"], w["att_mix"], w["ffn_mix"] = wd, u, att_mix, ffn_mix
+        num["Hp"], num["Wp"], num["quarter"] = res[0], res[1], int(C * att.channel_gamma)
+        return w, num
 
     def forward(self, x, patch_resolution):
         if self.layer_id == 0:

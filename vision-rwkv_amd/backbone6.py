@@ -11,7 +11,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .backbone import VRWKV, eval_cached, _proj, _matmul, _bmm, _as_built, _block_may_fuse, _block_weights
-from .ops import (HEAD_SIZE, RUN_CUDA_RWKV6, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, maa_mix, groupnorm_gate, block_weights_fit, block_forward, PRE_NONE, PRE_RELU_SQ, POST_NONE,
+from .ops import (HEAD_SIZE, RUN_CUDA_RWKV6, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, maa_mix, groupnorm_gate, block_takes, block_weights_fit, block_forward, PRE_NONE, PRE_RELU_SQ, POST_NONE,
                   POST_SIGMOID_GATE, POST_RESIDUAL)
 
 
@@ -150,14 +150,16 @@ class Block6(nn.Module):
 
     def _native(self, x, res):
         """The block in one native call (vrwkv_block6_fwd) where that computes the same; None elsewhere."""
+        if not block_takes(x):
+            return None
         try:
             fields = self._native_fields(x, res)
         except KeyError:                                     # a parameter or module that is held otherwise than built
             return None
-        return None if fields is None else block_forward(x, *fields[:-1], **fields[-1])
+        return block_forward(x, fields[0], fields[1], **fields[2]) if fields is not None else None
 
     def _native_fields(self, x, res):
-        if not _block_may_fuse(self, VRWKV_SpatialMix_V6, VRWKV_ChannelMix_V6, x):
+        if not _block_may_fuse(self, VRWKV_SpatialMix_V6, VRWKV_ChannelMix_V6):
             return None
         att, ffn = self._modules["att"], self._modules["ffn"]
         T, C = x.shape[1:]
@@ -184,7 +186,8 @@ class Block6(nn.Module):
         if not block_weights_fit(x, (*w.values(), *low.values())):
             return None
         params = {**low, **vec, **{n: w.pop(n) for n in ("att_kn_w", "att_kn_b") if n in w}}
-        return w, params, dict(num, Hp=res[0], Wp=res[1], heads=att.n_head, quarter=HEAD_SIZE // 4, gn_eps=ln_x.eps)
+        num.update(Hp=res[0], Wp=res[1], heads=att.n_head, quarter=HEAD_SIZE // 4, gn_eps=ln_x.eps)
+        return w, params, num
 
     def forward(self, x, patch_resolution):
         if self.layer_id == 0:
