@@ -180,19 +180,24 @@ def test_cut_sequence_with_a_decay_out_of_range(ops):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T", [300, 577, 1056, 1057])
-def test_one_rule_cuts_sequences_with_and_without_gradients(ops, T, dtype):
-    """The call that autograd records, the same call under no_grad with the bonus as a parameter, and the plain entry run the
-    same kernels on the same segments: bit-identical y."""
+def test_sequences_are_cut_where_autograd_records_nothing(ops, T, dtype):
+    """Under no_grad and inference_mode the bonus being a parameter changes nothing: bit-identical to the plain entry, which cuts.
+    What autograd records is whole in 16 bits up to 1056 tokens, and then the same in any batch."""
     H = 3
     assert ops.lib().vrwkv_wkv6_fwd_workspace_bytes(1, T, 64 * H, H) > 0
     r, k, v, w, u = (torch.from_numpy(x).cuda() for x in gen(1, T, H, seed=T, w_mean=-3.0, w_std=0.5))
     r, k, v, w = (x.to(dtype) for x in (r, k, v, w))
     u = torch.nn.Parameter(u)
-    want = ops.wkv6_forward(1, T, 64 * H, H, r, k, v, w, u.detach())
-    trained = ops.RUN_CUDA_RWKV6(1, T, 64 * H, H, r.requires_grad_(), k, v, w, u)
-    with torch.no_grad():
-        evaluated = ops.RUN_CUDA_RWKV6(1, T, 64 * H, H, r, k, v, w, u)
-    assert trained.grad_fn is not None and torch.equal(trained, want) and torch.equal(evaluated, want)
+    args = (1, T, 64 * H, H, r, k, v, w)
+    cut, whole = ops.wkv6_forward(*args, u.detach()), ops.wkv6_forward(*args, u.detach(), whole=True)
+    assert not torch.equal(cut, whole)
+    recorded = ops.RUN_CUDA_RWKV6(*args, u)
+    assert recorded.grad_fn is not None and torch.equal(recorded, whole if T <= 1056 and dtype == torch.bfloat16 else cut)
+    assert torch.equal(ops.RUN_CUDA_RWKV6(*args, u.detach()), cut)               # nothing requires a gradient
+    for mode in (torch.no_grad, torch.inference_mode):
+        with mode():
+            y = ops.RUN_CUDA_RWKV6(*args, u)
+        assert torch.equal(y, cut) and not y.requires_grad
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])

@@ -28,7 +28,7 @@ constexpr int BWD_SEG_FLOATS = 4 * SEG_STATE + HN;   // backward: S up, G up, S 
 
 // Segments of a sequence: the number with the least estimated time, where that is a fifth less than uncut.  Sequences of up to
 // 256 tokens stay whole, forward and backward: the results of a (b,h) then do not depend on how many others are in the call.
-// Those of longer sequences do, in their last bits, in both.  Costs are microseconds measured on bf16 calls: a step (one chunk) of the main kernel while its CU holds one workgroup, and more per further workgroup that its CU has to run
+// Those of longer sequences do, in their last bits (a caller that minds leaves the forward's workspace away).  Costs are microseconds measured on bf16 calls: a step (one chunk) of the main kernel while its CU holds one workgroup, and more per further workgroup that its CU has to run
 // (two at a time fit); the state kernel's step per workgroup on a CU; the scan and the extra launches.
 struct SegCosts { double one, each, state, fixed, per_segment; };
 // forward: at 24 sequences of 130 chunks uncut 358, 6 segments 103, 10 69, 21 64, 32 72; at 48 of 32 chunks uncut 90, 10

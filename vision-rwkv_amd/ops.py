@@ -190,9 +190,8 @@ def wkv6_forward(B, T, C, H, r, k, v, w, u, w_is_ew=False, out=None, whole=False
     that dtype, u (H,64); returns y (B,T,C) fp32.  With w_is_ew=False, w is the raw decay logit
     (the kernel applies d = exp(-exp(w))); with True it is ew = -exp(w_raw) as the reference
     extension receives it.  Sequences of more than 256 tokens are cut into segments where there are few of them, by their
-    number and length alone, in training as at inference; the last bits of y then depend on how many sequences there are.
-    whole: none is cut (a call without workspace), and they do not.  (Either is equally far from float64, 5.0e-6 in bf16 at
-    300 to 1024 tokens, and so are the gradients of twelve bf16 blocks from the fp32 model's, 2.7e-2 in the mean.)"""
+    number and length; the last bits of y then depend on how many sequences there are.  whole: none is cut (a call without
+    workspace), and they do not.  (Either is equally far from float64, 5.0e-6 in bf16 at 300 to 1024 tokens.)"""
     for t, n in ((r, "r"), (k, "k"), (v, "v"), (w, "w"), (u, "u")):
         _check_input(t, n)
     if tuple(r.shape) != (B, T, C) or k.shape != r.shape or v.shape != r.shape or w.shape != r.shape:
@@ -274,7 +273,18 @@ class WKV_6(torch.autograd.Function):
             assert w.is_contiguous()
             assert u.is_contiguous()
             ctx.save_for_backward(r, k, v, w, u)
-            return wkv6_forward(B, T, C, H, r, k, v, w, u)
+            return wkv6_forward(B, T, C, H, r, k, v, w, u, whole=WKV_6.stays_whole(T, r.dtype) and any(ctx.needs_input_grad))
+
+    # A 16-bit network rounds y again in every block and amplifies last bits: its gradients move by 3e-2 of their norm (twelve
+    # blocks, 400 to 1024 tokens, neither side closer to the fp32 model) when the forward is cut instead of whole, those of an fp32
+    # network by 4e-4 at most.  So a 16-bit forward that autograd records stays whole up to 33 chunks -- the 32 x 32 patches of a
+    # 512 x 512 image and a class token -- and a sample's y is the same in any batch; that costs up to 66 us a layer (3 / 24 / 96
+    # sequences of 1056 tokens: 92 / 94 / 95 us whole, 26 / 35 / 67 cut).  Longer chains cost more (2048 tokens: 175 whole, 34 to 115
+    # cut) and are cut.  The backward is cut from 257 tokens on in either type: gradients depend on the batch there, by 1.4e-2 in
+    # 16 bits.
+    @staticmethod
+    def stays_whole(T, dtype):
+        return T <= 33 * 32 and dtype != torch.float32
 
     @staticmethod
     def backward(ctx, gy):
@@ -287,9 +297,20 @@ class WKV_6(torch.autograd.Function):
             return (None, None, None, None, gr, gk, gv, gw, gu)
 
 
+class _WKV_6Unrecorded(WKV_6):
+    """WKV_6 where autograd records nothing.  Inside forward that cannot be seen: grad mode is off there anyway, and
+    needs_input_grad is set as soon as the bonus is a parameter."""
+
+    @staticmethod
+    def forward(ctx, B, T, C, H, r, k, v, w, u):
+        assert HEAD_SIZE == C // H
+        assert r.is_contiguous() and k.is_contiguous() and v.is_contiguous() and w.is_contiguous() and u.is_contiguous()
+        return wkv6_forward(B, T, C, H, r, k, v, w, u)
+
+
 def RUN_CUDA_RWKV6(B, T, C, H, r, k, v, w, u):
     """vrwkv6.py:72-73."""
-    return WKV_6.apply(B, T, C, H, r, k, v, w, u)
+    return (WKV_6 if torch.is_grad_enabled() else _WKV_6Unrecorded).apply(B, T, C, H, r, k, v, w, u)
 
 
 def q_shift(input, shift_pixel=1, gamma=1 / 4, patch_resolution=None):
