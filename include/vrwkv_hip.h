@@ -42,7 +42,7 @@ const char* vrwkv_last_error(void);      /* thread-local, never NULL */
  * that of the environment variable VRWKV_<NAME> when the library first looks at any switch; the entry points never read the environment afterwards.
  * vrwkv_set_option rejects (VRWKV_INVALID_ARG) a value the plans would ignore: biwkv_l takes 0, 4, 8, 16, 25, 28 (tokens
  * per wave), biwkv_s 0 or 2..8 (waves per workgroup), biwkv_grid 0 or a positive workgroup count, wkv6_segments 0..64 (segments a sequence
- * is cut into), linear_tile 0, 1, 2, 4, 8 (16 to 128 results on a side), wgrad_splits 0 or a positive count of token ranges, the
+ * is cut into), linear_tile 0, 1, 2, 4, 8 (16 to 128 results on a side), 16 (256 channels wide), wgrad_splits 0 or a positive count of token ranges, the
  * others 0 or 1. */
 int vrwkv_set_option(const char* name, int value);
 int vrwkv_get_option(const char* name, int* value);
@@ -267,6 +267,18 @@ typedef struct vrwkv_block6_params {
     int fp32_vectors;
 } vrwkv_block6_params;
 int vrwkv_block6_fwd(const vrwkv_block_args* args, const vrwkv_block6_params* params, void* hip_stream);
+
+/* ---- projections: several products of token matrices with weights in one launch ----
+ * out (M, N) = epilogue(a w^T): a (M, K) with rows at pitch lda, w (N, K) row-major, all of `dtype`, fp32 accumulation.  epi: bit 0 relu^2,
+ * bit 1 tanh, then, each optional (NULL): * sigmoid(gate) (M, N), * vec (N) (with bit 2: + vec), + res (M, N).  1 to 5 problems of the
+ * same M; N a multiple of 16, K of 32, lda of 8, every pointer 16-byte aligned.  The reference has no native code here (nn.Linear). */
+typedef struct vrwkv_linear {
+    const void *a, *w;
+    void* out;
+    const void *gate, *vec, *res;
+    int N, K, lda, epi;
+} vrwkv_linear;
+int vrwkv_linear_group(const vrwkv_linear* problems, int n, int M, int dtype, void* hip_stream);
 
 /* ---- weight gradients of the projections ----
  * out[z] (O, I) = sum over m of g[z][m][o] x[z][m][i], z < n: rows of g and x at pitches ldg, ldx (elements, multiples of 8),

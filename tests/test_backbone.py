@@ -627,7 +627,7 @@ def _small_backbone(kind, C, dtype, key_norm, post_norm, cls, hw, device="cuda")
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tile", [0, 1, 2, 4, 8])
+@pytest.mark.parametrize("tile", [0, 1, 2, 4, 8, 16])
 @pytest.mark.parametrize("kind,C,dtype,key_norm,post_norm,cls,hw,batch", [
     ("v4", 192, torch.bfloat16, False, False, False, (14, 14), 1), ("v4", 64, torch.float16, True, False, False, (1, 3), 24),
     ("v4", 416, torch.bfloat16, False, True, False, (7, 9), 3), ("v4", 256, torch.float16, True, True, False, (16, 15), 2),
@@ -768,6 +768,58 @@ def test_native_blocks_where_they_measured_faster(v6, dtype, M, C, called, recor
     for capturing, want in ((False, called), (True, recorded)):
         monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
         assert _native_size(x, 4 * C, v6) == want
+
+
+@pytest.mark.parametrize("v6,dtype,M,C,called,recorded", [
+    (False, torch.bfloat16, 12544, 768, True, True), (False, torch.bfloat16, 1568, 768, True, False), (False, torch.float16, 12544, 192, True, True),
+    (True, torch.bfloat16, 1568, 768, True, True), (True, torch.float16, 25088, 576, True, True), (False, torch.bfloat16, 12544, 640, False, False),
+    (False, torch.bfloat16, 12544, 1024, False, False), (False, torch.float32, 12544, 768, False, False),
+    (False, torch.bfloat16, 1 << 18, 768, False, False)])
+def test_native_blocks_of_wide_tiles_where_they_measured_faster(v6, dtype, M, C, called, recorded, monkeypatch):
+    """The rule against the measured points: called eagerly, and recorded into a graph (the last one: 32-bit offsets)."""
+    from vision_rwkv_amd.backbone import _native_wide
+    x = torch.empty(1, M, C, dtype=dtype, device="meta")
+    for capturing, want in ((False, called), (True, recorded)):
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+        assert _native_wide(x, 4 * C, v6) == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,Ns", [(1, 192, (16,)), (127, 128, (256, 272)), (160, 192, (768, 768, 768)), (1793, 192, (528, 64)), (225, 384, (784,)),
+                                    (449, 256, (240, 16, 512, 256, 32)), (24000, 192, (512,)), (20000, 128, (1024,)), (321, 1152, (32, 768))])
+def test_linear_group_of_wide_tiles(M, K, Ns, dtype):
+    """Partial tiles of tokens and channels, one and several rounds of workgroups, both counts of stages, every epilogue.  Against float64 of the
+    same 16-bit operands: the result's rounding (2^-9, 2^-12 relative) and K fp32 additions (K 2^-24 of the sum of magnitudes);
+    relu^2 doubles relative errors, so three times the rounding of the largest value bounds each."""
+    import ctypes
+    from vision_rwkv_amd import _lib, lib, option
+    torch.manual_seed(M + K)
+    d, n = "cuda", len(Ns)
+    A = [torch.randn(M, K + 8 * i, device=d).to(dtype)[:, :K] if i else torch.randn(M, K, device=d).to(dtype) for i in range(n)]
+    A = [a if a.stride(0) % 8 == 0 else a.contiguous() for a in A]
+    W = [(torch.randn(N, K, device=d) * K ** -0.5).to(dtype) for N in Ns]
+    for epi, extras in ((0, ()), (1, ("gate",)), (0, ("gate", "vec", "res")), (4, ("vec",))):
+        extra = [{"gate": torch.randn(M, N, device=d).to(dtype), "vec": torch.randn(N, device=d).to(dtype), "res": torch.randn(M, N, device=d).to(dtype)}
+                 for N in Ns]
+        out = [torch.full((M + 1, N), 7.0, device=d, dtype=dtype) for N in Ns]
+        ps = (_lib.Linear * n)(*[_lib.Linear(a=a.data_ptr(), w=w.data_ptr(), out=o.data_ptr(), N=N, K=K, lda=a.stride(0), epi=epi,
+                                             **{k: e[k].data_ptr() for k in extras}) for a, w, o, N, e in zip(A, W, out, Ns, extra)])
+        with option("linear_tile", 16):
+            _lib.check(lib().vrwkv_linear_group(ps, n, M, 1 if dtype == torch.bfloat16 else 2, torch.cuda.current_stream().cuda_stream))
+        for a, w, o, e in zip(A, W, out, extra):
+            ref = a.double() @ w.double().t()
+            if epi & 1:
+                ref = ref.relu().square()
+            if "gate" in extras:
+                ref = ref * torch.sigmoid(e["gate"].double())
+            if "vec" in extras:
+                ref = ref + e["vec"].double() if epi & 4 else ref * e["vec"].double()
+            if "res" in extras:
+                ref = ref + e["res"].double()
+            unit = 2.0 ** (-9 if dtype == torch.bfloat16 else -12)
+            assert (o[:M].double() - ref).abs().max() <= 3 * unit * max(ref.abs().max().item(), 1.0)
+            assert (o[M] == 7).all()
 
 
 @pytest.mark.gpu

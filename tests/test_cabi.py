@@ -173,6 +173,25 @@ def test_block_entries_validate_without_device(lib):
     assert lib.vrwkv_block6_fwd(None, None, None) == 1 and lib.vrwkv_block_fwd(None, None) == 1
 
 
+def test_linear_group_validates_without_device(lib):
+    from vision_rwkv_amd import _lib
+
+    def call(n=2, M=5, dtype=1, **change):
+        f = dict(a=4096, w=4096, out=4096, N=32, K=64, lda=64, epi=0)
+        return lib.vrwkv_linear_group((_lib.Linear * 2)(_lib.Linear(**f), _lib.Linear(**{**f, **change})), n, M, dtype, None)
+
+    assert call(n=0) == 1 and call(n=6) == 1 and lib.vrwkv_linear_group(None, 1, 1, 1, None) == 1
+    for name in ("a", "w", "out"):
+        assert call(**{name: 0}) == 1 and call(**{name: 4104}) == 1
+    for name in ("gate", "vec", "res"):
+        assert call(**{name: 4104}) == 1
+    assert call(epi=8) == 1
+    refused = call(dtype=9)
+    assert refused not in (0, 1)
+    for change in (dict(M=0), dict(N=24), dict(K=48), dict(lda=56), dict(lda=68), dict(M=1 << 24), dict(N=1 << 23)):
+        assert call(**change) not in (0, 1, refused), change
+
+
 def test_more_sequences_than_a_grid_holds_are_not_cut(lib):
     """A forced number of segments does not apply to more sequences than the fold kernel's grid has rows."""
     import vision_rwkv_amd as ops

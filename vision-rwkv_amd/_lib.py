@@ -29,6 +29,12 @@ class BlockArgs(ctypes.Structure):
                 + [(n, ctypes.c_void_p) for n in POINTERS_B] + [(n, ctypes.c_int) for n in INTS] + [(n, ctypes.c_float) for n in FLOATS])
 
 
+class Linear(ctypes.Structure):
+    """vrwkv_linear of include/vrwkv_hip.h."""
+    POINTERS = ("a", "w", "out", "gate", "vec", "res")
+    _fields_ = [(n, ctypes.c_void_p) for n in POINTERS] + [(n, ctypes.c_int) for n in ("N", "K", "lda", "epi")]
+
+
 class Block6Params(ctypes.Structure):
     """vrwkv_block6_params of include/vrwkv_hip.h."""
     POINTERS = ("maa_w1", "maa_w2", "decay_w1", "decay_w2", "maa_x", "maa_w", "maa_k", "maa_v", "maa_r", "maa_g", "ffn_mix_k", "ffn_mix_r",
@@ -128,6 +134,8 @@ def _declare(lib):
     lib.vrwkv_block_fwd.restype = i
     lib.vrwkv_block6_fwd.argtypes = [c.POINTER(BlockArgs), c.POINTER(Block6Params), vp]
     lib.vrwkv_block6_fwd.restype = i
+    lib.vrwkv_linear_group.argtypes = [c.POINTER(Linear), i, i, i, vp]
+    lib.vrwkv_linear_group.restype = i
     ll = c.c_longlong
     lib.vrwkv_wgrad_workspace_bytes.argtypes = [i, i, i, i]
     lib.vrwkv_wgrad_workspace_bytes.restype = sz

@@ -254,6 +254,24 @@ def _native_size(x, hidden, v6):
     return called and (recorded or not torch.cuda.is_current_stream_capturing())
 
 
+# In 16 bits the projections of many tokens go to a kernel of 256-channel tiles (csrc/linear_wide.hip) with three stages where C and the
+# hidden width are multiples of 192, and up to 768 channels such a block is ahead called eagerly at every size, recorded but for a
+# stretch where a block with key norms is 2 % behind (2352 x 768 1716 | 1753).  Operators -> native, eager | replayed:
+#   VRWKV  bf16  1568 x 768   3559 -> 1483 | 1595 -> 1480      3136 x 768, key norms 3597 -> 1901 | 1900 -> 1884      6272 x 768 3587 -> 2388 | 3064 -> 2384
+#                12544 x 768  4923 -> 3799 | 4887 -> 3785      25088 x 768  9237 -> 7356 | 9191 -> 7357      12544 x 192 3562 -> 1169 | 1483 -> 1158
+#   VRWKV6 bf16  1568 x 768   5887 -> 2246 | 2678 -> 2269      12544 x 768  7433 -> 6389 | 7422 -> 6383      12544 x 192 6272 -> 2069 | 2686 -> 2054
+NATIVE_WIDE, NATIVE_WIDE_GAP = 768, (600_000_000, 1_600_000_000)
+
+
+def _native_wide(x, hidden, v6):
+    """The rule above, and the offsets as there."""
+    B, T, C = x.shape
+    if (x.dtype == torch.float32 or C > NATIVE_WIDE or C % 192 or hidden % 192 or hidden == 0 or B * T * max(C, hidden) * 2 >= 1 << 30):
+        return False
+    lo, hi = NATIVE_WIDE_GAP
+    return v6 or C <= NATIVE_NARROW or not lo < B * T * C * C < hi or not torch.cuda.is_current_stream_capturing()
+
+
 def _as_built(module, kind):
     """True when calling `module` does what `kind`'s own forward does with the module's parameters and nothing else."""
     return (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks and "forward" not in module.__dict__)
@@ -268,7 +286,7 @@ def _block_weights(block, att, ffn, x):
     weight = key._parameters["weight"] if type(key) is nn.Linear else None
     hidden = weight.shape[0] if weight is not None else 0
     if not (C % 32 == 0 and hidden % 32 == 0 and 0 < hidden <= 4096 and att.fused_shift and ffn.fused_shift
-            and att.shift_pixel == ffn.shift_pixel and _native_size(x, hidden, "gate" in am)):
+            and att.shift_pixel == ffn.shift_pixel and (_native_wide(x, hidden, "gate" in am) or _native_size(x, hidden, "gate" in am))):
         return None
     w, num = {}, dict(hidden=hidden, shift_pixel=att.shift_pixel, post_norm=int(block.post_norm))
     for name, lin, shape in (("key", am["key"], (C, C)), ("value", am["value"], (C, C)), ("receptance", am["receptance"], (C, C)),

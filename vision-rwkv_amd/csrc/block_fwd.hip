@@ -6,7 +6,7 @@
 // library picks tiles of 192 x 256 for 196 x 192 results (13 us a product).  Issued from here a VRWKV block is 9 launches:
 //   LN | shift + mixes | key, value, receptance | Bi-WKV with gate | output + residual
 //   LN | shift + mixes | key with relu^2, receptance | value, gate, residual
-#include "gemm_tile.h"
+#include "linear.h"
 #include <algorithm>
 #include <type_traits>
 
@@ -20,19 +20,6 @@ namespace {
 // everything lies in the L2s and latency counts: a workgroup owns a tile of (16 MT)^2 results, its four waves take every
 // fourth slice of 64 bytes of k each with D slices requested ahead, and add up through LDS in a fixed order.  The weights are the
 // first operand, so a lane ends up with four neighbouring channels of a token: 8-byte accesses in the epilogue.
-enum { EPI_RELU_SQ = 1, EPI_TANH = 2, EPI_ADD_VEC = 4 };
-struct LinProblem {
-    const void *a, *w;
-    void* out;
-    const void *gate, *vec, *res;   // all optional: v *= sigmoid(gate); v *= vec (or v += vec with EPI_ADD_VEC); v += res
-    int N, K, lda, epi, tile0;
-};
-constexpr int LIN_MAX = 5;
-struct LinGroup {
-    LinProblem p[LIN_MAX];
-    int n, M;
-};
-
 using gemm::f32x4;
 using gemm::u32x4;
 // one 16-byte fragment of either operand: 32 k in 16 bits; in fp32 16 k as four products of 4, lane group g taking the k
@@ -51,31 +38,9 @@ template <typename IO> __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f
 // epilogue of four neighbouring channels n .. of token m
 template <typename IO>
 __device__ __forceinline__ void finish(const LinProblem& P, int m, int n, f32x4 s) {
-    const IO *gate = (const IO*)P.gate, *vec = (const IO*)P.vec, *res = (const IO*)P.res;
-    float v[4], x[4];
-    const size_t off = (size_t)m * P.N + n;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        v[e] = s[e];
-        if (P.epi & EPI_RELU_SQ) { const float r = fmaxf(v[e], 0.f); v[e] = r * r; }
-        if (P.epi & EPI_TANH) v[e] = tanhf(v[e]);
-    }
-    if (gate) {
-        load_vec<IO, 4>(gate + off, x);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] *= fast_rcp(1.f + fast_exp2(-LOG2E * x[e]));
-    }
-    if (vec) {
-        load_vec<IO, 4>(vec + n, x);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = P.epi & EPI_ADD_VEC ? v[e] + x[e] : v[e] * x[e];
-    }
-    if (res) {
-        load_vec<IO, 4>(res + off, x);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] += x[e];
-    }
-    store_vec<IO, 4>((IO*)P.out + off, v);
+    float v[4] = {s[0], s[1], s[2], s[3]};
+    epilogue<IO, 4>(P, m, n, v);
+    store_vec<IO, 4>((IO*)P.out + (size_t)m * P.N + n, v);
 }
 
 template <typename IO, int MT>
@@ -142,7 +107,7 @@ void linear_group_kernel(LinGroup G)
 }
 
 // The same with 128 x 128 tiles staged in LDS, for 16-bit calls that fill enough compute units with them: 64 x 64 tiles read
-// every operand piece twice as often straight from the L2s (12544 x 768, twelve blocks: 9957 us, with these 5472 us).
+// every operand piece twice as often straight from the L2s (three of 3136 x 768 x 768: 43 us, with these 21 us).
 template <typename IO>
 __global__ __launch_bounds__(256, 2)
 void linear_tile_kernel(LinGroup G)
@@ -187,22 +152,33 @@ void launch_group(LinGroup& G, int dtype, hipStream_t st) {
     else if (dtype == VRWKV_F16) hipLaunchKernelGGL((linear_group_kernel<__half, MT>), dim3(tiles), dim3(256), 0, st, G);
     else hipLaunchKernelGGL((linear_group_kernel<float, MT>), dim3(tiles), dim3(256), 0, st, G);
 }
-// Tile by the size of the result: larger tiles read less from the L2s, smaller ones give more workgroups and shorten the
-// chain of a wave.  Twelve bf16 blocks replayed as a graph, tiles of 64 / 128 on a side throughout, in us: 1568 x 768 2010 / 1751
-// (mixed by this rule 1721), 3136 x 384 1398 / 1297, 6272 x 384 2064 / 1550, 12544 x 768 9957 / 5472, 784 x 768 1339 / 1660; of
-// 16 / 32 / 64, eager: 784 x 768 2509 / 1672 / 1359, 3136 x 384 2499 / 1607 / 1417, 392 x 768 1544 / 1204 / 1163.
+}  // namespace
+
+// Kernel and tile by the number of results: larger tiles read less from the L2s, smaller ones give more workgroups and shorten the chain
+// of a wave.  64 x 64 from 128 tiles of that size on, 32 x 32 likewise; from 70 tiles of 128 x 128 on the wide kernel where it applies, else
+// 128 x 128.  (Between 70 and 256 such tiles the two are alike on rows that lie in the caches, as below, but inside a block, where they do not,
+// the wide kernel with its loads further ahead is faster: twelve blocks of 1568 x 768 1686 -> 1490 us, 12544 x 192 1322 -> 1160.)  us in bf16 with tiles of 16 / 32 / 64 / 128 / the wide kernel:
+//   784 x 192 x 192   3.2  3.1  4.6  6.6  7.3     784 x 768 x 768     16.3 11.0  9.2 12.9 13.4     784 x 3072 x 768      55   34   26   40   37
+//   three of them     5.6  4.7  4.9  6.9  7.7     three of them       39.7 24.0 15.6 14.2 14.6     1568 x 768 x 768      28.1 16.5 14.9 13.5 14.1
+//   6272 x 192 x 192, three  -  -   12.3 10.0  9.4 3136 x 384 x 384, three   -  -  17.2 10.7 11.6  6272 x 768 x 768      -    -    31.3 19.2 15.2
+//   3136 x 768 x 768  -    -   20.4 14.0 14.3     three of them       -    -   43.1 21.1 17.4      12544 x 768 x 768 three  -  -   158  64.1 52.5
+// (M x K x N)
 int linear_group(LinGroup& G, int dtype, hipStream_t st) {
     long long area = 0;
     for (int i = 0; i < G.n; ++i) area += (long long)G.M * G.p[i].N;
     const int force = option(OPT_LINEAR_TILE);
-    const bool wide = dtype != VRWKV_F32;                // 128 x 128 tiles are for 16 bits
-    const int mt = force && (wide || force < 8) ? force : wide && area >= 128LL * 128 * 110 ? 8 : area >= 64LL * 64 * 256 ? 4 : area >= 32LL * 32 * 128 ? 2 : 1;
+    const bool wide = dtype != VRWKV_F32;                // 128 x 128 tiles and wider ones are for 16 bits
+    if ((force ? force == 16 : area >= 128LL * 128 * 70) && wide_takes(G, dtype)) return wide_group(G, dtype, st);
+    const int mt = force && (wide || force < 8) ? std::min(force, 8)
+                   : wide ? (area >= 128LL * 128 * 70 ? 8 : area >= 64LL * 64 * 128 ? 4 : area >= 32LL * 32 * 128 ? 2 : 1)
+                          : (area >= 64LL * 64 * 256 ? 4 : area >= 32LL * 32 * 128 ? 2 : 1);
     if (mt == 8) launch_group<8>(G, dtype, st);
     else if (mt == 4) launch_group<4>(G, dtype, st);
     else if (mt == 2) launch_group<2>(G, dtype, st);
     else launch_group<1>(G, dtype, st);
     return check_launch("linear_group");
 }
+namespace {
 LinProblem linear(const void* a, const void* w, void* out, int N, int K, int lda = 0, int epi = 0) {
     return LinProblem{a, w, out, nullptr, nullptr, nullptr, N, K, lda ? lda : K, epi, 0};
 }
@@ -445,6 +421,41 @@ static int block_fwd(const vrwkv_block_args* args, const vrwkv_block6_params* pa
     LinProblem p = linear(hid, a->ffn_value, nullptr, C, hidden);
     p.gate = fr;
     return residual(p, x1, a->out, a->gamma2, a->ln2_w, a->ln2_b, a->ln2_eps, ftmp);
+}
+
+extern "C" int vrwkv_linear_group(const vrwkv_linear* problems, int n, int M, int dtype, void* hip_stream)
+{
+    using namespace vrwkv;
+    if (!problems || n <= 0 || n > LIN_MAX) {
+        set_error("linear_group: null argument, or not 1 to %d problems", LIN_MAX);
+        return VRWKV_INVALID_ARG;
+    }
+    if (dtype != VRWKV_F32 && dtype != VRWKV_BF16 && dtype != VRWKV_F16) {
+        set_error("linear_group: unknown dtype %d", dtype);
+        return VRWKV_UNSUPPORTED_DTYPE;
+    }
+    LinGroup G;
+    G.n = n;
+    G.M = M;
+    const long long es = dtype == VRWKV_F32 ? 4 : 2;
+    for (int i = 0; i < n; ++i) {
+        const vrwkv_linear& p = problems[i];
+        if (!p.a || !p.w || !p.out || (((size_t)p.a | (size_t)p.w | (size_t)p.out | (size_t)p.gate | (size_t)p.vec | (size_t)p.res) & 15)) {
+            set_error("linear_group: null or misaligned (16 bytes) pointer argument");
+            return VRWKV_INVALID_ARG;
+        }
+        if (M <= 0 || p.N <= 0 || p.K <= 0 || p.N % 16 || p.K % 32 || p.lda < p.K || p.lda % 8 || (M + 256LL) * std::max(p.lda, p.N) * es >= (1LL << 30) ||
+            (p.N + 256LL) * p.K * es >= (1LL << 30)) {
+            set_error("linear_group: unsupported sizes (M=%d N=%d K=%d lda=%d)", M, p.N, p.K, p.lda);
+            return VRWKV_UNSUPPORTED_SHAPE;
+        }
+        if (p.epi & ~(EPI_RELU_SQ | EPI_TANH | EPI_ADD_VEC)) {
+            set_error("linear_group: unknown epilogue %d", p.epi);
+            return VRWKV_INVALID_ARG;
+        }
+        G.p[i] = LinProblem{p.a, p.w, p.out, p.gate, p.vec, p.res, p.N, p.K, p.lda, p.epi, 0};
+    }
+    return linear_group(G, dtype, static_cast<hipStream_t>(hip_stream));
 }
 
 extern "C" int vrwkv_block_fwd(const vrwkv_block_args* args, void* hip_stream) { return block_fwd(args, nullptr, hip_stream); }

@@ -81,7 +81,7 @@ extern "C" int vrwkv_set_option(const char* name, int value) {
     if (i == vrwkv::OPT_BIWKV_S) ok = value == 0 || (value >= 2 && value <= 8);
     if (i == vrwkv::OPT_BIWKV_GRID) ok = value >= 0;
     if (i == vrwkv::OPT_WKV6_SEGMENTS) ok = value >= 0 && value <= 64;
-    if (i == vrwkv::OPT_LINEAR_TILE) ok = value == 0 || value == 1 || value == 2 || value == 4 || value == 8;
+    if (i == vrwkv::OPT_LINEAR_TILE) ok = value == 0 || value == 1 || value == 2 || value == 4 || value == 8 || value == 16;
     if (i == vrwkv::OPT_WGRAD_SPLITS) ok = value >= 0;
     if (!ok) {
         vrwkv::set_error("vrwkv_set_option: %d is no value of '%s'", value, name);

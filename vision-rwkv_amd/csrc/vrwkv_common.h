@@ -28,7 +28,7 @@ enum Option {
     OPT_WKV6_BWD_SCALAR,    // sequential wkv6 backward sweeps
     OPT_WKV6_BWD_UNFUSED,   // accepted, no effect (the backward is one kernel)
     OPT_WKV6_SEGMENTS,      // segments a wkv6 sequence is cut into
-    OPT_LINEAR_TILE,        // tile of the block entry's projections (1, 2, 4, 8: 16 to 128 results on a side)
+    OPT_LINEAR_TILE,        // tile of the block entry's projections (1, 2, 4, 8: 16 to 128 results on a side; 16: 256 channels wide)
     OPT_WGRAD_SPLITS,       // token ranges of a weight gradient
     N_OPTIONS
 };
