@@ -270,15 +270,20 @@ int vrwkv_block6_fwd(const vrwkv_block_args* args, const vrwkv_block6_params* pa
 
 /* ---- projections: several products of token matrices with weights in one launch ----
  * out (M, N) = epilogue(a w^T): a (M, K) with rows at pitch lda, w (N, K) row-major, all of `dtype`, fp32 accumulation.  epi: bit 0 relu^2,
- * bit 1 tanh, then, each optional (NULL): * sigmoid(gate) (M, N), * vec (N) (with bit 2: + vec), + res (M, N).  1 to 5 problems of the
- * same M; N a multiple of 16, K of 32, lda of 8, every pointer 16-byte aligned.  The reference has no native code here (nn.Linear). */
+ * bit 1 tanh, then, each optional (NULL): * sigmoid(gate) (M, N) (with bit 3: * 2 max(gate, 0), the derivative of relu^2 where gate was its
+ * argument), * vec (N) (with bit 2: + vec), + res (M, N).  raw (M, N), optional: the product itself as well;
+ * bit 4: the steps see the product rounded to `dtype`, as separate operators would.  1 to 5 problems of the same M; N a multiple of 16, K of 32, lda of 8, every pointer 16-byte aligned.  The reference has no native code here (nn.Linear). */
 typedef struct vrwkv_linear {
     const void *a, *w;
     void* out;
     const void *gate, *vec, *res;
+    void* raw;
     int N, K, lda, epi;
 } vrwkv_linear;
 int vrwkv_linear_group(const vrwkv_linear* problems, int n, int M, int dtype, void* hip_stream);
+/* dst[i] (cols, rows) = the transpose of src[i] (rows, cols), i < n <= 5, 16-bit elements, rows and cols multiples of 8 up to 65536,
+ * 16-byte aligned: the weights as the gradients of the projections' inputs take them. */
+int vrwkv_transpose_group(const void* const* src, void* const* dst, const int* rows, const int* cols, int n, void* hip_stream);
 
 /* ---- weight gradients of the projections ----
  * out[z] (O, I) = sum over m of g[z][m][o] x[z][m][i], z < n: rows of g and x at pitches ldg, ldx (elements, multiples of 8),

@@ -770,6 +770,92 @@ def test_native_blocks_where_they_measured_faster(v6, dtype, M, C, called, recor
         assert _native_size(x, 4 * C, v6) == want
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("shapes", [((8, 8),), ((72, 136), (64, 64), (8, 200)), ((768, 768), (3072, 768), (768, 3072), (192, 40), (40, 192))])
+def test_weights_transposed_in_one_launch(shapes):
+    from vision_rwkv_amd.ops import transposed
+    ws = [torch.randn(*s, device="cuda").bfloat16() for s in shapes]
+    for w, t in zip(ws, transposed(ws)):
+        assert torch.equal(t, w.t())
+
+
+def _norm_errors(got, plain, exact):
+    return [((a.double() - e).norm() / e.norm(), (b.double() - e).norm() / e.norm()) for a, b, e in zip(got, plain, exact)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,T,C,hidden", [(1, 6001, 192, 768), (2, 900, 768, 768), (3, 1500, 256, 512), (1, 4097, 384, 1152)])
+def test_projections_in_one_launch_and_channel_mix_against_float64(B, T, C, hidden, dtype, monkeypatch):
+    """Values and every gradient of grouped projections and of a channel mix whose element-wise steps are epilogues, against float64 of the
+    same 16-bit weights and inputs: the grouped path rounds at a subset of the places where the operators round (the weight
+    gradients are the same code), so it is no further off than they are; both errors are random, 1.1 is far outside their scatter over
+    10^5 elements and more."""
+    from vision_rwkv_amd import backbone as bb
+    monkeypatch.setattr(bb, "CHANNEL_MIX_TILES", 0)
+    torch.manual_seed(T)
+    d = "cuda"
+    ffn = bb.VRWKV_ChannelMix(C, 2, 0, hidden_rate=1).to(d)
+    ffn.key, ffn.value = torch.nn.Linear(C, hidden, bias=False, device=d), torch.nn.Linear(hidden, C, bias=False, device=d)
+    ffn.to(dtype)
+    lins = [torch.nn.Linear(C, C, bias=False, device=d).to(dtype) for _ in range(3)]
+    xs = [torch.randn(B, T, C, device=d).to(dtype).requires_grad_() for _ in range(3)]
+    gs = [torch.randn(B, T, C, device=d).to(dtype) for _ in range(4)]
+    params = [l.weight for l in (*lins, ffn.key, ffn.receptance, ffn.value)]
+
+    def run():
+        ys = bb._projs(lins, xs) + [bb._channel_mix(ffn, xs[0], xs[1])]
+        assert type(ys[0].grad_fn).__name__ == type(ys[1].grad_fn).__name__
+        return ys[0].grad_fn.name(), ys[3].grad_fn.name(), [y.detach() for y in ys] + list(torch.autograd.grad(ys, xs + params, gs))
+
+    n0, n3, got = run()
+    assert "_Projections" in n0 and "_ChannelMix" in n3
+    with torch.no_grad():                                    # without autograd: the same launches
+        for a, b in zip(bb._projs(lins, xs) + [bb._channel_mix(ffn, xs[0], xs[1])], got):
+            assert torch.equal(a, b)
+    monkeypatch.setattr(bb, "_own_weights", lambda *a: None)
+    n0, n3, plain = run()
+    assert "_Projections" not in n0 and "_ChannelMix" not in n3
+    x6, p6 = [x.detach().double().requires_grad_() for x in xs], [p.detach().double().requires_grad_() for p in params]
+    ys = [x @ w.t() for x, w in zip(x6, p6)]
+    ys.append(torch.sigmoid(x6[1] @ p6[4].t()) * ((x6[0] @ p6[3].t()).relu().square() @ p6[5].t()))
+    exact = [y.detach() for y in ys] + list(torch.autograd.grad(ys, x6 + p6, [g.double() for g in gs]))
+    for i, (a, b) in enumerate(_norm_errors(got, plain, exact)):
+        assert a <= 1.1 * b, (i, a, b)
+
+
+@pytest.mark.gpu
+def test_projections_with_hooks_frozen_parts_and_second_derivatives():
+    from vision_rwkv_amd import backbone as bb
+    torch.manual_seed(3)
+    d, C = "cuda", 192
+    lins = [torch.nn.Linear(C, C, bias=False, device=d).bfloat16() for _ in range(3)]
+    xs = [torch.randn(1, 6000, C, device=d).bfloat16().requires_grad_(i != 1) for i in range(3)]
+    lins[2].weight.requires_grad_(False)
+    ys = bb._projs(lins, xs)
+    assert "_Projections" in ys[0].grad_fn.name()
+    sum(y.float().square().sum() for y in ys).backward()
+    assert xs[0].grad is not None and xs[1].grad is None and lins[1].weight.grad is not None and lins[2].weight.grad is None
+    for add in ("register_forward_hook", "register_full_backward_hook"):
+        fired = []
+        handle = getattr(lins[1], add)(lambda *a: fired.append(1))
+        ys = bb._projs(lins, xs)
+        assert "_Projections" not in ys[0].grad_fn.name()
+        handle.remove()
+    # a gradient that is itself differentiated goes through tensor ops: d/dx of |dy/dx g|^2 of a relu^2 product
+    ffn = bb.VRWKV_ChannelMix(C, 2, 0).to(d).bfloat16()
+    x, r = (torch.randn(1, 22000, C, device=d).bfloat16().requires_grad_() for _ in range(2))
+    y = bb._channel_mix(ffn, x, r)
+    assert "_ChannelMix" in y.grad_fn.name()
+    g, = torch.autograd.grad(y, x, torch.ones_like(y), create_graph=True)
+    gg, = torch.autograd.grad(g.float().square().sum(), x)
+    X, R = x.detach().double().requires_grad_(), r.detach().double()
+    wk, wr, wv = (l.weight.detach().double() for l in (ffn.key, ffn.receptance, ffn.value))
+    G, = torch.autograd.grad((torch.sigmoid(R @ wr.t()) * ((X @ wk.t()).relu().square() @ wv.t())).sum(), X, create_graph=True)
+    GG, = torch.autograd.grad(G.square().sum(), X)
+    assert (gg.double() - GG).norm() <= 3e-2 * GG.norm()      # some eight bf16 roundings of 2^-9 = 2e-3, each of a differing sign pattern
+
+
 @pytest.mark.parametrize("v6,dtype,M,C,called,recorded", [
     (False, torch.bfloat16, 12544, 768, True, True), (False, torch.bfloat16, 1568, 768, True, False), (False, torch.float16, 12544, 192, True, True),
     (True, torch.bfloat16, 1568, 768, True, True), (True, torch.float16, 25088, 576, True, True), (False, torch.bfloat16, 12544, 640, False, False),

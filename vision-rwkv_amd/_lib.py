@@ -31,7 +31,7 @@ class BlockArgs(ctypes.Structure):
 
 class Linear(ctypes.Structure):
     """vrwkv_linear of include/vrwkv_hip.h."""
-    POINTERS = ("a", "w", "out", "gate", "vec", "res")
+    POINTERS = ("a", "w", "out", "gate", "vec", "res", "raw")
     _fields_ = [(n, ctypes.c_void_p) for n in POINTERS] + [(n, ctypes.c_int) for n in ("N", "K", "lda", "epi")]
 
 
@@ -136,6 +136,8 @@ def _declare(lib):
     lib.vrwkv_block6_fwd.restype = i
     lib.vrwkv_linear_group.argtypes = [c.POINTER(Linear), i, i, i, vp]
     lib.vrwkv_linear_group.restype = i
+    lib.vrwkv_transpose_group.argtypes = [c.POINTER(vp), c.POINTER(vp), c.POINTER(i), c.POINTER(i), i, vp]
+    lib.vrwkv_transpose_group.restype = i
     ll = c.c_longlong
     lib.vrwkv_wgrad_workspace_bytes.argtypes = [i, i, i, i]
     lib.vrwkv_wgrad_workspace_bytes.restype = sz

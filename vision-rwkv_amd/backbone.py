@@ -15,7 +15,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch.nn.modules import module as _hooks
 
-from .ops import (RUN_CUDA, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, weight_grad, block_takes, block_weights_fit, block_forward, _equal_quarters, _transformed, batched_cotangent, PRE_NONE, PRE_RELU_SQ, POST_NONE,
+from . import ops
+from .ops import (RUN_CUDA, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, weight_grad, linear_takes, linear_group, transposed, sigmoid_gate_backward, EPI_RELU_SQ, EPI_RELU_SQ_BWD, EPI_ROUND, block_takes, block_weights_fit, block_forward, _equal_quarters, _transformed, batched_cotangent, PRE_NONE, PRE_RELU_SQ, POST_NONE,
                   POST_SIGMOID_GATE, POST_RESIDUAL)
 
 
@@ -202,6 +203,136 @@ def _proj(linear, x):
     return linear(x)
 
 
+def _rows(t):
+    return t.reshape(-1, t.shape[-1])
+
+
+def _plain_backward(*tensors):
+    """True where a backward may launch kernels: nothing records, batches or traces it."""
+    return not torch.is_grad_enabled() and not batched_cotangent(*tensors) and not _transformed()
+
+
+def _weight_product(g, x):
+    """The gradient g^T x of a projection's weight (see _SplitKLinear)."""
+    return _token_product(_rows(g), _rows(x), 4 if g.shape[-1] * x.shape[-1] >= 1 << 21 else 8)
+
+
+class _Projections(torch.autograd.Function):
+    """[x @ W^T for x, W in zip(xs, ws)] as one launch (vrwkv_linear_group), the gradients of the inputs likewise."""
+
+    @staticmethod
+    def forward(ctx, *xw):
+        ctx.save_for_backward(*xw)
+        n = len(xw) // 2
+        outs = linear_group([dict(a=_rows(x), w=w) for x, w in zip(xw[:n], xw[n:])])
+        return tuple(o.reshape(*x.shape[:-1], -1) for o, x in zip(outs, xw))
+
+    @staticmethod
+    def backward(ctx, *gs):
+        xw, n = ctx.saved_tensors, len(gs)
+        xs, ws = xw[:n], xw[n:]
+        gx, gw = [None] * n, [None] * n
+        need = [i for i in range(n) if ctx.needs_input_grad[i]]
+        if _plain_backward(*gs) and len(need) > 1:
+            outs = linear_group([dict(a=_rows(gs[i]), w=wt) for i, wt in zip(need, transposed([ws[i] for i in need]))])
+            for i, o in zip(need, outs):
+                gx[i] = o.reshape(xs[i].shape)
+        else:
+            for i in need:
+                gx[i] = gs[i] @ ws[i]
+        for i in range(n):
+            if ctx.needs_input_grad[n + i]:
+                gw[i] = _weight_product(gs[i], xs[i])
+        return (*gx, *gw)
+
+
+class _ChannelMix(torch.autograd.Function):
+    """sigmoid(xr @ Wr^T) * (relu^2(xk @ Wk^T) @ Wv^T) (vrwkv.py:250-261 without key_norm): key and receptance in one launch, and every
+    element-wise step, forward and backward, in the epilogue of the product before it: the (tokens, hidden) matrices, four times as
+    wide as x, are written once and not read again to be squared or masked.  The steps see the products rounded, as the
+    operators one by one do: a network of 16-bit activations amplifies last bits (VRWKV6: 3e-2 of its gradients' norm)."""
+
+    @staticmethod
+    def forward(ctx, xk, xr, wk, wr, wv):
+        (kk, k), r = linear_group([dict(a=_rows(xk), w=wk, epi=EPI_RELU_SQ | EPI_ROUND, raw=True), dict(a=_rows(xr), w=wr)])
+        out, y = linear_group([dict(a=kk, w=wv, gate=r, epi=EPI_ROUND, raw=True)])[0]
+        ctx.save_for_backward(xk, xr, wk, wr, wv, k, kk, r, y)
+        return out.reshape(xk.shape)
+
+    @staticmethod
+    def backward(ctx, g):
+        xk, xr, wk, wr, wv, k, kk, r, y = ctx.saved_tensors
+        plain = _plain_backward(g)
+        g2 = _rows(g)
+        if plain:
+            g2 = g2.to(y.dtype).contiguous()
+            plain = g2.data_ptr() % 16 == 0
+        if plain:
+            gy, gr = sigmoid_gate_backward(y, r, g2)
+            wkt, wrt, wvt = transposed([wk, wr, wv])
+            gk = linear_group([dict(a=gy, w=wvt, gate=k, epi=EPI_RELU_SQ_BWD | EPI_ROUND)])[0]
+            gxk, gxr = (t.reshape(xk.shape) for t in linear_group([dict(a=gk, w=wkt), dict(a=gr, w=wrt)]))
+        else:                                                # from the inputs anew, so that it can be differentiated again
+            k, r = F.linear(_rows(xk), wk), F.linear(_rows(xr), wr)
+            kk = torch.square(torch.relu(k))
+            s = torch.sigmoid(r)
+            gy, gr = g2 * s, g2 * F.linear(kk, wv) * s * (1 - s)
+            gk = (gy @ wv) * (2 * torch.relu(k))
+            gxk, gxr = (gk @ wk).reshape(g.shape), (gr @ wr).reshape(g.shape)
+        need = ctx.needs_input_grad
+        return (gxk if need[0] else None, gxr if need[1] else None, _weight_product(gk, xk) if need[2] else None,
+                _weight_product(gr, xr) if need[3] else None, _weight_product(gy, kk) if need[4] else None)
+
+
+# Where the grouped launches take the place of the library's products.  Two or more projections of one shape on M tokens in one launch
+# are ahead from 70 tiles of 128 x 128 each on; a single one without an epilogue stays with the library.  M x K x N, library / own, us:
+#   three of 784 x 768 x 768 23 / 15    4096 35 / 22    8192 46 / 37    11760 60 / 53    12544 79 / 52    (one: 7.6 / 13, 12 / 15, 15 / 17, 20 / 21, 27 / 21)
+#   three of 784 x 1024 x 1024 27 / 19  4096 41 / 33    9216 90 / 65    10816 79 / 84    12544 84 / 82    three of 12544 x 384 x 384 33 / 23
+# A whole channel mix without key_norm takes them from 256 tiles on, where the passes they save (28 us forward, 43 back at 12544 x 3072)
+# outweigh a slower product: 4096 x 3072 x 768 30 / 39, 8192 44 / 41, 12544 60 / 55; 12544 x 768 x 3072 64 / 67; 12544 x 4096 x 1024 83 / 90.
+# Training steps of 64 images of 224 x 224, start and both of these: VRWKV-B 16195 -> 15108 us, VRWKV6-B 25761 -> 24499, bit for bit the same.
+CHANNEL_MIX_TILES = 256 * 128 * 128
+
+
+def _own_weights(linears, x):
+    """The weights of projections whose module call does nothing but multiply, and which vrwkv_linear_group takes; else None."""
+    if (_hooks._global_forward_hooks or _hooks._global_forward_pre_hooks or _hooks._global_backward_hooks
+            or _hooks._global_backward_pre_hooks):
+        return None
+    for l in linears:
+        if not _as_built(l, nn.Linear) or l._backward_hooks or l._backward_pre_hooks or l.bias is not None or type(l._parameters.get("weight")) is not nn.Parameter:
+            return None
+    ws = [l.weight for l in linears]
+    return ws if linear_takes(x, ws) else None
+
+
+def _projs(linears, xs):
+    """[linear(x) for linear, x in zip(linears, xs)] for projections of one shape."""
+    ws = _own_weights(linears, xs[0]) if type(xs[0]) is torch.Tensor and all(x.shape == xs[0].shape and x.dtype == xs[0].dtype for x in xs) else None
+    if ws is None:
+        return [_proj(l, x) for l, x in zip(linears, xs)]
+    if torch.is_grad_enabled() and any(t.requires_grad for t in (*xs, *ws)):
+        return list(_Projections.apply(*xs, *ws))
+    return [o.reshape(*x.shape[:-1], -1) for o, x in zip(linear_group([dict(a=_rows(x), w=w) for x, w in zip(xs, ws)]), xs)]
+
+
+def _channel_mix(ffn, xk, xr):
+    """What a channel mix makes of its two mixed inputs (vrwkv.py:250-261), by the rules above."""
+    kn = ffn.key_norm
+    if kn is None and ops.ROW_FUSE_ENABLED and type(xk) is type(xr) is torch.Tensor and xk.shape == xr.shape and xk.dtype == xr.dtype and xk.numel() >= CHANNEL_MIX_TILES:
+        ws = _own_weights((ffn.key, ffn.receptance, ffn.value), xk)
+        if ws is not None:
+            wk, wr, wv = ws
+            if torch.is_grad_enabled() and any(t.requires_grad for t in (xk, xr, *ws)):
+                return _ChannelMix.apply(xk, xr, wk, wr, wv)
+            kk, r = linear_group([dict(a=_rows(xk), w=wk, epi=EPI_RELU_SQ | EPI_ROUND), dict(a=_rows(xr), w=wr)])
+            return linear_group([dict(a=kk, w=wv, gate=r, epi=EPI_ROUND)])[0].reshape(xk.shape)
+    # relu^2 (+ key_norm) and the sigmoid gate (vrwkv.py:256-261), one pass each; tensor ops under autograd
+    k = row_fuse(_proj(ffn.key, xk), None, kn.weight if kn is not None else None, kn.bias if kn is not None else None, None,
+                 PRE_RELU_SQ, POST_NONE, kn.eps if kn is not None else 1e-5)
+    return row_fuse(_proj(ffn.value, k), _proj(ffn.receptance, xr), None, None, None, PRE_NONE, POST_SIGMOID_GATE)
+
+
 def _layer_norm(ln, x):
     """nn.LayerNorm over the channels through the fused row kernel (forward and backward); tensor ops where it does
     not apply."""
@@ -352,7 +483,7 @@ class VRWKV_SpatialMix(nn.Module):
                               self.channel_gamma, patch_resolution, self.fused_shift)
         else:
             xk = xv = xr = x
-        k, v, r = _proj(self.key, xk), _proj(self.value, xv), _proj(self.receptance, xr)
+        k, v, r = _projs((self.key, self.value, self.receptance), (xk, xv, xr))
         wd = self.spatial_decay.dtype
         if torch.is_grad_enabled() or k.dtype != (wd if wd in (torch.half, torch.bfloat16) else torch.float32):
             y = RUN_CUDA(self.spatial_decay / T, self.spatial_first / T, k, v)  # vrwkv.py:183
@@ -394,11 +525,7 @@ class VRWKV_ChannelMix(nn.Module):
                           patch_resolution, self.fused_shift)
         else:
             xk = xr = x
-        # relu^2 (+ key_norm) and the sigmoid gate (vrwkv.py:256-261), one pass each; tensor ops under autograd
-        kn = self.key_norm
-        k = row_fuse(_proj(self.key, xk), None, kn.weight if kn is not None else None, kn.bias if kn is not None else None, None,
-                     PRE_RELU_SQ, POST_NONE, kn.eps if kn is not None else 1e-5)
-        return row_fuse(_proj(self.value, k), _proj(self.receptance, xr), None, None, None, PRE_NONE, POST_SIGMOID_GATE)
+        return _channel_mix(self, xk, xr)
 
 
 class Block(nn.Module):

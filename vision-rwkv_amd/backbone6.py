@@ -10,7 +10,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .backbone import VRWKV, eval_cached, _proj, _matmul, _bmm, _as_built, _block_may_fuse, _block_weights
+from .backbone import VRWKV, eval_cached, _proj, _projs, _channel_mix, _matmul, _bmm, _as_built, _block_may_fuse, _block_weights
 from .ops import (HEAD_SIZE, RUN_CUDA_RWKV6, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, maa_mix, groupnorm_gate, block_takes, block_weights_fit, block_forward, PRE_NONE, PRE_RELU_SQ, POST_NONE,
                   POST_SIGMOID_GATE, POST_RESIDUAL)
 
@@ -93,8 +93,7 @@ class VRWKV_SpatialMix_V6(nn.Module):
         if not torch.is_grad_enabled() and x.is_cuda:
             table = eval_cached(self, "maa_table", maas, x.device, lambda: stack_mixes(maas, x.device))
         xw, xk, xv, xr, xg = maa_mix(x, sx, m, maas, table)
-        r, k, v = _proj(self.receptance, xr), _proj(self.key, xk), _proj(self.value, xv)
-        gate = _proj(self.gate, xg)
+        r, k, v, gate = _projs((self.receptance, self.key, self.value, self.gate), (xr, xk, xv, xg))
         w = self.time_decay + _matmul(torch.tanh(_matmul(xw, self.time_decay_w1)), self.time_decay_w2)
         y = RUN_CUDA_RWKV6(B, T, C, self.n_head, r.contiguous(), k.contiguous(), v.contiguous(),
                            w.contiguous(), self.time_faaaa.float())                  # vrwkv6.py:217 (w as it is: the
@@ -126,10 +125,7 @@ class VRWKV_ChannelMix_V6(nn.Module):
         xk, xr = _shift_and_mix(self, x, lambda: [self.spatial_mix_k, self.spatial_mix_r], self.shift_pixel,
                                 patch_resolution, self.with_cls_token, self.fused_shift,
                                 (self.spatial_mix_k, self.spatial_mix_r))
-        kn = self.key_norm                                   # relu^2 (+ key_norm), then the sigmoid gate: one pass each
-        k = row_fuse(_proj(self.key, xk), None, kn.weight if kn is not None else None, kn.bias if kn is not None else None, None,
-                     PRE_RELU_SQ, POST_NONE, kn.eps if kn is not None else 1e-5)
-        return row_fuse(_proj(self.value, k), _proj(self.receptance, xr), None, None, None, PRE_NONE, POST_SIGMOID_GATE)
+        return _channel_mix(self, xk, xr)
 
 
 class Block6(nn.Module):

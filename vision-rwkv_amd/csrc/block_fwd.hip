@@ -180,7 +180,7 @@ int linear_group(LinGroup& G, int dtype, hipStream_t st) {
 }
 namespace {
 LinProblem linear(const void* a, const void* w, void* out, int N, int K, int lda = 0, int epi = 0) {
-    return LinProblem{a, w, out, nullptr, nullptr, nullptr, N, K, lda ? lda : K, epi, 0};
+    return LinProblem{a, w, out, nullptr, nullptr, nullptr, N, K, lda ? lda : K, epi, 0, nullptr};
 }
 
 // ---- the block -----------------------------------------------------------------------------------------------------------
@@ -440,7 +440,7 @@ extern "C" int vrwkv_linear_group(const vrwkv_linear* problems, int n, int M, in
     const long long es = dtype == VRWKV_F32 ? 4 : 2;
     for (int i = 0; i < n; ++i) {
         const vrwkv_linear& p = problems[i];
-        if (!p.a || !p.w || !p.out || (((size_t)p.a | (size_t)p.w | (size_t)p.out | (size_t)p.gate | (size_t)p.vec | (size_t)p.res) & 15)) {
+        if (!p.a || !p.w || !p.out || (((size_t)p.a | (size_t)p.w | (size_t)p.out | (size_t)p.gate | (size_t)p.vec | (size_t)p.res | (size_t)p.raw) & 15)) {
             set_error("linear_group: null or misaligned (16 bytes) pointer argument");
             return VRWKV_INVALID_ARG;
         }
@@ -449,11 +449,11 @@ extern "C" int vrwkv_linear_group(const vrwkv_linear* problems, int n, int M, in
             set_error("linear_group: unsupported sizes (M=%d N=%d K=%d lda=%d)", M, p.N, p.K, p.lda);
             return VRWKV_UNSUPPORTED_SHAPE;
         }
-        if (p.epi & ~(EPI_RELU_SQ | EPI_TANH | EPI_ADD_VEC)) {
+        if (p.epi & ~(EPI_RELU_SQ | EPI_TANH | EPI_ADD_VEC | EPI_RELU_SQ_BWD | EPI_ROUND) || (p.epi & EPI_RELU_SQ_BWD && !p.gate)) {
             set_error("linear_group: unknown epilogue %d", p.epi);
             return VRWKV_INVALID_ARG;
         }
-        G.p[i] = LinProblem{p.a, p.w, p.out, p.gate, p.vec, p.res, p.N, p.K, p.lda, p.epi, 0};
+        G.p[i] = LinProblem{p.a, p.w, p.out, p.gate, p.vec, p.res, p.N, p.K, p.lda, p.epi, 0, p.raw};
     }
     return linear_group(G, dtype, static_cast<hipStream_t>(hip_stream));
 }

@@ -6,12 +6,13 @@
 namespace vrwkv {
 
 // A (M, K) with row pitch lda, W (N, K), out (M, N), of one type, with fp32 accumulation.
-enum { EPI_RELU_SQ = 1, EPI_TANH = 2, EPI_ADD_VEC = 4 };
+enum { EPI_RELU_SQ = 1, EPI_TANH = 2, EPI_ADD_VEC = 4, EPI_RELU_SQ_BWD = 8, EPI_ROUND = 16 };
 struct LinProblem {
     const void *a, *w;
     void* out;
-    const void *gate, *vec, *res;   // all optional: v *= sigmoid(gate); v *= vec (or v += vec with EPI_ADD_VEC); v += res
+    const void *gate, *vec, *res;   // all optional: v *= sigmoid(gate) (2 max(gate, 0) with EPI_RELU_SQ_BWD); v *= vec (or v += vec with EPI_ADD_VEC); v += res
     int N, K, lda, epi, tile0;
+    void* raw;                      // optional: the product itself, beside the result.  EPI_ROUND: the steps above see it rounded to its type
 };
 constexpr int LIN_MAX = 5;
 struct LinGroup {
@@ -25,6 +26,11 @@ __device__ __forceinline__ void epilogue(const LinProblem& P, int m, int n, floa
     const IO *gate = (const IO*)P.gate, *vec = (const IO*)P.vec, *res = (const IO*)P.res;
     const size_t off = (size_t)m * P.N + n;
     float x[V];
+    if (P.epi & EPI_ROUND) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[e] = to_f32(from_f32<IO>(v[e]));
+    }
+    if (P.raw) store_vec<IO, V>((IO*)P.raw + off, v);
     if (P.epi & EPI_RELU_SQ) {
 #pragma unroll
         for (int e = 0; e < V; ++e) { const float r = fmaxf(v[e], 0.f); v[e] = r * r; }
@@ -36,7 +42,7 @@ __device__ __forceinline__ void epilogue(const LinProblem& P, int m, int n, floa
     if (gate) {
         load_vec<IO, V>(gate + off, x);
 #pragma unroll
-        for (int e = 0; e < V; ++e) v[e] *= fast_rcp(1.f + fast_exp2(-LOG2E * x[e]));
+        for (int e = 0; e < V; ++e) v[e] *= P.epi & EPI_RELU_SQ_BWD ? 2.f * fmaxf(x[e], 0.f) : fast_rcp(1.f + fast_exp2(-LOG2E * x[e]));
     }
     if (vec) {
         load_vec<IO, V>(vec + n, x);

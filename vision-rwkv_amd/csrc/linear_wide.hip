@@ -180,11 +180,17 @@ void linear_wide_kernel(LinGroup G, int tiles)
         // counted).  The rows that an epilogue reads are requested a token ahead.
         typedef BufRaw<16>::type piece_t;
         const unsigned bytes = (unsigned)G.M * P.N * 2u;
-        const __amdgpu_buffer_rsrc_t ro = make_rsrc(P.out, bytes), rg = make_rsrc(P.gate, bytes), rr = make_rsrc(P.res, bytes);
+        const __amdgpu_buffer_rsrc_t ro = make_rsrc(P.out, bytes), rg = make_rsrc(P.gate, bytes), rr = make_rsrc(P.res, bytes), rp = make_rsrc(P.raw, bytes);
         const int n = n0 + 64 * wn + 16 * g4;
         auto at = [&](int i) {
             const int m = m0 + (wm * FM + i) * 16 + c16;
             return m < G.M && n < P.N ? ((unsigned)m * P.N + n) * 2u : OOB_OFFSET;
+        };
+        auto pack = [](piece_t& p, const float (&v)[8]) {
+            IO b[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) b[e] = from_f32<IO>(v[e]);
+            __builtin_memcpy(&p, b, 16);
         };
         piece_t gate[2], res[2], vec[2] = {};
         auto fetch = [&](unsigned o) {
@@ -205,11 +211,25 @@ void linear_wide_kernel(LinGroup G, int tiles)
             piece_t out[2];
 #pragma unroll
             for (int j = 0; j < FN; ++j) asm volatile("" : "+a"(acc[i][j]));         // not copied out before its turn
+            if (P.raw) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    float v[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] = acc[i][2 * h + (e >> 2)][e & 3];
+                    pack(out[h], v);
+                    BufRaw<16>::st(out[h], rp, o, 16 * h);
+                }
+            }
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 float v[8], x[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) v[e] = acc[i][2 * h + (e >> 2)][e & 3];
+                if (P.epi & EPI_ROUND) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] = to_f32(from_f32<IO>(v[e]));
+                }
                 if (P.epi & EPI_RELU_SQ) {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) { const float r = fmaxf(v[e], 0.f); v[e] = r * r; }
@@ -217,7 +237,8 @@ void linear_wide_kernel(LinGroup G, int tiles)
                 if (P.gate) {
                     widen_raw16<IO, 8>(gate[h], x);
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) v[e] *= fast_rcp(1.f + fast_exp2(-LOG2E * x[e]));
+                    for (int e = 0; e < 8; ++e)
+                        v[e] *= P.epi & EPI_RELU_SQ_BWD ? 2.f * fmaxf(x[e], 0.f) : fast_rcp(1.f + fast_exp2(-LOG2E * x[e]));
                 }
                 if (P.vec) {
                     widen_raw16<IO, 8>(vec[h], x);
@@ -229,10 +250,7 @@ void linear_wide_kernel(LinGroup G, int tiles)
 #pragma unroll
                     for (int e = 0; e < 8; ++e) v[e] += x[e];
                 }
-                IO b[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) b[e] = from_f32<IO>(v[e]);
-                __builtin_memcpy(&out[h], b, 16);
+                pack(out[h], v);
             }
             if (i + 1 < FM) fetch(at(i + 1));
 #pragma unroll
@@ -294,6 +312,37 @@ void launch_tile(LinGroup& G, hipStream_t st) {
     default: return launch<IO, 7, 2>(G, cus, st);
     }
 }
+// ---- weights with the contraction index innermost, for the gradients of the inputs (g W = g (W^T)^T) ----
+// 64 x 64 tiles turned through LDS, 16-byte accesses on either side; one launch for the matrices of a backward (3 x 768 x 768: 4 us).
+struct Turn { const void* src[LIN_MAX]; void* dst[LIN_MAX]; int rows[LIN_MAX], cols[LIN_MAX], tile0[LIN_MAX], n; };
+__global__ __launch_bounds__(256)
+void transpose_kernel(Turn T)
+{
+    __shared__ unsigned short tile[64][66];               // 33 banks a row: neither direction meets a bank twice
+    int q = 0;
+    while (q + 1 < T.n && (int)blockIdx.x >= T.tile0[q + 1]) ++q;
+    const int rows = T.rows[q], cols = T.cols[q], nc = (cols + 63) / 64, l = blockIdx.x - T.tile0[q], r0 = l / nc * 64, c0 = l % nc * 64;
+    const unsigned short* src = (const unsigned short*)T.src[q];
+    unsigned short* dst = (unsigned short*)T.dst[q];
+    const int x = 8 * (threadIdx.x & 7), y = threadIdx.x >> 3;
+#pragma unroll
+    for (int i = 0; i < 64; i += 32)
+        if (r0 + y + i < rows && c0 + x < cols) {
+            const nt_u32x4 v = load_raw16<false>(src + (size_t)(r0 + y + i) * cols + c0 + x);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { tile[y + i][x + 2 * e] = (unsigned short)v[e]; tile[y + i][x + 2 * e + 1] = (unsigned short)(v[e] >> 16); }
+        }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 64; i += 32)
+        if (c0 + y + i < cols && r0 + x < rows) {
+            nt_u32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = tile[x + 2 * e][y + i] | (unsigned)tile[x + 2 * e + 1][y + i] << 16;
+            *reinterpret_cast<nt_u32x4*>(dst + (size_t)(c0 + y + i) * rows + r0 + x) = v;
+        }
+}
+
 }  // namespace
 
 // 16-bit problems whose contraction is a whole number of turns of the loop (and whose epilogue is not the low-rank maps' tanh); byte
@@ -319,3 +368,29 @@ int wide_group(LinGroup& G, int dtype, hipStream_t st) {
 }
 
 }  // namespace vrwkv
+
+extern "C" int vrwkv_transpose_group(const void* const* src, void* const* dst, const int* rows, const int* cols, int n, void* hip_stream)
+{
+    using namespace vrwkv;
+    if (!src || !dst || !rows || !cols || n <= 0 || n > LIN_MAX) {
+        set_error("transpose_group: null argument, or not 1 to %d matrices", LIN_MAX);
+        return VRWKV_INVALID_ARG;
+    }
+    Turn T;
+    T.n = n;
+    int tiles = 0;
+    for (int i = 0; i < n; ++i) {
+        if (!src[i] || !dst[i] || (((size_t)src[i] | (size_t)dst[i]) & 15)) {
+            set_error("transpose_group: null or misaligned (16 bytes) pointer argument");
+            return VRWKV_INVALID_ARG;
+        }
+        if (rows[i] <= 0 || cols[i] <= 0 || rows[i] % 8 || cols[i] % 8 || rows[i] > 65536 || cols[i] > 65536) {
+            set_error("transpose_group: unsupported sizes (%d x %d)", rows[i], cols[i]);
+            return VRWKV_UNSUPPORTED_SHAPE;
+        }
+        T.src[i] = src[i]; T.dst[i] = dst[i]; T.rows[i] = rows[i]; T.cols[i] = cols[i]; T.tile0[i] = tiles;
+        tiles += ((rows[i] + 63) / 64) * ((cols[i] + 63) / 64);
+    }
+    hipLaunchKernelGGL(transpose_kernel, dim3(tiles), dim3(256), 0, static_cast<hipStream_t>(hip_stream), T);
+    return check_launch("transpose_group");
+}

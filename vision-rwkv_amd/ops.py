@@ -834,3 +834,68 @@ def weight_grad(g, x):
         _lib.check(L.vrwkv_wgrad(g3.data_ptr(), x3.data_ptr(), out.data_ptr(), n, M, O, I, gs[1], xs[1], gs[0], xs[0],
                                  _DT[g.dtype], ws.data_ptr(), ws_bytes, _stream_ptr(g.device)))
     return out
+
+
+EPI_RELU_SQ, EPI_RELU_SQ_BWD, EPI_ROUND = 1, 8, 16
+
+
+def linear_takes(x, weights):
+    """True where linear_group may stand in for x @ W^T on the GPU: 16-bit token matrices and weights of one type outside autocast and
+    every kind of transform, sizes that the kernel of the large tiles takes (include/vrwkv_hip.h, csrc/linear_wide.hip) and that fill
+    the chip with them: 70 tiles of 128 x 128."""
+    M, K = x.numel() // max(x.shape[-1], 1), x.shape[-1]
+    if not (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and M > 0 and not torch.is_autocast_enabled("cuda") and not _transformed()):
+        return False
+    for w in weights:
+        N, k = w.shape
+        if not (w.dtype == x.dtype and w.device == x.device and w.is_contiguous() and w.data_ptr() % 16 == 0
+                and (N % 192 == k % 192 == 0 or N % 128 == k % 128 == 0)):
+            return False
+        if M * N < 70 * 128 * 128 or (M + 256) * max(N, k) >= 1 << 29 or (N + 256) * (k + 256) >= 1 << 29:
+            return False
+    return True
+
+
+def linear_group(problems):
+    """vrwkv_linear_group: one launch of out = epilogue(a w^T) for 1 to 5 dicts of a (M, K), w (N, K) and, optional, gate, res (M, N), vec (N),
+    epi, raw (True: the product itself is returned as well).  Returns the results (out, or (out, raw)) in order; no autograd."""
+    M, dt, dev = problems[0]["a"].shape[0], problems[0]["a"].dtype, problems[0]["a"].device
+    n = len(problems)
+    structs, results, keep = (_lib.Linear * n)(), [], []
+    for s, p in zip(structs, problems):
+        a, w = p["a"], p["w"]
+        a = a if a.stride(1) == 1 and a.stride(0) % 8 == 0 and a.stride(0) >= a.shape[1] and a.data_ptr() % 16 == 0 else a.clone(memory_format=torch.contiguous_format)
+        keep.append(a)
+        out = torch.empty((M, w.shape[0]), dtype=dt, device=dev)
+        raw = torch.empty_like(out) if p.get("raw") else None
+        s.a, s.w, s.out, s.N, s.K, s.lda, s.epi = a.data_ptr(), w.data_ptr(), out.data_ptr(), w.shape[0], w.shape[1], a.stride(0), p.get("epi", 0)
+        for name in ("gate", "vec", "res"):
+            if p.get(name) is not None:
+                setattr(s, name, p[name].data_ptr())
+        if raw is not None:
+            s.raw = raw.data_ptr()
+        results.append(out if raw is None else (out, raw))
+    with _on(dev):
+        _lib.check(_lib.lib().vrwkv_linear_group(structs, n, M, _DT[dt], _stream_ptr(dev)))
+    return results
+
+
+def transposed(weights):
+    """The transposes of 1 to 5 contiguous 16-bit matrices, one launch (vrwkv_transpose_group)."""
+    n, dev = len(weights), weights[0].device
+    outs = [torch.empty(w.shape[1], w.shape[0], dtype=w.dtype, device=dev) for w in weights]
+    P, I = ctypes.c_void_p * n, ctypes.c_int * n
+    with _on(dev):
+        _lib.check(_lib.lib().vrwkv_transpose_group(P(*[w.data_ptr() for w in weights]), P(*[o.data_ptr() for o in outs]),
+                                                    I(*[w.shape[0] for w in weights]), I(*[w.shape[1] for w in weights]), n, _stream_ptr(dev)))
+    return outs
+
+
+def sigmoid_gate_backward(y, r, g):
+    """Gradients of sigmoid(r) * y for y and r (vrwkv_rowfuse_bwd); all contiguous token matrices of one type."""
+    gy, gr = torch.empty_like(y), torch.empty_like(r)
+    with _on(y.device):
+        _lib.check(_lib.lib().vrwkv_rowfuse_bwd_like(y.data_ptr(), r.data_ptr(), None, None, None, g.data_ptr(), gy.data_ptr(), gr.data_ptr(), None,
+                                                     y.numel() // y.shape[-1], y.shape[-1], PRE_NONE, POST_SIGMOID_GATE, 0.0, _DT[y.dtype],
+                                                     None, 0, _stream_ptr(y.device)))
+    return gy, gr
