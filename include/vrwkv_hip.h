@@ -294,6 +294,12 @@ size_t vrwkv_wgrad_workspace_bytes(int n, int M, int O, int I);
 int vrwkv_wgrad(const void* g, const void* x, void* out, int n, int M, int O, int I, int ldg, int ldx, long long stride_g,
                 long long stride_x, int dtype, void* workspace, size_t workspace_bytes, void* hip_stream);
 
+/* The gradients of 1 to 5 weights over the same M tokens in one launch of 256 x 256 tiles: out[i] (O[i], I[i]) = g[i]^T x[i], rows of g[i]
+ * (M, O[i]) and x[i] (M, I[i]) at pitches ldg[i], ldx[i]; as above otherwise.  M pitch < 2^30. */
+size_t vrwkv_wgrad_group_workspace_bytes(const int* O, const int* I, int n, int M);
+int vrwkv_wgrad_group(const void* const* g, const void* const* x, void* const* out, const int* O, const int* I, const int* ldg, const int* ldx,
+                      int n, int M, int dtype, void* workspace, size_t workspace_bytes, void* hip_stream);
+
 /* ---- the same backwards with the gradients of the parameters (gparam; gmix; gparam; gw and gu) in io_dtype, rounded once from
  * the fp32 sums: what autograd asks of a 16-bit model's parameters ---- */
 int vrwkv_rowfuse_bwd_like(const void* a, const void* other, const void* ln_weight, const void* ln_bias, const void* gamma, const void* gout, void* ga, void* gother, void* gparam, long long rows, int N, int pre, int post, float eps, int io_dtype, void* workspace, size_t workspace_bytes, void* hip_stream);

@@ -143,6 +143,11 @@ def _declare(lib):
     lib.vrwkv_wgrad_workspace_bytes.restype = sz
     lib.vrwkv_wgrad.argtypes = [vp, vp, vp, i, i, i, i, i, i, ll, ll, i, vp, sz, vp]
     lib.vrwkv_wgrad.restype = i
+    pi, pv = c.POINTER(i), c.POINTER(vp)
+    lib.vrwkv_wgrad_group_workspace_bytes.argtypes = [pi, pi, i, i]
+    lib.vrwkv_wgrad_group_workspace_bytes.restype = sz
+    lib.vrwkv_wgrad_group.argtypes = [pv, pv, pv, pi, pi, pi, pi, i, i, i, vp, sz, vp]
+    lib.vrwkv_wgrad_group.restype = i
     for name in ("rowfuse_bwd", "qshift_mix_bwd", "groupnorm_gate_bwd", "biwkv_bwd"):
         like = getattr(lib, f"vrwkv_{name}_like")
         like.argtypes, like.restype = getattr(lib, f"vrwkv_{name}").argtypes, i

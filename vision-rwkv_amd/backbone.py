@@ -16,7 +16,7 @@ import torch.nn.functional as F
 from torch.nn.modules import module as _hooks
 
 from . import ops
-from .ops import (RUN_CUDA, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, weight_grad, linear_takes, linear_group, transposed, sigmoid_gate_backward, EPI_RELU_SQ, EPI_RELU_SQ_BWD, EPI_ROUND, block_takes, block_weights_fit, block_forward, _equal_quarters, _transformed, batched_cotangent, PRE_NONE, PRE_RELU_SQ, POST_NONE,
+from .ops import (RUN_CUDA, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, weight_grad, weight_grad_group, linear_takes, linear_group, transposed, sigmoid_gate_backward, EPI_RELU_SQ, EPI_RELU_SQ_BWD, EPI_ROUND, block_takes, block_weights_fit, block_forward, _equal_quarters, _transformed, batched_cotangent, PRE_NONE, PRE_RELU_SQ, POST_NONE,
                   POST_SIGMOID_GATE, POST_RESIDUAL)
 
 
@@ -92,7 +92,7 @@ OWN_WEIGHT_GRAD = ((650_000, 100_000_000_000), (1 << 20, 10_000_000_000))       
 
 
 def _token_product(a, b, splits):
-    """a^T b over the rows (tokens) of a (M, O), b (M, I) or of stacks of them: the own kernel (fp32 sums, rounded once), or
+    """a^T b over the rows (tokens) of a (M, O), b (M, I) or of stacks of them: an own kernel (fp32 sums, rounded once), or
     `splits` batched partial products of the library.  A gradient that is itself to be differentiated, batched or traced takes tensor
     ops."""
     (M, O), I = a.shape[-2:], b.shape[-1]
@@ -122,7 +122,8 @@ class _SplitKLinear(torch.autograd.Function):
         gx = g @ weight if ctx.needs_input_grad[0] else None
         gw = None
         if ctx.needs_input_grad[1]:
-            gw = _token_product(g.reshape(-1, g.shape[-1]), x.reshape(-1, x.shape[-1]), S)
+            gw = (_weight_products([g], [x])[0] if weight.numel() >= 1 << 21
+                  else _token_product(g.reshape(-1, g.shape[-1]), x.reshape(-1, x.shape[-1]), S))
         return gx, gw, None
 
 
@@ -212,9 +213,18 @@ def _plain_backward(*tensors):
     return not torch.is_grad_enabled() and not batched_cotangent(*tensors) and not _transformed()
 
 
-def _weight_product(g, x):
-    """The gradient g^T x of a projection's weight (see _SplitKLinear)."""
-    return _token_product(_rows(g), _rows(x), 4 if g.shape[-1] * x.shape[-1] >= 1 << 21 else 8)
+def _weight_products(gs, xs):
+    """The gradients g^T x of several projections' weights (see _SplitKLinear), in one launch where kernels may be launched (12544 tokens,
+    own kernel one by one / the library / together: three of 768 x 768 110 / 127 / 60 us, 3072 x 768, 768 x 3072 and 768 x 768 263 / 200 / 137);
+    of single ones the large (3072 x 768 93 / 83 / 67, 4096 x 1024 156 / 115 / 102, but 768 x 768 34 / 43 / 36)."""
+    gs, xs = [_rows(g) for g in gs], [_rows(x) for x in xs]
+    M = gs[0].shape[0] if gs else 0
+    if (gs and (len(gs) > 1 or gs[0].shape[1] * xs[0].shape[1] >= 1 << 21) and M > 0 and gs[0].dtype in (torch.bfloat16, torch.float16) and _plain_backward(*gs)
+            and all(t.is_cuda and t.dtype == gs[0].dtype and t.shape[0] == M and t.shape[1] % 8 == 0 and t.shape[1] <= 65536 for t in (*gs, *xs))
+            and all((M + 256) * max(t.stride(0), t.shape[1]) < 1 << 30 for t in (*gs, *xs))
+            and all(g.shape[1] * x.shape[1] <= 1 << 28 for g, x in zip(gs, xs))):
+        return weight_grad_group(gs, xs)
+    return [_token_product(g, x, 4 if g.shape[1] * x.shape[1] >= 1 << 21 else 8) for g, x in zip(gs, xs)]
 
 
 class _Projections(torch.autograd.Function):
@@ -240,9 +250,9 @@ class _Projections(torch.autograd.Function):
         else:
             for i in need:
                 gx[i] = gs[i] @ ws[i]
-        for i in range(n):
-            if ctx.needs_input_grad[n + i]:
-                gw[i] = _weight_product(gs[i], xs[i])
+        need = [i for i in range(n) if ctx.needs_input_grad[n + i]]
+        for i, w in zip(need, _weight_products([gs[i] for i in need], [xs[i] for i in need])):
+            gw[i] = w
         return (*gx, *gw)
 
 
@@ -280,8 +290,10 @@ class _ChannelMix(torch.autograd.Function):
             gk = (gy @ wv) * (2 * torch.relu(k))
             gxk, gxr = (gk @ wk).reshape(g.shape), (gr @ wr).reshape(g.shape)
         need = ctx.needs_input_grad
-        return (gxk if need[0] else None, gxr if need[1] else None, _weight_product(gk, xk) if need[2] else None,
-                _weight_product(gr, xr) if need[3] else None, _weight_product(gy, kk) if need[4] else None)
+        of = [(gk, xk), (gr, xr), (gy, kk)]
+        which = [i for i in range(3) if need[2 + i]]
+        gw = dict(zip(which, _weight_products([of[i][0] for i in which], [of[i][1] for i in which])))
+        return (gxk if need[0] else None, gxr if need[1] else None, gw.get(0), gw.get(1), gw.get(2))
 
 
 # Where the grouped launches take the place of the library's products.  Two or more projections of one shape on M tokens in one launch

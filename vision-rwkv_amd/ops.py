@@ -836,6 +836,24 @@ def weight_grad(g, x):
     return out
 
 
+def weight_grad_group(gs, xs):
+    """[g^T x for g, x in zip(gs, xs)] over the rows of 1 to 5 pairs of token matrices g (M, O), x (M, I) of one 16-bit type, O and I
+    multiples of 8: the gradients of several weights (O, I) in one launch (vrwkv_wgrad_group), fp32 sums rounded once."""
+    gs, xs = [_token_rows(g[None])[0] for g in gs], [_token_rows(x[None])[0] for x in xs]
+    n, M, dev = len(gs), gs[0].shape[0], gs[0].device
+    outs = [torch.empty(g.shape[1], x.shape[1], dtype=g.dtype, device=dev) for g, x in zip(gs, xs)]
+    P, I = ctypes.c_void_p * n, ctypes.c_int * n
+    o, i = I(*[g.shape[1] for g in gs]), I(*[x.shape[1] for x in xs])
+    L = _lib.lib()
+    ws_bytes = L.vrwkv_wgrad_group_workspace_bytes(o, i, n, M)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    with _on(dev):
+        _lib.check(L.vrwkv_wgrad_group(P(*[t.data_ptr() for t in gs]), P(*[t.data_ptr() for t in xs]), P(*[t.data_ptr() for t in outs]), o, i,
+                                       I(*[t.stride(0) for t in gs]), I(*[t.stride(0) for t in xs]), n, M, _DT[gs[0].dtype],
+                                       ws.data_ptr(), ws_bytes, _stream_ptr(dev)))
+    return outs
+
+
 EPI_RELU_SQ, EPI_RELU_SQ_BWD, EPI_ROUND = 1, 8, 16
 
 
