@@ -300,6 +300,12 @@ size_t vrwkv_wgrad_group_workspace_bytes(const int* O, const int* I, int n, int 
 int vrwkv_wgrad_group(const void* const* g, const void* const* x, void* const* out, const int* O, const int* I, const int* ldg, const int* ldx,
                       int n, int M, int dtype, void* workspace, size_t workspace_bytes, void* hip_stream);
 
+/* ---- the Bi-WKV operator with w and u as a model holds them: of wu_dtype (aligned to their elements), times `factor` in that type, rounded
+ * to it (1: as they are; 1 / T: the block's division, vrwkv.py:183).  Backward: gw, gu of wu_dtype, rounded from the fp32 sums, then times
+ * `factor` and rounded again. ---- */
+int vrwkv_biwkv_fwd_as(const void* w, const void* u, int wu_dtype, float factor, const void* k, const void* v, void* y, int B, int T, int C, int io_dtype, void* workspace, size_t workspace_bytes, void* hip_stream);
+int vrwkv_biwkv_bwd_as(const void* w, const void* u, int wu_dtype, float factor, const void* k, const void* v, const void* gy, void* gw, void* gu, void* gk, void* gv, int B, int T, int C, int io_dtype, void* workspace, size_t workspace_bytes, void* hip_stream);
+
 /* ---- the same backwards with the gradients of the parameters (gparam; gmix; gparam; gw and gu) in io_dtype, rounded once from
  * the fp32 sums: what autograd asks of a 16-bit model's parameters ---- */
 int vrwkv_rowfuse_bwd_like(const void* a, const void* other, const void* ln_weight, const void* ln_bias, const void* gamma, const void* gout, void* ga, void* gother, void* gparam, long long rows, int N, int pre, int post, float eps, int io_dtype, void* workspace, size_t workspace_bytes, void* hip_stream);

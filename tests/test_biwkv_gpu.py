@@ -285,3 +285,43 @@ def test_error_behaviour(ops):
         ops.bi_wkv_forward(w.cpu(), w, k, k)
     with pytest.raises(RuntimeError):
         ops.bi_wkv_forward(w[:32].contiguous(), w, k, k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,T,C,offset", [(2, 196, 192, 0), (1, 49, 65, 1), (3, 577, 64, 0), (2, 700, 130, 3), (2, 1500, 768, 0), (1, 5, 33, 2)])
+def test_parameters_read_as_they_are_held(B, T, C, offset, dtype):
+    """w and u in the model's type, divided inside the kernels: bit for bit what the casts and divisions by tensor ops in front of
+    the kernels give, results and gradients, on every kernel (one and several super-chunks, the one-launch kernel of 16-bit
+    rows, rows that cannot be staged, sequences redone outside the plain sums), and w and u that lie at any element."""
+    from vision_rwkv_amd import ops
+    torch.manual_seed(T + C)
+    hold = torch.randn(2, C + 8, device="cuda")
+    hold[0, offset + C // 2:offset + C // 2 + 2] = 60.0 * T                 # two channels outside the plain-sum regime
+    w, u = (h[offset:offset + C] for h in hold.to(dtype))
+    assert offset == 0 or w.data_ptr() % 16 != 0
+    k, v, g = (torch.randn(B, T, C, device="cuda").to(dtype) for _ in range(3))
+
+    def run(fn):
+        ts = [t.detach().requires_grad_() for t in (w, u, k, v)]
+        assert ts[0].data_ptr() == w.data_ptr()
+        y = fn(*ts)
+        return [y.detach()] + list(torch.autograd.grad(y, ts, g))
+
+    class CastFirst(torch.autograd.Function):                               # the operator on fp32 vectors
+        @staticmethod
+        def forward(ctx, w, u, k, v):
+            w, u = w.float().contiguous(), u.float().contiguous()
+            ctx.save_for_backward(w, u, k, v)
+            return ops.bi_wkv_forward(w, u, k, v)
+
+        @staticmethod
+        def backward(ctx, gy):
+            return tuple(ops.bi_wkv_backward(*ctx.saved_tensors, gy, like_inputs=True))
+
+    cast = CastFirst.apply
+    for a, b in zip(run(ops.RUN_CUDA), run(cast)):
+        assert torch.equal(a, b)
+    assert ops.divided_takes(w, u, k, v)
+    for a, b in zip(run(lambda w, u, k, v: ops.wkv_divided(w, u, T, k, v)), run(lambda w, u, k, v: cast(w / T, u / T, k, v))):
+        assert torch.equal(a, b)

@@ -143,6 +143,10 @@ def _declare(lib):
     lib.vrwkv_wgrad_workspace_bytes.restype = sz
     lib.vrwkv_wgrad.argtypes = [vp, vp, vp, i, i, i, i, i, i, ll, ll, i, vp, sz, vp]
     lib.vrwkv_wgrad.restype = i
+    lib.vrwkv_biwkv_fwd_as.argtypes = [vp, vp, i, c.c_float, vp, vp, vp, i, i, i, i, vp, sz, vp]
+    lib.vrwkv_biwkv_fwd_as.restype = i
+    lib.vrwkv_biwkv_bwd_as.argtypes = [vp, vp, i, c.c_float, vp, vp, vp, vp, vp, vp, vp, i, i, i, i, vp, sz, vp]
+    lib.vrwkv_biwkv_bwd_as.restype = i
     pi, pv = c.POINTER(i), c.POINTER(vp)
     lib.vrwkv_wgrad_group_workspace_bytes.argtypes = [pi, pi, i, i]
     lib.vrwkv_wgrad_group_workspace_bytes.restype = sz

@@ -16,7 +16,7 @@ import torch.nn.functional as F
 from torch.nn.modules import module as _hooks
 
 from . import ops
-from .ops import (RUN_CUDA, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, weight_grad, weight_grad_group, linear_takes, linear_group, transposed, sigmoid_gate_backward, EPI_RELU_SQ, EPI_RELU_SQ_BWD, EPI_ROUND, block_takes, block_weights_fit, block_forward, _equal_quarters, _transformed, batched_cotangent, PRE_NONE, PRE_RELU_SQ, POST_NONE,
+from .ops import (RUN_CUDA, divided_takes, wkv_divided, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, weight_grad, weight_grad_group, linear_takes, linear_group, transposed, sigmoid_gate_backward, EPI_RELU_SQ, EPI_RELU_SQ_BWD, EPI_ROUND, block_takes, block_weights_fit, block_forward, _equal_quarters, _transformed, batched_cotangent, PRE_NONE, PRE_RELU_SQ, POST_NONE,
                   POST_SIGMOID_GATE, POST_RESIDUAL)
 
 
@@ -498,7 +498,8 @@ class VRWKV_SpatialMix(nn.Module):
         k, v, r = _projs((self.key, self.value, self.receptance), (xk, xv, xr))
         wd = self.spatial_decay.dtype
         if torch.is_grad_enabled() or k.dtype != (wd if wd in (torch.half, torch.bfloat16) else torch.float32):
-            y = RUN_CUDA(self.spatial_decay / T, self.spatial_first / T, k, v)  # vrwkv.py:183
+            w, u = self.spatial_decay, self.spatial_first
+            y = wkv_divided(w, u, T, k, v) if divided_takes(w, u, k, v) else RUN_CUDA(w / T, u / T, k, v)      # vrwkv.py:183
         else:
             # what WKV.forward does with these arguments, the scaled fp32 copies of w and u kept between calls
             w, u = eval_cached(self, "wu", (self.spatial_decay, self.spatial_first), T,

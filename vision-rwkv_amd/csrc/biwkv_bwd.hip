@@ -28,7 +28,7 @@ using namespace biwkv_bwd_detail;
 
 template <typename IO>
 __global__ __launch_bounds__(64)
-void biwkv_bwd_serial_kernel(const float* __restrict__ w_, const float* __restrict__ u_,
+void biwkv_bwd_serial_kernel(const ParamVec w_, const ParamVec u_,
                              const IO* __restrict__ k_, const IO* __restrict__ v_, const IO* __restrict__ gy_,
                              IO* __restrict__ gk_, IO* __restrict__ gv_, float* __restrict__ ws,
                              float* __restrict__ gw_part, float* __restrict__ gu_part, int B, int T, int C)
@@ -85,7 +85,7 @@ BwdPlan make_bwd_plan(int B, int T, int C) {
 }
 
 template <typename IO, int L>
-void launch_tiled(const BwdPlan& p, const float* w, const float* u, const IO* k, const IO* v, const IO* gy, IO* gk, IO* gv,
+void launch_tiled(const BwdPlan& p, const ParamVec& w, const ParamVec& u, const IO* k, const IO* v, const IO* gy, IO* gk, IO* gv,
                   float* ws, float* agg1, float* agg2, float* gw_part, float* gu_part, int B, int T, int C, hipStream_t st) {
     BwdGeom geo;
     geo.n_ctile = (C + WAVE - 1) / WAVE;
@@ -117,7 +117,7 @@ void launch_tiled(const BwdPlan& p, const float* w, const float* u, const IO* k,
 }
 
 template <typename IO>
-int launch(const float* w, const float* u, const void* k, const void* v, const void* gy, SumOut gw, SumOut gu,
+int launch(const ParamVec& w, const ParamVec& u, const void* k, const void* v, const void* gy, SumOut gw, SumOut gu,
            void* gk, void* gv, float* ws, int B, int T, int C, hipStream_t st) {
     const BwdPlan p = make_bwd_plan(B, T, C);
     float* agg1 = ws + p.planes;
@@ -139,7 +139,7 @@ int launch(const float* w, const float* u, const void* k, const void* v, const v
             hipLaunchKernelGGL((biwkv_bwd_serial_kernel<IO>), dim3((C + 63) / 64, B), dim3(64), 0, st, w, u,
                                kk, vv, gg, ok, ov, ws, gw_part, gu_part, B, T, C);
     }
-    launch_batch_sum(gw_part, gw, gu_part, gu, B * p.nSC, C, st);
+    launch_batch_sum(gw_part, gw, gu_part, gu, B * p.nSC, C, st, w.factor);
     return check_launch("biwkv_bwd");
 }
 
@@ -153,7 +153,7 @@ extern "C" size_t vrwkv_biwkv_bwd_workspace_bytes(int B, int T, int C, int io_dt
     return make_bwd_plan(B, T, C).total * sizeof(float);
 }
 
-static int biwkv_bwd(const float* w, const float* u, const void* k, const void* v, const void* gy,
+static int biwkv_bwd(const ParamVec& w, const ParamVec& u, const void* k, const void* v, const void* gy,
                                SumOut gw, SumOut gu, void* gk, void* gv, int B, int T, int C, int io_dtype,
                                void* workspace, size_t workspace_bytes, void* hip_stream)
 {
@@ -170,7 +170,7 @@ static int biwkv_bwd(const float* w, const float* u, const void* k, const void* 
     }
     const size_t esz = io_dtype == VRWKV_F32 ? 4 : 2;
     if ((((uintptr_t)k | (uintptr_t)v | (uintptr_t)gy | (uintptr_t)gk | (uintptr_t)gv) & (esz - 1)) ||
-        (((uintptr_t)w | (uintptr_t)u | (uintptr_t)workspace) & 3) ||
+        !w.aligned() || !u.aligned() || ((uintptr_t)workspace & 3) ||
         (((uintptr_t)gw.p | (uintptr_t)gu.p) & (gw.dtype == VRWKV_F32 ? 3 : 1))) {
         set_error("biwkv_bwd: pointers must be aligned to their element size");
         return VRWKV_INVALID_ARG;
@@ -197,3 +197,13 @@ extern "C" int vrwkv_biwkv_bwd_like(const float* w, const float* u, const void* 
     return biwkv_bwd(w, u, k, v, gy, SumOut(gw, io_dtype), SumOut(gu, io_dtype), gk, gv, B, T, C, io_dtype, workspace, workspace_bytes, hip_stream);
 }
 
+extern "C" int vrwkv_biwkv_bwd_as(const void* w, const void* u, int wu_dtype, float factor, const void* k, const void* v, const void* gy,
+                                  void* gw, void* gu, void* gk, void* gv, int B, int T, int C, int io_dtype,
+                                  void* workspace, size_t workspace_bytes, void* hip_stream) {
+    if (wu_dtype != VRWKV_F32 && wu_dtype != VRWKV_BF16 && wu_dtype != VRWKV_F16) {
+        set_error("biwkv_bwd_as: unknown dtype %d of w and u", wu_dtype);
+        return VRWKV_UNSUPPORTED_DTYPE;
+    }
+    return biwkv_bwd(ParamVec(w, wu_dtype, factor), ParamVec(u, wu_dtype, factor), k, v, gy, SumOut(gw, wu_dtype), SumOut(gu, wu_dtype), gk, gv, B, T, C,
+                     io_dtype, workspace, workspace_bytes, hip_stream);
+}

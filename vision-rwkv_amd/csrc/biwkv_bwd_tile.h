@@ -86,7 +86,7 @@ struct BwdGeom {
 // LDS in 16-byte pieces (buffer_load ... lds) while this tile is computed; gy stays a register load.
 template <typename IO, int L, int MODE, bool STAGED = false>
 __global__ __launch_bounds__(BWD_SMAX * WAVE)
-void biwkv_bwd_tile_kernel(const float* __restrict__ w_, const float* __restrict__ u_,
+void biwkv_bwd_tile_kernel(const ParamVec w_, const ParamVec u_,
                            const IO* __restrict__ k_, const IO* __restrict__ v_, const IO* __restrict__ gy_,
                            IO* __restrict__ gk_, IO* __restrict__ gv_,
                            float* __restrict__ ws, float* __restrict__ agg1, float* __restrict__ agg2,

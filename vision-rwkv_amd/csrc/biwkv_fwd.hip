@@ -6,9 +6,9 @@
 
 namespace vrwkv {
 namespace biwkv_fwd_detail {
-extern template int biwkv_fwd_launch_io<float>(const Plan&, const float*, const float*, const void*, const void*, const void*, void*, float*, int, int, int, hipStream_t);
-extern template int biwkv_fwd_launch_io<__hip_bfloat16>(const Plan&, const float*, const float*, const void*, const void*, const void*, void*, float*, int, int, int, hipStream_t);
-extern template int biwkv_fwd_launch_io<__half>(const Plan&, const float*, const float*, const void*, const void*, const void*, void*, float*, int, int, int, hipStream_t);
+extern template int biwkv_fwd_launch_io<float>(const Plan&, const ParamVec&, const ParamVec&, const void*, const void*, const void*, void*, float*, int, int, int, hipStream_t);
+extern template int biwkv_fwd_launch_io<__hip_bfloat16>(const Plan&, const ParamVec&, const ParamVec&, const void*, const void*, const void*, void*, float*, int, int, int, hipStream_t);
+extern template int biwkv_fwd_launch_io<__half>(const Plan&, const ParamVec&, const ParamVec&, const void*, const void*, const void*, void*, float*, int, int, int, hipStream_t);
 }
 namespace {
 using namespace biwkv_fwd_detail;
@@ -131,7 +131,7 @@ int launch_gate_in_place(const void* r, void* y, size_t n, hipStream_t st) {
 }
 
 // the forward, with the gate when r is given
-int biwkv_fwd_common(const char* who, const float* w, const float* u, const void* k, const void* v, const void* r, void* y,
+int biwkv_fwd_common(const char* who, const ParamVec& w, const ParamVec& u, const void* k, const void* v, const void* r, void* y,
                      int B, int T, int C, int io_dtype, void* workspace, size_t workspace_bytes, void* hip_stream) {
     int rc = validate(B, T, C, io_dtype);
     if (rc != VRWKV_OK) return rc;
@@ -140,7 +140,7 @@ int biwkv_fwd_common(const char* who, const float* w, const float* u, const void
         return VRWKV_INVALID_ARG;
     }
     const size_t esz = io_dtype == VRWKV_F32 ? 4 : 2;
-    if ((((uintptr_t)k | (uintptr_t)v | (uintptr_t)y | (uintptr_t)r) & (esz - 1)) || (((uintptr_t)w | (uintptr_t)u) & 3)) {
+    if ((((uintptr_t)k | (uintptr_t)v | (uintptr_t)y | (uintptr_t)r) & (esz - 1)) || !w.aligned() || !u.aligned()) {
         set_error("%s: pointers must be aligned to their element size", who);
         return VRWKV_INVALID_ARG;
     }
@@ -196,6 +196,16 @@ extern "C" int vrwkv_biwkv_fwd_gate(const float* w, const float* u, const void* 
         return VRWKV_INVALID_ARG;
     }
     return biwkv_fwd_common("biwkv_fwd_gate", w, u, k, v, r, y, B, T, C, io_dtype, workspace, workspace_bytes, hip_stream);
+}
+
+extern "C" int vrwkv_biwkv_fwd_as(const void* w, const void* u, int wu_dtype, float factor, const void* k, const void* v, void* y,
+                                  int B, int T, int C, int io_dtype, void* workspace, size_t workspace_bytes, void* hip_stream) {
+    if (wu_dtype != VRWKV_F32 && wu_dtype != VRWKV_BF16 && wu_dtype != VRWKV_F16) {
+        set_error("biwkv_fwd_as: unknown dtype %d of w and u", wu_dtype);
+        return VRWKV_UNSUPPORTED_DTYPE;
+    }
+    return biwkv_fwd_common("biwkv_fwd_as", ParamVec(w, wu_dtype, factor), ParamVec(u, wu_dtype, factor), k, v, nullptr, y, B, T, C, io_dtype,
+                            workspace, workspace_bytes, hip_stream);
 }
 
 extern "C" size_t vrwkv_biwkv_fwd_static_max_workspace_bytes(void) { return kStaticWorkspaceBytes; }

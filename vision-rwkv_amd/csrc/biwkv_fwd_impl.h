@@ -150,8 +150,7 @@ struct BiwkvTile {
     static constexpr int STAGE_ELEMS = 2 * LR * WAVE;                     // per wave: k rows, v rows
     static constexpr int YSTAGE_ELEMS = OUT_STAGED ? LR * WAVE : 8;       // per wave: y rows
 
-    const float* __restrict__ w_;
-    const float* __restrict__ u_;
+    ParamVec w_, u_;
     const IO* __restrict__ k_;
     const IO* __restrict__ v_;
     const IO* __restrict__ r_;  // GATE: receptance (B,T,C)
@@ -192,7 +191,7 @@ struct BiwkvTile {
     // sequence: wave 0 those of the earlier super-chunks (farthest first), wave 1 those of the later ones (farthest
     // first), up to NBF each -- a whole tile ahead, so that folding them (fold_others) waits for no memory round trip.
     static constexpr int NBF = MODE == 2 ? 16 : 1;
-    struct WU { float w[VEC], u[VEC]; float fr[NBF], f0[NBF], f1[NBF]; };
+    struct WU { unsigned w[VEC], u[VEC]; float fr[NBF], f0[NBF], f1[NBF]; };
 
     // super-chunk whose entry is the i-th one folded by `wave` (0: earlier ones ascending, 1: later ones descending)
     __device__ __forceinline__ int fold_source(int i) const { return wave == 0 ? i : g.nSC - 1 - i; }
@@ -207,8 +206,8 @@ struct BiwkvTile {
         const Where q = locate(tile);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-            wu.w[e] = q.cok ? w_[q.c0 + e] : 0.f;
-            wu.u[e] = q.cok ? u_[q.c0 + e] : 0.f;
+            wu.w[e] = q.cok ? w_.fetch(q.c0 + e) : 0u;      // 0 is 0 in every type
+            wu.u[e] = q.cok ? u_.fetch(q.c0 + e) : 0u;
         }
         if (MODE == 2 && wave < 2) {                     // wave-uniform
 #pragma unroll
@@ -327,12 +326,12 @@ struct BiwkvTile {
     // consumed) issues the loads of `next` into Kn, Vn when next < n_tiles.
     // True when any channel of the tile is outside the plain-sum regime (wave-uniform, and the
     // same for every wave and every super-chunk of a channel tile).
-    __device__ __forceinline__ bool tile_is_robust(const WU& wu, float (&om)[VEC], float (&mu)[VEC]) const {
+    __device__ __forceinline__ bool tile_is_robust(const Where& q, const WU& wu, float (&om)[VEC], float (&mu)[VEC]) const {
         bool bad = false;
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-            om[e] = wu.w[e] * LOG2E;
-            mu[e] = wu.u[e] * LOG2E;
+            om[e] = w_.value(wu.w[e], q.c0 + e) * LOG2E;
+            mu[e] = u_.value(wu.u[e], q.c0 + e) * LOG2E;
             bad = bad || outside_plain_sum(om[e], mu[e], T);
         }
         return __builtin_amdgcn_ballot_w64(bad) != 0ull;
@@ -358,7 +357,7 @@ struct BiwkvTile {
         VRWKV_STAMP(wave, round, 0);                      // tile entered
 
         float om[VEC], mu[VEC];
-        if (tile_is_robust(wu, om, mu)) {
+        if (tile_is_robust(q, wu, om, mu)) {
             // workgroup-uniform branch; the barrier stands in for the exchange barrier of a computed tile
             if (STAGED) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); else lds_barrier();
             if (next < g.n_tiles) {
@@ -663,10 +662,10 @@ struct BiwkvTile {
         WU wu;
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-            wu.w[e] = q.cok ? w_[q.c0 + e] : 0.f;
-            wu.u[e] = q.cok ? u_[q.c0 + e] : 0.f;
+            wu.w[e] = q.cok ? w_.fetch(q.c0 + e) : 0u;      // 0 is 0 in every type
+            wu.u[e] = q.cok ? u_.fetch(q.c0 + e) : 0u;
         }
-        if (!tile_is_robust(wu, om, mu)) return;
+        if (!tile_is_robust(q, wu, om, mu)) return;
 
         const unsigned row = (unsigned)(C * sizeof(IO));
         const __amdgpu_buffer_rsrc_t ry = make_rsrc(y_ + q.slab, (unsigned)((size_t)T * C * sizeof(IO)));
@@ -793,7 +792,7 @@ struct BiwkvTile {
 
 template <typename IO, int VEC, int L, int MODE, bool STAGED = false, bool GATE = false>
 __global__ __launch_bounds__(smax_for(L, VEC) * WAVE)
-void biwkv_fwd_kernel(const float* __restrict__ w_, const float* __restrict__ u_,
+void biwkv_fwd_kernel(const ParamVec w_, const ParamVec u_,
                       const IO* __restrict__ k_, const IO* __restrict__ v_, IO* __restrict__ y_,
                       float* __restrict__ ws, int T, int C, TileGeom g, const IO* __restrict__ r_ = nullptr)
 {
@@ -917,7 +916,7 @@ constexpr int GATE_NOT_FUSED = -100;
 
 // r: null, or the receptance whose sigmoid gates y inside the emitting kernel.
 template <typename IO, int VEC, int L>
-int launch_L(const Plan& p, const float* w, const float* u, const void* k, const void* v, const void* r, void* y,
+int launch_L(const Plan& p, const ParamVec& w, const ParamVec& u, const void* k, const void* v, const void* r, void* y,
              float* ws, int B, int T, int C, hipStream_t st) {
     const dim3 block(p.S * WAVE);
     const dim3 grid(p.grid);
@@ -975,7 +974,7 @@ int launch_L(const Plan& p, const float* w, const float* u, const void* k, const
 }
 
 template <typename IO, int VEC>
-int launch_VEC(const Plan& p, const float* w, const float* u, const void* k, const void* v, const void* r, void* y,
+int launch_VEC(const Plan& p, const ParamVec& w, const ParamVec& u, const void* k, const void* v, const void* r, void* y,
                float* ws, int B, int T, int C, hipStream_t st) {
     switch (p.L) {
 #define VRWKV_CASE(LL) case LL: return launch_L<IO, VEC, LL>(p, w, u, k, v, r, y, ws, B, T, C, st); break;
@@ -987,7 +986,7 @@ int launch_VEC(const Plan& p, const float* w, const float* u, const void* k, con
 }
 
 template <typename IO>
-int biwkv_fwd_launch_io(const Plan& p, const float* w, const float* u, const void* k, const void* v, const void* r, void* y,
+int biwkv_fwd_launch_io(const Plan& p, const ParamVec& w, const ParamVec& u, const void* k, const void* v, const void* r, void* y,
                         float* ws, int B, int T, int C, hipStream_t st) {
     return launch_VEC<IO, 1>(p, w, u, k, v, r, y, ws, B, T, C, st);
 }

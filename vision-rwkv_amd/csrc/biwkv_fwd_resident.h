@@ -109,7 +109,7 @@ __device__ __forceinline__ void agg_get(const float (*__restrict__ agg)[NSLOT][W
 // One sequence outside the plain-sum regime: the renormalising recurrence of BiwkvTile::run_robust, first the
 // aggregates of every super-chunk (into the workspace), then the outputs.
 template <typename IO, int NSC, int L>
-__device__ __forceinline__ void resident_robust(const float* w_, const float* u_, const IO* k_, const IO* v_, IO* y_,
+__device__ __forceinline__ void resident_robust(const ParamVec w_, const ParamVec u_, const IO* k_, const IO* v_, IO* y_,
                                                           float* ws, int T, int C, int n_ctile, int n_seq, int b, int ctile,
                                                           float (*agg0)[NSLOT][WAVE], float (*agg1)[NSLOT][WAVE]) {
     TileGeom g;
@@ -131,7 +131,7 @@ __device__ __forceinline__ void resident_robust(const float* w_, const float* u_
 
 template <typename IO, int NSC, int L>
 __global__ __launch_bounds__(8 * WAVE)
-void biwkv_fwd_resident_kernel(const float* __restrict__ w_, const float* __restrict__ u_,
+void biwkv_fwd_resident_kernel(const ParamVec w_, const ParamVec u_,
                                const IO* __restrict__ k_, const IO* __restrict__ v_, IO* __restrict__ y_,
                                float* __restrict__ ws, int T, int C, int n_ctile, int n_seq)
 {

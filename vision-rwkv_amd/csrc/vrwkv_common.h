@@ -187,6 +187,36 @@ __device__ __forceinline__ void stamp(int wave, int slot, int point) {
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
+// A parameter vector of the Bi-WKV operator (decay, bonus) as the caller holds it: fp32, bf16 or fp16, times a factor in the same type
+// (the block's division by T, which tensor ops carry out as a multiplication by the reciprocal).  Read where it is used, so that no
+// call begins with casts and divisions of 768 numbers (a launch of 2 to 3 us each, four of them a layer in training).
+// The word that holds an element is fetched as it lies and picked apart at its use: the fetch can be ahead, and has no branch.
+struct ParamVec {
+    const void* p;
+    int dtype;
+    float factor;                                         // 1: as it is
+    ParamVec() = default;
+    ParamVec(const float* q) : p(q), dtype(VRWKV_F32), factor(1.f) {}
+    ParamVec(const void* q, int dt, float f) : p(q), dtype(dt), factor(f) {}
+    explicit operator bool() const { return p != nullptr; }
+    bool aligned() const { return ((size_t)p & (dtype == VRWKV_F32 ? 3 : 1)) == 0; }
+    __device__ __forceinline__ size_t address(int c) const { return (size_t)p + ((size_t)c << (dtype == VRWKV_F32 ? 2 : 1)); }
+    __device__ __forceinline__ unsigned fetch(int c) const { return *reinterpret_cast<const unsigned*>(address(c) & ~(size_t)3); }
+    __device__ __forceinline__ float value(unsigned word, int c) const {
+        const unsigned short half = (unsigned short)(address(c) & 2 ? word >> 16 : word);
+        float x = __builtin_bit_cast(float, word);
+        if (dtype == VRWKV_BF16) x = __builtin_bit_cast(float, (unsigned)half << 16);
+        else if (dtype == VRWKV_F16) x = (float)__builtin_bit_cast(_Float16, half);
+        if (factor != 1.f) {
+            x *= factor;
+            if (dtype == VRWKV_BF16) x = to_f32(from_f32<__hip_bfloat16>(x));
+            else if (dtype == VRWKV_F16) x = to_f32(from_f32<__half>(x));
+        }
+        return x;
+    }
+    __device__ __forceinline__ float operator[](int c) const { return value(fetch(c), c); }
+};
+
 // out[c] = sum_b part[b*C + c] for up to two (part, out) pairs (the second may be null).  1024 threads = 32 columns
 // (one 128-byte piece of a row per half wave) x 32 slices of the batch, sixteen loads of a slice in flight at a time
 // (512 partial rows in one round of loads); the slices are added in a fixed order (deterministic).
@@ -196,7 +226,7 @@ constexpr int BATCH_SUM_THREADS = 1024, BATCH_SUM_COLS = 32, BATCH_SUM_SLICES = 
 template <typename O>
 __global__ __launch_bounds__(1024) inline void batch_sum_kernel(const float* __restrict__ part0, O* __restrict__ out0,
                                                                 const float* __restrict__ part1, O* __restrict__ out1,
-                                                                int B, int C) {
+                                                                int B, int C, float factor = 1.f) {
     constexpr int NS = BATCH_SUM_SLICES, U = 16;
     __shared__ float red[2][NS][BATCH_SUM_COLS];
     const int cl = threadIdx.x % BATCH_SUM_COLS, slice = threadIdx.x / BATCH_SUM_COLS;
@@ -228,6 +258,10 @@ __global__ __launch_bounds__(1024) inline void batch_sum_kernel(const float* __r
         for (int i = 0; i < NS; ++i) { t0 += red[0][i][cl]; t1 += red[1][i][cl]; }
         out0[c] = from_f32<O>(t0);
         if (part1) out1[c] = from_f32<O>(t1);
+        if (factor != 1.f) {                              // of the sum in its own type, like a multiplication of its own
+            out0[c] = from_f32<O>(to_f32(from_f32<O>(t0)) * factor);
+            if (part1) out1[c] = from_f32<O>(to_f32(from_f32<O>(t1)) * factor);
+        }
     }
 }
 // Where the sums go, and as what.
@@ -238,12 +272,12 @@ struct SumOut {
     SumOut(void* q, int dt) : p(q), dtype(dt) {}
     explicit operator bool() const { return p != nullptr; }
 };
-inline void launch_batch_sum(const float* part0, SumOut out0, const float* part1, SumOut out1, int B, int C, hipStream_t st) {
+inline void launch_batch_sum(const float* part0, SumOut out0, const float* part1, SumOut out1, int B, int C, hipStream_t st, float factor = 1.f) {
     const dim3 grid((C + BATCH_SUM_COLS - 1) / BATCH_SUM_COLS), block(BATCH_SUM_THREADS);
-    if (out0.dtype == VRWKV_F32) hipLaunchKernelGGL((batch_sum_kernel<float>), grid, block, 0, st, part0, (float*)out0.p, part1, (float*)out1.p, B, C);
+    if (out0.dtype == VRWKV_F32) hipLaunchKernelGGL((batch_sum_kernel<float>), grid, block, 0, st, part0, (float*)out0.p, part1, (float*)out1.p, B, C, factor);
     else if (out0.dtype == VRWKV_BF16)
-        hipLaunchKernelGGL((batch_sum_kernel<__hip_bfloat16>), grid, block, 0, st, part0, (__hip_bfloat16*)out0.p, part1, (__hip_bfloat16*)out1.p, B, C);
-    else hipLaunchKernelGGL((batch_sum_kernel<__half>), grid, block, 0, st, part0, (__half*)out0.p, part1, (__half*)out1.p, B, C);
+        hipLaunchKernelGGL((batch_sum_kernel<__hip_bfloat16>), grid, block, 0, st, part0, (__hip_bfloat16*)out0.p, part1, (__hip_bfloat16*)out1.p, B, C, factor);
+    else hipLaunchKernelGGL((batch_sum_kernel<__half>), grid, block, 0, st, part0, (__half*)out0.p, part1, (__half*)out1.p, B, C, factor);
 }
 #endif
 

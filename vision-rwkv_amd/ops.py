@@ -125,19 +125,66 @@ def bi_wkv_backward(w, u, k, v, gy, out=None, like_inputs=False):
     return [gw, gu, gk, gv]
 
 
+def _wkv_forward(w, u, k, v, factor=1.0):
+    """bi_wkv_forward with w and u of one type as they are, times factor in that type (vrwkv_biwkv_fwd_as)."""
+    for t, n in ((w, "w"), (u, "u"), (k, "k"), (v, "v")):
+        _check_input(t, n)
+    if k.dim() != 3 or v.shape != k.shape:
+        raise RuntimeError("k and v must all be (B,T,C) of one dtype")
+    B, T, C = k.shape
+    if w.numel() != C or u.numel() != C:
+        raise RuntimeError("w and u must have C elements")
+    if k.dtype not in _DT or v.dtype != k.dtype:
+        raise RuntimeError("k and v must share one of float32 / bfloat16 / float16")
+    L = _lib.lib()
+    dt = _DT[k.dtype]
+    y = torch.empty_like(k)
+    if y.numel() == 0:
+        return y
+    ws_bytes = L.vrwkv_biwkv_fwd_workspace_bytes(B, T, C, dt)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=k.device) if ws_bytes else None
+    with _on(k.device):
+        _lib.check(L.vrwkv_biwkv_fwd_as(w.data_ptr(), u.data_ptr(), _DT[w.dtype], factor, k.data_ptr(), v.data_ptr(), y.data_ptr(), B, T, C, dt,
+                                        ws.data_ptr() if ws is not None else None, ws_bytes, _stream_ptr(k.device)))
+    return y
+
+
+def _wkv_backward(w, u, k, v, gy, factor=1.0):
+    """The gradients of _wkv_forward, gw and gu of the type of w (vrwkv_biwkv_bwd_as)."""
+    gw, gu, gk, gv = torch.empty_like(w), torch.empty_like(u), torch.empty_like(k), torch.empty_like(k)
+    if gy.shape != k.shape or gy.dtype != k.dtype:
+        raise RuntimeError("gy must have the shape and dtype of k")
+    if k.numel() == 0:
+        return gw.zero_(), gu.zero_(), gk, gv
+    B, T, C = k.shape
+    L = _lib.lib()
+    dt = _DT[k.dtype]
+    ws_bytes = L.vrwkv_biwkv_bwd_workspace_bytes(B, T, C, dt)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=k.device)
+    with _on(k.device):
+        _lib.check(L.vrwkv_biwkv_bwd_as(w.data_ptr(), u.data_ptr(), _DT[w.dtype], factor, k.data_ptr(), v.data_ptr(), gy.data_ptr(), gw.data_ptr(),
+                                        gu.data_ptr(), gk.data_ptr(), gv.data_ptr(), B, T, C, dt, ws.data_ptr(), ws_bytes, _stream_ptr(k.device)))
+    return gw, gu, gk, gv
+
+
 class WKV(torch.autograd.Function):
     """Bi-WKV with the reference's dtype rule: arithmetic in fp32, the result is fp32 unless
     the *parameter* w is half / bfloat16, in which case it has w's dtype (vrwkv.py:31-44).
     When k and v already arrive in that 16-bit dtype they are consumed as they are
-    (no up-cast copies, no separate down-cast of y)."""
+    (no up-cast copies, no separate down-cast of y), and w and u as well when they share a type."""
 
     @staticmethod
     def forward(ctx, w, u, k, v):
         out_dtype = w.dtype if w.dtype in (torch.half, torch.bfloat16) else torch.float32
+        ctx.out_dtype = out_dtype
+        ctx.as_held = w.dtype == u.dtype == k.dtype == v.dtype == out_dtype
+        if ctx.as_held:
+            wc, uc = w.contiguous(), u.contiguous()
+            ctx.save_for_backward(wc, uc, k, v)
+            return _wkv_forward(wc, uc, k.contiguous(), v.contiguous())
         wf = w.float().contiguous()
         uf = u.float().contiguous()
         ctx.save_for_backward(wf, uf, k, v)                # the fp32 copies serve the backward too
-        ctx.out_dtype = out_dtype
         if k.dtype == out_dtype and v.dtype == out_dtype:
             return bi_wkv_forward(wf, uf, k.contiguous(), v.contiguous())
         y = bi_wkv_forward(wf, uf, k.float().contiguous(), v.float().contiguous())
@@ -148,6 +195,8 @@ class WKV(torch.autograd.Function):
         # vrwkv.py:47-61: gradients in fp32, returned in w's dtype when that is half / bfloat16
         wf, uf, k, v = ctx.saved_tensors
         out_dtype = ctx.out_dtype
+        if ctx.as_held:
+            return _wkv_backward(wf, uf, k.contiguous(), v.contiguous(), gy.to(out_dtype).contiguous())
         if k.dtype == out_dtype and v.dtype == out_dtype and out_dtype != torch.float32:
             return tuple(bi_wkv_backward(wf, uf, k.contiguous(), v.contiguous(), gy.to(out_dtype).contiguous(), like_inputs=True))
         gw, gu, gk, gv = bi_wkv_backward(wf, uf, k.float().contiguous(), v.float().contiguous(), gy.float().contiguous())
@@ -155,6 +204,34 @@ class WKV(torch.autograd.Function):
             return (gw, gu, gk, gv)
         gwu = torch.stack((gw, gu)).to(out_dtype)           # one cast for both parameter gradients
         return (gwu[0], gwu[1], gk.to(out_dtype), gv.to(out_dtype))
+
+
+class _WKVDivided(torch.autograd.Function):
+    """WKV of w / n and u / n (vrwkv.py:183) for parameters, k and v of one type: the divisions, and those of their gradients, inside the
+    kernels that read the vectors and write the sums.  Tensor ops divide by a number through its fp32 reciprocal; so do the kernels."""
+
+    @staticmethod
+    def forward(ctx, w, u, n, k, v):
+        ctx.factor = ctypes.c_float(1.0 / n).value
+        ctx.save_for_backward(w, u, k, v)
+        return _wkv_forward(w, u, k, v, ctx.factor)
+
+    @staticmethod
+    def backward(ctx, gy):
+        w, u, k, v = ctx.saved_tensors
+        gw, gu, gk, gv = _wkv_backward(w, u, k, v, gy.to(k.dtype).contiguous(), ctx.factor)
+        return gw, gu, None, gk, gv
+
+
+def divided_takes(w, u, k, v):
+    """True where wkv_divided computes RUN_CUDA(w / n, u / n, k, v): plain contiguous GPU tensors of one type outside every transform."""
+    return (type(w) in (torch.Tensor, torch.nn.Parameter) and type(u) is type(w) and type(k) is type(v) is torch.Tensor and w.is_cuda
+            and w.dtype == u.dtype == k.dtype == v.dtype and w.dtype in _DT and w.dim() == 1
+            and all(t.is_contiguous() and t.device == w.device for t in (w, u, k, v)) and not _transformed())
+
+
+def wkv_divided(w, u, n, k, v):
+    return _WKVDivided.apply(w, u, n, k, v)
 
 
 class _WKVLegacy(torch.autograd.Function):
