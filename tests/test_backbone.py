@@ -794,6 +794,35 @@ def test_weight_gradients_in_one_launch(M, shapes, splits, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind,C,dtype,hw,shift,batch,cls", [
+    ("v4", 192, torch.bfloat16, (14, 14), 1, 1, False), ("v4", 64, torch.float16, (1, 3), 1, 5, False), ("v4", 64, torch.bfloat16, (3, 1), 1, 2, False),
+    ("v4", 1024, torch.bfloat16, (5, 7), 2, 2, False), ("v4", 512, torch.float32, (6, 9), 1, 3, False), ("v4", 256, torch.float32, (4, 4), 3, 1, False),
+    ("v4", 96, torch.bfloat16, (7, 2), 5, 2, False), ("v6", 192, torch.bfloat16, (14, 13), 1, 1, True), ("v6", 64, torch.float16, (1, 1), 1, 7, True),
+    ("v6", 576, torch.bfloat16, (4, 9), 2, 2, False)])
+def test_norm_shift_and_mixes_in_one_launch(kind, C, dtype, hw, shift, batch, cls):
+    """Images whose rows and columns are shorter than a workgroup's four tokens or than the shift, class tokens, rows of one and two
+    pieces a lane: a block natively (one launch for norm, shift and mixes) is bit for bit the block with those as two launches,
+    which more images in the batch get (the tail of a batch that is past the size of the rule)."""
+    from vision_rwkv_amd import lib
+    net = _small_backbone(kind, C, dtype, False, False, cls, hw)
+    for l in net.layers:
+        l.att.shift_pixel = l.ffn.shift_pixel = shift
+    T = hw[0] * hw[1] + cls
+    many = 700000 // (T * C) // batch * batch + batch
+    x = torch.randn(many, T, C, device="cuda").to(dtype)
+    with torch.no_grad():
+        for b in (0, many - batch):
+            few = x[b:b + batch].contiguous()
+            assert all(l._native(few, hw) is not None for l in net.layers)
+        from vision_rwkv_amd import option
+        with option("linear_tile", 1):                       # the same products in either
+            assert net.layers[1]._native(x, hw) is not None
+            whole = net.layers[1](x, hw)
+            part = torch.cat([net.layers[1](x[b:b + batch].contiguous(), hw) for b in (0, many - batch)])
+    assert torch.equal(torch.cat((whole[:batch], whole[many - batch:])), part)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("shapes", [((8, 8),), ((72, 136), (64, 64), (8, 200)), ((768, 768), (3072, 768), (768, 3072), (192, 40), (40, 192))])
 def test_weights_transposed_in_one_launch(shapes):
     from vision_rwkv_amd.ops import transposed

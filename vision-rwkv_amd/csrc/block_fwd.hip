@@ -352,13 +352,22 @@ static int block_fwd(const vrwkv_block_args* args, const vrwkv_block6_params* pa
 
     const void* x = a->x;
     const void* src = x;                                  // input of a half
-    if (!a->post_norm) { TRY(vrwkv_rowfuse(x, nullptr, a->ln1_w, a->ln1_b, nullptr, ln, M, C, 0, 0, a->ln1_eps, dt, st)); src = ln; }
+    // a half's first steps: the pre-norm, the shift and the mixes; `keep`: the normalised rows are wanted as well
+    const int g = H ? 16 : a->quarter;
+    auto mixes = [&](const void* in, const void* w, const void* b, float eps, const float* mix, void* const* out, int n, bool keep) -> int {
+        if (a->post_norm) return vrwkv_qshift_mix(in, mix, out, n, B, T, C, a->Hp, a->Wp, a->shift_pixel, g, hd, dt, st);
+        if (ln_shift_mix_takes(B, T, C, g, hd, a->shift_pixel, dt))
+            return ln_shift_mix(in, w, b, eps, mix, out, n, keep ? ln : nullptr, B, T, C, a->Hp, a->Wp, a->shift_pixel, g, hd, dt, st);
+        TRY(vrwkv_rowfuse(in, nullptr, w, b, nullptr, ln, M, C, 0, 0, eps, dt, st));
+        return vrwkv_qshift_mix(ln, mix, out, n, B, T, C, a->Hp, a->Wp, a->shift_pixel, g, hd, dt, st);
+    };
+    if (!a->post_norm) src = ln;
     char* half = at;                                      // both halves use what follows
     void* y;
     if (!H) {
         void* m[3] = {take(L.n), take(L.n), take(L.n)};
         void *k = take(L.n), *v = take(L.n), *r = take(L.n);
-        TRY(vrwkv_qshift_mix(src, a->att_mix, m, 3, B, T, C, a->Hp, a->Wp, a->shift_pixel, a->quarter, 0, dt, st));
+        TRY(mixes(x, a->ln1_w, a->ln1_b, a->ln1_eps, a->att_mix, m, 3, false));
         G.n = 3;
         G.p[0] = linear(m[0], a->key, k, C, C);
         G.p[1] = linear(m[1], a->value, v, C, C);
@@ -380,7 +389,7 @@ static int block_fwd(const vrwkv_block_args* args, const vrwkv_block6_params* pa
         for (void*& p : m) p = take(L.n);
         float *yf = (float*)take(2 * L.n), *yn = (float*)take(2 * L.n);
         void *lo = take(al((size_t)M * 160 * es)), *dlo = take(al((size_t)M * 64 * es));
-        TRY(vrwkv_qshift_mix(src, a->att_mix, s, 2, B, T, C, a->Hp, a->Wp, a->shift_pixel, 16, hd, dt, st));
+        TRY(mixes(x, a->ln1_w, a->ln1_b, a->ln1_eps, a->att_mix, s, 2, true));
         G.n = 1;
         G.p[0] = linear(s[1], a->maa_w1, lo, 160, C, 0, EPI_TANH);
         TRY(linear_group(G, dt, st));
@@ -409,10 +418,8 @@ static int block_fwd(const vrwkv_block_args* args, const vrwkv_block6_params* pa
     }
     TRY(residual(linear(y, a->output, nullptr, C, C), x, x1, a->gamma1, a->ln1_w, a->ln1_b, a->ln1_eps, ln));
     at = half;
-    src = x1;
-    if (!a->post_norm) { TRY(vrwkv_rowfuse(x1, nullptr, a->ln2_w, a->ln2_b, nullptr, ln, M, C, 0, 0, a->ln2_eps, dt, st)); src = ln; }
     void *f[2] = {take(L.n), take(L.n)}, *fr = take(L.n), *ftmp = take(L.n);
-    TRY(vrwkv_qshift_mix(src, a->ffn_mix, f, 2, B, T, C, a->Hp, a->Wp, a->shift_pixel, H ? 16 : a->quarter, hd, dt, st));
+    TRY(mixes(x1, a->ln2_w, a->ln2_b, a->ln2_eps, a->ffn_mix, f, 2, false));
     G.n = 2;
     G.p[0] = linear(f[0], a->ffn_key, a->ffn_kn_w ? hid_raw : hid, hidden, C, 0, a->ffn_kn_w ? 0 : EPI_RELU_SQ);
     G.p[1] = linear(f[1], a->ffn_receptance, fr, C, C);

@@ -59,6 +59,12 @@ __device__ __forceinline__ void epilogue(const LinProblem& P, int m, int n, floa
 // Runs a group; picks kernel and tile by the size of the results (block_fwd.hip).  16-byte aligned pointers, N a multiple of 16, K of 32,
 // lda of 8, byte offsets below 2^30: the callers' checks.
 int linear_group(LinGroup& G, int dtype, hipStream_t st);
+// LayerNorm, Q-Shift and two or three token mixes in one launch (ln_shift_mix.hip): whether it is the faster way, and the launch.  Tensors
+// 16-byte aligned, x (B, T, C).  ln_out: optional, the normalised rows as well.
+constexpr long long LN_SHIFT_MIX_MOST = 700000;          // values of x
+bool ln_shift_mix_takes(int B, int T, int C, int g, int head_dim, int shift, int dtype);
+int ln_shift_mix(const void* x, const void* ln_w, const void* ln_b, float eps, const float* mix, void* const* out, int n_mix, void* ln_out,
+                 int B, int T, int C, int Hp, int Wp, int shift, int g, int head_dim, int dtype, hipStream_t st);
 // The wide kernel (linear_wide.hip): whether it can run a group, and the launch.
 bool wide_takes(const LinGroup& G, int dtype);
 int wide_group(LinGroup& G, int dtype, hipStream_t st);

@@ -20,32 +20,13 @@
 // A wave recomputes the row statistics from `a` and keeps the per-channel sums of its lanes' channels in registers; the
 // waves of a workgroup add theirs in LDS and write one partial row per gradient, which batch_sum_kernel adds over the
 // workgroups in a fixed order.
-#include "vrwkv_common.h"
+#include "wave_sum.h"
 
 namespace vrwkv {
 namespace {
 
 enum { PRE_NONE = 0, PRE_RELU_SQ = 1 };
 enum { POST_NONE = 0, POST_SIGMOID_GATE = 1, POST_RESIDUAL = 2 };
-
-// Sum over the 64 lanes, the same value in every lane: four DPP steps inside each row of 16 lanes (quad swaps, half-row
-// and row mirrors), then the four row sums through scalar registers.  All lanes must be active.
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float x) {
-    return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float wave_sum(float x) {
-    x = dpp_add<0xB1>(x);      // quad_perm [1,0,3,2]
-    x = dpp_add<0x4E>(x);      // quad_perm [2,3,0,1]
-    x = dpp_add<0x141>(x);     // row_half_mirror
-    x = dpp_add<0x140>(x);     // row_mirror
-    const int xi = __builtin_bit_cast(int, x);
-    const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(xi, 0)),
-                r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(xi, 16)),
-                r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(xi, 32)),
-                r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(xi, 48));
-    return (r0 + r1) + (r2 + r3);
-}
 
 // W waves share a row (1: a wave per row, short rows; 4: the workgroup's four waves, long rows), a thread keeps VPL
 // 16-byte vectors of it.  A group takes R rows whose loads are all issued before the first value is used, so a thread
