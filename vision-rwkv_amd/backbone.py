@@ -298,10 +298,12 @@ class _ChannelMix(torch.autograd.Function):
 
 # Where the grouped launches take the place of the library's products.  Two or more projections of one shape on M tokens in one launch
 # are ahead from 70 tiles of 128 x 128 each on; a single one without an epilogue stays with the library.  M x K x N, library / own, us:
-#   three of 784 x 768 x 768 23 / 15    4096 35 / 22    8192 46 / 37    11760 60 / 53    12544 79 / 52    (one: 7.6 / 13, 12 / 15, 15 / 17, 20 / 21, 27 / 21)
-#   three of 784 x 1024 x 1024 27 / 19  4096 41 / 33    9216 90 / 65    10816 79 / 84    12544 84 / 82    three of 12544 x 384 x 384 33 / 23
+#   three of 784 x 768 x 768 23 / 14    4096 36 / 21    8192 47 / 34    11760 63 / 52    12544 80 / 52    (one: 7.6 / 13, 12 / 15, 15 / 17, 20 / 21, 27 / 21)
+#   three of 784 x 1024 x 1024 27 / 19  4096 41 / 33    9216 89 / 61    10816 80 / 80    12544 79 / 82    three of 12544 x 384 x 384 33 / 23
 # A whole channel mix without key_norm takes them from 256 tiles on, where the passes they save (28 us forward, 43 back at 12544 x 3072)
-# outweigh a slower product: 4096 x 3072 x 768 30 / 39, 8192 44 / 41, 12544 60 / 55; 12544 x 768 x 3072 64 / 67; 12544 x 4096 x 1024 83 / 90.
+# outweigh a slower product: 4096 x 3072 x 768 28 / 34, 8192 42 / 40, 12544 62 / 54; 12544 x 768 x 3072 66 / 67; 12544 x 4096 x 1024 86 / 91.
+# With key_norm the products stay the library's: inside VRWKV-L, whose weights come from memory, a value product with the gate as its epilogue
+# takes 93 us at 9216 x 4096 x 1024 (two stages; 67 on weights that lie in the caches), the library's and the gate's pass 67 + 10.
 # Training steps of 64 images of 224 x 224, start and both of these: VRWKV-B 16195 -> 15108 us, VRWKV6-B 25761 -> 24499, bit for bit the same.
 CHANNEL_MIX_TILES = 256 * 128 * 128
 

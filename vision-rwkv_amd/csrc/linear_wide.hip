@@ -19,8 +19,8 @@
 // A lane ends up with 16 neighbouring channels of a token: the weights are the first operand of a product (result rows = channels),
 // and LDS row 16 f + 4 q + e of a wave's 64 channels holds channel 16 q + 4 f + e.
 //
-// us, three products of one shape in one launch here / three calls of the library: 12544 x 768 x 768 54 / 85, 9216 x 1024 x 1024 62 / 91;
-// one: 21 / 29, 23 / 31; 12544 x 768 x 3072 65 / 58, 12544 x 3072 x 768 56 / 64, 9216 x 1024 x 4096 74 / 68, 9216 x 4096 x 1024 80 / 65.
+// us, three products of one shape in one launch here / three calls of the library: 12544 x 768 x 768 52 / 80, 9216 x 1024 x 1024 61 / 89;
+// one: 21 / 28, 24 / 31; 12544 x 768 x 3072 67 / 66, 12544 x 3072 x 768 54 / 62, 9216 x 1024 x 4096 79 / 79, 9216 x 4096 x 1024 67 / 71.
 #include "linear.h"
 #include <algorithm>
 
@@ -30,7 +30,7 @@ using gemm::f32x4;
 using gemm::u32x4;
 
 constexpr int WM = 2, WN = 4, FN = 4, NT = 64 * WM * WN, TN = WN * FN * 16;
-// s_waitcnt for at most `vm` vector memory operations in flight (loads and stores return in order); LDS operations too
+// s_waitcnt for at most `vm` vector memory operations in flight; LDS operations too
 constexpr int wait_vm(int vm) { return 0x0F70 | (vm & 15) | (vm >> 4 << 14); }
 constexpr int wait_vm_lds(int vm) { return wait_vm(vm) & ~0x0F00; }
 
@@ -43,7 +43,7 @@ template <typename IO, int FM, int STAGES>
 __global__ __launch_bounds__(NT, 2)
 void linear_wide_kernel(LinGroup G, int tiles)
 {
-    constexpr int TM = WM * FM * 16, ROWS = TN + TM, PW = TN * 8 / NT, PER = PW + (TM * 8 + NT - 1) / NT, STORES = FM * FN / 2;
+    constexpr int TM = WM * FM * 16, ROWS = TN + TM, PW = TN * 8 / NT, PER = PW + (TM * 8 + NT - 1) / NT;
     // separate arrays: the compiler lets a read of one pass loads in flight to another
     __shared__ __attribute__((aligned(16))) char L0[ROWS * 128];
     __shared__ __attribute__((aligned(16))) char L1[ROWS * 128];
@@ -145,7 +145,6 @@ void linear_wide_kernel(LinGroup G, int tiles)
     __builtin_amdgcn_s_barrier();
 #pragma unroll
     for (int q = 0; q < FM + FN; ++q) read(L0, 0, q);
-    bool stored = false;
     for (int round = 0;; ++round) {
         const int t = tile_of(round);
         if (t >= tiles) break;
@@ -156,12 +155,11 @@ void linear_wide_kernel(LinGroup G, int tiles)
         for (int i = 0; i < FM; ++i)
 #pragma unroll
             for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        // One slice: behind the barrier everyone has read all of L, and the next stage has landed.  The stores of the tile before
-        // are younger than what the first slice waits for.
+        // One slice: behind the barrier everyone has read all of L, and the next stage has landed.  (After a tile that waits for its
+        // stores as well; counting them out measured the same, and nothing then hangs on the order in which loads and stores retire.)
 #define SLICE(L, NEXT)                                                                       \
         products(std::false_type{}, L, L, 0);                                                \
-        if (stored) { __builtin_amdgcn_s_waitcnt(wait_vm_lds((STAGES - 2) * PER + STORES)); stored = false; } \
-        else __builtin_amdgcn_s_waitcnt(wait_vm_lds((STAGES - 2) * PER));                                     \
+        __builtin_amdgcn_s_waitcnt(wait_vm_lds((STAGES - 2) * PER));                         \
         __builtin_amdgcn_s_barrier();                                                        \
         __builtin_amdgcn_sched_barrier(0);                                                   \
         products(std::true_type{}, L, NEXT, 1);
@@ -176,8 +174,8 @@ void linear_wide_kernel(LinGroup G, int tiles)
             }
         }
 #undef SLICE
-        // the epilogue, a token's sixteen channels as two pieces of eight; outside the result reads give 0 and stores are dropped (but
-        // counted).  The rows that an epilogue reads are requested a token ahead.
+        // the epilogue, a token's sixteen channels as two pieces of eight; outside the result reads give 0 and stores are
+        // dropped.  The rows that an epilogue reads are requested a token ahead.
         typedef BufRaw<16>::type piece_t;
         const unsigned bytes = (unsigned)G.M * P.N * 2u;
         const __amdgpu_buffer_rsrc_t ro = make_rsrc(P.out, bytes), rg = make_rsrc(P.gate, bytes), rr = make_rsrc(P.res, bytes), rp = make_rsrc(P.raw, bytes);
@@ -257,7 +255,6 @@ void linear_wide_kernel(LinGroup G, int tiles)
             for (int h = 0; h < 2; ++h) BufRaw<16>::st(out[h], ro, o, 16 * h);
             __builtin_amdgcn_sched_barrier(0);
         }
-        stored = true;
     }
     __builtin_amdgcn_s_waitcnt(wait_vm(0));               // nothing may land in LDS once the workgroup has left it
 }
