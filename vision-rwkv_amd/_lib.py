@@ -4,6 +4,7 @@ The library is loaded from this directory; it is never compiled at import time a
 is no fallback: a missing library is a hard error.
 """
 import ctypes
+import importlib.util
 import os
 import subprocess
 
@@ -15,6 +16,7 @@ STATUS_NAMES = {0: "OK", 1: "INVALID_ARG", 2: "UNSUPPORTED_DTYPE", 3: "UNSUPPORT
                 4: "LAUNCH_FAILED", 5: "WORKSPACE_TOO_SMALL"}
 
 _lib = None
+_host = None
 
 
 class BlockArgs(ctypes.Structure):
@@ -51,8 +53,23 @@ class VrwkvError(RuntimeError):
         self.status = status
 
 
+def host():
+    """The compiled module of csrc/host: the operators' host side in C++.  It stands or falls with the library."""
+    global _host
+    if _host is None:
+        lib()
+        path = os.path.join(_HERE, "_host.so")
+        if not os.path.exists(path):
+            raise ImportError(f"{path} is missing: build it first (make -C vision-rwkv_amd/csrc)")
+        spec = importlib.util.spec_from_file_location("_host", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host
+
+
 def build(force=True):
-    """Compile libvrwkv_hip.so for gfx950 with the Makefile in csrc/ (hipcc cross-compiles
+    """Compile libvrwkv_hip.so for gfx950 and _host.so with the Makefile in csrc/ (hipcc cross-compiles
     without a GPU)."""
     cmd = ["make", "-C", os.path.join(_HERE, "csrc"), "-j8"]
     if force:

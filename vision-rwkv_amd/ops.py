@@ -231,7 +231,8 @@ def divided_takes(w, u, k, v):
 
 
 def wkv_divided(w, u, n, k, v):
-    return _WKVDivided.apply(w, u, n, k, v)
+    y = _lib.host().wkv(w, u, k, v, 1.0 / n)
+    return _WKVDivided.apply(w, u, n, k, v) if y is None else y
 
 
 class _WKVLegacy(torch.autograd.Function):
@@ -248,10 +249,19 @@ class _WKVLegacy(torch.autograd.Function):
         return (None, None, None) + tuple(WKV.backward(ctx, gy))
 
 
+def _plain_call(x):
+    """Whether to ask the compiled operators (csrc/host/host_ops.cpp), which look at the arguments themselves and answer None where a
+    Python class has to decide."""
+    return type(x) is torch.Tensor and x.is_cuda and not torch.compiler.is_compiling()
+
+
 def RUN_CUDA(*args):
     """RUN_CUDA(w, u, k, v) (vrwkv.py:64-65) or legacy RUN_CUDA(B, T, C, w, u, k, v)."""
     if len(args) == 4:
         w, u, k, v = args
+        y = _lib.host().wkv(w, u, k, v, 1.0) if _plain_call(k) else None
+        if y is not None:
+            return y
         return WKV.apply(w.cuda(), u.cuda(), k.cuda(), v.cuda())
     if len(args) == 7:
         B, T, C, w, u, k, v = args
@@ -387,6 +397,10 @@ class _WKV_6Unrecorded(WKV_6):
 
 def RUN_CUDA_RWKV6(B, T, C, H, r, k, v, w, u):
     """vrwkv6.py:72-73."""
+    if _plain_call(r):
+        y = _lib.host().wkv6(B, T, C, H, r, k, v, w, u, WKV_6.stays_whole(T, r.dtype))
+        if y is not None:
+            return y
     return (WKV_6 if torch.is_grad_enabled() else _WKV_6Unrecorded).apply(B, T, C, H, r, k, v, w, u)
 
 
@@ -850,37 +864,15 @@ def block_takes(x):
 
 def block_weights_fit(x, weights):
     """True when every weight is a plain contiguous parameter of x's type and device."""
-    dt, dev, kind = x.dtype, x.get_device(), torch.nn.Parameter
-    for p in weights:
-        if type(p) is not kind or p.dtype != dt or p.get_device() != dev or not p.is_contiguous():
-            return False
-    return True
+    return _lib.host().weights_fit(x, weights)
 
 
 def block_forward(x, tensors, params=None, **scalars):
     """vrwkv_block_fwd on the current stream: tensors and scalars fill the like-named fields of vrwkv_block_args; with params
     (fields of vrwkv_block6_params) vrwkv_block6_fwd.  None when a tensor is not aligned for 16-byte accesses."""
-    L = _lib.lib()
-    B, T, C = x.shape
-    out = torch.empty_like(x)
-    ptrs = {n: t.data_ptr() for n, t in tensors.items()}
-    ptrs["x"], ptrs["out"] = x.data_ptr(), out.data_ptr()
-    bits = 0
-    for p in ptrs.values():
-        bits |= p
-    if bits & 15:
-        return None
-    a = _lib.BlockArgs(B=B, T=T, C=C, dtype=_DT[x.dtype], **ptrs, **scalars)
-    a.workspace_bytes = L.vrwkv_block_fwd_workspace_bytes(B, T, C, a.hidden, a.heads, a.dtype)
-    ws = torch.empty(a.workspace_bytes, dtype=torch.uint8, device=x.device)
-    a.workspace = ws.data_ptr()
-    with _on(x.device):
-        if params is None:
-            _lib.check(L.vrwkv_block_fwd(ctypes.byref(a), _stream_ptr(x.device)))
-        else:
-            fp32 = sum(1 << i for i, n in enumerate(_lib.Block6Params.POINTERS[4:13]) if params[n].dtype == torch.float32)
-            p = _lib.Block6Params(fp32_vectors=fp32, **{n: t.data_ptr() for n, t in params.items()})
-            _lib.check(L.vrwkv_block6_fwd(ctypes.byref(a), ctypes.byref(p), _stream_ptr(x.device)))
+    out = _lib.host().block_forward(x, tensors, params, scalars)
+    if type(out) is int:
+        _lib.check(out)
     return out
 
 
