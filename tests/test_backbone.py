@@ -1245,3 +1245,60 @@ def test_table_resize_of_a_batch_of_cotangents(adjoint, monkeypatch):
         assert torch.allclose(b, single, rtol=1e-5, atol=1e-5)
         # the pair are each other's adjoint
         assert abs(float((y.detach() * g).sum() - (t.detach() * single).sum())) < 1e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n_mix,through,C,head,cls,shift", [(1, 1, 64, 64, 0, 1), (2, 2, 128, 64, 1, 1), (3, 1, 192, 0, 0, 1), (2, 1, 20, 0, 0, 2), (3, 2, 768, 0, 0, 1)])
+def test_shift_backward_adds_the_other_uses_gradients(dtype, n_mix, through, C, head, cls, shift):
+    """x's gradients from its other uses, added in the shift's backward kernel: what the kernel without them gives for fp32 inputs of the same
+    values, plus those, rounded once (half a unit of the type; 2^-21 of the terms for the fp32 sums)."""
+    from vision_rwkv_amd.ops import q_shift_mix_autograd
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    B, res = 3, (5, 7)
+    T = 35 + cls
+    x = rand(B, T, C).to(dtype).requires_grad_()
+    mixes = [rand(C).to(dtype).requires_grad_() for _ in range(n_mix)]
+    outs = q_shift_mix_autograd(x, mixes, shift, 1 / 4, res, head, through)
+    assert len(outs) == n_mix + through and all(torch.equal(o, x) for o in outs[n_mix:])
+    gs = [rand(B, T, C).to(dtype) for _ in outs]
+    got = torch.autograd.grad(outs, [x, *mixes], gs, retain_graph=True)
+    xf, mf = x.detach().float().requires_grad_(), [m.detach().float().requires_grad_() for m in mixes]
+    want = torch.autograd.grad(q_shift_mix_autograd(xf, mf, shift, 1 / 4, res, head), [xf, *mf], [t.float() for t in gs[:n_mix]])
+    full = want[0].double() + sum(t.double() for t in gs[n_mix:])
+    size = want[0].abs() + sum(t.float().abs() for t in gs[n_mix:])
+    unit = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    assert ((got[0].double() - full).abs() <= unit * full.abs() + 2.0 ** -21 * size + (6e-8 if dtype is torch.float16 else 0)).all()
+    assert all(torch.equal(a, b.to(dtype)) for a, b in zip(got[1:], want[1:]))
+    # a use that has no gradient, and only such uses
+    some = torch.autograd.grad(outs[:n_mix], x, gs[:n_mix], retain_graph=True)[0]
+    assert torch.equal(some, want[0].to(dtype))
+    assert torch.equal(torch.autograd.grad(outs[-1], x, gs[-1], retain_graph=True)[0], gs[-1])
+    # one that is to be differentiated again keeps its graph
+    s = rand(B, T, C).to(dtype).requires_grad_()
+    first = torch.autograd.grad((outs[-1] * s).sum(), x, create_graph=True)[0]
+    assert torch.equal(torch.autograd.grad(first.sum(), s)[0], torch.ones_like(s))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["v4", "v6"])
+@pytest.mark.parametrize("post", [True, False])
+def test_residual_gradients_added_in_the_shift_are_those_of_autograd(kind, post):
+    """Blocks whose residual branches go through the token shift against the same blocks called with hooks, which take x itself (fp32:
+    1e-5 of the norm, a sum's rounding over two blocks)."""
+    net = _small_backbone(kind, 64, torch.float32, post, True, False, (3, 4), "cuda")
+    img = torch.randn(2, 3, 48, 64, device="cuda")
+    def grads():
+        net.zero_grad(set_to_none=True)
+        out = net(img)
+        out = out[0] if isinstance(out, tuple) else out
+        (out * torch.linspace(-1, 1, out.numel(), device="cuda").view_as(out)).sum().backward()
+        return out.detach(), [p.grad for p in net.parameters() if p.grad is not None]
+    out, got = grads()
+    seen = []
+    handles = [m.register_forward_hook(lambda *a: seen.append(1)) for l in net.layers for m in (l.att, l.ffn)]
+    ref, want = grads()
+    [h.remove() for h in handles]
+    assert len(seen) == 2 * len(net.layers) and torch.equal(out, ref) and len(got) == len(want)
+    assert all((a - b).norm() <= 1e-5 * b.norm() + 1e-12 for a, b in zip(got, want))

@@ -70,16 +70,16 @@ def eval_cached(module, name, params, extra, make):
     return hit[1]
 
 
-def _mix(module, x, mixes, shift_pixel, gamma, patch_resolution, fused, head_dim=0):
-    """[x*m + q_shift(x)*(1-m) for m in mixes]: one fused kernel (forward, and backward under autograd); tensor ops
-    when `fused` is off or the tensors are not on the GPU."""
+def _mix(module, x, mixes, shift_pixel, gamma, patch_resolution, fused, head_dim=0, through=0):
+    """[x*m + q_shift(x)*(1-m) for m in mixes], and x itself `through` times for its other uses (see _branch): one fused kernel
+    (forward, and backward under autograd); tensor ops when `fused` is off or the tensors are not on the GPU."""
     if fused and x.is_cuda:
         if torch.is_grad_enabled() and (x.requires_grad or any(m.requires_grad for m in mixes)):
-            return q_shift_mix_autograd(x, mixes, shift_pixel, gamma, patch_resolution, head_dim)
+            return q_shift_mix_autograd(x, mixes, shift_pixel, gamma, patch_resolution, head_dim, through)
         table = eval_cached(module, "mix_table", mixes, x.device, lambda: stack_mixes(mixes, x.device))
-        return q_shift_mix(x.contiguous(), mixes, shift_pixel, gamma, patch_resolution, head_dim, mix_table=table)
+        return q_shift_mix(x.contiguous(), mixes, shift_pixel, gamma, patch_resolution, head_dim, mix_table=table) + [x] * through
     xx = q_shift(x, shift_pixel, gamma, patch_resolution)
-    return [x * m + xx * (1 - m) for m in mixes]
+    return [x * m + xx * (1 - m) for m in mixes] + [x] * through
 
 
 # Whose weight gradient is the framework's own kernel, by the weight's elements and the multiplications: its deep split pays until
@@ -422,6 +422,16 @@ def _as_built(module, kind):
     return (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks and "forward" not in module.__dict__)
 
 
+def _branch(mix, kind, x, res):
+    """mix(x), and x as the residual branch beside it takes it: where autograd records, what the token shift hands on, so that the shift's
+    backward kernel adds the residual branch's gradient and no pass over the tokens does.  A module with hooks is called as it is."""
+    if (torch.is_grad_enabled() and type(x) is torch.Tensor and x.is_cuda and x.requires_grad and _as_built(mix, kind)
+            and not mix._backward_hooks and not mix._backward_pre_hooks and not _hooks._global_forward_hooks and not _hooks._global_forward_pre_hooks
+            and not _hooks._global_backward_hooks and not _hooks._global_backward_pre_hooks and not _transformed()):
+        return mix.with_residual(x, res)
+    return mix(x, res), x
+
+
 def _block_weights(block, att, ffn, x):
     """The weights of a block that one native call can run (its linear maps with the shapes and without the biases they are
     built with, the norms with both vectors) and the numbers that go with them, as fields of vrwkv_block_args; None for any
@@ -491,10 +501,15 @@ class VRWKV_SpatialMix(nn.Module):
         self.fused_gate = True     # inference without key_norm: sigmoid(r) * y inside the Bi-WKV kernel
 
     def forward(self, x, patch_resolution):
+        return self.with_residual(x, patch_resolution)[0]
+
+    def with_residual(self, x, patch_resolution):
+        """forward(x), and x as the residual branch is to take it (see _branch)."""
         B, T, C = x.shape
+        res = x
         if self.shift_pixel > 0:
-            xk, xv, xr = _mix(self, x, [self.spatial_mix_k, self.spatial_mix_v, self.spatial_mix_r], self.shift_pixel,
-                              self.channel_gamma, patch_resolution, self.fused_shift)
+            xk, xv, xr, res = _mix(self, x, [self.spatial_mix_k, self.spatial_mix_v, self.spatial_mix_r], self.shift_pixel,
+                                   self.channel_gamma, patch_resolution, self.fused_shift, through=1)
         else:
             xk = xv = xr = x
         k, v, r = _projs((self.key, self.value, self.receptance), (xk, xv, xr))
@@ -509,14 +524,14 @@ class VRWKV_SpatialMix(nn.Module):
                                         (self.spatial_first / T).float().contiguous()))
             if self.key_norm is None and self.fused_gate and r.dtype == k.dtype:
                 # the receptance gate (vrwkv.py:185-186) applied inside the operator, before y is stored
-                return _proj(self.output, bi_wkv_forward(w, u, k.contiguous(), v.contiguous(), gate=r.contiguous()))
+                return _proj(self.output, bi_wkv_forward(w, u, k.contiguous(), v.contiguous(), gate=r.contiguous())), res
             y = bi_wkv_forward(w, u, k.contiguous(), v.contiguous())
         y = y.to(r.dtype)
         # key_norm and the sigmoid gate (vrwkv.py:184-186) in one pass; tensor ops under autograd
         kn = self.key_norm
         y = row_fuse(y, r, kn.weight if kn is not None else None, kn.bias if kn is not None else None, None,
                      PRE_NONE, POST_SIGMOID_GATE, kn.eps if kn is not None else 1e-5)
-        return _proj(self.output, y)
+        return _proj(self.output, y), res
 
 
 class VRWKV_ChannelMix(nn.Module):
@@ -535,12 +550,17 @@ class VRWKV_ChannelMix(nn.Module):
         self.value = nn.Linear(hidden, n_embd, bias=False)
 
     def forward(self, x, patch_resolution):
+        return self.with_residual(x, patch_resolution)[0]
+
+    def with_residual(self, x, patch_resolution):
+        """forward(x), and x as the residual branch is to take it (see _branch)."""
+        res = x
         if self.shift_pixel > 0:
-            xk, xr = _mix(self, x, [self.spatial_mix_k, self.spatial_mix_r], self.shift_pixel, self.channel_gamma,
-                          patch_resolution, self.fused_shift)
+            xk, xr, res = _mix(self, x, [self.spatial_mix_k, self.spatial_mix_r], self.shift_pixel, self.channel_gamma,
+                               patch_resolution, self.fused_shift, through=1)
         else:
             xk = xr = x
-        return _channel_mix(self, xk, xr)
+        return _channel_mix(self, xk, xr), res
 
 
 class Block(nn.Module):
@@ -609,8 +629,8 @@ class Block(nn.Module):
         # residual with layer scale (vrwkv.py:300-313): x + gamma * ln(branch(x)) or x + gamma * branch(ln(x)), the
         # scale, the add and the post-norm in one pass; tensor ops under autograd
         if self.post_norm:
-            x = row_fuse(self.att(x, patch_resolution), x, self.ln1.weight, self.ln1.bias, g1, PRE_NONE, POST_RESIDUAL, self.ln1.eps)
-            x = row_fuse(self.ffn(x, patch_resolution), x, self.ln2.weight, self.ln2.bias, g2, PRE_NONE, POST_RESIDUAL, self.ln2.eps)
+            x = row_fuse(*_branch(self.att, VRWKV_SpatialMix, x, patch_resolution), self.ln1.weight, self.ln1.bias, g1, PRE_NONE, POST_RESIDUAL, self.ln1.eps)
+            x = row_fuse(*_branch(self.ffn, VRWKV_ChannelMix, x, patch_resolution), self.ln2.weight, self.ln2.bias, g2, PRE_NONE, POST_RESIDUAL, self.ln2.eps)
         else:
             x = row_fuse(self.att(_layer_norm(self.ln1, x), patch_resolution), x, None, None, g1, PRE_NONE, POST_RESIDUAL)
             x = row_fuse(self.ffn(_layer_norm(self.ln2, x), patch_resolution), x, None, None, g2, PRE_NONE, POST_RESIDUAL)

@@ -10,7 +10,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .backbone import VRWKV, eval_cached, _proj, _projs, _channel_mix, _matmul, _bmm, _as_built, _block_may_fuse, _block_weights
+from .backbone import VRWKV, eval_cached, _proj, _projs, _channel_mix, _matmul, _bmm, _as_built, _branch, _block_may_fuse, _block_weights
 from .ops import (HEAD_SIZE, RUN_CUDA_RWKV6, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, maa_mix, groupnorm_gate, block_takes, block_weights_fit, block_forward, PRE_NONE, PRE_RELU_SQ, POST_NONE,
                   POST_SIGMOID_GATE, POST_RESIDUAL)
 
@@ -27,18 +27,18 @@ def q_shift_multihead(x, shift_pixel=1, head_dim=HEAD_SIZE, patch_resolution=Non
     return torch.cat((out, x[:, -1:]), dim=1) if with_cls_token else out
 
 
-def _shift_and_mix(module, x, mixes, shift_pixel, patch_resolution, with_cls_token, fused, params):
-    """[x*m + shift(x)*(1-m) for m in mixes()]; one HIP kernel (forward, and backward under autograd), tensor ops when
+def _shift_and_mix(module, x, mixes, shift_pixel, patch_resolution, with_cls_token, fused, params, through):
+    """[x*m + shift(x)*(1-m) for m in mixes()], and x itself `through` times for its other uses; one HIP kernel (forward, and backward under autograd), tensor ops when
     `fused` is off or off the GPU.  `mixes` is a callable (the vectors may be derived from `params`); at inference
     its stacked fp32 table is kept on the module."""
     if fused and x.is_cuda:
         if torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in params)):
-            return q_shift_mix_autograd(x, mixes(), shift_pixel, 1 / 4, patch_resolution, HEAD_SIZE)
+            return q_shift_mix_autograd(x, mixes(), shift_pixel, 1 / 4, patch_resolution, HEAD_SIZE, through)
         table = eval_cached(module, "mix_table", params, x.device, lambda: stack_mixes(mixes(), x.device))
         return q_shift_mix(x.contiguous(), [None] * table.shape[0], shift_pixel, 1 / 4, patch_resolution,
-                           head_dim=HEAD_SIZE, mix_table=table)
+                           head_dim=HEAD_SIZE, mix_table=table) + [x] * through
     sx = q_shift_multihead(x, shift_pixel, HEAD_SIZE, patch_resolution, with_cls_token)
-    return [x * m + sx * (1 - m) for m in mixes()]
+    return [x * m + sx * (1 - m) for m in mixes()] + [x] * through
 
 
 def _layer_norm(ln, x):
@@ -80,11 +80,15 @@ class VRWKV_SpatialMix_V6(nn.Module):
         self.ln_x = nn.GroupNorm(n_head, n_embd, eps=1e-5)
 
     def forward(self, x, patch_resolution):
+        return self.with_residual(x, patch_resolution)[0]
+
+    def with_residual(self, x, patch_resolution):
+        """forward(x), and x as the residual branch is to take it."""
         B, T, C = x.shape
         # shift(x) and x + (shift(x) - x) * maa_x = x*(1 - maa_x) + shift(x)*maa_x in one pass over x
-        sx, xxx = _shift_and_mix(self, x, lambda: [torch.zeros_like(self.time_maa_x), 1 - self.time_maa_x],
+        sx, xxx, x, res = _shift_and_mix(self, x, lambda: [torch.zeros_like(self.time_maa_x), 1 - self.time_maa_x],
                                  self.shift_pixel, patch_resolution, self.with_cls_token, self.fused_shift,
-                                 (self.time_maa_x,))
+                                 (self.time_maa_x,), 2)
         lo = torch.tanh(_matmul(xxx, self.time_maa_w1)).view(B * T, 5, -1).transpose(0, 1)
         m = _bmm(lo, self.time_maa_w2).view(5, B, T, C)
         # xw..xg = x + (sx - x) * (time_maa_* + m_*)  (vrwkv6.py:190-194): one pass at inference
@@ -102,7 +106,7 @@ class VRWKV_SpatialMix_V6(nn.Module):
             y = self.key_norm(y.to(gate.dtype))
         # ln_x over each head's channels, times silu(gate) (vrwkv6.py:199, 205-211): one pass at inference
         y = groupnorm_gate(y, gate, self.ln_x.weight, self.ln_x.bias, self.ln_x.num_groups, self.ln_x.eps)
-        return _proj(self.output, y)
+        return _proj(self.output, y), res
 
 
 class VRWKV_ChannelMix_V6(nn.Module):
@@ -122,10 +126,14 @@ class VRWKV_ChannelMix_V6(nn.Module):
         self.value = nn.Linear(hidden, n_embd, bias=False)
 
     def forward(self, x, patch_resolution):
-        xk, xr = _shift_and_mix(self, x, lambda: [self.spatial_mix_k, self.spatial_mix_r], self.shift_pixel,
-                                patch_resolution, self.with_cls_token, self.fused_shift,
-                                (self.spatial_mix_k, self.spatial_mix_r))
-        return _channel_mix(self, xk, xr)
+        return self.with_residual(x, patch_resolution)[0]
+
+    def with_residual(self, x, patch_resolution):
+        """forward(x), and x as the residual branch is to take it."""
+        xk, xr, res = _shift_and_mix(self, x, lambda: [self.spatial_mix_k, self.spatial_mix_r], self.shift_pixel,
+                                     patch_resolution, self.with_cls_token, self.fused_shift,
+                                     (self.spatial_mix_k, self.spatial_mix_r), 1)
+        return _channel_mix(self, xk, xr), res
 
 
 class Block6(nn.Module):
@@ -194,8 +202,8 @@ class Block6(nn.Module):
         g1 = self.gamma1 if self.layer_scale else None
         g2 = self.gamma2 if self.layer_scale else None
         if self.post_norm:                                   # scale, add and post-norm in one pass
-            x = row_fuse(self.att(x, patch_resolution), x, self.ln1.weight, self.ln1.bias, g1, PRE_NONE, POST_RESIDUAL, self.ln1.eps)
-            x = row_fuse(self.ffn(x, patch_resolution), x, self.ln2.weight, self.ln2.bias, g2, PRE_NONE, POST_RESIDUAL, self.ln2.eps)
+            x = row_fuse(*_branch(self.att, VRWKV_SpatialMix_V6, x, patch_resolution), self.ln1.weight, self.ln1.bias, g1, PRE_NONE, POST_RESIDUAL, self.ln1.eps)
+            x = row_fuse(*_branch(self.ffn, VRWKV_ChannelMix_V6, x, patch_resolution), self.ln2.weight, self.ln2.bias, g2, PRE_NONE, POST_RESIDUAL, self.ln2.eps)
         else:
             x = row_fuse(self.att(_layer_norm(self.ln1, x), patch_resolution), x, None, None, g1, PRE_NONE, POST_RESIDUAL)
             x = row_fuse(self.ffn(_layer_norm(self.ln2, x), patch_resolution), x, None, None, g2, PRE_NONE, POST_RESIDUAL)

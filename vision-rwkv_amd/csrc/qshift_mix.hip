@@ -125,10 +125,13 @@ __device__ __forceinline__ int qs_dst(int t, int dir, int Hp, int Wp, int shift,
     return (sx >= 0 && sx < Wp && sy >= 0 && sy < Hp) ? sy * Wp + sx : -1;
 }
 
-template <typename IO, int VEC, int NMIX>
+// NADD: gradients that x has from elsewhere (its residual branch, another use of it), a0 and a1, are added to gx before it is rounded.  What
+// bounds the kernel is memory; an addend costs one read of a token matrix here and two reads and a write as a pass of its own.  64 x 196 x 768
+// bf16 with 0 / 1 / 2 addends: two mixes 21.7 / 25.2 / 29.2 us, three 28.1 / 30.8 / 35.0, a pass that adds two matrices 9.8 (10.8 in a training step).
+template <typename IO, int VEC, int NMIX, int NADD>
 __global__ __launch_bounds__(QS_CX * QS_TY)
 void qshift_mix_bwd_kernel(const IO* __restrict__ x_, const float* __restrict__ mix_, const IO* __restrict__ g0,
-                           const IO* __restrict__ g1, const IO* __restrict__ g2, IO* __restrict__ gx_,
+                           const IO* __restrict__ g1, const IO* __restrict__ g2, const IO* __restrict__ a0, const IO* __restrict__ a1, IO* __restrict__ gx_,
                            float* __restrict__ gmix_part, int T, int C, int Hp, int Wp, int shift, int g, int head_dim,
                            int n_grid_tokens, int n_tchunk, int gx, int gz)
 {
@@ -154,7 +157,7 @@ void qshift_mix_bwd_kernel(const IO* __restrict__ x_, const float* __restrict__ 
     using Packed = typename RawVec<sizeof(IO) * VEC>::type;
     if (cok) {
         for (int t0 = t_begin + ty; t0 < t_end; t0 += QS_TOK * QS_TY) {
-            Packed pxs[QS_TOK], pgt[QS_TOK][NMIX], pgd[QS_TOK][NMIX];
+            Packed pxs[QS_TOK], pgt[QS_TOK][NMIX], pgd[QS_TOK][NMIX], pa[QS_TOK][NADD ? NADD : 1];
             float keep_d[QS_TOK];
             int tt[QS_TOK];
 #pragma unroll
@@ -166,6 +169,8 @@ void qshift_mix_bwd_kernel(const IO* __restrict__ x_, const float* __restrict__ 
                 // a neighbour outside the grid is read from the token itself and masked: no divergent branches
                 keep_d[j] = td >= 0 ? 1.f : 0.f;
                 pxs[j] = load_packed<IO, VEC>(x_ + slab + (size_t)tl * C);
+                if (NADD > 0) pa[j][0] = load_packed<IO, VEC>(a0 + slab + (size_t)tl * C);
+                if (NADD > 1) pa[j][NADD - 1] = load_packed<IO, VEC>(a1 + slab + (size_t)tl * C);
 #pragma unroll
                 for (int m = 0; m < NMIX; ++m) {
                     pgt[j][m] = load_packed<IO, VEC>(gs[m] + slab + (size_t)tl * C);
@@ -196,6 +201,13 @@ void qshift_mix_bwd_kernel(const IO* __restrict__ x_, const float* __restrict__ 
                         acc[m][e] = fmaf(xs[e], diff, acc[m][e]);
                     }
                 }
+#pragma unroll
+                for (int a = 0; a < NADD; ++a) {
+                    float ga[VEC];
+                    widen_packed<IO, VEC>(pa[j][a], ga);
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) gx[e] += ga[e];
+                }
                 if constexpr (sizeof(IO) * VEC == 16) store_vec_nt<IO, VEC>(gx_ + slab + (size_t)tt[j] * C, gx);
                 else store_vec<IO, VEC>(gx_ + slab + (size_t)tt[j] * C, gx);
             }
@@ -219,8 +231,14 @@ void qshift_mix_bwd_kernel(const IO* __restrict__ x_, const float* __restrict__ 
     }
 }
 
+// The gradients of x from elsewhere: up to two token matrices.
+struct Addends {
+    const void* p[2];
+    int n;
+};
+
 template <typename IO, int VEC>
-int launch_bwd(const void* x, const float* mix, const void* const* gout, void* gx, SumOut gmix, float* part, int n_mix,
+int launch_bwd(const void* x, const float* mix, const void* const* gout, const Addends& add, void* gx, SumOut gmix, float* part, int n_mix,
                int B, int T, int C, int Hp, int Wp, int shift, int g, int head_dim, int n_grid, hipStream_t st) {
     const int ncv = C / VEC;
     const dim3 block(QS_CX * QS_TY);
@@ -241,10 +259,20 @@ int launch_bwd(const void* x, const float* mix, const void* const* gout, void* g
     const IO* g1 = n_mix > 1 ? static_cast<const IO*>(gout[1]) : nullptr;
     const IO* g2 = n_mix > 2 ? static_cast<const IO*>(gout[2]) : nullptr;
     IO* pgx = static_cast<IO*>(gx);
-    switch (n_mix) {
-        case 1: hipLaunchKernelGGL((qshift_mix_bwd_kernel<IO, VEC, 1>), grid, block, 0, st, xx, mix, g0, g1, g2, pgx, part, T, C, Hp, Wp, shift, g, head_dim, n_grid, n_tchunk, gbx, B); break;
-        case 2: hipLaunchKernelGGL((qshift_mix_bwd_kernel<IO, VEC, 2>), grid, block, 0, st, xx, mix, g0, g1, g2, pgx, part, T, C, Hp, Wp, shift, g, head_dim, n_grid, n_tchunk, gbx, B); break;
-        case 3: hipLaunchKernelGGL((qshift_mix_bwd_kernel<IO, VEC, 3>), grid, block, 0, st, xx, mix, g0, g1, g2, pgx, part, T, C, Hp, Wp, shift, g, head_dim, n_grid, n_tchunk, gbx, B); break;
+    const IO *a0 = static_cast<const IO*>(add.p[0]), *a1 = static_cast<const IO*>(add.p[1]);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, st, xx, mix, g0, g1, g2, a0, a1, pgx, part, T, C, Hp, Wp, shift, g, head_dim, n_grid, n_tchunk, gbx, B);
+    };
+    switch (n_mix * 3 + add.n) {
+        case 3: go(qshift_mix_bwd_kernel<IO, VEC, 1, 0>); break;
+        case 4: go(qshift_mix_bwd_kernel<IO, VEC, 1, 1>); break;
+        case 5: go(qshift_mix_bwd_kernel<IO, VEC, 1, 2>); break;
+        case 6: go(qshift_mix_bwd_kernel<IO, VEC, 2, 0>); break;
+        case 7: go(qshift_mix_bwd_kernel<IO, VEC, 2, 1>); break;
+        case 8: go(qshift_mix_bwd_kernel<IO, VEC, 2, 2>); break;
+        case 9: go(qshift_mix_bwd_kernel<IO, VEC, 3, 0>); break;
+        case 10: go(qshift_mix_bwd_kernel<IO, VEC, 3, 1>); break;
+        case 11: go(qshift_mix_bwd_kernel<IO, VEC, 3, 2>); break;
     }
     // gmix[m][c] = sum over the B * n_tchunk partial rows: the rows are (n_mix * C) wide
     const int wide = n_mix * C;
@@ -253,15 +281,15 @@ int launch_bwd(const void* x, const float* mix, const void* const* gout, void* g
 }
 
 template <typename IO>
-int launch_bwd_io(const void* x, const float* mix, const void* const* gout, void* gx, SumOut gmix, float* part, int n_mix,
+int launch_bwd_io(const void* x, const float* mix, const void* const* gout, const Addends& add, void* gx, SumOut gmix, float* part, int n_mix,
                   int B, int T, int C, int Hp, int Wp, int shift, int g, int head_dim, int n_grid, bool vec_ok, hipStream_t st) {
     // four channels per thread: 16-byte accesses of fp32, 8-byte ones of 16-bit elements (eight channels per thread
     // cost 153 registers with three mixes, three waves per SIMD: measured 10-13 % slower)
     constexpr int V = 4;
     const int period = head_dim > 0 ? head_dim : C;
     if (vec_ok && C % V == 0 && g % V == 0 && period % V == 0)
-        return launch_bwd<IO, V>(x, mix, gout, gx, gmix, part, n_mix, B, T, C, Hp, Wp, shift, g, head_dim, n_grid, st);
-    return launch_bwd<IO, 1>(x, mix, gout, gx, gmix, part, n_mix, B, T, C, Hp, Wp, shift, g, head_dim, n_grid, st);
+        return launch_bwd<IO, V>(x, mix, gout, add, gx, gmix, part, n_mix, B, T, C, Hp, Wp, shift, g, head_dim, n_grid, st);
+    return launch_bwd<IO, 1>(x, mix, gout, add, gx, gmix, part, n_mix, B, T, C, Hp, Wp, shift, g, head_dim, n_grid, st);
 }
 
 template <typename IO, int VEC>
@@ -354,7 +382,7 @@ extern "C" size_t vrwkv_qshift_mix_bwd_workspace_bytes(int n_mix, int B, int T, 
     return (size_t)B * ((T + QS_TCH - 1) / QS_TCH) * n_mix * C * sizeof(float);
 }
 
-static int qshift_mix_bwd(const void* x, const float* mix, const void* const* gout, int n_mix,
+static int qshift_mix_bwd(const void* x, const float* mix, const void* const* gout, int n_mix, const Addends& add,
                                     void* gx, SumOut gmix, int B, int T, int C, int Hp, int Wp, int shift_pixel,
                                     int quarter_width, int head_dim, int io_dtype,
                                     void* workspace, size_t workspace_bytes, void* hip_stream)
@@ -390,6 +418,10 @@ static int qshift_mix_bwd(const void* x, const float* mix, const void* const* go
         if (!gout[m]) { set_error("qshift_mix_bwd: null gradient pointer %d", m); return VRWKV_INVALID_ARG; }
         bits |= (uintptr_t)gout[m];
     }
+    for (int a = 0; a < add.n; ++a) {
+        if (!add.p[a]) { set_error("qshift_mix_bwd: null addend %d", a); return VRWKV_INVALID_ARG; }
+        bits |= (uintptr_t)add.p[a];
+    }
     const size_t need = vrwkv_qshift_mix_bwd_workspace_bytes(n_mix, B, T, C);
     if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 3)) {
         set_error("qshift_mix_bwd: a 4-byte aligned workspace of %zu bytes is required", need);
@@ -399,9 +431,9 @@ static int qshift_mix_bwd(const void* x, const float* mix, const void* const* go
     hipStream_t st = static_cast<hipStream_t>(hip_stream);
     float* part = static_cast<float*>(workspace);
     switch (io_dtype) {
-        case VRWKV_F32:  return launch_bwd_io<float>(x, mix, gout, gx, gmix, part, n_mix, B, T, C, Hp, Wp, shift_pixel, quarter_width, head_dim, n_grid, vec_ok, st);
-        case VRWKV_BF16: return launch_bwd_io<__hip_bfloat16>(x, mix, gout, gx, gmix, part, n_mix, B, T, C, Hp, Wp, shift_pixel, quarter_width, head_dim, n_grid, vec_ok, st);
-        case VRWKV_F16:  return launch_bwd_io<__half>(x, mix, gout, gx, gmix, part, n_mix, B, T, C, Hp, Wp, shift_pixel, quarter_width, head_dim, n_grid, vec_ok, st);
+        case VRWKV_F32:  return launch_bwd_io<float>(x, mix, gout, add, gx, gmix, part, n_mix, B, T, C, Hp, Wp, shift_pixel, quarter_width, head_dim, n_grid, vec_ok, st);
+        case VRWKV_BF16: return launch_bwd_io<__hip_bfloat16>(x, mix, gout, add, gx, gmix, part, n_mix, B, T, C, Hp, Wp, shift_pixel, quarter_width, head_dim, n_grid, vec_ok, st);
+        case VRWKV_F16:  return launch_bwd_io<__half>(x, mix, gout, add, gx, gmix, part, n_mix, B, T, C, Hp, Wp, shift_pixel, quarter_width, head_dim, n_grid, vec_ok, st);
     }
     return VRWKV_UNSUPPORTED_DTYPE;
 }
@@ -410,13 +442,29 @@ extern "C" int vrwkv_qshift_mix_bwd(const void* x, const float* mix, const void*
                                     void* gx, float* gmix, int B, int T, int C, int Hp, int Wp, int shift_pixel,
                                     int quarter_width, int head_dim, int io_dtype,
                                     void* workspace, size_t workspace_bytes, void* hip_stream) {
-    return qshift_mix_bwd(x, mix, gout, n_mix, gx, gmix, B, T, C, Hp, Wp, shift_pixel, quarter_width, head_dim, io_dtype, workspace, workspace_bytes, hip_stream);
+    return qshift_mix_bwd(x, mix, gout, n_mix, Addends{}, gx, gmix, B, T, C, Hp, Wp, shift_pixel, quarter_width, head_dim, io_dtype, workspace, workspace_bytes, hip_stream);
 }
 
 extern "C" int vrwkv_qshift_mix_bwd_like(const void* x, const float* mix, const void* const* gout, int n_mix,
                                     void* gx, void* gmix, int B, int T, int C, int Hp, int Wp, int shift_pixel,
                                     int quarter_width, int head_dim, int io_dtype,
                                     void* workspace, size_t workspace_bytes, void* hip_stream) {
-    return qshift_mix_bwd(x, mix, gout, n_mix, gx, SumOut(gmix, io_dtype), B, T, C, Hp, Wp, shift_pixel, quarter_width, head_dim, io_dtype, workspace, workspace_bytes, hip_stream);
+    return qshift_mix_bwd(x, mix, gout, n_mix, Addends{}, gx, SumOut(gmix, io_dtype), B, T, C, Hp, Wp, shift_pixel, quarter_width, head_dim, io_dtype, workspace, workspace_bytes, hip_stream);
 }
 
+extern "C" int vrwkv_qshift_mix_bwd_add(const void* x, const float* mix, const void* const* gout, int n_mix, const void* const* add, int n_add,
+                                        void* gx, void* gmix, int gmix_dtype, int B, int T, int C, int Hp, int Wp, int shift_pixel,
+                                        int quarter_width, int head_dim, int io_dtype,
+                                        void* workspace, size_t workspace_bytes, void* hip_stream) {
+    if (n_add < 0 || n_add > 2 || (n_add && !add)) {
+        set_error("qshift_mix_bwd: 0 to 2 addends (got %d)", n_add);
+        return VRWKV_INVALID_ARG;
+    }
+    if (gmix_dtype != VRWKV_F32 && gmix_dtype != io_dtype) {
+        set_error("qshift_mix_bwd: the table's gradient is fp32 or of the type of x");
+        return VRWKV_UNSUPPORTED_DTYPE;
+    }
+    Addends a = {{nullptr, nullptr}, n_add};
+    for (int i = 0; i < n_add; ++i) a.p[i] = add[i];
+    return qshift_mix_bwd(x, mix, gout, n_mix, a, gx, SumOut(gmix, gmix_dtype), B, T, C, Hp, Wp, shift_pixel, quarter_width, head_dim, io_dtype, workspace, workspace_bytes, hip_stream);
+}

@@ -728,19 +728,21 @@ def groupnorm_gate(y, gate, gn_weight, gn_bias, n_groups, eps=1e-5):
 
 
 class _QShiftMix(torch.autograd.Function):
-    """q_shift + mix lerps with a hand-written backward (vrwkv_qshift_mix / vrwkv_qshift_mix_bwd); the mix vectors
+    """q_shift + mix lerps with a hand-written backward (vrwkv_qshift_mix / vrwkv_qshift_mix_bwd_add); the mix vectors
     enter as one (n_mix, C) table of their own type, so whatever produced them (parameters, 1 - parameter, ...) is differentiated
-    by autograd outside."""
+    by autograd outside.  through: as many more results, each x itself: what uses x next to the mixes takes one of these, and the
+    backward kernel adds its gradient where autograd would run a pass over the tokens."""
 
     @staticmethod
-    def forward(ctx, x, table, shift_pixel, gamma, Hp, Wp, head_dim):
+    def forward(ctx, x, table, shift_pixel, gamma, Hp, Wp, head_dim, through=0):
         x = x.contiguous()
         ctx.table_dtype = table.dtype
         table = table.float().contiguous()
         ctx.save_for_backward(x, table)
         ctx.meta = (shift_pixel, gamma, Hp, Wp, head_dim)
+        ctx.set_materialize_grads(False)
         outs = q_shift_mix(x, [None] * table.shape[0], shift_pixel, gamma, (Hp, Wp), head_dim, mix_table=table)
-        return tuple(outs)
+        return (*outs, *(x.view_as(x) for _ in range(through)))
 
     @staticmethod
     def backward(ctx, *gouts):
@@ -748,7 +750,11 @@ class _QShiftMix(torch.autograd.Function):
         shift_pixel, gamma, Hp, Wp, head_dim = ctx.meta
         B, T, C = x.shape
         n_mix = table.shape[0]
-        gs = [g.to(x.dtype).contiguous() for g in gouts]
+        gs = [g.to(x.dtype).contiguous() if g is not None else torch.zeros_like(x) for g in gouts[:n_mix]]
+        add, apart = [g for g in gouts[n_mix:] if g is not None], []
+        if torch.is_grad_enabled():                              # to be differentiated again: what has a graph is added by tensor ops
+            add, apart = [g for g in add if not g.requires_grad], [g for g in add if g.requires_grad]
+        add = [g.to(x.dtype).contiguous() for g in add]
         gx = torch.empty_like(x)
         like = ctx.table_dtype == x.dtype                        # the table's gradient rounded by the kernel, or cast below
         gmix = torch.empty_like(table, dtype=x.dtype if like else torch.float32)
@@ -756,18 +762,21 @@ class _QShiftMix(torch.autograd.Function):
         ws_bytes = L.vrwkv_qshift_mix_bwd_workspace_bytes(n_mix, B, T, C)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
         ptrs = (ctypes.c_void_p * n_mix)(*[g.data_ptr() for g in gs])
+        adds = (ctypes.c_void_p * 2)(*[g.data_ptr() for g in add])
         g = head_dim // 4 if head_dim else int(C * gamma)
         with _on(x.device):
-            fn = L.vrwkv_qshift_mix_bwd_like if like else L.vrwkv_qshift_mix_bwd
-            _lib.check(fn(x.data_ptr(), table.data_ptr(), ptrs, n_mix, gx.data_ptr(), gmix.data_ptr(),
-                          B, T, C, Hp, Wp, shift_pixel, g, head_dim, _DT[x.dtype],
-                          ws.data_ptr(), ws_bytes, _stream_ptr(x.device)))
-        return gx, gmix.to(ctx.table_dtype), None, None, None, None, None
+            _lib.check(L.vrwkv_qshift_mix_bwd_add(x.data_ptr(), table.data_ptr(), ptrs, n_mix, adds, len(add), gx.data_ptr(), gmix.data_ptr(),
+                                                  _DT[gmix.dtype], B, T, C, Hp, Wp, shift_pixel, g, head_dim, _DT[x.dtype],
+                                                  ws.data_ptr(), ws_bytes, _stream_ptr(x.device)))
+        for a in apart:
+            gx = gx + a
+        return gx, gmix.to(ctx.table_dtype), None, None, None, None, None, None
 
 
-def q_shift_mix_autograd(x, mixes, shift_pixel=1, gamma=1 / 4, patch_resolution=None, head_dim=0):
+def q_shift_mix_autograd(x, mixes, shift_pixel=1, gamma=1 / 4, patch_resolution=None, head_dim=0, through=0):
     """q_shift_mix for training: the same fused forward kernel, and one fused backward kernel in place of autograd
-    through the slice copies and lerps.  `mixes` may be parameters or tensors derived from parameters."""
+    through the slice copies and lerps.  `mixes` may be parameters or tensors derived from parameters.  through (0 to 2): so many
+    more results, x for its other uses, whose gradients the backward kernel adds."""
     _check_input(x, "x")
     if x.dim() != 3 or x.dtype not in _DT:
         raise RuntimeError("x must be (B,T,C) float32 / bfloat16 / float16")
@@ -776,8 +785,8 @@ def q_shift_mix_autograd(x, mixes, shift_pixel=1, gamma=1 / 4, patch_resolution=
     if not _equal_quarters(x.shape[-1], gamma, head_dim):
         table = table.float()
         xx = q_shift(x, shift_pixel, gamma, patch_resolution)
-        return [(x.float() * m + xx.float() * (1 - m)).to(x.dtype) for m in table]
-    return list(_QShiftMix.apply(x, table, shift_pixel, gamma, Hp, Wp, head_dim))
+        return [(x.float() * m + xx.float() * (1 - m)).to(x.dtype) for m in table] + [x] * through
+    return list(_QShiftMix.apply(x, table, shift_pixel, gamma, Hp, Wp, head_dim, through))
 
 
 class _TableResize(torch.autograd.Function):
