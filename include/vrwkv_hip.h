@@ -310,6 +310,10 @@ int vrwkv_biwkv_bwd_as(const void* w, const void* u, int wu_dtype, float factor,
  * the fp32 sums: what autograd asks of a 16-bit model's parameters ---- */
 int vrwkv_rowfuse_bwd_like(const void* a, const void* other, const void* ln_weight, const void* ln_bias, const void* gamma, const void* gout, void* ga, void* gother, void* gparam, long long rows, int N, int pre, int post, float eps, int io_dtype, void* workspace, size_t workspace_bytes, void* hip_stream);
 int vrwkv_qshift_mix_bwd_like(const void* x, const float* mix, const void* const* gout, int n_mix, void* gx, void* gmix, int B, int T, int C, int Hp, int Wp, int shift_pixel, int quarter_width, int head_dim, int io_dtype, void* workspace, size_t workspace_bytes, void* hip_stream);
+/* out (C) = the sums over the rows of x (rows, C), both of dtype: fp32 sums in a fixed order, rounded once.  The gradient of a vector that is
+ * added to every token.  workspace: vrwkv_column_sums_workspace_bytes(rows, C) bytes. */
+size_t vrwkv_column_sums_workspace_bytes(long long rows, int C);
+int vrwkv_column_sums(const void* x, void* out, long long rows, int C, int dtype, void* workspace, size_t workspace_bytes, void* hip_stream);
 /* With the gradients that x has from elsewhere: add[i] (B, T, C) of io_dtype, i < n_add <= 2, go into gx before it is rounded; gmix of gmix_dtype,
  * fp32 or io_dtype. */
 int vrwkv_qshift_mix_bwd_add(const void* x, const float* mix, const void* const* gout, int n_mix, const void* const* add, int n_add, void* gx, void* gmix, int gmix_dtype, int B, int T, int C, int Hp, int Wp, int shift_pixel, int quarter_width, int head_dim, int io_dtype, void* workspace, size_t workspace_bytes, void* hip_stream);

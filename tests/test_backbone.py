@@ -1302,3 +1302,25 @@ def test_residual_gradients_added_in_the_shift_are_those_of_autograd(kind, post)
     [h.remove() for h in handles]
     assert len(seen) == 2 * len(net.layers) and torch.equal(out, ref) and len(got) == len(want)
     assert all((a - b).norm() <= 1e-5 * b.norm() + 1e-12 for a, b in zip(got, want))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,T,C,skip", [(1, 1, 64, 0), (3, 11, 768, 0), (2, 17, 65, 0), (4, 196, 192, 1), (64, 196, 768, 0), (1, 33, 8, 0), (2, 4000, 1024, 0)])
+def test_vector_added_to_every_token_and_its_gradient(dtype, B, T, C, skip):
+    """The vector's gradient against float64: half a unit of the type (fp16: its subnormals too) and, for fp32 sums of at most 8 row lanes of a
+    chunk and 1024 chunks in 32 slices, 2^-24 of the summed sizes for each of 256 additions one after the other at most."""
+    from vision_rwkv_amd.ops import add_to_tokens
+    g = torch.Generator(device="cuda").manual_seed(5)
+    vec = torch.randn(1, 1, C, generator=g, device="cuda").to(dtype).requires_grad_()
+    x = torch.randn(B, T, C, generator=g, device="cuda").to(dtype).requires_grad_()
+    gy = torch.randn(B * T * C + skip, generator=g, device="cuda").to(dtype)[skip:].view(B, T, C)
+    y = add_to_tokens(vec, x)
+    assert torch.equal(y, vec + x) and "AddToTokens" in type(y.grad_fn).__name__
+    gv, gx = torch.autograd.grad(y, [vec, x], gy, retain_graph=True)
+    want, size = gy.double().sum((0, 1), keepdim=True), gy.double().abs().sum((0, 1), keepdim=True)
+    unit = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    assert torch.equal(gx, gy) and gv.shape == vec.shape and gv.dtype == dtype
+    assert ((gv.double() - want).abs() <= unit * want.abs() + 256 * 2.0 ** -24 * size + (6e-8 if dtype is torch.float16 else 0)).all()
+    twice = torch.autograd.grad((y * y).sum(), vec, create_graph=True)[0]
+    assert torch.equal(torch.autograd.grad(twice.sum(), vec)[0], torch.full_like(vec, 2 * B * T))

@@ -125,6 +125,10 @@ def _declare(lib):
     lib.vrwkv_qshift_mix_bwd_workspace_bytes.restype = sz
     lib.vrwkv_qshift_mix_bwd.argtypes = [vp, fp, c.POINTER(c.c_void_p), i, vp, fp, i, i, i, i, i, i, i, i, i, vp, sz, vp]
     lib.vrwkv_qshift_mix_bwd.restype = i
+    lib.vrwkv_column_sums_workspace_bytes.argtypes = [c.c_longlong, i]
+    lib.vrwkv_column_sums_workspace_bytes.restype = sz
+    lib.vrwkv_column_sums.argtypes = [vp, vp, c.c_longlong, i, i, vp, sz, vp]
+    lib.vrwkv_column_sums.restype = i
     lib.vrwkv_qshift_mix_bwd_add.argtypes = [vp, fp, c.POINTER(c.c_void_p), i, c.POINTER(c.c_void_p), i, vp, vp, i, i, i, i, i, i, i, i, i, i, vp, sz, vp]
     lib.vrwkv_qshift_mix_bwd_add.restype = i
     lib.vrwkv_rowfuse.argtypes = [vp, vp, vp, vp, vp, vp, c.c_longlong, i, i, i, c.c_float, i, vp]

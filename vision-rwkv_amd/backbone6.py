@@ -11,7 +11,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .backbone import VRWKV, eval_cached, _proj, _projs, _channel_mix, _matmul, _bmm, _as_built, _branch, _block_may_fuse, _block_weights
-from .ops import (HEAD_SIZE, RUN_CUDA_RWKV6, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, maa_mix, groupnorm_gate, block_takes, block_weights_fit, block_forward, PRE_NONE, PRE_RELU_SQ, POST_NONE,
+from .ops import (HEAD_SIZE, RUN_CUDA_RWKV6, add_to_tokens, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, maa_mix, groupnorm_gate, block_takes, block_weights_fit, block_forward, PRE_NONE, PRE_RELU_SQ, POST_NONE,
                   POST_SIGMOID_GATE, POST_RESIDUAL)
 
 
@@ -98,7 +98,7 @@ class VRWKV_SpatialMix_V6(nn.Module):
             table = eval_cached(self, "maa_table", maas, x.device, lambda: stack_mixes(maas, x.device))
         xw, xk, xv, xr, xg = maa_mix(x, sx, m, maas, table)
         r, k, v, gate = _projs((self.receptance, self.key, self.value, self.gate), (xr, xk, xv, xg))
-        w = self.time_decay + _matmul(torch.tanh(_matmul(xw, self.time_decay_w1)), self.time_decay_w2)
+        w = add_to_tokens(self.time_decay, _matmul(torch.tanh(_matmul(xw, self.time_decay_w1)), self.time_decay_w2))
         y = RUN_CUDA_RWKV6(B, T, C, self.n_head, r.contiguous(), k.contiguous(), v.contiguous(),
                            w.contiguous(), self.time_faaaa.float())                  # vrwkv6.py:217 (w as it is: the
         # kernel widens a 16-bit decay logit itself, the same values the reference's `w.float()` holds)

@@ -976,6 +976,42 @@ def linear_group(problems):
     return results
 
 
+def column_sums(x):
+    """The sums of a contiguous (..., C) GPU tensor over all but the channels (vrwkv_column_sums): fp32, rounded once."""
+    C = x.shape[-1]
+    rows = x.numel() // C
+    out = torch.empty(C, dtype=x.dtype, device=x.device)
+    L = _lib.lib()
+    ws_bytes = L.vrwkv_column_sums_workspace_bytes(rows, C)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
+    with _on(x.device):
+        _lib.check(L.vrwkv_column_sums(x.data_ptr(), out.data_ptr(), rows, C, _DT[x.dtype], ws.data_ptr(), ws_bytes, _stream_ptr(x.device)))
+    return out
+
+
+class _AddToTokens(torch.autograd.Function):
+    """vector + x for a vector (1, 1, C) and x (B, T, C) of its type, with the vector's gradient in column_sums."""
+
+    @staticmethod
+    def forward(ctx, vector, x):
+        return vector + x
+
+    @staticmethod
+    def backward(ctx, g):
+        if not ctx.needs_input_grad[0]:
+            return None, g
+        own = g.is_cuda and g.numel() > 0 and not torch.is_grad_enabled() and not batched_cotangent(g) and not _transformed()
+        return (column_sums(g.contiguous()).view(1, 1, -1) if own else g.sum((0, 1), keepdim=True)), g
+
+
+def add_to_tokens(vector, x):
+    """vector + x, a vector (1, 1, C) added to every token of x (B, T, C)."""
+    if (x.is_cuda and torch.is_grad_enabled() and vector.requires_grad and x.dtype in _DT and vector.dtype == x.dtype and x.dim() == 3
+            and tuple(vector.shape) == (1, 1, x.shape[-1]) and vector.device == x.device and not torch.is_autocast_enabled("cuda") and not _transformed()):
+        return _AddToTokens.apply(vector, x)
+    return vector + x
+
+
 def transposed(weights):
     """The transposes of 1 to 5 contiguous 16-bit matrices, one launch (vrwkv_transpose_group)."""
     n, dev = len(weights), weights[0].device
