@@ -310,6 +310,11 @@ int vrwkv_biwkv_bwd_as(const void* w, const void* u, int wu_dtype, float factor,
  * the fp32 sums: what autograd asks of a 16-bit model's parameters ---- */
 int vrwkv_rowfuse_bwd_like(const void* a, const void* other, const void* ln_weight, const void* ln_bias, const void* gamma, const void* gout, void* ga, void* gother, void* gparam, long long rows, int N, int pre, int post, float eps, int io_dtype, void* workspace, size_t workspace_bytes, void* hip_stream);
 int vrwkv_qshift_mix_bwd_like(const void* x, const float* mix, const void* const* gout, int n_mix, void* gx, void* gmix, int B, int T, int C, int Hp, int Wp, int shift_pixel, int quarter_width, int head_dim, int io_dtype, void* workspace, size_t workspace_bytes, void* hip_stream);
+/* vrwkv_maa_mix with the low-rank products of vrwkv6.py:183-186 inside: m_i = lo_i w2_i, lo (rows, 5 x 32), w2 (5, 32, C), 16-bit types, C a multiple
+ * of 64.  The backward forms m again; gm (5, rows, C) are the gradients of the products.  The token matrices are 16-byte aligned. */
+int vrwkv_maa_lora_mix(const void* x, const void* sx, const void* lo, const void* w2, const float* maa, void* const* out, long long rows, int C, int io_dtype, void* hip_stream);
+size_t vrwkv_maa_lora_mix_bwd_workspace_bytes(long long rows, int C);
+int vrwkv_maa_lora_mix_bwd(const void* x, const void* sx, const void* lo, const void* w2, const float* maa, const void* const* gout, void* gx, void* gsx, void* gm, float* gmaa, long long rows, int C, int io_dtype, void* workspace, size_t workspace_bytes, void* hip_stream);
 /* out (C) = the sums over the rows of x (rows, C), both of dtype: fp32 sums in a fixed order, rounded once.  The gradient of a vector that is
  * added to every token.  workspace: vrwkv_column_sums_workspace_bytes(rows, C) bytes. */
 size_t vrwkv_column_sums_workspace_bytes(long long rows, int C);

@@ -1324,3 +1324,73 @@ def test_vector_added_to_every_token_and_its_gradient(dtype, B, T, C, skip):
     assert ((gv.double() - want).abs() <= unit * want.abs() + 256 * 2.0 ** -24 * size + (6e-8 if dtype is torch.float16 else 0)).all()
     twice = torch.autograd.grad((y * y).sum(), vec, create_graph=True)[0]
     assert torch.equal(torch.autograd.grad(twice.sum(), vec)[0], torch.full_like(vec, 2 * B * T))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,T,C", [(1, 1, 64), (1, 16, 128), (2, 33, 192), (3, 197, 384), (1, 2000, 768), (64, 196, 768), (2, 70, 1024)])
+def test_mixes_with_their_low_rank_products_inside(dtype, B, T, C, monkeypatch):
+    """Against the same steps in float64 from the same 16-bit values: m rounded to the type first (as a product's result is), then one rounding
+    per result.  A gradient sum's fp32 terms add 2^-21 of their sizes; where m falls on a rounding boundary, its two neighbours differ
+    by a unit of the type."""
+    from vision_rwkv_amd.ops import maa_lora_mix
+    g = torch.Generator(device="cuda").manual_seed(9)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dtype).requires_grad_()
+    x, sx, lo, w2, maas = rand(B, T, C), rand(B, T, C), rand(B * T, 160), rand(5, 32, C), [rand(1, 1, C) for _ in range(5)]
+    product = lambda a, b: torch.bmm(a.transpose(1, 2).contiguous(), b)
+    outs = maa_lora_mix(x, sx, lo, w2, maas, product)
+    with torch.no_grad():
+        assert all(torch.equal(a, b) for a, b in zip(outs, maa_lora_mix(x, sx, lo, w2, maas, product)))
+    gs = [torch.randn(B, T, C, generator=g, device="cuda").to(dtype) for _ in range(5)]
+    got = torch.autograd.grad(outs, [x, sx, *maas], gs, retain_graph=True)
+    glo, gw2 = torch.autograd.grad(outs, [lo, w2], gs, retain_graph=True)
+    unit = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    tiny = 6e-8 if dtype is torch.float16 else 0.0
+    d = lambda t: t.detach().double()
+    stack = lo.detach().view(B * T, 5, 32).transpose(0, 1)
+    exact = torch.bmm(d(stack), d(w2)).view(5, B, T, C)
+    m = exact.to(dtype).double()
+    off = 2 * unit * exact.abs() + 2.0 ** -20 * torch.bmm(d(stack).abs(), d(w2).abs()).view(5, B, T, C) + tiny      # of m, at most
+    f, xx = torch.stack([d(a) for a in maas]).view(5, 1, 1, C) + m, d(sx) - d(x)
+    G = torch.stack([d(t) for t in gs])
+    near = lambda a, want, slack: ((d(a) - want).abs() <= unit * (want.abs() + slack) + slack + 2.0 ** -21 + tiny).all()
+    for i in range(5):
+        assert near(outs[i], d(x) + xx * f[i], xx.abs() * off[i] + 2.0 ** -21 * (d(x).abs() + (xx * f[i]).abs()))
+    assert near(got[0], (G * (1 - f)).sum(0), (G.abs() * off).sum(0) + 2.0 ** -21 * (G.abs() * (1 + f.abs())).sum(0))
+    assert near(got[1], (G * f).sum(0), (G.abs() * off).sum(0) + 2.0 ** -21 * (G.abs() * f.abs()).sum(0))
+    gm = (G * xx).view(5, B * T, C)
+    for i in range(5):
+        want, size = gm[i].sum(0), gm[i].abs().sum(0)
+        assert ((d(got[2 + i]).view(-1) - want).abs() <= unit * want.abs() + 2.0 ** -16 * size + tiny).all()
+    gm16 = gm.to(dtype)
+    for a, want, size in ((glo, torch.bmm(gm, d(w2).transpose(1, 2)).transpose(0, 1).reshape(lo.shape), torch.bmm(gm.abs(), d(w2).abs().transpose(1, 2)).transpose(0, 1).reshape(lo.shape)),
+                          (gw2, torch.bmm(d(stack).transpose(1, 2), gm), torch.bmm(d(stack).abs().transpose(1, 2), gm.abs()))):
+        assert ((d(a) - want).abs() <= unit * want.abs() + (unit + 2.0 ** -16) * size + tiny).all()      # gm rounded once before the products
+    # to be differentiated again: tensor ops, the same values within their roundings, and a graph
+    again = torch.autograd.grad(outs, x, gs, create_graph=True)[0]
+    assert again.requires_grad and ((d(again) - d(got[0])).norm() <= 8 * unit * d(got[0]).norm())
+    assert maa_lora_mix(x.float(), sx.float(), lo.float(), w2.float(), [a.float() for a in maas], product) is None
+    assert maa_lora_mix(x[..., :60], sx[..., :60], lo, w2[..., :60], [a[..., :60] for a in maas], product) is None
+    with torch.autocast("cuda"):
+        assert maa_lora_mix(x, sx, lo, w2, maas, product) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("post", [True, False])
+def test_model_with_mixes_inside_is_the_model_without(post, monkeypatch):
+    """VRWKV6 blocks with the products inside the mixes against products of their own: the forward bit for bit, the gradients within bf16's
+    rounding of two blocks."""
+    from vision_rwkv_amd import backbone6
+    net = _small_backbone("v6", 128, torch.bfloat16, False, post, True, (5, 7), "cuda").train()
+    img = torch.randn(3, 3, 80, 112, device="cuda").bfloat16()
+    def run():
+        net.zero_grad(set_to_none=True)
+        out = net(img)
+        out = out[0] if isinstance(out, tuple) else out
+        (out.float() * torch.linspace(-1, 1, out.numel(), device="cuda").view_as(out)).sum().backward()
+        return out.detach(), {n: p.grad.double() for n, p in net.named_parameters() if p.grad is not None}
+    out, got = run()
+    monkeypatch.setattr(backbone6, "maa_lora_mix", lambda *a: None)
+    ref, want = run()
+    assert torch.equal(out, ref) and got.keys() == want.keys()
+    assert all((got[n] - want[n]).norm() <= 3e-2 * want[n].norm() + 1e-9 for n in got), {n: ((got[n] - want[n]).norm() / want[n].norm()).item() for n in got}

@@ -125,6 +125,12 @@ def _declare(lib):
     lib.vrwkv_qshift_mix_bwd_workspace_bytes.restype = sz
     lib.vrwkv_qshift_mix_bwd.argtypes = [vp, fp, c.POINTER(c.c_void_p), i, vp, fp, i, i, i, i, i, i, i, i, i, vp, sz, vp]
     lib.vrwkv_qshift_mix_bwd.restype = i
+    lib.vrwkv_maa_lora_mix.argtypes = [vp, vp, vp, vp, fp, c.POINTER(c.c_void_p), c.c_longlong, i, i, vp]
+    lib.vrwkv_maa_lora_mix.restype = i
+    lib.vrwkv_maa_lora_mix_bwd_workspace_bytes.argtypes = [c.c_longlong, i]
+    lib.vrwkv_maa_lora_mix_bwd_workspace_bytes.restype = sz
+    lib.vrwkv_maa_lora_mix_bwd.argtypes = [vp, vp, vp, vp, fp, c.POINTER(c.c_void_p), vp, vp, vp, fp, c.c_longlong, i, i, vp, sz, vp]
+    lib.vrwkv_maa_lora_mix_bwd.restype = i
     lib.vrwkv_column_sums_workspace_bytes.argtypes = [c.c_longlong, i]
     lib.vrwkv_column_sums_workspace_bytes.restype = sz
     lib.vrwkv_column_sums.argtypes = [vp, vp, c.c_longlong, i, i, vp, sz, vp]

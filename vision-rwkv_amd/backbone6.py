@@ -10,8 +10,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .backbone import VRWKV, eval_cached, _proj, _projs, _channel_mix, _matmul, _bmm, _as_built, _branch, _block_may_fuse, _block_weights
-from .ops import (HEAD_SIZE, RUN_CUDA_RWKV6, add_to_tokens, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, maa_mix, groupnorm_gate, block_takes, block_weights_fit, block_forward, PRE_NONE, PRE_RELU_SQ, POST_NONE,
+from .backbone import VRWKV, eval_cached, _proj, _projs, _channel_mix, _matmul, _bmm, _token_product, _as_built, _branch, _block_may_fuse, _block_weights
+from .ops import (HEAD_SIZE, RUN_CUDA_RWKV6, add_to_tokens, maa_lora_mix, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, maa_mix, groupnorm_gate, block_takes, block_weights_fit, block_forward, PRE_NONE, PRE_RELU_SQ, POST_NONE,
                   POST_SIGMOID_GATE, POST_RESIDUAL)
 
 
@@ -89,14 +89,17 @@ class VRWKV_SpatialMix_V6(nn.Module):
         sx, xxx, x, res = _shift_and_mix(self, x, lambda: [torch.zeros_like(self.time_maa_x), 1 - self.time_maa_x],
                                  self.shift_pixel, patch_resolution, self.with_cls_token, self.fused_shift,
                                  (self.time_maa_x,), 2)
-        lo = torch.tanh(_matmul(xxx, self.time_maa_w1)).view(B * T, 5, -1).transpose(0, 1)
-        m = _bmm(lo, self.time_maa_w2).view(5, B, T, C)
-        # xw..xg = x + (sx - x) * (time_maa_* + m_*)  (vrwkv6.py:190-194): one pass at inference
+        lo = torch.tanh(_matmul(xxx, self.time_maa_w1)).view(B * T, -1)
+        # xw..xg = x + (sx - x) * (time_maa_* + m_*)  (vrwkv6.py:183-194): one pass, the low-rank products inside where that applies
         maas = (self.time_maa_w, self.time_maa_k, self.time_maa_v, self.time_maa_r, self.time_maa_g)
         table = None
         if not torch.is_grad_enabled() and x.is_cuda:
             table = eval_cached(self, "maa_table", maas, x.device, lambda: stack_mixes(maas, x.device))
-        xw, xk, xv, xr, xg = maa_mix(x, sx, m, maas, table)
+        mixed = maa_lora_mix(x, sx, lo, self.time_maa_w2, maas, lambda a, b: _token_product(a, b, 8), table)
+        if mixed is None:
+            m = _bmm(lo.view(B * T, 5, -1).transpose(0, 1), self.time_maa_w2).view(5, B, T, C)
+            mixed = maa_mix(x, sx, m, maas, table)
+        xw, xk, xv, xr, xg = mixed
         r, k, v, gate = _projs((self.receptance, self.key, self.value, self.gate), (xr, xk, xv, xg))
         w = add_to_tokens(self.time_decay, _matmul(torch.tanh(_matmul(xw, self.time_decay_w1)), self.time_decay_w2))
         y = RUN_CUDA_RWKV6(B, T, C, self.n_head, r.contiguous(), k.contiguous(), v.contiguous(),

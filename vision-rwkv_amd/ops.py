@@ -648,6 +648,71 @@ def maa_mix(x, sx, m, maas, maa_table=None):
     return _maa_mix_launch(xc, sxc, mc, table)
 
 
+class _MaaLoraMix(torch.autograd.Function):
+    """The five mixes with their low-rank products inside (vrwkv_maa_lora_mix and its backward, which forms the products again); lo (M, 160),
+    w2 (5, 32, C), table as for _MaaMix."""
+
+    @staticmethod
+    def forward(ctx, x, sx, lo, w2, table, token_product):
+        ctx.save_for_backward(x, sx, lo, w2, table)
+        ctx.token_product = token_product
+        return tuple(_maa_lora_launch(x, sx, lo, w2, table))
+
+    @staticmethod
+    def backward(ctx, *gouts):
+        x, sx, lo, w2, table = ctx.saved_tensors
+        C = x.shape[-1]
+        rows = x.numel() // C
+        stack = lo.view(rows, 5, -1).transpose(0, 1)
+        gs = [g.to(x.dtype) for g in gouts]
+        if torch.is_grad_enabled() or batched_cotangent(*gs) or _transformed():
+            f = [t + m.view(x.shape) for t, m in zip(table.to(x.dtype), torch.bmm(stack, w2))]
+            gx, gsx = sum(g * (1 - t) for g, t in zip(gs, f)), sum(g * t for g, t in zip(gs, f))
+            gm = torch.stack([(g * (sx - x)).reshape(rows, C) for g in gs])
+            gtable = gm.float().sum(1)
+        else:
+            gs = [g.contiguous() for g in gs]
+            gx, gsx, gtable = torch.empty_like(x), torch.empty_like(x), torch.empty_like(table)
+            gm = torch.empty((5, rows, C), dtype=x.dtype, device=x.device)
+            L = _lib.lib()
+            ws_bytes = L.vrwkv_maa_lora_mix_bwd_workspace_bytes(rows, C)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
+            with _on(x.device):
+                _lib.check(L.vrwkv_maa_lora_mix_bwd(x.data_ptr(), sx.data_ptr(), lo.data_ptr(), w2.data_ptr(), table.data_ptr(),
+                                                    (ctypes.c_void_p * 5)(*[g.data_ptr() for g in gs]), gx.data_ptr(), gsx.data_ptr(), gm.data_ptr(),
+                                                    gtable.data_ptr(), rows, C, _DT[x.dtype], ws.data_ptr(), ws_bytes, _stream_ptr(x.device)))
+        need = ctx.needs_input_grad
+        glo = torch.bmm(gm, w2.transpose(1, 2)).transpose(0, 1).reshape(lo.shape) if need[2] else None
+        gw2 = ctx.token_product(stack, gm) if need[3] else None
+        return gx, gsx, glo, gw2, gtable, None
+
+
+def _maa_lora_launch(x, sx, lo, w2, table):
+    C = x.shape[-1]
+    outs = [torch.empty_like(x) for _ in range(5)]
+    with _on(x.device):
+        _lib.check(_lib.lib().vrwkv_maa_lora_mix(x.data_ptr(), sx.data_ptr(), lo.data_ptr(), w2.data_ptr(), table.data_ptr(),
+                                                 (ctypes.c_void_p * 5)(*[o.data_ptr() for o in outs]), x.numel() // C, C, _DT[x.dtype],
+                                                 _stream_ptr(x.device)))
+    return outs
+
+
+def maa_lora_mix(x, sx, lo, w2, maas, token_product, maa_table=None):
+    """maa_mix(x, sx, m, maas) with m_i = lo_i w2_i formed inside (vrwkv6.py:183-194): lo (B*T, 160), w2 (5, 32, C), 16-bit tensors.  None where
+    the kernels do not apply.  token_product(a, b): a^T b over the tokens, for the gradient of w2."""
+    C = x.shape[-1]
+    tensors = (x, sx, lo, w2, *maas)
+    if not (ROW_FUSE_ENABLED and x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and x.dim() == 3 and x.numel() > 0 and C % 64 == 0 and C <= 65536
+            and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == x.dtype and t.device == x.device for t in tensors)
+            and sx.shape == x.shape and tuple(w2.shape) == (5, 32, C) and tuple(lo.shape) == (x.numel() // C, 160) and all(m.numel() == C for m in maas)
+            and all(t.is_contiguous() for t in (x, sx, lo, w2)) and _vec_ok(x, sx, lo, w2) and x.numel() // C <= 65535 * 64
+            and not torch.is_autocast_enabled("cuda") and not _transformed()):
+        return None
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return list(_MaaLoraMix.apply(x, sx, lo, w2, torch.stack([a.reshape(-1) for a in maas]).float(), token_product))
+    return _maa_lora_launch(x, sx, lo, w2, maa_table if maa_table is not None else stack_mixes(maas, x.device))
+
+
 def groupnorm_gate_tensor_ops(y, gate, gn_weight, gn_bias, n_groups, eps=1e-5):
     """vrwkv6.py:205-211 and :199: ln_x on the (B*T, C) view, times silu(gate).  The group statistics are written out
     with mean / var instead of torch.nn.functional.group_norm: on a GPU that function's backward returns wrong weight
