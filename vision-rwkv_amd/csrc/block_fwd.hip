@@ -3,7 +3,8 @@
 //
 // A block of one 224 x 224 image (196 tokens) is 16 (VRWKV) or 26 (VRWKV6) operator calls of 2-20 us of GPU work each, and a call
 // through the Python operators and the library costs about 20 us of host time, so the host sets the pace; on top the
-// library picks tiles of 192 x 256 for 196 x 192 results (13 us a product).  Issued from here a VRWKV block is 9 launches:
+// library picks tiles of 192 x 256 for 196 x 192 results (13 us a product).  Issued from here a VRWKV block is 9 launches, 7 on few tokens,
+// where the norm and the shift behind it are one (ln_shift_mix.hip):
 //   LN | shift + mixes | key, value, receptance | Bi-WKV with gate | output + residual
 //   LN | shift + mixes | key with relu^2, receptance | value, gate, residual
 #include "linear.h"
@@ -393,11 +394,16 @@ static int block_fwd(const vrwkv_block_args* args, const vrwkv_block6_params* pa
         G.n = 1;
         G.p[0] = linear(s[1], a->maa_w1, lo, 160, C, 0, EPI_TANH);
         TRY(linear_group(G, dt, st));
+        if (params && dt != VRWKV_F32 && !((uintptr_t)params->maa_w2 & 15)) {         // w, k, v, r, g, the five maps formed inside
+            TRY(vrwkv_maa_lora_mix(src, s[0], lo, params->maa_w2, a->maa, m, M, C, dt, st));
+        } else {
+            G.n = 5;
+            for (int i = 0; i < 5; ++i)                   // the five maps as one (5, M, C) tensor
+                G.p[i] = linear((const char*)lo + 32 * es * i, (const char*)a->maa_w2 + (size_t)i * C * 32 * es, maps + (size_t)i * M * C * es, C, 32, 160);
+            TRY(linear_group(G, dt, st));
+            TRY(vrwkv_maa_mix(src, s[0], maps, a->maa, m, M, C, dt, st));
+        }
         G.n = 5;
-        for (int i = 0; i < 5; ++i)                       // the five maps as one (5, M, C) tensor
-            G.p[i] = linear((const char*)lo + 32 * es * i, (const char*)a->maa_w2 + (size_t)i * C * 32 * es, maps + (size_t)i * M * C * es, C, 32, 160);
-        TRY(linear_group(G, dt, st));
-        TRY(vrwkv_maa_mix(src, s[0], maps, a->maa, m, M, C, dt, st));                 // w, k, v, r, g
         G.p[0] = linear(m[0], a->decay_w1, dlo, 64, C, 0, EPI_TANH);
         G.p[1] = linear(m[1], a->key, five[1], C, C);
         G.p[2] = linear(m[2], a->value, five[2], C, C);

@@ -16,6 +16,7 @@
 //  vrwkv_groupnorm_gate_bwd  s = silu(gate), yn = xh w + b:  g_gate = g yn s',  gyn = g s,  g_w[c] = sum_rows gyn xh,
 //                            g_b[c] = sum_rows gyn,  gy = rstd (w gyn - mean_grp(w gyn) - xh mean_grp(w gyn xh))
 #include "vrwkv_common.h"
+#include <type_traits>
 
 namespace vrwkv {
 namespace {
@@ -46,7 +47,11 @@ void maa_mix_kernel(const IO* __restrict__ x_, const IO* __restrict__ sx_, const
         for (int e4 = 0; e4 < V; e4 += 4)
             load_vec<float, 4>(maa_ + (size_t)i * C + c + e4, *reinterpret_cast<float(*)[4]>(&a[e4]));
 #pragma unroll
-        for (int e = 0; e < V; ++e) r[e] = fmaf(d[e], a[e] + m[e], x[e]);
+        for (int e = 0; e < V; ++e) {
+            r[e] = fmaf(d[e], a[e] + m[e], x[e]);
+            // in fp32 first, like mix6_lora.hip: in fp16 some results would be rounded from the exact sum at once otherwise
+            if constexpr (std::is_same<IO, __half>::value) asm volatile("" : "+v"(r[e]));
+        }
         store_vec<IO, V>(outs[i] + e0, r);
     }
 }

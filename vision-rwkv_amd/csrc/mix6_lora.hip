@@ -12,8 +12,8 @@
 // workgroup's tokens in five registers (80 sums a lane, added up at the end, spill); LDS adds the four waves, and one partial row per workgroup
 // leaves for batch_sum_kernel.
 //
-// bf16, product and mix of their own -> here, forward | backward (the product's gradients come after it in either), us, the five products bit for bit
-// the library's: 12544 x 768 70 -> 38 | 89 -> 73     12544 x 384 40 -> 19 | 57 -> 36     12544 x 192 36 -> 13 | 27 -> 22     1568 x 768 19 -> 9 | 18 -> 16
+// bf16, product and mix of their own -> here, forward | backward (the product's gradients come after it in either), us, results bit for bit
+// the same: 12544 x 768 70 -> 38 | 89 -> 73     12544 x 384 40 -> 19 | 57 -> 36     12544 x 192 36 -> 13 | 27 -> 22     1568 x 768 19 -> 9 | 18 -> 16
 // 196 x 192 20 -> 5 | 12 -> 9.  The bytes at 5 TB/s: 12544 x 768 28 | 54.
 #include "gemm_tile.h"
 #include "wkv6_chunk_common.h"
@@ -74,7 +74,14 @@ __device__ __forceinline__ void factors(const LoraLds<IO>& L, int i, u32x4 lo, i
         const f32x4 m = gemm::mfma16<IO>(w, lo, f32x4{0.f, 0.f, 0.f, 0.f});
         const f32x4 a = *reinterpret_cast<const f32x4*>(&L.A[i][32 * (q >> 1) + 8 * g4 + 4 * (q & 1)]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) f[4 * q + e] = a[e] + to_f32(from_f32<IO>(m[e]));
+        for (int e = 0; e < 4; ++e) {
+            IO r = from_f32<IO>(m[e]);
+            unsigned short bits;
+            __builtin_memcpy(&bits, &r, 2);
+            asm volatile("" : "+v"(bits));                 // a rounding to fp16 and back is contracted away otherwise
+            __builtin_memcpy(&r, &bits, 2);
+            f[4 * q + e] = a[e] + to_f32(r);
+        }
     }
 }
 
@@ -95,7 +102,12 @@ __device__ __forceinline__ void widen16(const Raw16& r, float (&v)[16]) {
     for (int e = 0; e < 16; ++e) v[e] = to_f32(t[e]);
 }
 template <typename IO>
-__device__ __forceinline__ void store16(void* p, size_t e0, const float (&v)[16]) {
+__device__ __forceinline__ void store16(void* p, size_t e0, float (&v)[16]) {
+    if constexpr (std::is_same<IO, __half>::value) {
+        // fp32 values, as the other kernels round them: a mixed-precision multiply-add would round the exact sum to fp16 at once
+#pragma unroll
+        for (int e = 0; e < 16; ++e) asm volatile("" : "+v"(v[e]));
+    }
     store_vec<IO, 8>(static_cast<IO*>(p) + e0, *reinterpret_cast<const float(*)[8]>(&v[0]));
     store_vec<IO, 8>(static_cast<IO*>(p) + e0 + 32, *reinterpret_cast<const float(*)[8]>(&v[8]));
 }
