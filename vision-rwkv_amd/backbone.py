@@ -405,7 +405,7 @@ def _native_size(x, hidden, v6):
 #   VRWKV  bf16  1568 x 768   3559 -> 1483 | 1595 -> 1480      3136 x 768, key norms 3597 -> 1901 | 1900 -> 1884      6272 x 768 3587 -> 2388 | 3064 -> 2384
 #                12544 x 768  4923 -> 3799 | 4887 -> 3785      25088 x 768  9237 -> 7356 | 9191 -> 7357      12544 x 192 3562 -> 1169 | 1483 -> 1158
 #   VRWKV6 bf16  1568 x 768   5887 -> 2246 | 2678 -> 2269      12544 x 768  7433 -> 6389 | 7422 -> 6383      12544 x 192 6272 -> 2069 | 2686 -> 2054
-# (VRWKV6 before the mixes formed their low-rank products inside, which takes 30 us a block off either: 12544 x 768 native 5890 since.)
+# (VRWKV6 before the mixes formed their low-rank products inside, which takes 30 to 40 us a block of 12544 x 768 off either.)
 NATIVE_WIDE, NATIVE_WIDE_GAP = 768, (600_000_000, 1_600_000_000)
 
 
