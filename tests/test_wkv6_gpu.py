@@ -215,3 +215,26 @@ def test_results_of_a_sequence_of_up_to_256_tokens_do_not_depend_on_the_batch(op
         yb = ops.RUN_CUDA_RWKV6(1, T, 64 * H, H, *one, u)
         assert torch.equal(yb[0], y[b])
         assert all(torch.equal(p[0], q[b]) for p, q in zip(torch.autograd.grad(yb, one, gy[b:b + 1].contiguous()), grads))
+
+
+@pytest.mark.parametrize("B,T,H,dtype", [(8, 577, 6, torch.float32), (8, 577, 6, torch.bfloat16), (16, 577, 6, torch.bfloat16), (10, 370, 6, torch.float16),
+                                         (1, 4150, 3, torch.float16), (2, 577, 6, torch.bfloat16), (2, 300, 12, torch.float32)])
+def test_the_planned_cut_is_the_whole_sequence(ops, B, T, H, dtype):
+    """Sequences cut as the plan of their type has it against uncut ones: either is 5e-6 of the norm from float64 at most, so 1e-5 apart; the workspace
+    that is asked for serves every type."""
+    C = 64 * H
+    g = torch.Generator(device="cuda").manual_seed(2)
+    r, k, v = (torch.randn(B, T, C, generator=g, device="cuda").to(dtype) for _ in range(3))
+    w = (torch.randn(B, T, C, generator=g, device="cuda") - 3).to(dtype)
+    u = torch.randn(H, 64, generator=g, device="cuda") * 0.1
+    whole = ops.wkv6_forward(B, T, C, H, r, k, v, w, u, whole=True)
+    y = ops.wkv6_forward(B, T, C, H, r, k, v, w, u)
+    assert not torch.equal(y, whole) and (y - whole).norm() <= 1e-5 * whole.norm()
+    L = ops.lib()
+    dt = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}[dtype]
+    need = L.vrwkv_wkv6_fwd_workspace_bytes(B, T, C, H)
+    out, ws = torch.empty_like(whole), torch.empty(need, dtype=torch.uint8, device="cuda")
+    args = [t.data_ptr() for t in (r, k, v, w, u, out)] + [B, T, C, H, dt, dt, 0, ws.data_ptr()]
+    assert L.vrwkv_wkv6_fwd(*args, need, None) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out, y)
