@@ -194,3 +194,18 @@ def test_parameter_gradients_of_the_inputs_type_are_the_rounded_fp32_sums(B, T, 
     like = bi_wkv_backward(w, u, k, v, gy, like_inputs=True)
     assert all(a.dtype == dtype for a in like)
     assert all(torch.equal(a.to(dtype), b) for a, b in zip(full, like))
+
+
+@pytest.mark.parametrize("B,T,C", [(1, 225, 64), (2, 577, 384), (1, 1025, 192), (8, 577, 384), (1, 1793, 70), (2, 4150, 64), (20, 300, 128), (3, 640, 1024)])
+@pytest.mark.parametrize("tokens", [0, 16, 25, 28])
+def test_super_chunks_of_every_length(ops, B, T, C, tokens):
+    """Long sequences by 16, 25 and 28 tokens a wave, and by the plan, against the C oracle (the fp32 bounds of the other tests here)."""
+    from oracle import clib
+    rng = np.random.default_rng(T + C)
+    k, v, gy = (rng.standard_normal((B, T, C)).astype(np.float32) for _ in range(3))
+    w = (rng.uniform(-5, 3, C) / T).astype(np.float32)
+    u = rng.uniform(-1, 1, C).astype(np.float32)
+    with ops.option("biwkv_l", tokens):
+        got = run(ops, w, u, k, v, gy)[:4]
+    for a, r, bound in zip(got, clib.biwkv_bwd(w, u, k, v, gy), (2e-4, 1e-4, 1e-4, 1e-4)):
+        assert rel_err(a, r) <= bound

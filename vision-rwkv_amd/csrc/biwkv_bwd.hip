@@ -61,6 +61,28 @@ struct BwdPlan {
     size_t planes = 0, agg1 = 0, agg2 = 0, parts = 0, total = 0;
 };
 
+// Tokens per wave of a sequence cut into super-chunks of eight waves.  The tiles (sequence, super-chunk, 64 channels) go to as many workgroups
+// as there are compute units, in rounds: the length with the shortest rounds together, a round being its tokens and a share that does not depend
+// on them (25 fits the sweep below).  Beyond eight rounds 28, the fewest tiles.  28 / 25 / 16 tokens a wave, us:
+//   fp32  2 x 4150 x 768 (456 / 504 / 792 tiles)   86.5 / 85.0 / 135.2     8 x 1025 x 768 (480 / 576 / 864)     74.1 / 93.6 / 100.8
+//         16 x 577 x 384 (288 / 288 / 480)         63.8 / 61.8 / 52.4      24 x 577 x 1024 (1152 / 1152 / 1920)  159.7 / 155.8 / 184.6
+//         1 x 1025 x 192 (15 / 18 / 27)            30.0 / 29.2 / 26.0      4 x 4150 x 768 (912 / 1008 / 1584)    160.5 / 163.4 / 231.2
+//   bf16  24 x 577 x 1024 138.5 / 128.6 / 159.6    16 x 577 x 384 56.5 / 52.9 / 46.7    32 x 300 x 768 (768 / 768 / 1152) 81.5 / 77.6 / 96.9
+// The forward keeps 28: its 16-bit kernels read sequences of two or three super-chunks of that length once, and a 16-bit network amplifies the last bits
+// that the cut decides (fp32 gains 3 % at 2 x 4150 x 768).
+int super_chunk_tokens(int B, int T, int C) {
+    const long long columns = (long long)B * ((C + WAVE - 1) / WAVE), cus = biwkv_fwd_detail::num_cus();
+    int best = 28;
+    long long least = -1;
+    for (int L : {28, 25, 16}) {
+        const long long tiles = columns * ((T + BWD_SMAX * L - 1) / (BWD_SMAX * L)), rounds = (tiles + cus - 1) / cus;
+        if (L != 28 && rounds > 8) continue;
+        const long long cost = rounds * (L + 25);
+        if (least < 0 || cost < least) { best = L; least = cost; }
+    }
+    return best;
+}
+
 BwdPlan make_bwd_plan(int B, int T, int C) {
     BwdPlan p;
     static const int kL[] = {4, 8, 16, 25, 28};
@@ -72,7 +94,8 @@ BwdPlan make_bwd_plan(int B, int T, int C) {
         if (p.L) {
             p.S = (T + p.L - 1) / p.L;
         } else {
-            p.L = 28; p.S = BWD_SMAX;
+            p.L = el == 28 || el == 25 || el == 16 ? el : super_chunk_tokens(B, T, C);
+            p.S = BWD_SMAX;
             p.nSC = (T + p.S * p.L - 1) / (p.S * p.L);
         }
     }
@@ -106,7 +129,7 @@ void launch_tiled(const BwdPlan& p, const ParamVec& w, const ParamVec& u, const 
         }
         hipLaunchKernelGGL((biwkv_bwd_tile_kernel<IO, L, 0>), g, blk, 0, st, w, u, k, v, gy, gk, gv, ws, agg1, agg2,
                            gw_part, gu_part, B, T, C, geo);
-    } else if constexpr (L == 28) {
+    } else if constexpr (L == 28 || L == 25 || L == 16) {
         hipLaunchKernelGGL((biwkv_bwd_tile_kernel<IO, L, 1>), g, blk, 0, st, w, u, k, v, gy, gk, gv, ws, agg1, agg2,
                            gw_part, gu_part, B, T, C, geo);
         hipLaunchKernelGGL((biwkv_bwd_tile_kernel<IO, L, 2>), g, blk, 0, st, w, u, k, v, gy, gk, gv, ws, agg1, agg2,
