@@ -1394,3 +1394,50 @@ def test_model_with_mixes_inside_is_the_model_without(post, monkeypatch):
     ref, want = run()
     assert torch.equal(out, ref) and got.keys() == want.keys()
     assert all((got[n] - want[n]).norm() <= 3e-2 * want[n].norm() + 1e-9 for n in got), {n: ((got[n] - want[n]).norm() / want[n].norm()).item() for n in got}
+
+
+MISFITS = [("key", (192, 768)), ("receptance", (192, 384)), ("value", (384, 384)), ("value", (1536, 384)), ("receptance", (384, 192)), ("receptance", (384, 768)),
+           ("value", (768, 192)), ("value", (768, 768))]
+
+
+def test_weights_that_do_not_fit_their_inputs_are_not_the_grouped_launchs():
+    """The rule of the grouped launch for a channel mix of 384 channels and 768 hidden ones, every tensor but the device's name as on a
+    GPU: every weight has its input's width."""
+    from types import SimpleNamespace
+    from vision_rwkv_amd.ops import linear_takes
+    x = SimpleNamespace(shape=(2, 4096, 384), numel=lambda: 2 * 4096 * 384, is_cuda=True, dtype=torch.bfloat16, device=torch.device("cpu"))
+    weight = lambda i, o: torch.zeros(o, i, dtype=torch.bfloat16)
+    fits = dict(key=weight(384, 768), receptance=weight(384, 384), value=weight(768, 384))
+    assert linear_takes(x, [fits["receptance"]] * 3)
+    for wrong in (weight(192, 384), weight(768, 384), torch.zeros(384, dtype=torch.bfloat16)):
+        assert not linear_takes(x, [fits["receptance"], wrong])
+    rule = lambda ws: linear_takes(x, list(ws.values()), (384, 384, ws["key"].shape[0]))
+    assert rule(fits)
+    for name, size in MISFITS[:4]:
+        assert not rule({**fits, name: weight(*size)}), (name, size)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("name,size", MISFITS)
+def test_channel_mixes_whose_weights_do_not_fit_raise_as_the_operators_do(name, size, grad):
+    """Layers replaced by ones of another width: what nn.Linear and the gate's product raise.  (384 channels, 768 hidden, 8192 tokens.)"""
+    from vision_rwkv_amd import backbone as bb, ops
+    d = "cuda"
+    ffn = bb.VRWKV_ChannelMix(384, 2, 0, hidden_rate=2).to(d).bfloat16()
+    x = torch.randn(2, 4096, 384, device=d).bfloat16().requires_grad_(grad)
+    setattr(ffn, name, torch.nn.Linear(*size, bias=False, device=d).bfloat16())
+    with torch.set_grad_enabled(grad):
+        with pytest.raises(RuntimeError):
+            bb._channel_mix(ffn, x, x)
+        if name == "value" and size[0] == 768:               # ... and both of one other width
+            ffn.receptance = torch.nn.Linear(384, size[1], bias=False, device=d).bfloat16()
+            assert bb._channel_mix(ffn, x, x).shape == (2, 4096, size[1])
+        lins = [torch.nn.Linear(i, 384, bias=False, device=d).bfloat16() for i in (384, size[0] if size[0] != 384 else 192)]
+        with pytest.raises(RuntimeError):
+            bb._projs(lins, [x, x])
+        a, w = x.detach().view(-1, 384), lins[1].weight.detach()
+        with pytest.raises(RuntimeError, match="must be"):
+            ops.linear_group([dict(a=a, w=w)])
+        with pytest.raises(RuntimeError, match="must be"):
+            ops.linear_group([dict(a=a, w=lins[0].weight.detach(), gate=a[:, :192].contiguous())])

@@ -308,8 +308,9 @@ class _ChannelMix(torch.autograd.Function):
 CHANNEL_MIX_TILES = 256 * 128 * 128
 
 
-def _own_weights(linears, x):
-    """The weights of projections whose module call does nothing but multiply, and which vrwkv_linear_group takes; else None."""
+def _own_weights(linears, x, widths=None):
+    """The weights of projections whose module call does nothing but multiply, and which vrwkv_linear_group takes; else None.  widths: of
+    the projections' inputs, where they are not x."""
     if (_hooks._global_forward_hooks or _hooks._global_forward_pre_hooks or _hooks._global_backward_hooks
             or _hooks._global_backward_pre_hooks):
         return None
@@ -317,7 +318,7 @@ def _own_weights(linears, x):
         if not _as_built(l, nn.Linear) or l._backward_hooks or l._backward_pre_hooks or l.bias is not None or type(l._parameters.get("weight")) is not nn.Parameter:
             return None
     ws = [l.weight for l in linears]
-    return ws if linear_takes(x, ws) else None
+    return ws if linear_takes(x, ws, widths) else None
 
 
 def _projs(linears, xs):
@@ -334,8 +335,9 @@ def _channel_mix(ffn, xk, xr):
     """What a channel mix makes of its two mixed inputs (vrwkv.py:250-261), by the rules above."""
     kn = ffn.key_norm
     if kn is None and ops.ROW_FUSE_ENABLED and type(xk) is type(xr) is torch.Tensor and xk.shape == xr.shape and xk.dtype == xr.dtype and xk.numel() >= CHANNEL_MIX_TILES:
-        ws = _own_weights((ffn.key, ffn.receptance, ffn.value), xk)
-        if ws is not None:
+        C, wk = xk.shape[-1], ffn.key._parameters.get("weight")
+        ws = _own_weights((ffn.key, ffn.receptance, ffn.value), xk, (C, C, wk.shape[0] if wk is not None else 0))
+        if ws is not None and ws[1].shape[0] == ws[2].shape[0] == C:
             wk, wr, wv = ws
             if torch.is_grad_enabled() and any(t.requires_grad for t in (xk, xr, *ws)):
                 return _ChannelMix.apply(xk, xr, wk, wr, wv)

@@ -1000,14 +1000,17 @@ def weight_grad_group(gs, xs):
 EPI_RELU_SQ, EPI_RELU_SQ_BWD, EPI_ROUND = 1, 8, 16
 
 
-def linear_takes(x, weights):
+def linear_takes(x, weights, widths=None):
     """True where linear_group may stand in for x @ W^T on the GPU: 16-bit token matrices and weights of one type outside autocast and
     every kind of transform, sizes that the kernel of the large tiles takes (include/vrwkv_hip.h, csrc/linear_wide.hip) and that fill
-    the chip with them: 70 tiles of 128 x 128."""
+    the chip with them: 70 tiles of 128 x 128.  widths: what each weight's input has for columns, x's by default; a weight that does not fit
+    its input is left to the operators, which refuse it."""
     M, K = x.numel() // max(x.shape[-1], 1), x.shape[-1]
     if not (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and M > 0 and not torch.is_autocast_enabled("cuda") and not _transformed()):
         return False
-    for w in weights:
+    for w, width in zip(weights, widths if widths is not None else [K] * len(weights)):
+        if w.dim() != 2 or w.shape[1] != width:
+            return False
         N, k = w.shape
         if not (w.dtype == x.dtype and w.device == x.device and w.is_contiguous() and w.data_ptr() % 16 == 0
                 and (N % 192 == k % 192 == 0 or N % 128 == k % 128 == 0)):
@@ -1025,14 +1028,19 @@ def linear_group(problems):
     structs, results, keep = (_lib.Linear * n)(), [], []
     for s, p in zip(structs, problems):
         a, w = p["a"], p["w"]
+        if w.dim() != 2 or a.shape != (M, w.shape[1]) or any(t.dtype != dt or t.device != dev for t in (a, w)) or not w.is_contiguous():
+            raise RuntimeError(f"a {tuple(a.shape)} and a contiguous w {tuple(w.shape)} must be (M, K) and (N, K) of one dtype")
         a = a if a.stride(1) == 1 and a.stride(0) % 8 == 0 and a.stride(0) >= a.shape[1] and a.data_ptr() % 16 == 0 else a.clone(memory_format=torch.contiguous_format)
         keep.append(a)
         out = torch.empty((M, w.shape[0]), dtype=dt, device=dev)
         raw = torch.empty_like(out) if p.get("raw") else None
         s.a, s.w, s.out, s.N, s.K, s.lda, s.epi = a.data_ptr(), w.data_ptr(), out.data_ptr(), w.shape[0], w.shape[1], a.stride(0), p.get("epi", 0)
         for name in ("gate", "vec", "res"):
-            if p.get(name) is not None:
-                setattr(s, name, p[name].data_ptr())
+            t = p.get(name)
+            if t is not None:
+                if t.shape != (out.shape if name != "vec" else out.shape[1:]) or t.dtype != dt or t.device != dev or not t.is_contiguous():
+                    raise RuntimeError(f"{name} must be contiguous, of the result's dtype and shape (vec: its columns)")
+                setattr(s, name, t.data_ptr())
         if raw is not None:
             s.raw = raw.data_ptr()
         results.append(out if raw is None else (out, raw))
