@@ -1441,3 +1441,39 @@ def test_channel_mixes_whose_weights_do_not_fit_raise_as_the_operators_do(name, 
             ops.linear_group([dict(a=a, w=w)])
         with pytest.raises(RuntimeError, match="must be"):
             ops.linear_group([dict(a=a, w=lins[0].weight.detach(), gate=a[:, :192].contiguous())])
+
+
+def test_a_level_of_forward_mode_differentiation_is_a_transform():
+    from vision_rwkv_amd.ops import _transformed
+    assert not _transformed()
+    with torch.autograd.forward_ad.dual_level():
+        assert _transformed()
+    assert not _transformed()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("kind", ["v4", "v6"])
+def test_tangents_pass_through_frozen_blocks_up_to_the_operators_refusal(kind, grad):
+    """Forward-mode tangents with frozen weights, at a size of the grouped launches (384 channels, 3 x 4096 tokens): the projections' and a channel
+    mix's are those of tensor ops (bf16: some ten roundings of 2^-9 in the mix), the operators refuse as they do on their own."""
+    import torch.autograd.forward_ad as fw
+    from vision_rwkv_amd import backbone as bb
+    net = _small_backbone(kind, 384, torch.bfloat16, False, False, False, (64, 64))
+    net.requires_grad_(False)
+    block, hw = net.layers[1], (64, 64)
+    x, t = (torch.randn(3, 4096, 384, device="cuda").bfloat16() for _ in range(2))
+    lins = (block.att.key, block.att.value, block.att.receptance)
+    with torch.set_grad_enabled(grad), fw.dual_level():
+        dual = fw.make_dual(x, t)
+        for lin, y in zip(lins, bb._projs(lins, [dual] * 3)):
+            assert torch.equal(fw.unpack_dual(y).tangent, torch.nn.functional.linear(t, lin.weight))
+        got = fw.unpack_dual(block.ffn(dual, hw)).tangent
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            block.att(dual, hw)
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            block(dual, hw)
+    ffn = type(block.ffn)(**({} if kind == "v4" else dict(n_head=6)), n_embd=384, n_layer=2, layer_id=1, hidden_rate=4).double()
+    ffn.load_state_dict({n: p.double().cpu() for n, p in block.ffn.state_dict().items()})
+    _, want = torch.func.jvp(lambda z: ffn(z, hw), (x.double().cpu(),), (t.double().cpu(),))
+    assert (got.double().cpu() - want).norm() <= 3e-2 * want.norm()

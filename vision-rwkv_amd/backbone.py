@@ -16,7 +16,7 @@ import torch.nn.functional as F
 from torch.nn.modules import module as _hooks
 
 from . import ops
-from .ops import (RUN_CUDA, divided_takes, wkv_divided, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, weight_grad, weight_grad_group, linear_takes, linear_group, transposed, sigmoid_gate_backward, EPI_RELU_SQ, EPI_RELU_SQ_BWD, EPI_ROUND, block_takes, block_weights_fit, block_forward, _equal_quarters, _transformed, batched_cotangent, PRE_NONE, PRE_RELU_SQ, POST_NONE,
+from .ops import (RUN_CUDA, divided_takes, wkv_divided, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, weight_grad, weight_grad_group, linear_takes, linear_group, transposed, sigmoid_gate_backward, EPI_RELU_SQ, EPI_RELU_SQ_BWD, EPI_ROUND, block_takes, block_weights_fit, block_forward, _equal_quarters, _forward_mode, _transformed, batched_cotangent, PRE_NONE, PRE_RELU_SQ, POST_NONE,
                   POST_SIGMOID_GATE, POST_RESIDUAL)
 
 
@@ -73,7 +73,7 @@ def eval_cached(module, name, params, extra, make):
 def _mix(module, x, mixes, shift_pixel, gamma, patch_resolution, fused, head_dim=0, through=0):
     """[x*m + q_shift(x)*(1-m) for m in mixes], and x itself `through` times for its other uses (see _branch): one fused kernel
     (forward, and backward under autograd); tensor ops when `fused` is off or the tensors are not on the GPU."""
-    if fused and x.is_cuda:
+    if fused and x.is_cuda and not _forward_mode():
         if torch.is_grad_enabled() and (x.requires_grad or any(m.requires_grad for m in mixes)):
             return q_shift_mix_autograd(x, mixes, shift_pixel, gamma, patch_resolution, head_dim, through)
         table = eval_cached(module, "mix_table", mixes, x.device, lambda: stack_mixes(mixes, x.device))
@@ -517,7 +517,7 @@ class VRWKV_SpatialMix(nn.Module):
             xk = xv = xr = x
         k, v, r = _projs((self.key, self.value, self.receptance), (xk, xv, xr))
         wd = self.spatial_decay.dtype
-        if torch.is_grad_enabled() or k.dtype != (wd if wd in (torch.half, torch.bfloat16) else torch.float32):
+        if torch.is_grad_enabled() or _forward_mode() or k.dtype != (wd if wd in (torch.half, torch.bfloat16) else torch.float32):
             w, u = self.spatial_decay, self.spatial_first
             y = wkv_divided(w, u, T, k, v) if divided_takes(w, u, k, v) else RUN_CUDA(w / T, u / T, k, v)      # vrwkv.py:183
         else:

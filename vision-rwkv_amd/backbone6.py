@@ -11,7 +11,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .backbone import VRWKV, eval_cached, _proj, _projs, _channel_mix, _matmul, _bmm, _token_product, _as_built, _branch, _block_may_fuse, _block_weights
-from .ops import (HEAD_SIZE, RUN_CUDA_RWKV6, add_to_tokens, maa_lora_mix, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, maa_mix, groupnorm_gate, block_takes, block_weights_fit, block_forward, PRE_NONE, PRE_RELU_SQ, POST_NONE,
+from .ops import (HEAD_SIZE, RUN_CUDA_RWKV6, add_to_tokens, maa_lora_mix, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, maa_mix, groupnorm_gate, block_takes, block_weights_fit, block_forward, _forward_mode, PRE_NONE, PRE_RELU_SQ, POST_NONE,
                   POST_SIGMOID_GATE, POST_RESIDUAL)
 
 
@@ -31,7 +31,7 @@ def _shift_and_mix(module, x, mixes, shift_pixel, patch_resolution, with_cls_tok
     """[x*m + shift(x)*(1-m) for m in mixes()], and x itself `through` times for its other uses; one HIP kernel (forward, and backward under autograd), tensor ops when
     `fused` is off or off the GPU.  `mixes` is a callable (the vectors may be derived from `params`); at inference
     its stacked fp32 table is kept on the module."""
-    if fused and x.is_cuda:
+    if fused and x.is_cuda and not _forward_mode():
         if torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in params)):
             return q_shift_mix_autograd(x, mixes(), shift_pixel, 1 / 4, patch_resolution, HEAD_SIZE, through)
         table = eval_cached(module, "mix_table", params, x.device, lambda: stack_mixes(mixes(), x.device))

@@ -554,7 +554,7 @@ def row_fuse(a, other=None, ln_weight=None, ln_bias=None, gamma=None, pre=PRE_NO
     vec = 4 if a.dtype == torch.float32 else 8
     need_grad = torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
     sums = ln_weight is not None or (post == POST_RESIDUAL and gamma is not None)
-    fits = (ROW_FUSE_ENABLED and a.is_cuda and a.dtype in _DT and N % vec == 0 and N // vec <= 1024 and a.numel() > 0
+    fits = (ROW_FUSE_ENABLED and not _forward_mode() and a.is_cuda and a.dtype in _DT and N % vec == 0 and N // vec <= 1024 and a.numel() > 0
             and (other is None or (other.shape == a.shape and other.dtype == a.dtype))
             and not (need_grad and sums and N > 1024))
     if not fits:
@@ -631,7 +631,7 @@ def maa_mix(x, sx, m, maas, maa_table=None):
     vec = 4 if x.dtype == torch.float32 else 8
     tensors = [x, sx, m] + list(maas)
     need_grad = torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
-    fits = (ROW_FUSE_ENABLED and x.is_cuda and x.dtype in _DT and C % vec == 0 and x.numel() > 0
+    fits = (ROW_FUSE_ENABLED and not _forward_mode() and x.is_cuda and x.dtype in _DT and C % vec == 0 and x.numel() > 0
             and sx.shape == x.shape and sx.dtype == x.dtype and m.dtype == x.dtype and tuple(m.shape) == (5,) + tuple(x.shape)
             and not (need_grad and x.numel() // C > 65535 * 32))
     if not fits:
@@ -775,7 +775,7 @@ def groupnorm_gate(y, gate, gn_weight, gn_bias, n_groups, eps=1e-5):
     group = C // n_groups if n_groups > 0 and C % n_groups == 0 else 0
     tensors = [y, gate, gn_weight, gn_bias]
     need_grad = torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
-    fits = (ROW_FUSE_ENABLED and y.is_cuda and gate.dtype in (torch.float32, torch.bfloat16, torch.float16) and y.shape == gate.shape
+    fits = (ROW_FUSE_ENABLED and not _forward_mode() and y.is_cuda and gate.dtype in (torch.float32, torch.bfloat16, torch.float16) and y.shape == gate.shape
             and y.dtype in (torch.float32, gate.dtype) and group in (8, 16, 32, 64, 128) and y.numel() > 0
             and not (need_grad and C > 1024))
     if not fits:
@@ -905,11 +905,16 @@ def batched_cotangent(*tensors):
     return any(torch._C._functorch.is_legacy_batchedtensor(t) for t in tensors)
 
 
+def _forward_mode():
+    """True inside a level of forward-mode differentiation: a kernel's result has no tangent, whatever its arguments carry."""
+    return torch.autograd.forward_ad._current_level >= 0
+
+
 def _transformed():
-    """True inside torch.compile, jit tracing, a functorch transform or a dispatch / function mode, which are to see the
-    tensor ops."""
+    """True inside torch.compile, jit tracing, a functorch transform, a level of forward-mode differentiation or a dispatch /
+    function mode, which are to see the tensor ops."""
     return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0)
+            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0 or _forward_mode())
 
 
 def resize_table(table, src_shape, dst_shape):
