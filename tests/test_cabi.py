@@ -3,6 +3,8 @@ declares, and rejects bad arguments with a status and a message before touching 
 import ctypes
 import os
 import re
+import shutil
+import subprocess
 
 import pytest
 
@@ -243,3 +245,38 @@ def test_extension_module_stand_ins_and_torch_ops_namespaces():
     k = torch.randn(2, 8, 64)
     with pytest.raises(RuntimeError, match="CUDA tensor"):
         ops.ext.wkv.forward(2, 8, 64, torch.zeros(64), torch.zeros(64), k, k, torch.empty_like(k))
+
+
+PARAM_VEC = r"""
+#include "vrwkv_common.h"
+#include <cstdlib>
+#include <cstring>
+int main() {
+    for (int dtype : {VRWKV_F32, VRWKV_BF16, VRWKV_F16})
+        for (int C : {1, 2, 3, 5, 8, 65}) {
+            const int es = dtype == VRWKV_F32 ? 4 : 2;
+            char* p = (char*)malloc((size_t)C * es);                  // ends where the vector ends
+            for (int i = 0; i < C * es; ++i) p[i] = (char)(i + 1);
+            const vrwkv::ParamVec v(p, dtype, 1.f);
+            for (int c = 0; c < C; ++c) {
+                unsigned want = 0;
+                memcpy(&want, p + c * es, es);
+                if (v.fetch(c) != want) return 1;
+            }
+            free(p);
+        }
+    return 0;
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+def test_a_parameter_vector_is_read_element_by_element(tmp_path):
+    """vrwkv_biwkv_fwd_as / _bwd_as ask for w and u aligned to their elements and for nothing around them: the fetch, compiled for the host under
+    its address sanitizer, on vectors with nothing behind their last element."""
+    (tmp_path / "v.hip").write_text(PARAM_VEC)
+    csrc = os.path.join(ROOT, "vision-rwkv_amd", "csrc")
+    build = "hipcc -O1 -std=c++17 --offload-arch=gfx950 --cuda-host-only -w -Xarch_host -fsanitize=address"
+    subprocess.run([*build.split(), f"-I{csrc}", "-o", str(tmp_path / "v"), str(tmp_path / "v.hip")], check=True)
+    done = subprocess.run([str(tmp_path / "v")], capture_output=True, text=True)
+    assert done.returncode == 0, done.stderr[:2000]

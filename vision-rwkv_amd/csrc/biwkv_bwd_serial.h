@@ -36,7 +36,7 @@ void biwkv_bwd_serial_seq(const ParamVec w_, const ParamVec u_,
                           float* __restrict__ gw_part, float* __restrict__ gu_part, int B, int T, int C, int b, int c,
                           int rows_per_batch = 1)
 {
-    const float om = w_[c] * LOG2E, mu = u_[c] * LOG2E;
+    const float om = w_.value(w_.fetch(c)) * LOG2E, mu = u_.value(u_.fetch(c)) * LOG2E;
     const size_t base = (size_t)b * T * C + c;
     const size_t plane = (size_t)B * T * C;
     float* W0 = ws;                 // a      -> later z mantissa

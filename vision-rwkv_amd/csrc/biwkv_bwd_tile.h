@@ -147,8 +147,8 @@ void biwkv_bwd_tile_kernel(const ParamVec w_, const ParamVec u_,
         const int tw = (sc * S + wave) * L;
         const unsigned voff0 = cok ? (unsigned)(((size_t)tw * C + c0) * sizeof(IO)) : OOB_OFFSET;
         const size_t slab = (size_t)b * T * C;
-        const float om = (cok ? w_[c0] : 0.f) * LOG2E;
-        const float mu = (cok ? u_[c0] : 0.f) * LOG2E;
+        const unsigned wr = cok ? w_.fetch(c0) : 0u, ur = cok ? u_.fetch(c0) : 0u;      // 0 is 0 in every type
+        const float om = w_.value(wr) * LOG2E, mu = u_.value(ur) * LOG2E;
         const int next_tile = tile + gridDim.x;
         if (!bwd_tile_is_fast(om, mu, T)) {                   // workgroup-uniform: same channels in every wave
             if (STAGED && next_tile < n_tiles) {
@@ -498,8 +498,8 @@ void biwkv_bwd_tile_kernel(const ParamVec w_, const ParamVec u_,
         const int ctile = pair % n_ctile, b = pair / n_ctile;
         const int c0 = ctile * WAVE + lane;
         const bool cok = c0 < C;
-        const float om = (cok ? w_[c0] : 0.f) * LOG2E;
-        const float mu = (cok ? u_[c0] : 0.f) * LOG2E;
+        const unsigned wr = cok ? w_.fetch(c0) : 0u, ur = cok ? u_.fetch(c0) : 0u;      // 0 is 0 in every type
+        const float om = w_.value(wr) * LOG2E, mu = u_.value(ur) * LOG2E;
         if (bwd_tile_is_fast(om, mu, T)) continue;
         if (cok) biwkv_bwd_serial_seq<IO>(w_, u_, k_, v_, gy_, gk_, gv_, ws, gw_part, gu_part, B, T, C, b, c0, nSC);
     }

@@ -123,7 +123,7 @@ struct TileGeom {
 // previous tile is computed, and each wave then reads its own rows back lane-per-channel.
 // GATE: the emitted rows leave as sigmoid(r) * y (the receptance gate of vrwkv.py:186 applied before the store); r is
 // fetched lane-per-channel at the top of the tile, ahead of the next tile's rows, and waits packed in registers.
-template <typename IO, int VEC, int L, int MODE, bool STAGED = false, bool GATE = false>
+template <typename IO, int VEC, int L, int MODE, bool STAGED = false, bool GATE = false, typename PV = ParamVec>
 struct BiwkvTile {
     static_assert(!GATE || (VEC == 1 && MODE != 1), "the gate is applied where y is emitted, one channel per lane");
     static constexpr int SMAX = smax_for(L, VEC);
@@ -150,7 +150,7 @@ struct BiwkvTile {
     static constexpr int STAGE_ELEMS = 2 * LR * WAVE;                     // per wave: k rows, v rows
     static constexpr int YSTAGE_ELEMS = OUT_STAGED ? LR * WAVE : 8;       // per wave: y rows
 
-    ParamVec w_, u_;
+    PV w_, u_;
     const IO* __restrict__ k_;
     const IO* __restrict__ v_;
     const IO* __restrict__ r_;  // GATE: receptance (B,T,C)
@@ -326,12 +326,12 @@ struct BiwkvTile {
     // consumed) issues the loads of `next` into Kn, Vn when next < n_tiles.
     // True when any channel of the tile is outside the plain-sum regime (wave-uniform, and the
     // same for every wave and every super-chunk of a channel tile).
-    __device__ __forceinline__ bool tile_is_robust(const Where& q, const WU& wu, float (&om)[VEC], float (&mu)[VEC]) const {
+    __device__ __forceinline__ bool tile_is_robust(const WU& wu, float (&om)[VEC], float (&mu)[VEC]) const {
         bool bad = false;
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-            om[e] = w_.value(wu.w[e], q.c0 + e) * LOG2E;
-            mu[e] = u_.value(wu.u[e], q.c0 + e) * LOG2E;
+            om[e] = w_.value(wu.w[e]) * LOG2E;
+            mu[e] = u_.value(wu.u[e]) * LOG2E;
             bad = bad || outside_plain_sum(om[e], mu[e], T);
         }
         return __builtin_amdgcn_ballot_w64(bad) != 0ull;
@@ -357,7 +357,7 @@ struct BiwkvTile {
         VRWKV_STAMP(wave, round, 0);                      // tile entered
 
         float om[VEC], mu[VEC];
-        if (tile_is_robust(q, wu, om, mu)) {
+        if (tile_is_robust(wu, om, mu)) {
             // workgroup-uniform branch; the barrier stands in for the exchange barrier of a computed tile
             if (STAGED) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); else lds_barrier();
             if (next < g.n_tiles) {
@@ -665,7 +665,7 @@ struct BiwkvTile {
             wu.w[e] = q.cok ? w_.fetch(q.c0 + e) : 0u;      // 0 is 0 in every type
             wu.u[e] = q.cok ? u_.fetch(q.c0 + e) : 0u;
         }
-        if (!tile_is_robust(q, wu, om, mu)) return;
+        if (!tile_is_robust(wu, om, mu)) return;
 
         const unsigned row = (unsigned)(C * sizeof(IO));
         const __amdgpu_buffer_rsrc_t ry = make_rsrc(y_ + q.slab, (unsigned)((size_t)T * C * sizeof(IO)));
@@ -790,13 +790,13 @@ struct BiwkvTile {
 };
 
 
-template <typename IO, int VEC, int L, int MODE, bool STAGED = false, bool GATE = false>
+template <typename IO, int VEC, int L, int MODE, bool STAGED = false, bool GATE = false, typename PV = ParamVec>
 __global__ __launch_bounds__(smax_for(L, VEC) * WAVE)
-void biwkv_fwd_kernel(const ParamVec w_, const ParamVec u_,
+void biwkv_fwd_kernel(const PV w_, const PV u_,
                       const IO* __restrict__ k_, const IO* __restrict__ v_, IO* __restrict__ y_,
                       float* __restrict__ ws, int T, int C, TileGeom g, const IO* __restrict__ r_ = nullptr)
 {
-    using Tile = BiwkvTile<IO, VEC, L, MODE, STAGED, GATE>;
+    using Tile = BiwkvTile<IO, VEC, L, MODE, STAGED, GATE, PV>;
     __shared__ float s_agg[2][Tile::SMAX][NSLOT][Tile::CH];   // fast path: slot 2 carries the wave maxima
     __shared__ __attribute__((aligned(16))) IO s_stage[STAGED ? Tile::SMAX : 1][STAGED ? Tile::STAGE_ELEMS : 1];
     __shared__ __attribute__((aligned(16))) IO s_y[Tile::OUT_STAGED ? Tile::SMAX : 1][Tile::YSTAGE_ELEMS];
@@ -915,8 +915,8 @@ inline Plan make_plan(int B, int T, int C, int io_dtype) {
 constexpr int GATE_NOT_FUSED = -100;
 
 // r: null, or the receptance whose sigmoid gates y inside the emitting kernel.
-template <typename IO, int VEC, int L>
-int launch_L(const Plan& p, const ParamVec& w, const ParamVec& u, const void* k, const void* v, const void* r, void* y,
+template <typename IO, int VEC, int L, typename PV>
+int launch_L(const Plan& p, const PV& w, const PV& u, const void* k, const void* v, const void* r, void* y,
              float* ws, int B, int T, int C, hipStream_t st) {
     const dim3 block(p.S * WAVE);
     const dim3 grid(p.grid);
@@ -929,8 +929,8 @@ int launch_L(const Plan& p, const ParamVec& w, const ParamVec& u, const void* k,
         const bool aligned = C % (16 / (int)sizeof(IO)) == 0 && (((uintptr_t)k | (uintptr_t)v | (uintptr_t)y) & 15) == 0;
         if (aligned && !option(OPT_BIWKV_NO_STAGE)) {
             if (!p.multi()) {
-                if (rr) hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 0, true, true>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
-                else hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 0, true>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
+                if (rr) hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 0, true, true, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
+                else hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 0, true, false, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
             } else if (sizeof(IO) == 2 && L == 28 && p.nSC <= 3 && !option(OPT_BIWKV_NO_RESIDENT)) {
                 if (rr) return GATE_NOT_FUSED;
                 // two or three super-chunks of 16-bit rows fit a workgroup's registers: one launch, k and v read once
@@ -942,39 +942,44 @@ int launch_L(const Plan& p, const ParamVec& w, const ParamVec& u, const void* k,
                     const bool short_chunks = T <= p.nSC * 8 * 24;        // 24-token chunks need no spills with three super-chunks
                     const int RL = short_chunks ? 24 : 28;
                     const dim3 rblock(((T + p.nSC * RL - 1) / (p.nSC * RL)) * WAVE);
-#define VRWKV_RESIDENT(NSC_, L_) hipLaunchKernelGGL((biwkv_fwd_resident_kernel<IO, NSC_, L_>), rgrid, rblock, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom.n_ctile, n_seq)
-                    if (p.nSC == 2) { if (short_chunks) VRWKV_RESIDENT(2, 24); else VRWKV_RESIDENT(2, 28); }
-                    else            { if (short_chunks) VRWKV_RESIDENT(3, 24); else VRWKV_RESIDENT(3, 28); }
-#undef VRWKV_RESIDENT
+                    auto resident = [&](auto wp, auto up) {
+                        using R = decltype(wp);
+                        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, rgrid, rblock, 0, st, wp, up, kk, vv, yy, ws, T, C, p.geom.n_ctile, n_seq); };
+                        if (p.nSC == 2) { if (short_chunks) go(biwkv_fwd_resident_kernel<IO, 2, 24, R>); else go(biwkv_fwd_resident_kernel<IO, 2, 28, R>); }
+                        else            { if (short_chunks) go(biwkv_fwd_resident_kernel<IO, 3, 24, R>); else go(biwkv_fwd_resident_kernel<IO, 3, 28, R>); }
+                    };
+                    if (w.dtype == VRWKV_F32) resident(TypedVec<float>(w), TypedVec<float>(u));
+                    else if (w.dtype == type_code<IO>) resident(TypedVec<IO>(w), TypedVec<IO>(u));
+                    else resident(w, u);
                 }
             } else {
                 // fp32 rows: the emitting kernel of long sequences has no registers left for r (measured at 2 x 4150 x 768:
                 // 61 us with the gate inside against 50 us with the gate as a pass of its own); 16-bit rows: 32 against 37 us
                 if (rr && sizeof(IO) == 4) return GATE_NOT_FUSED;
-                hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 1, true>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
+                hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 1, true, false, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
                 if constexpr (sizeof(IO) == 2) {
                     if (rr) {
-                        hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 2, true, true>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
+                        hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 2, true, true, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
                         return check_launch("biwkv_fwd");
                     }
                 }
-                hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 2, true>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
+                hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 2, true, false, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
             }
             return check_launch("biwkv_fwd");
         }
     }
     if (rr) return GATE_NOT_FUSED;
     if (!p.multi()) {
-        hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 0>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
+        hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 0, false, false, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
     } else {
-        hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 1>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
-        hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 2>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
+        hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 1, false, false, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
+        hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 2, false, false, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
     }
     return check_launch("biwkv_fwd");
 }
 
-template <typename IO, int VEC>
-int launch_VEC(const Plan& p, const ParamVec& w, const ParamVec& u, const void* k, const void* v, const void* r, void* y,
+template <typename IO, int VEC, typename PV>
+int launch_VEC(const Plan& p, const PV& w, const PV& u, const void* k, const void* v, const void* r, void* y,
                float* ws, int B, int T, int C, hipStream_t st) {
     switch (p.L) {
 #define VRWKV_CASE(LL) case LL: return launch_L<IO, VEC, LL>(p, w, u, k, v, r, y, ws, B, T, C, st); break;
@@ -988,6 +993,9 @@ int launch_VEC(const Plan& p, const ParamVec& w, const ParamVec& u, const void* 
 template <typename IO>
 int biwkv_fwd_launch_io(const Plan& p, const ParamVec& w, const ParamVec& u, const void* k, const void* v, const void* r, void* y,
                         float* ws, int B, int T, int C, hipStream_t st) {
+    if constexpr (sizeof(IO) == 4) {
+        if (w.dtype == VRWKV_F32) return launch_VEC<IO, 1>(p, TypedVec<float>(w), TypedVec<float>(u), k, v, r, y, ws, B, T, C, st);
+    }
     return launch_VEC<IO, 1>(p, w, u, k, v, r, y, ws, B, T, C, st);
 }
 

@@ -108,8 +108,8 @@ __device__ __forceinline__ void agg_get(const float (*__restrict__ agg)[NSLOT][W
 
 // One sequence outside the plain-sum regime: the renormalising recurrence of BiwkvTile::run_robust, first the
 // aggregates of every super-chunk (into the workspace), then the outputs.
-template <typename IO, int NSC, int L>
-__device__ __forceinline__ void resident_robust(const ParamVec w_, const ParamVec u_, const IO* k_, const IO* v_, IO* y_,
+template <typename IO, int NSC, int L, typename PV>
+__device__ __forceinline__ void resident_robust(const PV w_, const PV u_, const IO* k_, const IO* v_, IO* y_,
                                                           float* ws, int T, int C, int n_ctile, int n_seq, int b, int ctile,
                                                           float (*agg0)[NSLOT][WAVE], float (*agg1)[NSLOT][WAVE]) {
     TileGeom g;
@@ -117,21 +117,21 @@ __device__ __forceinline__ void resident_robust(const ParamVec w_, const ParamVe
     const int lane = threadIdx.x & (WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int S = blockDim.x >> 6;
-    BiwkvTile<IO, 1, L, 1, false> t1;
+    BiwkvTile<IO, 1, L, 1, false, false, PV> t1;
     t1.w_ = w_; t1.u_ = u_; t1.k_ = k_; t1.v_ = v_; t1.y_ = y_; t1.ws = ws; t1.T = T; t1.C = C; t1.g = g;
     t1.lane = lane; t1.wave = wave; t1.S = S; t1.s_agg0 = agg0; t1.s_agg1 = agg1; t1.s_stage = nullptr; t1.s_y = nullptr; t1.s_fold = nullptr;
     for (int sc = 0; sc < NSC; ++sc) t1.run_robust((b * NSC + sc) * n_ctile + ctile);
     __threadfence();
     __syncthreads();
-    BiwkvTile<IO, 1, L, 2, false> t2;
+    BiwkvTile<IO, 1, L, 2, false, false, PV> t2;
     t2.w_ = w_; t2.u_ = u_; t2.k_ = k_; t2.v_ = v_; t2.y_ = y_; t2.ws = ws; t2.T = T; t2.C = C; t2.g = g;
     t2.lane = lane; t2.wave = wave; t2.S = S; t2.s_agg0 = agg0; t2.s_agg1 = agg1; t2.s_stage = nullptr; t2.s_y = nullptr; t2.s_fold = nullptr;
     for (int sc = 0; sc < NSC; ++sc) t2.run_robust((b * NSC + sc) * n_ctile + ctile);
 }
 
-template <typename IO, int NSC, int L>
+template <typename IO, int NSC, int L, typename PV>
 __global__ __launch_bounds__(8 * WAVE)
-void biwkv_fwd_resident_kernel(const ParamVec w_, const ParamVec u_,
+void biwkv_fwd_resident_kernel(const PV w_, const PV u_,
                                const IO* __restrict__ k_, const IO* __restrict__ v_, IO* __restrict__ y_,
                                float* __restrict__ ws, int T, int C, int n_ctile, int n_seq)
 {
@@ -198,14 +198,14 @@ void biwkv_fwd_resident_kernel(const ParamVec w_, const ParamVec u_,
         const int ctile = seq % n_ctile, b = seq / n_ctile;
         const int c0 = ctile * WAVE + lane;
         const bool cok = c0 < C;
-        const float wv = cok ? w_[c0] : 0.f, uv = cok ? u_[c0] : 0.f;
-        const float om = wv * LOG2E, mu = uv * LOG2E;
+        const unsigned wr = cok ? w_.fetch(c0) : 0u, ur = cok ? u_.fetch(c0) : 0u;      // 0 is 0 in every type
+        const float om = w_.value(wr) * LOG2E, mu = u_.value(ur) * LOG2E;
         const bool bad = outside_plain_sum(om, mu, T);
         if (__builtin_amdgcn_ballot_w64(bad) != 0ull) {
             // outside the plain-sum regime: the renormalising recurrence, super-chunk aggregates through the workspace
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // the rows already on their way must land first
             __syncthreads();
-            resident_robust<IO, NSC, L>(w_, u_, k_, v_, y_, ws, T, C, n_ctile, n_seq, b, ctile, s_agg, s_agg);
+            resident_robust<IO, NSC, L, PV>(w_, u_, k_, v_, y_, ws, T, C, n_ctile, n_seq, b, ctile, s_agg, s_agg);
 #pragma unroll
             for (int sc = 0; sc < NSC; ++sc, ++n)                         // what its super-chunks would have asked for
                 issue_rows(n + NREG - 1, STATIC_REG ? (sc + NREG - 1) % NREG : (n + NREG - 1) % NREG);
