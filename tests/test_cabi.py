@@ -247,6 +247,17 @@ def test_extension_module_stand_ins_and_torch_ops_namespaces():
         ops.ext.wkv.forward(2, 8, 64, torch.zeros(64), torch.zeros(64), k, k, torch.empty_like(k))
 
 
+@pytest.mark.parametrize("sequences,chunks", [(72, 9), (96, 10), (120, 10), (108, 11), (120, 13), (108, 14), (132, 19), (144, 24), (192, 130), (300, 130)])
+def test_wkv6_sequences_that_are_faster_whole_are_not_cut(lib, sequences, chunks):
+    """Shapes at which every count of segments measured slower than none, in any type (32-token chunks; 256 compute units): no workspace."""
+    assert lib.vrwkv_wkv6_fwd_workspace_bytes(1, 32 * chunks, 64 * sequences, sequences) == 0
+
+
+@pytest.mark.parametrize("sequences,chunks", [(1, 9), (3, 130), (12, 19), (48, 19), (36, 130), (84, 33), (96, 19)])
+def test_wkv6_few_long_sequences_are_cut(lib, sequences, chunks):
+    assert lib.vrwkv_wkv6_fwd_workspace_bytes(1, 32 * chunks, 64 * sequences, sequences) > 0
+
+
 PARAM_VEC = r"""
 #include "vrwkv_common.h"
 #include <cstdlib>

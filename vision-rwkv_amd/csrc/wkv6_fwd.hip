@@ -2,7 +2,6 @@
 #include "wkv6_fwd_scalar.h"
 #include "wkv6_fwd_chunk.h"
 #include <algorithm>
-#include <type_traits>
 #include <cstdlib>
 #include <cstring>
 
@@ -37,13 +36,13 @@ int validate(int B, int T, int C, int H, int rkv_dtype, int w_dtype) {
 }
 
 // Segments per sequence of a call (1: not split); OPT_WKV6_SEGMENTS forces a number (testing).
-int segments(int B, int T, int H, bool exact) {            // exact: bf16 values
+int segments(int B, int T, int H, int rkv_dtype) {
     const int nchunk = (T + LC - 1) / LC, forced = option(OPT_WKV6_SEGMENTS);
     if (forced > 0 && (long long)B * H <= SEG_SEQUENCES) {
         const int n = forced < nchunk ? forced : nchunk, cps = (nchunk + n - 1) / n;
         return (nchunk + cps - 1) / cps;
     }
-    return forced > 0 ? 1 : wkv6_segments((long long)B * H, nchunk, device_cus(), exact ? SEG_FWD : SEG_FWD_SPLIT);
+    return forced > 0 ? 1 : wkv6_fwd_segments((long long)B * H, nchunk, device_cus(), SEG_FWD[rkv_dtype]);
 }
 
 template <typename IO, typename WT>
@@ -75,7 +74,7 @@ int launch_chunked(const void* r, const void* k, const void* v, const void* w, c
     const IO* vv = static_cast<const IO*>(v);
     const WT* ww = static_cast<const WT*>(w);
     const long long sequences = (long long)B * H;
-    int nseg = segments(B, T, H, std::is_same<IO, __hip_bfloat16>::value);
+    int nseg = segments(B, T, H, type_code<IO>);
     // (the state kernel reads pairs of elements: 4-byte accesses of 16-bit rows; wider accesses need no more than 4 bytes either)
     if (!ws || ws_bytes < seg_bytes(sequences, nseg, SEG_FLOATS) || ((uintptr_t)ws & 15) || (((uintptr_t)k | (uintptr_t)v | (uintptr_t)w) & 3)) nseg = 1;
     float* states = nullptr;
@@ -141,8 +140,8 @@ extern "C" int vrwkv_wkv6_fwd_phases(const void* r, const void* k, const void* v
 extern "C" size_t vrwkv_wkv6_fwd_workspace_bytes(int B, int T, int C, int H) {
     (void)C;
     if (B <= 0 || T <= 0 || H <= 0) return 0;
-    // the same for every type: the larger of the two plans
-    return std::max(seg_bytes((long long)B * H, segments(B, T, H, true), SEG_FLOATS), seg_bytes((long long)B * H, segments(B, T, H, false), SEG_FLOATS));
+    // the same for every type: the largest of the plans
+    return seg_bytes((long long)B * H, std::max({segments(B, T, H, VRWKV_F32), segments(B, T, H, VRWKV_BF16), segments(B, T, H, VRWKV_F16)}), SEG_FLOATS);
 }
 
 extern "C" int vrwkv_wkv6_fwd(const void* r, const void* k, const void* v, const void* w, const float* u,

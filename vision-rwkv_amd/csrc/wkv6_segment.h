@@ -26,34 +26,56 @@ constexpr int SEG_STATE = HN * HN;                   // floats of one state
 constexpr int SEG_FLOATS = 2 * SEG_STATE + HN;       // forward: up state, down state, total decay per channel
 constexpr int BWD_SEG_FLOATS = 4 * SEG_STATE + HN;   // backward: S up, G up, S down, G down, total decay per channel
 
-// Segments of a sequence: the number with the least estimated time, where that is less than uncut by the margin below (a tenth, a fifth).  Sequences of up to
+// Segments of a sequence: the number with the least estimated time, where that is less than uncut by a margin.  Sequences of up to
 // 256 tokens stay whole, forward and backward: the results of a (b,h) then do not depend on how many others are in the call.
-// Those of longer sequences do, in their last bits (a caller that minds leaves the forward's workspace away).  Costs are microseconds measured on bf16 calls: a step (one chunk) of the main kernel while its CU holds one workgroup, and more per further workgroup that its CU has to run
-// (two at a time fit); the state kernel's step per workgroup on a CU; the extra launches; the scan by a sequence's segments, and the states' way out
-// of the state kernel, through the scan and into the main kernel (32 or 64 KB a segment, two to four times) by all of them, in thousands.
-struct SegCosts { double one, each, state, fixed, per_segment, per_thousand, margin; };
-// forward, by the main kernel's step: bf16 values go to the matrix cores as they are, fp16 and fp32 ones split in two.  Fitted to 3 to 192 sequences of
-// 10 to 130 chunks, each uncut and in 2 to 44 segments; the counts chosen are within 1 % (bf16) and 2 % (fp32) of the best ones on average.  bf16 / fp32, us:
-//   24 sequences of 130 chunks  uncut 356 / 370   10 segments 71 / 82   19 segments 67 / 87   33 segments 80
-//   48 of 19                    uncut 57 / 58      5 segments 33 / 35   10 segments 34 / 42
-//   96 of 19                    uncut 58 / 60      5 segments 47 / 58   12 of 19   10 segments 23 / 24   19 segments 27 / 31
-//   192 of 33                   uncut 105 / 120, best cut 113 / 130     144 of 10  uncut 35 / 35
-// (without the states' traffic in the estimate 48 sequences of 19 chunks went to 10 segments, 12 of them to 19, and 96 of them stayed uncut)
-constexpr SegCosts SEG_FWD = {3.45, 2.5, 0.55, 3.6, 0.3, 24.4, 0.9}, SEG_FWD_SPLIT = {2.75, 2.9, 1.57, 3.5, 0.32, 25.1, 0.9};
-// backward (both sweeps): at 24 sequences of 130 chunks uncut 1381, 10 segments 194, 21 163, 32 193; at 192 of 32 chunks
+// Those of longer sequences do, in their last bits (a caller that minds leaves the forward's workspace away).
+//
+// Backward (both sweeps), in microseconds measured on bf16 calls: a step (one chunk) of the main kernel while its CU holds one workgroup, and more per
+// further workgroup that its CU has to run (two at a time fit); the state kernel's step per workgroup on a CU; the scan and the extra launches.
+// At 24 sequences of 130 chunks uncut 1381, 10 segments 194, 21 163, 32 193; at 192 of 32 chunks
 // uncut 376, 4 segments 310; at 9 of 7 chunks uncut 78, 7 segments 42; at 192 of 7 chunks uncut 84, best cut 103
-constexpr SegCosts SEG_BWD = {11.5, 9.0, 1.5, 32.0, 0.1, 0.0, 0.8};
+struct SegCosts { double one, each, state, fixed, per_segment; };
+constexpr SegCosts SEG_BWD = {11.5, 9.0, 1.5, 32.0, 0.1};
 inline int wkv6_segments(long long sequences, int nchunk, int cus, const SegCosts& k) {
     auto time = [&](int nseg) {
         const int cps = (nchunk + nseg - 1) / nseg;
         const long long per_cu = (sequences * nseg + cus - 1) / cus;
         const double main = cps * (per_cu == 1 ? k.one : k.each * per_cu);
-        return nseg == 1 ? main : main + cps * k.state * per_cu + k.fixed + k.per_segment * nseg + k.per_thousand * 1e-3 * (double)(sequences * nseg);
+        return nseg == 1 ? main : main + cps * k.state * per_cu + k.fixed + k.per_segment * nseg;
     };
     int best = 1;
-    double best_time = k.margin * time(1);
+    double best_time = 0.8 * time(1);
     for (int nseg = 2; nchunk > 8 && nseg <= SEG_MAX && nseg <= nchunk && sequences * nseg <= 4LL * cus; ++nseg) {
         const double t = time(nseg);
+        if (t < best_time) { best = nseg; best_time = t; }
+    }
+    const int cps = (nchunk + best - 1) / best;
+    return (nchunk + cps - 1) / cps;                 // every segment non-empty
+}
+
+// Forward: the estimate follows the launches as they are.  The grid has a multiple of eight workgroups per segment number (seg_grid), and a compute
+// unit runs one to four of them: `step` is a chunk in the main and the state kernel together for each of those counts; `traffic` is the states' way out
+// of the state kernel, through the scan and into the main kernel by the thousand segments, `token_traffic` the rows' by the thousand chunks; `fixed` the
+// extra launches.  In microseconds, fitted for each type of r, k, v to 1 to 252 sequences of 9 to 130 chunks, uncut and in 2 to 64 segments: 19 000 times, the
+// estimate 4.5 % off (standard deviation).  Counts chosen against the best of the sweep: 0.2 % behind on average, 4 (fp32 7) at most.  On 3 200 further shapes
+// they are 10 % ahead on average of what the backward's estimate would choose, and at most 6 % behind that or uncut.  us, uncut | segments:
+//   bf16   24 sequences of 130 chunks 354 | 8 84, 10 69, 12 84, 19 64          fp32   36 of 130  364 | 6 113, 7 162, 10 127
+//          96 of 10                    32 | 2 36, 3 43, 4 38, 5 33                    48 of 24    71 | 6 52, 8 47, 12 56
+//         132 of 12                    38 | 2 54, 3 45                                84 of 24    72 | 2 68, 3 84, 5 65
+//          84 of 33                    93 | 2 83, 3 84, 5 64                         120 of 33    98 | 2 95, 4 99
+struct FwdSegCosts { double uncut, uncut_fixed, uncut_traffic, step[4], fixed, per_segment, traffic, token_traffic; };
+constexpr FwdSegCosts SEG_FWD[3] = {{2.72, 4.0, 2.23, {3.73, 7.06, 11.09, 14.80}, 9.8, 0.14, 28.5, 3.39},       // VRWKV_F32
+                                    {2.65, 5.1, 1.09, {3.53, 5.14, 8.16, 10.48}, 10.8, 0.14, 20.3, 3.44},       // VRWKV_BF16
+                                    {2.80, 4.9, 1.33, {3.99, 7.28, 10.68, 14.05}, 9.6, 0.14, 29.9, 1.70}};      // VRWKV_F16
+inline int wkv6_fwd_segments(long long sequences, int nchunk, int cus, const FwdSegCosts& k) {
+    const long long padded = (sequences + 7) / 8 * 8;
+    if (nchunk <= 8 || padded > cus) return 1;       // more sequences than compute units: a cut only adds work
+    int best = 1;
+    const double chunks = 1e-3 * (double)nchunk * (double)sequences;
+    double best_time = 0.95 * (nchunk * k.uncut + k.uncut_fixed + k.uncut_traffic * chunks);
+    for (int nseg = 2; nseg <= SEG_MAX && nseg <= nchunk && padded * nseg <= 4LL * cus; ++nseg) {
+        const int cps = (nchunk + nseg - 1) / nseg, per_cu = (int)((padded * nseg + cus - 1) / cus);
+        const double t = cps * k.step[per_cu - 1] + k.fixed + k.per_segment * nseg + k.traffic * 1e-3 * (double)(sequences * nseg) + k.token_traffic * chunks;
         if (t < best_time) { best = nseg; best_time = t; }
     }
     const int cps = (nchunk + best - 1) / best;
