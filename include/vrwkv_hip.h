@@ -94,7 +94,8 @@ int vrwkv_biwkv_fwd_static(const float* w, const float* u, const void* k, const 
  *   backward(B,T,C,w,u,k,v,gy,gw,gu,gk,gv) (.../backbones/cuda/wkv_op.cpp:9-11).
  * w, u, gw, gu: (C,) fp32, gw and gu already summed over batch and tokens (fully overwritten,
  * no need to zero them); k, v, gy, gk, gv: (B,T,C) of io_dtype.  The workspace (always needed)
- * replaces the three scratch tensors the reference allocates (bi_wkv_kernel.cu:415-417). */
+ * replaces the three scratch tensors the reference allocates (bi_wkv_kernel.cu:415-417).  A sample's gk and gv do not depend on the
+ * others in the call, but for the last bits of fp32 ones of more than 224 tokens. */
 size_t vrwkv_biwkv_bwd_workspace_bytes(int B, int T, int C, int io_dtype);
 int vrwkv_biwkv_bwd(const float* w, const float* u, const void* k, const void* v, const void* gy,
                     float* gw, float* gu, void* gk, void* gv, int B, int T, int C, int io_dtype,

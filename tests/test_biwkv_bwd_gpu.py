@@ -196,7 +196,10 @@ def test_parameter_gradients_of_the_inputs_type_are_the_rounded_fp32_sums(B, T, 
     assert all(torch.equal(a.to(dtype), b) for a, b in zip(full, like))
 
 
-@pytest.mark.parametrize("B,T,C", [(1, 225, 64), (2, 577, 384), (1, 1025, 192), (8, 577, 384), (1, 1793, 70), (2, 4150, 64), (20, 300, 128), (3, 640, 1024)])
+SUPER_CHUNK_SHAPES = [(1, 225, 64), (2, 577, 384), (1, 1025, 192), (8, 577, 384), (1, 1793, 70), (2, 4150, 64), (20, 300, 128), (3, 640, 1024)]
+
+
+@pytest.mark.parametrize("B,T,C", SUPER_CHUNK_SHAPES)
 @pytest.mark.parametrize("tokens", [0, 16, 25, 28])
 def test_super_chunks_of_every_length(ops, B, T, C, tokens):
     """Long sequences by 16, 25 and 28 tokens a wave, and by the plan, against the C oracle (the fp32 bounds of the other tests here)."""
@@ -209,3 +212,39 @@ def test_super_chunks_of_every_length(ops, B, T, C, tokens):
         got = run(ops, w, u, k, v, gy)[:4]
     for a, r, bound in zip(got, clib.biwkv_bwd(w, u, k, v, gy), (2e-4, 1e-4, 1e-4, 1e-4)):
         assert rel_err(a, r) <= bound
+
+
+@pytest.mark.parametrize("B,T,C", SUPER_CHUNK_SHAPES)
+@pytest.mark.parametrize("tokens", [0, 16, 25, 28])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_super_chunks_of_every_length_in_16_bits(ops, B, T, C, tokens, dtype):
+    """The same with 16-bit rows, on the values they hold: the fp32 bounds above; gk and gv are rounded to the rows' type on the way out: with 8
+    and 11 bits of significand by up to 2^-8 and 2^-11 of the value."""
+    from oracle import clib
+    g = torch.Generator().manual_seed(T + C)
+    k, v, gy = (torch.randn(B, T, C, generator=g).to(dtype) for _ in range(3))
+    w, u = (torch.rand(C, generator=g) * 8 - 5) / T, torch.rand(C, generator=g) * 2 - 1
+    with ops.option("biwkv_l", tokens):
+        got = ops.bi_wkv_backward(*(t.cuda() for t in (w, u, k, v, gy)))
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    want = clib.biwkv_bwd(*(t.float().numpy() for t in (w, u, k, v, gy)))
+    for a, r, bound in zip(got, want, (2e-4, 1e-4, 1e-4 + unit, 1e-4 + unit)):
+        assert rel_err(a.float().cpu().numpy(), r) <= bound
+
+
+@pytest.mark.parametrize("T", [225, 256, 257, 400, 401, 577, 1025, 2048])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_a_samples_gradients_in_16_bits_do_not_depend_on_the_batch(ops, T, dtype):
+    """gk and gv of a sample alone and among others (few and many tiles for the compute units), bit for bit."""
+    C, B = 768, 33
+    g = torch.Generator(device="cuda").manual_seed(T)
+    k, v, gy = (torch.randn(B, T, C, generator=g, device="cuda").to(dtype) for _ in range(3))
+    w, u = ((torch.rand(C, generator=g, device="cuda") * 8 - 5) / T).to(dtype), torch.zeros(C, device="cuda", dtype=dtype)
+
+    def grads(n, at):
+        xs = [t[at:at + n].clone().requires_grad_() for t in (k, v)]
+        return torch.autograd.grad(ops.RUN_CUDA(w, u, *xs), xs, gy[at:at + n].contiguous())
+
+    whole = grads(B, 0)
+    for n, at in ((1, 32), (4, 8), (12, 20)):
+        assert all(torch.equal(a, b[at:at + n]) for a, b in zip(grads(n, at), whole))

@@ -61,21 +61,29 @@ struct BwdPlan {
     size_t planes = 0, agg1 = 0, agg2 = 0, parts = 0, total = 0;
 };
 
-// Tokens per wave of a sequence cut into super-chunks of eight waves.  The tiles (sequence, super-chunk, 64 channels) go to as many workgroups
-// as there are compute units, in rounds: the length with the shortest rounds together, a round being its tokens and a share that does not depend
-// on them (25 fits the sweep below).  Beyond eight rounds 28, the fewest tiles.  28 / 25 / 16 tokens a wave, us:
-//   fp32  2 x 4150 x 768 (456 / 504 / 792 tiles)   86.5 / 85.0 / 135.2     8 x 1025 x 768 (480 / 576 / 864)     74.1 / 93.6 / 100.8
-//         16 x 577 x 384 (288 / 288 / 480)         63.8 / 61.8 / 52.4      24 x 577 x 1024 (1152 / 1152 / 1920)  159.7 / 155.8 / 184.6
-//         1 x 1025 x 192 (15 / 18 / 27)            30.0 / 29.2 / 26.0      4 x 4150 x 768 (912 / 1008 / 1584)    160.5 / 163.4 / 231.2
-//   bf16  24 x 577 x 1024 138.5 / 128.6 / 159.6    16 x 577 x 384 56.5 / 52.9 / 46.7    32 x 300 x 768 (768 / 768 / 1152) 81.5 / 77.6 / 96.9
-// The forward keeps 28: its 16-bit kernels read sequences of two or three super-chunks of that length once, and a 16-bit network amplifies the last bits
-// that the cut decides (fp32 gains 3 % at 2 x 4150 x 768).
-int super_chunk_tokens(int B, int T, int C) {
+// Tokens per wave of a sequence cut into super-chunks of eight waves.
+//
+// 16-bit rows: by the length of the sequence alone, since the cut decides the last bits of gk and gv, which a 16-bit network amplifies: a sample's are the
+// same whatever else is in the call.  The shortest of 28, 25 and 16 that makes no more super-chunks than 28: as many tiles, each of them shorter.
+// 28 / 25 / 16 tokens a wave, us in bf16 (fp16 alike):
+//   T = 256   4 x 768 31.9 / 30.7 / 25.7     64 x 768 152 / 142 / 118      T = 577   4 x 768 33.0 / 31.1 / 28.2     64 x 768 237 / 222 / 287
+//   T = 400   4 x 768 31.7 / 30.1 / 26.9     64 x 768 162 / 155 / 225      T = 1025  4 x 768 34.5 / 56.2 / 50.0     64 x 768 389 / 434 / 533
+//
+// fp32 rows: the tiles (sequence, super-chunk, 64 channels) go to as many workgroups as there are compute units, in rounds: the length with the shortest
+// rounds together, a round being its tokens and a share that does not depend on them (25 fits the sweep below).  Beyond eight rounds 28, the fewest tiles.
+// A sample's last bits then depend on how many others are in the call.  28 / 25 / 16 tokens a wave, us:
+//   2 x 4150 x 768 (456 / 504 / 792 tiles)   86.5 / 85.0 / 135.2     8 x 1025 x 768 (480 / 576 / 864)      74.1 / 93.6 / 100.8
+//   16 x 577 x 384 (288 / 288 / 480)         63.8 / 61.8 / 52.4      24 x 577 x 1024 (1152 / 1152 / 1920)  159.7 / 155.8 / 184.6
+//   1 x 1025 x 192 (15 / 18 / 27)            30.0 / 29.2 / 26.0      4 x 4150 x 768 (912 / 1008 / 1584)    160.5 / 163.4 / 231.2
+// The forward keeps 28: its 16-bit kernels read sequences of two or three super-chunks of that length once (fp32 gains 3 % at 2 x 4150 x 768).
+int super_chunk_tokens(int B, int T, int C, int io_dtype) {
+    auto super_chunks = [&](int L) { return (T + BWD_SMAX * L - 1) / (BWD_SMAX * L); };
+    if (io_dtype != VRWKV_F32) return super_chunks(16) == super_chunks(28) ? 16 : super_chunks(25) == super_chunks(28) ? 25 : 28;
     const long long columns = (long long)B * ((C + WAVE - 1) / WAVE), cus = biwkv_fwd_detail::num_cus();
     int best = 28;
     long long least = -1;
     for (int L : {28, 25, 16}) {
-        const long long tiles = columns * ((T + BWD_SMAX * L - 1) / (BWD_SMAX * L)), rounds = (tiles + cus - 1) / cus;
+        const long long tiles = columns * super_chunks(L), rounds = (tiles + cus - 1) / cus;
         if (L != 28 && rounds > 8) continue;
         const long long cost = rounds * (L + 25);
         if (least < 0 || cost < least) { best = L; least = cost; }
@@ -83,7 +91,7 @@ int super_chunk_tokens(int B, int T, int C) {
     return best;
 }
 
-BwdPlan make_bwd_plan(int B, int T, int C) {
+BwdPlan make_bwd_plan(int B, int T, int C, int io_dtype) {
     BwdPlan p;
     static const int kL[] = {4, 8, 16, 25, 28};
     const int el = option(OPT_BIWKV_L);                      // tuning override: tokens per wave
@@ -94,7 +102,7 @@ BwdPlan make_bwd_plan(int B, int T, int C) {
         if (p.L) {
             p.S = (T + p.L - 1) / p.L;
         } else {
-            p.L = el == 28 || el == 25 || el == 16 ? el : super_chunk_tokens(B, T, C);
+            p.L = el == 28 || el == 25 || el == 16 ? el : super_chunk_tokens(B, T, C, io_dtype);
             p.S = BWD_SMAX;
             p.nSC = (T + p.S * p.L - 1) / (p.S * p.L);
         }
@@ -142,7 +150,7 @@ void launch_tiled(const BwdPlan& p, const ParamVec& w, const ParamVec& u, const 
 template <typename IO>
 int launch(const ParamVec& w, const ParamVec& u, const void* k, const void* v, const void* gy, SumOut gw, SumOut gu,
            void* gk, void* gv, float* ws, int B, int T, int C, hipStream_t st) {
-    const BwdPlan p = make_bwd_plan(B, T, C);
+    const BwdPlan p = make_bwd_plan(B, T, C, type_code<IO>);
     float* agg1 = ws + p.planes;
     float* agg2 = agg1 + p.agg1;
     float* gw_part = agg2 + p.agg2;
@@ -173,7 +181,7 @@ using namespace vrwkv;
 
 extern "C" size_t vrwkv_biwkv_bwd_workspace_bytes(int B, int T, int C, int io_dtype) {
     if (validate(B, T, C, io_dtype) != VRWKV_OK) return 0;
-    return make_bwd_plan(B, T, C).total * sizeof(float);
+    return make_bwd_plan(B, T, C, io_dtype).total * sizeof(float);
 }
 
 static int biwkv_bwd(const ParamVec& w, const ParamVec& u, const void* k, const void* v, const void* gy,
@@ -186,7 +194,7 @@ static int biwkv_bwd(const ParamVec& w, const ParamVec& u, const void* k, const 
         set_error("biwkv_bwd: null pointer argument");
         return VRWKV_INVALID_ARG;
     }
-    const size_t need = make_bwd_plan(B, T, C).total * sizeof(float);
+    const size_t need = make_bwd_plan(B, T, C, io_dtype).total * sizeof(float);
     if (!workspace || workspace_bytes < need) {
         set_error("biwkv_bwd: workspace of %zu bytes required (got %zu)", need, workspace ? workspace_bytes : (size_t)0);
         return VRWKV_WORKSPACE_TOO_SMALL;

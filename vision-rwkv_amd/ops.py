@@ -93,7 +93,8 @@ def bi_wkv_backward(w, u, k, v, gy, out=None, like_inputs=False):
     """Extension-level entry (bi_wkv.cpp:35-47): w,u (C,) fp32; k,v,gy (B,T,C) of one dtype;
     returns [gw, gu, gk, gv] with gw, gu (C,) fp32 summed over batch and tokens and gk, gv of the
     dtype of k.  out: caller-allocated (gw, gu, gk, gv).  like_inputs: gw, gu of the dtype of k as well, rounded from the
-    fp32 sums by the kernel."""
+    fp32 sums by the kernel.  A sample's gk and gv are the same whatever else is in the call, but for the last bits of fp32 ones of more than
+    224 tokens: how those are cut goes by the number of samples and channels too."""
     for t, n in ((w, "w"), (u, "u"), (k, "k"), (v, "v"), (gy, "gy")):
         _check_input(t, n)
     if k.dim() != 3 or v.shape != k.shape or gy.shape != k.shape:
