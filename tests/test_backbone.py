@@ -1,4 +1,6 @@
 """q_shift, the fused shift+mix kernel and the plain-PyTorch backbone."""
+import contextlib
+
 import numpy as np
 import pytest
 import torch
@@ -1477,3 +1479,35 @@ def test_tangents_pass_through_frozen_blocks_up_to_the_operators_refusal(kind, g
     ffn.load_state_dict({n: p.double().cpu() for n, p in block.ffn.state_dict().items()})
     _, want = torch.func.jvp(lambda z: ffn(z, hw), (x.double().cpu(),), (t.double().cpu(),))
     assert (got.double().cpu() - want).norm() <= 3e-2 * want.norm()
+
+
+def _other_strides(t):
+    return t.transpose(0, -1).contiguous().transpose(0, -1)
+
+
+def _other_place(t):
+    return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,C,hw,batch", [("v4", 384, (64, 64), 3), ("v6", 384, (64, 64), 3), ("v4", 192, (14, 14), 2), ("v6", 192, (14, 14), 2)])
+@pytest.mark.parametrize("unpack", [_other_strides, _other_place])
+@pytest.mark.parametrize("key_norm", [False, True])
+def test_saved_tensors_may_come_back_with_other_strides(kind, C, hw, batch, unpack, key_norm):
+    """Hooks on saved tensors promise the values, not the strides or the place: the gradients are those without hooks (12288 tokens
+    of 384 channels: the sizes of the grouped launches).  Not bit for bit: the library's products take other kernels for operands that lie otherwise, so
+    their results move by a rounding to bf16, 2^-9 of the value on average, some ten of which follow one another in a block: 3e-2.
+    (Tensors of one column come back as they were: torch's LayerNorm reads its own statistics as dense.)"""
+    net = _small_backbone(kind, C, torch.bfloat16, key_norm, True, False, hw)
+    x = torch.randn(batch, hw[0] * hw[1], C, device="cuda").bfloat16()
+    g = torch.randn_like(x)
+
+    def grads(hooks):
+        xs = x.clone().requires_grad_()
+        with hooks:
+            y = net.layers[1](xs, hw)
+        return torch.autograd.grad(y, [xs, *net.layers[1].parameters()], g)
+
+    want = grads(contextlib.nullcontext())
+    got = grads(torch.autograd.graph.saved_tensors_hooks(lambda t: t.detach(), lambda t: unpack(t) if t.dim() and t.shape[-1] > 1 else t))
+    assert all((a - b).norm() <= 3e-2 * b.norm() for a, b in zip(got, want))

@@ -16,7 +16,7 @@ import torch.nn.functional as F
 from torch.nn.modules import module as _hooks
 
 from . import ops
-from .ops import (RUN_CUDA, divided_takes, wkv_divided, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, weight_grad, weight_grad_group, linear_takes, linear_group, transposed, sigmoid_gate_backward, EPI_RELU_SQ, EPI_RELU_SQ_BWD, EPI_ROUND, block_takes, block_weights_fit, block_forward, _equal_quarters, _forward_mode, _transformed, batched_cotangent, PRE_NONE, PRE_RELU_SQ, POST_NONE,
+from .ops import (RUN_CUDA, divided_takes, wkv_divided, bi_wkv_forward, q_shift, q_shift_mix, q_shift_mix_autograd, stack_mixes, row_fuse, resize_table, weight_grad, weight_grad_group, linear_takes, linear_group, transposed, sigmoid_gate_backward, EPI_RELU_SQ, EPI_RELU_SQ_BWD, EPI_ROUND, block_takes, block_weights_fit, block_forward, _dense, _equal_quarters, _forward_mode, _transformed, batched_cotangent, PRE_NONE, PRE_RELU_SQ, POST_NONE,
                   POST_SIGMOID_GATE, POST_RESIDUAL)
 
 
@@ -244,7 +244,7 @@ class _Projections(torch.autograd.Function):
         gx, gw = [None] * n, [None] * n
         need = [i for i in range(n) if ctx.needs_input_grad[i]]
         if _plain_backward(*gs) and len(need) > 1:
-            outs = linear_group([dict(a=_rows(gs[i]), w=wt) for i, wt in zip(need, transposed([ws[i] for i in need]))])
+            outs = linear_group([dict(a=_rows(gs[i]), w=wt) for i, wt in zip(need, transposed([_dense(ws[i]) for i in need]))])
             for i, o in zip(need, outs):
                 gx[i] = o.reshape(xs[i].shape)
         else:
@@ -278,6 +278,7 @@ class _ChannelMix(torch.autograd.Function):
             g2 = g2.to(y.dtype).contiguous()
             plain = g2.data_ptr() % 16 == 0
         if plain:
+            wk, wr, wv, k, r, y = (_dense(t) for t in (wk, wr, wv, k, r, y))
             gy, gr = sigmoid_gate_backward(y, r, g2)
             wkt, wrt, wvt = transposed([wk, wr, wv])
             gk = linear_group([dict(a=gy, w=wvt, gate=k, epi=EPI_RELU_SQ_BWD | EPI_ROUND)])[0]

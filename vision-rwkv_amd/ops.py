@@ -197,7 +197,7 @@ class WKV(torch.autograd.Function):
         wf, uf, k, v = ctx.saved_tensors
         out_dtype = ctx.out_dtype
         if ctx.as_held:
-            return _wkv_backward(wf, uf, k.contiguous(), v.contiguous(), gy.to(out_dtype).contiguous())
+            return _wkv_backward(wf.contiguous(), uf.contiguous(), k.contiguous(), v.contiguous(), gy.to(out_dtype).contiguous())
         if k.dtype == out_dtype and v.dtype == out_dtype and out_dtype != torch.float32:
             return tuple(bi_wkv_backward(wf, uf, k.contiguous(), v.contiguous(), gy.to(out_dtype).contiguous(), like_inputs=True))
         gw, gu, gk, gv = bi_wkv_backward(wf, uf, k.float().contiguous(), v.float().contiguous(), gy.float().contiguous())
@@ -219,7 +219,7 @@ class _WKVDivided(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gy):
-        w, u, k, v = ctx.saved_tensors
+        w, u, k, v = _saved(ctx)
         gw, gu, gk, gv = _wkv_backward(w, u, k, v, gy.to(k.dtype).contiguous(), ctx.factor)
         return gw, gu, None, gk, gv
 
@@ -482,6 +482,16 @@ def _vec_ok(*tensors):
     return all(t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0) for t in tensors)
 
 
+def _dense(t):
+    """t as the kernels read it, dense and on 16 bytes."""
+    return t if _vec_ok(t) else t.clone(memory_format=torch.contiguous_format)
+
+
+def _saved(ctx):
+    """The saved tensors as the kernels read them: a hook on saved tensors may hand back other strides or a piece of a larger tensor."""
+    return tuple(_dense(t) for t in ctx.saved_tensors)
+
+
 def row_fuse_tensor_ops(a, other=None, ln_weight=None, ln_bias=None, gamma=None, pre=PRE_NONE, post=POST_NONE, eps=1e-5):
     """The PyTorch-op sequence row_fuse replaces (what the reference runs: vrwkv.py:184-186, :256-261, :300-313);
     used under autograd and wherever the kernel does not apply."""
@@ -507,7 +517,7 @@ class _RowFuse(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gout):
-        a, other, ln_weight, ln_bias, gamma = ctx.saved_tensors
+        a, other, ln_weight, ln_bias, gamma = _saved(ctx)
         pre, post, eps = ctx.meta
         N = a.shape[-1]
         rows = a.numel() // N
@@ -597,7 +607,7 @@ class _MaaMix(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, *gouts):
-        x, sx, m, table = ctx.saved_tensors
+        x, sx, m, table = _saved(ctx)
         C = x.shape[-1]
         rows = x.numel() // C
         gs = [g.to(x.dtype).contiguous() for g in gouts]
@@ -664,7 +674,7 @@ class _MaaLoraMix(torch.autograd.Function):
         x, sx, lo, w2, table = ctx.saved_tensors
         C = x.shape[-1]
         rows = x.numel() // C
-        stack = lo.view(rows, 5, -1).transpose(0, 1)
+        stack = lo.reshape(rows, 5, -1).transpose(0, 1)
         gs = [g.to(x.dtype) for g in gouts]
         if torch.is_grad_enabled() or batched_cotangent(*gs) or _transformed():
             f = [t + m.view(x.shape) for t, m in zip(table.to(x.dtype), torch.bmm(stack, w2))]
@@ -672,7 +682,7 @@ class _MaaLoraMix(torch.autograd.Function):
             gm = torch.stack([(g * (sx - x)).reshape(rows, C) for g in gs])
             gtable = gm.float().sum(1)
         else:
-            gs = [g.contiguous() for g in gs]
+            x, sx, lo, w2, table, *gs = (_dense(t) for t in (x, sx, lo, w2, table, *gs))
             gx, gsx, gtable = torch.empty_like(x), torch.empty_like(x), torch.empty_like(table)
             gm = torch.empty((5, rows, C), dtype=x.dtype, device=x.device)
             L = _lib.lib()
@@ -741,7 +751,7 @@ class _GroupNormGate(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gout):
-        y, gate, w, b = ctx.saved_tensors
+        y, gate, w, b = _saved(ctx)
         group, eps = ctx.meta
         C = y.shape[-1]
         rows = y.numel() // C
@@ -812,7 +822,7 @@ class _QShiftMix(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, *gouts):
-        x, table = ctx.saved_tensors
+        x, table = _saved(ctx)
         shift_pixel, gamma, Hp, Wp, head_dim = ctx.meta
         B, T, C = x.shape
         n_mix = table.shape[0]
