@@ -1511,3 +1511,19 @@ def test_saved_tensors_may_come_back_with_other_strides(kind, C, hw, batch, unpa
     want = grads(contextlib.nullcontext())
     got = grads(torch.autograd.graph.saved_tensors_hooks(lambda t: t.detach(), lambda t: unpack(t) if t.dim() and t.shape[-1] > 1 else t))
     assert all((a - b).norm() <= 3e-2 * b.norm() for a, b in zip(got, want))
+
+
+def test_batched_products_take_dense_right_operands(monkeypatch):
+    """The batched products of the low-rank maps' gradients are given no transposed views on the right, which the library's 16-bit ones are not to be
+    trusted with on this target."""
+    from types import SimpleNamespace
+    from vision_rwkv_amd import backbone as bb, ops
+    seen, bmm = [], torch.bmm
+    monkeypatch.setattr(torch, "bmm", lambda a, b: seen.append(b.is_contiguous()) or bmm(a, b))
+    x, w = torch.randn(5, 24, 32, requires_grad=True), torch.randn(5, 32, 64)
+    torch.autograd.grad(bb._SplitKBmm.apply(x, w, 8).sum(), x)
+    B, T, C = 2, 3, 64
+    saved = torch.randn(B, T, C), torch.randn(B, T, C), torch.randn(B * T, 160), torch.randn(5, 32, C), torch.randn(5, C)
+    ctx = SimpleNamespace(saved_tensors=saved, needs_input_grad=[True] * 5, token_product=lambda a, b: a.transpose(1, 2) @ b)
+    gx, gsx, glo, gw2, gtable, _ = ops._MaaLoraMix.backward(ctx, *torch.randn(5, B, T, C))
+    assert glo.shape == (B * T, 160) and len(seen) == 4 and all(seen)

@@ -162,7 +162,7 @@ class _SplitKBmm(torch.autograd.Function):
     def backward(ctx, g):
         x, weight = ctx.saved_tensors
         S = ctx.splits
-        gx = torch.bmm(g, weight.transpose(1, 2)) if ctx.needs_input_grad[0] else None
+        gx = torch.bmm(g, weight.transpose(1, 2).contiguous()) if ctx.needs_input_grad[0] else None
         gw = None
         if ctx.needs_input_grad[1]:
             gw = _token_product(x, g, S)

@@ -693,7 +693,7 @@ class _MaaLoraMix(torch.autograd.Function):
                                                     (ctypes.c_void_p * 5)(*[g.data_ptr() for g in gs]), gx.data_ptr(), gsx.data_ptr(), gm.data_ptr(),
                                                     gtable.data_ptr(), rows, C, _DT[x.dtype], ws.data_ptr(), ws_bytes, _stream_ptr(x.device)))
         need = ctx.needs_input_grad
-        glo = torch.bmm(gm, w2.transpose(1, 2)).transpose(0, 1).reshape(lo.shape) if need[2] else None
+        glo = torch.bmm(gm, w2.transpose(1, 2).contiguous()).transpose(0, 1).reshape(lo.shape) if need[2] else None
         gw2 = ctx.token_product(stack, gm) if need[3] else None
         return gx, gsx, glo, gw2, gtable, None
 
