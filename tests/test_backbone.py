@@ -1527,3 +1527,31 @@ def test_batched_products_take_dense_right_operands(monkeypatch):
     ctx = SimpleNamespace(saved_tensors=saved, needs_input_grad=[True] * 5, token_product=lambda a, b: a.transpose(1, 2) @ b)
     gx, gsx, glo, gw2, gtable, _ = ops._MaaLoraMix.backward(ctx, *torch.randn(5, B, T, C))
     assert glo.shape == (B * T, 160) and len(seen) == 4 and all(seen)
+
+
+def test_weights_too_wide_to_transpose_are_not_the_grouped_launchs():
+    from types import SimpleNamespace
+    from vision_rwkv_amd.ops import linear_takes
+    x = SimpleNamespace(shape=(4096, 1024), numel=lambda: 4096 * 1024, is_cuda=True, dtype=torch.bfloat16, device=torch.device("cpu"))
+    for n, takes in ((65536, True), (65536 + 128, False)):
+        assert linear_takes(x, [torch.zeros(n, 1024, dtype=torch.bfloat16)]) is takes
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("C", [8192, 8320])
+def test_channel_mixes_wider_than_the_gates_backward_kernel(C, monkeypatch):
+    """Rows of 8192 channels and more: the gradients of the tensor ops (bf16 products of up to C terms with fp32 sums, each result rounded: three roundings
+    of 2^-9 follow one another, 1e-2)."""
+    from vision_rwkv_amd import backbone as bb, ops
+    torch.manual_seed(3)
+    ffn = bb.VRWKV_ChannelMix(C, 2, 0, hidden_rate=1).cuda().bfloat16()
+    with torch.no_grad():
+        for p in (ffn.key.weight, ffn.value.weight, ffn.receptance.weight):
+            p.normal_(0, C ** -0.5)
+    xs = [torch.randn(520, C, device="cuda").bfloat16().requires_grad_() for _ in range(2)]
+    over = [*xs, ffn.key.weight, ffn.receptance.weight, ffn.value.weight]
+    g = torch.randn(520, C, device="cuda").bfloat16()
+    got = torch.autograd.grad(bb._channel_mix(ffn, *xs), over, g)
+    monkeypatch.setattr(ops, "ROW_FUSE_ENABLED", False)
+    want = torch.autograd.grad(bb._channel_mix(ffn, *xs), over, g)
+    assert all((a - b).norm() <= 1e-2 * b.norm() for a, b in zip(got, want))

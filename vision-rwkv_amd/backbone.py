@@ -338,7 +338,7 @@ def _channel_mix(ffn, xk, xr):
     if kn is None and ops.ROW_FUSE_ENABLED and type(xk) is type(xr) is torch.Tensor and xk.shape == xr.shape and xk.dtype == xr.dtype and xk.numel() >= CHANNEL_MIX_TILES:
         C, wk = xk.shape[-1], ffn.key._parameters.get("weight")
         ws = _own_weights((ffn.key, ffn.receptance, ffn.value), xk, (C, C, wk.shape[0] if wk is not None else 0))
-        if ws is not None and ws[1].shape[0] == ws[2].shape[0] == C:
+        if ws is not None and ws[1].shape[0] == ws[2].shape[0] == C <= 8192:       # (the gate's backward kernel takes rows of up to that)
             wk, wr, wv = ws
             if torch.is_grad_enabled() and any(t.requires_grad for t in (xk, xr, *ws)):
                 return _ChannelMix.apply(xk, xr, wk, wr, wv)

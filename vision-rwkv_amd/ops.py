@@ -1018,8 +1018,8 @@ EPI_RELU_SQ, EPI_RELU_SQ_BWD, EPI_ROUND = 1, 8, 16
 
 def linear_takes(x, weights, widths=None):
     """True where linear_group may stand in for x @ W^T on the GPU: 16-bit token matrices and weights of one type outside autocast and
-    every kind of transform, sizes that the kernel of the large tiles takes (include/vrwkv_hip.h, csrc/linear_wide.hip) and that fill
-    the chip with them: 70 tiles of 128 x 128.  widths: what each weight's input has for columns, x's by default; a weight that does not fit
+    every kind of transform, sizes that the kernel of the large tiles takes, and the transpose that the backward makes of the weights
+    (include/vrwkv_hip.h, csrc/linear_wide.hip), and that fill the chip with them: 70 tiles of 128 x 128.  widths: what each weight's input has for columns, x's by default; a weight that does not fit
     its input is left to the operators, which refuse it."""
     M, K = x.numel() // max(x.shape[-1], 1), x.shape[-1]
     if not (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and M > 0 and not torch.is_autocast_enabled("cuda") and not _transformed()):
@@ -1031,7 +1031,7 @@ def linear_takes(x, weights, widths=None):
         if not (w.dtype == x.dtype and w.device == x.device and w.is_contiguous() and w.data_ptr() % 16 == 0
                 and (N % 192 == k % 192 == 0 or N % 128 == k % 128 == 0)):
             return False
-        if M * N < 70 * 128 * 128 or (M + 256) * max(N, k) >= 1 << 29 or (N + 256) * (k + 256) >= 1 << 29:
+        if M * N < 70 * 128 * 128 or max(N, k) > 65536 or (M + 256) * max(N, k) >= 1 << 29 or (N + 256) * (k + 256) >= 1 << 29:
             return False
     return True
 
