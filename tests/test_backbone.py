@@ -1555,3 +1555,12 @@ def test_channel_mixes_wider_than_the_gates_backward_kernel(C, monkeypatch):
     monkeypatch.setattr(ops, "ROW_FUSE_ENABLED", False)
     want = torch.autograd.grad(bb._channel_mix(ffn, *xs), over, g)
     assert all((a - b).norm() <= 1e-2 * b.norm() for a, b in zip(got, want))
+
+
+def test_a_compiled_module_is_called_as_it_is():
+    """module.compile() changes what a call runs: neither a projection nor a mix is then taken apart."""
+    from vision_rwkv_amd import backbone as bb
+    lin = torch.nn.Linear(8, 8, bias=False)
+    assert bb._as_built(lin, torch.nn.Linear)
+    lin.compile()
+    assert not bb._as_built(lin, torch.nn.Linear)

@@ -423,7 +423,8 @@ def _native_wide(x, hidden, v6):
 
 def _as_built(module, kind):
     """True when calling `module` does what `kind`'s own forward does with the module's parameters and nothing else."""
-    return (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks and "forward" not in module.__dict__)
+    return (type(module) is kind and not module._forward_hooks and not module._forward_pre_hooks and "forward" not in module.__dict__
+            and module._compiled_call_impl is None)
 
 
 def _branch(mix, kind, x, res):
