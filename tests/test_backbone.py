@@ -1564,3 +1564,31 @@ def test_a_compiled_module_is_called_as_it_is():
     assert bb._as_built(lin, torch.nn.Linear)
     lin.compile()
     assert not bb._as_built(lin, torch.nn.Linear)
+
+
+class _Adapted(torch.nn.Linear):
+    def forward(self, x):
+        return 2 * super().forward(x)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["subclass", "sequential", "backward hook", "global hook"])
+def test_projections_that_do_more_than_multiply_are_called(kind):
+    """4096 tokens in training, where a plain projection's weight gradient is split: replaced layers and hooked ones run their own call."""
+    from torch.nn.modules import module as hooks
+    from vision_rwkv_amd import backbone as bb
+    lin = (_Adapted if kind == "subclass" else torch.nn.Linear)(192, 192, bias=False).cuda().bfloat16()
+    x = torch.randn(4096, 192, device="cuda").bfloat16().requires_grad_()
+    called, handle = [], None
+    if kind == "backward hook":
+        handle = lin.register_full_backward_hook(lambda m, gi, go: called.append(m) or None)
+    elif kind == "global hook":
+        handle = hooks.register_module_forward_hook(lambda m, i, o: called.append(m) or None)
+    fn = torch.nn.Sequential(lin) if kind == "sequential" else lin
+    try:
+        y = bb._proj(fn, x)
+        y.sum().backward()
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert torch.equal(y, lin(x)) and (handle is None or lin in called)

@@ -190,14 +190,18 @@ def _matmul(x, weight):
     return x @ weight
 
 
+def _only_multiplies(*linears):
+    """True for projections whose module call does nothing but multiply with their weight: no hook, no bias, no other class or forward."""
+    return (not _hooks._global_forward_hooks and not _hooks._global_forward_pre_hooks and not _hooks._global_backward_hooks
+            and not _hooks._global_backward_pre_hooks
+            and all(_as_built(l, nn.Linear) and not l._backward_hooks and not l._backward_pre_hooks and l.bias is None for l in linears))
+
+
 def _proj(linear, x):
     """linear(x) for the bias-free projections of a block; under autograd on the GPU with many tokens the weight gradient
     is split over the tokens (see _SplitKLinear)."""
-    w = linear.weight
-    hooked = linear._forward_hooks or linear._forward_pre_hooks       # hooks fire only through linear(x)
-    if (linear.bias is None and not hooked and x.is_cuda and torch.is_grad_enabled() and w.requires_grad
-            and x.dtype == w.dtype and x.dtype in (torch.bfloat16, torch.float16)):
-        M = x.numel() // x.shape[-1]
+    if x.is_cuda and torch.is_grad_enabled() and x.dtype in (torch.bfloat16, torch.float16) and _only_multiplies(linear) and linear.weight.requires_grad and x.dtype == linear.weight.dtype:
+        w, M = linear.weight, x.numel() // x.shape[-1]
         S = 4 if w.numel() >= (1 << 21) else 8
         if M >= 4096 and M % S == 0:
             return _SplitKLinear.apply(x, w, S)
@@ -312,12 +316,8 @@ CHANNEL_MIX_TILES = 256 * 128 * 128
 def _own_weights(linears, x, widths=None):
     """The weights of projections whose module call does nothing but multiply, and which vrwkv_linear_group takes; else None.  widths: of
     the projections' inputs, where they are not x."""
-    if (_hooks._global_forward_hooks or _hooks._global_forward_pre_hooks or _hooks._global_backward_hooks
-            or _hooks._global_backward_pre_hooks):
+    if not _only_multiplies(*linears) or any(type(l._parameters.get("weight")) is not nn.Parameter for l in linears):
         return None
-    for l in linears:
-        if not _as_built(l, nn.Linear) or l._backward_hooks or l._backward_pre_hooks or l.bias is not None or type(l._parameters.get("weight")) is not nn.Parameter:
-            return None
     ws = [l.weight for l in linears]
     return ws if linear_takes(x, ws, widths) else None
 
