@@ -291,3 +291,19 @@ def test_a_parameter_vector_is_read_element_by_element(tmp_path):
     subprocess.run([*build.split(), f"-I{csrc}", "-o", str(tmp_path / "v"), str(tmp_path / "v.hip")], check=True)
     done = subprocess.run([str(tmp_path / "v")], capture_output=True, text=True)
     assert done.returncode == 0, done.stderr[:2000]
+
+
+@pytest.mark.parametrize("fault", ["missing", "another torch"])
+def test_without_its_host_module_the_library_serves_the_python_classes(lib, fault, tmp_path, monkeypatch):
+    """The compiled host side belongs to the torch that it was built with; the library does not, and used to serve the operators alone."""
+    import torch
+    from vision_rwkv_amd import _lib, ops
+    monkeypatch.setattr(_lib, "_host", None)
+    if fault == "missing":
+        monkeypatch.setattr(_lib, "_HERE", str(tmp_path))
+    else:
+        monkeypatch.setattr(torch, "__version__", "1.0.0+other")
+    with pytest.warns(RuntimeWarning, match="missing" if fault == "missing" else "built with torch"):
+        host = _lib.host()
+    assert host.wkv(1, 2, 3, 4, 1.0) is None and host.wkv6(*range(10)) is None and _lib.host() is host
+    assert ops.block_weights_fit(torch.zeros(1, 1, 1), []) is False and ops.block_forward(torch.zeros(1, 1, 1), {}) is None

@@ -146,3 +146,23 @@ def test_recorded_into_a_graph_forward_and_backward():
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(outs, run(python)))
+
+
+@pytest.mark.parametrize("kind", ["wkv", "divided", "wkv6"])
+def test_the_operators_without_the_compiled_module(kind, monkeypatch):
+    xs, native, _ = _inputs(kind, torch.bfloat16)
+    run = lambda: (lambda y: (y, *torch.autograd.grad(y, xs, torch.ones_like(y))))(native(*xs))
+    want = run()
+    monkeypatch.setattr(_lib, "_host", _lib._NoHost)
+    got = run()
+    assert type(got[0].grad_fn).__name__ == {"wkv": "WKV", "divided": "_WKVDivided", "wkv6": "WKV_6"}[kind] + "Backward" and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_a_block_without_the_compiled_module(monkeypatch):
+    net = ops.VRWKV(img_size=32, patch_size=16, embed_dims=64, depth=1).to(DEV, torch.bfloat16).eval()
+    x = torch.randn(2, 3, 32, 32, generator=torch.Generator().manual_seed(3)).to(DEV, torch.bfloat16)
+    with torch.no_grad():
+        want = net(x).float()
+        monkeypatch.setattr(_lib, "_host", _lib._NoHost)
+        got = net(x).float()
+    assert (got - want).norm() <= 2 ** -6 * want.norm()      # a few roundings to 8 bits that the native call leaves out

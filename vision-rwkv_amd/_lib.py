@@ -7,6 +7,9 @@ import ctypes
 import importlib.util
 import os
 import subprocess
+import warnings
+
+import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libvrwkv_hip.so")
@@ -53,18 +56,43 @@ class VrwkvError(RuntimeError):
         self.status = status
 
 
+class _NoHost:
+    """What host() answers without the compiled module: None and False, with which the classes of ops.py go on by themselves."""
+    @staticmethod
+    def wkv(*args):
+        return None
+
+    wkv6 = block_forward = wkv
+
+    @staticmethod
+    def weights_fit(*args):
+        return False
+
+
+def _load_host(path):
+    """The module at path, or an ImportError that says why it cannot be this process's."""
+    if not os.path.exists(path):
+        raise ImportError(f"{path} is missing")
+    spec = importlib.util.spec_from_file_location("_host", path)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    built, here = module.torch_version, torch.__version__.split("+")[0]
+    if built != here:                                        # it passes torch's own objects: another build's layout may differ
+        raise ImportError(f"{path} was built with torch {built}, this is {here}")
+    return module
+
+
 def host():
-    """The compiled module of csrc/host: the operators' host side in C++.  It stands or falls with the library."""
+    """The compiled module of csrc/host: the operators' host side in C++.  It belongs to the torch that it was built with; where it is missing or
+    another's, the operators run through the classes of ops.py, the same kernels at more host time a call, after one warning."""
     global _host
     if _host is None:
         lib()
-        path = os.path.join(_HERE, "_host.so")
-        if not os.path.exists(path):
-            raise ImportError(f"{path} is missing: build it first (make -C vision-rwkv_amd/csrc)")
-        spec = importlib.util.spec_from_file_location("_host", path)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
-        _host = module
+        try:
+            _host = _load_host(os.path.join(_HERE, "_host.so"))
+        except ImportError as e:
+            warnings.warn(f"{e}: operators are called through Python, which takes longer (make -C vision-rwkv_amd/csrc builds it)", RuntimeWarning)
+            _host = _NoHost
     return _host
 
 

@@ -16,6 +16,7 @@
 #include <string_view>
 #include <unordered_map>
 #include <torch/extension.h>
+#include <torch/version.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -293,6 +294,7 @@ py::object block_forward(py::handle x_, py::dict tensors, py::object params, py:
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
+    m.attr("torch_version") = TORCH_VERSION;               // what the module's calls into torch were compiled against
     m.def("weights_fit", &weights_fit);
     m.def("block_forward", &block_forward);
     m.def("wkv", &wkv);
