@@ -200,10 +200,11 @@ def _only_multiplies(*linears):
 def _proj(linear, x):
     """linear(x) for the bias-free projections of a block; under autograd on the GPU with many tokens the weight gradient
     is split over the tokens (see _SplitKLinear)."""
-    if x.is_cuda and torch.is_grad_enabled() and x.dtype in (torch.bfloat16, torch.float16) and _only_multiplies(linear) and linear.weight.requires_grad and x.dtype == linear.weight.dtype:
-        w, M = linear.weight, x.numel() // x.shape[-1]
+    if (x.is_cuda and torch.is_grad_enabled() and x.dtype in (torch.bfloat16, torch.float16) and x.numel() >= 4096 * x.shape[-1]
+            and _only_multiplies(linear) and linear.weight.requires_grad and x.dtype == linear.weight.dtype):
+        w = linear.weight
         S = 4 if w.numel() >= (1 << 21) else 8
-        if M >= 4096 and M % S == 0:
+        if x.numel() // x.shape[-1] % S == 0:
             return _SplitKLinear.apply(x, w, S)
     return linear(x)
 
@@ -316,10 +317,10 @@ CHANNEL_MIX_TILES = 256 * 128 * 128
 def _own_weights(linears, x, widths=None):
     """The weights of projections whose module call does nothing but multiply, and which vrwkv_linear_group takes; else None.  widths: of
     the projections' inputs, where they are not x."""
-    if not _only_multiplies(*linears) or any(type(l._parameters.get("weight")) is not nn.Parameter for l in linears):
+    if any(type(l) is not nn.Linear or type(l._parameters.get("weight")) is not nn.Parameter for l in linears):
         return None
-    ws = [l.weight for l in linears]
-    return ws if linear_takes(x, ws, widths) else None
+    ws = [l._parameters["weight"] for l in linears]
+    return ws if linear_takes(x, ws, widths) and _only_multiplies(*linears) else None       # (sizes first: few tokens are the usual no)
 
 
 def _projs(linears, xs):

@@ -484,7 +484,7 @@ def _vec_ok(*tensors):
 
 def _dense(t):
     """t as the kernels read it, dense and on 16 bytes."""
-    return t if _vec_ok(t) else t.clone(memory_format=torch.contiguous_format)
+    return t if t is None or (t.is_contiguous() and not t.data_ptr() & 15) else t.clone(memory_format=torch.contiguous_format)
 
 
 def _saved(ctx):
@@ -1022,18 +1022,18 @@ def linear_takes(x, weights, widths=None):
     (include/vrwkv_hip.h, csrc/linear_wide.hip), and that fill the chip with them: 70 tiles of 128 x 128.  widths: what each weight's input has for columns, x's by default; a weight that does not fit
     its input is left to the operators, which refuse it."""
     M, K = x.numel() // max(x.shape[-1], 1), x.shape[-1]
-    if not (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and M > 0 and not torch.is_autocast_enabled("cuda") and not _transformed()):
+    if torch.compiler.is_compiling() or not (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and M > 0):
         return False
     for w, width in zip(weights, widths if widths is not None else [K] * len(weights)):
         if w.dim() != 2 or w.shape[1] != width:
             return False
         N, k = w.shape
-        if not (w.dtype == x.dtype and w.device == x.device and w.is_contiguous() and w.data_ptr() % 16 == 0
-                and (N % 192 == k % 192 == 0 or N % 128 == k % 128 == 0)):
-            return False
         if M * N < 70 * 128 * 128 or max(N, k) > 65536 or (M + 256) * max(N, k) >= 1 << 29 or (N + 256) * (k + 256) >= 1 << 29:
             return False
-    return True
+        if not (w.dtype == x.dtype and w.device == x.device and (N % 192 == k % 192 == 0 or N % 128 == k % 128 == 0)):
+            return False
+    return (not torch.is_autocast_enabled("cuda") and not _transformed()
+            and all(w.is_contiguous() and w.data_ptr() % 16 == 0 for w in weights))        # (memory last: not every traced tensor has any)
 
 
 def linear_group(problems):
@@ -1044,7 +1044,8 @@ def linear_group(problems):
     structs, results, keep = (_lib.Linear * n)(), [], []
     for s, p in zip(structs, problems):
         a, w = p["a"], p["w"]
-        if w.dim() != 2 or a.shape != (M, w.shape[1]) or any(t.dtype != dt or t.device != dev for t in (a, w)) or not w.is_contiguous():
+        if (w.dim() != 2 or a.shape != (M, w.shape[1]) or a.dtype != dt or w.dtype != dt or a.device != dev or w.device != dev
+                or not w.is_contiguous()):
             raise RuntimeError(f"a {tuple(a.shape)} and a contiguous w {tuple(w.shape)} must be (M, K) and (N, K) of one dtype")
         a = a if a.stride(1) == 1 and a.stride(0) % 8 == 0 and a.stride(0) >= a.shape[1] and a.data_ptr() % 16 == 0 else a.clone(memory_format=torch.contiguous_format)
         keep.append(a)
