@@ -309,7 +309,8 @@ class _ChannelMix(torch.autograd.Function):
 # A whole channel mix without key_norm takes them from 256 tiles on, where the passes they save (28 us forward, 43 back at 12544 x 3072)
 # outweigh a slower product: 4096 x 3072 x 768 28 / 34, 8192 42 / 40, 12544 62 / 54; 12544 x 768 x 3072 66 / 67; 12544 x 4096 x 1024 86 / 91.
 # With key_norm the products stay the library's: inside VRWKV-L, whose weights come from memory, a value product with the gate as its epilogue
-# takes 93 us at 9216 x 4096 x 1024 (two stages; 67 on weights that lie in the caches), the library's and the gate's pass 67 + 10.
+# takes 93 us at 9216 x 4096 x 1024 (two stages; 66 on operands that lie in the caches), the library's and the gate's pass 67 + 10.  All of these but the
+# last were taken on operands in the caches; on others the own kernel gives up more (csrc/linear_wide.hip).
 # Training steps of 64 images of 224 x 224, start and both of these: VRWKV-B 16195 -> 15108 us, VRWKV6-B 25761 -> 24499, bit for bit the same.
 CHANNEL_MIX_TILES = 256 * 128 * 128
 
@@ -358,28 +359,30 @@ def _layer_norm(ln, x):
 
 
 # Whether a block runs as one native call (vrwkv_block_fwd), by M C C, the multiplications of a (C, C) projection on M tokens.
-# Operator by operator the host takes 290 us a block (VRWKV6 490) and sets the pace up to some thousand tokens; the native call
-# takes it 58 (83), so called eagerly it gains until its time on the GPU reaches the host's or the library's, whichever is longer.
+# Operator by operator the host takes 215 to 290 us a block (VRWKV6 340 to 430) and sets the pace up to some thousand tokens; the native call
+# takes it 36 at most (VRWKV6 69), so called eagerly it gains until its time on the GPU reaches the host's or the library's, whichever is longer.
 # Recorded into a graph only the time on the GPU counts.  There the native call saves launches and passes over the tokens, and
-# its products are slower than the library's where the contraction is long: 6 to 15 % of a 16-bit block from about 1000 tokens of 768
-# or more channels on.  Up to 512 channels it is ahead in 16 bits.  (VRWKV6, whose operators are more, is within 1 % on the GPU at the
+# its products are slower than the library's where the contraction is long: up to 17 % of a 16-bit block from about 1000 tokens of 768
+# or more channels on.  Up to 512 channels it is ahead in 16 bits.  (VRWKV6, whose operators are more, is within a few % on the GPU at the
 # eager line; its operators would also record the forming of their tables, which its native call does not leave behind.)  Twelve blocks
-# of tokens x channels, operators ->
+# of tokens x channels, pre-norm without key norms, operators ->
 # native, eager | replayed, in us:
-#   VRWKV  bf16  784 x 768   3535 -> 1371 | 1415 -> 1362      1568 x 768   3532 -> 1704 | 1597 -> 1693      392 x 1024 3512 -> 1377 | 1508 -> 1375
-#                784 x 1024  3506 -> 1874 | 1648 -> 1868      3136 x 1024  3514 -> 2813 | 2466 -> 2806      6272 x 768 3566 -> 2964 | 3047 -> 2966
-#                6272 x 1024 3665 -> 4118 | 3674 -> 4109      12544 x 768  4892 -> 5334 | 4866 -> 5316      196 x 192  3529 ->  702 | 1492 ->  469
-#                3136 x 512  3528 -> 1452 | 1587 -> 1444      12544 x 512  3530 -> 2944 | 3287 -> 2926      12544 x 192 3521 -> 1388 | 1473 -> 1379
-#   VRWKV6 bf16  6272 x 768  6010 -> 4367 | 4720 -> 4335      3136 x 1024  5971 -> 3795 | 3830 -> 3766      6272 x 1024 5938 -> 5711 | 5628 -> 5680
-#                12544 x 768 7758 -> 7692 | 7659 -> 7660      12544 x 1024 8965 -> 10822 | 8879 -> 10797
+#   VRWKV  bf16  784 x 768   3323 -> 1185 | 1410 -> 1185      1568 x 768   2980 -> 1446 | 1449 -> 1446      392 x 1024 3328 -> 1444 | 1508 -> 1444
+#                784 x 1024  3280 -> 1555 | 1645 -> 1558      3136 x 1024  2969 -> 2720 | 2317 -> 2718      6272 x 768 2588 -> 2428 | 2581 -> 2430
+#                6272 x 1024 3930 -> 3804 | 3907 -> 3804      12544 x 768  4193 -> 3802 | 4174 -> 3799      196 x 192  3496 ->  430 | 1505 ->  388
+#                3136 x 512  2948 -> 1355 | 1465 -> 1359      12544 x 512  2639 -> 2423 | 2615 -> 2452      12544 x 192 2925 -> 1173 | 1413 -> 1177
+#   VRWKV6 bf16  6272 x 768  4041 -> 3673 | 3870 -> 3648      3136 x 1024  4575 -> 3634 | 3408 -> 3629      6272 x 1024 5511 -> 5260 | 5513 -> 5251
+#                12544 x 768 6377 -> 5912 | 6440 -> 5916      12544 x 1024 8959 -> 8563 | 8932 -> 8581      196 x 192  5066 ->  833 | 2484 ->  829
+# The 16-bit lines were drawn before the native call's projections of many tokens went to the wide kernel (widths in multiples of 128 as well): called
+# eagerly 6272 and 12544 x 1024 are 3 and 4 % ahead natively today, and 784 x 1024 recorded 5 %, which the lines leave to the operators.
 # fp32: a gap between few tokens, where launches count, and many, where the products of either are alike and the passes over the
 # tokens count: there the library's products are ahead (784 x 768, 1568 x 768, 392 and 784 x 1024, 1960 and 2352 x 512).
-#   VRWKV        392 x 768   3446 -> 1761 | 1892 -> 1760      784 x 768    3476 -> 2494 | 2274 -> 2485      1568 x 768 3481 -> 3915 | 3326 -> 3907
-#                3136 x 768  7010 -> 6330 | 6990 -> 6325      784 x 1024   3539 -> 3860 | 3394 -> 3853      1568 x 1024 5558 -> 5423 | 5524 -> 5411
-#                3136 x 384  3490 -> 2452 | 2400 -> 2438      6272 x 384   5768 -> 4026 | 5742 -> 3995      1568 x 512  3454 -> 2254 | 2349 -> 2233
-#                1960 x 512  3521 -> 2452 | 2174 -> 2454      3136 x 448   3859 -> 2970 | 3829 -> 2957      43904 x 192 7935 -> 8006 | 7917 -> 7999
-#   VRWKV6       784 x 768   5810 -> 3363 | 3357 -> 3339      1568 x 768   5825 -> 4994 | 4637 -> 4960      1568 x 1024 7193 -> 6854 | 7101 -> 6826
-#                2352 x 512  5943 -> 4005 | 4012 -> 3945      25088 x 192  7842 -> 7431 | 7718 -> 7419      3136 x 1024 13259 -> 12425 | 13180 -> 12409
+#   VRWKV        392 x 768   3226 -> 1757 | 1893 -> 1761      784 x 768    3267 -> 2481 | 2261 -> 2484      1568 x 768 3348 -> 3875 | 3319 -> 3876
+#                3136 x 768  6996 -> 6275 | 6975 -> 6277      784 x 1024   3411 -> 3842 | 3392 -> 3844      1568 x 1024 5550 -> 5390 | 5512 -> 5397
+#                3136 x 384  3296 -> 2441 | 2392 -> 2433      6272 x 384   5733 -> 3964 | 5728 -> 3964      1568 x 512  3309 -> 2223 | 2336 -> 2226
+#                1960 x 512  3506 -> 2441 | 2170 -> 2437      3136 x 448   3877 -> 2937 | 3822 -> 2933      43904 x 192 7934 -> 7932 | 7905 -> 7933
+#   VRWKV6       784 x 768   5200 -> 3322 | 3362 -> 3324      1568 x 768   5247 -> 4912 | 4632 -> 4919      1568 x 1024 7079 -> 6769 | 7069 -> 6768
+#                2352 x 512  5298 -> 3957 | 3993 -> 3951      25088 x 192  7745 -> 7315 | 7729 -> 7325      3136 x 1024 13191 -> 12315 | 13177 -> 12304
 NATIVE_NARROW = 512
 NATIVE_WORK = {False: (600_000_000, 3_800_000_000), True: (7_500_000_000, 7_500_000_000)}       # VRWKV6: most work recorded if wider, most work
 NATIVE_FP32_GAP = {                                   # (VRWKV6, narrow): the work left to the operators, recorded and called
@@ -405,11 +408,13 @@ def _native_size(x, hidden, v6):
 
 # In 16 bits the projections of many tokens go to a kernel of 256-channel tiles (csrc/linear_wide.hip) with three stages where C and the
 # hidden width are multiples of 192, and up to 768 channels such a block is ahead called eagerly at every size, recorded but for a
-# stretch where a block with key norms is 2 % behind (2352 x 768 1716 | 1753).  Operators -> native, eager | replayed:
-#   VRWKV  bf16  1568 x 768   3559 -> 1483 | 1595 -> 1480      3136 x 768, key norms 3597 -> 1901 | 1900 -> 1884      6272 x 768 3587 -> 2388 | 3064 -> 2384
-#                12544 x 768  4923 -> 3799 | 4887 -> 3785      25088 x 768  9237 -> 7356 | 9191 -> 7357      12544 x 192 3562 -> 1169 | 1483 -> 1158
-#   VRWKV6 bf16  1568 x 768   5887 -> 2246 | 2678 -> 2269      12544 x 768  7433 -> 6389 | 7422 -> 6383      12544 x 192 6272 -> 2069 | 2686 -> 2054
-# (VRWKV6 before the mixes formed their low-rank products inside, which takes 30 to 40 us a block of 12544 x 768 off either.)
+# stretch where a block with key norms is 8 % behind (2352 x 768; 5 % at 3136 x 768, past the stretch).  Of VRWKV6's projections
+# the output and the channel mix's go there: key, value, receptance and gate share their launch with the decay's first product, whose tanh
+# the wide kernel does not take, and stay on tiles of 128 x 128.  Operators -> native, eager | replayed:
+#   VRWKV  bf16  1568 x 768   2980 -> 1446 | 1449 -> 1446      2352 x 768, key norms 3185 -> 1818 | 1677 -> 1811      6272 x 768 2588 -> 2428 | 2581 -> 2430
+#                12544 x 768  4193 -> 3802 | 4174 -> 3799      3136 x 768, key norms 3195 -> 1957 | 1871 -> 1966      25088 x 768 7840 -> 7131 | 7850 -> 7142
+#                12544 x 192  2925 -> 1173 | 1413 -> 1177
+#   VRWKV6 bf16  1568 x 768   4611 -> 2115 | 2244 -> 2086      12544 x 768  6377 -> 5912 | 6440 -> 5916      12544 x 192 4546 -> 1931 | 2244 -> 1927
 NATIVE_WIDE, NATIVE_WIDE_GAP = 768, (600_000_000, 1_600_000_000)
 
 

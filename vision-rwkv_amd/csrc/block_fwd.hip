@@ -206,7 +206,8 @@ Layout layout(int B, int T, int C, int hidden, int heads, int dtype) {
 // ---- VRWKV6: the weights that the block wants otherwise than the modules hold them -----------------------------------------
 // The low-rank matrices with the contraction index innermost (32 x 32 tiles turned through LDS) and the vectors in fp32.  Formed
 // in every call, so that a write to a parameter leaves nothing behind: 448 C values, one launch of 3 us (twelve blocks of 784 x 768
-// bf16 1953 -> 1990 us, of 196 x 192 893 -> 935, against copies kept between calls).
+// bf16 1953 -> 1990 us, of 196 x 192 893 -> 935, against copies kept between calls).  160 C of them are maa_w2, which only fp32 blocks and
+// a misaligned maa_w2 read: the mixes of 16-bit ones take the matrix as it lies.
 // Grid: 14 C / 32 tiles, then C / 256 (rounded up) workgroups for the vectors.
 struct Weights6 {
     vrwkv_block6_params p;

@@ -3,7 +3,7 @@
 //
 // A workgroup is eight waves (two per SIMD) on a tile of 32 FM tokens x 256 channels, a wave on 16 FM x 64 of them (FM x 4 products
 // of 16 x 16 x 32 per 32 k).  Slices of 64 k of both operands go straight from memory to LDS (whole 128-byte lines: with slices of 32 k,
-// which fetch every line twice, 12544 x 3072 x 768 takes 70 us instead of 64), into one of two or three stages; a row's eight
+// which fetch every line twice, 12544 x 3072 x 768 on tiles of 160 tokens in two stages takes 70 us instead of 64), into one of two or three stages; a row's eight
 // 16-byte pieces lie rotated by an exclusive-or with the row, so that the fragment reads meet no bank twice (SQ_LDS_BANK_CONFLICT 0).
 // The fragments of the next 32 k are read into a second set of registers during the products of the present ones.  A stage is
 // refilled behind the barrier in the middle of its slice, when its last fragments are in registers: two half slices ahead
@@ -19,8 +19,13 @@
 // A lane ends up with 16 neighbouring channels of a token: the weights are the first operand of a product (result rows = channels),
 // and LDS row 16 f + 4 q + e of a wave's 64 channels holds channel 16 q + 4 f + e.
 //
-// us, three products of one shape in one launch here / three calls of the library: 12544 x 768 x 768 52 / 80, 9216 x 1024 x 1024 61 / 89;
-// one: 21 / 28, 24 / 31; 12544 x 768 x 3072 67 / 66, 12544 x 3072 x 768 54 / 62, 9216 x 1024 x 4096 79 / 79, 9216 x 4096 x 1024 67 / 71.
+// us (M x K x N), this kernel / the library, on the same operands again and again, which the caches then hold | on operands in rotation, more than they hold:
+//   three of 12544 x 768 x 768, here one launch  53 / 81 | 57 / 86      three of 9216 x 1024 x 1024  60 / 92 | 66 / 94
+//   one                                          22 / 30 | 22 / 29      one                          23 / 31 | 29 / 32
+//   12544 x 768 x 3072                           70 / 61 | 71 / 60      9216 x 1024 x 4096           79 / 73 | 85 / 74
+//   12544 x 3072 x 768                           51 / 59 | 55 / 63      9216 x 4096 x 1024           66 / 66 | 87 / 70
+// In a training step of 64 images of 224 x 224 at 768 channels, between other kernels and with epilogues, three of 12544 x 768 x 768 take 65 to 75, the
+// key's product with its two results 106 to 110.  The figures further down are of the first kind.
 #include "linear.h"
 #include <algorithm>
 
