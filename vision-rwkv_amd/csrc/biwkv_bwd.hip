@@ -126,24 +126,25 @@ void launch_tiled(const BwdPlan& p, const ParamVec& w, const ParamVec& u, const 
     int grid = biwkv_fwd_detail::num_cus() * per_cu;
     if (grid > geo.n_tiles) grid = geo.n_tiles;
     const dim3 g(grid), blk(p.S * WAVE);
+    // with fp32 vectors their type is known to the kernel (see TypedVec)
+    auto go = [&](auto mode, auto staged) {
+        auto with = [&](auto wp, auto up) {
+            hipLaunchKernelGGL((biwkv_bwd_tile_kernel<IO, L, decltype(mode)::value, decltype(staged)::value, decltype(wp)>), g, blk, 0, st, wp, up,
+                               k, v, gy, gk, gv, ws, agg1, agg2, gw_part, gu_part, B, T, C, geo);
+        };
+        if (w.dtype == VRWKV_F32) with(TypedVec<float>(w), TypedVec<float>(u));
+        else with(w, u);
+    };
     if (p.nSC == 1) {
         if constexpr (sizeof(IO) == 4) {
             const bool aligned = C % 4 == 0 && (((uintptr_t)k | (uintptr_t)v) & 15) == 0;
-            if (aligned && !option(OPT_BIWKV_NO_STAGE)) {
-                hipLaunchKernelGGL((biwkv_bwd_tile_kernel<IO, L, 0, true>), g, blk, 0, st, w, u, k, v, gy, gk, gv, ws, agg1, agg2,
-                                   gw_part, gu_part, B, T, C, geo);
-                return;
-            }
+            if (aligned && !option(OPT_BIWKV_NO_STAGE)) return go(std::integral_constant<int, 0>{}, std::true_type{});
         }
-        hipLaunchKernelGGL((biwkv_bwd_tile_kernel<IO, L, 0>), g, blk, 0, st, w, u, k, v, gy, gk, gv, ws, agg1, agg2,
-                           gw_part, gu_part, B, T, C, geo);
+        go(std::integral_constant<int, 0>{}, std::false_type{});
     } else if constexpr (L == 28 || L == 25 || L == 16) {
-        hipLaunchKernelGGL((biwkv_bwd_tile_kernel<IO, L, 1>), g, blk, 0, st, w, u, k, v, gy, gk, gv, ws, agg1, agg2,
-                           gw_part, gu_part, B, T, C, geo);
-        hipLaunchKernelGGL((biwkv_bwd_tile_kernel<IO, L, 2>), g, blk, 0, st, w, u, k, v, gy, gk, gv, ws, agg1, agg2,
-                           gw_part, gu_part, B, T, C, geo);
-        hipLaunchKernelGGL((biwkv_bwd_tile_kernel<IO, L, 3>), g, blk, 0, st, w, u, k, v, gy, gk, gv, ws, agg1, agg2,
-                           gw_part, gu_part, B, T, C, geo);
+        go(std::integral_constant<int, 1>{}, std::false_type{});
+        go(std::integral_constant<int, 2>{}, std::false_type{});
+        go(std::integral_constant<int, 3>{}, std::false_type{});
     }
 }
 

@@ -28,9 +28,9 @@ struct Scan {
 };
 
 // One lane: the whole sequence of batch element b, channel c (c < C).
-template <typename IO>
+template <typename IO, typename PV>
 __device__ __forceinline__
-void biwkv_bwd_serial_seq(const ParamVec w_, const ParamVec u_,
+void biwkv_bwd_serial_seq(const PV w_, const PV u_,
                           const IO* __restrict__ k_, const IO* __restrict__ v_, const IO* __restrict__ gy_,
                           IO* __restrict__ gk_, IO* __restrict__ gv_, float* __restrict__ ws,
                           float* __restrict__ gw_part, float* __restrict__ gu_part, int B, int T, int C, int b, int c,

@@ -84,9 +84,9 @@ struct BwdGeom {
 
 // STAGED (MODE 0, fp32 I/O, C % 4 == 0, 16-byte aligned k, v): the next tile's k, v rows are fetched straight into
 // LDS in 16-byte pieces (buffer_load ... lds) while this tile is computed; gy stays a register load.
-template <typename IO, int L, int MODE, bool STAGED = false>
+template <typename IO, int L, int MODE, bool STAGED, typename PV>
 __global__ __launch_bounds__(BWD_SMAX * WAVE)
-void biwkv_bwd_tile_kernel(const ParamVec w_, const ParamVec u_,
+void biwkv_bwd_tile_kernel(const PV w_, const PV u_,
                            const IO* __restrict__ k_, const IO* __restrict__ v_, const IO* __restrict__ gy_,
                            IO* __restrict__ gk_, IO* __restrict__ gv_,
                            float* __restrict__ ws, float* __restrict__ agg1, float* __restrict__ agg2,

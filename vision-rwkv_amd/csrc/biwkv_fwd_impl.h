@@ -915,8 +915,8 @@ inline Plan make_plan(int B, int T, int C, int io_dtype) {
 constexpr int GATE_NOT_FUSED = -100;
 
 // r: null, or the receptance whose sigmoid gates y inside the emitting kernel.
-template <typename IO, int VEC, int L, typename PV>
-int launch_L(const Plan& p, const PV& w, const PV& u, const void* k, const void* v, const void* r, void* y,
+template <typename IO, int VEC, int L>
+int launch_L(const Plan& p, const ParamVec& w, const ParamVec& u, const void* k, const void* v, const void* r, void* y,
              float* ws, int B, int T, int C, hipStream_t st) {
     const dim3 block(p.S * WAVE);
     const dim3 grid(p.grid);
@@ -924,13 +924,30 @@ int launch_L(const Plan& p, const PV& w, const PV& u, const void* k, const void*
     const IO* vv = static_cast<const IO*>(v);
     const IO* rr = static_cast<const IO*>(r);
     IO* yy = static_cast<IO*>(y);
+    typedef std::integral_constant<int, 0> whole;
+    typedef std::integral_constant<int, 1> aggregate;
+    typedef std::integral_constant<int, 2> emit;
+    // with fp32 vectors their type is known to the kernel (see TypedVec), but for the emitting kernel of rows that are not staged: that one spills,
+    // fp32 rows a quarter more with TypedVec (11 x 1528 x 293: 76 us instead of 55)
+    auto launch = [&](auto mode, auto staged, auto gate) {
+        constexpr int MODE = decltype(mode)::value;
+        constexpr bool STAGED = decltype(staged)::value, GATE = decltype(gate)::value;
+        auto go = [&](auto wp, auto up) {
+            hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, MODE, STAGED, GATE, decltype(wp)>), grid, block, 0, st, wp, up, kk, vv, yy, ws, T, C, p.geom, rr);
+        };
+        if constexpr (STAGED || MODE != 2) {
+            if (w.dtype == VRWKV_F32) return go(TypedVec<float>(w), TypedVec<float>(u));
+        }
+        go(w, u);
+    };
+    const std::true_type yes;
+    const std::false_type no;
     // fp32 rows are staged through LDS in 16-byte pieces when the layout allows it
     if constexpr (VEC == 1) {
         const bool aligned = C % (16 / (int)sizeof(IO)) == 0 && (((uintptr_t)k | (uintptr_t)v | (uintptr_t)y) & 15) == 0;
         if (aligned && !option(OPT_BIWKV_NO_STAGE)) {
             if (!p.multi()) {
-                if (rr) hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 0, true, true, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
-                else hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 0, true, false, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
+                if (rr) launch(whole{}, yes, yes); else launch(whole{}, yes, no);
             } else if (sizeof(IO) == 2 && L == 28 && p.nSC <= 3 && !option(OPT_BIWKV_NO_RESIDENT)) {
                 if (rr) return GATE_NOT_FUSED;
                 // two or three super-chunks of 16-bit rows fit a workgroup's registers: one launch, k and v read once
@@ -956,30 +973,30 @@ int launch_L(const Plan& p, const PV& w, const PV& u, const void* k, const void*
                 // fp32 rows: the emitting kernel of long sequences has no registers left for r (measured at 2 x 4150 x 768:
                 // 61 us with the gate inside against 50 us with the gate as a pass of its own); 16-bit rows: 32 against 37 us
                 if (rr && sizeof(IO) == 4) return GATE_NOT_FUSED;
-                hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 1, true, false, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
+                launch(aggregate{}, yes, no);
                 if constexpr (sizeof(IO) == 2) {
                     if (rr) {
-                        hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 2, true, true, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
+                        launch(emit{}, yes, yes);
                         return check_launch("biwkv_fwd");
                     }
                 }
-                hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 2, true, false, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
+                launch(emit{}, yes, no);
             }
             return check_launch("biwkv_fwd");
         }
     }
     if (rr) return GATE_NOT_FUSED;
     if (!p.multi()) {
-        hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 0, false, false, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
+        launch(whole{}, no, no);
     } else {
-        hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 1, false, false, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
-        hipLaunchKernelGGL((biwkv_fwd_kernel<IO, VEC, L, 2, false, false, PV>), grid, block, 0, st, w, u, kk, vv, yy, ws, T, C, p.geom, rr);
+        launch(aggregate{}, no, no);
+        launch(emit{}, no, no);
     }
     return check_launch("biwkv_fwd");
 }
 
-template <typename IO, int VEC, typename PV>
-int launch_VEC(const Plan& p, const PV& w, const PV& u, const void* k, const void* v, const void* r, void* y,
+template <typename IO, int VEC>
+int launch_VEC(const Plan& p, const ParamVec& w, const ParamVec& u, const void* k, const void* v, const void* r, void* y,
                float* ws, int B, int T, int C, hipStream_t st) {
     switch (p.L) {
 #define VRWKV_CASE(LL) case LL: return launch_L<IO, VEC, LL>(p, w, u, k, v, r, y, ws, B, T, C, st); break;
@@ -993,9 +1010,6 @@ int launch_VEC(const Plan& p, const PV& w, const PV& u, const void* k, const voi
 template <typename IO>
 int biwkv_fwd_launch_io(const Plan& p, const ParamVec& w, const ParamVec& u, const void* k, const void* v, const void* r, void* y,
                         float* ws, int B, int T, int C, hipStream_t st) {
-    if constexpr (sizeof(IO) == 4) {
-        if (w.dtype == VRWKV_F32) return launch_VEC<IO, 1>(p, TypedVec<float>(w), TypedVec<float>(u), k, v, r, y, ws, B, T, C, st);
-    }
     return launch_VEC<IO, 1>(p, w, u, k, v, r, y, ws, B, T, C, st);
 }
 

@@ -216,9 +216,10 @@ struct ParamVec {
         return x;
     }
 };
-// The same for vectors whose type is known at the launch, for kernels where the branches show: the fp32 forward, which is bound by memory and
-// waits for w and u among its rows (64 x 196 x 768: 23.9 us with ParamVec, 23.5 with TypedVec), and the forward that keeps 16-bit rows in registers
-// (16 x 577 x 768: bf16 22.1 and 21.5, fp16 22.5 and 21.6).
+// The same for vectors whose type is known at the launch: fp32 ones, which inference and the extension's own calls hand over, in nearly every kernel, and
+// those of the rows' type in the forward that keeps 16-bit rows in registers.  The branches of ParamVec are small beside a kernel of 20 us, but all
+// waves pass them while nothing else is on its way.  us, ParamVec / TypedVec: fp32 64 x 196 x 768 23.9 / 23.5, 30 x 196 x 767 18.5 / 17.7, backward 38.2 / 36.6;
+// fp32 vectors beside bf16 rows 2 x 4150 x 768 27.6 / 26.1, 4 x 1024 x 768 with the gate 20.9 / 19.3; 16 x 577 x 768 bf16 22.1 / 21.5, fp16 22.5 / 21.6.
 template <typename T> constexpr int type_code = std::is_same<T, float>::value ? VRWKV_F32 : std::is_same<T, __hip_bfloat16>::value ? VRWKV_BF16 : VRWKV_F16;
 template <typename T>
 struct TypedVec {
