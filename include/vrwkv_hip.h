@@ -119,8 +119,9 @@ int vrwkv_wkv6_fwd(const void* r, const void* k, const void* v, const void* w, c
                    float* y, int B, int T, int C, int H, int rkv_dtype, int w_dtype, int w_is_ew,
                    void* workspace, size_t workspace_bytes, void* hip_stream);
 
-/* Profiling twin of vrwkv_wkv6_fwd (no counterpart in the reference; for benchmarks and tuning): the same kernel
- * for bf16 r, k, v and fp32 raw-logit w, with every wave storing the shader clock at the boundaries of its stages.
+/* Profiling twin of vrwkv_wkv6_fwd (no counterpart in the reference; for benchmarks and tuning): the chunked kernel
+ * for bf16 r, k, v and fp32 raw-logit w, with every wave storing the shader clock at the boundaries of its stages
+ * (that kernel serves sequences of more than 256 tokens; shorter ones are stamped in it and then run as they are).
  * stamps: device buffer of vrwkv_wkv6_fwd_phases_bytes(B, T, H) bytes, laid out as uint64
  * [B*H][8 waves][ceil(T/32) chunk steps][8 points]: 0 element-wise stage entered, 1 its operands written (before the
  * barrier), 2 behind that barrier, 4 matrix stage entered, 5 y stored and the next decay sums formed (before the

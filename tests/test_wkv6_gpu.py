@@ -178,6 +178,28 @@ def test_cut_sequence_with_a_decay_out_of_range(ops):
     assert rel_err(y, clib.wkv6_fwd(*inputs, u, 2)) <= TOL
 
 
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 32, 33, 96, 127, 128, 129, 160, 161, 225, 256])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_sequences_as_one_or_two_products(ops, T, dtype):
+    """Up to 256 tokens in one or two parts of 16-token tiles against the sequential recurrence (5e-7 of the norm): every operand rounded at its 18th bit
+    (r~, k~, A or the state) and the tail x tail products left out, 2^-18 each, are 1.6e-5 at most.  A decay of 1.4 a token is beyond a part's range from
+    about 100 tokens on (the chunked kernel's code takes over), single strong tokens are not; 16-bit rows off 4 bytes take the chunked kernel."""
+    H = 2
+    for w_mean, spikes in ((-3.0, False), (0.3, False), (-3.0, True)):
+        x = [torch.from_numpy(a).cuda() for a in gen(2, T, H, seed=T, w_mean=w_mean, w_std=0.3)]
+        u = x.pop()
+        if spikes:
+            x[3][1, 5::40, 64:] = 2.3                                    # e^-10 at these tokens
+        x = [a.to(dtype) for a in x]
+        y = ops.wkv6_forward(2, T, 64 * H, H, *x, u)
+        with ops.option("wkv6_fwd_scalar", 1):
+            ref = ops.wkv6_forward(2, T, 64 * H, H, *x, u)
+        assert (y - ref).norm() <= 1.6e-5 * ref.norm(), (w_mean, spikes)
+        if dtype != torch.float32:
+            off = [torch.empty(a.numel() + 1, dtype=dtype, device="cuda")[1:].view_as(a).copy_(a) for a in x]
+            assert (ops.wkv6_forward(2, T, 64 * H, H, *off, u) - ref).norm() <= 1.6e-5 * ref.norm()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T", [300, 577, 1056, 1057])
 def test_sequences_are_cut_where_autograd_records_nothing(ops, T, dtype):

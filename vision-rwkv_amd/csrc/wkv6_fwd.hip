@@ -1,6 +1,7 @@
 // wkv6 forward entry points.
 #include "wkv6_fwd_scalar.h"
 #include "wkv6_fwd_chunk.h"
+#include "wkv6_fwd_tile.h"
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
@@ -35,14 +36,16 @@ int validate(int B, int T, int C, int H, int rkv_dtype, int w_dtype) {
     return VRWKV_OK;
 }
 
-// Segments per sequence of a call (1: not split); OPT_WKV6_SEGMENTS forces a number (testing).
-int segments(int B, int T, int H, int rkv_dtype) {
+// Segments per sequence of a call (1: not split); OPT_WKV6_SEGMENTS forces a number (testing).  parts: the tile kernels run them (bf16).
+int segments(int B, int T, int H, int rkv_dtype, bool& parts) {
     const int nchunk = (T + LC - 1) / LC, forced = option(OPT_WKV6_SEGMENTS);
     if (forced > 0 && (long long)B * H <= SEG_SEQUENCES) {
         const int n = forced < nchunk ? forced : nchunk, cps = (nchunk + n - 1) / n;
+        parts = rkv_dtype == VRWKV_BF16 && cps * LC <= TILE_TOKENS;
         return (nchunk + cps - 1) / cps;
     }
-    return forced > 0 ? 1 : wkv6_fwd_segments((long long)B * H, nchunk, device_cus(), SEG_FWD[rkv_dtype]);
+    parts = false;
+    return forced > 0 ? 1 : wkv6_fwd_segments((long long)B * H, nchunk, device_cus(), SEG_FWD[rkv_dtype], rkv_dtype == VRWKV_BF16 ? &parts : nullptr);
 }
 
 template <typename IO, typename WT>
@@ -74,9 +77,11 @@ int launch_chunked(const void* r, const void* k, const void* v, const void* w, c
     const IO* vv = static_cast<const IO*>(v);
     const WT* ww = static_cast<const WT*>(w);
     const long long sequences = (long long)B * H;
-    int nseg = segments(B, T, H, type_code<IO>);
-    // (the state kernel reads pairs of elements: 4-byte accesses of 16-bit rows; wider accesses need no more than 4 bytes either)
-    if (!ws || ws_bytes < seg_bytes(sequences, nseg, SEG_FLOATS) || ((uintptr_t)ws & 15) || (((uintptr_t)k | (uintptr_t)v | (uintptr_t)w) & 3)) nseg = 1;
+    bool parts;
+    int nseg = segments(B, T, H, type_code<IO>, parts);
+    // (the state and tile kernels read several elements at a time: 16-bit rows on 4 bytes; wider accesses need no more either)
+    const bool aligned = !(((uintptr_t)r | (uintptr_t)k | (uintptr_t)v | (uintptr_t)w) & 3);
+    if (!ws || ws_bytes < seg_bytes(sequences, nseg, SEG_FLOATS) || ((uintptr_t)ws & 15) || !aligned) nseg = 1;
     float* states = nullptr;
     int* flags = nullptr;
     unsigned grid = (unsigned)sequences;
@@ -84,9 +89,27 @@ int launch_chunked(const void* r, const void* k, const void* v, const void* w, c
         states = static_cast<float*>(ws);
         flags = reinterpret_cast<int*>(states + (size_t)sequences * nseg * SEG_FLOATS);
         grid = seg_grid(sequences, nseg);
-        hipLaunchKernelGGL((wkv6_seg_state_kernel<IO, WT, EW>), dim3(grid), dim3(256), 0, st, kk, vv, ww, states, flags, T, C, H,
-                           sequences, nseg);
+        if constexpr (type_code<IO> == VRWKV_BF16) {
+            if (parts)
+                hipLaunchKernelGGL((wkv6_part_state_kernel<IO, WT, EW>), dim3(grid), dim3(64 * PART_WAVES), 0, st, kk, vv, ww, states, flags, T, C, H,
+                                   sequences, nseg);
+        }
+        if (!parts)
+            hipLaunchKernelGGL((wkv6_seg_state_kernel<IO, WT, EW>), dim3(grid), dim3(256), 0, st, kk, vv, ww, states, flags, T, C, H, sequences, nseg);
         hipLaunchKernelGGL((wkv6_seg_fold_kernel<2, false>), dim3(4, 2, (unsigned)sequences), dim3(256), 0, st, states, nseg);
+    }
+    // Up to 256 tokens in one or two parts (the tile kernel is ahead of the chunked one at every size measured, 3 to 768 sequences of 33 to 256 tokens in
+    // all types: 1.03 to 1.8 times, least where a second part is nearly empty); more tokens, and rows off 4 bytes, are the chunked kernel's.
+    const FwdTileArgs tile{r, k, v, w, u, y, T, C, H, (int)sequences, nseg, states, flags};
+    if (nseg == 1 && T <= TILE_TOKENS && aligned) {
+        hipLaunchKernelGGL((wkv6_fwd_tile_kernel<IO, WT, EW, false>), dim3(grid), dim3(64 * PART_WAVES), 0, st, tile);
+        return check_launch("wkv6_fwd (tile)");
+    }
+    if constexpr (type_code<IO> == VRWKV_BF16) {
+        if (nseg > 1 && parts) {
+            hipLaunchKernelGGL((wkv6_fwd_tile_kernel<IO, WT, EW, true>), dim3(grid), dim3(64 * PART_WAVES), 0, st, tile);
+            return check_launch("wkv6_fwd (tile, segments)");
+        }
     }
     hipLaunchKernelGGL((wkv6_fwd_chunk_kernel<IO, WT, EW>), dim3(grid), block, 0, st, rr, kk, vv, ww, u, y, T, C, H, (int)sequences,
                        nseg, states, flags, nullptr);
@@ -134,6 +157,9 @@ extern "C" int vrwkv_wkv6_fwd_phases(const void* r, const void* k, const void* v
                        static_cast<const __hip_bfloat16*>(k), static_cast<const __hip_bfloat16*>(v),
                        static_cast<const float*>(w), u, y, T, C, H, B * H, 1, (const float*)nullptr, (const int*)nullptr,
                        static_cast<unsigned long long*>(stamps));
+    // (sequences that vrwkv_wkv6_fwd leaves to the tile kernel: y is that one's)
+    if (T <= TILE_TOKENS)
+        return launch_any<__hip_bfloat16, float>(r, k, v, w, u, y, nullptr, 0, B, T, C, H, false, static_cast<hipStream_t>(hip_stream));
     return check_launch("wkv6_fwd_phases");
 }
 
@@ -141,7 +167,9 @@ extern "C" size_t vrwkv_wkv6_fwd_workspace_bytes(int B, int T, int C, int H) {
     (void)C;
     if (B <= 0 || T <= 0 || H <= 0) return 0;
     // the same for every type: the largest of the plans
-    return seg_bytes((long long)B * H, std::max({segments(B, T, H, VRWKV_F32), segments(B, T, H, VRWKV_BF16), segments(B, T, H, VRWKV_F16)}), SEG_FLOATS);
+    bool parts;
+    return seg_bytes((long long)B * H, std::max({segments(B, T, H, VRWKV_F32, parts), segments(B, T, H, VRWKV_BF16, parts), segments(B, T, H, VRWKV_F16, parts)}),
+                     SEG_FLOATS);
 }
 
 extern "C" int vrwkv_wkv6_fwd(const void* r, const void* k, const void* v, const void* w, const float* u,

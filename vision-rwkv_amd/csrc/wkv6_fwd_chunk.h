@@ -97,16 +97,15 @@ struct __attribute__((aligned(16))) FwdLds {
 //   4 stage M entered   5 y stored and next decays summed, before the barrier   6 after that barrier   3, 7 unused
 constexpr int FW_STAMP_POINTS = 8;
 
+// One (b,h) sequence, or the segment `seg` of one, by the first FW_WAVES waves of a workgroup (no other wave may still be running).
 template <typename IO, typename WT, bool W_IS_EW, bool STAMPS = false>
-__global__ __launch_bounds__(64 * FW_WAVES, 4)   // four waves per SIMD: at most 128 registers
-void wkv6_fwd_chunk_kernel(const IO* __restrict__ r_, const IO* __restrict__ k_, const IO* __restrict__ v_,
-                           const WT* __restrict__ w_, const float* __restrict__ u_, float* __restrict__ y_,
-                           int T, int C, int H, int sequences, int nseg, const float* __restrict__ seg_ws,
-                           const int* __restrict__ seg_flags, unsigned long long* __restrict__ stamps = nullptr)
+__device__ __forceinline__
+void fwd_chunk_sequence(FwdLds<!__is_same(IO, __hip_bfloat16)>* lds, int* sFlag, int bh, int seg, const IO* __restrict__ r_,
+                        const IO* __restrict__ k_, const IO* __restrict__ v_, const WT* __restrict__ w_, const float* __restrict__ u_,
+                        float* __restrict__ y_, int T, int C, int H, int nseg, const float* __restrict__ seg_ws,
+                        const int* __restrict__ seg_flags, unsigned long long* __restrict__ stamps = nullptr)
 {
-    constexpr bool VSPLIT = !(sizeof(IO) == 2 && __is_same(IO, __hip_bfloat16));
-    __shared__ FwdLds<VSPLIT> lds[2];
-    __shared__ int sFlag[2];                   // out-of-range flags, one per half-period parity
+    constexpr bool VSPLIT = !__is_same(IO, __hip_bfloat16);
     static_assert(sizeof(FwdLds<VSPLIT>) * 2 >= 4 * 2 * 3 * N * sizeof(float), "fallback staging must fit");
 
     const int lane = threadIdx.x & 63;
@@ -114,17 +113,12 @@ void wkv6_fwd_chunk_kernel(const IO* __restrict__ r_, const IO* __restrict__ k_,
     const int w4 = wave & 3;                     // token quarter in stage E, value-column quarter in stage M
     const bool asc = wave >= 4;                  // waves 4-7: ascending pass (with the bonus)
     FwdLds<VSPLIT>& L = lds[asc ? 1 : 0];
-    int bh = blockIdx.x, seg = 0;
-    if (nseg > 1) {
-        seg_of_block(blockIdx.x, nseg, bh, seg);
-        if (bh >= sequences) return;
-    }
     const int b = bh / H, h = bh % H;
     const size_t base = (size_t)b * T * C + (size_t)h * HN;
     const int cps = ((T + LC - 1) / LC + nseg - 1) / nseg, c0 = seg * cps;       // this segment's chunks: c0 .. c0 + nchunk - 1
     const int nchunk = min(cps, (T + LC - 1) / LC - c0);
     const float uj = asc ? u_[h * HN + lane] : 0.f;
-    if (threadIdx.x < 2) sFlag[threadIdx.x] = 0;
+    if (threadIdx.x < 2) sFlag[threadIdx.x] = 0;                                 // out-of-range flags, one per half-period parity
     __syncthreads();
     unsigned long long* stamp_row = nullptr;
     if constexpr (STAMPS) stamp_row = stamps + ((size_t)bh * FW_WAVES + wave) * nchunk * FW_STAMP_POINTS;
@@ -538,6 +532,23 @@ void wkv6_fwd_chunk_kernel(const IO* __restrict__ r_, const IO* __restrict__ k_,
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
         if (wave < 4) wkv6_scalar_pass<IO, WT, 0, W_IS_EW>(r_, k_, v_, w_, u_, y_, stage, bh, T, C, H);
     }
+}
+
+template <typename IO, typename WT, bool W_IS_EW, bool STAMPS = false>
+__global__ __launch_bounds__(64 * FW_WAVES, 4)   // four waves per SIMD: at most 128 registers
+void wkv6_fwd_chunk_kernel(const IO* __restrict__ r_, const IO* __restrict__ k_, const IO* __restrict__ v_,
+                           const WT* __restrict__ w_, const float* __restrict__ u_, float* __restrict__ y_,
+                           int T, int C, int H, int sequences, int nseg, const float* __restrict__ seg_ws,
+                           const int* __restrict__ seg_flags, unsigned long long* __restrict__ stamps = nullptr)
+{
+    __shared__ FwdLds<!__is_same(IO, __hip_bfloat16)> lds[2];
+    __shared__ int sFlag[2];
+    int bh = blockIdx.x, seg = 0;
+    if (nseg > 1) {
+        seg_of_block(blockIdx.x, nseg, bh, seg);
+        if (bh >= sequences) return;
+    }
+    fwd_chunk_sequence<IO, WT, W_IS_EW, STAMPS>(lds, sFlag, bh, seg, r_, k_, v_, w_, u_, y_, T, C, H, nseg, seg_ws, seg_flags, stamps);
 }
 
 }  // namespace wkv6_detail

@@ -16,6 +16,7 @@
 // a third of the main kernel's work per chunk.
 #pragma once
 #include "wkv6_chunk_common.h"
+#include <algorithm>
 
 namespace vrwkv {
 namespace wkv6_detail {
@@ -59,15 +60,21 @@ inline int wkv6_segments(long long sequences, int nchunk, int cus, const SegCost
 // extra launches.  In microseconds, fitted for each type of r, k, v to 1 to 252 sequences of 9 to 130 chunks, uncut and in 2 to 64 segments: 19 000 times, the
 // estimate 4.5 % off (standard deviation).  Counts chosen against the best of the sweep: 0.2 % behind on average, 4 (fp32 7) at most.  On 3 200 further shapes
 // they are 10 % ahead on average of what the backward's estimate would choose, and at most 6 % behind that or uncut.  us, uncut | segments:
-//   bf16   24 sequences of 130 chunks 354 | 8 84, 10 69, 12 84, 19 64          fp32   36 of 130  364 | 6 113, 7 162, 10 127
-//          96 of 10                    32 | 2 36, 3 43, 4 38, 5 33                    48 of 24    71 | 6 52, 8 47, 12 56
-//         132 of 12                    38 | 2 54, 3 45                                84 of 24    72 | 2 68, 3 84, 5 65
-//          84 of 33                    93 | 2 83, 3 84, 5 64                         120 of 33    98 | 2 95, 4 99
+//   fp32   36 sequences of 130 chunks 364 | 6 113, 7 162, 10 127
+//          48 of 24                    71 | 6 52, 8 47, 12 56
+//          84 of 24                    72 | 2 68, 3 84, 5 65
+//         120 of 33                    98 | 2 95, 4 99
+// bf16 sequences can also be cut into segments of 128 tokens, one part of the tile kernel each (wkv6_fwd_tile.h): `parts`.  That cut's time is estimated
+// from the segments, all of them and those of a sequence (the scan); for a few sequences finer segments of the chunked kernels are ahead (3 of 10 chunks
+// 16.5 against 20.3).  us, uncut | segments (the 128-token cut in brackets):
+//          24 of 130                  354 | 10 65, 17 61, 26 76, [33] 62            192 of 32    94 | 4 95, [8] 95, 11 119
+//          48 of 64                   174 | 8 59, 10 61, [16] 55, 32 81             192 of 13    41 | 2 58, [4] 50, 5 56
+//          96 of 19                    56 | 3 54, [5] 37, 10 54                      96 of 10    32 | 2 36, [3] 36, 5 35
 struct FwdSegCosts { double uncut, uncut_fixed, uncut_traffic, step[4], fixed, per_segment, traffic, token_traffic; };
 constexpr FwdSegCosts SEG_FWD[3] = {{2.72, 4.0, 2.23, {3.73, 7.06, 11.09, 14.80}, 9.8, 0.14, 28.5, 3.39},       // VRWKV_F32
                                     {2.65, 5.1, 1.09, {3.53, 5.14, 8.16, 10.48}, 10.8, 0.14, 20.3, 3.44},       // VRWKV_BF16
                                     {2.80, 4.9, 1.33, {3.99, 7.28, 10.68, 14.05}, 9.6, 0.14, 29.9, 1.70}};      // VRWKV_F16
-inline int wkv6_fwd_segments(long long sequences, int nchunk, int cus, const FwdSegCosts& k) {
+inline int wkv6_fwd_segments(long long sequences, int nchunk, int cus, const FwdSegCosts& k, bool* parts) {
     const long long padded = (sequences + 7) / 8 * 8;
     if (nchunk <= 8 || padded > cus) return 1;       // more sequences than compute units: a cut only adds work
     int best = 1;
@@ -77,6 +84,12 @@ inline int wkv6_fwd_segments(long long sequences, int nchunk, int cus, const Fwd
         const int cps = (nchunk + nseg - 1) / nseg, per_cu = (int)((padded * nseg + cus - 1) / cus);
         const double t = cps * k.step[per_cu - 1] + k.fixed + k.per_segment * nseg + k.traffic * 1e-3 * (double)(sequences * nseg) + k.token_traffic * chunks;
         if (t < best_time) { best = nseg; best_time = t; }
+    }
+    if (parts) {
+        const int cps = std::max(4, (nchunk + SEG_MAX - 1) / SEG_MAX), nseg = (nchunk + cps - 1) / cps;
+        const double t = std::max(19.0 + 0.45 * nseg, 15.0 + 0.25 * nseg + 0.052 * (double)(sequences * nseg));
+        *parts = t < (best == 1 ? 0.95 : 1.0) * best_time && cps * LC <= 2 * 128;
+        if (*parts) return nseg;
     }
     const int cps = (nchunk + best - 1) / best;
     return (nchunk + cps - 1) / cps;                 // every segment non-empty
@@ -138,6 +151,41 @@ __global__ __launch_bounds__(256) void wkv6_seg_fold_kernel(float* __restrict__ 
         d += U * step;
     }
 }
+
+// Operand arrays in LDS: rows of 64 bf16 (eight 16-byte chunks), chunk c of row t at place c ^ (t & 7), so that 16-byte accesses of eight rows and
+// 8-byte transposing reads of four fall into distinct banks without padding.
+__device__ __forceinline__ unsigned row_chunk(unsigned row, unsigned chunk) { return row * 128u + ((chunk ^ (row & 7u)) << 4); }
+// 16 channels (tile ct) of an array x the 32 tokens of block q, as an operand: slot (g4, e) is token 4 g4 + e (e < 4), 16 + 4 g4 + e - 4 (e >= 4)
+__device__ __forceinline__ bf16x8 read_across(const unsigned char* arr, int q, int ct, int lane) {
+    const int g4 = lane >> 4, c16 = lane & 15;
+    const unsigned char* p = arr + row_chunk(4 * g4 + (c16 >> 2), 2 * ct + ((c16 >> 1) & 1)) + 8 * (c16 & 1) + 4096 * q;
+    return cat8(lds_read_tr4(reinterpret_cast<const __bf16*>(p)), lds_read_tr4(reinterpret_cast<const __bf16*>(p + 2048)));
+}
+// eight packed elements of a row, in 16-byte pieces, widened
+template <typename T>
+__device__ __forceinline__ void widen8(const u32x4* raw, float (&o)[8]) {
+    T t[8];
+    __builtin_memcpy(t, raw, sizeof(t));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = to_f32(t[e]);
+}
+// Log2 decays of a row's eight channels from its logits, summed over the row's predecessors among the wave's 16 tokens (lanes of a row of 16)
+template <typename WT, bool W_IS_EW>
+__device__ __forceinline__ void summed_decays(const u32x4* raw, bool past, float (&x)[8]) {
+    widen8<WT>(raw, x);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        float d = W_IS_EW ? x[e] * LOG2E : -fast_exp2(fmaf(x[e], LOG2E, LOG2_LOG2E));
+        d = past ? 0.f : d;
+        d += dpp_get<0x111>(d);                      // row_shr:1, 2, 4, 8
+        d += dpp_get<0x112>(d);
+        d += dpp_get<0x114>(d);
+        d += dpp_get<0x118>(d);
+        x[e] = d;
+    }
+}
+
+constexpr int PART_WAVES = 8, PART = 16 * PART_WAVES;                     // waves of a workgroup, tokens it holds at a time
 
 template <typename IO> struct SegLds {
     static constexpr bool VSPLIT = !__is_same(IO, __hip_bfloat16);
@@ -281,6 +329,149 @@ void wkv6_seg_state_kernel(const IO* __restrict__ k_, const IO* __restrict__ v_,
     // every wave's half waves saw the same chunk totals: wave 0's first half speaks for all
     if (w4 == 0) {
         if (lane < 32) *reinterpret_cast<f32x2*>(out + 2 * SEG_STATE + cp) = f32x2{fast_exp2(base_p[0]), fast_exp2(base_p[1])};
+        const bool any = __builtin_amdgcn_ballot_w64(out_of_range) != 0ull;
+        if (lane == 0) flags[(size_t)bh * nseg + seg] = any ? 1 : 0;
+    }
+}
+
+// The same in parts of up to 128 tokens: eight waves, a wave prepares 16 tokens in the layout of the matrix operands (lane = token c16, eight channels of
+// each half) and then forms a quarter of the columns x half the rows of both states over the part's tokens.  All exponents are <= 0.  Two barriers per 128
+// tokens where the kernel above has two per 32; bound by the latency of its loads (two workgroups a compute unit) and by the states' way out.
+// 24 sequences of 4150 tokens in 17 segments 22 -> 17.6 us.  bf16 only: the operands of a split v leave room for one workgroup (fp32 21 -> 29 us).
+template <typename IO, typename WT, bool W_IS_EW>
+__global__ __launch_bounds__(64 * PART_WAVES, 4)
+void wkv6_part_state_kernel(const IO* __restrict__ k_, const IO* __restrict__ v_, const WT* __restrict__ w_,
+                           float* __restrict__ ws, int* __restrict__ flags, int T, int C, int H, long long sequences, int nseg)
+{
+    static_assert(__is_same(IO, __hip_bfloat16), "v exact in bf16: the operands of a split v leave room for one workgroup a compute unit");
+    constexpr unsigned ES = (unsigned)sizeof(IO), WS = (unsigned)sizeof(WT), ARR = PART * 128u;
+    constexpr unsigned AH = 0, AL = ARR, DH = 2 * ARR, DL = 3 * ARR, VH = 4 * ARR;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[5 * ARR];
+    int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int bh, seg;
+    seg_of_block(blockIdx.x, nseg, bh, seg);
+    if (bh >= sequences) return;
+    const size_t base = (size_t)(bh / H) * T * C + (size_t)(bh % H) * HN;
+    const int nchunk = (T + LC - 1) / LC, cps = (nchunk + nseg - 1) / nseg;
+    const int first = seg * cps * LC, n = min(cps * LC, T - first);
+    // rows past T (last part only) lie outside the descriptors and read 0: k = 0 switches such a token off, and its decay is set to 1
+    auto fetch = [&](const void* p, int t0, auto& raw, unsigned es) {
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(static_cast<const char*>(p) + base * es, (unsigned)(((size_t)(T - 1) * C + HN) * es));
+        constexpr int pieces = sizeof(raw[0]) / 16;
+        const unsigned vo = ((unsigned)(lane & 15) * C + 8 * (lane >> 4)) * es, so = (unsigned)(t0 + 16 * wave) * C * es;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int i = 0; i < pieces; ++i) raw[kb][i] = BufRaw<16>::ld(rs, vo + 32u * kb * es + 16u * i, so);
+    };
+    const int jt0 = 2 * (wave >> 2), it0 = wave & 3;                      // the wave's tiles: rows 16 (jt0 + q) + 4 g4 + r, column 16 it0 + c16
+    f32x4 A[2], D[2];                                                     // up and down states
+    A[0] = A[1] = D[0] = D[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float base_p = 0.f;                                                   // log2 decay from the segment's start to the part, channel `lane`
+    bool out_of_range = false;
+    u32x4 wraw[2][WS / 2], kraw[2][ES / 2], vraw[2][ES / 2];
+    fetch(w_, first, wraw, WS);
+    fetch(k_, first, kraw, ES);
+    fetch(v_, first, vraw, ES);
+#pragma unroll 1
+    for (int at = 0; at < n; at += PART) {
+        asm volatile("" : "+v"(lane));
+        const int np = min(n - at, PART), nb = (np + LC - 1) / LC, g4 = lane >> 4, c16 = lane & 15;
+        float x[2][8];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            summed_decays<WT, W_IS_EW>(wraw[kb], 16 * wave + c16 >= np, x[kb]);
+            if (c16 == 15) {
+#pragma unroll
+                for (int hf = 0; hf < 2; ++hf)
+                    *reinterpret_cast<f32x4*>(lds + AH + 256 * wave + 128 * kb + 32 * g4 + 16 * hf) =
+                        f32x4{x[kb][4 * hf], x[kb][4 * hf + 1], x[kb][4 * hf + 2], x[kb][4 * hf + 3]};
+            }
+        }
+        lds_barrier();
+        float total = 0.f;
+        {
+            float before = 0.f, t[PART_WAVES];
+#pragma unroll
+            for (int g = 0; g < PART_WAVES; ++g) {
+                t[g] = *reinterpret_cast<const float*>(lds + AH + 256 * g + 4 * lane);
+                before += g < wave ? t[g] : 0.f;
+                total += t[g];
+            }
+#pragma unroll
+            for (int g = 0; g < PART_WAVES; g += 2) out_of_range |= !(t[g] + t[g + 1] >= -SAFE_DECAY * LOG2E);    // a 32-token chunk
+            float* const own = reinterpret_cast<float*>(lds + AL + 2048 * wave);                                  // (in the wave's own rows)
+            own[lane] = before;
+            own[HN + lane] = total;
+            own[2 * HN + lane] = base_p;
+        }
+        lds_barrier();                                                    // the sums are read: their place is written below
+        f32x4 bs[2][2], tt[2][2], bp[2][2];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int hf = 0; hf < 2; ++hf) {
+                const unsigned char* own = lds + AL + 2048 * wave + 128 * kb + 32 * g4 + 16 * hf;
+                bs[kb][hf] = *reinterpret_cast<const f32x4*>(own);
+                tt[kb][hf] = *reinterpret_cast<const f32x4*>(own + 256) - bs[kb][hf];         // from the wave's start to the part's end
+                bp[kb][hf] = *reinterpret_cast<const f32x4*>(own + 512) + bs[kb][hf];         // from the segment's start to the wave's
+            }
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            const unsigned to = row_chunk(16 * wave + c16, 4 * kb + g4);
+            float k8[8], o8[8];
+            bf16x8 hi, lo;
+            widen8<IO>(kraw[kb], k8);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o8[e] = k8[e] * fast_exp2(tt[kb][e >> 2][e & 3] - x[kb][e]);
+            split8<true>(o8, hi, lo);
+            *reinterpret_cast<bf16x8*>(lds + AH + to) = hi;
+            *reinterpret_cast<bf16x8*>(lds + AL + to) = lo;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o8[e] = k8[e] * fast_exp2(bp[kb][e >> 2][e & 3] + dpp_get<0x111>(x[kb][e]));
+            split8<true>(o8, hi, lo);
+            *reinterpret_cast<bf16x8*>(lds + DH + to) = hi;
+            *reinterpret_cast<bf16x8*>(lds + DL + to) = lo;
+            *reinterpret_cast<u32x4*>(lds + VH + to) = vraw[kb][0];
+        }
+        lds_barrier();
+        if (at + PART < n) {
+            fetch(w_, first + at + PART, wraw, WS);
+            fetch(k_, first + at + PART, kraw, ES);
+            fetch(v_, first + at + PART, vraw, ES);
+        }
+        if (at > 0) {                                                     // the up state over this part's decay
+            const float f = fast_exp2(total);
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) A[q][e] *= __shfl(f, 16 * (jt0 + q) + 4 * g4 + e);
+        }
+#pragma unroll 1
+        for (int q = 0; q < nb; ++q) {
+            const bf16x8 vv = read_across(lds + VH, q, it0, lane);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const bf16x8 ah = read_across(lds + AH, q, jt0 + j, lane), al = read_across(lds + AL, q, jt0 + j, lane);
+                const bf16x8 dh = read_across(lds + DH, q, jt0 + j, lane), dl = read_across(lds + DL, q, jt0 + j, lane);
+                A[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, vv, A[j], 0, 0, 0);
+                D[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dh, vv, D[j], 0, 0, 0);
+                A[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, vv, A[j], 0, 0, 0);
+                D[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dl, vv, D[j], 0, 0, 0);
+            }
+        }
+        base_p += total;
+        lds_barrier();                                                    // the operands' place is written next
+    }
+    float* out = ws + ((size_t)bh * nseg + seg) * SEG_FLOATS;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        *reinterpret_cast<f32x4*>(out + seg_frag(it0, jt0 + q, lane)) = A[q];
+        *reinterpret_cast<f32x4*>(out + SEG_STATE + seg_frag(it0, jt0 + q, lane)) = D[q];
+    }
+    if (wave == 0) {                                                      // every wave saw all totals
+        out[2 * SEG_STATE + lane] = fast_exp2(base_p);
         const bool any = __builtin_amdgcn_ballot_w64(out_of_range) != 0ull;
         if (lane == 0) flags[(size_t)bh * nseg + seg] = any ? 1 : 0;
     }
