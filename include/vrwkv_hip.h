@@ -118,6 +118,10 @@ size_t vrwkv_wkv6_fwd_workspace_bytes(int B, int T, int C, int H);
 int vrwkv_wkv6_fwd(const void* r, const void* k, const void* v, const void* w, const float* u,
                    float* y, int B, int T, int C, int H, int rkv_dtype, int w_dtype, int w_is_ew,
                    void* workspace, size_t workspace_bytes, void* hip_stream);
+/* The same uncut and 32 tokens at a time at every length: y then has the same bits whatever the number of sequences, and the tokens
+ * in front of a position are summed the same way in sequences of any length.  For 16-bit networks in training, which amplify last bits. */
+int vrwkv_wkv6_fwd_whole(const void* r, const void* k, const void* v, const void* w, const float* u, float* y,
+                         int B, int T, int C, int H, int rkv_dtype, int w_dtype, int w_is_ew, void* hip_stream);
 
 /* Profiling twin of vrwkv_wkv6_fwd (no counterpart in the reference; for benchmarks and tuning): the chunked kernel
  * for bf16 r, k, v and fp32 raw-logit w, with every wave storing the shader clock at the boundaries of its stages

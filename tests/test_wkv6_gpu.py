@@ -183,7 +183,7 @@ def test_cut_sequence_with_a_decay_out_of_range(ops):
 def test_sequences_as_one_or_two_products(ops, T, dtype):
     """Up to 256 tokens in one or two parts of 16-token tiles against the sequential recurrence (5e-7 of the norm): every operand rounded at its 18th bit
     (r~, k~, A or the state) and the tail x tail products left out, 2^-18 each, are 1.6e-5 at most.  A decay of 1.4 a token is beyond a part's range from
-    about 100 tokens on (the chunked kernel's code takes over), single strong tokens are not; 16-bit rows off 4 bytes take the chunked kernel."""
+    about 100 tokens on (the chunked kernel's code takes over), single strong tokens are not; 16-bit rows off 4 bytes give the same bits."""
     H = 2
     for w_mean, spikes in ((-3.0, False), (0.3, False), (-3.0, True)):
         x = [torch.from_numpy(a).cuda() for a in gen(2, T, H, seed=T, w_mean=w_mean, w_std=0.3)]
@@ -197,7 +197,24 @@ def test_sequences_as_one_or_two_products(ops, T, dtype):
         assert (y - ref).norm() <= 1.6e-5 * ref.norm(), (w_mean, spikes)
         if dtype != torch.float32:
             off = [torch.empty(a.numel() + 1, dtype=dtype, device="cuda")[1:].view_as(a).copy_(a) for a in x]
-            assert (ops.wkv6_forward(2, T, 64 * H, H, *off, u) - ref).norm() <= 1.6e-5 * ref.norm()
+            assert torch.equal(ops.wkv6_forward(2, T, 64 * H, H, *off, u), y)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T", [1, 32, 129, 196, 256])
+def test_what_autograd_records_in_16_bits_goes_chunk_by_chunk(ops, T, dtype):
+    """A 16-bit forward that is recorded has the bits of the uncut entry at every length, through the host module and through the Python class; y is within
+    the rounding of the split operands of the one that is not recorded (either 5e-6 of the norm from float64)."""
+    H = 2
+    x = [torch.from_numpy(a).cuda() for a in gen(2, T, H, seed=T, w_mean=-3.0, w_std=0.5)]
+    u = x.pop()
+    x = [a.to(dtype).requires_grad_() for a in x]
+    args = (2, T, 64 * H, H, *x, u)
+    with torch.no_grad():
+        whole, plain = ops.wkv6_forward(*args, whole=True), ops.RUN_CUDA_RWKV6(*args)
+    assert (whole - plain).norm() <= 1.6e-5 * whole.norm()
+    for y in (ops.RUN_CUDA_RWKV6(*args), ops.WKV_6.apply(*args)):
+        assert torch.equal(y, plain if dtype == torch.float32 else whole)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])

@@ -135,6 +135,8 @@ def _declare(lib):
     lib.vrwkv_wkv6_fwd_workspace_bytes.restype = sz
     lib.vrwkv_wkv6_fwd.argtypes = [vp, vp, vp, vp, fp, vp, i, i, i, i, i, i, i, vp, sz, vp]
     lib.vrwkv_wkv6_fwd.restype = i
+    lib.vrwkv_wkv6_fwd_whole.argtypes = [vp, vp, vp, vp, fp, vp, i, i, i, i, i, i, i, vp]
+    lib.vrwkv_wkv6_fwd_whole.restype = i
     lib.vrwkv_wkv6_fwd_phases_bytes.argtypes = [i, i, i]
     lib.vrwkv_wkv6_fwd_phases_bytes.restype = sz
     lib.vrwkv_wkv6_fwd_phases.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, i, vp, sz, vp]

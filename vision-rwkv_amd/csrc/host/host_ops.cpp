@@ -135,7 +135,12 @@ at::Tensor wkv6_forward(const at::Tensor& r, const at::Tensor& k, const at::Tens
     const int B = (int)r.size(0), T = (int)r.size(1), C = (int)r.size(2);
     Guard guard(r.device());
     at::Tensor y = at::empty_like(r, r.options().dtype(at::kFloat)), ws;
-    const size_t n = whole ? 0 : vrwkv_wkv6_fwd_workspace_bytes(B, T, C, H);
+    if (whole) {
+        const int rc = vrwkv_wkv6_fwd_whole(r.data_ptr(), k.data_ptr(), v.data_ptr(), w.data_ptr(), (const float*)u.data_ptr(), (float*)y.data_ptr(),
+                                            B, T, C, H, code(r.scalar_type()), code(w.scalar_type()), 0, stream_of(r));
+        return rc == VRWKV_OK ? y : at::Tensor();
+    }
+    const size_t n = vrwkv_wkv6_fwd_workspace_bytes(B, T, C, H);
     if (n) ws = bytes(n, r);
     const int rc = vrwkv_wkv6_fwd(r.data_ptr(), k.data_ptr(), v.data_ptr(), w.data_ptr(), (const float*)u.data_ptr(), (float*)y.data_ptr(), B, T, C, H,
                                   code(r.scalar_type()), code(w.scalar_type()), 0, n ? ws.data_ptr() : nullptr, n, stream_of(r));

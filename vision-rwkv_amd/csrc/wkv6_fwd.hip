@@ -70,18 +70,18 @@ int launch_scalar(const void* r, const void* k, const void* v, const void* w, co
 // recurrence; few long sequences are cut into segments first (wkv6_segment.h) when the caller's workspace allows it.
 template <typename IO, typename WT, bool EW>
 int launch_chunked(const void* r, const void* k, const void* v, const void* w, const float* u, float* y, void* ws, size_t ws_bytes,
-                   int B, int T, int C, int H, hipStream_t st) {
+                   int B, int T, int C, int H, bool whole, hipStream_t st) {
     const dim3 block(64 * FW_WAVES);
     const IO* rr = static_cast<const IO*>(r);
     const IO* kk = static_cast<const IO*>(k);
     const IO* vv = static_cast<const IO*>(v);
     const WT* ww = static_cast<const WT*>(w);
     const long long sequences = (long long)B * H;
-    bool parts;
-    int nseg = segments(B, T, H, type_code<IO>, parts);
-    // (the state and tile kernels read several elements at a time: 16-bit rows on 4 bytes; wider accesses need no more either)
-    const bool aligned = !(((uintptr_t)r | (uintptr_t)k | (uintptr_t)v | (uintptr_t)w) & 3);
-    if (!ws || ws_bytes < seg_bytes(sequences, nseg, SEG_FLOATS) || ((uintptr_t)ws & 15) || !aligned) nseg = 1;
+    bool parts = false;
+    int nseg = whole ? 1 : segments(B, T, H, type_code<IO>, parts);
+    // (the state kernels read several elements at a time: 16-bit rows on 4 bytes; wider accesses need no more either)
+    const bool cut = !(((uintptr_t)k | (uintptr_t)v | (uintptr_t)w) & 3), loose = !cut || ((uintptr_t)r & 3);
+    if (!ws || ws_bytes < seg_bytes(sequences, nseg, SEG_FLOATS) || ((uintptr_t)ws & 15) || !cut) nseg = 1;
     float* states = nullptr;
     int* flags = nullptr;
     unsigned grid = (unsigned)sequences;
@@ -99,15 +99,23 @@ int launch_chunked(const void* r, const void* k, const void* v, const void* w, c
         hipLaunchKernelGGL((wkv6_seg_fold_kernel<2, false>), dim3(4, 2, (unsigned)sequences), dim3(256), 0, st, states, nseg);
     }
     // Up to 256 tokens in one or two parts (the tile kernel is ahead of the chunked one at every size measured, 3 to 768 sequences of 33 to 256 tokens in
-    // all types: 1.03 to 1.8 times, least where a second part is nearly empty); more tokens, and rows off 4 bytes, are the chunked kernel's.
+    // all types: 1.03 to 1.8 times, least where a second part is nearly empty); more tokens, and calls that ask for it (vrwkv_wkv6_fwd_whole),
+    // are the chunked kernel's.
     const FwdTileArgs tile{r, k, v, w, u, y, T, C, H, (int)sequences, nseg, states, flags};
-    if (nseg == 1 && T <= TILE_TOKENS && aligned) {
+    if (nseg == 1 && T <= TILE_TOKENS && !whole) {
+        if constexpr (sizeof(IO) == 2) {
+            if (loose) {
+                hipLaunchKernelGGL((wkv6_fwd_tile_kernel<IO, WT, EW, false, true>), dim3(grid), dim3(64 * PART_WAVES), 0, st, tile);
+                return check_launch("wkv6_fwd (tile, rows off 4 bytes)");
+            }
+        }
         hipLaunchKernelGGL((wkv6_fwd_tile_kernel<IO, WT, EW, false>), dim3(grid), dim3(64 * PART_WAVES), 0, st, tile);
         return check_launch("wkv6_fwd (tile)");
     }
     if constexpr (type_code<IO> == VRWKV_BF16) {
         if (nseg > 1 && parts) {
-            hipLaunchKernelGGL((wkv6_fwd_tile_kernel<IO, WT, EW, true>), dim3(grid), dim3(64 * PART_WAVES), 0, st, tile);
+            if (loose) hipLaunchKernelGGL((wkv6_fwd_tile_kernel<IO, WT, EW, true, true>), dim3(grid), dim3(64 * PART_WAVES), 0, st, tile);
+            else hipLaunchKernelGGL((wkv6_fwd_tile_kernel<IO, WT, EW, true>), dim3(grid), dim3(64 * PART_WAVES), 0, st, tile);
             return check_launch("wkv6_fwd (tile, segments)");
         }
     }
@@ -120,10 +128,10 @@ bool force_scalar() { return option(OPT_WKV6_FWD_SCALAR) != 0; }   // testing ov
 
 template <typename IO, typename WT>
 int launch_any(const void* r, const void* k, const void* v, const void* w, const float* u, float* y,
-               void* ws, size_t ws_bytes, int B, int T, int C, int H, bool w_is_ew, hipStream_t st) {
+               void* ws, size_t ws_bytes, int B, int T, int C, int H, bool w_is_ew, bool whole, hipStream_t st) {
     if (force_scalar()) return launch_scalar<IO, WT>(r, k, v, w, u, y, B, T, C, H, w_is_ew, st);
-    return w_is_ew ? launch_chunked<IO, WT, true>(r, k, v, w, u, y, ws, ws_bytes, B, T, C, H, st)
-                   : launch_chunked<IO, WT, false>(r, k, v, w, u, y, ws, ws_bytes, B, T, C, H, st);
+    return w_is_ew ? launch_chunked<IO, WT, true>(r, k, v, w, u, y, ws, ws_bytes, B, T, C, H, whole, st)
+                   : launch_chunked<IO, WT, false>(r, k, v, w, u, y, ws, ws_bytes, B, T, C, H, whole, st);
 }
 
 }  // namespace
@@ -159,7 +167,7 @@ extern "C" int vrwkv_wkv6_fwd_phases(const void* r, const void* k, const void* v
                        static_cast<unsigned long long*>(stamps));
     // (sequences that vrwkv_wkv6_fwd leaves to the tile kernel: y is that one's)
     if (T <= TILE_TOKENS)
-        return launch_any<__hip_bfloat16, float>(r, k, v, w, u, y, nullptr, 0, B, T, C, H, false, static_cast<hipStream_t>(hip_stream));
+        return launch_any<__hip_bfloat16, float>(r, k, v, w, u, y, nullptr, 0, B, T, C, H, false, false, static_cast<hipStream_t>(hip_stream));
     return check_launch("wkv6_fwd_phases");
 }
 
@@ -172,9 +180,10 @@ extern "C" size_t vrwkv_wkv6_fwd_workspace_bytes(int B, int T, int C, int H) {
                      SEG_FLOATS);
 }
 
-extern "C" int vrwkv_wkv6_fwd(const void* r, const void* k, const void* v, const void* w, const float* u,
-                              float* y, int B, int T, int C, int H, int rkv_dtype, int w_dtype, int w_is_ew,
-                              void* workspace, size_t workspace_bytes, void* hip_stream) {
+namespace vrwkv {
+namespace {
+int forward(const void* r, const void* k, const void* v, const void* w, const float* u, float* y, int B, int T, int C, int H, int rkv_dtype,
+            int w_dtype, int w_is_ew, bool whole, void* workspace, size_t workspace_bytes, void* hip_stream) {
     int rc = validate(B, T, C, H, rkv_dtype, w_dtype);
     if (rc != VRWKV_OK) return rc;
     if (!r || !k || !v || !w || !u || !y) {
@@ -191,15 +200,27 @@ extern "C" int vrwkv_wkv6_fwd(const void* r, const void* k, const void* v, const
     const bool ew = w_is_ew != 0;
     switch (rkv_dtype) {
         case VRWKV_F32:
-            return launch_any<float, float>(r, k, v, w, u, y, workspace, workspace_bytes, B, T, C, H, ew, st);
+            return launch_any<float, float>(r, k, v, w, u, y, workspace, workspace_bytes, B, T, C, H, ew, whole, st);
         case VRWKV_BF16:
             return w_dtype == VRWKV_F32
-                       ? launch_any<__hip_bfloat16, float>(r, k, v, w, u, y, workspace, workspace_bytes, B, T, C, H, ew, st)
-                       : launch_any<__hip_bfloat16, __hip_bfloat16>(r, k, v, w, u, y, workspace, workspace_bytes, B, T, C, H, ew, st);
+                       ? launch_any<__hip_bfloat16, float>(r, k, v, w, u, y, workspace, workspace_bytes, B, T, C, H, ew, whole, st)
+                       : launch_any<__hip_bfloat16, __hip_bfloat16>(r, k, v, w, u, y, workspace, workspace_bytes, B, T, C, H, ew, whole, st);
         case VRWKV_F16:
             return w_dtype == VRWKV_F32
-                       ? launch_any<__half, float>(r, k, v, w, u, y, workspace, workspace_bytes, B, T, C, H, ew, st)
-                       : launch_any<__half, __half>(r, k, v, w, u, y, workspace, workspace_bytes, B, T, C, H, ew, st);
+                       ? launch_any<__half, float>(r, k, v, w, u, y, workspace, workspace_bytes, B, T, C, H, ew, whole, st)
+                       : launch_any<__half, __half>(r, k, v, w, u, y, workspace, workspace_bytes, B, T, C, H, ew, whole, st);
     }
     return VRWKV_UNSUPPORTED_DTYPE;
+}
+}  // namespace
+}  // namespace vrwkv
+
+extern "C" int vrwkv_wkv6_fwd(const void* r, const void* k, const void* v, const void* w, const float* u,
+                              float* y, int B, int T, int C, int H, int rkv_dtype, int w_dtype, int w_is_ew,
+                              void* workspace, size_t workspace_bytes, void* hip_stream) {
+    return forward(r, k, v, w, u, y, B, T, C, H, rkv_dtype, w_dtype, w_is_ew, false, workspace, workspace_bytes, hip_stream);
+}
+extern "C" int vrwkv_wkv6_fwd_whole(const void* r, const void* k, const void* v, const void* w, const float* u, float* y,
+                                    int B, int T, int C, int H, int rkv_dtype, int w_dtype, int w_is_ew, void* hip_stream) {
+    return forward(r, k, v, w, u, y, B, T, C, H, rkv_dtype, w_dtype, w_is_ew, true, nullptr, 0, hip_stream);
 }

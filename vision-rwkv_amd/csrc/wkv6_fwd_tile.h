@@ -45,7 +45,8 @@ struct FwdTileArgs {
     const int* seg_flags;
 };
 
-template <typename IO, typename WT, bool W_IS_EW, bool SEG>
+// LOOSE: 16-bit rows that do not lie on 4 bytes, fetched element by element (the same results, in a kernel of its own: the packing takes registers).
+template <typename IO, typename WT, bool W_IS_EW, bool SEG, bool LOOSE = false>
 __global__ __launch_bounds__(64 * PART_WAVES, 4)
 void wkv6_fwd_tile_kernel(FwdTileArgs A)
 {
@@ -98,9 +99,18 @@ void wkv6_fwd_tile_kernel(FwdTileArgs A)
         constexpr int pieces = sizeof(raw[0]) / 16;
         const unsigned vo = ((unsigned)c16 * C + 8 * g4) * es, so = (unsigned)(t0 + 16 * wave) * C * es;
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+        for (int kb = 0; kb < 2; ++kb) {
+            if constexpr (LOOSE && pieces == 1) {
+                unsigned e8[8];
 #pragma unroll
-            for (int i = 0; i < pieces; ++i) raw[kb][i] = BufRaw<16>::ld(rs, vo + 32u * kb * es + 16u * i, so);
+                for (int e = 0; e < 8; ++e) e8[e] = (unsigned short)BufRaw<2>::ld(rs, vo + 64u * kb + 2u * e, so);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) raw[kb][0][i] = e8[2 * i] | e8[2 * i + 1] << 16;
+            } else {
+#pragma unroll
+                for (int i = 0; i < pieces; ++i) raw[kb][i] = BufRaw<16>::ld(rs, vo + 32u * kb * es + 16u * i, so);
+            }
+        }
     };
     // y of the wave's tokens: value channels 16 vt + 4 g4 .. + 3 of token c16
     auto y_lane = [&]() { return ((unsigned)c16 * C + 4 * g4) * 4u; };

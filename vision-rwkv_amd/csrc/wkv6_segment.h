@@ -66,7 +66,7 @@ inline int wkv6_segments(long long sequences, int nchunk, int cus, const SegCost
 //         120 of 33                    98 | 2 95, 4 99
 // bf16 sequences can also be cut into segments of 128 tokens, one part of the tile kernel each (wkv6_fwd_tile.h): `parts`.  That cut's time is estimated
 // from the segments, all of them and those of a sequence (the scan); for a few sequences finer segments of the chunked kernels are ahead (3 of 10 chunks
-// 16.5 against 20.3).  us, uncut | segments (the 128-token cut in brackets):
+// 16.5 against 20.3), and where the others leave a sequence whole it has to be a fifth faster by the estimate, which is that far off (192 of 13).  us, uncut | segments (the 128-token cut in brackets):
 //          24 of 130                  354 | 10 65, 17 61, 26 76, [33] 62            192 of 32    94 | 4 95, [8] 95, 11 119
 //          48 of 64                   174 | 8 59, 10 61, [16] 55, 32 81             192 of 13    41 | 2 58, [4] 50, 5 56
 //          96 of 19                    56 | 3 54, [5] 37, 10 54                      96 of 10    32 | 2 36, [3] 36, 5 35
@@ -88,7 +88,7 @@ inline int wkv6_fwd_segments(long long sequences, int nchunk, int cus, const Fwd
     if (parts) {
         const int cps = std::max(4, (nchunk + SEG_MAX - 1) / SEG_MAX), nseg = (nchunk + cps - 1) / cps;
         const double t = std::max(19.0 + 0.45 * nseg, 15.0 + 0.25 * nseg + 0.052 * (double)(sequences * nseg));
-        *parts = t < (best == 1 ? 0.95 : 1.0) * best_time && cps * LC <= 2 * 128;
+        *parts = t < (best == 1 ? 0.84 : 1.0) * best_time && cps * LC <= 2 * 128;
         if (*parts) return nseg;
     }
     const int cps = (nchunk + best - 1) / best;

@@ -278,8 +278,8 @@ def wkv6_forward(B, T, C, H, r, k, v, w, u, w_is_ew=False, out=None, whole=False
     that dtype, u (H,64); returns y (B,T,C) fp32.  With w_is_ew=False, w is the raw decay logit
     (the kernel applies d = exp(-exp(w))); with True it is ew = -exp(w_raw) as the reference
     extension receives it.  Sequences of more than 256 tokens are cut into segments where there are few of them, by their
-    number and length; the last bits of y then depend on how many sequences there are.  whole: none is cut (a call without
-    workspace), and they do not.  (Either is equally far from float64, 5.0e-6 in bf16 at 300 to 1024 tokens.)"""
+    number and length; the last bits of y then depend on how many sequences there are.  whole: none is cut and all go 32 tokens at
+    a time, and they do not.  (Either is equally far from float64, 5.0e-6 in bf16 at 300 to 1024 tokens.)"""
     for t, n in ((r, "r"), (k, "k"), (v, "v"), (w, "w"), (u, "u")):
         _check_input(t, n)
     if tuple(r.shape) != (B, T, C) or k.shape != r.shape or v.shape != r.shape or w.shape != r.shape:
@@ -296,7 +296,12 @@ def wkv6_forward(B, T, C, H, r, k, v, w, u, w_is_ew=False, out=None, whole=False
          else _check_out(out, "y", (B, T, C), torch.float32, r))      # the reference passes y in (wkv6_op.cpp:7-9)
     if y.numel() == 0:
         return y
-    ws_bytes = 0 if whole else L.vrwkv_wkv6_fwd_workspace_bytes(B, T, C, H)
+    if whole:
+        with _on(r.device):
+            _lib.check(L.vrwkv_wkv6_fwd_whole(r.data_ptr(), k.data_ptr(), v.data_ptr(), w.data_ptr(), uf.data_ptr(), y.data_ptr(), B, T, C, H,
+                                              _DT[r.dtype], _DT[w.dtype], 1 if w_is_ew else 0, _stream_ptr(r.device)))
+        return y
+    ws_bytes = L.vrwkv_wkv6_fwd_workspace_bytes(B, T, C, H)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=r.device) if ws_bytes else None
     with _on(r.device):
         _lib.check(L.vrwkv_wkv6_fwd(r.data_ptr(), k.data_ptr(), v.data_ptr(), w.data_ptr(), uf.data_ptr(),
@@ -368,7 +373,8 @@ class WKV_6(torch.autograd.Function):
     # network by 4e-4 at most.  So a 16-bit forward that autograd records stays whole up to 33 chunks -- the 32 x 32 patches of a
     # 512 x 512 image and a class token -- and a sample's y is the same in any batch; that costs up to 66 us a layer (3 / 24 / 96
     # sequences of 1056 tokens: 92 / 94 / 95 us whole, 26 / 35 / 67 cut).  Longer chains cost more (2048 tokens: 175 whole, 34 to 115
-    # cut) and are cut.  The backward is cut from 257 tokens on in either type: gradients depend on the batch there, by 1.4e-2 in
+    # cut) and are cut.  For the same reason it takes up to 256 tokens 32 at a time, not as one or two products: with those the gradients
+    # of VRWKV6-B (64 images, 196 tokens) move by 3.3e-2 at a last-bit difference of 7e-6 in y (62 us a layer of 257, 46 of 243).  The backward is cut from 257 tokens on in either type: gradients depend on the batch there, by 1.4e-2 in
     # 16 bits.
     @staticmethod
     def stays_whole(T, dtype):
