@@ -247,6 +247,34 @@ def test_decay_regimes_mixed_over_the_heads_of_one_call(ops, seed, B, T, H, dtyp
             assert e <= TOL, (name, e)
 
 
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 32, 33, 96, 127, 128, 161, 193, 224, 225, 256])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_gradients_of_sequences_as_one_or_two_products(ops, T, dtype):
+    """Against the sequential sweeps (5e-7 of the norm).  gr, gk, gv: a rounding of 2^-18 each in D, rf, kf and the state, 1.6e-5 at most.  gw sums that of up
+    to T tokens, with signs that are as good as random, times its own decay.  Decays of 1.4 a token leave the range of a part, single strong tokens do not."""
+    B, H = 2, 2
+    C = 64 * H
+    g = torch.Generator(device="cuda").manual_seed(T)
+    r, k, v = (torch.randn(B, T, C, generator=g, device="cuda").to(dtype) for _ in range(3))
+    gy, u = torch.randn(B, T, C, generator=g, device="cuda"), torch.randn(H, 64, generator=g, device="cuda") * 0.3
+    noise = torch.randn(B, T, C, generator=g, device="cuda") * 0.3
+    for w_mean, spikes in ((-3.0, False), (-1.0, False), (0.3, False), (-3.0, True)):
+        w = w_mean + noise
+        if spikes:
+            w[1, 5::40, 64:] = 2.3
+        w = w.to(dtype)
+        got = ops.wkv6_backward(B, T, C, H, r, k, v, w, u, gy)
+        with ops.option("wkv6_bwd_scalar", 1):
+            ref = ops.wkv6_backward(B, T, C, H, r, k, v, w, u, gy)
+        for x, y in zip(got[:3] + got[4:], ref[:3] + ref[4:]):
+            assert (x - y).norm() <= 1.6e-5 * y.norm(), (w_mean, spikes)
+        terms = w.float().exp() * ((r.float() * ref[0]).abs() + (k.float() * ref[1]).abs())
+        assert (got[3] - ref[3]).norm() <= 1.6e-5 * T ** 0.5 * terms.norm(), (w_mean, spikes)
+        if dtype != torch.float32:
+            off = [torch.empty(a.numel() + 1, dtype=dtype, device="cuda")[1:].view_as(a).copy_(a) for a in (r, k, v, w)]
+            assert all(torch.equal(x, y) for x, y in zip(ops.wkv6_backward(B, T, C, H, *off, u, gy), got))
+
+
 @pytest.mark.parametrize("T,segments", [(33, 2), (65, 3), (200, 3), (250, 8), (577, 5)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_backward_of_sequences_cut_into_segments(ops, T, segments, dtype):

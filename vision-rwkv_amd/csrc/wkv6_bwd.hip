@@ -15,7 +15,7 @@
 //             a_n = r_n[j] (S_n gy_n)[j],  b_n = k_n[j] (G_{n+1} v_n)[j]
 // (the last line follows from X_n = sum_i S_n[j,i] G_n[j,i]:  d_n * dL/dd_n = X_n - a_n = X_{n+1} - b_n;
 //  gw is the gradient w.r.t. the raw decay logit, as in wkv6_cuda.cu:248,277.)
-#include "wkv6_bwd_sweep.h"
+#include "wkv6_bwd_tile.h"
 #include <cstdlib>
 #include <type_traits>
 
@@ -63,6 +63,15 @@ int segments(int B, int T, int H) {
     return forced > 0 ? 1 : wkv6_segments((long long)B * H, nchunk, device_cus(), SEG_BWD);
 }
 
+// Uncut sequences in one or two products (wkv6_bwd_tile.h).  By length and type alone, so that a sample's gradients do not depend on the batch.  Two parts
+// are three steps whatever the second one holds: up to 160 tokens (fp32, which spills, 192) the sweeps' five (six) chunks are ahead where compute units have
+// two sequences each.  us, sweeps -> products: 64 x 12 sequences of 128 tokens, bf16 119 -> 73, fp32 128 -> 90; of 129, fp16 141 -> 141, fp32 148 -> 166; of
+// 196, bf16 197 -> 155, fp16 195 -> 167, fp32 213 -> 193; of 256, fp16 232 -> 180, fp32 254 -> 213; 22 x 12 of 129, fp16 85 -> 92; of 161, fp16 99 -> 97,
+// fp32 99 -> 108; of 196, fp32 113 -> 119; 8 x 3 of 196, bf16 81 -> 50, fp32 77 -> 58.
+bool bwd_tile_takes(int T, int rkv_dtype) {
+    return T <= PART || (T > (rkv_dtype == VRWKV_F32 ? 192 : 160) && T <= BWD_TILE_TOKENS);
+}
+
 // Workspace: [fp32 sums gr, gk, gv (16-bit results only)] [gw (16-bit decay logits only)] [a of both passes] [partial gu] [states] [flags]
 struct Plan {
     bool out16, w16;
@@ -97,18 +106,21 @@ int launch_all(const void* r, const void* k, const void* v, const void* w, const
     A.a_size = p.n;
     A.gu_part = take((size_t)B * p.nseg * C);
     q = ws + (((size_t)(q - ws) + 3) & ~(size_t)3);      // states: 16-byte aligned
-    // gv leaves the sweep in pieces of four channels; where its 16-bit rows do not lie on 4 bytes, the sums are rounded afterwards
-    const bool apart = p.out16 && ((uintptr_t)gv & 3);
+    // results leave the kernels in pieces of several channels; where 16-bit rows do not lie on 4 bytes, the sums are rounded afterwards
+    const bool apart = p.out16 && (((uintptr_t)gr | (uintptr_t)gk | (uintptr_t)gv) & 3), w_apart = p.w16 && ((uintptr_t)gw & 3);
     if (apart) { A.gr = A.pr; A.gk = A.pk; A.gv = A.pv; }
-    A.T = T; A.C = C; A.H = H; A.sequences = B * H; A.nseg = p.nseg; A.out16 = p.out16 && !apart; A.w16 = p.w16;
+    if (w_apart) A.gw = A.pw;
+    A.T = T; A.C = C; A.H = H; A.sequences = B * H; A.nseg = p.nseg; A.out16 = p.out16 && !apart; A.w16 = p.w16 && !w_apart;
     A.seg_ws = q;
     int* flags = reinterpret_cast<int*>(q + (size_t)A.sequences * p.nseg * BWD_SEG_FLOATS);
     A.seg_flags = flags;
     const IO *rr = static_cast<const IO*>(r), *kk = static_cast<const IO*>(k), *vv = static_cast<const IO*>(v);
     const WT* ww = static_cast<const WT*>(w);
     int part_rows = B;
+    const dim3 rg((unsigned)((p.n + 1023) / 1024 < 8192 ? (p.n + 1023) / 1024 : 8192));
+    auto round_w = [&]() { hipLaunchKernelGGL((round_kernel<WT>), rg, dim3(256), 0, st, A.pw, static_cast<WT*>(gw), p.n); };
     auto round_rkv = [&]() {
-        const dim3 rg((unsigned)((p.n + 1023) / 1024 < 8192 ? (p.n + 1023) / 1024 : 8192)), block(256);
+        const dim3 block(256);
         hipLaunchKernelGGL((round_kernel<IO>), rg, block, 0, st, A.pr, static_cast<IO*>(gr), p.n);
         hipLaunchKernelGGL((round_kernel<IO>), rg, block, 0, st, A.pk, static_cast<IO*>(gk), p.n);
         hipLaunchKernelGGL((round_kernel<IO>), rg, block, 0, st, A.pv, static_cast<IO*>(gv), p.n);
@@ -121,9 +133,19 @@ int launch_all(const void* r, const void* k, const void* v, const void* w, const
                                (long long)A.sequences, p.nseg);
             hipLaunchKernelGGL((wkv6_seg_fold_kernel<4, true>), dim3(4, 4, (unsigned)A.sequences), dim3(256), 0, st, q, p.nseg);
         }
-        hipLaunchKernelGGL((wkv6_bwd_sweep_kernel<IO, WT, EW>), dim3(grid), dim3(512), 0, st, A);
+        if (p.nseg == 1 && bwd_tile_takes(T, type_code<IO>)) {
+            bool loose = false;
+            if constexpr (sizeof(IO) == 2) {
+                loose = (((uintptr_t)r | (uintptr_t)k | (uintptr_t)v | (uintptr_t)w) & 3) != 0;
+                if (loose) hipLaunchKernelGGL((wkv6_bwd_tile_kernel<IO, WT, EW, true>), dim3(grid), dim3(64 * PART_WAVES), 0, st, A);
+            }
+            if (!loose) hipLaunchKernelGGL((wkv6_bwd_tile_kernel<IO, WT, EW>), dim3(grid), dim3(64 * PART_WAVES), 0, st, A);
+        } else {
+            hipLaunchKernelGGL((wkv6_bwd_sweep_kernel<IO, WT, EW>), dim3(grid), dim3(512), 0, st, A);
+        }
         part_rows = B * p.nseg;
         if (apart) round_rkv();
+        if (w_apart) round_w();
     } else {
         const dim3 grid(A.sequences), block(256);
         // descending pass first (writes), ascending pass second (accumulates), as in the forward
@@ -133,9 +155,8 @@ int launch_all(const void* r, const void* k, const void* v, const void* w, const
         hipLaunchKernelGGL((wkv6_bwd_seq_s<IO, WT, 0, EW>), grid, block, 0, st, rr, kk, vv, ww, u, gy, A.pr, A.a, A.gu_part, T, C, H);
         hipLaunchKernelGGL((wkv6_bwd_seq_g<IO, WT, 0, EW>), grid, block, 0, st, rr, kk, vv, ww, u, gy, A.a, A.pk, A.pw, T, C, H);
         hipLaunchKernelGGL((wkv6_bwd_seq_v<IO, WT, 0, EW>), grid, block, 0, st, rr, kk, ww, u, gy, A.pv, T, C, H);
-        const dim3 rg((unsigned)((p.n + 1023) / 1024 < 8192 ? (p.n + 1023) / 1024 : 8192));
         if (p.out16) round_rkv();
-        if (p.w16) hipLaunchKernelGGL((round_kernel<WT>), rg, block, 0, st, A.pw, static_cast<WT*>(gw), p.n);
+        if (p.w16) round_w();
     }
     // torch.sum(gu, 0), vrwkv6.py:69
     launch_batch_sum(A.gu_part, gu, nullptr, SumOut((float*)nullptr), part_rows, C, st);

@@ -252,25 +252,18 @@ __device__ __forceinline__ void matrix_stage(const __bf16 (*Qh)[BP], const __bf1
     }
 }
 
+// One (b,h) sequence, or the segment `seg` of one, by a workgroup of eight waves (no wave may still be using L).
 template <typename IO, typename WT, bool W_IS_EW>
-__global__ __launch_bounds__(512, 4)                 // four waves per SIMD: at most 128 registers
-void wkv6_bwd_sweep_kernel(BwdArgs A)
+__device__ __forceinline__
+void bwd_sweep_sequence(const BwdArgs& A, BwdLds<!__is_same(IO, __hip_bfloat16)>& L, int& sFlag, int bh, int seg)
 {
     constexpr bool EXACT = __is_same(IO, __hip_bfloat16);
     constexpr unsigned ES = (unsigned)sizeof(IO), WS = (unsigned)sizeof(WT);
-    using Lds = BwdLds<!EXACT>;
-    __shared__ Lds L;
-    __shared__ int sFlag;
-    static_assert(sizeof(Lds) >= 2 * SEQ_STAGE_FLOATS * sizeof(float), "the sequential sweeps' staging must fit");
+    static_assert(sizeof(BwdLds<!EXACT>) >= 2 * SEQ_STAGE_FLOATS * sizeof(float), "the sequential sweeps' staging must fit");
 
     const int lane = threadIdx.x & 63;                                    // channel in the element-wise and closing stages
     const int w8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // token group there (tokens 4 w8 .. 4 w8 + 3 of the chunk)
     const int T = A.T, C = A.C, nseg = A.nseg;
-    int bh = blockIdx.x, seg = 0;
-    if (nseg > 1) {
-        seg_of_block(blockIdx.x, nseg, bh, seg);
-        if (bh >= A.sequences) return;
-    }
     const int b = bh / A.H, h = bh % A.H;
     const size_t base = (size_t)b * T * C + (size_t)h * HN;
     const int cps = ((T + LC - 1) / LC + nseg - 1) / nseg, c0 = seg * cps;
@@ -661,6 +654,20 @@ void wkv6_bwd_sweep_kernel(BwdArgs A)
             if (WS == 2 && A.w16) static_cast<WT*>(A.gw)[o] = from_f32<WT>(A.pw[o]);
         }
     }
+}
+
+template <typename IO, typename WT, bool W_IS_EW>
+__global__ __launch_bounds__(512, 4)                 // four waves per SIMD: at most 128 registers
+void wkv6_bwd_sweep_kernel(BwdArgs A)
+{
+    __shared__ BwdLds<!__is_same(IO, __hip_bfloat16)> L;
+    __shared__ int sFlag;
+    int bh = blockIdx.x, seg = 0;
+    if (A.nseg > 1) {
+        seg_of_block(blockIdx.x, A.nseg, bh, seg);
+        if (bh >= A.sequences) return;
+    }
+    bwd_sweep_sequence<IO, WT, W_IS_EW>(A, L, sFlag, bh, seg);
 }
 
 }  // namespace wkv6_detail
