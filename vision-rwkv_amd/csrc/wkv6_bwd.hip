@@ -16,6 +16,7 @@
 // (the last line follows from X_n = sum_i S_n[j,i] G_n[j,i]:  d_n * dL/dd_n = X_n - a_n = X_{n+1} - b_n;
 //  gw is the gradient w.r.t. the raw decay logit, as in wkv6_cuda.cu:248,277.)
 #include "wkv6_bwd_tile.h"
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -53,16 +54,6 @@ void round_kernel(const float* __restrict__ x, OT* __restrict__ y, size_t n) {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) y[i] = from_f32<OT>(x[i]);
 }
 
-// Segments per sequence of a call (1: not cut); OPT_WKV6_SEGMENTS forces a number (testing).
-int segments(int B, int T, int H) {
-    const int nchunk = (T + LC - 1) / LC, forced = option(OPT_WKV6_SEGMENTS);
-    if (forced > 0 && (long long)B * H <= SEG_SEQUENCES) {
-        const int n = forced < nchunk ? forced : nchunk, cps = (nchunk + n - 1) / n;
-        return (nchunk + cps - 1) / cps;
-    }
-    return forced > 0 ? 1 : wkv6_segments((long long)B * H, nchunk, device_cus(), SEG_BWD);
-}
-
 // Uncut sequences in one or two products (wkv6_bwd_tile.h).  By length and type alone, so that a sample's gradients do not depend on the batch.  Two parts
 // are three steps whatever the second one holds: up to 160 tokens (fp32, which spills, 192) the sweeps' five (six) chunks are ahead where compute units have
 // two sequences each.  us, sweeps -> products: 64 x 12 sequences of 128 tokens, bf16 119 -> 73, fp32 128 -> 90; of 129, fp16 141 -> 141, fp32 148 -> 166; of
@@ -72,9 +63,32 @@ bool bwd_tile_takes(int T, int rkv_dtype) {
     return T <= PART || (T > (rkv_dtype == VRWKV_F32 ? 192 : 160) && T <= BWD_TILE_TOKENS);
 }
 
+// Segments per sequence of a call (1: not cut); OPT_WKV6_SEGMENTS forces a number (testing).  parts: of 128 tokens, one part of wkv6_bwd_tile.h each.  Those
+// take three launches and BWD_PARTS_US whatever the sequences' number and length, as long as every segment has a compute unit and there are not more than
+// eight in a sequence (each folds the states of all others); the sweeps are ahead where they find short segments for all of them.  us, sweeps -> parts,
+// bf16 / fp32: 48 sequences of 577 tokens 80 -> 55 / 79 -> 65, of 400 84 -> 51 / 85 -> 60, 24 of 1024 87 -> 51 / 92 -> 62, 24 of 577 57 -> 47 / 59 -> 58,
+// 24 of 300 43 -> 45 / 43 -> 55, 3 of 577 41 -> 44 / 42 -> 53.
+constexpr int BWD_TILE_SEGMENTS = 8;
+constexpr double BWD_PARTS_US[3] = {62., 52., 55.};      // VRWKV_F32, VRWKV_BF16, VRWKV_F16
+int segments(int B, int T, int H, int rkv_dtype, bool& parts) {
+    const int nchunk = (T + LC - 1) / LC, forced = option(OPT_WKV6_SEGMENTS);
+    const long long sequences = (long long)B * H;
+    parts = false;
+    if (forced > 0 && sequences <= SEG_SEQUENCES) {
+        const int n = forced < nchunk ? forced : nchunk, cps = (nchunk + n - 1) / n, nseg = (nchunk + cps - 1) / cps;
+        parts = nseg > 1 && nseg <= BWD_TILE_SEGMENTS && cps * LC <= PART;
+        return nseg;
+    }
+    if (forced > 0) return 1;
+    double us;
+    const int nseg = wkv6_segments(sequences, nchunk, device_cus(), SEG_BWD, us), nparts = (nchunk + PART / LC - 1) / (PART / LC);
+    parts = nchunk > 8 && nparts <= BWD_TILE_SEGMENTS && (sequences + 7) / 8 * 8 * nparts <= device_cus() && us > BWD_PARTS_US[rkv_dtype];
+    return parts ? nparts : nseg;
+}
+
 // Workspace: [fp32 sums gr, gk, gv (16-bit results only)] [gw (16-bit decay logits only)] [a of both passes] [partial gu] [states] [flags]
 struct Plan {
-    bool out16, w16;
+    bool out16, w16, parts;
     int nseg;
     size_t n, sums, states, bytes;                       // elements of a tensor; floats in front of `a`; bytes of the state block
 };
@@ -82,10 +96,12 @@ Plan plan(int B, int T, int C, int H, int rkv_dtype, int w_dtype, int grad_dtype
     Plan p;
     p.out16 = grad_dtypes_of_inputs && rkv_dtype != VRWKV_F32;
     p.w16 = grad_dtypes_of_inputs && w_dtype != VRWKV_F32;
-    p.nseg = cut ? segments(B, T, H) : 1;
+    p.nseg = 1;
+    p.parts = false;
+    if (cut) p.nseg = segments(B, T, H, rkv_dtype, p.parts);
     p.n = (size_t)B * T * C;
     p.sums = (p.out16 ? 3 * p.n : 0) + (p.w16 ? p.n : 0);
-    p.states = seg_bytes((long long)B * H, p.nseg, BWD_SEG_FLOATS);
+    p.states = seg_bytes((long long)B * H, p.nseg, BWD_SEG_FLOATS * (p.parts ? 2 : 1));
     p.bytes = ((p.sums + 2 * p.n + (size_t)B * p.nseg * C + 3) & ~(size_t)3) * sizeof(float) + p.states;
     return p;
 }
@@ -112,7 +128,8 @@ int launch_all(const void* r, const void* k, const void* v, const void* w, const
     if (w_apart) A.gw = A.pw;
     A.T = T; A.C = C; A.H = H; A.sequences = B * H; A.nseg = p.nseg; A.out16 = p.out16 && !apart; A.w16 = p.w16 && !w_apart;
     A.seg_ws = q;
-    int* flags = reinterpret_cast<int*>(q + (size_t)A.sequences * p.nseg * BWD_SEG_FLOATS);
+    A.seg_own = q + (size_t)A.sequences * p.nseg * BWD_SEG_FLOATS;
+    int* flags = reinterpret_cast<int*>(p.parts ? A.seg_own + (A.seg_own - q) : A.seg_own);
     A.seg_flags = flags;
     const IO *rr = static_cast<const IO*>(r), *kk = static_cast<const IO*>(k), *vv = static_cast<const IO*>(v);
     const WT* ww = static_cast<const WT*>(w);
@@ -129,11 +146,15 @@ int launch_all(const void* r, const void* k, const void* v, const void* w, const
         unsigned grid = (unsigned)A.sequences;
         if (p.nseg > 1) {
             grid = seg_grid(A.sequences, p.nseg);
-            hipLaunchKernelGGL((wkv6_bwd_seg_state_kernel<IO, WT, EW>), dim3(grid), dim3(256), 0, st, rr, kk, vv, ww, gy, q, flags, T, C, H,
+            if (p.parts)
+                hipLaunchKernelGGL((wkv6_bwd_part_state_kernel<IO, WT, EW>), dim3(grid), dim3(64 * PART_WAVES), 0, st, r, k, v, w, gy, q, flags, T, C, H,
+                                   A.sequences, p.nseg);
+            else
+                hipLaunchKernelGGL((wkv6_bwd_seg_state_kernel<IO, WT, EW>), dim3(grid), dim3(256), 0, st, rr, kk, vv, ww, gy, q, flags, T, C, H,
                                (long long)A.sequences, p.nseg);
-            hipLaunchKernelGGL((wkv6_seg_fold_kernel<4, true>), dim3(4, 4, (unsigned)A.sequences), dim3(256), 0, st, q, p.nseg);
+            if (!p.parts) hipLaunchKernelGGL((wkv6_seg_fold_kernel<4, true>), dim3(4, 4, (unsigned)A.sequences), dim3(256), 0, st, q, p.nseg);
         }
-        if (p.nseg == 1 && bwd_tile_takes(T, type_code<IO>)) {
+        if (p.nseg == 1 ? bwd_tile_takes(T, type_code<IO>) : p.parts) {
             bool loose = false;
             if constexpr (sizeof(IO) == 2) {
                 loose = (((uintptr_t)r | (uintptr_t)k | (uintptr_t)v | (uintptr_t)w) & 3) != 0;
@@ -226,7 +247,10 @@ using namespace vrwkv;
 
 extern "C" size_t vrwkv_wkv6_bwd_workspace_bytes(int B, int T, int C, int H) {
     if (B <= 0 || T <= 0 || C <= 0 || H <= 0) return 0;
-    return plan(B, T, C, H, VRWKV_F32, VRWKV_F32, 0).bytes;
+    // the same for every type: the largest of the plans
+    size_t bytes = 0;
+    for (int dt : {VRWKV_F32, VRWKV_BF16, VRWKV_F16}) bytes = std::max(bytes, plan(B, T, C, H, dt, VRWKV_F32, 0).bytes);
+    return bytes;
 }
 extern "C" size_t vrwkv_wkv6_bwd_like_workspace_bytes(int B, int T, int C, int H, int rkv_dtype, int w_dtype) {
     if (B <= 0 || T <= 0 || C <= 0 || H <= 0) return 0;

@@ -52,7 +52,8 @@ struct BwdArgs {
     float *pr, *pk, *pv, *pw;                        // fp32 sums of the upward sweep (the results themselves when they are fp32)
     float *a, *gu_part;                              // sequential fallback's (2, B,T,C) scratch; (B*nseg, C) partial gu
     size_t a_size;                                   // elements of a tensor
-    const float* seg_ws;                             // states entering the segments (nseg > 1)
+    const float* seg_ws;                             // states entering the segments (nseg > 1); wkv6_bwd_tile.h: those that the segments leave by themselves
+    float* seg_own;                                  // room for the former beside the latter
     const int* seg_flags;
     int T, C, H, sequences, nseg, out16, w16;
 };

@@ -55,8 +55,8 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
     constexpr unsigned RFH = 0, RFL = ARR, RBH = 2 * ARR, RBL = 3 * ARR, GYH = 4 * ARR, GYL = 5 * ARR;
     constexpr unsigned KFH = 0, KFL = ARR, KBH = 2 * ARR, KBL = 3 * ARR, VH = 4 * ARR, VL = 5 * ARR;
     constexpr unsigned LVH = 6 * ARR, LVL = 7 * ARR;                      // (KFH, KFL, RBH, RBL, GYH, GYL beside them)
-    // scaled states, row j: 64 value channels, head and tail; G of the second part's states from behind apart (formed while the other is still read)
-    constexpr unsigned ZS = 6 * ARR, ZG = 7 * ARR, ZG_BEHIND = 8 * ARR, ZTAIL = ARR / 2, TAB = 9 * ARR;
+    // scaled states, row j: 64 value channels, head and tail; apart the G that is formed or waits while the other is read
+    constexpr unsigned ZS = 6 * ARR, ZG = 7 * ARR, ZG_BEHIND = 8 * ARR, ZG_FRONT = ZG_BEHIND, ZTAIL = ARR / 2, TAB = 9 * ARR;
     struct Tables { float Tot[PART_WAVES][HN], Before[PART_WAVES][2][HN], Q[PART_WAVES][HN], X[2][HN]; };
     __shared__ __attribute__((aligned(16))) unsigned char lds[TAB + sizeof(Tables)];
     __shared__ int sFlag;
@@ -165,38 +165,46 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
     };
     constexpr std::integral_constant<bool, VSPLIT> v_split{};
     constexpr std::true_type is_split{};
-    const float* const seg_in = A.seg_ws + ((size_t)bh * nseg + seg) * BWD_SEG_FLOATS;
-    auto load_state = [&](const float* m, f32x4 (&X)[2]) {
+    // The states that enter the segment from the front (up) or from behind: those that the segments there leave by themselves, each over the decay of the
+    // segments in between.  (A launch that folds them first costs more for up to eight segments.)
+    auto local_state = [&](int s, int m, f32x4 (&X)[2]) {
+        const float* const p = A.seg_ws + ((size_t)bh * nseg + s) * BWD_SEG_FLOATS + m * SEG_STATE;
 #pragma unroll
-        for (int q = 0; q < 2; ++q) X[q] = *reinterpret_cast<const f32x4*>(m + seg_frag(jt, ct0 + q, lane));
+        for (int q = 0; q < 2; ++q) X[q] = *reinterpret_cast<const f32x4*>(p + seg_frag(jt, ct0 + q, lane));
+    };
+    auto segment_decay = [&](int s) { return A.seg_ws[((size_t)bh * nseg + s) * BWD_SEG_FLOATS + 4 * SEG_STATE + 16 * jt + c16]; };
+    auto entering = [&](bool up, f32x4 (&S)[2], f32x4 (&G)[2]) {
+        S[0] = S[1] = G[0] = G[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int count = up ? seg : nseg - 1 - seg, m = up ? 0 : 2;
+        constexpr int U = 4;
+#pragma unroll 1
+        for (int q = 0; q < count; q += U) {
+            f32x4 ls[U][2], lg[U][2];
+            float d[U];
+#pragma unroll
+            for (int i = 0; i < U; ++i)
+                if (q + i < count) {
+                    const int s = up ? q + i : nseg - 1 - q - i;
+                    local_state(s, m, ls[i]);
+                    local_state(s, m + 1, lg[i]);
+                    d[i] = segment_decay(s);
+                }
+#pragma unroll
+            for (int i = 0; i < U; ++i)
+                if (q + i < count) {
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        S[e] = S[e] * d[i] + ls[i][e];
+                        G[e] = G[e] * d[i] + lg[i][e];
+                    }
+                }
+        }
     };
 
     const float uj = A.u[h * HN + lane];
     float xrun = 0.f, c_both = 0.f, gu = 0.f;        // of channel `lane`: the sum of q behind the part; c of both parts; gu of channel gu_at
     int gu_at = 0;
     f32x4 XS[2], XG[2];
-    if (nseg > 1 && !bail) {
-        if (seg + 1 < nseg) {
-            // X at the segment's end: sum over the value channels of S G of both passes, the states that enter the next segment from the front with those
-            // that enter this one from behind
-            const float* const next = seg_in + BWD_SEG_FLOATS;
-            float x = 0.f;
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                f32x4 p[2], q[2];
-                load_state(next + i * SEG_STATE, p);
-                load_state(seg_in + (3 - i) * SEG_STATE, q);
-#pragma unroll
-                for (int m = 0; m < 2; ++m)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) x = fmaf(p[m][e], q[m][e], x);
-            }
-            x += __shfl_xor(x, 16);
-            x += __shfl_xor(x, 32);
-            if (lane < 16) L.X[wave >> 2][16 * jt + lane] = x;
-        }
-    }
-
 #pragma unroll 1
     for (int step = two ? 0 : 2; step < 3 && !bail; ++step) {
         const int part = step == 1 ? 1 : 0, t0 = first + (part ? n1 : 0), np = part ? n - n1 : n1, nb = (np + LC - 1) / LC;
@@ -208,6 +216,27 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
         fetch(A.r, t0, rraw, ES);
         fetch(A.gy, t0, graw, 4u);
         fetch(A.v, t0, vraw, ES);
+        f32x4 XD[2], YD[2], XU[2], YU[2];            // S and G that enter a segment from behind and from the front
+        if (nseg > 1) {
+            entering(false, XD, YD);
+            entering(true, XU, YU);
+            // X at the segment's end: sum over the value channels of S G of both passes
+            f32x4 ls[2], lg[2];
+            local_state(seg, 0, ls);
+            local_state(seg, 1, lg);
+            const float d = segment_decay(seg);
+            float x = 0.f;
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    x = fmaf(fmaf(XU[q][e], d, ls[q][e]), YD[q][e], x);
+                    x = fmaf(fmaf(YU[q][e], d, lg[q][e]), XD[q][e], x);
+                }
+            x += __shfl_xor(x, 16);
+            x += __shfl_xor(x, 32);
+            if (lane < 16) L.X[wave >> 2][16 * jt + lane] = x;
+        }
         const bool past = 16 * wave + c16 >= np;
         float x[2][8];                               // log2 decays summed over the wave's tokens, channel 32 kb + 8 g4 + e
         float c_part;
@@ -324,11 +353,9 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
                 XG[q] = __builtin_nondeterministic_value(XG[q]);
             }
         } else if (nseg > 1) {
-            f32x4 X[2];
-            load_state(seg_in + 2 * SEG_STATE, X);
-            put_state(c_part, X, ZS);
-            load_state(seg_in + 3 * SEG_STATE, X);
-            put_state(c_part, X, ZG);
+            put_state(c_part, XD, ZS);
+            put_state(c_part, YD, ZG);
+            put_state(c_part, YU, ZG_FRONT);
         }
         lds_barrier();
 
@@ -475,16 +502,10 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
             state_gkv(ZG_BEHIND, KF, gkd);
         } else if (nseg > 1) {
             state_gkv(ZG, KF, gkd);
+            state_gkv(ZG_FRONT, KB, gku);
             state_gr(grd);
-            f32x4 XU[2], XV[2];
-            load_state(seg_in, XU);
-            load_state(seg_in + SEG_STATE, XV);
-            lds_barrier();
+            lds_barrier();                           // (S from behind is read)
             put_state(c_part, XU, ZS);
-            put_state(c_part, XV, ZG);
-            lds_barrier();
-            renew();
-            state_gkv(ZG, KB, gku);
         }
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
@@ -570,7 +591,7 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
         gu += row_sums16(gu16, lane, gu_at);
         lds_barrier();
         {
-            if (nseg > 1 && seg + 1 < nseg) xrun = L.X[0][lane] + L.X[1][lane];
+            if (nseg > 1) xrun = L.X[0][lane] + L.X[1][lane];
             float after = 0.f, total = 0.f;
 #pragma unroll
             for (int g = 0; g < PART_WAVES; ++g) {
@@ -601,6 +622,21 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
         }
     }
     if (bail) {
+        if (nseg > 1) {
+            // the sweeps take the states that enter the segment from memory
+            float* const own = A.seg_own + ((size_t)bh * nseg + seg) * BWD_SEG_FLOATS;
+#pragma unroll 1
+            for (int m = 0; m < 4; m += 2) {
+                f32x4 S[2], G[2];
+                entering(m == 0, S, G);
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    *reinterpret_cast<f32x4*>(own + m * SEG_STATE + seg_frag(jt, ct0 + q, lane)) = S[q];
+                    *reinterpret_cast<f32x4*>(own + (m + 1) * SEG_STATE + seg_frag(jt, ct0 + q, lane)) = G[q];
+                }
+            }
+            A.seg_ws = A.seg_own;
+        }
         __syncthreads();
         bwd_sweep_sequence<IO, WT, W_IS_EW>(A, *reinterpret_cast<Sweep*>(lds), sFlag, bh, seg);
         return;
@@ -613,6 +649,144 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
 #pragma unroll
         for (int g = 0; g < PART_WAVES; ++g) x += L.Q[g][threadIdx.x];
         A.gu_part[((size_t)b * nseg + seg) * C + h * HN + threadIdx.x] = x;
+    }
+}
+
+// What every segment of up to 128 tokens leaves behind it in both directions by itself, S (k, v) and G (r, gy), with its decay and whether it is out of range:
+// wkv6_bwd_seg_state_kernel's results, a part at a time (two pairs of barriers in place of two for every 32 tokens; the up states' factors first, then, in
+// their place, the down states').  All exponents are <= 0.  One workgroup on a compute unit (136 KB of LDS), for calls that do not have more.
+template <typename IO, typename WT, bool W_IS_EW>
+__global__ __launch_bounds__(64 * PART_WAVES, 2)
+void wkv6_bwd_part_state_kernel(const void* r_, const void* k_, const void* v_, const void* w_, const float* gy_, float* ws, int* flags, int T, int C, int H,
+                                int sequences, int nseg)
+{
+    constexpr bool VSPLIT = !__is_same(IO, __hip_bfloat16);
+    constexpr unsigned ES = (unsigned)sizeof(IO), WS = (unsigned)sizeof(WT), ARR = PART * 128u;
+    constexpr unsigned KH = 0, KL = ARR, RH = 2 * ARR, RL = 3 * ARR, GYH = 4 * ARR, GYL = 5 * ARR, VH = 6 * ARR, VL = 7 * ARR, TAB = (VSPLIT ? 8 : 7) * ARR;
+    struct Tables { float Tot[PART_WAVES][HN], Before[PART_WAVES][2][HN]; };
+    __shared__ __attribute__((aligned(16))) unsigned char lds[TAB + sizeof(Tables)];
+    Tables& L = *reinterpret_cast<Tables*>(lds + TAB);
+    const int lane = threadIdx.x & 63, g4 = lane >> 4, c16 = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int bh, seg;
+    seg_of_block(blockIdx.x, nseg, bh, seg);
+    if (bh >= sequences) return;
+    const size_t base = (size_t)(bh / H) * T * C + (size_t)(bh % H) * HN;
+    const unsigned n_el = (unsigned)((size_t)(T - 1) * C + HN);
+    const int nchunk = (T + LC - 1) / LC, cps = (nchunk + nseg - 1) / nseg;
+    const int first = seg * cps * LC, n = min(cps * LC, T - first), nb = (n + LC - 1) / LC;
+    auto fetch = [&](const void* p, auto& raw, unsigned es) {
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(static_cast<const char*>(p) + base * es, n_el * es);
+        constexpr int pieces = sizeof(raw[0]) / 16;
+        const unsigned vo = ((unsigned)c16 * C + 8 * g4) * es, so = (unsigned)(first + 16 * wave) * C * es;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int i = 0; i < pieces; ++i) raw[kb][i] = BufRaw<16>::ld(rs, vo + 32u * kb * es + 16u * i, so);
+    };
+    u32x4 wraw[2][WS / 2], rraw[2][ES / 2], kraw[2][ES / 2], vraw[2][ES / 2], graw[2][2];
+    fetch(w_, wraw, WS);
+    fetch(k_, kraw, ES);
+    fetch(r_, rraw, ES);
+    fetch(v_, vraw, ES);
+    fetch(gy_, graw, 4u);
+    float x[2][8];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+        summed_decays<WT, W_IS_EW>(wraw[kb], 16 * wave + c16 >= n, x[kb]);
+        if (c16 == 15) {
+#pragma unroll
+            for (int hf = 0; hf < 2; ++hf)
+                *reinterpret_cast<f32x4*>(&L.Tot[wave][32 * kb + 8 * g4 + 4 * hf]) = f32x4{x[kb][4 * hf], x[kb][4 * hf + 1], x[kb][4 * hf + 2], x[kb][4 * hf + 3]};
+        }
+    }
+    auto store = [&](unsigned arr, int kb, const bf16x8& o) { *reinterpret_cast<bf16x8*>(lds + arr + row_chunk(16 * wave + c16, 4 * kb + g4)) = o; };
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+        float o8[8];
+        bf16x8 hi, lo;
+        widen8<float>(graw[kb], o8);
+        split8<true>(o8, hi, lo);
+        store(GYH, kb, hi);
+        store(GYL, kb, lo);
+        if constexpr (VSPLIT) {
+            widen8<IO>(vraw[kb], o8);
+            split8<true>(o8, hi, lo);
+            store(VH, kb, hi);
+            store(VL, kb, lo);
+        } else {
+            store(VH, kb, __builtin_bit_cast(bf16x8, vraw[kb][0]));
+        }
+    }
+    lds_barrier();
+    float before = 0.f, total = 0.f, t[PART_WAVES];
+#pragma unroll
+    for (int g = 0; g < PART_WAVES; ++g) {
+        t[g] = L.Tot[g][lane];
+        before += g < wave ? t[g] : 0.f;
+        total += t[g];
+    }
+    bool out_of_range = false;
+#pragma unroll
+    for (int g = 0; g < PART_WAVES; g += 2) out_of_range |= !(t[g] + t[g + 1] >= -SAFE_DECAY * LOG2E);        // a 32-token chunk
+    L.Before[wave][0][lane] = before;
+    L.Before[wave][1][lane] = total - before;
+    float* const out = ws + ((size_t)bh * nseg + seg) * BWD_SEG_FLOATS;
+    if (wave == 0) {                                                      // every wave saw all totals
+        out[4 * SEG_STATE + lane] = fast_exp2(total);
+        const bool any = __builtin_amdgcn_ballot_w64(out_of_range) != 0ull;
+        if (lane == 0) flags[(size_t)bh * nseg + seg] = any ? 1 : 0;
+    }
+    const int jt = wave & 3, ct0 = 2 * (wave >> 2);                       // column j = 16 jt + c16, rows (value channels) 16 (ct0 + q) + 4 g4 + r
+#pragma unroll
+    for (int dn = 0; dn < 2; ++dn) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            float f[8];
+#pragma unroll
+            for (int hf = 0; hf < 2; ++hf) {
+                const f32x4 b = *reinterpret_cast<const f32x4*>(&L.Before[wave][1 - dn][32 * kb + 8 * g4 + 4 * hf]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) f[4 * hf + e] = fast_exp2(dn ? b[e] + dpp_get<0x111>(x[kb][4 * hf + e]) : b[e] - x[kb][4 * hf + e]);
+            }
+            auto times = [&](const u32x4* raw, unsigned h, unsigned l) {
+                float o8[8];
+                bf16x8 hi, lo;
+                widen8<IO>(raw, o8);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o8[e] *= f[e];
+                split8<true>(o8, hi, lo);
+                store(h, kb, hi);
+                store(l, kb, lo);
+            };
+            times(kraw[kb], KH, KL);
+            times(rraw[kb], RH, RL);
+        }
+        lds_barrier();
+        f32x4 S[2], G[2];
+        S[0] = S[1] = G[0] = G[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int q = 0; q < nb; ++q) {
+            const bf16x8 kh = tile_across(lds + KH, 32 * q, jt, lane), kl = tile_across(lds + KL, 32 * q, jt, lane);
+            const bf16x8 rh = tile_across(lds + RH, 32 * q, jt, lane), rl = tile_across(lds + RL, 32 * q, jt, lane);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const bf16x8 vh = tile_across(lds + VH, 32 * q, ct0 + i, lane), gh = tile_across(lds + GYH, 32 * q, ct0 + i, lane),
+                             gl = tile_across(lds + GYL, 32 * q, ct0 + i, lane);
+                S[i] = mfma(vh, kh, S[i]);
+                G[i] = mfma(gh, rh, G[i]);
+                S[i] = mfma(vh, kl, S[i]);
+                G[i] = mfma(gh, rl, G[i]);
+                if constexpr (VSPLIT) S[i] = mfma(tile_across(lds + VL, 32 * q, ct0 + i, lane), kh, S[i]);
+                G[i] = mfma(gl, rh, G[i]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            *reinterpret_cast<f32x4*>(out + 2 * dn * SEG_STATE + seg_frag(jt, ct0 + i, lane)) = S[i];
+            *reinterpret_cast<f32x4*>(out + (2 * dn + 1) * SEG_STATE + seg_frag(jt, ct0 + i, lane)) = G[i];
+        }
+        if (dn == 0) lds_barrier();                                       // the operands' place is written next
     }
 }
 

@@ -37,7 +37,7 @@ constexpr int BWD_SEG_FLOATS = 4 * SEG_STATE + HN;   // backward: S up, G up, S 
 // uncut 376, 4 segments 310; at 9 of 7 chunks uncut 78, 7 segments 42; at 192 of 7 chunks uncut 84, best cut 103
 struct SegCosts { double one, each, state, fixed, per_segment; };
 constexpr SegCosts SEG_BWD = {11.5, 9.0, 1.5, 32.0, 0.1};
-inline int wkv6_segments(long long sequences, int nchunk, int cus, const SegCosts& k) {
+inline int wkv6_segments(long long sequences, int nchunk, int cus, const SegCosts& k, double& us) {
     auto time = [&](int nseg) {
         const int cps = (nchunk + nseg - 1) / nseg;
         const long long per_cu = (sequences * nseg + cus - 1) / cus;
@@ -50,6 +50,7 @@ inline int wkv6_segments(long long sequences, int nchunk, int cus, const SegCost
         const double t = time(nseg);
         if (t < best_time) { best = nseg; best_time = t; }
     }
+    us = time(best);
     const int cps = (nchunk + best - 1) / best;
     return (nchunk + cps - 1) / cps;                 // every segment non-empty
 }
