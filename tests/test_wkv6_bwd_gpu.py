@@ -275,7 +275,7 @@ def test_gradients_of_sequences_as_one_or_two_products(ops, T, dtype):
             assert all(torch.equal(x, y) for x, y in zip(ops.wkv6_backward(B, T, C, H, *off, u, gy), got))
 
 
-@pytest.mark.parametrize("T,segments", [(33, 2), (65, 3), (200, 3), (250, 8), (577, 5)])
+@pytest.mark.parametrize("T,segments", [(33, 2), (65, 3), (200, 3), (250, 8), (577, 5), (280, 9)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_backward_of_sequences_cut_into_segments(ops, T, segments, dtype):
     """Forced numbers of segments (one chunk each, a last segment of one token) against the uncut sequences, which the

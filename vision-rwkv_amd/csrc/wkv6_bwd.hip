@@ -65,11 +65,11 @@ bool bwd_tile_takes(int T, int rkv_dtype) {
 
 // Segments per sequence of a call (1: not cut); OPT_WKV6_SEGMENTS forces a number (testing).  parts: of 128 tokens, one part of wkv6_bwd_tile.h each.  Those
 // take three launches and BWD_PARTS_US whatever the sequences' number and length, as long as every segment has a compute unit and there are not more than
-// eight in a sequence (each folds the states of all others); the sweeps are ahead where they find short segments for all of them.  us, sweeps -> parts,
-// bf16 / fp32: 48 sequences of 577 tokens 80 -> 55 / 79 -> 65, of 400 84 -> 51 / 85 -> 60, 24 of 1024 87 -> 51 / 92 -> 62, 24 of 577 57 -> 47 / 59 -> 58,
-// 24 of 300 43 -> 45 / 43 -> 55, 3 of 577 41 -> 44 / 42 -> 53.
-constexpr int BWD_TILE_SEGMENTS = 8;
-constexpr double BWD_PARTS_US[3] = {62., 52., 55.};      // VRWKV_F32, VRWKV_BF16, VRWKV_F16
+// sixteen in a sequence (each folds the states of all others); the sweeps are ahead where they find short segments for all of them.  us, sweeps -> parts,
+// bf16 / fp32: 48 sequences of 577 tokens 80 -> 55 / 79 -> 65, of 400 84 -> 51 / 85 -> 60, 24 of 1024 87 -> 51 / 92 -> 62, 12 of 1025 77 -> 50 / 80 -> 59,
+// 24 of 577 57 -> 47 / 59 -> 58, 24 of 300 43 -> 45 / 43 -> 55, 3 of 577 41 -> 44 / 42 -> 53.
+constexpr int BWD_TILE_SEGMENTS = 16;
+constexpr double BWD_PARTS_US[3] = {59.5, 52., 55.};    // VRWKV_F32, VRWKV_BF16, VRWKV_F16
 int segments(int B, int T, int H, int rkv_dtype, bool& parts) {
     const int nchunk = (T + LC - 1) / LC, forced = option(OPT_WKV6_SEGMENTS);
     const long long sequences = (long long)B * H;
@@ -157,10 +157,11 @@ int launch_all(const void* r, const void* k, const void* v, const void* w, const
         if (p.nseg == 1 ? bwd_tile_takes(T, type_code<IO>) : p.parts) {
             bool loose = false;
             if constexpr (sizeof(IO) == 2) {
-                loose = (((uintptr_t)r | (uintptr_t)k | (uintptr_t)v | (uintptr_t)w) & 3) != 0;
-                if (loose) hipLaunchKernelGGL((wkv6_bwd_tile_kernel<IO, WT, EW, true>), dim3(grid), dim3(64 * PART_WAVES), 0, st, A);
+                loose = (((uintptr_t)r | (uintptr_t)k | (uintptr_t)v | (uintptr_t)w) & 3) != 0;               // (then uncut)
+                if (loose) hipLaunchKernelGGL((wkv6_bwd_tile_kernel<IO, WT, EW, false, true>), dim3(grid), dim3(64 * PART_WAVES), 0, st, A);
             }
-            if (!loose) hipLaunchKernelGGL((wkv6_bwd_tile_kernel<IO, WT, EW>), dim3(grid), dim3(64 * PART_WAVES), 0, st, A);
+            if (p.nseg > 1) hipLaunchKernelGGL((wkv6_bwd_tile_kernel<IO, WT, EW, true>), dim3(grid), dim3(64 * PART_WAVES), 0, st, A);
+            else if (!loose) hipLaunchKernelGGL((wkv6_bwd_tile_kernel<IO, WT, EW, false>), dim3(grid), dim3(64 * PART_WAVES), 0, st, A);
         } else {
             hipLaunchKernelGGL((wkv6_bwd_sweep_kernel<IO, WT, EW>), dim3(grid), dim3(512), 0, st, A);
         }

@@ -20,6 +20,11 @@
 // the channels in the order in which a lane holds its token's rows (token c16, channels 32 kb + 8 g4 .. + 7), so that the results meet r, k and the factors
 // there and gw is summed along the rows of 16 lanes.  Computed operands are split into bf16 head + tail as in the sweeps, tail x tail included for gr and gk.
 //
+// Bound by latency and vector work: two waves a SIMD issue 6 200 vector instructions, 730 products and 970 LDS accesses each at 64 x 196 x 768, matrix cores
+// busy 19 %, LDS 25 %, vector ALUs 40 %; of a full part's 42 000 cycles 6 500 wait for its rows, 4 500 form operands, 11 000 + 7 000 are products and 8 000 the
+// results.  us there, sweeps -> here: bf16 197 -> 150, fp32 213 -> 185; one sequence 81 -> 48.  Measured and left out: rows brought into the L2s ahead
+// (166 -> 172), pieces of four channels (the loads' halves have to be moved: 166 -> 188), places in LDS with twice the bank conflicts (166 -> 167).
+//
 // Range: |P_end| <= 200 in a part, and 60 nats over 32 tokens as in the sweeps (gw is a difference of sums whose neighbouring tokens do not decay: the more
 // the others do, the less of it is left).  Sequences beyond go through the sweeps' code, which leaves the latter to the sequential sweeps.
 #pragma once
@@ -44,8 +49,9 @@ __device__ __forceinline__ bf16x8 tile_across_owned(const unsigned char* arr, un
     return cat8(lds_read_tr4(reinterpret_cast<const __bf16*>(p)), lds_read_tr4(reinterpret_cast<const __bf16*>(p + 2048)));
 }
 
-// LOOSE: 16-bit rows that do not lie on 4 bytes, fetched element by element.
-template <typename IO, typename WT, bool W_IS_EW, bool LOOSE = false>
+// SEG: segments of cut sequences (a kernel of its own: either path's registers would hold the other back, 155 -> 176 us uncut).  LOOSE: 16-bit rows that do
+// not lie on 4 bytes, fetched element by element.
+template <typename IO, typename WT, bool W_IS_EW, bool SEG, bool LOOSE = false>
 __global__ __launch_bounds__(64 * PART_WAVES, 2)
 void wkv6_bwd_tile_kernel(BwdArgs A)
 {
@@ -75,10 +81,10 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
         c16 = lane & 15;
     };
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int T = A.T, C = A.C, nseg = A.nseg;
+    const int T = A.T, C = A.C, nseg = SEG ? A.nseg : 1;
     int bh = blockIdx.x, seg = 0;
     bool bail = false;
-    if (nseg > 1) {
+    if constexpr (SEG) {
         seg_of_block(blockIdx.x, nseg, bh, seg);
         if (bh >= A.sequences) return;
         const int f = lane < nseg ? A.seg_flags[(size_t)bh * nseg + lane] : 0;
@@ -89,7 +95,7 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
     const unsigned n_el = (unsigned)((size_t)(T - 1) * C + HN);          // elements from the block's first to its last
     const int nchunk = (T + LC - 1) / LC, cps = (nchunk + nseg - 1) / nseg;
     const int first = seg * cps * LC, n = min(cps * LC, T - first);
-    const bool two = n > PART;
+    const bool two = !SEG && n > PART;
     const int n1 = two ? (n - PART + LC - 1) / LC * LC : n;              // tokens of the first part
 
     constexpr int PI = (int)ES / 2, PW = (int)WS / 2;
@@ -166,7 +172,7 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
     constexpr std::integral_constant<bool, VSPLIT> v_split{};
     constexpr std::true_type is_split{};
     // The states that enter the segment from the front (up) or from behind: those that the segments there leave by themselves, each over the decay of the
-    // segments in between.  (A launch that folds them first costs more for up to eight segments.)
+    // segments in between.  (A launch that folds them first costs 11 us at 48 sequences of five segments.)
     auto local_state = [&](int s, int m, f32x4 (&X)[2]) {
         const float* const p = A.seg_ws + ((size_t)bh * nseg + s) * BWD_SEG_FLOATS + m * SEG_STATE;
 #pragma unroll
@@ -217,7 +223,7 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
         fetch(A.gy, t0, graw, 4u);
         fetch(A.v, t0, vraw, ES);
         f32x4 XD[2], YD[2], XU[2], YU[2];            // S and G that enter a segment from behind and from the front
-        if (nseg > 1) {
+        if constexpr (SEG) {
             entering(false, XD, YD);
             entering(true, XU, YU);
             // X at the segment's end: sum over the value channels of S G of both passes
@@ -352,7 +358,7 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
                 XS[q] = __builtin_nondeterministic_value(XS[q]);
                 XG[q] = __builtin_nondeterministic_value(XG[q]);
             }
-        } else if (nseg > 1) {
+        } else if constexpr (SEG) {
             put_state(c_part, XD, ZS);
             put_state(c_part, YD, ZG);
             put_state(c_part, YU, ZG_FRONT);
@@ -500,7 +506,7 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
             state_gkv(ZG, KB, gku);
         } else if (two) {
             state_gkv(ZG_BEHIND, KF, gkd);
-        } else if (nseg > 1) {
+        } else if constexpr (SEG) {
             state_gkv(ZG, KF, gkd);
             state_gkv(ZG_FRONT, KB, gku);
             state_gr(grd);
@@ -548,7 +554,7 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
             for (int q = own + 1; q < nb; ++q) gather(KBH, KBL, q, pair(dt_tile(2 * q), dt_tile(2 * q + 1)), grd);
         }
         if (two && step == 2) state_gr(grd);
-        else if (step == 1 || nseg > 1) state_gr(gru);
+        else if (SEG || step == 1) state_gr(gru);
         if (step == 1) {
             f32x4 X[2];
             form_state(KBH, KBL, VH, VL, v_split, nb, X);
@@ -591,7 +597,7 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
         gu += row_sums16(gu16, lane, gu_at);
         lds_barrier();
         {
-            if (nseg > 1) xrun = L.X[0][lane] + L.X[1][lane];
+            if constexpr (SEG) xrun = L.X[0][lane] + L.X[1][lane];
             float after = 0.f, total = 0.f;
 #pragma unroll
             for (int g = 0; g < PART_WAVES; ++g) {
@@ -622,7 +628,7 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
         }
     }
     if (bail) {
-        if (nseg > 1) {
+        if constexpr (SEG) {
             // the sweeps take the states that enter the segment from memory
             float* const own = A.seg_own + ((size_t)bh * nseg + seg) * BWD_SEG_FLOATS;
 #pragma unroll 1
