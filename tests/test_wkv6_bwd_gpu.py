@@ -275,6 +275,31 @@ def test_gradients_of_sequences_as_one_or_two_products(ops, T, dtype):
             assert all(torch.equal(x, y) for x, y in zip(ops.wkv6_backward(B, T, C, H, *off, u, gy), got))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,segments", [(300, 3), (577, 5), (1100, 9)])
+def test_cut_sequences_whose_parts_are_out_of_range(ops, T, segments, dtype):
+    """1.8 log2 a token: 225 over a part of 128 tokens, whose factors hold 200, 39 nats over a chunk, whose factors hold 60.  The chunked kernels' code takes
+    such segments over, from the states that every workgroup folds for itself.  Bounds as above."""
+    B, H = 2, 2
+    C = 64 * H
+    g = torch.Generator(device="cuda").manual_seed(T)
+    r, k, v = (torch.randn(B, T, C, generator=g, device="cuda").to(dtype) for _ in range(3))
+    gy, u = torch.randn(B, T, C, generator=g, device="cuda"), torch.randn(H, 64, generator=g, device="cuda") * 0.3
+    w = torch.full((B, T, C), -3.0, device="cuda")
+    w[0] = 0.2
+    w = (w + 0.05 * torch.randn(B, T, C, generator=g, device="cuda")).to(dtype)
+    with ops.option("wkv6_segments", segments):
+        y, got = ops.wkv6_forward(B, T, C, H, r, k, v, w, u), ops.wkv6_backward(B, T, C, H, r, k, v, w, u, gy)
+    with ops.option("wkv6_fwd_scalar", 1), ops.option("wkv6_bwd_scalar", 1):
+        want, ref = ops.wkv6_forward(B, T, C, H, r, k, v, w, u), ops.wkv6_backward(B, T, C, H, r, k, v, w, u, gy)
+    terms = w.float().exp() * ((r.float() * ref[0]).abs() + (k.float() * ref[1]).abs())
+    for b in range(B):
+        for x, y_ in zip((y,) + tuple(got[:3]), (want,) + tuple(ref[:3])):
+            assert (x[b] - y_[b]).norm() <= 1.6e-5 * y_[b].norm()
+        assert (got[3][b] - ref[3][b]).norm() <= 1.6e-5 * T ** 0.5 * terms[b].norm()
+    assert (got[4] - ref[4]).norm() <= 1.6e-5 * ref[4].norm()
+
+
 @pytest.mark.parametrize("T,segments", [(33, 2), (65, 3), (200, 3), (250, 8), (577, 5), (280, 9)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_backward_of_sequences_cut_into_segments(ops, T, segments, dtype):

@@ -41,12 +41,16 @@ int segments(int B, int T, int H, int rkv_dtype, bool& parts) {
     const int nchunk = (T + LC - 1) / LC, forced = option(OPT_WKV6_SEGMENTS);
     if (forced > 0 && (long long)B * H <= SEG_SEQUENCES) {
         const int n = forced < nchunk ? forced : nchunk, cps = (nchunk + n - 1) / n;
-        parts = rkv_dtype == VRWKV_BF16 && cps * LC <= TILE_TOKENS;
+        parts = rkv_dtype == VRWKV_BF16 ? cps * LC <= TILE_TOKENS : cps * LC <= PART && (nchunk + cps - 1) / cps <= FOLD_SEGMENTS;
         return (nchunk + cps - 1) / cps;
     }
     parts = false;
-    return forced > 0 ? 1 : wkv6_fwd_segments((long long)B * H, nchunk, device_cus(), SEG_FWD[rkv_dtype], rkv_dtype == VRWKV_BF16 ? &parts : nullptr);
+    return forced > 0 ? 1 : wkv6_fwd_segments((long long)B * H, nchunk, device_cus(), rkv_dtype, parts);
 }
+// Segments of one part fold the states themselves where there are few, without a launch that does it first (bf16, 48 sequences of 577 tokens: 29.9 and 26.9
+// us), and want room for the result.
+bool folds(int T, int nseg, bool parts) { return parts && nseg <= FOLD_SEGMENTS && ((T + LC - 1) / LC + nseg - 1) / nseg * LC <= PART; }
+size_t states_bytes(long long sequences, int T, int nseg, bool parts) { return seg_bytes(sequences, nseg, SEG_FLOATS * (folds(T, nseg, parts) ? 2 : 1)); }
 
 template <typename IO, typename WT>
 int launch_scalar(const void* r, const void* k, const void* v, const void* w, const float* u, float* y,
@@ -81,43 +85,58 @@ int launch_chunked(const void* r, const void* k, const void* v, const void* w, c
     int nseg = whole ? 1 : segments(B, T, H, type_code<IO>, parts);
     // (the state kernels read several elements at a time: 16-bit rows on 4 bytes; wider accesses need no more either)
     const bool cut = !(((uintptr_t)k | (uintptr_t)v | (uintptr_t)w) & 3), loose = !cut || ((uintptr_t)r & 3);
-    if (!ws || ws_bytes < seg_bytes(sequences, nseg, SEG_FLOATS) || ((uintptr_t)ws & 15) || !cut) nseg = 1;
-    float* states = nullptr;
+    if (!ws || ws_bytes < states_bytes(sequences, T, nseg, parts) || ((uintptr_t)ws & 15) || !cut) nseg = 1;
+    float *states = nullptr, *own = nullptr;
     int* flags = nullptr;
     unsigned grid = (unsigned)sequences;
     if (nseg > 1) {
         states = static_cast<float*>(ws);
-        flags = reinterpret_cast<int*>(states + (size_t)sequences * nseg * SEG_FLOATS);
+        const size_t all = (size_t)sequences * nseg * SEG_FLOATS;
+        if (folds(T, nseg, parts)) own = states + all;
+        flags = reinterpret_cast<int*>((own ? own : states) + all);
         grid = seg_grid(sequences, nseg);
-        if constexpr (type_code<IO> == VRWKV_BF16) {
-            if (parts)
-                hipLaunchKernelGGL((wkv6_part_state_kernel<IO, WT, EW>), dim3(grid), dim3(64 * PART_WAVES), 0, st, kk, vv, ww, states, flags, T, C, H,
-                                   sequences, nseg);
-        }
-        if (!parts)
+        if (parts)
+            hipLaunchKernelGGL((wkv6_part_state_kernel<IO, WT, EW>), dim3(grid), dim3(64 * PART_WAVES), 0, st, kk, vv, ww, states, flags, T, C, H,
+                               sequences, nseg);
+        else
             hipLaunchKernelGGL((wkv6_seg_state_kernel<IO, WT, EW>), dim3(grid), dim3(256), 0, st, kk, vv, ww, states, flags, T, C, H, sequences, nseg);
-        hipLaunchKernelGGL((wkv6_seg_fold_kernel<2, false>), dim3(4, 2, (unsigned)sequences), dim3(256), 0, st, states, nseg);
+        if (!own) hipLaunchKernelGGL((wkv6_seg_fold_kernel<2, false>), dim3(4, 2, (unsigned)sequences), dim3(256), 0, st, states, nseg);
     }
     // Up to 256 tokens in one or two parts (the tile kernel is ahead of the chunked one at every size measured, 3 to 768 sequences of 33 to 256 tokens in
     // all types: 1.03 to 1.8 times, least where a second part is nearly empty); more tokens, and calls that ask for it (vrwkv_wkv6_fwd_whole),
     // are the chunked kernel's.
-    const FwdTileArgs tile{r, k, v, w, u, y, T, C, H, (int)sequences, nseg, states, flags};
+    const FwdTileArgs tile{r, k, v, w, u, y, T, C, H, (int)sequences, nseg, states, flags, own};
     if (nseg == 1 && T <= TILE_TOKENS && !whole) {
         if constexpr (sizeof(IO) == 2) {
             if (loose) {
-                hipLaunchKernelGGL((wkv6_fwd_tile_kernel<IO, WT, EW, false, true>), dim3(grid), dim3(64 * PART_WAVES), 0, st, tile);
+                hipLaunchKernelGGL((wkv6_fwd_tile_kernel<IO, WT, EW, 0, true>), dim3(grid), dim3(64 * PART_WAVES), 0, st, tile);
                 return check_launch("wkv6_fwd (tile, rows off 4 bytes)");
             }
         }
-        hipLaunchKernelGGL((wkv6_fwd_tile_kernel<IO, WT, EW, false>), dim3(grid), dim3(64 * PART_WAVES), 0, st, tile);
+        hipLaunchKernelGGL((wkv6_fwd_tile_kernel<IO, WT, EW, 0>), dim3(grid), dim3(64 * PART_WAVES), 0, st, tile);
         return check_launch("wkv6_fwd (tile)");
     }
-    if constexpr (type_code<IO> == VRWKV_BF16) {
-        if (nseg > 1 && parts) {
-            if (loose) hipLaunchKernelGGL((wkv6_fwd_tile_kernel<IO, WT, EW, true, true>), dim3(grid), dim3(64 * PART_WAVES), 0, st, tile);
-            else hipLaunchKernelGGL((wkv6_fwd_tile_kernel<IO, WT, EW, true>), dim3(grid), dim3(64 * PART_WAVES), 0, st, tile);
-            return check_launch("wkv6_fwd (tile, segments)");
+    if (nseg > 1 && parts) {
+        auto go = [&](auto segments, auto off) {
+            hipLaunchKernelGGL((wkv6_fwd_tile_kernel<IO, WT, EW, decltype(segments)::value, decltype(off)::value>), dim3(grid), dim3(64 * PART_WAVES), 0, st, tile);
+        };
+        constexpr std::integral_constant<int, 1> folded{};
+        constexpr std::integral_constant<int, 2> fold{};
+        if constexpr (type_code<IO> == VRWKV_BF16) {                     // (the other types have no segments that do not fold)
+            if (!own) {
+                if (loose) go(folded, std::true_type{});
+                else go(folded, std::false_type{});
+                return check_launch("wkv6_fwd (tile, segments)");
+            }
         }
+        if constexpr (sizeof(IO) == 2) {
+            if (loose) {
+                go(fold, std::true_type{});
+                return check_launch("wkv6_fwd (tile, segments, r off 4 bytes)");
+            }
+        }
+        go(fold, std::false_type{});
+        return check_launch("wkv6_fwd (tile, segments)");
     }
     hipLaunchKernelGGL((wkv6_fwd_chunk_kernel<IO, WT, EW>), dim3(grid), block, 0, st, rr, kk, vv, ww, u, y, T, C, H, (int)sequences,
                        nseg, states, flags, nullptr);
@@ -175,9 +194,13 @@ extern "C" size_t vrwkv_wkv6_fwd_workspace_bytes(int B, int T, int C, int H) {
     (void)C;
     if (B <= 0 || T <= 0 || H <= 0) return 0;
     // the same for every type: the largest of the plans
-    bool parts;
-    return seg_bytes((long long)B * H, std::max({segments(B, T, H, VRWKV_F32, parts), segments(B, T, H, VRWKV_BF16, parts), segments(B, T, H, VRWKV_F16, parts)}),
-                     SEG_FLOATS);
+    size_t bytes = 0;
+    for (int dt : {VRWKV_F32, VRWKV_BF16, VRWKV_F16}) {
+        bool parts;
+        const int nseg = segments(B, T, H, dt, parts);
+        bytes = std::max(bytes, states_bytes((long long)B * H, T, nseg, parts));
+    }
+    return bytes;
 }
 
 namespace vrwkv {

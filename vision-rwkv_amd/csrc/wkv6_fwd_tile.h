@@ -41,16 +41,19 @@ struct FwdTileArgs {
     const float* u;
     float* y;
     int T, C, H, sequences, nseg;
-    const float* seg_ws;
+    const float* seg_ws;                             // the segments' states
     const int* seg_flags;
+    float* seg_own;                                  // SEGMENTS 2: room for the states that enter the segments
 };
 
-// LOOSE: 16-bit rows that do not lie on 4 bytes, fetched element by element (the same results, in a kernel of its own: the packing takes registers).
-template <typename IO, typename WT, bool W_IS_EW, bool SEG, bool LOOSE = false>
+// SEGMENTS: of cut sequences, 1 with the states that enter them, 2 with those that they leave by themselves (of one part; in a kernel of its own, for the
+// registers).  LOOSE: 16-bit rows that do not lie on 4 bytes, fetched element by element (the same results, in a kernel of its own: the packing takes registers).
+template <typename IO, typename WT, bool W_IS_EW, int SEGMENTS, bool LOOSE = false>
 __global__ __launch_bounds__(64 * PART_WAVES, 4)
 void wkv6_fwd_tile_kernel(FwdTileArgs A)
 {
     constexpr bool VSPLIT = !__is_same(IO, __hip_bfloat16);
+    constexpr bool SEG = SEGMENTS != 0, FOLD = SEGMENTS == 2;
     constexpr unsigned ES = (unsigned)sizeof(IO), WS = (unsigned)sizeof(WT), ARR = PART * 128u;
     constexpr unsigned KFH = 0, KFL = ARR, KBH = 2 * ARR, KBL = 3 * ARR, VH = 4 * ARR, VL = 5 * ARR;
     __shared__ __attribute__((aligned(16))) unsigned char lds[(VSPLIT ? 6 : 5) * ARR];
@@ -85,7 +88,7 @@ void wkv6_fwd_tile_kernel(FwdTileArgs A)
     const int b = bh / A.H, h = bh % A.H;
     const size_t base = (size_t)b * T * C + (size_t)h * HN;
     const int first = seg * cps * LC, n = min(cps * LC, T - first);
-    const bool two = n > PART;
+    const bool two = !FOLD && n > PART;
     const int n1 = two ? ((n + LC - 1) / LC + 1) / 2 * LC : n;           // tokens of the first part
 
     // eight channels 32 kb + 8 g4 .. + 7 of a row, packed as they lie, in 16-byte pieces
@@ -158,6 +161,32 @@ void wkv6_fwd_tile_kernel(FwdTileArgs A)
 #pragma unroll
         for (int q = 0; q < 2; ++q) X[q] = *reinterpret_cast<const f32x4v*>(in + seg_frag(it0, jt0 + q, lane));
     };
+    // the same from the states that the segments in front of this one, or behind it, leave by themselves, each over the decays in between
+    auto fold_states = [&](bool down, f32x4v (&S)[2]) {
+        constexpr int U = 4;
+        const int count = down ? nseg - 1 - seg : seg;
+        S[0] = S[1] = f32x4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int i0 = 0; i0 < count; i0 += U) {
+            f32x4v l[U][2], d[U][2];
+#pragma unroll
+            for (int i = 0; i < U; ++i)
+                if (i0 + i < count) {
+                    const float* p = A.seg_ws + ((size_t)bh * nseg + (down ? nseg - 1 - i0 - i : i0 + i)) * SEG_FLOATS;
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        l[i][q] = *reinterpret_cast<const f32x4v*>(p + (down ? SEG_STATE : 0) + seg_frag(it0, jt0 + q, lane));
+                        d[i][q] = *reinterpret_cast<const f32x4v*>(p + 2 * SEG_STATE + 16 * (jt0 + q) + 4 * g4);
+                    }
+                }
+#pragma unroll
+            for (int i = 0; i < U; ++i)
+                if (i0 + i < count) {
+                    S[0] = S[0] * d[i][0] + l[i][0];
+                    S[1] = S[1] * d[i][1] + l[i][1];
+                }
+        }
+    };
     auto across = [&](unsigned arr, int q, int ct) { return read_across(lds + arr, q, ct, lane); };
 
     u32x4 wraw[2][PW];
@@ -173,6 +202,11 @@ void wkv6_fwd_tile_kernel(FwdTileArgs A)
         fetch(A.r, t0, rraw, ES);
         fetch(A.k, t0, kraw, ES);
         fetch(A.v, t0, vraw, ES);
+        f32x4v XF[2];                                // the state from the front, where it is folded here
+        if constexpr (FOLD) {                        // (of one part)
+            fold_states(true, X);
+            fold_states(false, XF);
+        }
         float x[2][8];                               // log2 decays summed over the wave's tokens
         const bool past = 16 * wave + c16 >= np;
 #pragma unroll
@@ -264,7 +298,7 @@ void wkv6_fwd_tile_kernel(FwdTileArgs A)
         // states that enter the part: from behind (the second part's, or the segment's), from the front (the segment's, of a first part)
         if (SEG || (two && part == 0)) {
             if constexpr (SEG) {
-                if (part == 1 || !two) load_state(true);
+                if (!FOLD && (part == 1 || !two)) load_state(true);
             }
             put_state(part ? c_second : two ? c_first + c_second : c_first);
             lds_barrier();
@@ -272,7 +306,8 @@ void wkv6_fwd_tile_kernel(FwdTileArgs A)
             lds_barrier();
             if constexpr (SEG) {
                 if (part == 0) {
-                    load_state(false);
+                    if constexpr (FOLD) { X[0] = XF[0]; X[1] = XF[1]; }
+                    else load_state(false);
                     put_state(c_first);
                     lds_barrier();
                     add_state(RFh, RFl, accY);
@@ -407,10 +442,21 @@ void wkv6_fwd_tile_kernel(FwdTileArgs A)
         }
     }
     if (bail) {
+        const float* states = A.seg_ws;
+        if constexpr (FOLD) {                        // the chunked kernel's code takes the states that enter the segment from memory
+            float* const own = A.seg_own + ((size_t)bh * nseg + seg) * SEG_FLOATS;
+#pragma unroll 1
+            for (int down = 0; down < 2; ++down) {
+                fold_states(down, X);
+#pragma unroll
+                for (int q = 0; q < 2; ++q) *reinterpret_cast<f32x4v*>(own + down * SEG_STATE + seg_frag(it0, jt0 + q, lane)) = X[q];
+            }
+            states = A.seg_own;
+        }
         __syncthreads();
         fwd_chunk_sequence<IO, WT, W_IS_EW>(reinterpret_cast<FwdLds<VSPLIT>*>(lds), reinterpret_cast<int*>(lds + sizeof(FwdLds<VSPLIT>) * 2), bh, seg,
                                             static_cast<const IO*>(A.r), static_cast<const IO*>(A.k), static_cast<const IO*>(A.v),
-                                            static_cast<const WT*>(A.w), A.u, A.y, T, C, A.H, nseg, A.seg_ws, A.seg_flags);
+                                            static_cast<const WT*>(A.w), A.u, A.y, T, C, A.H, nseg, states, A.seg_flags);
     }
 }
 

@@ -71,11 +71,17 @@ inline int wkv6_segments(long long sequences, int nchunk, int cus, const SegCost
 //          24 of 130                  354 | 10 65, 17 61, 26 76, [33] 62            192 of 32    94 | 4 95, [8] 95, 11 119
 //          48 of 64                   174 | 8 59, 10 61, [16] 55, 32 81             192 of 13    41 | 2 58, [4] 50, 5 56
 //          96 of 19                    56 | 3 54, [5] 37, 10 54                      96 of 10    32 | 2 36, [3] 36, 5 35
+// In fp16 and fp32 a part's operands leave room for one workgroup a compute unit: where all have one, and no sequence more than sixteen, as each folds the
+// states of the others; sequences that the others leave whole stay so unless a third is gained.  us, chunked kernels -> parts, fp16 / fp32: 48 sequences of 577 tokens 33 -> 23 / 34 -> 26, 24 of 1024 32 -> 24 / 32 -> 27,
+// 24 of 300 23 -> 21 / 23.6 -> 23.4, 12 of 2048 35 -> 26 / 34 -> 30, 3 of 577 20.2 -> 20.2 / 20.6 -> 23.5.
+constexpr int FOLD_SEGMENTS = 16;
 struct FwdSegCosts { double uncut, uncut_fixed, uncut_traffic, step[4], fixed, per_segment, traffic, token_traffic; };
 constexpr FwdSegCosts SEG_FWD[3] = {{2.72, 4.0, 2.23, {3.73, 7.06, 11.09, 14.80}, 9.8, 0.14, 28.5, 3.39},       // VRWKV_F32
                                     {2.65, 5.1, 1.09, {3.53, 5.14, 8.16, 10.48}, 10.8, 0.14, 20.3, 3.44},       // VRWKV_BF16
                                     {2.80, 4.9, 1.33, {3.99, 7.28, 10.68, 14.05}, 9.6, 0.14, 29.9, 1.70}};      // VRWKV_F16
-inline int wkv6_fwd_segments(long long sequences, int nchunk, int cus, const FwdSegCosts& k, bool* parts) {
+inline int wkv6_fwd_segments(long long sequences, int nchunk, int cus, int type, bool& parts) {
+    const FwdSegCosts& k = SEG_FWD[type];
+    parts = false;
     const long long padded = (sequences + 7) / 8 * 8;
     if (nchunk <= 8 || padded > cus) return 1;       // more sequences than compute units: a cut only adds work
     int best = 1;
@@ -86,11 +92,16 @@ inline int wkv6_fwd_segments(long long sequences, int nchunk, int cus, const Fwd
         const double t = cps * k.step[per_cu - 1] + k.fixed + k.per_segment * nseg + k.traffic * 1e-3 * (double)(sequences * nseg) + k.token_traffic * chunks;
         if (t < best_time) { best = nseg; best_time = t; }
     }
-    if (parts) {
+    if (type == 1) {
         const int cps = std::max(4, (nchunk + SEG_MAX - 1) / SEG_MAX), nseg = (nchunk + cps - 1) / cps;
         const double t = std::max(19.0 + 0.45 * nseg, 15.0 + 0.25 * nseg + 0.052 * (double)(sequences * nseg));
-        *parts = t < (best == 1 ? 0.84 : 1.0) * best_time && cps * LC <= 2 * 128;
-        if (*parts) return nseg;
+        parts = t < (best == 1 ? 0.84 : 1.0) * best_time && cps * LC <= 2 * 128;
+        if (parts) return nseg;
+    } else {
+        const int nseg = (nchunk + 3) / 4;
+        const double t = (type == 0 ? 21.5 : 19.0) + 0.4 * nseg + 0.01 * (double)(sequences * nseg);
+        parts = nseg <= FOLD_SEGMENTS && padded * nseg <= cus && t < (best == 1 ? 0.73 : 0.95) * best_time;
+        if (parts) return nseg;
     }
     const int cps = (nchunk + best - 1) / best;
     return (nchunk + cps - 1) / cps;                 // every segment non-empty
@@ -338,16 +349,17 @@ void wkv6_seg_state_kernel(const IO* __restrict__ k_, const IO* __restrict__ v_,
 // The same in parts of up to 128 tokens: eight waves, a wave prepares 16 tokens in the layout of the matrix operands (lane = token c16, eight channels of
 // each half) and then forms a quarter of the columns x half the rows of both states over the part's tokens.  All exponents are <= 0.  Two barriers per 128
 // tokens where the kernel above has two per 32; bound by the latency of its loads (two workgroups a compute unit) and by the states' way out.
-// 24 sequences of 4150 tokens in 17 segments 22 -> 17.6 us.  bf16 only: the operands of a split v leave room for one workgroup (fp32 21 -> 29 us).
+// 24 sequences of 4150 tokens in 17 segments 22 -> 17.6 us.  The operands of a split v leave room for one workgroup (fp32 there 21 -> 29 us): for calls that
+// do not have more.
 template <typename IO, typename WT, bool W_IS_EW>
 __global__ __launch_bounds__(64 * PART_WAVES, 4)
 void wkv6_part_state_kernel(const IO* __restrict__ k_, const IO* __restrict__ v_, const WT* __restrict__ w_,
                            float* __restrict__ ws, int* __restrict__ flags, int T, int C, int H, long long sequences, int nseg)
 {
-    static_assert(__is_same(IO, __hip_bfloat16), "v exact in bf16: the operands of a split v leave room for one workgroup a compute unit");
+    constexpr bool VSPLIT = !__is_same(IO, __hip_bfloat16);
     constexpr unsigned ES = (unsigned)sizeof(IO), WS = (unsigned)sizeof(WT), ARR = PART * 128u;
-    constexpr unsigned AH = 0, AL = ARR, DH = 2 * ARR, DL = 3 * ARR, VH = 4 * ARR;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[5 * ARR];
+    constexpr unsigned AH = 0, AL = ARR, DH = 2 * ARR, DL = 3 * ARR, VH = 4 * ARR, VL = 5 * ARR;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[(VSPLIT ? 6 : 5) * ARR];
     int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int bh, seg;
@@ -434,7 +446,14 @@ void wkv6_part_state_kernel(const IO* __restrict__ k_, const IO* __restrict__ v_
             split8<true>(o8, hi, lo);
             *reinterpret_cast<bf16x8*>(lds + DH + to) = hi;
             *reinterpret_cast<bf16x8*>(lds + DL + to) = lo;
-            *reinterpret_cast<u32x4*>(lds + VH + to) = vraw[kb][0];
+            if constexpr (!VSPLIT) {
+                *reinterpret_cast<u32x4*>(lds + VH + to) = vraw[kb][0];
+            } else {
+                widen8<IO>(vraw[kb], o8);
+                split8<true>(o8, hi, lo);
+                *reinterpret_cast<bf16x8*>(lds + VH + to) = hi;
+                *reinterpret_cast<bf16x8*>(lds + VL + to) = lo;
+            }
         }
         lds_barrier();
         if (at + PART < n) {
@@ -460,6 +479,11 @@ void wkv6_part_state_kernel(const IO* __restrict__ k_, const IO* __restrict__ v_
                 D[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dh, vv, D[j], 0, 0, 0);
                 A[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, vv, A[j], 0, 0, 0);
                 D[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dl, vv, D[j], 0, 0, 0);
+                if constexpr (VSPLIT) {
+                    const bf16x8 vl = read_across(lds + VL, q, it0, lane);
+                    A[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, vl, A[j], 0, 0, 0);
+                    D[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dh, vl, D[j], 0, 0, 0);
+                }
             }
         }
         base_p += total;
