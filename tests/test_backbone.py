@@ -825,6 +825,27 @@ def test_norm_shift_and_mixes_in_one_launch(kind, C, dtype, hw, shift, batch, cl
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("C,dtype,hw,shift,batch,key_norm", [
+    (192, torch.bfloat16, (14, 14), 1, 1, False), (192, torch.float16, (5, 7), 2, 3, True), (64, torch.bfloat16, (1, 1), 1, 1, False),
+    (64, torch.float16, (3, 1), 1, 7, False), (64, torch.bfloat16, (2, 8), 3, 33, False), (256, torch.bfloat16, (3, 24), 1, 2, False),
+    (320, torch.bfloat16, (4, 4), 1, 5, False), (384, torch.float16, (11, 17), 1, 1, True), (512, torch.bfloat16, (5, 3), 1, 1, False)])
+def test_norm_shift_and_mixes_inside_the_projections(C, dtype, hw, shift, batch, key_norm):
+    """Tiles of 16 tokens across images and past the last one, rows of half a wave and more, up to all 64 rows a workgroup holds: bit for bit the block that
+    forms them in front of the projections, which a forced tile does (one order of the products in either)."""
+    from vision_rwkv_amd import option
+    net = _small_backbone("v4", C, dtype, key_norm, False, False, hw)
+    for l in net.layers:
+        l.att.shift_pixel = l.ffn.shift_pixel = shift
+    x = torch.randn(batch, hw[0] * hw[1], C, device="cuda").to(dtype)
+    with torch.no_grad():
+        for l in net.layers:
+            got = l._native(x, hw)
+            with option("linear_tile", 1):
+                want = l._native(x, hw)
+            assert got is not None and torch.equal(got, want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("shapes", [((8, 8),), ((72, 136), (64, 64), (8, 200)), ((768, 768), (3072, 768), (768, 3072), (192, 40), (40, 192))])
 def test_weights_transposed_in_one_launch(shapes):
     from vision_rwkv_amd.ops import transposed

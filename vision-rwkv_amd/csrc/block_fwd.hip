@@ -7,7 +7,9 @@
 // where the norm and the shift behind it are one (ln_shift_mix.hip):
 //   LN | shift + mixes | key, value, receptance | Bi-WKV with gate | output + residual
 //   LN | shift + mixes | key with relu^2, receptance | value, gate, residual
+// and 5 on fewer still, where the norm, the shift and the mixes are inside the projections of a half (linear_mix_kernel).
 #include "linear.h"
+#include "wave_sum.h"
 #include <algorithm>
 #include <type_traits>
 
@@ -107,6 +109,136 @@ void linear_group_kernel(LinGroup G)
     }
 }
 
+// A pre-norm half's first steps inside the projections that take them: problem q multiplies mix q of LayerNorm(x) and its shifted rows.  On few tokens
+// the launch in front (ln_shift_mix.hip) waits for its rows and sums, this one for its operands, and the host for either.  A workgroup owns 16 tokens x 64
+// results: it normalises the rows that the mix of its tokens reads, those and the steps up and down around (a wave every fourth row, or pair of rows where
+// half a wave holds one), forms the mix in LDS, rounded as the separate kernels round it and in their order, and every wave multiplies it with 16 rows of
+// the weights, requested at the start.  What it costs is the rows normalised again by every workgroup of a token's results.
+struct MixIn {
+    const void *x, *ln_w, *ln_b;
+    const float* mix;
+    int T, Hp, Wp, shift, g, head_dim;
+    float eps;
+};
+constexpr int MIX_TOKENS = 16, MIX_COLS = 64, MIX_ROWS = 64;     // of a workgroup; most rows that it normalises
+__host__ __device__ inline unsigned mix_pitch(int C, unsigned es) { return C * es + 16u; }     // (16 more: rows begin in distinct banks)
+
+template <typename IO, bool PAIRS>
+__global__ __launch_bounds__(256)
+void linear_mix_kernel(LinGroup G, MixIn X)
+{
+    constexpr int V = 16 / (int)sizeof(IO), RW = PAIRS ? 8 : 4, U = MIX_ROWS / RW, D = 6;
+    constexpr unsigned ES = sizeof(IO);
+    extern __shared__ __attribute__((aligned(16))) unsigned char rows[];
+    const int lane = threadIdx.x & 63, g4 = lane >> 4, c16 = lane & 15;
+    const int w4 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int q = 0;
+    while (q + 1 < G.n && (int)blockIdx.x >= G.p[q + 1].tile0) ++q;
+    const LinProblem& P = G.p[q];
+    const int N = P.N, C = P.K, M = G.M, nt = N / MIX_COLS, nvec = C / V;
+    const int tile = (int)blockIdx.x - P.tile0, m0 = tile / nt * MIX_TOKENS, n0 = tile % nt * MIX_COLS + 16 * w4;
+    const int reach = X.shift * X.Wp, lo = max(m0 - reach, 0), R = min(m0 + MIX_TOKENS + reach, M) - lo;
+    const unsigned pitch = mix_pitch(C, ES);
+    unsigned char* const mixed = rows + (MIX_TOKENS + 2 * reach) * pitch;
+    // ---- everything is requested together ----
+    const int piece = PAIRS ? lane & 31 : lane, sub = PAIRS ? 2 * w4 + (lane >> 5) : w4;
+    const __amdgpu_buffer_rsrc_t rsx = make_rsrc(X.x, (unsigned)M * C * ES), rsw = make_rsrc(P.w, (unsigned)N * C * ES);
+    u32x4 raw[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+        raw[i] = u32x4{0u, 0u, 0u, 0u};
+        if (RW * i < R) raw[i] = BufRaw<16>::ld(rsx, piece < nvec && RW * i + sub < R ? (unsigned)(lo + RW * i + sub) * C * ES + 16u * piece : OOB_OFFSET, 0);
+    }
+    nt_u32x4 lw = {0u, 0u, 0u, 0u}, lb = lw;
+    if (piece < nvec) {
+        lw = load_raw16<false>((const IO*)X.ln_w + piece * V);
+        lb = load_raw16<false>((const IO*)X.ln_b + piece * V);
+    }
+    const unsigned ow = (unsigned)(n0 + c16) * C * ES + 16u * g4;
+    const int steps = C * (int)ES / 64;
+    u32x4 fw[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) fw[d] = BufRaw<16>::ld(rsw, d < steps ? ow : OOB_OFFSET, 64u * d);
+    // ---- LayerNorm ----
+    auto row_sum = [&](float x) {                         // as wave_sum; over the row's half wave where two share a wave
+        x = dpp_add<0x140>(dpp_add<0x141>(dpp_add<0x4E>(dpp_add<0xB1>(x))));
+        const int xi = __builtin_bit_cast(int, x);
+        const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(xi, 0)), r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(xi, 16)),
+                    r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(xi, 32)), r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(xi, 48));
+        return PAIRS ? (lane < 32 ? r0 + r1 : r2 + r3) : (r0 + r1) + (r2 + r3);
+    };
+    float lnw[V], lnb[V];
+    widen_raw16<IO, V>(lw, lnw);
+    widen_raw16<IO, V>(lb, lnb);
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+        if (RW * i >= R) break;
+        float v[V], s = 0.f, sq = 0.f;
+        widen_raw16<IO, V>(__builtin_bit_cast(nt_u32x4, raw[i]), v);
+#pragma unroll
+        for (int e = 0; e < V; ++e) s += v[e];
+        const float mean = row_sum(s) / (float)C;
+        if (piece < nvec) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) { const float d = v[e] - mean; sq = fmaf(d, d, sq); }
+        }
+        const float rstd = rsqrtf(row_sum(sq) / (float)C + X.eps);
+        IO n[V];
+#pragma unroll
+        for (int e = 0; e < V; ++e) n[e] = from_f32<IO>(fmaf((v[e] - mean) * rstd, lnw[e], lnb[e]));
+        if (piece < nvec && RW * i + sub < R) __builtin_memcpy(rows + (RW * i + sub) * pitch + 16 * piece, n, 16);
+    }
+    __syncthreads();
+    // ---- the mix of the 16 tokens: a thread keeps its token and takes every sixteenth piece ----
+    {
+        const int m = m0 + (threadIdx.x & 15), t = m % X.T, y0 = t / X.Wp, x0 = t % X.Wp;
+        const bool in = t < X.Hp * X.Wp;                  // (a class token stands alone)
+        const unsigned char* const own = rows + (m - lo) * pitch;
+        for (int p = threadIdx.x >> 4; p < nvec; p += 16) {
+            const int c = p * V, cq = X.head_dim > 0 ? c % X.head_dim : c, dir = X.g > 0 && cq < 4 * X.g ? cq / X.g : 4;
+            nt_u32x4 out = {0u, 0u, 0u, 0u};
+            if (m < M) {
+                const bool moved = in && dir < 4;
+                const bool there = !moved || (dir == 0 ? x0 >= X.shift : dir == 1 ? x0 + X.shift < X.Wp : dir == 2 ? y0 >= X.shift : y0 + X.shift < X.Hp);
+                const int step = !moved || !there ? 0 : dir == 0 ? -X.shift : dir == 1 ? X.shift : dir == 2 ? -reach : reach;
+                float xs[V], xx[V], mu[V];
+                widen_raw16<IO, V>(*reinterpret_cast<const nt_u32x4*>(own + 16 * p), xs);
+                widen_raw16<IO, V>(*reinterpret_cast<const nt_u32x4*>(own + step * (int)pitch + 16 * p), xx);
+#pragma unroll
+                for (int e = 0; e < V; e += 4) {
+                    const float4 f = *reinterpret_cast<const float4*>(X.mix + (size_t)q * C + c + e);
+                    mu[e] = f.x; mu[e + 1] = f.y; mu[e + 2] = f.z; mu[e + 3] = f.w;
+                }
+                IO o[V];
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                    const float x = there ? xx[e] : 0.f;
+                    o[e] = from_f32<IO>(xs[e] * mu[e] + x * (1.f - mu[e]));
+                }
+                __builtin_memcpy(&out, o, 16);
+            }
+            *reinterpret_cast<nt_u32x4*>(mixed + (threadIdx.x & 15) * pitch + 16 * p) = out;
+        }
+    }
+    __syncthreads();
+    // ---- the products; slices of k in the order of linear_group_kernel: four sums over every fourth ----
+    f32x4 acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < steps; s0 += 2 * D) {
+#pragma unroll
+        for (int d = 0; d < 2 * D; ++d) {
+            const int s = s0 + d;
+            if (s >= steps) break;                        // uniform
+            const u32x4 fa = *reinterpret_cast<const u32x4*>(mixed + c16 * pitch + 64 * s + 16 * g4);
+            acc[d & 3] = mfma<IO>(fw[d % D], fa, acc[d & 3]);
+            if (s + D < steps) fw[d % D] = BufRaw<16>::ld(rsw, ow, 64u * (s + D));
+        }
+    }
+    const int m = m0 + c16;
+    if (m < M) finish<IO>(P, m, n0 + 4 * g4, (acc[0] + acc[1]) + (acc[2] + acc[3]));
+}
+
 // The same with 128 x 128 tiles staged in LDS, for 16-bit calls that fill enough compute units with them: 64 x 64 tiles read
 // every operand piece twice as often straight from the L2s (three of 3136 x 768 x 768: 43 us, with these 21 us).
 template <typename IO>
@@ -180,6 +312,36 @@ int linear_group(LinGroup& G, int dtype, hipStream_t st) {
     return check_launch("linear_group");
 }
 namespace {
+// 16-bit rows of few tokens: the rows normalised again grow with tokens, channels and results alike.  Twelve blocks, two launches / this one, us (the host
+// sets the pace of the small ones): 196 x 192 511 / 456 (replayed as a graph 424 / 383), 784 x 192 522 / 475, 1568 x 192 668 / 642, 3136 x 192 842 / 881;
+// 196 x 384 547 / 530, 392 x 384 601 / 607, 784 x 384 764 / 903; fp32 196 x 192 584 / 585, 784 x 192 618 / 635.
+constexpr long long LINEAR_MIX_PAIRS = 58000000, LINEAR_MIX_WIDE = 30000000;   // tokens x channels^2, with two rows a wave and with one
+bool linear_mix_takes(const LinGroup& G, const MixIn& X, int C, int dtype) {
+    const int es = 2, V = 16 / es, period = X.head_dim > 0 ? X.head_dim : C;
+    if (dtype == VRWKV_F32 || option(OPT_LINEAR_TILE) || C / V > WAVE || (long long)G.M * C * C > (C / V <= 32 ? LINEAR_MIX_PAIRS : LINEAR_MIX_WIDE) || C % V || X.g < 0 || X.g % V || period % V || 4LL * X.g > period || C % period) return false;
+    if (X.shift < 0 || X.Wp <= 0 || X.Hp <= 0 || X.shift > X.Wp || ((long long)X.Hp * X.Wp != X.T && (long long)X.Hp * X.Wp != X.T - 1)) return false;
+    for (int i = 0; i < G.n; ++i)
+        if (G.p[i].N % MIX_COLS) return false;
+    const long long rows = MIX_TOKENS + 2LL * X.shift * X.Wp;
+    return rows <= MIX_ROWS && (rows + MIX_TOKENS) * mix_pitch(C, es) <= 64 * 1024;
+}
+template <typename IO>
+void launch_mix(LinGroup& G, const MixIn& X, int C, hipStream_t st) {
+    int tiles = 0;
+    for (int i = 0; i < G.n; ++i) {
+        G.p[i].tile0 = tiles;
+        tiles += (G.M + MIX_TOKENS - 1) / MIX_TOKENS * (G.p[i].N / MIX_COLS);
+    }
+    const unsigned lds = (2 * MIX_TOKENS + 2 * X.shift * X.Wp) * mix_pitch(C, sizeof(IO));
+    if (C * (int)sizeof(IO) / 16 <= 32) hipLaunchKernelGGL((linear_mix_kernel<IO, true>), dim3(tiles), dim3(256), lds, st, G, X);
+    else hipLaunchKernelGGL((linear_mix_kernel<IO, false>), dim3(tiles), dim3(256), lds, st, G, X);
+}
+int linear_mix(LinGroup& G, const MixIn& X, int C, int dtype, hipStream_t st) {
+    if (dtype == VRWKV_BF16) launch_mix<__hip_bfloat16>(G, X, C, st);
+    else launch_mix<__half>(G, X, C, st);
+    return check_launch("linear_mix");
+}
+
 LinProblem linear(const void* a, const void* w, void* out, int N, int K, int lda = 0, int epi = 0) {
     return LinProblem{a, w, out, nullptr, nullptr, nullptr, N, K, lda ? lda : K, epi, 0, nullptr};
 }
@@ -363,18 +525,24 @@ static int block_fwd(const vrwkv_block_args* args, const vrwkv_block6_params* pa
         TRY(vrwkv_rowfuse(in, nullptr, w, b, nullptr, ln, M, C, 0, 0, eps, dt, st));
         return vrwkv_qshift_mix(ln, mix, out, n, B, T, C, a->Hp, a->Wp, a->shift_pixel, g, hd, dt, st);
     };
+    // ... and the projections of the mixes, in one launch where that is the faster way (problem i takes mix i)
+    auto mixed = [&](const void* in, const void* w, const void* b, float eps, const float* mix, void* const* out) -> int {
+        const MixIn X{in, w, b, mix, T, a->Hp, a->Wp, a->shift_pixel, g, hd, eps};
+        if (!a->post_norm && linear_mix_takes(G, X, C, dt)) return linear_mix(G, X, C, dt, st);
+        TRY(mixes(in, w, b, eps, mix, out, G.n, false));
+        return linear_group(G, dt, st);
+    };
     if (!a->post_norm) src = ln;
     char* half = at;                                      // both halves use what follows
     void* y;
     if (!H) {
         void* m[3] = {take(L.n), take(L.n), take(L.n)};
         void *k = take(L.n), *v = take(L.n), *r = take(L.n);
-        TRY(mixes(x, a->ln1_w, a->ln1_b, a->ln1_eps, a->att_mix, m, 3, false));
         G.n = 3;
         G.p[0] = linear(m[0], a->key, k, C, C);
         G.p[1] = linear(m[1], a->value, v, C, C);
         G.p[2] = linear(m[2], a->receptance, r, C, C);
-        TRY(linear_group(G, dt, st));
+        TRY(mixed(x, a->ln1_w, a->ln1_b, a->ln1_eps, a->att_mix, m));
         y = m[0];
         if (a->att_kn_w) {
             TRY(vrwkv_biwkv_fwd(a->w, a->u, k, v, m[1], B, T, C, dt, L.op ? op_ws : nullptr, L.op, st));
@@ -426,11 +594,10 @@ static int block_fwd(const vrwkv_block_args* args, const vrwkv_block6_params* pa
     TRY(residual(linear(y, a->output, nullptr, C, C), x, x1, a->gamma1, a->ln1_w, a->ln1_b, a->ln1_eps, ln));
     at = half;
     void *f[2] = {take(L.n), take(L.n)}, *fr = take(L.n), *ftmp = take(L.n);
-    TRY(mixes(x1, a->ln2_w, a->ln2_b, a->ln2_eps, a->ffn_mix, f, 2, false));
     G.n = 2;
     G.p[0] = linear(f[0], a->ffn_key, a->ffn_kn_w ? hid_raw : hid, hidden, C, 0, a->ffn_kn_w ? 0 : EPI_RELU_SQ);
     G.p[1] = linear(f[1], a->ffn_receptance, fr, C, C);
-    TRY(linear_group(G, dt, st));
+    TRY(mixed(x1, a->ln2_w, a->ln2_b, a->ln2_eps, a->ffn_mix, f));
     if (a->ffn_kn_w) TRY(vrwkv_rowfuse(hid_raw, nullptr, a->ffn_kn_w, a->ffn_kn_b, nullptr, hid, M, hidden, 1, 0, a->ffn_kn_eps, dt, st));
     LinProblem p = linear(hid, a->ffn_value, nullptr, C, hidden);
     p.gate = fr;
