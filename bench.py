@@ -142,8 +142,8 @@ def cpu_baseline(torch, n_calls):
 
 def wkv6_section(torch, ops, steps, warmup, with_cpu):
     """Secondary line of the metric: wkv6 forward at the VRWKV6-B shape (B=64, T=196, C=768, H=12,
-    bf16 r,k,v, fp32 w and y).  tokens/s = B*T per call; MFMA figures use the flops the chunked
-    kernel issues to the matrix cores (all split-bf16 products counted), end to end."""
+    bf16 r,k,v, fp32 w and y).  tokens/s = B*T per call; MFMA figures use the flops the kernel
+    issues to the matrix cores (all split-bf16 products counted), end to end."""
     Bw, Tw, Hw = 64, 196, 12
     Cw = Hw * 64
     dev = torch.device("cuda:0")
@@ -157,9 +157,12 @@ def wkv6_section(torch, ops, steps, warmup, with_cpu):
     us, reps = median_us(torch, fn, steps, warmup)
     r, k, v, w = sets[0]
     nchunk = (Tw + 31) // 32
-    # per chunk step a workgroup of eight waves issues 42 MFMA 16x16x32 per wave, 16384 flop each
+    # MFMA 16x16x32, 16384 flop each, of a sequence in two parts (csrc/wkv6_fwd_tile.h): two waves per 32 tokens, each 20 for a block of 32 tokens in
+    # front of it or behind and 26 for its own; 32 a block for the state a part leaves, 24 a wave for one that enters
     waves, mfma_per_wave_step, mfma_flop, mfma_cycles = 8, 42, 2 * 16 * 16 * 32, 16
-    mfma_flops = Bw * Hw * nchunk * waves * mfma_per_wave_step * mfma_flop
+    blocks = ((nchunk + 1) // 2, nchunk // 2)
+    products = sum(2 * n * (20 * (n - 1) + 26) + 32 * n for n in blocks) + 24 * (waves + (Tw - 32 * blocks[0] + 15) // 16)
+    mfma_flops = Bw * Hw * products * mfma_flop
     out = {
         "workload": f"wkv6 forward B={Bw} T={Tw} C={Cw} H={Hw}, bf16 r,k,v, fp32 w,y, {len(sets)} input sets in rotation",
         "us_per_call": round(us, 2),
@@ -169,8 +172,8 @@ def wkv6_section(torch, ops, steps, warmup, with_cpu):
         "mfma_issued_tflops": round(mfma_flops / (us * 1e-6) / 1e12, 2),
         "pct_bf16_mfma_peak_end_to_end": round(100.0 * mfma_flops / (us * 1e-6) / 2.5e15, 3),
     }
-    # Matrix-pipe share inside the contraction stage: the library's profiling entry runs the same kernel with the shader
-    # clock stamped by every wave on entering and leaving the matrix stage of every chunk step; a wave's 42 MFMAs occupy
+    # Matrix-pipe share inside the contraction stage of the chunked kernel (recorded 16-bit forwards, longer sequences): the
+    # library's profiling entry runs it with the shader clock stamped by every wave on entering and leaving the matrix stage of every chunk step; a wave's 42 MFMAs occupy
     # the pipe for 16 cycles each (measured: a chain of dependent v_mfma_f32_16x16x32_bf16 issues one per 16 cycles).
     try:
         import ctypes
@@ -192,7 +195,7 @@ def wkv6_section(torch, ops, steps, warmup, with_cpu):
         step = t[:, :, 1:, 0] - t[:, :, :-1, 0]
         busy = mfma_per_wave_step * mfma_cycles
         out["phases"] = {
-            "unit": "shader-clock cycles per wave and chunk step (mean over all waves and steps)",
+            "unit": "shader-clock cycles per wave and chunk step of the chunked kernel (mean over all waves and steps)",
             "matrix_stage": round(float(m_stage.mean()), 1), "elementwise_stage": round(float(e_stage.mean()), 1),
             "whole_step": round(float(step.mean()), 1),
             "mfma_pipe_cycles_per_wave_step": busy,
