@@ -374,7 +374,7 @@ class WKV_6(torch.autograd.Function):
     # 512 x 512 image and a class token -- and a sample's y is the same in any batch; that costs up to 66 us a layer (3 / 24 / 96
     # sequences of 1056 tokens: 92 / 94 / 95 us whole, 26 / 35 / 67 cut).  Longer chains cost more (2048 tokens: 175 whole, 34 to 115
     # cut) and are cut.  For the same reason it takes up to 256 tokens 32 at a time, not as one or two products: with those the gradients
-    # of VRWKV6-B (64 images, 196 tokens) move by 3.3e-2 at a last-bit difference of 7e-6 in y (62 us a layer of 257, 46 of 243).  The backward is cut from 257 tokens on in either type: gradients depend on the batch there, by 1.4e-2 in
+    # of VRWKV6-B (64 images, 196 tokens) move by 3.3e-2 at a last-bit difference of 7e-6 in y (62 us a layer in place of 46).  The backward is cut from 257 tokens on in either type: gradients depend on the batch there, by 1.4e-2 in
     # 16 bits.
     @staticmethod
     def stays_whole(T, dtype):
