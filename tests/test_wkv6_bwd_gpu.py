@@ -300,6 +300,30 @@ def test_cut_sequences_whose_parts_are_out_of_range(ops, T, segments, dtype):
     assert (got[4] - ref[4]).norm() <= 1.6e-5 * ref[4].norm()
 
 
+@pytest.mark.parametrize("T,segments", [(100, 0), (128, 0), (196, 0), (256, 0), (577, 5)])
+@pytest.mark.parametrize("dtype,log2_decay,size,gy_size", [
+    (torch.float32, 1.5, 1e-10, 1.), (torch.float32, 0.95, 1e-10, 1.), (torch.float32, 0.6, 1e-10, 1.), (torch.float32, 1.5, 1., 1e-12),
+    (torch.float32, 0.95, 3e10, 1.), (torch.bfloat16, 0.95, 3e10, 1.), (torch.float32, 1.5, 1e6, 1e6), (torch.float16, 1.5, 8e3, 1e3), (torch.float32, 1.5, 1., 1.)])
+def test_decays_over_a_part_with_rows_of_unusual_size(ops, dtype, log2_decay, size, gy_size, T, segments):
+    """The factors of a part reach 2^96 at 1.5 log2 a token: products of small rows times them would leave fp32 at its lower end, those of large ones at the
+    upper.  Against the sequential recurrence and sweeps with the bounds for rows of any size (see above)."""
+    B, H = 2, 2
+    C = 64 * H
+    g = torch.Generator(device="cuda").manual_seed(T)
+    r, k, v = ((torch.randn(B, T, C, generator=g, device="cuda") * size).to(dtype) for _ in range(3))
+    w = np.log(log2_decay * np.log(2)) + 0.02 * torch.randn(B, T, C, generator=g, device="cuda")
+    gy, u = torch.randn(B, T, C, generator=g, device="cuda") * gy_size, torch.randn(H, 64, generator=g, device="cuda") * 0.3
+    with ops.option("wkv6_segments", segments):
+        y, got = ops.wkv6_forward(B, T, C, H, r, k, v, w, u), ops.wkv6_backward(B, T, C, H, r, k, v, w, u, gy)
+    with ops.option("wkv6_fwd_scalar", 1), ops.option("wkv6_bwd_scalar", 1):
+        want, ref = ops.wkv6_forward(B, T, C, H, r, k, v, w, u), ops.wkv6_backward(B, T, C, H, r, k, v, w, u, gy)
+    error = lambda a, b: (a.double() - b.double()).norm()
+    for a, b in zip((y,) + tuple(got[:3]) + tuple(got[4:]), (want,) + tuple(ref[:3]) + tuple(ref[4:])):
+        assert error(a, b) <= 1.6e-5 * b.double().norm()
+    terms = w.double().exp() * ((r.double() * ref[0]).abs() + (k.double() * ref[1]).abs())
+    assert error(got[3], ref[3]) <= 1.6e-5 * T ** 0.5 * terms.norm()
+
+
 @pytest.mark.parametrize("T,segments", [(33, 2), (65, 3), (200, 3), (250, 8), (577, 5), (280, 9)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_backward_of_sequences_cut_into_segments(ops, T, segments, dtype):

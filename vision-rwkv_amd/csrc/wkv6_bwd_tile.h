@@ -25,8 +25,9 @@
 // results.  us there, sweeps -> here: bf16 197 -> 150, fp32 213 -> 185; one sequence 81 -> 48.  Measured and left out: rows brought into the L2s ahead
 // (166 -> 172), pieces of four channels (the loads' halves have to be moved: 166 -> 188), places in LDS with twice the bank conflicts (166 -> 167).
 //
-// Range: |P_end| <= 200 in a part, and 60 nats over 32 tokens as in the sweeps (gw is a difference of sums whose neighbouring tokens do not decay: the more
-// the others do, the less of it is left).  Sequences beyond go through the sweeps' code, which leaves the latter to the sequential sweeps.
+// Range: |P_end| <= 200 in a part, less for rows of unusual size (PART_FREE in wkv6_segment.h), and 60 nats over 32 tokens as in the sweeps (gw is a
+// difference of sums whose neighbouring tokens do not decay: the more the others do, the less of it is left).  Sequences beyond go through the sweeps' code,
+// which leaves the latter to the sequential sweeps.
 #pragma once
 #include "wkv6_bwd_sweep.h"
 
@@ -34,7 +35,6 @@ namespace vrwkv {
 namespace wkv6_detail {
 
 constexpr int BWD_TILE_TOKENS = 2 * PART;            // most tokens of an uncut sequence; a segment has PART
-constexpr float BWD_TILE_RANGE = 200.f;              // most log2 decay over a part
 
 // 32 rows (from row0) of an operand array (row_chunk) x 16 columns, 16 ct + c16, as an operand; slot (g4, e) is row 4 g4 + e (e < 4), 16 + 4 g4 + e - 4 (e >= 4)
 __device__ __forceinline__ bf16x8 tile_across(const unsigned char* arr, unsigned row0, int ct, int lane) {
@@ -63,7 +63,7 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
     constexpr unsigned LVH = 6 * ARR, LVL = 7 * ARR;                      // (KFH, KFL, RBH, RBL, GYH, GYL beside them)
     // scaled states, row j: 64 value channels, head and tail; apart the G that is formed or waits while the other is read
     constexpr unsigned ZS = 6 * ARR, ZG = 7 * ARR, ZG_BEHIND = 8 * ARR, ZG_FRONT = ZG_BEHIND, ZTAIL = ARR / 2, TAB = 9 * ARR;
-    struct Tables { float Tot[PART_WAVES][HN], Before[PART_WAVES][2][HN], Q[PART_WAVES][HN], X[2][HN]; };
+    struct Tables { float Tot[PART_WAVES][HN], Before[PART_WAVES][2][HN], Q[PART_WAVES][HN], X[2][HN], Max[PART_WAVES][4]; };
     __shared__ __attribute__((aligned(16))) unsigned char lds[TAB + sizeof(Tables)];
     __shared__ int sFlag;
     using Sweep = BwdLds<VSPLIT>;
@@ -265,10 +265,27 @@ void wkv6_bwd_tile_kernel(BwdArgs A)
                 total += t[g];
             }
             c_part = 0.5f * total;
-            bool in_range = total >= -BWD_TILE_RANGE;
+            bool in_range = total >= -PART_RANGE;
 #pragma unroll
             for (int g = 0; g < PART_WAVES; g += 2) in_range &= t[g] + t[g + 1] >= -SAFE_DECAY * LOG2E;
             if (__builtin_amdgcn_ballot_w64(!in_range) != 0ull) { bail = true; break; }                       // the same in every wave
+            if (__builtin_amdgcn_ballot_w64(!(total >= -PART_FREE)) != 0ull) {                                // ... and this
+                const float mr = largest_of_wave(mine ? largest16<IO>(rraw[0], rraw[1]) : 0.f), mk = largest_of_wave(mine ? largest16<IO>(kraw[0], kraw[1]) : 0.f),
+                            mv = largest_of_wave(mine ? largest16<IO>(vraw[0], vraw[1]) : 0.f), mg = largest_of_wave(mine ? largest16<float>(graw[0], graw[1]) : 0.f);
+                if (lane == 0) *reinterpret_cast<f32x4*>(L.Max[wave]) = f32x4{mr, mk, mv, mg};
+                lds_barrier();
+                f32x4 m = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int g = 0; g < PART_WAVES; ++g) {
+                    const f32x4 x = *reinterpret_cast<const f32x4*>(L.Max[g]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], x[e]);
+                }
+                const float lr = log2_of_largest(m[0]), lk = log2_of_largest(m[1]), lv = log2_of_largest(m[2]), lg = log2_of_largest(m[3]);
+                const float lo = fminf(lr, lk), hi = fmaxf(lr, lk);
+                const float smallest = fminf(fminf(lo, lo + lg + lv), fminf(lk + lv, lr + lg)), largest = fmaxf(fmaxf(hi, hi + lg + lv), fmaxf(lk + lv, lr + lg));
+                if (__builtin_amdgcn_ballot_w64(!(total >= -part_decay(smallest, largest))) != 0ull) { bail = true; break; }
+            }
             L.Before[wave][0][lane] = s - c_part;
             L.Before[wave][1][lane] = uj;
         }

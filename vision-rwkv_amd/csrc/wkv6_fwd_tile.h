@@ -24,8 +24,8 @@
 // matrix stage, and 768 sequences are one and a half rounds.  us, chunked kernel -> here, bf16 / fp32: 768 sequences of 196 tokens 65 -> 50 / 85 -> 71,
 // of 128 39 -> 22 / 56 -> 38, of 49 22 -> 15 / 31 -> 24; 3 sequences of 196 23.0 -> 16.8 / 23.2 -> 19.2.
 //
-// Range: |P_end| <= 200 in a part (factors up to 2^100 either way, e^-138 over it).  Sequences beyond go through the chunked kernel's code (range per 32
-// tokens, the sequential recurrence beyond that).
+// Range: |P_end| <= 200 in a part (e^-138 over it), less for rows of unusual size (PART_FREE in wkv6_segment.h).  Sequences beyond go through the chunked
+// kernel's code (range per 32 tokens, the sequential recurrence beyond that).
 #pragma once
 #include "wkv6_fwd_chunk.h"
 
@@ -34,7 +34,6 @@ namespace wkv6_detail {
 
 constexpr int TILE_TOKENS = 2 * PART;               // most tokens of a sequence or segment
 static_assert(PART_WAVES == FW_WAVES, "the chunked kernel's code runs on the same workgroup");
-constexpr float TILE_RANGE = 200.f;                  // most log2 decay over a part
 
 struct FwdTileArgs {
     const void *r, *k, *v, *w;
@@ -235,7 +234,21 @@ void wkv6_fwd_tile_kernel(FwdTileArgs A)
             own[lane] = s - 0.5f * total;
             own[HN + lane] = uj;
         }
-        if (__builtin_amdgcn_ballot_w64(!(total >= -TILE_RANGE)) != 0ull) { bail = true; break; }     // the same in every wave
+        if (__builtin_amdgcn_ballot_w64(!(total >= -PART_FREE)) != 0ull) {       // the same in every wave
+            const float mr = largest_of_wave(mine ? largest16<IO>(rraw[0], rraw[1]) : 0.f), mk = largest_of_wave(mine ? largest16<IO>(kraw[0], kraw[1]) : 0.f),
+                        mv = largest_of_wave(mine ? largest16<IO>(vraw[0], vraw[1]) : 0.f);
+            if (lane == 0) *reinterpret_cast<f32x4*>(lds + KFH + 2048 + 16 * wave) = f32x4{mr, mk, mv, 0.f};      // (behind the decay sums)
+            lds_barrier();
+            f32x4 m = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int g = 0; g < PART_WAVES; ++g) {
+                const f32x4 x = *reinterpret_cast<const f32x4*>(lds + KFH + 2048 + 16 * g);
+#pragma unroll
+                for (int e = 0; e < 3; ++e) m[e] = fmaxf(m[e], x[e]);
+            }
+            const float lr = log2_of_largest(m[0]), lk = log2_of_largest(m[1]), lkv = lk + log2_of_largest(m[2]);
+            if (__builtin_amdgcn_ballot_w64(!(total >= -part_decay(fminf(fminf(lr, lk), lkv), fmaxf(fmaxf(lr, lk), lkv)))) != 0ull) { bail = true; break; }
+        }
         lds_barrier();                               // the sums are read: their place is written below
         // bonus: sum_j r_t[j] u[j] k_t[j] of the lane's token, over the four lanes that share it
         f32x4 before[2][2];

@@ -199,6 +199,36 @@ __device__ __forceinline__ void summed_decays(const u32x4* raw, bool past, float
 
 constexpr int PART_WAVES = 8, PART = 16 * PART_WAVES;                     // waves of a workgroup, tokens it holds at a time
 
+// How far a part may decay.  The factors of wkv6_fwd_tile.h and wkv6_bwd_tile.h lie between 2^-c and 2^c, c = |P_end| / 2, on r, k, and through those on the
+// products of two or three rows that are summed next (k v, r gy, gy v r, gy v k), which have to stay in fp32: times 2^c below 2^114 (2^13 terms at most), and
+// times 2^-c above 2^-92 by the largest of the part (2^17 for the split operands' last bits and as much again for rows that are smaller than the largest).
+// c <= 100 in any case.  Up to c = 40, beyond which a model's decays hardly go, the data is not looked at: products from 2^-69 to 2^74 are good there, what
+// the chunked kernels ask for at the end of their own range (60 nats over 32 tokens).  What does not fit is those kernels'.  Looking costs the parts beyond
+// c = 40 a barrier and their rows' arrival ahead of it (64 x 196 x 768 bf16 forward 46.4 -> 47.6 to 49 us, backward 158 -> 170), the others nothing.
+constexpr float PART_FREE = 80.f, PART_RANGE = 200.f;                     // log2
+template <typename T>
+__device__ __forceinline__ float largest16(const u32x4* a, const u32x4* b) {         // |x| of a lane's 16 elements
+    float x[8], y[8], m = 0.f;
+    widen8<T>(a, x);
+    widen8<T>(b, y);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) m = fmaxf(m, fmaxf(fabsf(x[e]), fabsf(y[e])));
+    return m;
+}
+__device__ __forceinline__ float largest_of_wave(float m) {
+    m = fmaxf(m, dpp_get<0x111>(m));                 // row_shr:1, 2, 4, 8
+    m = fmaxf(m, dpp_get<0x112>(m));
+    m = fmaxf(m, dpp_get<0x114>(m));
+    m = fmaxf(m, dpp_get<0x118>(m));
+    const int x = __builtin_bit_cast(int, m);
+    auto row = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(x, l)); };
+    return fmaxf(fmaxf(row(15), row(31)), fmaxf(row(47), row(63)));
+}
+__device__ __forceinline__ float log2_of_largest(float m) { return m > 0.f ? __builtin_amdgcn_logf(m) : 0.f; }   // (rows of zeros take no part)
+__device__ __forceinline__ float part_decay(float smallest, float largest) {         // most log2 decay, from log2 of the products
+    return fminf(PART_RANGE, 2.f * fminf(92.f + smallest, 114.f - largest));
+}
+
 template <typename IO> struct SegLds {
     static constexpr bool VSPLIT = !__is_same(IO, __hip_bfloat16);
     __bf16 Ah[HN][PS], Al[HN][PS], Dh[HN][PS], Dl[HN][PS], Vt[HN][PS], Vtl[VSPLIT ? HN : 1][PS];   // [channel][token]
