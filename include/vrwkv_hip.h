@@ -123,14 +123,13 @@ int vrwkv_wkv6_fwd(const void* r, const void* k, const void* v, const void* w, c
 int vrwkv_wkv6_fwd_whole(const void* r, const void* k, const void* v, const void* w, const float* u, float* y,
                          int B, int T, int C, int H, int rkv_dtype, int w_dtype, int w_is_ew, void* hip_stream);
 
-/* Profiling twin of vrwkv_wkv6_fwd (no counterpart in the reference; for benchmarks and tuning): the chunked kernel
- * for bf16 r, k, v and fp32 raw-logit w, with every wave storing the shader clock at the boundaries of its stages
- * (that kernel serves sequences of more than 256 tokens; shorter ones are stamped in it and then run as they are).
+/* Profiling twin of vrwkv_wkv6_fwd_whole (no counterpart in the reference; for benchmarks and tuning): the chunked kernel
+ * for bf16 r, k, v and fp32 raw-logit w, with every wave storing the shader clock at the boundaries of its stages.
  * stamps: device buffer of vrwkv_wkv6_fwd_phases_bytes(B, T, H) bytes, laid out as uint64
  * [B*H][8 waves][ceil(T/32) chunk steps][8 points]: 0 element-wise stage entered, 1 its operands written (before the
  * barrier), 2 behind that barrier, 4 matrix stage entered, 5 y stored and the next decay sums formed (before the
  * barrier), 6 behind that barrier; 3 and 7 unused.  Waves 0-3 are the descending pass, 4-7 the ascending one.  y is
- * written as by vrwkv_wkv6_fwd.  Sequences whose decays fall outside the chunked kernel's range leave later steps
+ * that of vrwkv_wkv6_fwd_whole bit for bit.  Sequences whose decays fall outside the chunked kernel's range leave later steps
  * unstamped. */
 size_t vrwkv_wkv6_fwd_phases_bytes(int B, int T, int H);
 int vrwkv_wkv6_fwd_phases(const void* r, const void* k, const void* v, const void* w, const float* u,

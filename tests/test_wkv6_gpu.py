@@ -120,20 +120,21 @@ def test_error_behaviour(ops):
         ops.wkv6_forward(1, 4, 64, 1, x.cpu(), x, x, x, u)
 
 
-def test_phase_stamping_entry_point(ops):
+@pytest.mark.parametrize("T", [200, 300])
+def test_phase_stamping_entry_point(ops, T):
     """vrwkv_wkv6_fwd_phases (the chunked kernel writing a shader-clock stamp at six points of every wave's chunk
-    steps, which bench.py turns into its per-phase figures): same y as the plain entry point bit for bit, every stamp
+    steps, which bench.py turns into its per-phase figures): the chunked kernel's own y bit for bit, every stamp
     written, and the stamps of a wave in program order -- stage E entered, operands written, behind the barrier, matrix
     stage entered, y stored, behind the barrier -- within a step and from step to step.  Also its argument checks."""
     import ctypes
     lib = ops.lib()
     dev = "cuda:0"
-    B, T, H = 3, 200, 2
+    B, H = 3, 2
     C = H * 64
     r, k, v, w, u = gen(B, T, H, 77)
     tt = lambda a, d: torch.from_numpy(a).to(dev).to(d)
     rt, kt, vt, wt, ut = tt(r, torch.bfloat16), tt(k, torch.bfloat16), tt(v, torch.bfloat16), tt(w, torch.float32), tt(u, torch.float32)
-    want = ops.RUN_CUDA_RWKV6(B, T, C, H, rt, kt, vt, wt, ut)
+    want = ops.wkv6_forward(B, T, C, H, rt, kt, vt, wt, ut, whole=True)
     nb = lib.vrwkv_wkv6_fwd_phases_bytes(B, T, H)
     nchunk = (T + 31) // 32
     assert nb == B * H * 8 * nchunk * 8 * 8

@@ -184,9 +184,6 @@ extern "C" int vrwkv_wkv6_fwd_phases(const void* r, const void* k, const void* v
                        static_cast<const __hip_bfloat16*>(k), static_cast<const __hip_bfloat16*>(v),
                        static_cast<const float*>(w), u, y, T, C, H, B * H, 1, (const float*)nullptr, (const int*)nullptr,
                        static_cast<unsigned long long*>(stamps));
-    // (sequences that vrwkv_wkv6_fwd leaves to the tile kernel: y is that one's)
-    if (T <= TILE_TOKENS)
-        return launch_any<__hip_bfloat16, float>(r, k, v, w, u, y, nullptr, 0, B, T, C, H, false, false, static_cast<hipStream_t>(hip_stream));
     return check_launch("wkv6_fwd_phases");
 }
 
