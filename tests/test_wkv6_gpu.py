@@ -179,6 +179,28 @@ def test_cut_sequence_with_a_decay_out_of_range(ops):
     assert rel_err(y, clib.wkv6_fwd(*inputs, u, 2)) <= TOL
 
 
+@pytest.mark.parametrize("T,segments", [(300, 2), (577, 3), (2048, 8), (2080, 64), (2049, 17), (8300, 0)])
+@pytest.mark.parametrize("w_mean", [-3.0, -0.8, 0.2])
+def test_bf16_segments_of_two_parts_and_more_than_sixteen(ops, T, segments, w_mean):
+    """Segments of 129 to 256 tokens (forced, and as the plan has them beyond 8192 tokens) are two parts each, more than sixteen get their states from a launch
+    of its own; at 1.8 log2 a token the larger ones are out of a part's range and run the chunked kernel's code.  Against the sequential recurrence (bounds of
+    test_sequences_as_one_or_two_products); r alone off 4 bytes gives the same bits."""
+    H = 2
+    x = [torch.from_numpy(a).cuda() for a in gen(2, T, H, seed=T, w_mean=w_mean, w_std=0.05 if w_mean > -3 else 0.5)]
+    u = x.pop()
+    x = [a.to(torch.bfloat16) for a in x]
+    need = ops.lib().vrwkv_wkv6_fwd_workspace_bytes(2, T, 64 * H, H)
+    with ops.option("wkv6_segments", segments):
+        assert segments or need > 0
+        y = ops.wkv6_forward(2, T, 64 * H, H, *x, u)
+        x[0] = torch.empty(x[0].numel() + 1, dtype=torch.bfloat16, device="cuda")[1:].view_as(x[0]).copy_(x[0])
+        off = ops.wkv6_forward(2, T, 64 * H, H, *x, u)
+    with ops.option("wkv6_fwd_scalar", 1):
+        ref = ops.wkv6_forward(2, T, 64 * H, H, *x, u)
+    assert not torch.equal(y, ops.wkv6_forward(2, T, 64 * H, H, *x, u, whole=True))
+    assert (y - ref).norm() <= 1.6e-5 * ref.norm() and torch.equal(off, y)
+
+
 @pytest.mark.parametrize("T", [1, 15, 16, 17, 32, 33, 96, 127, 128, 129, 160, 161, 225, 256])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_sequences_as_one_or_two_products(ops, T, dtype):
