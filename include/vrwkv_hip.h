@@ -38,12 +38,13 @@ const char* vrwkv_last_error(void);      /* thread-local, never NULL */
 
 /* Tuning / testing switches, process-wide (no counterpart in the reference).  Names: "biwkv_l", "biwkv_s",
  * "biwkv_grid", "biwkv_no_stage", "biwkv_no_resident", "biwkv_bwd_serial", "wkv6_fwd_scalar", "wkv6_bwd_scalar",
- * "wkv6_bwd_unfused" (no effect: the backward is one kernel), "wkv6_segments", "linear_tile", "wgrad_splits"; 0 = default behaviour.  The initial value of <name> is
- * that of the environment variable VRWKV_<NAME> when the library first looks at any switch; the entry points never read the environment afterwards.
+ * "wkv6_bwd_unfused" (no effect: the backward is one kernel), "wkv6_segments", "linear_tile", "wgrad_splits", "linear_mix"; 0 = default behaviour.  The initial
+ * value of <name> is that of the environment variable VRWKV_<NAME> when the library first looks at any switch; the entry points never read the environment afterwards.
  * vrwkv_set_option rejects (VRWKV_INVALID_ARG) a value the plans would ignore: biwkv_l takes 0, 4, 8, 16, 25, 28 (tokens
  * per wave), biwkv_s 0 or 2..8 (waves per workgroup), biwkv_grid 0 or a positive workgroup count, wkv6_segments 0..64 (segments a sequence
- * is cut into), linear_tile 0, 1, 2, 4, 8 (16 to 128 results on a side), 16 (256 channels wide), wgrad_splits 0 or a positive count of token ranges, the
- * others 0 or 1. */
+ * is cut into), linear_tile 0, 1, 2, 4, 8 (16 to 128 results on a side), 16 (256 channels wide), wgrad_splits 0 or a positive count of token ranges,
+ * linear_mix 0, 1 (norm, shift and mixes inside the projections of a block's halves, VRWKV_UNSUPPORTED_SHAPE where the default would have them in front),
+ * 2 (in front), the others 0 or 1. */
 int vrwkv_set_option(const char* name, int value);
 int vrwkv_get_option(const char* name, int* value);
 

@@ -831,7 +831,8 @@ def test_norm_shift_and_mixes_in_one_launch(kind, C, dtype, hw, shift, batch, cl
     (320, torch.bfloat16, (4, 4), 1, 5, False), (384, torch.float16, (11, 17), 1, 1, True), (512, torch.bfloat16, (5, 3), 1, 1, False)])
 def test_norm_shift_and_mixes_inside_the_projections(C, dtype, hw, shift, batch, key_norm):
     """Tiles of 16 tokens across images and past the last one, rows of half a wave and more, up to all 64 rows a workgroup holds: bit for bit the block that
-    forms them in front of the projections, which a forced tile does (one order of the products in either)."""
+    forms them in front of the projections, which a forced tile does (one order of the products in either).  That the block by itself has them inside is
+    what the switch says, which makes anything else an error."""
     from vision_rwkv_amd import option
     net = _small_backbone("v4", C, dtype, key_norm, False, False, hw)
     for l in net.layers:
@@ -843,6 +844,29 @@ def test_norm_shift_and_mixes_inside_the_projections(C, dtype, hw, shift, batch,
             with option("linear_tile", 1):
                 want = l._native(x, hw)
             assert got is not None and torch.equal(got, want)
+            with option("linear_mix", 1):
+                assert torch.equal(l._native(x, hw), want)
+            with option("linear_mix", 2):
+                assert torch.equal(l._native(x, hw), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("C,dtype,hw,batch,inside", [
+    (64, torch.bfloat16, (2, 24), 1, True), (64, torch.bfloat16, (2, 25), 1, False),            # 64 and 66 rows of a workgroup
+    (256, torch.bfloat16, (17, 13), 4, True), (256, torch.bfloat16, (15, 12), 5, False),        # 884 and 900 tokens: 58.0 and 59.0 million by channels^2
+    (384, torch.float16, (7, 29), 1, False), (384, torch.float16, (29, 7), 1, True), (384, torch.float16, (17, 12), 1, False),      # 74 rows; 203 and 204 tokens
+    (576, torch.bfloat16, (1, 1), 1, False), (192, torch.float32, (2, 2), 1, False)])
+def test_which_blocks_have_norm_shift_and_mixes_inside_the_projections(C, dtype, hw, batch, inside):
+    """The rule's limits, on either side, by the switch that makes the other choice an error."""
+    from vision_rwkv_amd import option
+    l = _small_backbone("v4", C, dtype, False, False, False, hw).layers[0]
+    x = torch.randn(batch, hw[0] * hw[1], C, device="cuda").to(dtype)
+    with torch.no_grad(), option("linear_mix", 1):
+        if inside:
+            assert l._native(x, hw) is not None
+        else:
+            with pytest.raises(RuntimeError, match="not inside the projections"):
+                l._native(x, hw)
 
 
 @pytest.mark.gpu

@@ -528,7 +528,12 @@ static int block_fwd(const vrwkv_block_args* args, const vrwkv_block6_params* pa
     // ... and the projections of the mixes, in one launch where that is the faster way (problem i takes mix i)
     auto mixed = [&](const void* in, const void* w, const void* b, float eps, const float* mix, void* const* out) -> int {
         const MixIn X{in, w, b, mix, T, a->Hp, a->Wp, a->shift_pixel, g, hd, eps};
-        if (!a->post_norm && linear_mix_takes(G, X, C, dt)) return linear_mix(G, X, C, dt, st);
+        const int asked = option(OPT_LINEAR_MIX);
+        if (!a->post_norm && asked != 2 && linear_mix_takes(G, X, C, dt)) return linear_mix(G, X, C, dt, st);
+        if (asked == 1) {
+            set_error("block_fwd: norm, shift and mixes are not inside the projections of this call");
+            return VRWKV_UNSUPPORTED_SHAPE;
+        }
         TRY(mixes(in, w, b, eps, mix, out, G.n, false));
         return linear_group(G, dt, st);
     };

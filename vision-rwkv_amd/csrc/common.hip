@@ -22,7 +22,7 @@ void set_error(const char* fmt, ...) {
 namespace {
 const char* const kOptionNames[N_OPTIONS] = {
     "biwkv_l", "biwkv_s", "biwkv_grid", "biwkv_no_stage", "biwkv_no_resident", "biwkv_bwd_serial",
-    "wkv6_fwd_scalar", "wkv6_bwd_scalar", "wkv6_bwd_unfused", "wkv6_segments", "linear_tile", "wgrad_splits",
+    "wkv6_fwd_scalar", "wkv6_bwd_scalar", "wkv6_bwd_unfused", "wkv6_segments", "linear_tile", "wgrad_splits", "linear_mix",
 };
 std::atomic<int> g_options[N_OPTIONS];
 std::once_flag g_options_once;
@@ -83,6 +83,7 @@ extern "C" int vrwkv_set_option(const char* name, int value) {
     if (i == vrwkv::OPT_WKV6_SEGMENTS) ok = value >= 0 && value <= 64;
     if (i == vrwkv::OPT_LINEAR_TILE) ok = value == 0 || value == 1 || value == 2 || value == 4 || value == 8 || value == 16;
     if (i == vrwkv::OPT_WGRAD_SPLITS) ok = value >= 0;
+    if (i == vrwkv::OPT_LINEAR_MIX) ok = value >= 0 && value <= 2;
     if (!ok) {
         vrwkv::set_error("vrwkv_set_option: %d is no value of '%s'", value, name);
         return VRWKV_INVALID_ARG;

@@ -31,6 +31,7 @@ enum Option {
     OPT_WKV6_SEGMENTS,      // segments a wkv6 sequence is cut into
     OPT_LINEAR_TILE,        // tile of the block entry's projections (1, 2, 4, 8: 16 to 128 results on a side; 16: 256 channels wide)
     OPT_WGRAD_SPLITS,       // token ranges of a weight gradient
+    OPT_LINEAR_MIX,         // norm, shift and mixes inside a half's projections: 1 or an error, 2 never
     N_OPTIONS
 };
 int option(Option o);
