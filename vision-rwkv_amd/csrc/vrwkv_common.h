@@ -152,8 +152,9 @@ template <> struct BufRaw<8> {
 template <> struct BufRaw<16> {
     typedef unsigned int type __attribute__((ext_vector_type(4)));
     template <unsigned CP = 0> static __device__ __forceinline__ type ld(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned s) { return __builtin_amdgcn_raw_buffer_load_b128(r, v, s, CP); }
-    // The data stays in its registers for two cycles more.  A store of 16 bytes whose offset is a scalar register is held to need no wait before its data is
-    // overwritten; on gfx950 the fourth word of the last lanes was, now and then, the overwriting instruction's when that came next.
+    // The data stays in its registers for two cycles more.  The compiler leaves none between a store of 16 bytes whose offset is a scalar register and an
+    // instruction that overwrites its data.  In one kernel (fp32 results of the segmented wkv6 backward) the fourth word of the last lanes was then, now and
+    // then, the overwriting instruction's, and with the two cycles no more: an observation of that kernel on gfx950, not a documented property.
     template <unsigned CP = 0> static __device__ __forceinline__ void st(type d, __amdgpu_buffer_rsrc_t r, unsigned v, unsigned s) {
         __builtin_amdgcn_raw_buffer_store_b128(d, r, v, s, CP);
         asm volatile("s_nop 1" : : "v"(d));

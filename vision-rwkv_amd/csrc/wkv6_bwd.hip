@@ -55,10 +55,12 @@ void round_kernel(const float* __restrict__ x, OT* __restrict__ y, size_t n) {
 }
 
 // Uncut sequences in one or two products (wkv6_bwd_tile.h).  By length and type alone, so that a sample's gradients do not depend on the batch.  Two parts
-// are three steps whatever the second one holds: up to 160 tokens (fp32, which spills, 192) the sweeps' five (six) chunks are ahead where compute units have
-// two sequences each.  us, sweeps -> products: 64 x 12 sequences of 128 tokens, bf16 119 -> 73, fp32 128 -> 90; of 129, fp16 141 -> 141, fp32 148 -> 166; of
-// 196, bf16 197 -> 155, fp16 195 -> 167, fp32 213 -> 193; of 256, fp16 232 -> 180, fp32 254 -> 213; 22 x 12 of 129, fp16 85 -> 92; of 161, fp16 99 -> 97,
-// fp32 99 -> 108; of 196, fp32 113 -> 119; 8 x 3 of 196, bf16 81 -> 50, fp32 77 -> 58.
+// are three steps whatever the second one holds, the sweeps a step of two barriers more for every 32 tokens: short ones stay with the sweeps for the calls that
+// give every compute unit one to two sequences, where the sweeps run two at a time and the parts one.  us, sweeps -> products, 64 x 12 sequences: of 128 tokens
+// bf16 119 -> 71, fp32 126 -> 84; of 196 bf16 195 -> 152, fp16 190 -> 160, fp32 207 -> 186; of 256 bf16 230 -> 164, fp16 224 -> 172, fp32 249 -> 206.  At the
+// limits, 3 / 256 / 264 / 512 / 768 sequences: of 160 tokens bf16 60 -> 44, 65 -> 49, 87 -> 87, 92 -> 90, 146 -> 132, fp16 58 -> 45, 64 -> 51, 85 -> 91, 92 -> 94,
+// 145 -> 137; of 192 fp32 64 -> 52, 74 -> 63, 98 -> 109, 122 -> 118, 190 -> 175; of 193 fp32 73 -> 55, 83 -> 65, 110 -> 114, 131 -> 124, 204 -> 186.  (257 to 384
+// fp32 sequences of 193 to 224 tokens are 1 to 7 % behind the sweeps for it.)
 bool bwd_tile_takes(int T, int rkv_dtype) {
     return T <= PART || (T > (rkv_dtype == VRWKV_F32 ? 192 : 160) && T <= BWD_TILE_TOKENS);
 }
@@ -66,8 +68,8 @@ bool bwd_tile_takes(int T, int rkv_dtype) {
 // Segments per sequence of a call (1: not cut); OPT_WKV6_SEGMENTS forces a number (testing).  parts: of 128 tokens, one part of wkv6_bwd_tile.h each.  Those
 // take three launches and BWD_PARTS_US whatever the sequences' number and length, as long as every segment has a compute unit and there are not more than
 // sixteen in a sequence (each folds the states of all others); the sweeps are ahead where they find short segments for all of them.  us, sweeps -> parts,
-// bf16 / fp32: 48 sequences of 577 tokens 80 -> 55 / 79 -> 65, of 400 84 -> 51 / 85 -> 60, 24 of 1024 87 -> 51 / 92 -> 62, 12 of 1025 77 -> 50 / 80 -> 59,
-// 24 of 577 57 -> 47 / 59 -> 58, 24 of 300 43 -> 45 / 43 -> 55, 3 of 577 41 -> 44 / 42 -> 53.
+// bf16 / fp32: 48 sequences of 577 tokens 74 -> 43 / 76 -> 51, of 400 80 -> 41 / 82 -> 48, 24 of 1024 85 -> 43 / 90 -> 50, 12 of 1025 78 -> 42 / 81 -> 48 (the
+// sweeps' estimate is too low there for fp32 to take it), 24 of 577 59 -> 41 / 61 -> 47 (fp32 likewise), 24 of 300 43 -> 39 / 43 -> 45, 3 of 577 41 -> 39 / 41 -> 44.
 constexpr int BWD_TILE_SEGMENTS = 16;
 constexpr double BWD_PARTS_US[3] = {59.5, 52., 55.};    // VRWKV_F32, VRWKV_BF16, VRWKV_F16
 int segments(int B, int T, int H, int rkv_dtype, bool& parts) {

@@ -22,7 +22,7 @@
 //
 // Bound by latency and vector work: two waves a SIMD issue 6 200 vector instructions, 730 products and 970 LDS accesses each at 64 x 196 x 768, matrix cores
 // busy 19 %, LDS 25 %, vector ALUs 40 %; of a full part's 42 000 cycles 6 500 wait for its rows, 4 500 form operands, 11 000 + 7 000 are products and 8 000 the
-// results.  us there, sweeps -> here: bf16 197 -> 150, fp32 213 -> 185; one sequence 81 -> 48.  Measured and left out: rows brought into the L2s ahead
+// results.  us there, sweeps -> here: bf16 195 -> 152, fp32 207 -> 186; one sequence 79 -> 49.  Measured and left out: rows brought into the L2s ahead
 // (166 -> 172), pieces of four channels (the loads' halves have to be moved: 166 -> 188), places in LDS with twice the bank conflicts (166 -> 167).
 //
 // Range: |P_end| <= 200 in a part, less for rows of unusual size (PART_FREE in wkv6_segment.h), and 60 nats over 32 tokens as in the sweeps (gw is a

@@ -36,7 +36,7 @@ int validate(int B, int T, int C, int H, int rkv_dtype, int w_dtype) {
     return VRWKV_OK;
 }
 
-// Segments per sequence of a call (1: not split); OPT_WKV6_SEGMENTS forces a number (testing).  parts: the tile kernels run them (bf16).
+// Segments per sequence of a call (1: not split); OPT_WKV6_SEGMENTS forces a number (testing).  parts: the tile kernels run them.
 int segments(int B, int T, int H, int rkv_dtype, bool& parts) {
     const int nchunk = (T + LC - 1) / LC, forced = option(OPT_WKV6_SEGMENTS);
     if (forced > 0 && (long long)B * H <= SEG_SEQUENCES) {
@@ -103,8 +103,8 @@ int launch_chunked(const void* r, const void* k, const void* v, const void* w, c
         if (!own) hipLaunchKernelGGL((wkv6_seg_fold_kernel<2, false>), dim3(4, 2, (unsigned)sequences), dim3(256), 0, st, states, nseg);
     }
     // Up to 256 tokens in one or two parts (the tile kernel is ahead of the chunked one at every size measured, 3 to 768 sequences of 33 to 256 tokens in
-    // all types: 1.03 to 1.8 times, least where a second part is nearly empty); more tokens, and calls that ask for it (vrwkv_wkv6_fwd_whole),
-    // are the chunked kernel's.
+    // all types: 1.03 to 1.8 times, least where a second part is nearly empty); more tokens uncut, and calls that ask for it (vrwkv_wkv6_fwd_whole),
+    // are the chunked kernel's, cut sequences the tile kernel's where their segments are parts.
     const FwdTileArgs tile{r, k, v, w, u, y, T, C, H, (int)sequences, nseg, states, flags, own};
     if (nseg == 1 && T <= TILE_TOKENS && !whole) {
         if constexpr (sizeof(IO) == 2) {

@@ -14,15 +14,15 @@
 // Against the chunked kernel (two passes of 32-token chunks) a token and channel is prepared once and not twice, with three exponentials instead of
 // six, the 64 x 64 states are scaled and split once per part and not once per chunk, and y is not fetched again.
 //
-// A workgroup of eight waves holds a part, two share a compute unit; a wave owns 16 tokens.  Element-wise stage: lane = (token c16, eight
+// A workgroup of eight waves holds a part, two (fp16 and fp32, whose v is split: one) share a compute unit; a wave owns 16 tokens.  Element-wise stage: lane = (token c16, eight
 // channels of each half), the layout of the matrix operands, so rf and rb stay in registers and kf, kb, v (head and tail) leave for LDS in 16-byte pieces;
 // the decays are summed along a row of 16 lanes, then over the waves.  Matrix stage, no barrier inside: the wave walks the 32-token blocks of the part's
 // tokens i, A^T leaves its accumulators as the next product's operand, v is read across with ds_read_b64_tr_b16, y is transposed in accumulators.
 // Computed operands are split into bf16 head + tail, products head*head + head*tail + tail*head, as in the chunked kernel.
 //
-// Bound by latency: the two workgroups of a compute unit spend a third of their time on rows on their way, each part is a chain of an element-wise and a
-// matrix stage, and 768 sequences are one and a half rounds.  us, chunked kernel -> here, bf16 / fp32: 768 sequences of 196 tokens 65 -> 50 / 85 -> 71,
-// of 128 39 -> 22 / 56 -> 38, of 49 22 -> 15 / 31 -> 24; 3 sequences of 196 23.0 -> 16.8 / 23.2 -> 19.2.
+// Bound by latency: the workgroups of a compute unit spend a third of their time on rows on their way, each part is a chain of an element-wise and a
+// matrix stage, and 768 sequences are one and a half rounds.  us, chunked kernel -> here, bf16 / fp32: 768 sequences of 196 tokens 62 -> 46 / 80 -> 67,
+// of 128 36 -> 22 / 51 -> 35, of 49 22 -> 15 / 31 -> 22; 3 sequences of 196 23.0 -> 16.9 / 23.6 -> 18.7.
 //
 // Range: |P_end| <= 200 in a part (e^-138 over it), less for rows of unusual size (PART_FREE in wkv6_segment.h).  Sequences beyond go through the chunked
 // kernel's code (range per 32 tokens, the sequential recurrence beyond that).

@@ -21,6 +21,7 @@
 namespace vrwkv {
 namespace wkv6_detail {
 
+constexpr int PART_WAVES = 8, PART = 16 * PART_WAVES;   // waves of a workgroup of the tile kernels, tokens it holds at a time
 constexpr int SEG_MAX = 64;                          // segments per sequence (one flag per lane of a wave)
 constexpr int SEG_SEQUENCES = 65535;                 // sequences of a cut call (the fold kernel's grid; by the rule below, 4 per CU at most)
 constexpr int SEG_STATE = HN * HN;                   // floats of one state
@@ -92,14 +93,15 @@ inline int wkv6_fwd_segments(long long sequences, int nchunk, int cus, int type,
         const double t = cps * k.step[per_cu - 1] + k.fixed + k.per_segment * nseg + k.traffic * 1e-3 * (double)(sequences * nseg) + k.token_traffic * chunks;
         if (t < best_time) { best = nseg; best_time = t; }
     }
-    if (type == 1) {
-        const int cps = std::max(4, (nchunk + SEG_MAX - 1) / SEG_MAX), nseg = (nchunk + cps - 1) / cps;
+    constexpr int part = PART / LC;                  // chunks of a part
+    if (type == VRWKV_BF16) {
+        const int cps = std::max(part, (nchunk + SEG_MAX - 1) / SEG_MAX), nseg = (nchunk + cps - 1) / cps;
         const double t = std::max(19.0 + 0.45 * nseg, 15.0 + 0.25 * nseg + 0.052 * (double)(sequences * nseg));
-        parts = t < (best == 1 ? 0.84 : 1.0) * best_time && cps * LC <= 2 * 128;
+        parts = t < (best == 1 ? 0.84 : 1.0) * best_time && cps <= 2 * part;
         if (parts) return nseg;
     } else {
-        const int nseg = (nchunk + 3) / 4;
-        const double t = (type == 0 ? 21.5 : 19.0) + 0.4 * nseg + 0.01 * (double)(sequences * nseg);
+        const int nseg = (nchunk + part - 1) / part;
+        const double t = (type == VRWKV_F32 ? 21.5 : 19.0) + 0.4 * nseg + 0.01 * (double)(sequences * nseg);
         parts = nseg <= FOLD_SEGMENTS && padded * nseg <= cus && t < (best == 1 ? 0.73 : 0.95) * best_time;
         if (parts) return nseg;
     }
@@ -196,8 +198,6 @@ __device__ __forceinline__ void summed_decays(const u32x4* raw, bool past, float
         x[e] = d;
     }
 }
-
-constexpr int PART_WAVES = 8, PART = 16 * PART_WAVES;                     // waves of a workgroup, tokens it holds at a time
 
 // How far a part may decay.  The factors of wkv6_fwd_tile.h and wkv6_bwd_tile.h lie between 2^-c and 2^c, c = |P_end| / 2, on r, k, and through those on the
 // products of two or three rows that are summed next (k v, r gy, gy v r, gy v k), which have to stay in fp32: times 2^c below 2^114 (2^13 terms at most), and
